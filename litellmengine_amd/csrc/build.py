@@ -31,6 +31,7 @@ LIBRARIES: Dict[str, List[str]] = {
     "rope_kv": ["rope_kv.hip"],
     "attention": ["attention.hip"],
     "gemm": ["gemm.hip"],
+    "gemm_f32": ["gemm_f32.hip"],
     "sampling": ["sampling.hip"],
     "recurrent": ["recurrent.hip"],
     "latent": ["latent.hip"],

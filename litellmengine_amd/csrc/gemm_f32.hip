@@ -1,0 +1,253 @@
+// The float32 product of many rows, C[M, N] = A[M, K] . B[N, K]^T, on the bfloat16 matrix cores without losing a bit of
+// an operand.  A float32 number is the sum of three bfloat16 numbers, x = x1 + x2 + x3 (x1 = x rounded, x2 = what is left
+// rounded, x3 = the rest: 3 x 8 significand bits and two signs hold 24), so
+//   a b = a1 b1 + (a1 b2 + a2 b1) + (a1 b3 + a2 b2 + a3 b1) + what is below 2^-26 of it,
+// six products of the bfloat16 matrix instruction, each exact, added up in float32: less is lost than one float32
+// rounding of a b.  The float32 matrix instruction does 157 TFLOP/s, the bfloat16 one 2500, a sixth of which is 417.
+#include "common.h"
+#include <math.h>
+
+LLE_DEFINE_ERROR_STRING()
+
+typedef bf16_t sbf16x8 __attribute__((ext_vector_type(8)));
+typedef float sf32x4 __attribute__((ext_vector_type(4)));
+typedef float sf32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t su32x4 __attribute__((ext_vector_type(4)));
+
+#define SG_BK 32      // columns of K per step
+#define SG_PIECES 4   // 8-element pieces of a row of a step
+
+// two numbers as their three bfloat16 parts, packed
+__device__ __forceinline__ void split2(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
+    typedef bf16_t pair __attribute__((ext_vector_type(2)));
+    typedef float fpair __attribute__((ext_vector_type(2)));
+    auto pack = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(fpair{x, y}, pair)); };
+    p1 = pack(a, b);
+    a -= __builtin_bit_cast(float, p1 << 16);
+    b -= __builtin_bit_cast(float, p1 & 0xffff0000u);
+    p2 = pack(a, b);
+    a -= __builtin_bit_cast(float, p2 << 16);
+    b -= __builtin_bit_cast(float, p2 & 0xffff0000u);
+    p3 = pack(a, b);
+}
+
+// Tiles of 64 TM rows of A x 64 TN rows of B, four wavefronts of 32 TM x 32 TN.  A step of 32 columns is asked for while the
+// one before is multiplied, split in registers on its way to LDS (one buffer; two or more workgroups a CU fill each other's
+// gaps), its 16-byte pieces XOR-swizzled by the row, so that no read meets a bank conflict.  blockIdx.y: a slice of K, whose
+// sums go to C + blockIdx.y * M * N.
+//
+// Bound by the matrix cores: at 2048 x 24576 x 4096 the 256 x 128 tiles keep them busy 0.77 of the time, at the 1.8 GHz that
+// their power leaves: 1800 us, 229 TFLOP/s of float32 product (1.37 PFLOP/s of the instruction); the float32 instruction, in
+// 64 x 64 tiles, took 4160 us.  2048 x 4096 x 12288: 965 us against 1774; 2048 x 4096 x 4096: 321 against 590.  The error
+// against 64 bits is a tenth smaller (1.0e-6 against 1.1e-6 at K = 4096): fewer, exact products per rounding of a sum.
+template <int TM, int TN, int PER_SIMD>
+__global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                                      float* __restrict__ C, int M, int N, int K, int64_t lda,
+                                                                      int64_t ldb, int64_t ldc, int m_tiles, int n_tiles, int slice) {
+    constexpr int BM = 64 * TM, BN = 64 * TN;
+    extern __shared__ __attribute__((aligned(16))) unsigned char sg_lds[];
+    unsigned char* as = sg_lds;                            // [3 parts][BM][4 pieces of 16 bytes]
+    unsigned char* bs = sg_lds + 3 * BM * SG_BK * 2;       // [3 parts][BN][4 pieces]
+    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
+    // consecutive workgroups go to different dies: a die takes every eighth column of tiles, all its row tiles one after the
+    // other, so that its L2 sees few rows of B at a time
+    const int die = blockIdx.x % 8, at = blockIdx.x / 8;
+    const int nt = die + 8 * (at / m_tiles), mt = at % m_tiles;
+    if (nt >= n_tiles) return;
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int k_begin = blockIdx.y * slice, k_end = min(K, k_begin + slice);  // (a slice is a whole number of steps)
+    C += (int64_t)blockIdx.y * M * N;
+    // the copy: thread -> (row of 64, piece)
+    const int lr = threadIdx.x / SG_PIECES, lp = threadIdx.x % SG_PIECES;
+    const float *ap[TM], *bp[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) ap[i] = A + (int64_t)min(m0 + 64 * i + lr, M - 1) * lda;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bp[j] = B + (int64_t)min(n0 + 64 * j + lr, N - 1) * ldb;
+    const int dst = lr * (SG_BK * 2) + ((lp ^ ((lr >> 3) & 3)) * 16);
+    sf32x4 ar[TM][2], br[TN][2];
+    auto issue = [&](int k0) {
+        const int ka = min(k0 + 8 * lp, K - 4), kb = min(k0 + 8 * lp + 4, K - 4);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) ar[i][0] = *(const sf32x4*)(ap[i] + ka), ar[i][1] = *(const sf32x4*)(ap[i] + kb);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) br[j][0] = *(const sf32x4*)(bp[j] + ka), br[j][1] = *(const sf32x4*)(bp[j] + kb);
+    };
+    auto store = [&](unsigned char* base, int rows, int i, const sf32x4* v) {
+        su32x4 p1, p2, p3;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            uint32_t q1, q2, q3;
+            split2(v[h / 2][2 * (h % 2)], v[h / 2][2 * (h % 2) + 1], q1, q2, q3);
+            p1[h] = q1, p2[h] = q2, p3[h] = q3;
+        }
+        unsigned char* d = base + 64 * i * (SG_BK * 2) + dst;
+        *(su32x4*)d = p1;
+        *(su32x4*)(d + rows * SG_BK * 2) = p2;
+        *(su32x4*)(d + 2 * rows * SG_BK * 2) = p3;
+    };
+    const int wm = (wave / 2) * 32 * TM, wn = (wave % 2) * 32 * TN;
+    sf32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    // fragments of 32 rows x 16 columns: lane -> row lane % 32, eight columns from 8 (lane / 32) on
+    const int fr = lane % 32, fh = lane / 32;
+    const unsigned char* af = as + (wm + fr) * (SG_BK * 2);
+    const unsigned char* bf = bs + (wn + fr) * (SG_BK * 2);
+
+    issue(k_begin);
+    for (int k0 = k_begin; k0 < k_end; k0 += SG_BK) {
+        if (k0 + SG_BK > K) {  // past the end: zeros for A (B's repeated columns then count for nothing)
+            const sf32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (k0 + 8 * lp + 4 * h >= K) ar[i][h] = zero;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) store(as, BM, i, ar[i]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) store(bs, BN, j, br[j]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        issue(k0 + SG_BK);  // on its way while this step is multiplied (past the end: the last columns again)
+        __builtin_amdgcn_sched_barrier(0);  // (the compiler would ask for it where it is needed)
+        __builtin_amdgcn_s_setprio(1);  // matrix instructions ahead of the other workgroup's splitting: 3 % at 2048 x 24576 x 4096
+#pragma unroll
+        for (int s = 0; s < SG_BK / 16; ++s) {
+            const int piece = ((2 * s + fh) ^ ((fr >> 3) & 3)) * 16;
+            sbf16x8 b[TN][3];
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) b[j][p] = *(const sbf16x8*)(bf + (p * BN + 32 * j) * SG_BK * 2 + piece);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                sbf16x8 a[3];
+#pragma unroll
+                for (int p = 0; p < 3; ++p) a[p] = *(const sbf16x8*)(af + (p * BM + 32 * i) * SG_BK * 2 + piece);
+                // the smallest products first
+                constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[q]], b[j][pb[q]], acc[i][j], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // nobody reads this step any more
+    }
+    // lane holds C[m = 8 (e / 4) + 4 (lane / 32) + e % 4][n = lane % 32] of every 32 x 32 tile
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
+                const float v = acc[i][j][e];
+                odd |= (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u;
+                if (m < M && n < N) C[m * ldc + n] = v;
+            }
+    // An infinity has no parts (inf - inf is no number), and numbers within 2^-9 of the largest one round to infinity: a result
+    // that is not finite is made again in plain float32.
+    if (!odd) return;
+    for (int t = 0; t < TM * TN * 16; ++t) {
+        const int e = t % 16, j = t / 16 % TN, i = t / 16 / TN;
+        const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
+        if (m >= M || n >= N || (__builtin_bit_cast(uint32_t, C[m * ldc + n]) & 0x7f800000u) != 0x7f800000u) continue;
+        float v = 0.f;
+        for (int k = k_begin; k < k_end; ++k) v = fmaf(A[m * lda + k], B[n * ldb + k], v);
+        C[m * ldc + n] = v;
+    }
+}
+
+template <int TM, int TN, int PER_SIMD>
+static int launch_split(const float* A, const float* B, float* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+                        int slices, hipStream_t stream) {
+    constexpr int lds = 3 * 64 * (TM + TN) * SG_BK * 2;
+    const int m_tiles = (M + 64 * TM - 1) / (64 * TM), n_tiles = (N + 64 * TN - 1) / (64 * TN);
+    static bool ready = false;  // more than 64 KB of LDS has to be asked for once
+    if (!ready) {
+        if (hipFuncSetAttribute((const void*)gemm_nt_split_kernel<TM, TN, PER_SIMD>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+            return (int)hipGetLastError();
+        ready = true;
+    }
+    const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
+    if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
+    const int steps = (K + SG_BK - 1) / SG_BK, slice = (steps + slices - 1) / slices * SG_BK;
+    gemm_nt_split_kernel<TM, TN, PER_SIMD><<<dim3((int)blocks, slices), 256, lds, stream>>>(A, B, C, M, N, K, lda, ldb, ldc, m_tiles,
+                                                                                         n_tiles, slice);
+    LLE_RETURN_LAUNCH_STATUS();
+}
+
+// The tiles, and what a step of one costs (us): alone on a CU, and each of several that share one.  Large tiles read less and
+// lose where they leave CUs without work; measured over M from 66 to 2048 (see choose).
+struct SplitTile {
+    int tm, tn;
+    float alone, shared;
+};
+static const SplitTile split_tiles[4] = {{4, 2, 2.70f, 2.35f}, {2, 2, 1.63f, 1.28f}, {2, 1, 1.09f, 0.74f}, {1, 1, 0.70f, 0.43f}};
+
+static int units_of_device() {
+    static int units[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (units[dev] == 0 && hipDeviceGetAttribute(&units[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) units[dev] = 256;
+    return units[dev];
+}
+
+// The tiles, and the slices of K (up to `most`), that take the least time by the steps of the CU with the most tiles, plus the
+// way of the slices' sums to their reader and back at 5 TB/s.
+static void choose(int M, int N, int K, int most, int& tiles, int& slices) {
+    const int units = units_of_device(), steps = (K + SG_BK - 1) / SG_BK;
+    float best = 0.f;
+    tiles = 0, slices = 1;
+    for (int s = 1; s <= most; ++s)
+        for (int t = 0; t < 4; ++t) {
+            const SplitTile& v = split_tiles[t];
+            const int64_t count = (int64_t)((M + 64 * v.tm - 1) / (64 * v.tm)) * ((N + 64 * v.tn - 1) / (64 * v.tn)) * s;
+            const float each = fmaxf(v.alone, (float)((count + units - 1) / units) * v.shared);
+            const float us = (float)((steps + s - 1) / s) * each + (s > 1 ? (float)s * M * N * 8 / 5e6f : 0.f);
+            if (best == 0.f || us < best) best = us, tiles = t, slices = s;
+        }
+}
+
+// In how many slices of K (up to 8) a product is taken whose reader adds up partial sums; 1: whole.
+extern "C" int lle_gemm_nt_f32_slices(int M, int N, int K) {
+    int tiles, slices;
+    if (M <= 0 || N <= 0 || K <= 0) return 1;
+    choose(M, N, K, 8, tiles, slices);
+    return slices;
+}
+
+// float32 in, float32 out; K, lda and ldb multiples of 4.  slices > 1: C is [slices][M][N], contiguous, the sums of equal parts
+// of K (rounded up to whole steps).  tiles: which of split_tiles, below zero for the one that takes the least time.
+extern "C" int lle_gemm_nt_f32(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+                               int slices, int tiles, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || K % 4 != 0 || lda % 4 != 0 || ldb % 4 != 0 || slices < 1 || slices > 65535) return (int)hipErrorInvalidValue;
+    if (slices > 1 && ldc != N) return (int)hipErrorInvalidValue;
+    if (tiles < 0) {
+        int unused;
+        // (a slice's product is as long as a whole one of its part of K)
+        choose(M, N * slices, (K + slices - 1) / slices, 1, tiles, unused);
+    }
+    const float *a = (const float*)A, *b = (const float*)B;
+    float* c = (float*)C;
+    switch (tiles) {
+        case 0: return launch_split<4, 2, 2>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 1: return launch_split<2, 2, 3>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 2: return launch_split<2, 1, 4>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 3: return launch_split<1, 1, 6>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        default: return (int)hipErrorInvalidValue;
+    }
+}

@@ -296,9 +296,9 @@ class HipOps:
 
     def linear(self, x, weight, out_dtype=None, fold=None, sums_ok=False):
         """x [M, K] . weight [N, K]^T -> [M, N].  With `sums_ok` the caller takes the result also as
-        PartialSums (float32 [slices, M, N], what add_rmsnorm adds into the residual stream).  float32 operands take a true 32-bit
-        product: few rows the weight-streaming kernel, more rows a tiled kernel, both
-        with the float32 matrix instruction; the plain-FMA kernel where K is no multiple of 4.  bfloat16 operands: few rows take the
+        PartialSums (float32 [slices, M, N], what add_rmsnorm adds into the residual stream).  float32 operands take a
+        32-bit product: few rows the weight-streaming kernel (float32 matrix instruction), more rows a tiled kernel
+        (operands split exactly into three bfloat16 parts); the plain-FMA kernel where K is no multiple of 4.  bfloat16 operands: few rows take the
         weight-streaming matrix-core kernel, more rows the library product; both
         accumulate in 32-bit and write either result type.  `x` a Prenormed or `fold`
         a NormFold: see _linear_folded."""
@@ -338,19 +338,47 @@ class HipOps:
             # the library product accumulates in 32-bit and can leave the result so
             return torch.mm(x, weight.t()) if out_dtype == torch.bfloat16 else torch.mm(x, weight.t(), out_dtype=out_dtype)
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
-        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        if M <= self.tuning.skinny_f32_max_rows and K % 4 == 0 and not self.force_library_gemm:
+        # (up to 16 columns are one step of one of the weight-streaming kernel's sixteen wavefronts: nothing to stream, and in
+        # the tiles' kernel a row's result does not depend on how many rows there are)
+        if M <= self.tuning.skinny_f32_max_rows and K % 4 == 0 and K > 16 and not self.force_library_gemm:
+            out = torch.empty((M, N), dtype=out_dtype, device=x.device)
             # few rows: W streamed once, float32 matrix instruction
             self._run("gemm", "lle_gemm_skinny_f32", [_P, _P, _P, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
                       M, N, K)
             return out
         if K % 4 == 0 and not self.force_simt_gemm:
-            # many rows: 64 x 64 tiles through the float32 matrix instruction
-            self._run("gemm", "lle_gemm_nt_mfma_f32", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _P],
-                      _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N)
-            return out
+            slices = self.f32_slices_for(M, N, K) if sums_ok else 1
+            if slices > 1:
+                return PartialSums(self.linear_f32_tiles(x, weight, slices))
+            return self.linear_f32_tiles(x, weight)[0]
+        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
         self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
                   _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, dtype_code(x.dtype), dtype_code(out_dtype))
+        return out
+
+    _F32_TILES = [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P]
+
+    def f32_slices_for(self, M: int, N: int, K: int) -> int:
+        """In how many slices of K a float32 product of more rows than the weight-streaming kernel takes is cut, where its
+        reader adds up partial sums: as many as the tiles need to fill the CUs (the kernel library's model of its time);
+        1 for the whole product, and where the reader (add_rmsnorm) takes no partial sums of that width."""
+        if N > MAX_SUMMED_NORM_WIDTH or N % 4 != 0:
+            return 1
+        fn = getattr(build.load_library("gemm_f32"), "lle_gemm_nt_f32_slices")
+        fn.argtypes, fn.restype = [_I, _I, _I], _I
+        return int(fn(M, N, K))
+
+    def linear_f32_tiles(self, x, weight, slices: int = 1, tiles: int = -1) -> torch.Tensor:
+        """x [M, K] . weight [N, K]^T, float32, in tiles: [slices, M, N], the sums over `slices` parts of K (whole steps of
+        32 columns) to be added up by the reader.  `tiles`: which tile shape (below zero: the one that takes the least time)."""
+        _dev(x, "x", torch.float32)
+        _dev(weight, "weight", torch.float32)
+        M, K = x.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 4 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, slices,
+                  tiles)
         return out
 
     SLICED_MIN_ROWS, SLICED_MAX_ROWS = 17, 128  # (lle_gemm_mid_slices_max_rows)
@@ -888,8 +916,8 @@ class HipOps:
             b_ptr = weight.data_ptr() + 4 * h * O * K
             c_ptr = out.data_ptr() + 4 * h * O
             if quick:
-                self._run("gemm", "lle_gemm_nt_mfma_f32", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _P],
-                          a_ptr, b_ptr, c_ptr, N, O, K, heads * xw, K, heads * O)
+                self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, a_ptr, b_ptr, c_ptr, N, O, K, heads * xw, K,
+                          heads * O, 1, -1)
             else:
                 self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
                           a_ptr, b_ptr, c_ptr, N, O, K, heads * xw, K, heads * O, F32, F32)

@@ -1,0 +1,80 @@
+"""The float32 product of many rows (operands split into three bfloat16 parts) against float64: every tile shape at the edges
+of its tiles, slices of K, and values at the ends of float32's range."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TILES = [-1, 0, 1, 2, 3]
+
+
+def ops():
+    from litellmengine_amd.csrc.ops import default_ops
+
+    return default_ops()
+
+
+def operands(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(1000 * seed + M + 7 * N + 13 * K)
+    x = torch.randn(M, K, generator=g, device="cuda") * torch.exp2(torch.randint(-8, 9, (M, 1), generator=g, device="cuda").float())
+    return x, torch.randn(N, K, generator=g, device="cuda") * 0.02
+
+
+def check(got, x, w):
+    """Every element within what K float32 additions may lose of the sum of its products' sizes; all together within 6 x 2^-24 of
+    those (with random signs a sum stays sqrt(K) below its products' sizes, and so do its roundings; without the third parts
+    of the operands it would be 2^-18 sqrt(1 / K) or more off at these K)."""
+    want = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    K = x.shape[1]
+    off = (got.double() - want).abs()
+    assert bool((off <= 2.0 ** -24 * (K + 16) * size).all())
+    assert float(off.norm() / size.norm()) <= 2.0 ** -24 * 6 / math.sqrt(K) * max(1.0, K / 64)
+
+
+@pytest.mark.parametrize("tiles", TILES)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (65, 64, 32), (64, 129, 36), (257, 127, 100), (128, 256, 28), (300, 2049, 64), (66, 131, 4)])
+def test_tiles_at_their_edges(tiles, M, N, K):
+    x, w = operands(M, N, K)
+    check(ops().linear_f32_tiles(x, w, tiles=tiles)[0], x, w)
+
+
+@pytest.mark.parametrize("slices,K", [(2, 128), (3, 260), (8, 96), (5, 1028)])
+def test_slices_add_up(slices, K):
+    """(8 slices of three steps: the last ones are empty)"""
+    x, w = operands(70, 192, K, seed=1)
+    parts = ops().linear_f32_tiles(x, w, slices=slices)
+    assert parts.shape == (slices, 70, 192) and bool(torch.isfinite(parts).all())
+    check(parts.double().sum(0), x, w)
+
+
+def test_the_product_takes_slices_where_its_reader_adds_them_up():
+    from litellmengine_amd.parts import PartialSums
+
+    o = ops()
+    x, w = operands(100, 1024, 3072, seed=2)
+    whole, cut = o.linear(x, w), o.linear(x, w, sums_ok=True)
+    assert isinstance(cut, PartialSums) and cut.sums.shape[0] == o.f32_slices_for(100, 1024, 3072) > 1
+    check(whole, x, w)
+    check(cut.total(), x, w)
+    assert o.f32_slices_for(100, 1022, 3072) == 1 and o.f32_slices_for(100, 1 << 17, 4096) == 1
+
+
+@pytest.mark.parametrize("tiles", TILES)
+def test_values_at_the_ends_of_the_range(tiles):
+    """Infinities and NaN where plain float32 has them, numbers that round to infinity in bfloat16, and small ones."""
+    x, w = operands(70, 72, 40, seed=3)
+    x[3, 5], x[9, 0], x[11, 39] = math.inf, -math.inf, math.nan
+    w[7, 2] = math.inf
+    x[20] = 0.0
+    x[20, 8], w[:, 8] = 3.4e38, 2.0 ** -30 * w[:, 8].sign()
+    x[21], x[22] = x[21] * 2.0 ** -100, x[22] * 2.0 ** 90
+    got = ops().linear_f32_tiles(x, w, tiles=tiles)[0].cpu()
+    want = (x.double().cpu() @ w.double().cpu().T)  # (an infinity's sign follows the weights' signs in both)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()].double(), want[want.isinf()])
+    fine = want.isfinite()
+    size = torch.nan_to_num(x.double().cpu(), posinf=0, neginf=0).abs() @ torch.nan_to_num(w.double().cpu(), posinf=0).abs().T
+    assert bool(((got.double() - want).abs()[fine] <= (2.0 ** -24 * 56 * size)[fine] + 2.0 ** -126).all())
