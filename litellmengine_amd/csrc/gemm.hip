@@ -92,7 +92,26 @@ extern "C" int lle_gemm_nt_simt(const void* A, const void* B, void* C, int M, in
 typedef bf16_t gbf16x8 __attribute__((ext_vector_type(8)));
 typedef float gf32x4 __attribute__((ext_vector_type(4)));
 
-#define SK_KSTEP 64
+// An operand type T of the weight-streaming kernels: 16 bytes of it, and the product of 16 rows of W and of X over the columns
+// that the lanes hold 16 bytes of each (bfloat16: one instruction; float32: four of the float32 instruction, whose products and
+// sums are float32, element e of the lanes in instruction e).  A step is 128 bytes of a row.
+template <typename T> struct SkOp;
+template <> struct SkOp<bf16_t> {
+    typedef gbf16x8 vec;
+    static constexpr int E = 8;
+    static __device__ __forceinline__ gf32x4 mma(vec w, vec x, gf32x4 acc) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc, 0, 0, 0); }
+};
+template <> struct SkOp<float> {
+    typedef gf32x4 vec;
+    static constexpr int E = 4;
+    static __device__ __forceinline__ gf32x4 mma(vec w, vec x, gf32x4 acc) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], acc, 0, 0, 0);
+        return acc;
+    }
+};
+#define SK_KSTEP 64  // elements of a bfloat16 step
+template <typename T> constexpr int sk_step = 8 * SkOp<T>::E;  // elements of a step
 
 // GATED: W holds gate rows [0, N/2) and then up rows [N/2, N); a workgroup takes 16 gate rows
 // and the 16 up rows that go with them (NT = 2) and writes silu(gate) * up, C is [M, N/2].
@@ -134,13 +153,15 @@ __device__ __forceinline__ float gated_result(float g, float u, const NormFold& 
     return g / (1.0f + expf(-g)) * u;
 }
 
-template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL>
+template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL>
 // one tile of W and up to 16 rows of X: two workgroups of 16 wavefronts a CU (8 wavefronts a SIMD),
 // which 64 registers allow; the gated form measured faster with the registers it asks for
-__global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) void gemm_skinny_kernel(const bf16_t* __restrict__ X,
-                                                                         const bf16_t* __restrict__ W,
+__global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) void gemm_skinny_kernel(const T* __restrict__ X,
+                                                                         const T* __restrict__ W,
                                                                          TC* __restrict__ C, int M, int N, int K,
                                                                          int tile_rows, NormFold fold) {
+    using Vec = typename SkOp<T>::vec;
+    constexpr int E = SkOp<T>::E, STEP = sk_step<T>;
     static_assert(!(RESID || SCALED) || MT <= 2, "the norm is folded for up to 32 rows");
     // `tile_rows` (at most 16) rows of W per tile: fewer than 16 where that makes the number of tiles a
     // multiple of the number of CUs (see skinny_tile_rows); the lanes past them read the tile's last
@@ -188,43 +209,42 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
         for (int mt = 0; mt < MT; ++mt)
             resid_h[mt] = fold.hidden[(int64_t)min(16 * mt + (int)(threadIdx.x / 16) % 16, M - 1) * N + col];
     }
-    const bf16_t* wp[NT];
+    const T* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int rt = min(r16, tile_rows - 1);  // the lane's row of the tile
         const int64_t wrow = GATED ? min(n0 + rt, (int64_t)N / 2 - 1) + nt * ((int64_t)N / 2)
                                    : min(n0 + (NT == 1 ? rt : 16 * nt + r16), (int64_t)N - 1);
-        wp[nt] = W + wrow * K + 16 * c;
+        wp[nt] = W + wrow * K + 2 * E * c;
     }
     // rows of X beyond M are never written back, so their lanes may read any valid row
-    const bf16_t* xp[MT];
+    const T* xp[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xp[mt] = X + (int64_t)min(16 * mt + r16, M - 1) * K + 16 * c;
+    for (int mt = 0; mt < MT; ++mt) xp[mt] = X + (int64_t)min(16 * mt + r16, M - 1) * K + 2 * E * c;
     gf32x4 acc[NT][MT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    const gbf16x8 zero = {(bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f,
-                          (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f};
+    const Vec zero = {};
 
-    const int full_steps = K / SK_KSTEP;
+    const int full_steps = K / STEP;
     int ss = wave;
     // UNROLL steps at a time: all their loads are issued before the first product
     for (; ss + (UNROLL - 1) * SK_WAVES < full_steps; ss += UNROLL * SK_WAVES) {
-        gbf16x8 w0[UNROLL][NT], w1[UNROLL][NT], x0[UNROLL][MT], x1[UNROLL][MT];
+        Vec w0[UNROLL][NT], w1[UNROLL][NT], x0[UNROLL][MT], x1[UNROLL][MT];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            const int k0 = (ss + u * SK_WAVES) * SK_KSTEP;
+            const int k0 = (ss + u * SK_WAVES) * STEP;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
-                w0[u][nt] = *(const gbf16x8*)(wp[nt] + k0);
-                w1[u][nt] = *(const gbf16x8*)(wp[nt] + k0 + 8);
+                w0[u][nt] = *(const Vec*)(wp[nt] + k0);
+                w1[u][nt] = *(const Vec*)(wp[nt] + k0 + E);
             }
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                x0[u][mt] = *(const gbf16x8*)(xp[mt] + k0);
-                x1[u][mt] = *(const gbf16x8*)(xp[mt] + k0 + 8);
+                x0[u][mt] = *(const Vec*)(xp[mt] + k0);
+                x1[u][mt] = *(const Vec*)(xp[mt] + k0 + E);
             }
         }
 #pragma unroll
@@ -233,30 +253,30 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[u][nt], x0[u][mt], acc[nt][mt], 0, 0, 0);
-                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[u][nt], x1[u][mt], acc[nt][mt], 0, 0, 0);
+                    acc[nt][mt] = SkOp<T>::mma(w0[u][nt], x0[u][mt], acc[nt][mt]);
+                    acc[nt][mt] = SkOp<T>::mma(w1[u][nt], x1[u][mt], acc[nt][mt]);
                 }
     }
-    // what is left of K: single steps; the last one may be partial (K is a multiple of 8),
+    // what is left of K: single steps; the last one may be partial (K is a multiple of E),
     // and there both operands are zeroed beyond K so that nothing outside the matrices is read
-    const int all_steps = (K + SK_KSTEP - 1) / SK_KSTEP;
+    const int all_steps = (K + STEP - 1) / STEP;
     for (; ss < all_steps; ss += SK_WAVES) {
-        const int k0 = ss * SK_KSTEP;
-        const bool in0 = k0 + 16 * c + 8 <= K, in1 = k0 + 16 * c + 16 <= K;
-        gbf16x8 x0[MT], x1[MT];
+        const int k0 = ss * STEP;
+        const bool in0 = k0 + 2 * E * c + E <= K, in1 = k0 + 2 * E * c + 2 * E <= K;
+        Vec x0[MT], x1[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            x0[mt] = in0 ? *(const gbf16x8*)(xp[mt] + k0) : zero;
-            x1[mt] = in1 ? *(const gbf16x8*)(xp[mt] + k0 + 8) : zero;
+            x0[mt] = in0 ? *(const Vec*)(xp[mt] + k0) : zero;
+            x1[mt] = in1 ? *(const Vec*)(xp[mt] + k0 + E) : zero;
         }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const gbf16x8 w0 = in0 ? *(const gbf16x8*)(wp[nt] + k0) : zero;
-            const gbf16x8 w1 = in1 ? *(const gbf16x8*)(wp[nt] + k0 + 8) : zero;
+            const Vec w0 = in0 ? *(const Vec*)(wp[nt] + k0) : zero;
+            const Vec w1 = in1 ? *(const Vec*)(wp[nt] + k0 + E) : zero;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, x0[mt], acc[nt][mt], 0, 0, 0);
-                acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, x1[mt], acc[nt][mt], 0, 0, 0);
+                acc[nt][mt] = SkOp<T>::mma(w0, x0[mt], acc[nt][mt]);
+                acc[nt][mt] = SkOp<T>::mma(w1, x1[mt], acc[nt][mt]);
             }
         }
     }
@@ -321,8 +341,8 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                     for (int w = 0; w < SK_WAVES; ++w) sum += s_acc[w][0][mt][n][m16];
                     const float h = resid_h[mt] + sum;
                     fold.hidden[(int64_t)m * N + col] = h;
-                    fold.xw[(int64_t)m * N + col] =
-                        (bf16_t)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid_w : resid_w << 16));
+                    ((T*)fold.xw)[(int64_t)m * N + col] =
+                        (T)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid_w : resid_w << 16));
                     sq = h * h;
                 }
 #pragma unroll
@@ -534,14 +554,18 @@ extern "C" int lle_gemm_mid_slices_bf16(const void* X, const void* W, void* out,
 // more than 16 rows);
 // the head of the 0.6B sizes (151936 x 1024) at 32 rows: 73.6 us, against 112.1 for the
 // one-tile-per-workgroup kernel with four tiles a workgroup and 66.8 at 16 rows.
-template <bool GATED, bool SCALED, int XS, typename TC, int MT = 1>
-__global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(const bf16_t* __restrict__ X,
-                                                                              const bf16_t* __restrict__ W,
+template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT = 1>
+__global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(const T* __restrict__ X,
+                                                                              const T* __restrict__ W,
                                                                               TC* __restrict__ C, int M, int N, int K,
                                                                               int share, NormFold fold) {
+    using Vec = typename SkOp<T>::vec;
+    constexpr int E = SkOp<T>::E, STEP = sk_step<T>;
     constexpr int WAVES = 16;
     constexpr int NT = GATED ? 2 : 1;
     constexpr int SS = (XS % 2 == 0 && XS <= 6) ? 2 : 1;  // steps of a set (one where X takes most of the registers)
+    // sets of W operands: one is multiplied, the others are on their way (single steps of float32: four)
+    constexpr int SETS = std::is_same<T, float>::value && !GATED && SS == 1 && XS % 4 == 0 ? 4 : 2;
     constexpr int SPT = XS / SS;             // sets of a tile
     static_assert(MT == 1 || (MT == 2 && (XS <= 2 || (!GATED && XS <= 4))), "two tiles of X rows only while X fits the registers");
     __shared__ float s_acc[2][WAVES][NT][MT][16][17];  // tiles take the two halves in turn: one barrier a tile
@@ -554,28 +578,28 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
     auto tile_begin = [&](int t) { return (int)gridDim.x * 16 * t + (int)blockIdx.x * min(16, share - 16 * t); };
     auto tile_end = [&](int t) { return min(rows, tile_begin(t) + min(16, share - 16 * t)); };
 
-    // a set: SS 64-element steps of the tile (and of the up tile that goes with a gate tile)
+    // a set: SS steps of the tile (and of the up tile that goes with a gate tile)
     struct Set {
-        gbf16x8 g0[SS], g1[SS], u0[SS], u1[SS];
+        Vec g0[SS], g1[SS], u0[SS], u1[SS];
     };
     // the load cursor: tile and step of the set that is asked for next
     int load_tile = 0, load_step = 0;
-    const bf16_t* wp = nullptr;
+    const T* wp = nullptr;
     auto aim = [&]() {
         const int t = min(load_tile, tiles - 1);
         const int row = max(0, min(tile_begin(t) + r16, tile_end(t) - 1));  // a tile without rows reads rows that are there
-        wp = W + (int64_t)row * K + 16 * c + wave * SK_KSTEP;
+        wp = W + (int64_t)row * K + 2 * E * c + wave * STEP;
     };
     auto load = [&](Set& set) {
 #pragma unroll
         for (int i = 0; i < SS; ++i) {
-            const bf16_t* g = wp + (load_step + i) * (WAVES * SK_KSTEP);
-            set.g0[i] = *(const gbf16x8*)g;
-            set.g1[i] = *(const gbf16x8*)(g + 8);
+            const T* g = wp + (load_step + i) * (WAVES * STEP);
+            set.g0[i] = *(const Vec*)g;
+            set.g1[i] = *(const Vec*)(g + E);
             if (GATED) {
-                const bf16_t* u = g + (int64_t)rows * K;
-                set.u0[i] = *(const gbf16x8*)u;
-                set.u1[i] = *(const gbf16x8*)(u + 8);
+                const T* u = g + (int64_t)rows * K;
+                set.u0[i] = *(const Vec*)u;
+                set.u1[i] = *(const Vec*)(u + E);
             }
         }
         load_step += SS;
@@ -585,18 +609,19 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
             aim();
         }
     };
-    Set sets[2];
+    Set sets[SETS];
     aim();
-    load(sets[0]);
+#pragma unroll
+    for (int i = 0; i < SETS - 1; ++i) load(sets[i]);
     // rows of X beyond M are never written back, so their lanes may read any valid row
-    gbf16x8 x0[MT][XS], x1[MT][XS];
+    Vec x0[MT][XS], x1[MT][XS];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        const bf16_t* xp = X + (int64_t)min(16 * mt + r16, M - 1) * K + 16 * c + wave * SK_KSTEP;
+        const T* xp = X + (int64_t)min(16 * mt + r16, M - 1) * K + 2 * E * c + wave * STEP;
 #pragma unroll
         for (int j = 0; j < XS; ++j) {
-            x0[mt][j] = *(const gbf16x8*)(xp + j * (WAVES * SK_KSTEP));
-            x1[mt][j] = *(const gbf16x8*)(xp + j * (WAVES * SK_KSTEP) + 8);
+            x0[mt][j] = *(const Vec*)(xp + j * (WAVES * STEP));
+            x1[mt][j] = *(const Vec*)(xp + j * (WAVES * STEP) + E);
         }
     }
     if (SCALED) {
@@ -625,11 +650,11 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
         for (int i = 0; i < SS; ++i)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                acc_g[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(set.g0[i], x0[mt][j + i], acc_g[mt], 0, 0, 0);
-                acc_g[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(set.g1[i], x1[mt][j + i], acc_g[mt], 0, 0, 0);
+                acc_g[mt] = SkOp<T>::mma(set.g0[i], x0[mt][j + i], acc_g[mt]);
+                acc_g[mt] = SkOp<T>::mma(set.g1[i], x1[mt][j + i], acc_g[mt]);
                 if (GATED) {
-                    acc_u[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(set.u0[i], x0[mt][j + i], acc_u[mt], 0, 0, 0);
-                    acc_u[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(set.u1[i], x1[mt][j + i], acc_u[mt], 0, 0, 0);
+                    acc_u[mt] = SkOp<T>::mma(set.u0[i], x0[mt][j + i], acc_u[mt]);
+                    acc_u[mt] = SkOp<T>::mma(set.u1[i], x1[mt][j + i], acc_u[mt]);
                 }
             }
     };
@@ -683,7 +708,19 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
     using Buf0 = std::integral_constant<int, 0>;
     using Buf1 = std::integral_constant<int, 1>;
     int tile = 0;
-    if constexpr (SPT % 2 == 0) {
+    if constexpr (SETS > 2) {
+        auto run = [&](bool last) {
+#pragma unroll
+            for (int s = 0; s < SPT; ++s) {
+                if (!(last && s + SETS - 1 >= SPT)) load(sets[(s + SETS - 1) % SETS]);
+                multiply(sets[s % SETS], s * SS);
+            }
+            finish_tile(tile);
+        };
+        static_assert(SPT % SETS == 0, "a tile's sets go around the buffers in whole rounds");
+        for (; tile + 1 < tiles; ++tile) run(false);
+        run(true);
+    } else if constexpr (SPT % 2 == 0) {
         for (; tile + 1 < tiles; ++tile) run_tile(tile, Buf0{}, false);
         run_tile(tile, Buf0{}, true);
     } else {
@@ -716,31 +753,35 @@ static int gemm_compute_units() {
 // The streaming kernel takes the product when K is a number of whole rounds of its 16 wavefronts
 // (1024 elements a round) that its registers hold, X has up to 16 rows, and W has more than one
 // tile of rows for every CU.
-template <bool GATED, bool SCALED, typename TC>
-static bool launch_skinny_stream(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K,
+template <typename T, bool GATED, bool SCALED, typename TC>
+static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, int K,
                                  const NormFold& fold, hipStream_t stream) {
-    if (M > 32 || K % (SK_KSTEP * 16) != 0) return false;
+    constexpr int STEP = sk_step<T>;
+    if (M > 32 || K % (STEP * 16) != 0) return false;
     const int rows = GATED ? N / 2 : N;
     const int units = gemm_compute_units();
     const int share = (rows + units - 1) / units;
     if (share <= 16) return false;
+    // a float32 row of X in the registers costs a start that few rows of W and of X do not repay (6144 x 4096 at 1 row: 24.7
+    // against 21.2 us, at 8 rows 26.6 against 27.9; 24576 x 4096 at 8 rows 83.6 against 96.7)
+    if (std::is_same<T, float>::value && share <= 32 && M <= 4) return false;
     const int blocks = (rows + share - 1) / share;
     if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
-        if (K == SK_KSTEP * 16) {
-            gemm_skinny_stream_kernel<GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+        if (K == STEP * 16) {
+            gemm_skinny_stream_kernel<T, GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
             return true;
         }
-        if (K == 2 * SK_KSTEP * 16) {
-            gemm_skinny_stream_kernel<GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+        if (K == 2 * STEP * 16) {
+            gemm_skinny_stream_kernel<T, GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
             return true;
         }
         if constexpr (!GATED) {
-            if (K == 3 * SK_KSTEP * 16) {
-                gemm_skinny_stream_kernel<GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+            if (K == 3 * STEP * 16) {
+                gemm_skinny_stream_kernel<T, GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
                 return true;
             }
-            if (K == 4 * SK_KSTEP * 16) {
-                gemm_skinny_stream_kernel<GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+            if (K == 4 * STEP * 16) {
+                gemm_skinny_stream_kernel<T, GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
                 return true;
             }
         }
@@ -748,10 +789,10 @@ static bool launch_skinny_stream(const bf16_t* X, const bf16_t* W, TC* C, int M,
     }
 #define LLE_STREAM_CASE(XSV)                                                                                          \
     case XSV:                                                                                                         \
-        gemm_skinny_stream_kernel<GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
+        gemm_skinny_stream_kernel<T, GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
                                                                                                fold);                \
         return true;
-    switch (K / (SK_KSTEP * 16)) {
+    switch (K / (STEP * 16)) {
         LLE_STREAM_CASE(1)
         LLE_STREAM_CASE(2)
         LLE_STREAM_CASE(3)
@@ -760,11 +801,11 @@ static bool launch_skinny_stream(const bf16_t* X, const bf16_t* W, TC* C, int M,
         case 6:
         case 8:
             if constexpr (!GATED) {  // the gated form's two tiles leave no registers for this much of X
-                if (K / (SK_KSTEP * 16) == 6) {
-                    gemm_skinny_stream_kernel<GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
+                if (K / (STEP * 16) == 6) {
+                    gemm_skinny_stream_kernel<T, GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
                                                                                                           share, fold);
                 } else {
-                    gemm_skinny_stream_kernel<GATED, SCALED, 8, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
+                    gemm_skinny_stream_kernel<T, GATED, SCALED, 8, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
                                                                                                           share, fold);
                 }
                 return true;
@@ -801,8 +842,8 @@ extern "C" int lle_gemm_skinny_resid_parts(int N) {
     return (N + tr - 1) / tr;
 }
 
-template <typename TC, int NT, bool GATED>
-static int launch_skinny(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K, hipStream_t stream, const NormFold& none = {}) {
+template <typename T, typename TC, int NT, bool GATED>
+static int launch_skinny(const T* X, const T* W, TC* C, int M, int N, int K, hipStream_t stream, const NormFold& none = {}) {
     constexpr int WAVES = 16, UNROLL = 4 / NT;
     const int rows = GATED ? N / 2 : N;
     const int tile_rows = (GATED || NT == 1) ? skinny_tile_rows(rows) : 16;
@@ -810,10 +851,10 @@ static int launch_skinny(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, 
     const int blocks = (rows + per_block - 1) / per_block;
     const int mt = (M + 15) / 16;
     switch (mt) {
-        case 1: gemm_skinny_kernel<1, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
-        case 2: gemm_skinny_kernel<2, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
-        case 3: gemm_skinny_kernel<3, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
-        case 4: gemm_skinny_kernel<4, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
+        case 1: gemm_skinny_kernel<T, 1, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
+        case 2: gemm_skinny_kernel<T, 2, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
+        case 3: gemm_skinny_kernel<T, 3, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
+        case 4: gemm_skinny_kernel<T, 4, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
@@ -829,12 +870,12 @@ extern "C" int lle_gemm_skinny_bf16(const void* X, const void* W, void* C, int M
     // one tile of W rows per workgroup measured best up to 16 rows of X (two tiles share the X
     // operands but halve the number of workgroups; they only pay off from 16 rows on)
     if (out_dtype == LLE_F32) {
-        if (launch_skinny_stream<false, false, float>(x, w, (float*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
-        return launch_skinny<float, 1, false>(x, w, (float*)C, M, N, K, stream);
+        if (launch_skinny_stream<bf16_t, false, false, float>(x, w, (float*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+        return launch_skinny<bf16_t, float, 1, false>(x, w, (float*)C, M, N, K, stream);
     }
     if (out_dtype == LLE_BF16) {
-        if (launch_skinny_stream<false, false, bf16_t>(x, w, (bf16_t*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
-        return launch_skinny<bf16_t, 1, false>(x, w, (bf16_t*)C, M, N, K, stream);
+        if (launch_skinny_stream<bf16_t, false, false, bf16_t>(x, w, (bf16_t*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+        return launch_skinny<bf16_t, bf16_t, 1, false>(x, w, (bf16_t*)C, M, N, K, stream);
     }
     return (int)hipErrorInvalidValue;
 }
@@ -845,9 +886,9 @@ extern "C" int lle_gemm_skinny_gated_bf16(const void* X, const void* W, void* C,
                                           hipStream_t stream) {
     if (M <= 0 || N2 <= 0) return 0;
     if (M > 32 || K % 8 != 0 || K <= 0 || N2 % 2 != 0) return (int)hipErrorInvalidValue;
-    if (launch_skinny_stream<true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, NormFold{}, stream))
+    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, NormFold{}, stream))
         LLE_RETURN_LAUNCH_STATUS();
-    return launch_skinny<bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream);
+    return launch_skinny<bf16_t, bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream);
 }
 
 // The same with biases [N2] (or null) and the clamped activation: g = min(gate + b, limit), u = clamp(up + b, -limit, limit),
@@ -859,9 +900,9 @@ extern "C" int lle_gemm_skinny_clamped_bf16(const void* X, const void* W, const 
     NormFold fold = {};
     fold.act_bias = (const bf16_t*)bias;
     fold.act_limit = limit;
-    if (launch_skinny_stream<true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, fold, stream))
+    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, fold, stream))
         LLE_RETURN_LAUNCH_STATUS();
-    return launch_skinny<bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream, fold);
+    return launch_skinny<bf16_t, bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream, fold);
 }
 
 // The product BEFORE a folded norm: delta = X W^T [M, N] is added into `hidden` (float32 [M, N],
@@ -881,10 +922,10 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
     fold.ss_out = (float*)ss_part;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     if (M <= 16)
-        gemm_skinny_kernel<1, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
+        gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
             (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
     else
-        gemm_skinny_kernel<2, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
+        gemm_skinny_kernel<bf16_t, 2, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
             (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
     LLE_RETURN_LAUNCH_STATUS();
 }
@@ -899,20 +940,20 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
 template <typename TC>
 static void launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M, int N, int K, const NormFold& fold,
                                  hipStream_t stream) {
-    if (launch_skinny_stream<false, true, TC>(x, w, c, M, N, K, fold, stream)) return;
+    if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream)) return;
     const int threads = 16 * LLE_WAVE;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     if (M <= 16) {
-        gemm_skinny_kernel<1, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
+        gemm_skinny_kernel<bf16_t, 1, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
     } else if (N >= 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()) {
         // 17 to 32 rows of X are twice the bytes of a tile of W: with one tile a workgroup a product
         // with many tiles (an output head) spends its time on X; several tiles share what they read of it
         // (the head of the 0.6B sizes, 151936 x 1024, at 32 rows: 137.6 us with one tile, 126.8 with two, 112.1 with four)
         constexpr int NT = SCALED_TILES_AT_32_ROWS;
-        gemm_skinny_kernel<2, NT, false, false, true, TC, 16, 4 / NT>
+        gemm_skinny_kernel<bf16_t, 2, NT, false, false, true, TC, 16, 4 / NT>
             <<<(N + 16 * NT - 1) / (16 * NT), threads, 0, stream>>>(x, w, c, M, N, K, 16, fold);
     } else {
-        gemm_skinny_kernel<2, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
+        gemm_skinny_kernel<bf16_t, 2, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
     }
 }
 
@@ -935,20 +976,20 @@ extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C
             launch_skinny_scaled<float>(x, w, (float*)C, M, N, K, fold, stream);
         else
             launch_skinny_scaled<bf16_t>(x, w, c, M, N, K, fold, stream);
-    } else if (launch_skinny_stream<true, true, bf16_t>(x, w, c, M, N, K, fold, stream)) {
+    } else if (launch_skinny_stream<bf16_t, true, true, bf16_t>(x, w, c, M, N, K, fold, stream)) {
     } else {
         const int rows = N / 2;
         const int tr = skinny_tile_rows(rows), blocks = (rows + tr - 1) / tr;
         if (M <= 16)
-            gemm_skinny_kernel<1, 2, true, false, true, bf16_t, 16, 2><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
+            gemm_skinny_kernel<bf16_t, 1, 2, true, false, true, bf16_t, 16, 2><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
         else
-            gemm_skinny_kernel<2, 2, true, false, true, bf16_t, 16, 2><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
+            gemm_skinny_kernel<bf16_t, 2, 2, true, false, true, bf16_t, 16, 2><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
     }
     LLE_RETURN_LAUNCH_STATUS();
 }
 
 // ---------------------------------------------------------------------------------
-// The same for float32 operands: the true 32-bit path of decoding.  W is read once;
+// The same for float32 operands: decoding in 32-bit where the streaming kernel does not take the product.  W is read once;
 // v_mfma_f32_16x16x4_f32 multiplies and adds in float32 (no reduced-precision mode).
 // Lane (c, r) loads 16 contiguous bytes W[n0 + r][k0 + 4c .. + 3]; its four values are the
 // k slot c of four instructions, and the X operand is laid out the same way.
@@ -1025,13 +1066,16 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE) void gemm_skinny_f32_kernel(con
 }
 
 // X [M, K] and W [N, K] float32, contiguous; C [M, N] float32; 1 <= M <= 64; K a multiple of 4.
+// The streaming kernel takes what it holds a row of X of (K a multiple of 512 up to 4096; 2048 beyond 16 rows), as for
+// bfloat16: at 8 rows 24576 x 4096 96.7 -> 83.6 us, 151936 x 4096 555 -> 457, 151936 x 1024 at 32 rows 240 -> 124.
 extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (M > 64 || K % 4 != 0 || K <= 0) return (int)hipErrorInvalidValue;
-    const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     const float* x = (const float*)X;
     const float* w = (const float*)W;
     float* c = (float*)C;
+    if (launch_skinny_stream<float, false, false, float>(x, w, c, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+    const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     switch ((M + 15) / 16) {
         case 1: gemm_skinny_f32_kernel<1, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;
         case 2: gemm_skinny_f32_kernel<2, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;
@@ -1039,4 +1083,13 @@ extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M,
         default: gemm_skinny_f32_kernel<4, 16, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;
     }
     LLE_RETURN_LAUNCH_STATUS();
+}
+
+// silu(X gate^T) * (X up^T) as lle_gemm_skinny_gated_bf16; 1 <= M <= 32, K a multiple of 4.
+extern "C" int lle_gemm_skinny_gated_f32(const void* X, const void* W, void* C, int M, int N2, int K, hipStream_t stream) {
+    if (M <= 0 || N2 <= 0) return 0;
+    if (M > 32 || K % 4 != 0 || K <= 0 || N2 % 2 != 0) return (int)hipErrorInvalidValue;
+    const float *x = (const float*)X, *w = (const float*)W;
+    if (launch_skinny_stream<float, true, false, float>(x, w, (float*)C, M, N2, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+    return launch_skinny<float, float, 2, true>(x, w, (float*)C, M, N2, K, stream);
 }

@@ -341,6 +341,9 @@ class HipOps:
         # (up to 16 columns are one step of one of the weight-streaming kernel's sixteen wavefronts: nothing to stream, and in
         # the tiles' kernel a row's result does not depend on how many rows there are)
         if M <= self.tuning.skinny_f32_max_rows and K % 4 == 0 and K > 16 and not self.force_library_gemm:
+            slices = self.f32_slices_for(M, N, K) if sums_ok else 1
+            if slices > 1:
+                return PartialSums(self.linear_f32_slices(x, weight, slices))
             out = torch.empty((M, N), dtype=out_dtype, device=x.device)
             # few rows: W streamed once, float32 matrix instruction
             self._run("gemm", "lle_gemm_skinny_f32", [_P, _P, _P, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
@@ -359,14 +362,31 @@ class HipOps:
     _F32_TILES = [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P]
 
     def f32_slices_for(self, M: int, N: int, K: int) -> int:
-        """In how many slices of K a float32 product of more rows than the weight-streaming kernel takes is cut, where its
-        reader adds up partial sums: as many as the tiles need to fill the CUs (the kernel library's model of its time);
-        1 for the whole product, and where the reader (add_rmsnorm) takes no partial sums of that width."""
+        """In how many slices of K a float32 product is cut whose reader adds up partial sums, so that the CUs have work and no
+        workgroup reads more of x than it has to (the kernel library says how many); 1 for the whole product, and where the
+        reader (add_rmsnorm) takes no partial sums of that width."""
         if N > MAX_SUMMED_NORM_WIDTH or N % 4 != 0:
             return 1
+        if M <= self.tuning.skinny_f32_max_rows:
+            fn = getattr(build.load_library("gemm_f32"), "lle_gemm_slices_f32_count")
+            fn.argtypes, fn.restype = [_I, _I], _I
+            return int(fn(N, K))
         fn = getattr(build.load_library("gemm_f32"), "lle_gemm_nt_f32_slices")
         fn.argtypes, fn.restype = [_I, _I, _I], _I
         return int(fn(M, N, K))
+
+    def linear_f32_slices(self, x, weight, slices: int) -> torch.Tensor:
+        """x [M, K] . weight [N, K]^T, float32, up to 64 rows, as partial sums over `slices` parts of K: [slices, M, N], to be
+        added up by the reader in slice order."""
+        _dev(x, "x", torch.float32)
+        _dev(weight, "weight", torch.float32)
+        M, K = x.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 4 == 0 and M <= 64, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm_f32", "lle_gemm_slices_f32", [_P, _P, _P, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out), M, N, K,
+                  slices)
+        return out
 
     def linear_f32_tiles(self, x, weight, slices: int = 1, tiles: int = -1) -> torch.Tensor:
         """x [M, K] . weight [N, K]^T, float32, in tiles: [slices, M, N], the sums over `slices` parts of K (whole steps of
@@ -758,8 +778,9 @@ class HipOps:
 
     def gate_up_silu(self, x, weight) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows) -> silu(x gate^T) * (x up^T), [M, I].
-        Few bfloat16 rows run as ONE weight-streaming launch with the activation in its
-        epilogue; otherwise the product and silu_mul."""
+        Few rows run as ONE weight-streaming launch with the activation in its epilogue; otherwise the product and
+        silu_mul (in float32 also up to 16 rows with more than 2560 columns, which the streaming kernel's gated form does
+        not hold: 24576 x 4096 at 8 rows 83.6 + 5 against 93.4 us in one launch, at 32 rows 153 + 5 against 122)."""
         if isinstance(x, Prenormed):
             return self._linear_folded(x, weight, None, gated=True)
         _dev(x, "x")
@@ -771,6 +792,11 @@ class HipOps:
         if x.dtype == torch.bfloat16 and few and K % 8 == 0 and not self.force_library_gemm:
             out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
             self._run("gemm", "lle_gemm_skinny_gated_bf16", [_P, _P, _P, _I, _I, _I, _P],
+                      _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
+            return out
+        if x.dtype == torch.float32 and M <= 32 and K % 4 == 0 and (M > 16 or 16 < K <= 2560) and not self.force_library_gemm:
+            out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
+            self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
         return self.silu_mul(self.linear(x, weight))

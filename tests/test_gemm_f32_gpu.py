@@ -62,6 +62,28 @@ def test_the_product_takes_slices_where_its_reader_adds_them_up():
     assert o.f32_slices_for(100, 1022, 3072) == 1 and o.f32_slices_for(100, 1 << 17, 4096) == 1
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K,slices", [(64, 128, 1), (100, 260, 2), (1024, 3072, 16), (72, 1028, 7), (64, 4, 1)])
+def test_few_rows_in_slices(M, N, K, slices):
+    """One step for a wavefront, an odd number, a last step that is not whole, rows of the weight that fill no group."""
+    x, w = operands(M, N, K, seed=4)
+    check(ops().linear_f32_slices(x, w, slices).double().sum(0), x, w)
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 32])
+@pytest.mark.parametrize("K", [512, 1024, 1536, 2560, 3072, 4096, 520])
+def test_few_rows_streamed(M, K):
+    """More rows of the weight than sixteen for every CU: a row of x in the registers (and K that is not held), plain and gated."""
+    o = ops()
+    N = 2 * (17 * o.compute_units() + 5)
+    x, w = operands(M, N, K, seed=5)
+    check(o.linear(x, w), x, w)
+    x = x / x.abs().max()
+    gate, up = (x.double() @ w.double().T).chunk(2, dim=1)
+    want = torch.nn.functional.silu(gate) * up
+    assert float((o.gate_up_silu(x, w).double() - want).norm() / want.norm()) < 2.0 ** -24 * 6 * max(1.0, math.sqrt(K) / 8)
+
+
 @pytest.mark.parametrize("tiles", TILES)
 def test_values_at_the_ends_of_the_range(tiles):
     """Infinities and NaN where plain float32 has them, numbers that round to infinity in bfloat16, and small ones."""
