@@ -32,6 +32,7 @@ LIBRARIES: Dict[str, List[str]] = {
     "attention": ["attention.hip"],
     "gemm": ["gemm.hip"],
     "gemm_f32": ["gemm_f32.hip"],
+    "gemm_tile": ["gemm_tile.hip"],
     "sampling": ["sampling.hip"],
     "recurrent": ["recurrent.hip"],
     "latent": ["latent.hip"],

@@ -314,6 +314,9 @@ class HipOps:
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.bfloat16:
             if sums_ok and out_dtype == torch.bfloat16:
+                slices = self.tile_slices_for(M, N, K)
+                if slices:
+                    return PartialSums(self.linear_tile_sums(x, weight, slices))
                 slices = self.slices_for(M, N, K)
                 if slices:
                     return PartialSums(self.linear_slices(x, weight, slices))
@@ -438,6 +441,43 @@ class HipOps:
         if best_fill >= t.sliced_min_fill or (K >= 2 * N and N * K >= t.sliced_long_k_min_weight):
             return best
         return 0
+
+    def tile_slices_for(self, M: int, N: int, K: int) -> int:
+        """In how many slices of K the tiled product takes a delta of the residual stream (linear_tile_sums), or 0 where another
+        form stays.  It is taken where the whole product has too few tiles for the CUs and neither the sliced kernel of up to
+        128 rows nor the library's batched slices have better ones (measured with the norm, old -> new in us): up to 32 rows
+        weights that the sliced kernel does not take (5120 x 8192 31.0 -> 26.9) and large ones (5120 x 25600 68 -> 56); up to 128
+        rows also K >= 2 N (4096 x 12288 at 96 rows 40.4 -> 32.7; 4096 x 4096 gains nothing); beyond, square weights (4096 x 4096
+        at 160 / 512 rows 33.5 -> 23.4 / 37.7 -> 35.5, 5120 x 8192 57.8 -> 38.7 / 78 -> 64; at 700 rows 41.8 -> 47.8, not taken) and
+        the narrow ones of small models (1024 x 2048 at 1000 rows 24.1 -> 17.0)."""
+        if K % 64 != 0 or N % 4 != 0 or N > MAX_SUMMED_NORM_WIDTH or self.force_library_gemm or N * K < 1 << 20:
+            return 0
+        if M <= 32:
+            taken = M > 16 and (N * K >= 1 << 26 or self.slices_for(M, N, K) == 0)
+        elif M <= 128:
+            taken = K >= 2 * N or self.slices_for(M, N, K) == 0
+        else:
+            narrow = N <= 1024 and N * K <= 1 << 22
+            taken = M <= 2048 and (narrow or (K < 2 * N and (M <= 256 or (M <= 512 and N >= 4096))))
+        if not taken:
+            return 0
+        fn = getattr(build.load_library("gemm_tile"), "lle_gemm_tile_sums_slices")
+        fn.argtypes, fn.restype = [_I, _I, _I], _I
+        return int(fn(M, N, K))
+
+    def linear_tile_sums(self, x, weight, slices: int, tiles: int = -1) -> torch.Tensor:
+        """x [M, K] . weight [N, K]^T, bfloat16, as float32 partial sums over `slices` equal parts of K (whole stages of 64
+        columns): [slices, M, N], to be added up by the reader in slice order.  `tiles`: which tile shape (below zero: the one
+        that takes the least time)."""
+        _dev(x, "x", torch.bfloat16)
+        _dev(weight, "weight", torch.bfloat16)
+        M, K = x.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 64 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm_tile", "lle_gemm_tile_sums_bf16", [_P, _P, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
+                  M, N, K, slices, tiles)
+        return out
 
     def library_slices_for(self, M: int, N: int, K: int) -> int:
         """In how many slices of K the LIBRARY takes a product of more than 128 rows whose result is a
