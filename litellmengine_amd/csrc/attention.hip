@@ -551,6 +551,7 @@ struct FusedQKV {
     const float* cos_sin;   // [N, D / 2, 2]
     float eps;
     int write_kv;
+    const int32_t* order;   // the requests, longest first (lle_decode_order), or nullptr: as they come
 };
 
 // Eight consecutive norm weights (float32 or bfloat16) as they lie in memory; what they mean is
@@ -746,8 +747,16 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
                  "s"(page_stride), "s"(max_pages), "s"(window), "s"(scale_log2), "s"(fused.qkv), "s"(fused.slots),
                  "s"(fused.q_weight), "s"(fused.k_weight), "s"(fused.weight_dtype), "s"(fused.cos_sin),
                  "s"(fused.eps), "s"(fused.write_kv));
-    const int s = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z, nsplit = gridDim.z;
+    int s = blockIdx.x, kvh = blockIdx.y;
+    const int split = blockIdx.z, nsplit = gridDim.z;
     const int G = nq / nkv;
+    if (FUSED && fused.order) {
+        // More workgroups than CUs, which take one each and the next as they finish: with the longest requests first the
+        // last ones to start are short (all heads of a request before the next request).
+        const int id = blockIdx.y * gridDim.x + blockIdx.x;
+        s = fused.order[id / nkv];
+        kvh = id % nkv;
+    }
     const int q_start = cu_tokens[s], q_end = cu_tokens[s + 1], kv_len = kv_lens[s], seq_slot = seq_slots[s];
     asm volatile("" ::"s"(q_start), "s"(q_end), "s"(kv_len), "s"(seq_slot));
     const int q_len = q_end - q_start;
@@ -859,6 +868,27 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
             }
         }
     }
+}
+
+// order[0 .. S - 1]: the requests by falling length, equal ones as they come.  One workgroup, S <= 1024: a request's place is
+// the number of those before it.
+__global__ __launch_bounds__(1024) void decode_order_kernel(const int32_t* __restrict__ kv_lens, int32_t* __restrict__ order, int S) {
+    __shared__ int lens[1024];
+    const int i = threadIdx.x;
+    const int own = i < S ? kv_lens[i] : 0;
+    lens[i] = own;
+    __syncthreads();
+    if (i >= S) return;
+    int place = 0;
+    for (int j = 0; j < S; ++j) place += lens[j] > own || (lens[j] == own && j < i);
+    order[place] = i;
+}
+
+extern "C" int lle_decode_order(const void* kv_lens, void* order, int S, hipStream_t stream) {
+    if (S <= 0) return 0;
+    if (S > 1024) return (int)hipErrorInvalidValue;
+    decode_order_kernel<<<1, (S + LLE_WAVE - 1) / LLE_WAVE * LLE_WAVE, 0, stream>>>((const int32_t*)kv_lens, (int32_t*)order, S);
+    return (int)hipGetLastError();
 }
 
 // Merges the key splits.  grid = (tokens, q heads), one wavefront each; lane k holds (m, l) of
@@ -1817,7 +1847,7 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
                                                  const void* token_seq, void* out, void* ws_o, void* ws_ml, int N,
                                                  int S, int nq, int nkv, int d, int page_size, int64_t page_stride,
                                                  int max_pages, int window, float scale, int nsplit_decode,
-                                                 hipStream_t stream) {
+                                                 const void* order, hipStream_t stream) {
     if (!qkv || !cos_sin || !slots || d % 64 != 0) return (int)hipErrorInvalidValue;
     if ((q_weight == nullptr) != (k_weight == nullptr)) return (int)hipErrorInvalidValue;
     FusedQKV fused;
@@ -1829,6 +1859,7 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
     fused.cos_sin = (const float*)cos_sin;
     fused.eps = eps;
     fused.write_kv = write_kv;
+    fused.order = (const int32_t*)order;
     return paged_attention_mfma(nullptr, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, token_seq, out, ws_o,
                                 ws_ml, N, S, nq, nkv, d, page_size, page_stride, max_pages, window, scale, 1,
                                 nsplit_decode, 0, 1, 1, 0, fused, nullptr, 0, 0.f, stream);

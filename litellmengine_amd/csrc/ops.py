@@ -658,10 +658,11 @@ class HipOps:
 
     def qk_norm_rope_attention(self, qkv, slots, q_weight, k_weight, cos_sin, eps: float, kv_layer, nq: int,
                                nkv: int, d: int, write_kv: bool, block_table, seq_slots, cu_tokens, kv_lens,
-                               token_seq, window: Optional[int], scale: float, max_kv_len: int) -> torch.Tensor:
+                               token_seq, window: Optional[int], scale: float, max_kv_len: int, order=None) -> torch.Tensor:
         """qk_norm_rope_write and paged_attention of a decode step in one launch (see
         can_fuse_rope_attention): the workgroup whose keys include a new token's position writes
-        its K and V, every workgroup norms and rotates the q rows it multiplies."""
+        its K and V, every workgroup norms and rotates the q rows it multiplies.  `order` (int32 [S], or None):
+        the requests in the order in which they are started, see decode_order."""
         _dev(qkv, "qkv", torch.bfloat16)
         _dev(kv_layer, "kv_layer", torch.bfloat16)
         _dev(cos_sin, "cos_sin", torch.float32)
@@ -685,6 +686,9 @@ class HipOps:
         _need(cu_tokens.shape == (S + 1,) and kv_lens.shape == (S,), "cu_tokens [S + 1], kv_lens [S]")
         _need(nq % nkv == 0 and d % 64 == 0 and page_size % 16 == 0 and S <= 65535,
               "the fused decode attention does not take these sizes")
+        if order is not None:
+            _dev(order, "order", torch.int32)
+            _need(order.shape == (S,), "order must be [S]")
         win = int(window) if window else 0
         ns = self.decode_splits(S, nkv, max_kv_len, win)
         out = torch.empty((N, nq * d), dtype=torch.bfloat16, device=qkv.device)
@@ -694,12 +698,24 @@ class HipOps:
             ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=qkv.device)
         self._run("attention", "lle_qk_norm_rope_attention_decode",
                   [_P, _P, _P, _P, _I, _P, _F, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I,
-                   _F, _I, _P],
+                   _F, _I, _P, _P],
                   _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wcode, _ptr(cos_sin), float(eps),
                   int(bool(write_kv)), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens),
                   _ptr(kv_lens), _ptr(token_seq), _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size,
-                  kv_layer.stride(0), block_table.shape[1], win, float(scale), ns)
+                  kv_layer.stride(0), block_table.shape[1], win, float(scale), ns, _ptr(order))
         return out
+
+    def decode_order(self, kv_lens, num_kv_heads: int):
+        """The requests of a decode step by falling length (int32 [S], on the device), for qk_norm_rope_attention; None where its
+        workgroups, one for every request and key head, all start at once or there are over 1024 requests.  (A CU holds one
+        of them.  64 requests of 1000 to 4096 keys, 8 key heads: 130 us as they come, shortest first; 112 longest first.)"""
+        _dev(kv_lens, "kv_lens", torch.int32)
+        S = kv_lens.shape[0]
+        if S > 1024 or S * num_kv_heads <= self.compute_units():
+            return None
+        order = torch.empty((S,), dtype=torch.int32, device=kv_lens.device)
+        self._run("attention", "lle_decode_order", [_P, _P, _I, _P], _ptr(kv_lens), _ptr(order), S)
+        return order
 
     force_generic_attention = False  # tests flip this to compare the two families of kernels
     force_prefill_form = 0           # tests set 1, 2 or 3 to reach every shape of the prompt-portion workgroups

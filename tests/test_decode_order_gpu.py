@@ -1,0 +1,52 @@
+"""The order in which a decode step's requests are started: longest first, and no result depends on it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def ops():
+    from litellmengine_amd.csrc.ops import default_ops
+
+    return default_ops()
+
+
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 200, 1000, 1024])
+def test_longest_first_and_equal_ones_as_they_come(S):
+    o = ops()
+    lens = torch.randint(1, 50, (S,), generator=torch.Generator().manual_seed(S)).to(torch.int32)
+    got = o.decode_order(lens.cuda(), o.compute_units() + 1)
+    assert torch.equal(got.cpu().long(), torch.argsort(lens, descending=True, stable=True))
+
+
+def test_nothing_to_order():
+    o = ops()
+    lens = torch.ones(8, dtype=torch.int32, device="cuda")
+    assert o.decode_order(lens, 1) is None and o.decode_order(lens.repeat(200), 8) is None
+
+
+@pytest.mark.parametrize("nkv,group,lens", [(8, 4, [1, 33, 700, 64] * 10), (1, 16, [5] * 7), (3, 2, [40, 2000, 1])])
+def test_the_order_changes_no_result(nkv, group, lens):
+    """(the last: keys split over workgroups)"""
+    o = ops()
+    d, P, S, nq = 128, 16, len(lens), nkv * group
+    g = torch.Generator(device="cuda").manual_seed(3)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    pages = [-(-n // P) for n in lens]
+    table = torch.full((S, max(pages)), -1, dtype=torch.int32, device="cuda")
+    first = 0
+    for s, n in enumerate(pages):
+        table[s, :n] = torch.arange(first, first + n, dtype=torch.int32, device="cuda")
+        first += n
+    kv = torch.randn(first, 2, nkv, P, d, generator=g, device="cuda").bfloat16()
+    qkv = torch.randn(S, (nq + 2 * nkv) * d, generator=g, device="cuda").bfloat16()
+    w = torch.ones(d, device="cuda").bfloat16()
+    kv_lens = i32(lens)
+    slots = i32([int(table[s, (n - 1) // P]) * P + (n - 1) % P for s, n in enumerate(lens)])
+    inv = (1e4 ** (-torch.arange(0, d, 2) / d)).float().cuda()
+    cs = o.rope_table((kv_lens - 1).contiguous(), inv)
+    run = lambda pool, order: o.qk_norm_rope_attention(qkv, slots, w, w, cs, 1e-6, pool, nq, nkv, d, True, table, i32(range(S)), i32(range(S + 1)),
+                                                       kv_lens, i32(range(S)), None, d ** -0.5, max(lens), order)
+    a, b = kv.clone(), kv.clone()
+    plain, ordered = run(a, None), run(b, torch.argsort(kv_lens, descending=True, stable=True).to(torch.int32))
+    assert torch.equal(plain, ordered) and torch.equal(a, b) and not torch.equal(a, kv) and bool(plain.float().isfinite().all())
