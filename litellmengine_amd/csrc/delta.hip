@@ -11,9 +11,7 @@
 // Value head h reads the q and k of head h / (H / G).  Every value channel of a head is a recurrence of its
 // own over a vector of `dim` numbers (the column S[:, j]): a thread owns KI key channels of one column, the
 // DELTA_IG = 16 threads of a column are neighbours in a wavefront and add up their shares of S^T k and S^T q
-// through the lanes' cross-bar (no LDS, no barrier inside a token).  o is taken from the state BEFORE the
-// correction: S'^T q = g S^T q + w (k . q), so both sums are taken in one pass over the column and meet the
-// lanes' exchange together; k . q is made when the tokens are staged.  The state lies transposed in its row,
+// through the lanes' cross-bar (no LDS, no barrier inside a token).  The state lies transposed in its row,
 // [head][value][key], so a wavefront reads and writes one stretch of memory.
 // All of it is 32-bit in every mode; only u, gate and y have the activation type.
 #include "common.h"
@@ -24,7 +22,7 @@ LLE_DEFINE_ERROR_STRING()
 #define DELTA_TC 16   // tokens staged at a time
 #define DELTA_THREADS 256
 #define DELTA_VB (DELTA_THREADS / DELTA_IG)  // value channels of a workgroup
-static_assert(DELTA_VB == DELTA_TC, "the walk's kernel deals the staged tokens' k . q to its thread rows");
+static_assert(DELTA_VB * DELTA_TC == DELTA_THREADS, "a chunk's values are one element a thread");
 
 __device__ __forceinline__ float delta_silu(float x) { return x / (1.0f + expf(-x)); }
 
@@ -298,16 +296,16 @@ __device__ __forceinline__ float delta_row_sum(float x) {
 }
 
 // What a thread reads of one staged token: its share of k and q (CHANNEL: and of the channels' decays), and the
-// token's decay, beta and k . q.
+// token's decay and beta.
 template <int KI, bool CHANNEL>
 struct DeltaToken {
     float kk[KI], qq[KI], gg[CHANNEL ? KI : 1];
-    float g, beta, kq;
+    float g, beta;
 };
 
 template <int KI, bool CHANNEL>
 __device__ __forceinline__ void delta_read(DeltaToken<KI, CHANNEL>& d, const float* __restrict__ kt, const float* __restrict__ qt,
-                                           const float* __restrict__ gt, const float4* __restrict__ par) {
+                                           const float* __restrict__ gt, const float2* __restrict__ par) {
     if constexpr (CHANNEL) {
         if (KI % 4 == 0) {
 #pragma unroll
@@ -334,64 +332,57 @@ __device__ __forceinline__ void delta_read(DeltaToken<KI, CHANNEL>& d, const flo
             d.qq[ii] = qt[ii];
         }
     }
-    const float4 pr = *par;
-    d.g = pr.x, d.beta = pr.y, d.kq = pr.z;
+    const float2 pr = *par;
+    d.g = pr.x, d.beta = pr.y;
 }
 
-// One token of the walk for this thread's share of column j: both sums over the key channels in one pass, the
-// lanes' exchange, the correction; returns the read-out.
+// One token of the walk for this thread's share of column j: the sum over the key channels, the lanes' exchange, the
+// correction; returns the read-out, which the next token does not wait for.
 template <int KI, bool CHANNEL>
 __device__ __forceinline__ float delta_token(float (&S)[KI], const DeltaToken<KI, CHANNEL>& d, float v) {
-    float p = 0.f, r = 0.f, gS[KI];
-    if constexpr (CHANNEL) {  // the rows of S decay each at their own rate: the sums are taken over the decayed column
+    float p = 0.f, r = 0.f;
+    if constexpr (CHANNEL) {  // the rows of S decay each at their own rate
 #pragma unroll
         for (int ii = 0; ii < KI; ++ii) {
-            gS[ii] = d.gg[ii] * S[ii];
-            p = fmaf(gS[ii], d.kk[ii], p);
-            r = fmaf(gS[ii], d.qq[ii], r);
+            S[ii] *= d.gg[ii];
+            p = fmaf(S[ii], d.kk[ii], p);
         }
-        p = delta_row_sum(p);
-        r = delta_row_sum(r);
-        const float w = d.beta * (v - p);
+    } else {
 #pragma unroll
-        for (int ii = 0; ii < KI; ++ii) S[ii] = fmaf(d.kk[ii], w, gS[ii]);
-        return fmaf(w, d.kq, r);
+        for (int ii = 0; ii < KI; ++ii) {
+            S[ii] *= d.g;
+            p = fmaf(S[ii], d.kk[ii], p);
+        }
     }
+    const float w = d.beta * (v - delta_row_sum(p));
 #pragma unroll
     for (int ii = 0; ii < KI; ++ii) {
-        p = fmaf(S[ii], d.kk[ii], p);
+        S[ii] = fmaf(d.kk[ii], w, S[ii]);
         r = fmaf(S[ii], d.qq[ii], r);
-        gS[ii] = d.g * S[ii];
     }
-    p = delta_row_sum(p);
-    r = delta_row_sum(r);
-    const float w = d.beta * fmaf(-d.g, p, v);
-#pragma unroll
-    for (int ii = 0; ii < KI; ++ii) S[ii] = fmaf(d.kk[ii], w, gS[ii]);
-    return fmaf(w, d.kq, d.g * r);
+    return delta_row_sum(r);
 }
 
 // grid = (requests, heads, blocks of DELTA_VB value channels).  Thread (jl, ig) = (tid / 16, tid % 16) owns the
 // key channels [ig KI, (ig + 1) KI) of column j = block DELTA_VB + jl.  The tokens pass through LDS DELTA_TC at a
-// time; the next chunk's q, k, v, beta and decay inputs are asked for before the current chunk is walked and wait
-// in registers meanwhile, and inside a chunk every token's operands leave LDS one token ahead of their use.
-// Measured at 2048 tokens of 32 heads of 64 x 64: everything asked for when it was needed 916 us; the next chunk
-// ahead and whole chunks without a condition per token 591 us; operands read a token ahead, decay, beta and k . q
-// in one 16-byte read 348 us; the chunk's values through LDS, one load a thread 294 us; q and k staged 16 bytes at a
-// time 281 us; decays and betas made by a launch ahead of the walk 248 us.  Tried and not kept: all of a chunk's operands in registers before its first token
-// and k . q made in the walk (378 us, and two workgroups no longer share a CU: 194 against 116 us for four
-// requests of 512 tokens).
+// time, in two buffers (one for heads over 128 channels): the next chunk goes to LDS and the one behind it is asked for
+// before the current chunk is walked, one barrier a chunk, and inside a chunk every token's operands leave LDS one token
+// ahead of their use.  The read-out is the lane's whose number the token has, so a chunk's leave from the registers.
+// Measured at 2048 tokens of 32 heads of 64 x 64, a decay per channel: 267 us with three barriers a chunk, k . q made
+// ahead of the walk (the read-out taken from the state before the correction, in the same pass) and the read-outs through
+// LDS; NEW_C us so.  Tried and not kept: all of a chunk's operands in registers before its first token.
 template <int KI, bool CHANNEL>
 __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) {
     constexpr int KD = KI * DELTA_IG;
     constexpr int PER = DELTA_TC * KD / DELTA_THREADS;  // elements of q (and of k) of a chunk that a thread fetches
     static_assert(DELTA_TC * KD % DELTA_THREADS == 0, "a chunk's q and k are dealt to the threads in equal shares");
-    __shared__ __attribute__((aligned(16))) float s_q[DELTA_TC][KD];
-    __shared__ __attribute__((aligned(16))) float s_k[DELTA_TC][KD];
-    __shared__ __attribute__((aligned(16))) float s_g[CHANNEL ? DELTA_TC : 1][CHANNEL ? KD : 4];
-    __shared__ float4 s_par[DELTA_TC];  // (decay, beta, k . q, -) of every staged token
-    __shared__ float s_o[DELTA_TC][DELTA_VB];
-    __shared__ float s_v[DELTA_TC][DELTA_VB];
+    static_assert(DELTA_TC == DELTA_IG, "every lane of a column takes one token's read-out");
+    constexpr int BUFS = KI <= 8 ? 2 : 1;
+    __shared__ __attribute__((aligned(16))) float s_q[BUFS][DELTA_TC][KD];
+    __shared__ __attribute__((aligned(16))) float s_k[BUFS][DELTA_TC][KD];
+    __shared__ __attribute__((aligned(16))) float s_g[CHANNEL ? BUFS : 1][CHANNEL ? DELTA_TC : 1][CHANNEL ? KD : 4];
+    __shared__ float2 s_par[BUFS][DELTA_TC];  // (decay, beta) of every staged token
+    __shared__ __attribute__((aligned(16))) float s_v[BUFS][DELTA_VB][DELTA_TC + 4];
     const int s = blockIdx.x, h = blockIdx.y;
     const int tid = threadIdx.x, jl = tid / DELTA_IG, ig = tid % DELTA_IG;
     const int j0 = blockIdx.z * DELTA_VB, j = j0 + jl;
@@ -454,88 +445,92 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
             }
         }
     };
-    fetch(q0, min(DELTA_TC, q1 - q0));
-
-    for (int c0 = q0; c0 < q1; c0 += DELTA_TC) {
-        const int nt = min(DELTA_TC, q1 - c0);
-        __syncthreads();  // (the chunk before has been read, its results have left)
+    auto stage = [&](int buf, int nt) {  // what was fetched goes to LDS
         if (wide) {
 #pragma unroll
             for (int r = 0; r + 3 < PER; r += 4) {
                 const int e = (tid + DELTA_THREADS * (r / 4)) * 4, t = e / KD, i = e - t * KD;
-                *(float4*)&s_q[t][i] = float4{fq[r], fq[r + 1], fq[r + 2], fq[r + 3]};
-                *(float4*)&s_k[t][i] = float4{fk[r], fk[r + 1], fk[r + 2], fk[r + 3]};
-                if constexpr (CHANNEL) *(float4*)&s_g[t][i] = float4{fg[r], fg[r + 1], fg[r + 2], fg[r + 3]};
+                *(float4*)&s_q[buf][t][i] = float4{fq[r], fq[r + 1], fq[r + 2], fq[r + 3]};
+                *(float4*)&s_k[buf][t][i] = float4{fk[r], fk[r + 1], fk[r + 2], fk[r + 3]};
+                if constexpr (CHANNEL) *(float4*)&s_g[buf][t][i] = float4{fg[r], fg[r + 1], fg[r + 2], fg[r + 3]};
             }
         } else {
 #pragma unroll
             for (int r = 0; r < PER; ++r) {
                 const int e = tid + DELTA_THREADS * r, t = e / KD, i = e - t * KD;
-                s_q[t][i] = fq[r];
-                s_k[t][i] = fk[r];
-                if constexpr (CHANNEL) s_g[t][i] = fg[r];
+                s_q[buf][t][i] = fq[r];
+                s_k[buf][t][i] = fk[r];
+                if constexpr (CHANNEL) s_g[buf][t][i] = fg[r];
             }
         }
         if (tid < nt) {
-            float* par = (float*)&s_par[tid];
+            float2 par = {1.0f, 0.f};
             if (CHANNEL) {
-                par[1] = 1.0f / (1.0f + expf(-fb));
+                par.y = 1.0f / (1.0f + expf(-fb));
             } else if (a.gates) {
-                par[0] = fa;
-                par[1] = fb;
+                par = float2{fa, fb};
             } else {
                 const float x = fa + dt_bias;
                 const float softplus = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
-                par[0] = expf(-decay_rate * softplus);
-                par[1] = 1.0f / (1.0f + expf(-fb));
+                par = float2{expf(-decay_rate * softplus), 1.0f / (1.0f + expf(-fb))};
             }
+            s_par[buf][tid] = par;
         }
-        s_v[tid / DELTA_VB][tid % DELTA_VB] = fv;
-        if (c0 + DELTA_TC < q1) fetch(c0 + DELTA_TC, min(DELTA_TC, q1 - c0 - DELTA_TC));
-        __syncthreads();
+        s_v[buf][tid % DELTA_VB][tid / DELTA_VB] = fv;
+    };
+    auto count = [&](int c0) { return min(DELTA_TC, q1 - c0); };
+    fetch(q0, count(q0));
+    stage(0, count(q0));
+    if (q0 + DELTA_TC < q1) fetch(q0 + DELTA_TC, count(q0 + DELTA_TC));
+    __syncthreads();
+
+    int buf = 0;
+    for (int c0 = q0; c0 < q1; c0 += DELTA_TC) {
+        const int nt = count(c0), c1 = c0 + DELTA_TC, c2 = c1 + DELTA_TC;
+        if (BUFS == 2 && c1 < q1) {
+            stage(buf ^ 1, count(c1));
+            if (c2 < q1) fetch(c2, count(c2));
+        }
         float vv[DELTA_TC];
 #pragma unroll
-        for (int t = 0; t < DELTA_TC; ++t) vv[t] = s_v[t][jl];
-        {  // k . q of every token: the sixteen lanes of thread row jl take token jl (DELTA_VB == DELTA_TC)
-            float d = 0.f;
-            for (int i = ig; i < KD; i += DELTA_IG) d = fmaf(s_k[jl][i], s_q[jl][i], d);
-            d = delta_row_sum(d);
-            if (ig == 0) ((float*)&s_par[jl])[2] = d;
+        for (int t = 0; t < DELTA_TC; t += 4) {
+            const float4 x = *(const float4*)&s_v[buf][jl][t];
+            vv[t] = x.x, vv[t + 1] = x.y, vv[t + 2] = x.z, vv[t + 3] = x.w;
         }
-        __syncthreads();
-        const float* kt = &s_k[0][ig * KI];
-        const float* qt = &s_q[0][ig * KI];
+        const float* kt = &s_k[buf][0][ig * KI];
+        const float* qt = &s_q[buf][0][ig * KI];
         constexpr int GS = CHANNEL ? KD : 0;
-        const float* gt = CHANNEL ? &s_g[0][ig * KI] : &s_g[0][0];
-        float oo[DELTA_TC];
+        const float* gt = CHANNEL ? &s_g[buf][0][ig * KI] : &s_g[0][0][0];
+        float out = 0.f;  // of token ig
         if (nt == DELTA_TC) {  // a whole chunk: nothing under a condition, every token's operands read a token ahead
             DeltaToken<KI, CHANNEL> cur, nxt;
-            delta_read<KI, CHANNEL>(cur, kt, qt, gt, &s_par[0]);
+            delta_read<KI, CHANNEL>(cur, kt, qt, gt, &s_par[buf][0]);
 #pragma unroll
             for (int t = 0; t < DELTA_TC; ++t) {
-                if (t + 1 < DELTA_TC) delta_read<KI, CHANNEL>(nxt, kt + (t + 1) * KD, qt + (t + 1) * KD, gt + (t + 1) * GS, &s_par[t + 1]);
-                oo[t] = delta_token<KI, CHANNEL>(S, cur, vv[t]);
+                if (t + 1 < DELTA_TC) delta_read<KI, CHANNEL>(nxt, kt + (t + 1) * KD, qt + (t + 1) * KD, gt + (t + 1) * GS, &s_par[buf][t + 1]);
+                const float o = delta_token<KI, CHANNEL>(S, cur, vv[t]);
+                out = ig == t ? o : out;
                 cur = nxt;
             }
         } else {
 #pragma unroll
             for (int t = 0; t < DELTA_TC; ++t) {
-                oo[t] = 0.f;
                 if (t < nt) {
                     DeltaToken<KI, CHANNEL> cur;
-                    delta_read<KI, CHANNEL>(cur, kt + t * KD, qt + t * KD, gt + t * GS, &s_par[t]);
-                    oo[t] = delta_token<KI, CHANNEL>(S, cur, vv[t]);
+                    delta_read<KI, CHANNEL>(cur, kt + t * KD, qt + t * KD, gt + t * GS, &s_par[buf][t]);
+                    const float o = delta_token<KI, CHANNEL>(S, cur, vv[t]);
+                    out = ig == t ? o : out;
                 }
             }
         }
-        if (ig == 0) {
-#pragma unroll
-            for (int t = 0; t < DELTA_TC; ++t) s_o[t][jl] = oo[t];
-        }
-        __syncthreads();
-        for (int idx = tid; idx < nt * DELTA_VB; idx += DELTA_THREADS) {
-            const int t = idx / DELTA_VB, e = idx - t * DELTA_VB;
-            if (j0 + e < vdim) a.out[(int64_t)(c0 + t) * HV + h * vdim + j0 + e] = s_o[t][e];
+        if (ig < nt && live) a.out[(int64_t)(c0 + ig) * HV + h * vdim + j] = out;
+        __syncthreads();  // this chunk has been read, and the next one is in LDS
+        if (BUFS == 2) {
+            buf ^= 1;
+        } else if (c1 < q1) {
+            stage(0, count(c1));
+            if (c2 < q1) fetch(c2, count(c2));
+            __syncthreads();
         }
     }
     if (live) {
