@@ -88,6 +88,7 @@ class HipOps:
         if not torch.cuda.is_available():
             raise KernelError("litellmengine_amd needs a GPU: its kernels have no CPU form")
         self._fn = {}
+        self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta)
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives)
 
     # -- plumbing ---------------------------------------------------------
@@ -315,14 +316,12 @@ class HipOps:
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.bfloat16:
             if sums_ok and out_dtype == torch.bfloat16:
-                slices = self.tile_slices_for(M, N, K)
-                if slices:
+                form, slices = self._form_of_delta(x.dtype, M, N, K)
+                if form == "tiles":
                     return PartialSums(self.linear_tile_sums(x, weight, slices))
-                slices = self.slices_for(M, N, K)
-                if slices:
+                if form == "slices":
                     return PartialSums(self.linear_slices(x, weight, slices))
-                slices = self.library_slices_for(M, N, K)
-                if slices:
+                if form == "library":
                     # one batched library product over the slices of K, partial sums left in 32-bit
                     xs = x.view(M, slices, K // slices).permute(1, 0, 2)
                     ws = weight.view(N, slices, K // slices).permute(1, 2, 0)
@@ -345,7 +344,7 @@ class HipOps:
         # (up to 16 columns are one step of one of the weight-streaming kernel's sixteen wavefronts: nothing to stream, and in
         # the tiles' kernel a row's result does not depend on how many rows there are)
         if M <= self.tuning.skinny_f32_max_rows and K % 4 == 0 and K > 16 and not self.force_library_gemm:
-            slices = self.f32_slices_for(M, N, K) if sums_ok else 1
+            slices = self._form_of_delta(x.dtype, M, N, K)[1] if sums_ok else 1
             if slices > 1:
                 return PartialSums(self.linear_f32_slices(x, weight, slices))
             out = torch.empty((M, N), dtype=out_dtype, device=x.device)
@@ -354,7 +353,7 @@ class HipOps:
                       M, N, K)
             return out
         if K % 4 == 0 and not self.force_simt_gemm:
-            slices = self.f32_slices_for(M, N, K) if sums_ok else 1
+            slices = self._form_of_delta(x.dtype, M, N, K)[1] if sums_ok else 1
             # (splitting the rows of x is a launch of its own: small weights do not repay it, 513 x 1024 x 2052 49 against 51 us)
             if exponent is not None and M >= 96 and N * K >= 1 << 22:
                 out = self.linear_f32_halves(x, weight, exponent, slices)
@@ -365,6 +364,26 @@ class HipOps:
         self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
                   _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, dtype_code(x.dtype), dtype_code(out_dtype))
         return out
+
+    def _form_of_delta(self, dtype, M: int, N: int, K: int):
+        """(form, slices of K) in which a product is taken whose reader adds up partial sums.  The choice is made from the sizes
+        alone and kept for the next product of the same sizes: made anew each time it costs the host as much as the launch."""
+        key = (dtype, M, N, K, self.force_library_gemm)
+        form = self._forms.get(key)
+        if form is None:
+            if dtype == torch.float32:
+                form = ("f32", self.f32_slices_for(M, N, K))
+            else:
+                for name, choose in (("tiles", self.tile_slices_for), ("slices", self.slices_for), ("library", self.library_slices_for)):
+                    form = (name, choose(M, N, K))
+                    if form[1]:
+                        break
+                else:
+                    form = ("whole", 0)
+            if len(self._forms) >= 4096:
+                self._forms.clear()
+            self._forms[key] = form
+        return form
 
     _F32_TILES = [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P]
 
