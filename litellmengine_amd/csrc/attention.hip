@@ -1337,7 +1337,15 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
 //   * a request with at most 16 rows (token, head of the group): one tile of rows, the four
 //     wavefronts take every fourth 16-key step and are merged through LDS (decoding);
 //   * any other: a workgroup takes 64 rows, each wavefront a tile of 16 of them and all keys
-//     that its rows see.
+//     that its rows see; or (TILES == 2, heads of 64 and 128) 128 rows, two tiles a wavefront.
+// What bounds it: the matrix instruction (32 cycles for 1024 products) where the loads keep up.
+// Every wavefront loads K and V for itself, 16 KB a step of 16 keys of 128 elements, and one tile
+// multiplies them in 2048 cycles; two tiles halve the bytes and leave two independent chains of
+// scores.  The registers hold one step's K and one step's V, each asked for again as soon as its
+// product is through, so that two (two tiles) or three workgroups fit a CU; two steps' worth of them,
+// as it was, left one.  A 2048-token prompt of 32 / 8 heads of 128: 730 -> 372 us a layer (34 GFLOP:
+// 92 of the 154 TFLOP/s a large float32 product reaches), one of 4096 tokens 2455 -> 1386, 32
+// prompts of 64 tokens (16 / 8 heads) 31 -> 23; 64 requests decoding at 900 keys 102 -> 92.
 // grid = (kv heads, row blocks x key splits, requests); with key splits the partial (m, l, acc)
 // go to the workspaces and the combine kernel merges them.
 // Operands (lane = (c, r), c = lane / 16, r = lane % 16): a lane loads 16 bytes, four
@@ -1349,14 +1357,15 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
 // ---------------------------------------------------------------------------------
 #define F32_WAVES 4
 #define F32_KEYS 16
-template <int DQ, bool KEEP, bool CAP>
-__global__ __launch_bounds__(F32_WAVES* LLE_WAVE) void mfma_f32_attention_kernel(
+template <int DQ, int TILES, bool KEEP, bool CAP>
+__global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES == 2 ? 2 : 3) void mfma_f32_attention_kernel(
     const float* __restrict__ q, const float* __restrict__ kv_layer, const int32_t* __restrict__ block_tables,
     const int32_t* __restrict__ seq_slots, const int32_t* __restrict__ cu_tokens,
     const int32_t* __restrict__ kv_lens, float* __restrict__ out, float* __restrict__ ws_o,
     float* __restrict__ ws_ml, int nsplit, int nq, int nkv, int P, int64_t page_stride, int max_pages, int window,
-    int keep_first, float scale_log2, const float* __restrict__ sinks, float cap_log2) {
-    constexpr int D = 16 * DQ;
+    int keep_first, float scale_log2, const float* __restrict__ sinks, float cap_log2, int paired) {
+    static_assert(TILES == 1 || !KEEP, "kept first keys: one tile");
+    constexpr int D = 16 * DQ, ROWS = 16 * TILES;
     extern __shared__ float smem[];  // [waves][16][D] acc, then [waves][16] m, [waves][16] l
     float* s_o = smem;
     float* s_m = smem + F32_WAVES * 16 * D;
@@ -1370,154 +1379,224 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE) void mfma_f32_attention_kernel
     const int kv_len = kv_lens[s];
     const int past = kv_len - q_len;
     const int row_blocks = gridDim.y / nsplit;
-    const int split = blockIdx.y / row_blocks, yb = blockIdx.y % row_blocks;
+    const int split = blockIdx.y / row_blocks;
+    int yb = blockIdx.y % row_blocks;
     const bool few = nrows <= 16;  // the same for the whole workgroup
     const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
     const int c = lane / 16, r16 = lane % 16;
-    if (few ? yb != 0 : yb * (16 * F32_WAVES) >= nrows) return;
-    const int row0 = few ? 0 : yb * (16 * F32_WAVES) + wave * 16;
+    const int own = few ? 1 : (nrows + ROWS * F32_WAVES - 1) / (ROWS * F32_WAVES);  // the request's blocks
+    if (yb >= own) return;
+    // the last rows, which see the most keys, first; or (`paired`) the later half of the blocks from
+    // the longest on, then the earlier half from the shortest on
+    yb = paired && 2 * yb >= own ? yb - (own + 1) / 2 : own - 1 - yb;
+    const int row0 = few ? 0 : yb * (ROWS * F32_WAVES) + wave * ROWS;
     const bool wave_has_rows = row0 < nrows;
     const int32_t* table = block_tables + (int64_t)seq_slots[s] * max_pages;
 
-    // the lane's row
-    const int row = row0 + r16;
-    const bool exists = row < nrows;
-    const int tok = exists ? row / G : 0, g = exists ? row - tok * G : 0;
-    const int64_t head_row = (int64_t)(q_start + tok) * nq + kvh * G + g;
-    int pos = exists ? past + tok : -1;
-    int lo = (exists && window > 0) ? max(0, pos - window + 1) : 0;
-    f32x4 qf[DQ];
+    // the lane's row of each tile
+    bool exists[TILES];
+    int pos[TILES], lo[TILES], g[TILES];
+    int64_t head_row[TILES];
+    f32x4 qf[TILES][DQ];
 #pragma unroll
-    for (int i = 0; i < DQ; ++i)
-        qf[i] = exists ? *(const f32x4*)(q + head_row * D + 16 * i + 4 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TILES; ++t) {
+        const int row = row0 + 16 * t + r16;
+        exists[t] = row < nrows;
+        const int tok = exists[t] ? row / G : 0;
+        g[t] = exists[t] ? row - tok * G : 0;
+        head_row[t] = (int64_t)(q_start + tok) * nq + kvh * G + g[t];
+        pos[t] = exists[t] ? past + tok : -1;
+        lo[t] = (exists[t] && window > 0) ? max(0, pos[t] - window + 1) : 0;
+#pragma unroll
+        for (int i = 0; i < DQ; ++i)
+            qf[t][i] = exists[t] ? *(const f32x4*)(q + head_row[t] * D + 16 * i + 4 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 
-    // the keys of this wavefront's tile, in steps of 16, and its share of them
+    // the keys that each tile's rows see, in steps of 16, and the wavefront's share of them
     int step_begin = 0, step_end = 0, step_stride = 1;
+    int first[TILES], end[TILES];
     [[maybe_unused]] int kept_end = 0;  // steps of the kept first keys, which are the first split's work
-    if (wave_has_rows) {
-        const int last_row = min(nrows, row0 + 16) - 1;
-        const int hi = past + last_row / G;
-        const int lo_tile = window > 0 ? max(0, past + row0 / G - window + 1) : 0;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const int r0 = row0 + 16 * t;
+        first[t] = end[t] = 0;
+        if (r0 >= nrows) continue;
+        const int hi = past + (min(nrows, r0 + 16) - 1) / G;
+        const int lo_tile = window > 0 ? max(0, past + r0 / G - window + 1) : 0;
+        first[t] = lo_tile / F32_KEYS;
+        end[t] = hi / F32_KEYS + 1;
+        step_end = end[t];  // (a later tile's rows see no less far)
         if (KEEP && split == 0) kept_end = (min(keep_first, max(0, hi - window + 1)) + F32_KEYS - 1) / F32_KEYS;
-        const int first = lo_tile / F32_KEYS, end = hi / F32_KEYS + 1;
-        const int per_split = (end - first + nsplit - 1) / nsplit;
-        step_begin = first + split * per_split;
-        step_end = min(end, step_begin + per_split);
+    }
+    if (wave_has_rows) {
+        const int per_split = (step_end - first[0] + nsplit - 1) / nsplit;
+        step_begin = first[0] + split * per_split;
+        step_end = min(step_end, step_begin + per_split);
         if (few) {
             step_begin += wave;
             step_stride = F32_WAVES;
         }
     }
-    f32x4 o[DQ];
+    f32x4 o[TILES][DQ];
+    float m[TILES], l[TILES];
 #pragma unroll
-    for (int n = 0; n < DQ; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = NEG_BIG, l = 0.f;
+    for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+        for (int n = 0; n < DQ; ++n) o[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        m[t] = NEG_BIG;
+        l[t] = 0.f;
+    }
     const int64_t k_lane = ((int64_t)kvh * P + r16) * D + 4 * c;
     const int64_t v_lane = ((int64_t)nkv + kvh) * P * D + (int64_t)r16 * P + 4 * c;
-    constexpr int NBUF = DQ <= 8 ? 2 : 1;
-    f32x4 kf[NBUF][DQ], vf[NBUF][DQ];
-    auto load = [&](int buf, int step) {
+    f32x4 kf[DQ], vf[DQ];
+    auto place = [&](int step) {
         const int j0 = step * F32_KEYS;
-        const int lp = j0 / P, off = j0 - lp * P;  // 16 keys of a step lie in one page
-        const float* page = kv_layer + (int64_t)table[__builtin_amdgcn_readfirstlane(lp)] * page_stride;
-#pragma unroll
-        for (int i = 0; i < DQ; ++i) kf[buf][i] = *(const f32x4*)(page + k_lane + (int64_t)off * D + 16 * i);
-#pragma unroll
-        for (int n = 0; n < DQ; ++n) vf[buf][n] = *(const f32x4*)(page + v_lane + (int64_t)16 * n * P + off);
+        const int lp = j0 / P;  // 16 keys of a step lie in one page
+        return kv_layer + (int64_t)table[__builtin_amdgcn_readfirstlane(lp)] * page_stride;
     };
-    auto multiply = [&](int buf, int step) {
-        const int j0 = step * F32_KEYS;
-        f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+    auto load_k = [&](int step) {
+        const float* at = place(step) + k_lane + (int64_t)(step * F32_KEYS % P) * D;
+#pragma unroll
+        for (int i = 0; i < DQ; ++i) kf[i] = *(const f32x4*)(at + 16 * i);
+    };
+    auto load_v = [&](int step) {
+        const float* at = place(step) + v_lane + step * F32_KEYS % P;
+#pragma unroll
+        for (int n = 0; n < DQ; ++n) vf[n] = *(const f32x4*)(at + (int64_t)16 * n * P);
+    };
+    auto scores = [&](auto from, auto to, f32x4* sc) {
+        constexpr int T0 = decltype(from)::value, T1 = decltype(to)::value;
+#pragma unroll
+        for (int t = T0; t < T1; ++t) sc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < DQ; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[buf][i][e], qf[i][e], sc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = T0; t < T1; ++t)
+                    sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][e], qf[t][i][e], sc[t], 0, 0, 0);
+    };
+    // scores of a step to probabilities: the row's maximum and sum, and the factor its sums get
+    auto weigh = [&](int t, int step, const f32x4 sc, f32x4& p, float& alpha) {
+        const int j0 = step * F32_KEYS;
         float x[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int j = j0 + 4 * c + e;
             const float score = CAP ? cap_log2 * tanhf(sc[e] * scale_log2) : sc[e] * scale_log2;  // (CAP: scale / cap)
-            x[e] = (j < lo || j > pos) ? NEG_BIG : score;
+            x[e] = (j < lo[t] || j > pos[t]) ? NEG_BIG : score;
         }
         float top = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
         top = fmaxf(top, __shfl_xor(top, 16, LLE_WAVE));
         top = fmaxf(top, __shfl_xor(top, 32, LLE_WAVE));
-        const float new_m = fmaxf(m, top);
+        const float new_m = fmaxf(m[t], top);
         // while the row has seen no key new_m is NEG_BIG as its masked scores are, and
         // exp2(0) = 1 would count them: shift such rows so that they give 0
         const float base = new_m <= NEG_BIG ? 0.f : new_m;
-        const float alpha = exp2f(m - base);
-        m = new_m;
-        f32x4 p;
+        alpha = exp2f(m[t] - base);
+        m[t] = new_m;
         float psum = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             p[e] = exp2f(x[e] - base);
             psum += p[e];
         }
-        l = l * alpha + psum;
+        l[t] = l[t] * alpha + psum;
+    };
+    auto values = [&](auto from, auto to, const f32x4* p, const float* alpha) {
+        constexpr int T0 = decltype(from)::value, T1 = decltype(to)::value;
 #pragma unroll
         for (int n = 0; n < DQ; ++n) {
-            o[n] *= alpha;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[buf][n][e], p[e], o[n], 0, 0, 0);
+            for (int t = T0; t < T1; ++t) o[t][n] *= alpha[t];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = T0; t < T1; ++t)
+                    o[t][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[n][e], p[t][e], o[t][n], 0, 0, 0);
         }
     };
-    [[maybe_unused]] const int w_pos = pos, w_lo = lo, w_begin = step_begin, w_end = step_end;
+    using None = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    using All = std::integral_constant<int, TILES>;
+    [[maybe_unused]] const int w_pos = pos[0], w_lo = lo[0], w_begin = step_begin, w_end = step_end;
     for (int range = KEEP && kept_end > 0 ? 0 : 1; range < 2; ++range) {
     if constexpr (KEEP) {
-        pos = range == 0 ? (exists ? min(keep_first, w_lo) - 1 : -1) : w_pos;
-        lo = range == 0 ? 0 : w_lo;
+        pos[0] = range == 0 ? (exists[0] ? min(keep_first, w_lo) - 1 : -1) : w_pos;
+        lo[0] = range == 0 ? 0 : w_lo;
         step_begin = range == 0 ? (few ? wave : 0) : w_begin;
         step_end = range == 0 ? kept_end : w_end;
     }
-    if constexpr (NBUF == 2) {
-        // the operands of the next step are asked for before this one is multiplied
-        if (step_begin < step_end) load(0, step_begin);
-        int buf = 0;
-        for (int step = step_begin; step < step_end; step += step_stride) {
-            if (step + step_stride < step_end) {
-                if (buf == 0) load(1, step + step_stride); else load(0, step + step_stride);
+    if (step_begin >= step_end) continue;
+    // K of the next step is asked for before the values of this one are multiplied, V of it before
+    // its scores are: the loads fly under the other product and take no registers of their own
+    load_k(step_begin);
+    load_v(step_begin);
+    for (int step = step_begin; step < step_end; step += step_stride) {
+        const int next = step + step_stride;
+        f32x4 sc[TILES], p[TILES];
+        float alpha[TILES];
+        // a tile takes part in the steps that its own rows see and in no other: the sums are those
+        // of tiles that work alone
+        const bool first_in = TILES == 1 || step < end[0];
+        const bool second_in = TILES == 2 && step >= first[TILES - 1] && step < end[TILES - 1];
+        if (TILES == 1 || (first_in && second_in)) {
+            scores(None{}, All{}, sc);
+            if (next < step_end) load_k(next);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) weigh(t, step, sc[t], p[t], alpha[t]);
+            values(None{}, All{}, p, alpha);
+        } else {
+            if (first_in) scores(None{}, One{}, sc);
+            else if (second_in) scores(One{}, All{}, sc);
+            if (next < step_end) load_k(next);
+            if (first_in) {
+                weigh(0, step, sc[0], p[0], alpha[0]);
+                values(None{}, One{}, p, alpha);
+            } else if (second_in) {
+                weigh(TILES - 1, step, sc[TILES - 1], p[TILES - 1], alpha[TILES - 1]);
+                values(One{}, All{}, p, alpha);
             }
-            if (buf == 0) multiply(0, step); else multiply(1, step);
-            buf ^= 1;
         }
-    } else {  // heads over 128 elements: the registers hold one step's operands
-        for (int step = step_begin; step < step_end; step += step_stride) {
-            load(0, step);
-            multiply(0, step);
-        }
+        if (next < step_end) load_v(next);
     }
     }
-    l += __shfl_xor(l, 16, LLE_WAVE);
-    l += __shfl_xor(l, 32, LLE_WAVE);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        l[t] += __shfl_xor(l[t], 16, LLE_WAVE);
+        l[t] += __shfl_xor(l[t], 32, LLE_WAVE);
+    }
 
-    if (!few) {  // every wavefront writes the rows of its own tile
-        if (!exists) return;
-        if (nsplit > 1) {
-            float* po = ws_o + (head_row * nsplit + split) * D;
+    if (!few) {  // every wavefront writes the rows of its own tiles
 #pragma unroll
-            for (int n = 0; n < DQ; ++n) *(f32x4*)(po + 16 * n + 4 * c) = o[n];
-            if (c == 0) {
-                ws_ml[(head_row * nsplit + split) * 2] = m;
-                ws_ml[(head_row * nsplit + split) * 2 + 1] = l;
+        for (int t = 0; t < TILES; ++t) {
+            if (!exists[t]) continue;
+            if (nsplit > 1) {
+                float* po = ws_o + (head_row[t] * nsplit + split) * D;
+#pragma unroll
+                for (int n = 0; n < DQ; ++n) *(f32x4*)(po + 16 * n + 4 * c) = o[t][n];
+                if (c == 0) {
+                    ws_ml[(head_row[t] * nsplit + split) * 2] = m[t];
+                    ws_ml[(head_row[t] * nsplit + split) * 2 + 1] = l[t];
+                }
+                continue;
             }
-            return;
-        }
-        // (a sink: a place in the sum without a value)
-        const float inv = 1.0f / (sinks ? l + exp2f(sinks[kvh * G + g] * 1.44269504088896340736f - m) : l);
+            // (a sink: a place in the sum without a value)
+            const float sum = sinks ? l[t] + exp2f(sinks[kvh * G + g[t]] * 1.44269504088896340736f - m[t]) : l[t];
+            const float inv = 1.0f / sum;
 #pragma unroll
-        for (int n = 0; n < DQ; ++n) *(f32x4*)(out + head_row * D + 16 * n + 4 * c) = o[n] * inv;
+            for (int n = 0; n < DQ; ++n) *(f32x4*)(out + head_row[t] * D + 16 * n + 4 * c) = o[t][n] * inv;
+        }
         return;
     }
     // few rows: the four wavefronts hold parts of the same rows
-    if (exists) {
+    if (exists[0]) {
 #pragma unroll
-        for (int n = 0; n < DQ; ++n) *(f32x4*)(s_o + (wave * 16 + r16) * D + 16 * n + 4 * c) = o[n];
+        for (int n = 0; n < DQ; ++n) *(f32x4*)(s_o + (wave * 16 + r16) * D + 16 * n + 4 * c) = o[0][n];
     }
     if (c == 0) {
-        s_m[wave * 16 + r16] = m;
-        s_l[wave * 16 + r16] = l;
+        s_m[wave * 16 + r16] = m[0];
+        s_l[wave * 16 + r16] = l[0];
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < nrows * D; idx += blockDim.x) {
@@ -1579,9 +1658,10 @@ extern "C" int lle_paged_attention_mfma_f32(const void* q, const void* kv_layer,
                                             const void* seq_slots, const void* cu_tokens, const void* kv_lens,
                                             void* out, void* ws_o, void* ws_ml, int N, int S, int nq, int nkv, int d,
                                             int page_size, int64_t page_stride, int max_pages, int window,
-                                            int keep_first, float scale, int row_blocks, int nsplit, const void* sinks,
-                                            float softcap, hipStream_t stream) {
+                                            int keep_first, float scale, int row_blocks, int tiles, int paired, int nsplit,
+                                            const void* sinks, float softcap, hipStream_t stream) {
     if (N <= 0) return 0;
+    if (tiles < 1 || tiles > 2 || (tiles == 2 && ((d != 64 && d != 128) || keep_first > 0 || softcap > 0.f))) return (int)hipErrorInvalidValue;
     if (d % 16 != 0 || d > 256 || d <= 0 || page_size % 16 != 0 || nq % nkv != 0) return (int)hipErrorInvalidValue;
     if (S > 65535 || nkv <= 0 || row_blocks < 1 || nsplit < 1 || nsplit > 64 || (int64_t)row_blocks * nsplit > 65535)
         return (int)hipErrorInvalidValue;
@@ -1601,15 +1681,21 @@ extern "C" int lle_paged_attention_mfma_f32(const void* q, const void* kv_layer,
         kernel<<<grid, F32_WAVES * LLE_WAVE, smem, stream>>>(
             (const float*)q, (const float*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots,
             (const int32_t*)cu_tokens, (const int32_t*)kv_lens, (float*)out, (float*)ws_o, (float*)ws_ml, nsplit, nq, nkv,
-            page_size, page_stride, max_pages, window, keep_first, scale_log2, (const float*)sinks, cap_log2);
+            page_size, page_stride, max_pages, window, keep_first, scale_log2, (const float*)sinks, cap_log2, paired);
         return hipGetLastError();
     };
     hipError_t launched = hipSuccess;
-#define LLE_F32_CASE(DQV)                                                                \
-    case DQV:                                                                            \
-        launched = keep_first > 0 ? launch(mfma_f32_attention_kernel<DQV, true, false>)  \
-                   : softcap > 0.f ? launch(mfma_f32_attention_kernel<DQV, false, true>) \
-                                   : launch(mfma_f32_attention_kernel<DQV, false, false>); \
+#define LLE_F32_CASE(DQV)                                                                     \
+    case DQV:                                                                                 \
+        if constexpr (DQV == 4 || DQV == 8) {                                                 \
+            if (tiles == 2) {                                                                 \
+                launched = launch(mfma_f32_attention_kernel<DQV, 2, false, false>);           \
+                break;                                                                        \
+            }                                                                                 \
+        }                                                                                     \
+        launched = keep_first > 0 ? launch(mfma_f32_attention_kernel<DQV, 1, true, false>)    \
+                   : softcap > 0.f ? launch(mfma_f32_attention_kernel<DQV, 1, false, true>)   \
+                                   : launch(mfma_f32_attention_kernel<DQV, 1, false, false>); \
         break;
     switch (d / 16) {
         LLE_F32_CASE(1) LLE_F32_CASE(2) LLE_F32_CASE(3) LLE_F32_CASE(4) LLE_F32_CASE(5) LLE_F32_CASE(6)

@@ -670,17 +670,20 @@ class HipOps:
                 and S <= 65535 and not both and not self.force_generic_attention):
             # float32 on the matrix cores (float32 operands, products and sums)
             rows = max_q_len * group
-            row_blocks = 1 if rows <= 16 else -(-rows // 64)
-            ns = self.f32_attention_splits(S, nkv, row_blocks, max_q_len, max_kv_len, win)
+            span = min(max_kv_len, win + max_q_len) if win else max_kv_len
+            tiles, paired, rounds = self.f32_attention_form(N, nq, nkv, d, keep == 0 and cap == 0.0, max_q_len, span)
+            row_blocks = 1 if rows <= 16 else -(-rows // (64 * tiles))
+            ns = self.f32_attention_splits(S, nkv, row_blocks, max_q_len, max_kv_len, win, rounds)
             ws_o = ws_ml = None
             if ns > 1:
                 ws_o = torch.empty((N * nq * ns * d,), dtype=torch.float32, device=q.device)
                 ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=q.device)
             self._run("attention", "lle_paged_attention_mfma_f32",
-                      [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I, _I, _F, _I, _I, _P, _F, _P],
+                      [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I, _I, _F, _I, _I, _I, _I, _P, _F,
+                       _P],
                       _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens),
                       _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size, kv_layer.stride(0),
-                      block_table.shape[1], win, keep, float(scale), row_blocks, ns, _ptr(sinks), cap)
+                      block_table.shape[1], win, keep, float(scale), row_blocks, tiles, paired, ns, _ptr(sinks), cap)
             return out
         if not mfma:
             self._run("attention", "lle_paged_attention_generic",
@@ -852,16 +855,42 @@ class HipOps:
             return 1 if low <= units or (low <= resident and max_kv_len <= max_q_len and num_seqs <= 1) else 3
         return 1 if low <= resident else 2
 
+    def f32_attention_form(self, N: int, nq: int, num_kv_heads: int, d: int, plain: bool, max_q_len: int,
+                           span: int) -> tuple:
+        """(tiles of 16 rows that a wavefront of the float32 matrix-core kernel takes, whether its long
+        and short row blocks are paired, rounds of the CUs that key splits may fill).
+        Two tiles share what is loaded of K and V, but half as many workgroups are left: from one and a
+        half blocks of 128 rows per CU on (measured, 32 / 8 heads of 128: a 2048-token prompt 372 us, in
+        one tile 481; a 1024-token one 184 and 126), and for portions with at least as much behind them,
+        2048 keys or more, which key splits spread instead (300 tokens behind 4000: 239 us, in one tile
+        469; 512 behind 2048: 220 and 285; 128 behind 1000: 53 and 44).
+        Between one and two blocks per CU all of them start at once and nothing evens out what the CUs
+        got: the second one of a CU is the shortest left (a 2048-token prompt 480 -> 372 us, a 1024-token
+        one 178 -> 126); otherwise the longest first (4096 tokens: 1386 us, paired 1584)."""
+        cus, group = self.compute_units(), nq // num_kv_heads
+        if max_q_len * group <= 16:  # decoding: a block a request and key split
+            return 1, 0, 1
+
+        def blocks(tiles):  # (the rows of several requests share no block: a few more than this)
+            return num_kv_heads * -(-N * group // (64 * tiles))
+
+        if not plain or d not in (64, 128):
+            tiles = 1
+        elif max_q_len * group > 64 and span >= max(2048, 2 * max_q_len) and 2 * blocks(2) < 3 * cus:
+            return 2, 0, 2
+        else:
+            tiles = 2 if 2 * blocks(2) >= 3 * cus else 1
+        return tiles, int(cus < blocks(tiles) <= 2 * cus), 1
+
     def f32_attention_splits(self, num_seqs: int, num_kv_heads: int, row_blocks: int, max_q_len: int,
-                             max_kv_len: int, window: int) -> int:
-        """Key splits of the float32 matrix-core kernel: enough workgroups for one round of the CUs
-        (measured: more cost 10 % at batch 8 and at 512-token portions), at least 4 of its 16-key
-        steps each (measured at 512 keys: batch 1 in 2 / 8 splits 20 / 12 us, batch 8 in 2 / 4 splits
-        22 / 18 us)."""
+                             max_kv_len: int, window: int, rounds: int = 1) -> int:
+        """Key splits of the float32 matrix-core kernel: enough workgroups for `rounds` rounds of the
+        CUs (decoding: one; measured at 1000 keys, batch 16: 29 us, two rounds 30, three 39), at least 4
+        of its 16-key steps each (measured at 512 keys: batch 1 in 2 / 8 splits 20 / 12 us, batch 8 in
+        2 / 4 splits 22 / 18 us)."""
         span = min(max_kv_len, window + max_q_len) if window else max_kv_len
-        steps = (span + 15) // 16
-        by_work = max(1, steps // 4)
-        by_fill = max(1, self.compute_units() // max(1, num_seqs * num_kv_heads * row_blocks))
+        by_work = max(1, (span + 15) // 16 // 4)
+        by_fill = max(1, rounds * self.compute_units() // max(1, num_seqs * num_kv_heads * row_blocks))
         return int(min(by_work, by_fill, 64))
 
     def decode_splits(self, num_seqs: int, num_kv_heads: int, max_kv_len: int, window: int) -> int:
