@@ -370,7 +370,7 @@ __device__ __forceinline__ float delta_token(float (&S)[KI], const DeltaToken<KI
 // ahead of their use.  The read-out is the lane's whose number the token has, so a chunk's leave from the registers.
 // Measured at 2048 tokens of 32 heads of 64 x 64, a decay per channel: 267 us with three barriers a chunk, k . q made
 // ahead of the walk (the read-out taken from the state before the correction, in the same pass) and the read-outs through
-// LDS; NEW_C us so.  Tried and not kept: all of a chunk's operands in registers before its first token.
+// LDS; 239 us so.  Tried and not kept: all of a chunk's operands in registers before its first token.
 template <int KI, bool CHANNEL>
 __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) {
     constexpr int KD = KI * DELTA_IG;
