@@ -23,6 +23,7 @@ LLE_DEFINE_ERROR_STRING()
 
 #define SSD_CHUNK 64
 #define SSD_WALK 32
+#define SSD_HEADS 32
 typedef float ssd_f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float ssd_silu(float x) { return x / (1.0f + expf(-x)); }
@@ -335,90 +336,129 @@ __device__ __forceinline__ void ssd_chunk_steps(const SsdArgs& a, int h, int t0,
     l_lo = (float)(l - (double)l_hi);
 }
 
-// Pass 1.  grid = (requests x pieces, heads), 256 threads.  B and x (times its factor) of the chunk wait in LDS; the
-// contribution, [vdim, n] as the state lies, is taken in 16 x 16 tiles, four tokens an instruction: a lane (c, r) gives
-// token 4 k + c of row (column) r.  Row strides of 16 modulo 64 words spread the four tokens over the banks.
-template <int JT>  // tiles of value channels that a wavefront keeps side by side
+// four consecutive elements of a row of `n`, zeros past its end
+template <bool WIDE>
+__device__ __forceinline__ ssd_f32x4 ssd_quad(const float* row, int i, int n) {
+    ssd_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (WIDE) {  // (n a multiple of 4, rows aligned)
+        if (i < n) v = *(const ssd_f32x4*)(row + i);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i + e < n) v[e] = row[i + e];
+    }
+    return v;
+}
+
+// x of a chunk and head on its way to LDS: thread `tid` has the quads tid, tid + 256 .. of [SSD_CHUNK][VX 64]
+template <int VX, bool WIDE>
+struct SsdX {
+    ssd_f32x4 v[4 * VX];
+    __device__ __forceinline__ void load(const float* rows, int CC, int h, int vdim, int nt) {
+#pragma unroll
+        for (int k = 0; k < 4 * VX; ++k) {
+            const int e = k * 256 + threadIdx.x, t = e / (16 * VX), i = (e - t * (16 * VX)) * 4;
+            v[k] = ssd_quad<WIDE>(rows + (int64_t)min(t, nt - 1) * CC + h * vdim, i, vdim);
+        }
+    }
+    // (tokens past the chunk's last one have a factor of 0, but another token's x: they are left out)
+    __device__ __forceinline__ void store(float* s_x, int XS, const float* factor, int nt) const {
+#pragma unroll
+        for (int k = 0; k < 4 * VX; ++k) {
+            const int e = k * 256 + threadIdx.x, t = e / (16 * VX), i = (e - t * (16 * VX)) * 4;
+            *(ssd_f32x4*)(s_x + t * XS + i) = t < nt ? v[k] * factor[t] : ssd_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+};
+
+// Pass 1.  grid = (requests x pieces, heads / heads_a_group), 256 threads.  A wavefront has NT tiles of 16 state channels;
+// their B stays in its registers for all heads that the workgroup takes.  x times its factor waits in LDS, two buffers: the
+// next head's is asked for before this one's is multiplied, one barrier a head.  The contribution, [vdim, n] as the state
+// lies, is taken in 16 x 16 tiles, four tokens an instruction: a lane (c, r) gives token 4 k + c of row (column) r and
+// gets four neighbouring state channels of a value channel.  A row stride of 16 modulo 64 words spreads the four tokens
+// over the banks.  What bounds it: the part's 32 KB a chunk and head of 64 x 128 that are written.
+// 2048 tokens of 64 heads of 64 x 128, four heads a workgroup: 61 us with a workgroup a head, B in LDS beside x; 39 so.
+template <int NT, int VX, bool WIDE>
 __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
+    constexpr int XS = VX * 64 + 16;
     extern __shared__ float lds[];
-    const int s = blockIdx.x / a.pieces, piece = blockIdx.x % a.pieces, h = blockIdx.y;
+    const int s = blockIdx.x / a.pieces, piece = blockIdx.x % a.pieces, h0 = blockIdx.y * a.heads_a_group;
     const int q0 = a.cu_tokens[s], len = a.cu_tokens[s + 1] - q0;
     if (len <= SSD_WALK || piece * SSD_CHUNK >= len) return;
     const int t0 = q0 + piece * SSD_CHUNK, nt = min(SSD_CHUNK, len - piece * SSD_CHUNK);
-    const int n = a.n, vdim = a.vdim, grp = h / (a.H / a.G), inner = a.H * vdim;
-    const int BS = (n + 63) / 64 * 64 + 16, XS = (vdim + 63) / 64 * 64 + 16;
-    float* s_B = lds;                    // [SSD_CHUNK][BS]
-    float* s_x = s_B + SSD_CHUNK * BS;   // [SSD_CHUNK][XS]
-    float* s_f = s_x + SSD_CHUNK * XS;   // [SSD_CHUNK] exp(l_last - l_s) dt_s
-    const int tid = threadIdx.x, wave = tid / LLE_WAVE, lane = tid % LLE_WAVE, c = lane / 16, r = lane % 16;
+    const int n = a.n, vdim = a.vdim, grp = h0 / (a.H / a.G), inner = a.H * vdim;
+    float* s_x = lds;                        // [2][SSD_CHUNK][XS]
+    float* s_f = s_x + 2 * SSD_CHUNK * XS;   // [heads][SSD_CHUNK] exp(l_last - l_s) dt_s
+    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE, c = lane / 16, r = lane % 16;
     const int64_t slot = ssd_slot(q0, s) + piece;
-    if (wave == 0) {
-        float dt, hi, lo;
-        ssd_chunk_steps(a, h, t0, nt, dt, hi, lo);
-        const float hi_last = __shfl(hi, LLE_WAVE - 1, LLE_WAVE), lo_last = __shfl(lo, LLE_WAVE - 1, LLE_WAVE);
-        s_f[lane] = expf((hi_last - hi) + (lo_last - lo)) * dt;
-        if (lane == 0) a.part_decay[slot * a.H + h] = expf(hi_last);
-    }
-    const int np = BS - 16, vp = XS - 16;
     const float* rows = a.c + (int64_t)t0 * a.CC;
-    const int bcol = inner + grp * n;
-    const bool wide = n % 4 == 0 && vdim % 4 == 0 && a.CC % 4 == 0 && bcol % 4 == 0;
-    if (wide) {
-        for (int e = tid; e < SSD_CHUNK * np / 4; e += 256) {
-            const int t = e / (np / 4), i = (e - t * (np / 4)) * 4;
-            *(float4*)(s_B + t * BS + i) = (t < nt && i < n) ? *(const float4*)(rows + (int64_t)t * a.CC + bcol + i) : float4{0.f, 0.f, 0.f, 0.f};
-        }
-    } else {
-        for (int e = tid; e < SSD_CHUNK * np; e += 256) {
-            const int t = e / np, i = e - t * np;
-            s_B[t * BS + i] = (t < nt && i < n) ? rows[(int64_t)t * a.CC + bcol + i] : 0.f;
+    SsdX<VX, WIDE> x;
+    x.load(rows, a.CC, h0, vdim, nt);
+    float B[NT][SSD_CHUNK / 4];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int i = (wave * NT + q) * 16 + r;
+        const float* col = rows + inner + grp * n + min(i, n - 1);
+#pragma unroll
+        for (int k = 0; k < SSD_CHUNK / 4; ++k) {
+            const float v = col[(int64_t)min(4 * k + c, nt - 1) * a.CC];
+            B[q][k] = (i < n && 4 * k + c < nt) ? v : 0.f;
         }
     }
-    __syncthreads();
-    if (wide) {
-        for (int e = tid; e < SSD_CHUNK * vp / 4; e += 256) {
-            const int t = e / (vp / 4), i = (e - t * (vp / 4)) * 4;
-            float4 v = float4{0.f, 0.f, 0.f, 0.f};
-            if (t < nt && i < vdim) {
-                v = *(const float4*)(rows + (int64_t)t * a.CC + h * vdim + i);
-                const float f = s_f[t];
-                v = float4{v.x * f, v.y * f, v.z * f, v.w * f};
-            }
-            *(float4*)(s_x + t * XS + i) = v;
-        }
-    } else {
-        for (int e = tid; e < SSD_CHUNK * vp; e += 256) {
-            const int t = e / vp, i = e - t * vp;
-            s_x[t * XS + i] = (t < nt && i < vdim) ? rows[(int64_t)t * a.CC + h * vdim + i] * s_f[t] : 0.f;
-        }
+    for (int hh = wave; hh < a.heads_a_group; hh += 4) {  // a wavefront a head
+        float dt, hi, lo;
+        ssd_chunk_steps(a, h0 + hh, t0, nt, dt, hi, lo);
+        const float hi_last = __shfl(hi, LLE_WAVE - 1, LLE_WAVE), lo_last = __shfl(lo, LLE_WAVE - 1, LLE_WAVE);
+        s_f[hh * SSD_CHUNK + lane] = expf((hi_last - hi) + (lo_last - lo)) * dt;
+        if (lane == 0) a.part_decay[slot * a.H + h0 + hh] = expf(hi_last);
     }
     __syncthreads();
-    float* out = a.part + (slot * a.H + h) * (int64_t)vdim * n;
-    const int j_tiles = (vdim + 15) / 16, n_tiles = (n + 15) / 16;
-    for (int nt0 = wave; nt0 < n_tiles; nt0 += 4) {
-        for (int jt0 = 0; jt0 < j_tiles; jt0 += JT) {
-            ssd_f32x4 acc[JT];
+    const int j_tiles = (vdim + 15) / 16;
+    for (int hh = 0; hh < a.heads_a_group; ++hh) {
+        float* own_x = s_x + (hh & 1) * SSD_CHUNK * XS;
+        x.store(own_x, XS, s_f + hh * SSD_CHUNK, nt);
+        __syncthreads();  // (and the buffer that the next head writes has been read)
+        if (hh + 1 < a.heads_a_group) x.load(rows, a.CC, h0 + hh + 1, vdim, nt);
+        float* out = a.part + (slot * a.H + h0 + hh) * (int64_t)vdim * n;
+        auto tiles = [&](auto jt_, int jt0) {  // so many tiles of value channels side by side
+            constexpr int JT = decltype(jt_)::value;
+            ssd_f32x4 acc[NT][JT];
 #pragma unroll
-            for (int q = 0; q < JT; ++q) acc[q] = ssd_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-            for (int k = 0; k < SSD_CHUNK; k += 4) {
-                const float b = s_B[(k + c) * BS + nt0 * 16 + r];
+            for (int q = 0; q < NT; ++q)
 #pragma unroll
-                for (int q = 0; q < JT; ++q) {
-                    const int jt = min(jt0 + q, j_tiles - 1);
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_x[(k + c) * XS + jt * 16 + r], b, acc[q], 0, 0, 0);
+                for (int p = 0; p < JT; ++p) acc[q][p] = ssd_f32x4{0.f, 0.f, 0.f, 0.f};
+            // (value channels past the last tile lie in the padding of the row, as zeros)
+#pragma unroll
+            for (int k = 0; k < SSD_CHUNK / 4; ++k) {
+                const float* xk = own_x + (4 * k + c) * XS + jt0 * 16 + r;
+#pragma unroll
+                for (int p = 0; p < JT; ++p) {
+                    const float xv = xk[p * 16];
+#pragma unroll
+                    for (int q = 0; q < NT; ++q) acc[q][p] = __builtin_amdgcn_mfma_f32_16x16x4f32(B[q][k], xv, acc[q][p], 0, 0, 0);
                 }
             }
 #pragma unroll
-            for (int q = 0; q < JT; ++q) {
-                const int j = (jt0 + q) * 16 + 4 * c, col = nt0 * 16 + r;
-                if (col < n) {
+            for (int q = 0; q < NT; ++q) {
+                const int i = (wave * NT + q) * 16 + 4 * c;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (jt0 + q < j_tiles && j + e < vdim) out[(int64_t)(j + e) * n + col] = acc[q][e];
+                for (int p = 0; p < JT; ++p) {
+                    const int j = (jt0 + p) * 16 + r;
+                    if (j >= vdim) continue;
+                    if (WIDE) {
+                        if (i < n) *(ssd_f32x4*)(out + (int64_t)j * n + i) = acc[q][p];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (i + e < n) out[(int64_t)j * n + i + e] = acc[q][p][e];
+                    }
                 }
             }
-        }
+        };
+        if (j_tiles == 1) tiles(std::integral_constant<int, 1>{}, 0);
+        else if (j_tiles == 2) tiles(std::integral_constant<int, 2>{}, 0);
+        else
+            for (int jt0 = 0; jt0 < j_tiles; jt0 += 4) tiles(std::integral_constant<int, 4>{}, jt0);
     }
 }
 
@@ -454,47 +494,56 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs a) {
     *own = S;
 }
 
-// four consecutive elements of a row of `n`, zeros past its end
-template <bool WIDE>
-__device__ __forceinline__ ssd_f32x4 ssd_quad(const float* row, int i, int n) {
-    ssd_f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (WIDE) {  // (n a multiple of 4, rows aligned)
-        if (i < n) v = *(const ssd_f32x4*)(row + i);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (i + e < n) v[e] = row[i + e];
-    }
-    return v;
-}
-
 // Pass 2.  grid = (requests x pieces, heads / heads_a_group), 256 threads; wavefront w has the chunk's tokens
 // 16 w .. 16 w + 15, and the products C_t . B_s of its rows stay in registers for all heads that the workgroup takes.
 // A lane (c, r) loads four neighbouring elements of a contraction of row r; element e is slot c of instruction e:
 //   M^T = B C^T: the result leaves the lane with token t = r and keys s = 4 c .. 4 c + 3 of a tile: the second operand of
 //   Y^T += (x dt)^T M^T (contraction over s), whose first operand comes from LDS, and of
 //   Y^T += S C^T (contraction over n) with the entry state's rows straight from memory.
+// The entry state's rows of the next tile of value channels are on their way while this one's are multiplied (states of up
+// to 128 channels: two sets of registers; wider ones: one, asked for again behind the products), also over the end of a
+// head; so is the next head's x, and the step sizes of all heads are made at the start, a wavefront a head.
 // LDS: x dt [SSD_CHUNK][XS], XS = 4 modulo 64 words: the rows 4 c + e of an instruction lie in different banks.
-template <int NQ, bool WIDE>
+// Bounded by the products (19 us at the matrix instruction's rate) and what four wavefronts read of the entry state, each for
+// itself: at the sizes above 79 us with one set of registers and each head's x and step sizes made at its start; 64 so.
+template <int NQ, int VX, bool WIDE>
 __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdArgs a) {
+    constexpr int XS = VX * 64 + 4, SETS = NQ <= 8 ? 2 : 1;
     extern __shared__ float lds[];
-    __shared__ float s_dt[SSD_CHUNK];
     const int s = blockIdx.x / a.pieces, piece = blockIdx.x % a.pieces, h0 = blockIdx.y * a.heads_a_group;
     const int q0 = a.cu_tokens[s], len = a.cu_tokens[s + 1] - q0;
     if (len <= SSD_WALK || piece * SSD_CHUNK >= len) return;
     const int t0 = q0 + piece * SSD_CHUNK, nt = min(SSD_CHUNK, len - piece * SSD_CHUNK);
     const int n = a.n, vdim = a.vdim, grp = h0 / (a.H / a.G), inner = a.H * vdim;
-    const int XS = (vdim + 63) / 64 * 64 + 4, vp = XS - 4;
     float* s_x = lds;
-    const int tid = threadIdx.x, wave = tid / LLE_WAVE, lane = tid % LLE_WAVE, c = lane / 16, r = lane % 16;
+    float* s_dt = s_x + SSD_CHUNK * XS;                    // [heads][SSD_CHUNK]
+    float* s_hi = s_dt + a.heads_a_group * SSD_CHUNK;      // likewise
+    float* s_lo = s_hi + a.heads_a_group * SSD_CHUNK;
+    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE, c = lane / 16, r = lane % 16;
     const int64_t slot = ssd_slot(q0, s) + piece;
     const float* rows = a.c + (int64_t)t0 * a.CC;
     const int tok = wave * 16 + r;  // this lane's token of the chunk
+    const int j_tiles = (vdim + 15) / 16;
+    ssd_f32x4 sv[SETS][NQ];
+    auto entry_rows = [&](int set, int h, int jt) {
+        const float* row = a.part + (slot * a.H + h) * (int64_t)vdim * n + (int64_t)min(jt * 16 + r, vdim - 1) * n;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) sv[set][q] = ssd_quad<WIDE>(row, 16 * q + 4 * c, n);
+    };
+    SsdX<VX, WIDE> x;
+    x.load(rows, a.CC, h0, vdim, nt);
     ssd_f32x4 C[NQ], cb[4];
     {
         const float* crow = rows + (int64_t)min(tok, nt - 1) * a.CC + inner + (a.G + grp) * n;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) C[q] = ssd_quad<WIDE>(crow, 16 * q + 4 * c, n);
+    }
+    for (int hh = wave; hh < a.heads_a_group; hh += 4) {
+        float dt, hi, lo;  // of token `lane` of the chunk
+        ssd_chunk_steps(a, h0 + hh, t0, nt, dt, hi, lo);
+        s_dt[hh * SSD_CHUNK + lane] = dt;
+        s_hi[hh * SSD_CHUNK + lane] = hi;
+        s_lo[hh * SSD_CHUNK + lane] = lo;
     }
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
@@ -509,84 +558,82 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdArgs a) {
             }
         }
     }
-    for (int hh = 0; hh < a.heads_a_group; ++hh) {
+    entry_rows(0, h0, 0);
+    ssd_f32x4 m[4];
+    float entry = 0.f, D = 0.f;
+    // a tile of value channels of head h0 + hh; `set`: where its entry rows are
+    auto tile = [&](auto set_, int hh, int jt) {
+        constexpr int SET = decltype(set_)::value, OTHER = SETS - 1 - SET;
         const int h = h0 + hh;
-        // the entry state's first rows are asked for now, the later ones while the rows before them are multiplied
-        const float* S = a.part + (slot * a.H + h) * (int64_t)vdim * n;
-        ssd_f32x4 sv[NQ];
+        const bool last = jt + 1 == j_tiles;
+        const bool more = !last || hh + 1 < a.heads_a_group;
+        const int j = jt * 16 + 4 * c;
+        const ssd_f32x4 xj = ssd_quad<WIDE>(rows + (int64_t)min(tok, nt - 1) * a.CC + h * vdim, j, vdim);
+        if (SETS == 2 && more) entry_rows(OTHER, last ? h + 1 : h, last ? 0 : jt + 1);
+        // (two chains of sums: a product waits for the one before it in its own chain only)
+        ssd_f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) sv[q] = ssd_quad<WIDE>(S + (int64_t)min(r, vdim - 1) * n, 16 * q + 4 * c, n);
-        float dt, hi, lo;  // of token `lane` of the chunk (every wavefront makes them for itself)
-        ssd_chunk_steps(a, h, t0, nt, dt, hi, lo);
-        if (hh > 0) __syncthreads();  // (the head before has been read)
-        if (wave == 0) s_dt[lane] = dt;
-        __syncthreads();
-        if (WIDE) {
-            for (int e = tid; e < SSD_CHUNK * vp / 4; e += 256) {
-                const int t = e / (vp / 4), i = (e - t * (vp / 4)) * 4;
-                ssd_f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (t < nt && i < vdim) v = *(const ssd_f32x4*)(rows + (int64_t)t * a.CC + h * vdim + i) * s_dt[t];
-                *(ssd_f32x4*)(s_x + t * XS + i) = v;
-            }
-        } else {
-            for (int e = tid; e < SSD_CHUNK * vp; e += 256) {
-                const int t = e / vp, i = e - t * vp;
-                s_x[t * XS + i] = (t < nt && i < vdim) ? rows[(int64_t)t * a.CC + h * vdim + i] * s_dt[t] : 0.f;
+        for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[SET][q][e], C[q][e], acc, 0, 0, 0);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[SET][q][e + 1], C[q][e + 1], acc2, 0, 0, 0);
             }
         }
-        __syncthreads();
-        const float hi_t = __shfl(hi, tok, LLE_WAVE), lo_t = __shfl(lo, tok, LLE_WAVE);
-        ssd_f32x4 m[4];
+        if (SETS == 1 && more) entry_rows(0, last ? h + 1 : h, last ? 0 : jt + 1);
+        acc = (acc + acc2) * entry;
+        acc2 = ssd_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
+            if (st <= wave) {  // (the same for the whole wavefront)
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    const float* x2 = s_x + (st * 16 + 4 * c + e) * XS + jt * 16 + r;
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x2[0], m[st][e], acc, 0, 0, 0);
+                    acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x2[XS], m[st][e + 1], acc2, 0, 0, 0);
+                }
+            }
+        }
+        acc += acc2;
+        if (tok < nt) {
+            float* y = a.y + (int64_t)(t0 + tok) * inner + h * vdim;
+            if (WIDE) {
+                if (j < vdim) *(ssd_f32x4*)(y + j) = xj * D + acc;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (j + e < vdim) y[j + e] = fmaf(D, xj[e], acc[e]);
+            }
+        }
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, SETS - 1>;
+    for (int hh = 0; hh < a.heads_a_group; ++hh) {
+        __syncthreads();  // (step sizes are there; the head before has been read)
+        x.store(s_x, XS, s_dt + hh * SSD_CHUNK, nt);
+        __syncthreads();
+        if (hh + 1 < a.heads_a_group) x.load(rows, a.CC, h0 + hh + 1, vdim, nt);
+        const float *hi = s_hi + hh * SSD_CHUNK, *lo = s_lo + hh * SSD_CHUNK;
+        const float hi_t = hi[tok], lo_t = lo[tok];
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            const ssd_f32x4 hi_s = *(const ssd_f32x4*)(hi + st * 16 + 4 * c), lo_s = *(const ssd_f32x4*)(lo + st * 16 + 4 * c);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int key = st * 16 + 4 * c + e;
-                const float hi_s = __shfl(hi, key, LLE_WAVE), lo_s = __shfl(lo, key, LLE_WAVE);
                 // (later keys weigh nothing; their exponent would be above zero)
-                m[st][e] = key <= tok ? cb[st][e] * expf((hi_t - hi_s) + (lo_t - lo_s)) : 0.f;
+                m[st][e] = key <= tok ? cb[st][e] * expf((hi_t - hi_s[e]) + (lo_t - lo_s[e])) : 0.f;
             }
         }
-        const float entry = expf(hi_t), D = a.D[h];
-        for (int jt = 0; jt * 16 < vdim; ++jt) {
-            // (two chains of sums: a product waits for the one before it in its own chain only)
-            ssd_f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
+        entry = expf(hi_t);
+        D = a.D[h0 + hh];
+        for (int jt = 0; jt < j_tiles; jt += 2) {
+            tile(First{}, hh, jt);
+            if (jt + 1 < j_tiles) {
+                tile(Second{}, hh, jt + 1);
+            } else if (SETS == 2) {
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-#pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[q][e], C[q][e], acc, 0, 0, 0);
-                    acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[q][e + 1], C[q][e + 1], acc2, 0, 0, 0);
-                }
-            }
-            const float* next = S + (int64_t)min((jt + 1) * 16 + r, vdim - 1) * n;
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) sv[q] = ssd_quad<WIDE>(next, 16 * q + 4 * c, n);
-            acc = (acc + acc2) * entry;
-            acc2 = ssd_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st <= wave) {  // (the same for the whole wavefront)
-#pragma unroll
-                    for (int e = 0; e < 4; e += 2) {
-                        const float* x2 = s_x + (st * 16 + 4 * c + e) * XS + jt * 16 + r;
-                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x2[0], m[st][e], acc, 0, 0, 0);
-                        acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x2[XS], m[st][e + 1], acc2, 0, 0, 0);
-                    }
-                }
-            }
-            acc += acc2;
-            if (tok < nt) {
-                const int j = jt * 16 + 4 * c;
-                const float* x = rows + (int64_t)tok * a.CC + h * vdim;
-                float* y = a.y + (int64_t)(t0 + tok) * inner + h * vdim;
-                if (WIDE) {
-                    if (j < vdim) *(ssd_f32x4*)(y + j) = *(const ssd_f32x4*)(x + j) * D + acc;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (j + e < vdim) y[j + e] = fmaf(D, x[j + e], acc[e]);
-                }
+                for (int q = 0; q < NQ; ++q) sv[0][q] = sv[SETS - 1][q];
             }
         }
     }
@@ -609,6 +656,9 @@ extern "C" int lle_ssd_scan(const void* c, int CC, const void* dt_in, int dt_col
         pieces < 0 || heads_a_group <= 0 || (H / G) % heads_a_group || (int64_t)S * (pieces > 0 ? pieces : 1) > 0x7fffffff ||
         (pieces > 0 && (!part || !part_decay)))
         return (int)hipErrorInvalidValue;
+    // LDS holds the step sizes of a workgroup's heads: at most SSD_HEADS of them
+    for (int k = SSD_HEADS; heads_a_group > SSD_HEADS; --k)
+        if (heads_a_group % k == 0) heads_a_group = k;
     const SsdArgs a{(const float*)c, CC, (const float*)dt_in, dt_cols, (const float*)dt_bias, (const float*)a_log, (const float*)D,
                     (float*)state, state_stride, (const int32_t*)seq_slots, (const int32_t*)cu_tokens, (float*)y, H, G, vdim, n,
                     heads_a_group, pieces, (float*)part, (float*)part_decay, (uintptr_t)state % 16 == 0 && state_stride % 4 == 0};
@@ -623,48 +673,56 @@ extern "C" int lle_ssd_scan(const void* c, int CC, const void* dt_in, int dt_col
         if (e != hipSuccess || pieces == 0) return (int)e;
     }
     if (pieces == 0) return 0;
-    {
-        const int BS = (n + 63) / 64 * 64 + 16, XS = (vdim + 63) / 64 * 64 + 16;
-        const size_t lds = ((size_t)SSD_CHUNK * (BS + XS) + SSD_CHUNK) * sizeof(float);
-        auto go = [&](auto kernel) {
-            if (lds > 64 * 1024) {
-                const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                if (e != hipSuccess) return e;
-            }
-            kernel<<<dim3(S * pieces, H), 256, lds, stream>>>(a);
-            return hipGetLastError();
-        };
-        const hipError_t e = vdim <= 16 ? go(ssd_chunk_state_kernel<1>) : vdim <= 32 ? go(ssd_chunk_state_kernel<2>) : go(ssd_chunk_state_kernel<4>);
-        if (e != hipSuccess) return (int)e;
-    }
-    ssd_carry_kernel<<<dim3(S, H, (vdim * n + 255) / 256), 256, 0, stream>>>(a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
-    const size_t lds = (size_t)SSD_CHUNK * ((vdim + 63) / 64 * 64 + 4) * sizeof(float);
     const bool wide = n % 4 == 0 && vdim % 4 == 0;  // (then CC and every column offset are multiples of 4 too)
     const dim3 grid(S * pieces, H / heads_a_group);
-    auto go = [&](auto narrow_k, auto wide_k) {
-        const void* k = wide ? (const void*)wide_k : (const void*)narrow_k;
+    auto go = [&](auto kernel, size_t lds) {
         if (lds > 64 * 1024) {
-            const hipError_t e2 = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e2 != hipSuccess) return (int)e2;
+            const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
         }
-        if (wide) wide_k<<<grid, 256, lds, stream>>>(a);
-        else narrow_k<<<grid, 256, lds, stream>>>(a);
-        return (int)hipGetLastError();
+        kernel<<<grid, 256, lds, stream>>>(a);
+        return hipGetLastError();
     };
+    const int VX = (vdim + 63) / 64;
+    auto by_width = [&](auto launch) {  // launch(how many times 64 value channels, whether 16 bytes a load)
+        using No = std::false_type;
+        using Yes = std::true_type;
+        switch (VX) {
+            case 1: return wide ? launch(std::integral_constant<int, 1>{}, Yes{}) : launch(std::integral_constant<int, 1>{}, No{});
+            case 2: return wide ? launch(std::integral_constant<int, 2>{}, Yes{}) : launch(std::integral_constant<int, 2>{}, No{});
+            case 3: return wide ? launch(std::integral_constant<int, 3>{}, Yes{}) : launch(std::integral_constant<int, 3>{}, No{});
+            default: return wide ? launch(std::integral_constant<int, 4>{}, Yes{}) : launch(std::integral_constant<int, 4>{}, No{});
+        }
+    };
+    hipError_t e = by_width([&](auto vx, auto w) {
+        constexpr int V = decltype(vx)::value;
+        constexpr bool W = decltype(w)::value;
+        const size_t lds = ((size_t)2 * SSD_CHUNK * (V * 64 + 16) + heads_a_group * SSD_CHUNK) * sizeof(float);
+        if (n <= 64) return go(ssd_chunk_state_kernel<1, V, W>, lds);
+        if (n <= 128) return go(ssd_chunk_state_kernel<2, V, W>, lds);
+        return go(ssd_chunk_state_kernel<4, V, W>, lds);
+    });
+    if (e != hipSuccess) return (int)e;
+    ssd_carry_kernel<<<dim3(S, H, (vdim * n + 255) / 256), 256, 0, stream>>>(a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return (int)e;
+    return (int)by_width([&](auto vx, auto w) {
+        constexpr int V = decltype(vx)::value;
+        constexpr bool W = decltype(w)::value;
+        const size_t lds = ((size_t)SSD_CHUNK * (V * 64 + 4) + 3 * heads_a_group * SSD_CHUNK) * sizeof(float);
 #define SSD_OUT_CASE(NQ) \
-    if (n <= 16 * NQ) return go(ssd_chunk_out_kernel<NQ, false>, ssd_chunk_out_kernel<NQ, true>);
-    SSD_OUT_CASE(1)
-    SSD_OUT_CASE(2)
-    SSD_OUT_CASE(3)
-    SSD_OUT_CASE(4)
-    SSD_OUT_CASE(6)
-    SSD_OUT_CASE(8)
-    SSD_OUT_CASE(12)
-    SSD_OUT_CASE(16)
+    if (n <= 16 * NQ) return go(ssd_chunk_out_kernel<NQ, V, W>, lds);
+        SSD_OUT_CASE(1)
+        SSD_OUT_CASE(2)
+        SSD_OUT_CASE(3)
+        SSD_OUT_CASE(4)
+        SSD_OUT_CASE(6)
+        SSD_OUT_CASE(8)
+        SSD_OUT_CASE(12)
+        SSD_OUT_CASE(16)
 #undef SSD_OUT_CASE
-    return (int)hipErrorInvalidValue;
+        return hipErrorInvalidValue;
+    });
 }
 
 // ---------------------------------------------------------------------------------
