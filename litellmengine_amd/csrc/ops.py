@@ -88,7 +88,8 @@ class HipOps:
         if not torch.cuda.is_available():
             raise KernelError("litellmengine_amd needs a GPU: its kernels have no CPU form")
         self._fn = {}
-        self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta)
+        self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta) ...
+        self._forms_tuning = None  # ... with these numbers
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives)
 
     # -- plumbing ---------------------------------------------------------
@@ -368,6 +369,8 @@ class HipOps:
     def _form_of_delta(self, dtype, M: int, N: int, K: int):
         """(form, slices of K) in which a product is taken whose reader adds up partial sums.  The choice is made from the sizes
         alone and kept for the next product of the same sizes: made anew each time it costs the host as much as the launch."""
+        if self._forms_tuning is not self.tuning:  # (other numbers choose anew)
+            self._forms, self._forms_tuning = {}, self.tuning
         key = (dtype, M, N, K, self.force_library_gemm)
         form = self._forms.get(key)
         if form is None:

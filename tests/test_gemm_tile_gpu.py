@@ -47,3 +47,19 @@ def test_which_products_take_it():
     assert isinstance(cut, PartialSums) and o.linear(x, w).shape == (200, 4096)
     want = x.double() @ w.double().T
     assert float((cut.total().double() - want).norm() / want.norm()) < 2.0 ** -24 * 64  # (sqrt(K) roundings)
+
+
+def test_other_numbers_choose_anew(monkeypatch):
+    """The form that was chosen for a product's sizes is chosen again when the numbers behind the choice change."""
+    import dataclasses
+
+    from litellmengine_amd.csrc.ops import HipOps
+
+    o = ops()
+    sizes = [(m, n, k) for m in (17, 64, 100, 512) for n, k in ((4096, 4096), (4096, 12288), (1024, 3072))]
+    before = [o._form_of_delta(torch.bfloat16, *s) for s in sizes]
+    other = dataclasses.replace(o.tuning, sliced_min_fill=0.0, partial_sums_bytes_per_s=1e15, library_max_slices=1)
+    monkeypatch.setattr(o, "tuning", other)
+    assert [o._form_of_delta(torch.bfloat16, *s) for s in sizes] == [HipOps(tuning=other)._form_of_delta(torch.bfloat16, *s) for s in sizes]
+    monkeypatch.undo()
+    assert [o._form_of_delta(torch.bfloat16, *s) for s in sizes] == before
