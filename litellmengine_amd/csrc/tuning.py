@@ -25,7 +25,8 @@ class ProductTuning:
     # head of the 8B sizes: 41-43 against the library's 49 us, 239-250 against 270; qkv, 24 rows a CU,
     # is the library's: 15-17 against 15 us)
     stream_32_rows_min_share: int = 64
-    # the float32 twin takes up to this many rows (the tiled float32 kernel wastes its 64-row tiles on fewer)
+    # the float32 twins and the product in slices take up to this many rows (the tiled float32 kernels waste their
+    # 64-row tiles on fewer)
     skinny_f32_max_rows: int = 64
     # the sliced product (17 to 128 rows) is taken where its workgroups fill at least this share
     # of whole rounds of the CUs ...
