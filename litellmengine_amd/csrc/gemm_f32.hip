@@ -196,7 +196,6 @@ struct SplitTile {
     float alone, shared;
 };
 static const SplitTile split_tiles[4] = {{4, 2, 2.70f, 2.35f}, {2, 2, 1.63f, 1.28f}, {2, 1, 1.09f, 0.74f}, {1, 1, 0.70f, 0.43f}};
-static const SplitTile halves_tiles[4] = {{4, 2, 1.84f, 1.45f}, {2, 2, 1.04f, 0.87f}, {2, 1, 0.70f, 0.55f}, {1, 1, 0.55f, 0.41f}};
 
 static int units_of_device() {
     static int units[64] = {0};
@@ -208,13 +207,13 @@ static int units_of_device() {
 
 // The tiles, and the slices of K (up to `most`), that take the least time by the steps of the CU with the most tiles, plus the
 // way of the slices' sums to their reader and back at 5 TB/s.
-static void choose(const SplitTile* table, int M, int N, int K, int most, int& tiles, int& slices) {
+static void choose(int M, int N, int K, int most, int& tiles, int& slices) {
     const int units = units_of_device(), steps = (K + SG_BK - 1) / SG_BK;
     float best = 0.f;
     tiles = 0, slices = 1;
     for (int s = 1; s <= most; ++s)
         for (int t = 0; t < 4; ++t) {
-            const SplitTile& v = table[t];
+            const SplitTile& v = split_tiles[t];
             const int64_t count = (int64_t)((M + 64 * v.tm - 1) / (64 * v.tm)) * ((N + 64 * v.tn - 1) / (64 * v.tn)) * s;
             const float each = fmaxf(v.alone, (float)((count + units - 1) / units) * v.shared);
             const float us = (float)((steps + s - 1) / s) * each + (s > 1 ? (float)s * M * N * 8 / 5e6f : 0.f);
@@ -226,7 +225,7 @@ static void choose(const SplitTile* table, int M, int N, int K, int most, int& t
 extern "C" int lle_gemm_nt_f32_slices(int M, int N, int K) {
     int tiles, slices;
     if (M <= 0 || N <= 0 || K <= 0) return 1;
-    choose(split_tiles, M, N, K, 8, tiles, slices);
+    choose(M, N, K, 8, tiles, slices);
     return slices;
 }
 
@@ -240,7 +239,7 @@ extern "C" int lle_gemm_nt_f32(const void* A, const void* B, void* C, int M, int
     if (tiles < 0) {
         int unused;
         // (a slice's product is as long as a whole one of its part of K)
-        choose(split_tiles, M, N * slices, (K + slices - 1) / slices, 1, tiles, unused);
+        choose(M, N * slices, (K + slices - 1) / slices, 1, tiles, unused);
     }
     const float *a = (const float*)A, *b = (const float*)B;
     float* c = (float*)C;
@@ -249,254 +248,6 @@ extern "C" int lle_gemm_nt_f32(const void* A, const void* B, void* C, int M, int
         case 1: return launch_split<2, 2, 3>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
         case 2: return launch_split<2, 1, 4>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
         case 3: return launch_split<1, 1, 6>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
-        default: return (int)hipErrorInvalidValue;
-    }
-}
-
-// ---------------------------------------------------------------------------------
-// The same in half as many products where both operands have been looked over: a float32 number, times a power of two that
-// brings its row's largest to 2^12 .. 2^14, is the sum of two halves and a rest of 2^-24 of it at most (of 2^-25 itself where
-// it is below 2^-12 or so, 2^-37 of the row's largest), so
-//   a b = a1 b1 + (a1 b2 + a2 b1) + what is about 2^-24 of it, and 2^-37 of the largest product of the rows:
-// as much as one float32 rounding of a b.  A's rows are split ahead (split_rows_kernel: each has its own power of two); B is
-// split on the way to LDS with one power of two for all of it, which the caller vouches for (no row's largest below 2^-13 of
-// the largest of all).
-// ---------------------------------------------------------------------------------
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-// two numbers as their two half parts, packed
-__device__ __forceinline__ void halves2(float a, float b, uint32_t& p1, uint32_t& p2) {
-    const half2v h1 = {(_Float16)a, (_Float16)b};
-    const half2v h2 = {(_Float16)(a - (float)h1[0]), (_Float16)(b - (float)h1[1])};
-    p1 = __builtin_bit_cast(uint32_t, h1);
-    p2 = __builtin_bit_cast(uint32_t, h2);
-}
-
-// What lle_gemm_nt_f32_halves has to be told of B [N][K]: every workgroup's largest number and least row's largest (rows of
-// zeros aside), as bits without signs (a NaN is larger than an infinity), to bounds [gridDim.x][2].
-#define BOUNDS_BLOCKS 1024
-__global__ __launch_bounds__(256) void weight_bounds_kernel(const uint32_t* __restrict__ B, uint32_t* __restrict__ bounds, int N, int K) {
-    __shared__ uint32_t s_most[4], s_least[4];
-    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
-    uint32_t most = 0u, least = 0x7f7fffffu;
-    for (int n = blockIdx.x * 4 + wave; n < N; n += gridDim.x * 4) {
-        const uint32_t* row = B + (int64_t)n * K;
-        uint32_t big = 0u;
-        for (int k = 4 * lane; k < K; k += 4 * LLE_WAVE) {
-            const su32x4 x = *(const su32x4*)(row + k) & 0x7fffffffu;
-            big = max(max(big, max(x[0], x[1])), max(x[2], x[3]));
-        }
-#pragma unroll
-        for (int o = LLE_WAVE / 2; o > 0; o >>= 1) big = max(big, (uint32_t)__shfl_xor((int)big, o, LLE_WAVE));
-        most = max(most, big);
-        if (big) least = min(least, big);
-    }
-    if (lane == 0) s_most[wave] = most, s_least[wave] = least;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        bounds[2 * blockIdx.x] = max(max(s_most[0], s_most[1]), max(s_most[2], s_most[3]));
-        bounds[2 * blockIdx.x + 1] = min(min(s_least[0], s_least[1]), min(s_least[2], s_least[3]));
-    }
-}
-
-extern "C" int lle_weight_bounds_blocks(void) { return BOUNDS_BLOCKS; }
-extern "C" int lle_weight_bounds(const void* B, void* bounds, int N, int K, hipStream_t stream) {
-    if (N <= 0 || K <= 0 || K % 4 != 0) return (int)hipErrorInvalidValue;
-    weight_bounds_kernel<<<BOUNDS_BLOCKS, 256, 0, stream>>>((const uint32_t*)B, (uint32_t*)bounds, N, K);
-    LLE_RETURN_LAUNCH_STATUS();
-}
-
-// parts [2][M][KP] (KP: K up to a multiple of 32, zeros past K) of A [M][lda] times 2^(13 - exponent of the row's largest), and
-// back[m], the factor that takes it back.  A row without a number of its own (zeros, infinities, NaN) is taken as it is.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, int64_t lda, int K, int KP, uint32_t* __restrict__ parts,
-                                                         int64_t part_stride, float* __restrict__ back) {
-    __shared__ float red[16];
-    const int64_t m = blockIdx.x;
-    const float* row = A + m * lda;
-    float big = 0.f;
-    for (int k = 4 * threadIdx.x; k < K; k += 1024) {
-        const sf32x4 x = *(const sf32x4*)(row + k);
-        big = fmaxf(big, fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
-    }
-    big = block_max(big, red);
-    int e = (int)((__builtin_bit_cast(uint32_t, big) >> 23) & 255) - 127;  // (rows of numbers below 2^-113: up to 2^13 only)
-    if (big == 0.f || e == 128) e = 13;
-    const int up = min(13 - e, 126);
-    const float scale = __builtin_bit_cast(float, (uint32_t)(127 + up) << 23);
-    if (threadIdx.x == 0) back[m] = __builtin_bit_cast(float, (uint32_t)(127 - up) << 23);
-    uint32_t *p1 = parts + m * (KP / 2), *p2 = p1 + part_stride;
-    for (int k = 4 * threadIdx.x; k < KP; k += 1024) {
-        sf32x4 x = {0.f, 0.f, 0.f, 0.f};
-        if (k < K) x = *(const sf32x4*)(row + k);
-        uint32_t a, b, c, d;
-        halves2(x[0] * scale, x[1] * scale, a, b);
-        halves2(x[2] * scale, x[3] * scale, c, d);
-        *(uint2*)(p1 + k / 2) = make_uint2(a, c);
-        *(uint2*)(p2 + k / 2) = make_uint2(b, d);
-    }
-}
-
-// Tiles, slices and stages as gemm_nt_split_kernel.  2048 x 24576 x 4096: 1772 -> 1141 us with the splitting of A (361 TFLOP/s
-// of float32 product), 2048 x 4096 x 12288 986 -> 687, 300 x 24576 x 4096 433 -> 311, 100 x 24576 x 4096 190 -> 163; the error
-// against 64 bits 1.0e-6 -> 0.71e-6 at K = 4096 (half as many roundings of a sum).
-template <int TM, int TN, int PER_SIMD>
-__global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_halves_kernel(const float* __restrict__ A, const _Float16* __restrict__ parts,
-                                                                       int64_t part_stride, const float* __restrict__ back,
-                                                                       const float* __restrict__ B, float* __restrict__ C, int M, int N, int K,
-                                                                       int KP, float b_scale, float b_back, int m_tiles, int n_tiles, int slice) {
-    constexpr int BM = 64 * TM, BN = 64 * TN, PLANE = SG_BK * 2;
-    extern __shared__ __attribute__((aligned(16))) unsigned char sg_lds[];
-    unsigned char* as = sg_lds;                     // [2 parts][BM][4 pieces of 16 bytes]
-    unsigned char* bs = sg_lds + 2 * BM * PLANE;    // [2 parts][BN][4 pieces]
-    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
-    const int die = blockIdx.x % 8, at = blockIdx.x / 8;
-    const int nt = die + 8 * (at / m_tiles), mt = at % m_tiles;
-    if (nt >= n_tiles) return;
-    const int m0 = mt * BM, n0 = nt * BN;
-    const int k_begin = blockIdx.y * slice, k_end = min(K, k_begin + slice);  // (a slice is a whole number of steps)
-    C += (int64_t)blockIdx.y * M * N;
-    const int lr = threadIdx.x / SG_PIECES, lp = threadIdx.x % SG_PIECES;
-    const _Float16* ap[TM];
-    const float* bp[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) ap[i] = parts + (int64_t)min(m0 + 64 * i + lr, M - 1) * KP + 8 * lp;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bp[j] = B + (int64_t)min(n0 + 64 * j + lr, N - 1) * K;
-    const int dst = lr * PLANE + ((lp ^ ((lr >> 3) & 3)) * 16);
-    su32x4 ar[TM][2];
-    sf32x4 br[TN][2];
-    auto issue = [&](int k0) {
-        const int ka = min(k0 + 8 * lp, K - 4), kb = min(k0 + 8 * lp + 4, K - 4), kp = min(k0, KP - SG_BK);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) ar[i][0] = *(const su32x4*)(ap[i] + kp), ar[i][1] = *(const su32x4*)(ap[i] + part_stride + kp);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) br[j][0] = *(const sf32x4*)(bp[j] + ka), br[j][1] = *(const sf32x4*)(bp[j] + kb);
-    };
-    const int wm = (wave / 2) * 32 * TM, wn = (wave % 2) * 32 * TN;
-    sf32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    const int fr = lane % 32, fh = lane / 32;
-    const unsigned char* af = as + (wm + fr) * PLANE;
-    const unsigned char* bf = bs + (wn + fr) * PLANE;
-
-    issue(k_begin);
-    for (int k0 = k_begin; k0 < k_end; k0 += SG_BK) {  // (past the end A's parts are zeros, B's repeated columns count for nothing)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            unsigned char* d = as + 64 * i * PLANE + dst;
-            *(su32x4*)d = ar[i][0];
-            *(su32x4*)(d + BM * PLANE) = ar[i][1];
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            su32x4 p1, p2;
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                uint32_t q1, q2;
-                halves2(br[j][h / 2][2 * (h % 2)] * b_scale, br[j][h / 2][2 * (h % 2) + 1] * b_scale, q1, q2);
-                p1[h] = q1, p2[h] = q2;
-            }
-            unsigned char* d = bs + 64 * j * PLANE + dst;
-            *(su32x4*)d = p1;
-            *(su32x4*)(d + BN * PLANE) = p2;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        issue(k0 + SG_BK);  // on its way while this step is multiplied (past the end: the last columns again)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int s = 0; s < SG_BK / 16; ++s) {
-            const int piece = ((2 * s + fh) ^ ((fr >> 3) & 3)) * 16;
-            half8 b[TN][2];
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int p = 0; p < 2; ++p) b[j][p] = *(const half8*)(bf + (p * BN + 32 * j) * PLANE + piece);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                half8 a[2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p) a[p] = *(const half8*)(af + (p * BM + 32 * i) * PLANE + piece);
-                constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};  // the smallest products first
-#pragma unroll
-                for (int q = 0; q < 3; ++q)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[pa[q]], b[j][pb[q]], acc[i][j], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_s_setprio(0);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();  // nobody reads this step any more
-    }
-    // lane holds C[m = 8 (e / 4) + 4 (lane / 32) + e % 4][n = lane % 32] of every 32 x 32 tile
-    bool odd = false;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4;
-            const float row_back = back[min(m, M - 1)];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int n = n0 + wn + 32 * j + fr;
-                const float v = acc[i][j][e] * b_back * row_back;
-                odd |= (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u;
-                if (m < M && n < N) C[(int64_t)m * N + n] = v;
-            }
-        }
-    // infinities and NaN in A, or numbers of B outside the range that the caller has named: again in plain float32
-    if (!odd) return;
-    for (int t = 0; t < TM * TN * 16; ++t) {
-        const int e = t % 16, j = t / 16 % TN, i = t / 16 / TN;
-        const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
-        if (m >= M || n >= N || (__builtin_bit_cast(uint32_t, C[(int64_t)m * N + n]) & 0x7f800000u) != 0x7f800000u) continue;
-        float v = 0.f;
-        for (int k = k_begin; k < k_end; ++k) v = fmaf(A[(int64_t)m * K + k], B[(int64_t)n * K + k], v);
-        C[(int64_t)m * N + n] = v;
-    }
-}
-
-template <int TM, int TN, int PER_SIMD>
-static int launch_halves(const float* A, const _Float16* parts, int64_t part_stride, const float* back, const float* B, float* C, int M, int N,
-                         int K, int KP, float b_scale, float b_back, int slices, hipStream_t stream) {
-    constexpr int lds = 2 * 64 * (TM + TN) * SG_BK * 2;
-    const int m_tiles = (M + 64 * TM - 1) / (64 * TM), n_tiles = (N + 64 * TN - 1) / (64 * TN);
-    const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
-    if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-    const int steps = (K + SG_BK - 1) / SG_BK, slice = (steps + slices - 1) / slices * SG_BK;
-    gemm_nt_halves_kernel<TM, TN, PER_SIMD><<<dim3((int)blocks, slices), 256, lds, stream>>>(A, parts, part_stride, back, B, C, M, N, K, KP,
-                                                                                          b_scale, b_back, m_tiles, n_tiles, slice);
-    LLE_RETURN_LAUNCH_STATUS();
-}
-
-// The product of lle_gemm_nt_f32 for contiguous operands, A [M][K] and B [N][K], K a multiple of 4.  `parts`: scratch of
-// 2 M KP halves (KP: K up to a multiple of 32), `back`: scratch of M floats.  b_exponent: of B's largest number.
-extern "C" int lle_gemm_nt_f32_halves(const void* A, const void* B, void* C, void* parts, void* back, int b_exponent, int M, int N, int K,
-                                      int slices, int tiles, hipStream_t stream) {
-    if (M <= 0 || N <= 0) return 0;
-    if (K <= 0 || K % 4 != 0 || slices < 1 || slices > 65535 || b_exponent < -100 || b_exponent > 100) return (int)hipErrorInvalidValue;
-    if (tiles < 0) {
-        int unused;
-        choose(halves_tiles, M, N * slices, (K + slices - 1) / slices, 1, tiles, unused);
-    }
-    const int KP = (K + SG_BK - 1) / SG_BK * SG_BK;
-    const int64_t stride = (int64_t)M * KP;
-    const float *a = (const float*)A, *b = (const float*)B, up = ldexpf(1.f, 13 - b_exponent), down = ldexpf(1.f, b_exponent - 13);
-    split_rows_kernel<<<M, 256, 0, stream>>>(a, K, K, KP, (uint32_t*)parts, stride / 2, (float*)back);
-    const _Float16* p = (const _Float16*)parts;
-    switch (tiles) {
-        case 0: return launch_halves<4, 2, 2>(a, p, stride, (const float*)back, b, (float*)C, M, N, K, KP, up, down, slices, stream);
-        case 1: return launch_halves<2, 2, 3>(a, p, stride, (const float*)back, b, (float*)C, M, N, K, KP, up, down, slices, stream);
-        case 2: return launch_halves<2, 1, 4>(a, p, stride, (const float*)back, b, (float*)C, M, N, K, KP, up, down, slices, stream);
-        case 3: return launch_halves<1, 1, 6>(a, p, stride, (const float*)back, b, (float*)C, M, N, K, KP, up, down, slices, stream);
         default: return (int)hipErrorInvalidValue;
     }
 }

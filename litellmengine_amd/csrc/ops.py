@@ -6,7 +6,6 @@ CPU path: without a GPU or without the compiled libraries these raise.
 from __future__ import annotations
 
 import ctypes
-import math
 from typing import Optional
 
 import torch
@@ -297,14 +296,14 @@ class HipOps:
                   _ptr(xw), _ptr(sums), M, N, K)
         return Prenormed(xw, sums, fold.eps)
 
-    def linear(self, x, weight, out_dtype=None, fold=None, sums_ok=False, exponent=None):
+    def linear(self, x, weight, out_dtype=None, fold=None, sums_ok=False):
         """x [M, K] . weight [N, K]^T -> [M, N].  With `sums_ok` the caller takes the result also as
         PartialSums (float32 [slices, M, N], what add_rmsnorm adds into the residual stream).  float32 operands take a
         32-bit product: few rows the weight-streaming kernel (float32 matrix instruction), more rows a tiled kernel
         (operands split exactly into three bfloat16 parts); the plain-FMA kernel where K is no multiple of 4.  bfloat16 operands: few rows take the
         weight-streaming matrix-core kernel, more rows the library product; both
         accumulate in 32-bit and write either result type.  `x` a Prenormed or `fold`
-        a NormFold: see _linear_folded.  `exponent`: what product_exponents says of a float32 weight (None: not known)."""
+        a NormFold: see _linear_folded."""
         if fold is not None or isinstance(x, Prenormed):
             _need(out_dtype in (None, torch.bfloat16) or (fold is None and out_dtype == torch.float32),
                   "a product that makes a folded norm's input writes bfloat16")
@@ -355,11 +354,7 @@ class HipOps:
             return out
         if K % 4 == 0 and not self.force_simt_gemm:
             slices = self._form_of_delta(x.dtype, M, N, K)[1] if sums_ok else 1
-            # (splitting the rows of x is a launch of its own: small weights do not repay it, 513 x 1024 x 2052 49 against 51 us)
-            if exponent is not None and M >= 96 and N * K >= 1 << 22:
-                out = self.linear_f32_halves(x, weight, exponent, slices)
-            else:
-                out = self.linear_f32_tiles(x, weight, slices)
+            out = self.linear_f32_tiles(x, weight, slices)
             return PartialSums(out) if slices > 1 else out[0]
         out = torch.empty((M, N), dtype=out_dtype, device=x.device)
         self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
@@ -428,46 +423,6 @@ class HipOps:
         out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
         self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, slices,
                   tiles)
-        return out
-
-    def weight_bounds(self, weight):
-        """Looks a float32 weight [N, K] over that is laid out for many products: what product_exponents makes its exponent of,
-        on the device; None for a weight that no product in halves takes."""
-        if weight.dtype != torch.float32 or weight.dim() != 2 or weight.numel() < 1 << 22 or weight.shape[1] % 4 != 0:
-            return None
-        _dev(weight, "weight")
-        fn = getattr(build.load_library("gemm_f32"), "lle_weight_bounds_blocks")
-        fn.argtypes, fn.restype = [], _I
-        bounds = torch.empty((int(fn()), 2), dtype=torch.float32, device=weight.device)
-        self._run("gemm_f32", "lle_weight_bounds", [_P, _P, _I, _I, _P], _ptr(weight), _ptr(bounds), weight.shape[0], weight.shape[1])
-        return bounds
-
-    def product_exponents(self, bounds) -> list:
-        """For every weight_bounds in `bounds`: the exponent of the weight's largest number, where every row's largest lies
-        within 2^-13 of it (linear_f32_halves then loses no more than float32 does); else None.  Waits for the device once."""
-        if not bounds:
-            return []
-        all_ = torch.stack(list(bounds))
-        most, least = all_[:, :, 0].view(torch.int32).amax(1).view(torch.float32), all_[:, :, 1].amin(1)
-        out = []
-        for hi, lo in torch.stack([most, least], dim=1).tolist():
-            fine = 2.0 ** -100 < hi < 2.0 ** 100 and lo >= hi * 2.0 ** -13  # (no number among them: not)
-            out.append(math.frexp(hi)[1] - 1 if fine else None)
-        return out
-
-    def linear_f32_halves(self, x, weight, exponent: int, slices: int = 1, tiles: int = -1) -> torch.Tensor:
-        """linear_f32_tiles with both operands split into two half parts instead of three (product_exponents says for which
-        weights): half as many matrix instructions."""
-        _dev(x, "x", torch.float32)
-        _dev(weight, "weight", torch.float32)
-        M, K = x.shape
-        N = weight.shape[0]
-        _need(weight.shape[1] == K and K % 4 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
-        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
-        parts = torch.empty((2, M, -(-K // 32) * 32), dtype=torch.float16, device=x.device)
-        back = torch.empty((M,), dtype=torch.float32, device=x.device)
-        self._run("gemm_f32", "lle_gemm_nt_f32_halves", [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight),
-                  _ptr(out), _ptr(parts), _ptr(back), int(exponent), M, N, K, slices, tiles)
         return out
 
     SLICED_MIN_ROWS, SLICED_MAX_ROWS = 17, 128  # (lle_gemm_mid_slices_max_rows)
@@ -927,7 +882,7 @@ class HipOps:
                   _ptr(gate_up), _ptr(out), N, two_i // 2, dtype_code(gate_up.dtype))
         return out
 
-    def gate_up_silu(self, x, weight, exponent=None) -> torch.Tensor:
+    def gate_up_silu(self, x, weight) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows) -> silu(x gate^T) * (x up^T), [M, I].
         Few rows run as ONE weight-streaming launch with the activation in its epilogue; otherwise the product and
         silu_mul (in float32 also up to 16 rows with more than 2560 columns, which the streaming kernel's gated form does
@@ -950,7 +905,7 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
-        return self.silu_mul(self.linear(x, weight, exponent=exponent))
+        return self.silu_mul(self.linear(x, weight))
 
     def gate_up_clamped(self, x, weight, bias, limit: float) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows), bias [2 I] or None -> [M, I]: with g = min(x gate^T + b,

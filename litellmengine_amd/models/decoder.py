@@ -143,7 +143,6 @@ class DecoderLM:
             self.head.bind_tensor(self.embedding.weight, ctx)
         else:
             raise KeyError(head_name)
-        ctx.settle()
 
     # -- one step --------------------------------------------------------------
     def _injected(self, inject: Inject, delta, step) -> Injected:

@@ -26,17 +26,6 @@ class BuildContext:
     dtype: torch.dtype  # activation/weight type: torch.bfloat16 or torch.float32
     device: torch.device
     ops: Any  # the kernel operations (csrc.ops.HipOps)
-    # float32 projections whose weights have been looked over, and what was seen (on the device): read by settle()
-    looked_over: list = dataclasses.field(default_factory=list, compare=False, repr=False)
-
-    def settle(self) -> None:
-        """Once all weights are bound: hands every projection in `looked_over` what may be said of its weight, waiting for the
-        device once.  (A projection that is bound alone goes without.)"""
-        parts, bounds = [p for p, _ in self.looked_over], [b for _, b in self.looked_over]
-        self.looked_over.clear()
-        if parts:
-            for part, exponent in zip(parts, self.ops.product_exponents(bounds)):
-                part.known = {} if exponent is None else {"exponent": exponent}
 
 
 @dataclasses.dataclass(frozen=True)

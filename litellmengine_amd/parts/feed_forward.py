@@ -60,11 +60,11 @@ class GatedMLP(FeedForward):
     def forward(self, x, fold=None):
         ops = self.ctx.ops
         if self.fused:
-            return self.down.forward(ops.gate_up_silu(x, self.gate_up.weight, **self.gate_up.known), fold=fold)
+            return self.down.forward(ops.gate_up_silu(x, self.gate_up.weight), fold=fold)
         if self.limit is not None:
             a = ops.gate_up_clamped(x, self.gate_up.weight, self.gate_up.bias, self.limit)
         else:
-            a = ops.bias_act(ops.linear(x, self.gate_up.weight, **self.gate_up.known), self.activation, gated=True, bias=self.gate_up.bias)
+            a = ops.bias_act(ops.linear(x, self.gate_up.weight), self.activation, gated=True, bias=self.gate_up.bias)
         y = self.down.forward(a)
         return y if self.late_bias is None else Injected(y, self.late_bias, None, ops)
 
@@ -94,4 +94,4 @@ class PlainMLP(FeedForward):
 
     def forward(self, x, row_gate=None):
         ops = self.ctx.ops
-        return self.down.forward(ops.bias_act(ops.linear(x, self.up.weight, **self.up.known), self.activation, gated=False, row_gate=row_gate))
+        return self.down.forward(ops.bias_act(ops.linear(x, self.up.weight), self.activation, gated=False, row_gate=row_gate))

@@ -30,7 +30,6 @@ class Linear(Part):
             raise ValueError("a bias for every weight tensor, or none")
         self.weight: Optional[torch.Tensor] = None
         self.bias: Optional[torch.Tensor] = None
-        self.known = {}  # what the operations may be told of the weight (float32: its exponent, see BuildContext.settle)
 
     @property
     def has_bias(self) -> bool:
@@ -49,11 +48,6 @@ class Linear(Part):
         self.ctx = ctx
         parts = [weights[n].to(ctx.dtype) for n in self.names]
         self.weight = parts[0].contiguous() if len(parts) == 1 else torch.cat(parts, dim=0).contiguous()
-        self.known = {}
-        if ctx.dtype == torch.float32 and hasattr(ctx.ops, "weight_bounds"):
-            bounds = ctx.ops.weight_bounds(self.weight)
-            if bounds is not None:
-                ctx.looked_over.append((self, bounds))
         if self.bias_names:
             self.bias = torch.cat([weights[n].to(ctx.dtype).reshape(-1) for n in self.bias_names]).contiguous()
 
@@ -69,9 +63,9 @@ class Linear(Part):
         if self.bias is not None:
             if fold is not None:
                 raise ValueError("a projection with a bias cannot add into the residual stream for a folded norm")
-            return ops.add_bias(ops.linear(x, self.weight, out_dtype, **self.known), self.bias)
+            return ops.add_bias(ops.linear(x, self.weight, out_dtype), self.bias)
         if fold is None:
             if self.to_residual and out_dtype is None:
-                return ops.linear(x, self.weight, out_dtype, sums_ok=True, **self.known)
-            return ops.linear(x, self.weight, out_dtype, **self.known)
+                return ops.linear(x, self.weight, out_dtype, sums_ok=True)
+            return ops.linear(x, self.weight, out_dtype)
         return ops.linear(x, self.weight, out_dtype, fold=fold)
