@@ -387,8 +387,9 @@ class HipOps:
 
     def f32_slices_for(self, M: int, N: int, K: int) -> int:
         """In how many slices of K a float32 product is cut whose reader adds up partial sums, so that the CUs have work and no
-        workgroup reads more of x than it has to (the kernel library says how many); 1 for the whole product, and where the
-        reader (add_rmsnorm) takes no partial sums of that width."""
+        workgroup reads more of x than it has to (the kernel library says how many, from N and K: M only decides which
+        of the two kernels it is, so beyond those rows, and up to them, a row's sums do not depend on how many rows there are);
+        1 for the whole product, and where the reader (add_rmsnorm) takes no partial sums of that width."""
         if N > MAX_SUMMED_NORM_WIDTH or N % 4 != 0:
             return 1
         if M <= self.tuning.skinny_f32_max_rows:
@@ -396,8 +397,8 @@ class HipOps:
             fn.argtypes, fn.restype = [_I, _I], _I
             return int(fn(N, K))
         fn = getattr(build.load_library("gemm_f32"), "lle_gemm_nt_f32_slices")
-        fn.argtypes, fn.restype = [_I, _I, _I], _I
-        return int(fn(M, N, K))
+        fn.argtypes, fn.restype = [_I, _I], _I
+        return int(fn(N, K))
 
     def linear_f32_slices(self, x, weight, slices: int) -> torch.Tensor:
         """x [M, K] . weight [N, K]^T, float32, up to 64 rows, as partial sums over `slices` parts of K: [slices, M, N], to be

@@ -127,3 +127,17 @@ def test_all_bits_of_an_operand_count(M):
     x = x / x.abs().amax(1, keepdim=True) * 1e-3
     x[:, 7], w[:, 7] = 1e4, 0.0
     check(projection(w).forward(x), x, w)
+
+
+@pytest.mark.parametrize("N,K", [(1024, 3072), (4096, 4096), (2048, 1028), (1000, 512)])
+def test_a_row_does_not_depend_on_its_step(N, K):
+    """Beyond the few rows that the weight-streaming kernels take, a row's sums are the same to the last bit however many rows
+    there are, also where slices of K are left to the reader."""
+    o = ops()
+    x, w = operands(1100, N, K, seed=10)
+    whole, cut = o.linear(x, w), o.linear(x, w, sums_ok=True)
+    sums = lambda t: t.sums if hasattr(t, "sums") else t[None]
+    for M in (65, 100, 209, 513):
+        part = x[-M:].contiguous()
+        assert torch.equal(o.linear(part, w), whole[-M:]), M
+        assert torch.equal(sums(o.linear(part, w, sums_ok=True)), sums(cut)[:, -M:]), M
