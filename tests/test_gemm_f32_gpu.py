@@ -141,3 +141,33 @@ def test_a_row_does_not_depend_on_its_step(N, K):
         part = x[-M:].contiguous()
         assert torch.equal(o.linear(part, w), whole[-M:]), M
         assert torch.equal(sums(o.linear(part, w, sums_ok=True)), sums(cut)[:, -M:]), M
+
+
+@pytest.mark.parametrize("value", [math.nan, math.inf])
+def test_rows_that_are_no_numbers_are_not_waited_for(value):
+    """One request whose stream is no number any more shares every product with the others: one such row, or all of them, cost
+    no more than the float32 instruction takes for the tiles they are in (measured 2.5 and 2.9 times the product without them;
+    a loop over K for every element took a hundred times as long for 64 such rows)."""
+    o = ops()
+    x, w = operands(512, 4096, 4096, seed=11)
+
+    def seconds(x):
+        best = math.inf
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            o.linear(x, w)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    clean = seconds(x)
+    one, all_ = x.clone(), x.clone()
+    one[77, 5], all_[:, 5] = value, value
+    assert seconds(one) < 4 * clean and seconds(all_) < 12 * clean
+    got, plain = o.linear(one, w), o.linear(x, w)
+    others = torch.arange(512, device="cuda") != 77
+    assert not bool(torch.isfinite(got[77]).any())
+    check(got[others], x[others], w)
+    assert torch.equal(got[:64], plain[:64])  # (rows of other tiles: to the last bit)
