@@ -1269,19 +1269,20 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
                     [&](int n) { return *(const bf16x8*)(vt + v_read + n * 256); }, step * KSTEP, scale_log2,
                     cap_log2);
             }
-            // the loads just issued may stay in flight; the tile before them has landed
+            // the loads just issued may stay in flight; the tile before them has landed, and this one has been read (its
+            // buffer is the next one to be filled)
             if constexpr (LOADS == 2)
-                asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
             else
-                asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
         };
         dma(0);  // tile first_step
         dma(1);  // tile first_step + 1
         if constexpr (LOADS == 2)
-            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
         else
-            asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         for (int step = first_step; step < end_step; step += 3) {
             dma_step(step, 0, 2);

@@ -81,11 +81,11 @@ __global__ __launch_bounds__(WM* WN* LLE_WAVE, 2) void gemm_tile_kernel(const bf
     int buf = 0;
     for (int step = 0; step < steps; ++step) {
         // this stage has landed (what was asked for behind it may stay on its way), for every wavefront; and nobody reads the
-        // buffer of the stage before any more, which the next load takes
+        // buffer of the stage before any more, which the next load takes (lgkmcnt: the reads have arrived, not only been issued)
         if (step + STAGES - 1 <= steps)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
         else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (step + STAGES - 1 < steps) issue(step + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
