@@ -48,8 +48,13 @@ LIBRARIES: Dict[str, List[str]] = {
 HOST_LIBRARIES: Dict[str, List[str]] = {"host": ["host.cpp"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared"]
 HEADERS = ["common.h"]
-# headers that only one library includes
-OWN_HEADERS: Dict[str, List[str]] = {"sampling": ["sampling.h"]}
+# headers that not every library includes
+OWN_HEADERS: Dict[str, List[str]] = {
+    "sampling": ["sampling.h"],
+    "gemm": ["lds.h"],
+    "gemm_f32": ["lds.h"],
+    "gemm_tile": ["lds.h"],
+}
 # packed 32-bit float instructions are switched off on purpose (device flag); the first kernel
 # arguments come preloaded into scalar registers with the dispatch instead of being loaded by the
 # kernel's first instructions (every kernel here is short enough for that to count: measured

@@ -5,6 +5,7 @@
 // depend on what else is in the batch; gemm_f32.hip has the one for many rows), the bfloat16 weight-streaming product of decoding, and its 32-bit twin (32-bit
 // operands through the 32-bit matrix instruction: products and sums in float32).
 #include "common.h"
+#include "lds.h"
 #include <type_traits>
 
 LLE_DEFINE_ERROR_STRING()
@@ -511,13 +512,9 @@ extern "C" int lle_gemm_mid_slices_bf16(const void* X, const void* W, void* out,
         constexpr size_t tiles = (size_t)2 * 16 * T * MID_STAGE * sizeof(bf16_t);                           \
         constexpr size_t sums = (size_t)4 * MID_STEPS * T * 16 * 17 * sizeof(float);                                  \
         constexpr size_t lds = tiles > sums ? tiles : sums;                                                           \
-        static bool ready = false; /* more than 64 KB of LDS has to be asked for once */                              \
-        if (!ready) {                                                                                                 \
-            if (hipFuncSetAttribute((const void*)gemm_mid_slices_kernel<T, B>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                    (int)lds) != hipSuccess)                                                          \
-                return (int)hipGetLastError();                                                                        \
-            ready = true;                                                                                             \
-        }                                                                                                             \
+        static std::atomic<uint64_t> granted{0};                                                                      \
+        const hipError_t e = lle_grant_lds((const void*)gemm_mid_slices_kernel<T, B>, (int)lds, granted);             \
+        if (e != hipSuccess) return (int)e;                                                                           \
         gemm_mid_slices_kernel<T, B><<<grid, 4 * MID_STEPS * LLE_WAVE, lds, stream>>>(                                    \
             (const bf16_t*)X, (const bf16_t*)W, (float*)out, M, N, K, stages);                                        \
     }

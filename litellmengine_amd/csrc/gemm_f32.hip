@@ -5,6 +5,7 @@
 // six products of the bfloat16 matrix instruction, each exact, added up in float32: less is lost than one float32
 // rounding of a b.  The float32 matrix instruction does 157 TFLOP/s, the bfloat16 one 2500, a sixth of which is 417.
 #include "common.h"
+#include "lds.h"
 #include <math.h>
 
 LLE_DEFINE_ERROR_STRING()
@@ -193,12 +194,9 @@ static int launch_split(const float* A, const float* B, float* C, int M, int N, 
                         int slices, hipStream_t stream) {
     constexpr int lds = 3 * 64 * (TM + TN) * SG_BK * 2;
     const int m_tiles = (M + 64 * TM - 1) / (64 * TM), n_tiles = (N + 64 * TN - 1) / (64 * TN);
-    static bool ready = false;  // more than 64 KB of LDS has to be asked for once
-    if (!ready) {
-        if (hipFuncSetAttribute((const void*)gemm_nt_split_kernel<TM, TN, PER_SIMD>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-            return (int)hipGetLastError();
-        ready = true;
-    }
+    static std::atomic<uint64_t> granted{0};
+    const hipError_t e = lle_grant_lds((const void*)gemm_nt_split_kernel<TM, TN, PER_SIMD>, lds, granted);
+    if (e != hipSuccess) return (int)e;
     const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
     const int steps = (K + SG_BK - 1) / SG_BK, slice = (steps + slices - 1) / slices * SG_BK;

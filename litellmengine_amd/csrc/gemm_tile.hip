@@ -11,6 +11,7 @@
 // (256 x 256 tiles: 5120 x 8192 at 400 rows 92 us against 63 in 256 x 128.)
 // For whole products (gate_up, qkv) the library's tiles are as fast or faster.
 #include "common.h"
+#include "lds.h"
 #include <math.h>
 
 LLE_DEFINE_ERROR_STRING()
@@ -129,11 +130,9 @@ static int launch_tile(const void* X, const void* W, void* C, int M, int N, int 
     static_assert(lds <= 160 * 1024, "the LDS of a CU");
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     auto kernel = gemm_tile_kernel<WM, WN, TM, TN, STAGES>;
-    static bool ready = false;  // more than 64 KB of LDS has to be asked for once
-    if (!ready) {
-        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return (int)hipGetLastError();
-        ready = true;
-    }
+    static std::atomic<uint64_t> granted{0};
+    const hipError_t e = lle_grant_lds((const void*)kernel, lds, granted);
+    if (e != hipSuccess) return (int)e;
     const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
     kernel<<<dim3((int)blocks, slices), WM * WN * LLE_WAVE, lds, stream>>>((const bf16_t*)X, (const bf16_t*)W, (float*)C, M, N, K, m_tiles, n_tiles,

@@ -2,6 +2,7 @@
 import glob
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -26,3 +27,35 @@ def test_bare_barriers_wait_for_lds(path):
         waits = [w for w in before if "s_waitcnt" in w or "fence" in w]
         assert waits, f"{os.path.basename(path)}: {lines[at]} / {line}"
         assert all("lgkmcnt(0)" in w or "fence" in w for w in waits), (os.path.basename(path), waits)
+
+
+def test_lds_is_asked_for_on_every_device(tmp_path):
+    """A kernel that takes more than 64 KB of LDS asks for it once on each device of the process, and again after a refusal."""
+    source = tmp_path / "grant.cpp"
+    source.write_text(r'''
+#include "lds.h"
+static int device = 0, asked = 0;
+static hipError_t answer = hipSuccess;
+extern "C" hipError_t hipGetDevice(int* d) { return *d = device, hipSuccess; }
+extern "C" hipError_t hipGetLastError() { return answer; }
+extern "C" hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return ++asked, answer; }
+int main() {
+    std::atomic<uint64_t> one{0}, other{0};
+    auto launch = [&](int on, std::atomic<uint64_t>& kernel, hipError_t says = hipSuccess) {
+        device = on, asked = 0, answer = says;
+        return lle_grant_lds(nullptr, 1 << 17, kernel) != says ? -1 : asked;
+    };
+    const int got[] = {launch(0, one), launch(0, one), launch(1, one), launch(63, one), launch(64, one), launch(64, one), launch(1, one),
+                       launch(0, other, hipErrorInvalidValue), launch(0, other), launch(0, other)};
+    const int want[] = {1, 0, 1, 1, 1, 1, 0, 1, 1, 0};
+    for (int i = 0; i < 10; ++i)
+        if (got[i] != want[i]) return i + 1;
+    return 0;
+}
+''')
+    rocm = os.path.dirname(os.path.dirname(build._hipcc()))
+    program = tmp_path / "grant"
+    subprocess.run([build._host_compiler(), "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                    f"-I{os.path.dirname(build.__file__)}", str(source), "-o", str(program)], check=True)
+    assert subprocess.run([str(program)]).returncode == 0
+    assert not [p for p in SOURCES if re.search(r"static bool \w+ =", open(p).read())]  # (asked for once a process)
