@@ -112,7 +112,21 @@ template <> struct SkOp<float> {
     }
 };
 #define SK_KSTEP 64  // elements of a bfloat16 step
-template <typename T> constexpr int sk_step = 8 * SkOp<T>::E;  // elements of a step
+// How the wavefronts share the columns of a row, in rounds of 128 bytes a wavefront, each lane two pieces of 16 bytes a round:
+// bfloat16 wavefronts take 128 bytes in a row, a lane's pieces side by side; float32 ones 64 bytes of each half of the round,
+// as gemm_skinny_f32_kernel does: which of the float32 kernels takes a product follows the number of rows, and a row's sums must
+// not.  (The other way round that kernel is slower with few rows: 6144 x 4096 at 1 row 21 us, with 128 bytes in a row 26.
+// The streaming kernel, 128 bytes in a row against so: 24576 x 4096 at 1 / 16 rows 79 / 83 against 75 / 81 us, gated 6144 x 1024
+// at 32 rows 11.0 against 10.3, gated 12288 x 2048 at 8 rows 22.5 against 24.7, 151936 x 1024 at 32 rows 123 against 138.)
+template <typename T, int WAVES = 16> struct SkShare {
+    static constexpr bool HALVES = std::is_same<T, float>::value;
+    static constexpr int E = SkOp<T>::E;
+    static constexpr int ROUND = 8 * E * WAVES;               // elements of a round
+    static constexpr int WAVE = HALVES ? 4 * E : 8 * E;       // from a wavefront's first element to the next one's
+    static constexpr int LANE = HALVES ? E : 2 * E;           // from lane group c to c + 1
+    static constexpr int SECOND = HALVES ? ROUND / 2 : E;     // from a lane's first piece to its second
+    static constexpr int EXTENT = HALVES ? SECOND + WAVE : WAVE;  // from a wavefront's first element to behind its last of a round
+};
 
 // GATED: W holds gate rows [0, N/2) and then up rows [N/2, N); a workgroup takes 16 gate rows
 // and the 16 up rows that go with them (NT = 2) and writes silu(gate) * up, C is [M, N/2].
@@ -162,7 +176,8 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                                                                          TC* __restrict__ C, int M, int N, int K,
                                                                          int tile_rows, NormFold fold) {
     using Vec = typename SkOp<T>::vec;
-    constexpr int E = SkOp<T>::E, STEP = sk_step<T>;
+    using Share = SkShare<T, SK_WAVES>;
+    constexpr int E = SkOp<T>::E, SECOND = Share::SECOND;
     static_assert(!(RESID || SCALED) || MT <= 2, "the norm is folded for up to 32 rows");
     // `tile_rows` (at most 16) rows of W per tile: fewer than 16 where that makes the number of tiles a
     // multiple of the number of CUs (see skinny_tile_rows); the lanes past them read the tile's last
@@ -216,12 +231,12 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
         const int rt = min(r16, tile_rows - 1);  // the lane's row of the tile
         const int64_t wrow = GATED ? min(n0 + rt, (int64_t)N / 2 - 1) + nt * ((int64_t)N / 2)
                                    : min(n0 + (NT == 1 ? rt : 16 * nt + r16), (int64_t)N - 1);
-        wp[nt] = W + wrow * K + 2 * E * c;
+        wp[nt] = W + wrow * K + Share::LANE * c;
     }
     // rows of X beyond M are never written back, so their lanes may read any valid row
     const T* xp[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xp[mt] = X + (int64_t)min(16 * mt + r16, M - 1) * K + 2 * E * c;
+    for (int mt = 0; mt < MT; ++mt) xp[mt] = X + (int64_t)min(16 * mt + r16, M - 1) * K + Share::LANE * c;
     gf32x4 acc[NT][MT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -229,23 +244,22 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
     const Vec zero = {};
 
-    const int full_steps = K / STEP;
-    int ss = wave;
-    // UNROLL steps at a time: all their loads are issued before the first product
-    for (; ss + (UNROLL - 1) * SK_WAVES < full_steps; ss += UNROLL * SK_WAVES) {
+    int kw = wave * Share::WAVE;
+    // UNROLL rounds at a time: all their loads are issued before the first product
+    for (; kw + (UNROLL - 1) * Share::ROUND + Share::EXTENT <= K; kw += UNROLL * Share::ROUND) {
         Vec w0[UNROLL][NT], w1[UNROLL][NT], x0[UNROLL][MT], x1[UNROLL][MT];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            const int k0 = (ss + u * SK_WAVES) * STEP;
+            const int k0 = kw + u * Share::ROUND;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 w0[u][nt] = *(const Vec*)(wp[nt] + k0);
-                w1[u][nt] = *(const Vec*)(wp[nt] + k0 + E);
+                w1[u][nt] = *(const Vec*)(wp[nt] + k0 + SECOND);
             }
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 x0[u][mt] = *(const Vec*)(xp[mt] + k0);
-                x1[u][mt] = *(const Vec*)(xp[mt] + k0 + E);
+                x1[u][mt] = *(const Vec*)(xp[mt] + k0 + SECOND);
             }
         }
 #pragma unroll
@@ -258,22 +272,21 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                     acc[nt][mt] = SkOp<T>::mma(w1[u][nt], x1[u][mt], acc[nt][mt]);
                 }
     }
-    // what is left of K: single steps; the last one may be partial (K is a multiple of E),
+    // what is left of K: single rounds; the last one may be partial (K is a multiple of E),
     // and there both operands are zeroed beyond K so that nothing outside the matrices is read
-    const int all_steps = (K + STEP - 1) / STEP;
-    for (; ss < all_steps; ss += SK_WAVES) {
-        const int k0 = ss * STEP;
-        const bool in0 = k0 + 2 * E * c + E <= K, in1 = k0 + 2 * E * c + 2 * E <= K;
+    for (; kw < K; kw += Share::ROUND) {
+        const int k0 = kw;
+        const bool in0 = k0 + Share::LANE * c + E <= K, in1 = k0 + SECOND + Share::LANE * c + E <= K;
         Vec x0[MT], x1[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             x0[mt] = in0 ? *(const Vec*)(xp[mt] + k0) : zero;
-            x1[mt] = in1 ? *(const Vec*)(xp[mt] + k0 + E) : zero;
+            x1[mt] = in1 ? *(const Vec*)(xp[mt] + k0 + SECOND) : zero;
         }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const Vec w0 = in0 ? *(const Vec*)(wp[nt] + k0) : zero;
-            const Vec w1 = in1 ? *(const Vec*)(wp[nt] + k0 + E) : zero;
+            const Vec w1 = in1 ? *(const Vec*)(wp[nt] + k0 + SECOND) : zero;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 acc[nt][mt] = SkOp<T>::mma(w0, x0[mt], acc[nt][mt]);
@@ -557,8 +570,8 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
                                                                               TC* __restrict__ C, int M, int N, int K,
                                                                               int share, NormFold fold) {
     using Vec = typename SkOp<T>::vec;
-    constexpr int E = SkOp<T>::E, STEP = sk_step<T>;
     constexpr int WAVES = 16;
+    using Share = SkShare<T, WAVES>;
     constexpr int NT = GATED ? 2 : 1;
     constexpr int SS = (XS % 2 == 0 && XS <= 6) ? 2 : 1;  // steps of a set (one where X takes most of the registers)
     // sets of W operands: one is multiplied, the others are on their way (single steps of float32: four)
@@ -585,18 +598,18 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
     auto aim = [&]() {
         const int t = min(load_tile, tiles - 1);
         const int row = max(0, min(tile_begin(t) + r16, tile_end(t) - 1));  // a tile without rows reads rows that are there
-        wp = W + (int64_t)row * K + 2 * E * c + wave * STEP;
+        wp = W + (int64_t)row * K + Share::LANE * c + wave * Share::WAVE;
     };
     auto load = [&](Set& set) {
 #pragma unroll
         for (int i = 0; i < SS; ++i) {
-            const T* g = wp + (load_step + i) * (WAVES * STEP);
+            const T* g = wp + (load_step + i) * Share::ROUND;
             set.g0[i] = *(const Vec*)g;
-            set.g1[i] = *(const Vec*)(g + E);
+            set.g1[i] = *(const Vec*)(g + Share::SECOND);
             if (GATED) {
                 const T* u = g + (int64_t)rows * K;
                 set.u0[i] = *(const Vec*)u;
-                set.u1[i] = *(const Vec*)(u + E);
+                set.u1[i] = *(const Vec*)(u + Share::SECOND);
             }
         }
         load_step += SS;
@@ -614,11 +627,11 @@ __global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(co
     Vec x0[MT][XS], x1[MT][XS];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        const T* xp = X + (int64_t)min(16 * mt + r16, M - 1) * K + 2 * E * c + wave * STEP;
+        const T* xp = X + (int64_t)min(16 * mt + r16, M - 1) * K + Share::LANE * c + wave * Share::WAVE;
 #pragma unroll
         for (int j = 0; j < XS; ++j) {
-            x0[mt][j] = *(const Vec*)(xp + j * (WAVES * STEP));
-            x1[mt][j] = *(const Vec*)(xp + j * (WAVES * STEP) + E);
+            x0[mt][j] = *(const Vec*)(xp + j * Share::ROUND);
+            x1[mt][j] = *(const Vec*)(xp + j * Share::ROUND + Share::SECOND);
         }
     }
     if (SCALED) {
@@ -753,8 +766,8 @@ static int gemm_compute_units() {
 template <typename T, bool GATED, bool SCALED, typename TC>
 static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, int K,
                                  const NormFold& fold, hipStream_t stream) {
-    constexpr int STEP = sk_step<T>;
-    if (M > 32 || K % (STEP * 16) != 0) return false;
+    constexpr int ROUND = SkShare<T>::ROUND;
+    if (M > 32 || K % ROUND != 0) return false;
     const int rows = GATED ? N / 2 : N;
     const int units = gemm_compute_units();
     const int share = (rows + units - 1) / units;
@@ -764,20 +777,20 @@ static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, in
     if (std::is_same<T, float>::value && share <= 32 && M <= 4) return false;
     const int blocks = (rows + share - 1) / share;
     if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
-        if (K == STEP * 16) {
+        if (K == ROUND) {
             gemm_skinny_stream_kernel<T, GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
             return true;
         }
-        if (K == 2 * STEP * 16) {
+        if (K == 2 * ROUND) {
             gemm_skinny_stream_kernel<T, GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
             return true;
         }
         if constexpr (!GATED) {
-            if (K == 3 * STEP * 16) {
+            if (K == 3 * ROUND) {
                 gemm_skinny_stream_kernel<T, GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
                 return true;
             }
-            if (K == 4 * STEP * 16) {
+            if (K == 4 * ROUND) {
                 gemm_skinny_stream_kernel<T, GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
                 return true;
             }
@@ -789,7 +802,7 @@ static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, in
         gemm_skinny_stream_kernel<T, GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
                                                                                                fold);                \
         return true;
-    switch (K / (STEP * 16)) {
+    switch (K / ROUND) {
         LLE_STREAM_CASE(1)
         LLE_STREAM_CASE(2)
         LLE_STREAM_CASE(3)
@@ -798,7 +811,7 @@ static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, in
         case 6:
         case 8:
             if constexpr (!GATED) {  // the gated form's two tiles leave no registers for this much of X
-                if (K / (STEP * 16) == 6) {
+                if (K / ROUND == 6) {
                     gemm_skinny_stream_kernel<T, GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
                                                                                                           share, fold);
                 } else {

@@ -171,3 +171,19 @@ def test_rows_that_are_no_numbers_are_not_waited_for(value):
     assert not bool(torch.isfinite(got[77]).any())
     check(got[others], x[others], w)
     assert torch.equal(got[:64], plain[:64])  # (rows of other tiles: to the last bit)
+
+
+@pytest.mark.parametrize("few", [False, True])
+@pytest.mark.parametrize("K", [20, 512, 520, 1024, 1300, 2560, 3072, 4096])
+def test_a_decoded_row_does_not_depend_on_the_batch(K, few):
+    """Up to 64 rows: streamed or not, gated in one launch or in two, a row's sums are the same to the last bit."""
+    o = ops()
+    N = 500 if few else 2 * (17 * o.compute_units() + 5)
+    x, w = operands(64, N, K, seed=12)
+    x = x / x.abs().max()
+    want = o.linear(x, w)
+    check(want, x, w)
+    gated = o.silu_mul(want)
+    for M in (1, 4, 5, 16, 17, 32, 33, 63):
+        assert torch.equal(o.linear(x[:M].contiguous(), w), want[:M]), M
+        assert torch.equal(o.gate_up_silu(x[:M].contiguous(), w), gated[:M]), M
