@@ -25,11 +25,11 @@ typedef float tf32x16 __attribute__((ext_vector_type(16)));
 #define TILE_SWIZZLE(r) ((((r) >> 1) & 1) | ((((r) >> 3) & 3) << 1))
 
 // WM x WN wavefronts of TM x TN matrix tiles of 32 x 32; STAGES buffers of LDS, STAGES - 1 of them on their way.
-// The float32 sums of slice blockIdx.y of K go to C + blockIdx.y * M * N.
+// The float32 sums of a slice of K go to C + slice * M * N.
 template <int WM, int WN, int TM, int TN, int STAGES>
 __global__ __launch_bounds__(WM* WN* LLE_WAVE, 2) void gemm_tile_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                                                float* __restrict__ C, int M, int N, int K, int m_tiles,
-                                                                               int n_tiles, int slice_stages) {
+                                                                               int n_tiles, int slices, int slice_stages) {
     constexpr int WAVES = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
     constexpr int PIECES = BK / 8, ROW = BK * 2;  // 16-byte pieces of a row of a stage; its bytes
     constexpr int RPL = 64 / PIECES;         // rows that one wavefront's load brings
@@ -39,11 +39,14 @@ __global__ __launch_bounds__(WM* WN* LLE_WAVE, 2) void gemm_tile_kernel(const bf
     static_assert(GROUPS % WAVES == 0 && BM % RPL == 0, "every wavefront loads as much");
     extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    // consecutive workgroups go to different dies: a die takes every eighth part of W (a column of tiles in a slice of K), all
+    // its row tiles one after the other
     const int die = blockIdx.x % 8, at = blockIdx.x / 8;
-    const int nt = die + 8 * (at / m_tiles), mt = at % m_tiles;
-    if (nt >= n_tiles) return;
+    const int part = die + 8 * (at / m_tiles), mt = at % m_tiles;
+    if (part >= n_tiles * slices) return;
+    const int nt = part % n_tiles, slice = part / n_tiles;
     const int m0 = mt * BM, n0 = nt * BN;
-    const int first = blockIdx.y * slice_stages, steps = min(K / BK - first, slice_stages);
+    const int first = slice * slice_stages, steps = min(K / BK - first, slice_stages);
     const bf16_t* xb = X + (int64_t)m0 * K + first * BK;
     const bf16_t* wb = W + (int64_t)n0 * K + first * BK;
     // a load: eight rows of 128 bytes; lane -> row lane / 8, physical piece lane % 8, the logical piece that belongs there
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(WM* WN* LLE_WAVE, 2) void gemm_tile_kernel(const bf
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int n = n0 + wn + 32 * j + fr;
-                if (n < N) C[((int64_t)blockIdx.y * M + m) * N + n] = acc[i][j][e];
+                if (n < N) C[((int64_t)slice * M + m) * N + n] = acc[i][j][e];
             }
         }
 }
@@ -133,10 +136,10 @@ static int launch_tile(const void* X, const void* W, void* C, int M, int N, int 
     static std::atomic<uint64_t> granted{0};
     const hipError_t e = lle_grant_lds((const void*)kernel, lds, granted);
     if (e != hipSuccess) return (int)e;
-    const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
+    const int64_t blocks = (int64_t)8 * m_tiles * (((int64_t)n_tiles * slices + 7) / 8);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-    kernel<<<dim3((int)blocks, slices), WM * WN * LLE_WAVE, lds, stream>>>((const bf16_t*)X, (const bf16_t*)W, (float*)C, M, N, K, m_tiles, n_tiles,
-                                                                           (K / BK + slices - 1) / slices);
+    kernel<<<(int)blocks, WM * WN * LLE_WAVE, lds, stream>>>((const bf16_t*)X, (const bf16_t*)W, (float*)C, M, N, K, m_tiles, n_tiles, slices,
+                                                             (K / BK + slices - 1) / slices);
     LLE_RETURN_LAUNCH_STATUS();
 }
 
@@ -155,21 +158,25 @@ static int units_of_device() {
     return units[dev];
 }
 
-// The tiles and the slices of K that take the least time: rounds of workgroups over the CUs, each with a start of 3 us and its
-// operands at the shape's rate, but not less than W's way from memory (5.2 TB/s into all CUs); the sums' way to their reader and back
-// (5 TB/s), who asks for a slice after the other.
+// The tiles and the slices of K that take the least time: rounds of workgroups over the CUs of the die that gets most of them (a
+// die has whole parts of W, see the kernel: 28 columns of tiles in 3 slices are 11 parts for four dies, 33 workgroups of 129
+// rows in tiles of 64 for 32 CUs), each with a start of 3 us and its operands at the shape's rate, but not less than W's way from
+// memory (5.2 TB/s into all CUs); the sums' way to their reader and back (5 TB/s), who asks for a slice after the other.
+// Measured at 17 to 2048 rows of 73 weights from 512 x 1024 to 8192 x 16384, the choice is 1.6 % slower than the best of
+// all tiles and slices, over 10 % in 3 of 100 (with rounds over all CUs alike 3 %, and 8 of 100).
 static void choose(int M, int N, int K, int first, int last, int& tiles, int& slices) {
-    const int units = units_of_device(), stages = K / BK;
+    constexpr int DIES = 8;
+    const int units = units_of_device(), per_die = units >= DIES ? units / DIES : 1, stages = K / BK;
     const float from_memory = (float)N * K * 2 / 5.2e6f;
     float best = 0.f;
     tiles = 0, slices = first;
     for (int s = first; s <= last && s <= stages; ++s)
         for (int t = 0; t < 3; ++t) {
             const TileShape& v = tile_shapes[t];
-            const int64_t count = (int64_t)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * s;
-            const int64_t rounds = (count + units - 1) / units;
+            const int64_t m_tiles = (M + v.bm - 1) / v.bm, parts = (int64_t)((N + v.bn - 1) / v.bn) * s;
+            const int64_t rounds = ((parts + DIES - 1) / DIES * m_tiles + per_die - 1) / per_die;
             const float each = (float)((stages + s - 1) / s) * (v.bm + v.bn) * BK * 2 / (v.intake * 1e3f);
-            const float memory = from_memory * (float)(rounds * units) / count;  // (CUs without a tile take in nothing)
+            const float memory = from_memory * (float)(rounds * units) / (parts * m_tiles);  // (CUs without a tile take in nothing)
             const float us = fmaxf(rounds * (3.f + each), memory) + (float)s * M * N * 8 / 5e6f + 0.15f * s;
             if (best == 0.f || us < best) best = us, tiles = t, slices = s;
         }

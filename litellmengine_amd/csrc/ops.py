@@ -467,20 +467,29 @@ class HipOps:
     def tile_slices_for(self, M: int, N: int, K: int) -> int:
         """In how many slices of K the tiled product takes a delta of the residual stream (linear_tile_sums), or 0 where another
         form stays.  It is taken where the whole product has too few tiles for the CUs and neither the sliced kernel of up to
-        128 rows nor the library's batched slices have better ones (measured with the norm, old -> new in us): up to 32 rows
-        weights that the sliced kernel does not take (5120 x 8192 31.0 -> 26.9) and large ones (5120 x 25600 68 -> 56); up to 128
-        rows also K >= 2 N (4096 x 12288 at 96 rows 40.4 -> 32.7; 4096 x 4096 gains nothing); beyond, square weights (4096 x 4096
-        at 160 / 512 rows 33.5 -> 23.4 / 37.7 -> 35.5, 5120 x 8192 57.8 -> 38.7 / 78 -> 64; at 700 rows 41.8 -> 47.8, not taken) and
-        the narrow ones of small models (1024 x 2048 at 1000 rows 24.1 -> 17.0)."""
+        128 rows nor the library's batched slices have better ones.  Measured with the norm at 17 to 2048 rows of 73
+        weights, 512 to 8192 wide, other form -> this one in us:
+        * up to 32 rows weights that the sliced kernel does not take (5120 x 8192 31.0 -> 26.9; at most 8 % slower, 3072 x 2048
+          at 17 rows 11.3 -> 12.3) and large ones (5120 x 25600 68 -> 56); up to 128 rows also K >= 2 N (4096 x 12288 at 96 rows
+          40.4 -> 32.7; 4096 x 4096 gains nothing);
+        * beyond, weights of small models (1024 x 2048 at 1000 rows 24.1 -> 17.0); over 512 rows the library's four slices are
+          better for long K (1024 x 4096 at 1536 rows 27.9 -> 32.1, not taken; 1024 x 3072 25.6 -> 27.5 there, at 600 and 2048
+          18.8 -> 16.6 and 32.6 -> 30.9; 512 x 2048 at 1536 rows 0.77 of it);
+        * others with K < 2 N up to 256 rows (4096 x 4096 at 160 rows 33.5 -> 23.4, 5120 x 8192 57.8 -> 38.7), and up to 512 rows
+          where 128 x 128 tiles of the whole product leave a third of the CUs without work (4096 x 4096 at 512 rows 37.7 ->
+          35.5, 5120 x 8192 78 -> 64; 6144 x 4096 at 400 rows, three quarters, 43.2 -> 49.6, not taken) and K is long enough for
+          slices (5120 x 2048 at 512 rows 29.6 -> 32.4, not taken)."""
         if K % 64 != 0 or N % 4 != 0 or N > MAX_SUMMED_NORM_WIDTH or self.force_library_gemm or N * K < 1 << 20:
             return 0
         if M <= 32:
             taken = M > 16 and (N * K >= 1 << 26 or self.slices_for(M, N, K) == 0)
         elif M <= 128:
             taken = K >= 2 * N or self.slices_for(M, N, K) == 0
+        elif N <= 1024 and N * K <= 1 << 22:
+            taken = M <= 512 or (M <= 2048 and (K <= 3 * N or N * K <= 1 << 20))
         else:
-            narrow = N <= 1024 and N * K <= 1 << 22
-            taken = M <= 2048 and (narrow or (K < 2 * N and (M <= 256 or (M <= 512 and N >= 4096))))
+            whole_tiles = -(-M // 128) * -(-N // 128)
+            taken = K < 2 * N and (M <= 256 or (M <= 512 and 3 * whole_tiles <= 2 * self.compute_units() and 4 * K >= 3 * N))
         if not taken:
             return 0
         fn = getattr(build.load_library("gemm_tile"), "lle_gemm_tile_sums_slices")

@@ -42,6 +42,12 @@ def test_which_products_take_it():
     assert not took(96, 4096, 4096) and took(129, 4096, 4096) and took(512, 4096, 4096) and not took(513, 4096, 4096)
     assert took(17, 5120, 25600) and took(17, 5120, 8192) and took(2048, 1024, 2048) and not took(2049, 1024, 2048)
     assert not took(96, 4096, 12288 + 32) and not took(96, 8196, 32768) and not took(96, 64, 128)
+    # the library's tiles fill the CUs, or its slices of K are better (measured 6 to 24 % faster)
+    for m, n, k in ((400, 6144, 4096), (330, 8192, 8192), (512, 5120, 2048), (1536, 1024, 4096), (2048, 768, 4096)):
+        assert not took(m, n, k), (m, n, k)
+    assert took(512, 5120, 8192) and took(330, 4096, 4096) and took(1536, 512, 2048) and took(2048, 1024, 3072)
+    # in 3 slices and tiles of 64 rows a die would get 33 workgroups for its 32 CUs
+    assert o.tile_slices_for(129, 3584, 3584) != 3
     x, w = torch.randn(200, 4096, device="cuda").bfloat16(), torch.randn(4096, 4096, device="cuda").bfloat16()
     cut = o.linear(x, w, sums_ok=True)
     assert isinstance(cut, PartialSums) and o.linear(x, w).shape == (200, 4096)
