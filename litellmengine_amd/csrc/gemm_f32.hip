@@ -373,13 +373,16 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_slices_f32_kernel(const fl
     }
 }
 
-// In how many slices of K the product of up to 64 rows is taken: as many workgroups of 64 rows of B as there are CUs, a step
-// for every wavefront at least; 1 where the rows of B alone occupy the CUs.
+// In how many slices of K the product of up to 64 rows is taken: as many workgroups of 64 rows of B as there are CUs, six steps
+// for the four wavefronts of a row group at least; 1 where the rows of B alone occupy the CUs, and where K is so short that the
+// sums' way to the norm and back costs what the slices gain.  Product and norm, whole / in slices of four steps / so, at 1, 8
+// and 32 rows: 512 x 512 5.4, 5.8, 7.1 / 6.7, 7.9, 10.5 us / whole; 512 x 1024 5.8, 6.6, 9.3 / 6.6, 7.5, 10.1 / whole; 1024 x 2048
+// 8.3, 9.4, 14.4 / 8.4, 9.3, 12.5 / 7.8, 8.8, 11.4; 1024 x 3072 10.4, 11.3, 18.9 in 16 slices 8.4, 9.3, 12.4.
 extern "C" int lle_gemm_slices_f32_count(int N, int K) {
-    if (N <= 0 || K <= 0) return 1;
+    if (N <= 0 || K < 1536) return 1;
     const int groups = (N + FS_ROWS - 1) / FS_ROWS, steps = (K + FS_STEP - 1) / FS_STEP;
     int slices = units_of_device() / groups;
-    if (slices > steps / FS_KW) slices = steps / FS_KW;
+    if (slices > steps / 6) slices = steps / 6;
     if (slices < 2) return 1;
     const int each = (steps + slices - 1) / slices;
     return (steps + each - 1) / each;  // (none of them empty)
