@@ -173,6 +173,19 @@ def test_rows_that_are_no_numbers_are_not_waited_for(value):
     assert torch.equal(got[:64], plain[:64])  # (rows of other tiles: to the last bit)
 
 
+@pytest.mark.parametrize("tiles", TILES)
+@pytest.mark.parametrize("slices", [1, 2])
+def test_rows_beside_one_that_is_no_number_keep_their_bits(tiles, slices):
+    """Also those of the same matrix tile, which is made again."""
+    x, w = operands(300, 192, 260, seed=13)
+    odd = x.clone()
+    odd[77, 5], odd[200, 100], odd[299, 259] = math.nan, math.inf, -math.inf
+    got, plain = (ops().linear_f32_tiles(t, w, slices=slices, tiles=tiles) for t in (odd, x))
+    fine = got.isfinite()
+    assert int((~fine).sum()) == 3 * 192 and not bool(fine[:, [77, 200, 299]].all(0).any())
+    assert torch.equal(got[fine], plain[fine])
+
+
 @pytest.mark.parametrize("few", [False, True])
 @pytest.mark.parametrize("K", [20, 512, 520, 1024, 1300, 2560, 3072, 4096])
 def test_a_decoded_row_does_not_depend_on_the_batch(K, few):
