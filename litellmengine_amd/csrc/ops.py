@@ -895,8 +895,7 @@ class HipOps:
     def gate_up_silu(self, x, weight) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows) -> silu(x gate^T) * (x up^T), [M, I].
         Few rows run as ONE weight-streaming launch with the activation in its epilogue; otherwise the product and
-        silu_mul (in float32 also up to 16 rows with more than 2560 columns, which the streaming kernel's gated form does
-        not hold: 24576 x 4096 at 8 rows 83.6 + 5 against 93.4 us in one launch, at 32 rows 153 + 5 against 122)."""
+        silu_mul (in float32 also where _gated_f32_in_one says so)."""
         if isinstance(x, Prenormed):
             return self._linear_folded(x, weight, None, gated=True)
         _dev(x, "x")
@@ -910,12 +909,25 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_bf16", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
-        if x.dtype == torch.float32 and M <= 32 and K % 4 == 0 and (M > 16 or 16 < K <= 2560) and not self.force_library_gemm:
+        if x.dtype == torch.float32 and K % 4 == 0 and self._gated_f32_in_one(M, N2, K) and not self.force_library_gemm:
             out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
         return self.silu_mul(self.linear(x, weight))
+
+    def _gated_f32_in_one(self, M: int, N2: int, K: int) -> bool:
+        """Whether the float32 product of gate and up and its activation are one launch (the same sums either way).  Not
+        * over 32 rows, and up to 16 rows with more than 2560 columns, which the streaming kernel's gated form does not hold
+          (24576 x 4096 at 8 rows 83.6 + 5 against 93.4 us in one launch, at 32 rows 153 + 5 against 122);
+        * where the plain product's tiles of 16 rows are one for a CU at most: a gated one is two of them, so half of the CUs have
+          work or all of them low tiles, which costs more than a launch saves but for short rows and 9 to 16 rows of x (in two
+          launches / in one at 1, 8, 16 and 17 rows: 4096 x 1024 7.9, 8.4, 8.9, 9.5 / 6.4, 6.6, 7.3, 9.2 us; 2048 x 1536 7.9, 8.3,
+          9.4, 10.7 / 8.3, 8.9, 9.0, 12.5; 4096 x 2560 13.9, 15.8, 18.1, 19.2 / 15.0, 15.1, 17.3, 21.4; 4096 x 4096 at 17 rows
+          26.0 / 30.4; 5120 x 1536, over one round of tiles, 13.1, 13.4, 15.1, 18.0 / 10.3, 10.8, 11.8, 14.6)."""
+        if M > 32 or (M <= 16 and not 16 < K <= 2560):
+            return False
+        return K <= 1024 or N2 > 16 * self.compute_units() or 8 < M <= 16
 
     def gate_up_clamped(self, x, weight, bias, limit: float) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows), bias [2 I] or None -> [M, I]: with g = min(x gate^T + b,

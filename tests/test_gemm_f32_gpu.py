@@ -209,3 +209,20 @@ def test_short_products_are_not_cut():
         assert o.f32_slices_for(32, N, K) == 1, (N, K)
     if o.compute_units() == 256:
         assert o.f32_slices_for(1, 1024, 2048) == 10 and o.f32_slices_for(64, 1024, 3072) == 16 and o.f32_slices_for(8, 4096, 12288) == 4
+
+
+@pytest.mark.parametrize("M,N2,K,one", [(1, 2048, 1024, True), (32, 4096, 1024, True), (8, 4096, 1028, False), (9, 4096, 1028, True),
+                                        (16, 2048, 2560, True), (17, 2048, 2560, False), (1, 2048, 2560, False), (17, 4096, 4096, False),
+                                        (1, 4104, 2048, True), (17, 4104, 4096, True), (8, 8192, 4096, False), (33, 4104, 512, False)])
+def test_gate_and_up_in_one_launch_or_two(monkeypatch, M, N2, K, one):
+    """One where that is faster (4096 x 2048 at 17 rows took 14.8 us in two, 17.2 in one), and the same bits."""
+    o = ops()
+    if o.compute_units() != 256:
+        pytest.skip("the choice follows the number of CUs")
+    x, w = operands(M, N2, K, seed=14)
+    x = x / x.abs().max()
+    launched, run = [], o._run
+    monkeypatch.setattr(o, "_run", lambda lib, name, *a: (launched.append(name), run(lib, name, *a))[1])
+    got = o.gate_up_silu(x, w)
+    assert len(launched) == (1 if one else 2), launched
+    assert torch.equal(got, o.silu_mul(o.linear(x, w)))
