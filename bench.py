@@ -54,9 +54,9 @@ SIZES_32B = dict(
 )
 REFERENCE_TOK_S = 189.06  # readme.md:66: 32 requests x 64 new tokens, paged batch kernel, FP32, an unnamed CUDA GPU
 HBM_PEAK = 8.0e12  # bytes/s
-# dense peaks.  A 32-bit product of a prompt is three products of half-precision parts, at best a third of the 16-bit
-# rate (the float32 instruction alone: 157.3e12)
-MFMA_PEAK = {"bf16": 2.5e15, "fp32": 2.5e15 / 3}
+# dense peaks.  A 32-bit product of a prompt is six products of bfloat16 parts, at best a sixth of the 16-bit rate (the
+# float32 instruction alone: 157.3e12)
+MFMA_PEAK = {"bf16": 2.5e15, "fp32": 2.5e15 / 6}
 PAGE_SIZE = 16
 PREFILL_TOKENS = 2048
 
@@ -1632,7 +1632,8 @@ def main():
         points["decode_b64"] = round(64 / time_decode(model, cfg, 64, args.context, s, 4), 2)
         read_peak, mfma_peak = measure_peaks("bfloat16")
         if short == "fp32":
-            mfma_peak /= 3  # (as the published one)
+            mfma_peak /= 6  # (as the published one)
+            line["prefill"]["measured_f32_instruction_tflops"] = round(measure_peaks(args.dtype)[1] / 1e12, 1)
         line["roofline"]["measured_peak"] = round(read_peak / 1e9, 1)
         line["roofline"]["frac_of_measured"] = round(achieved / read_peak, 4)
         line["prefill"]["measured_peak_tflops"] = round(mfma_peak / 1e12, 1)

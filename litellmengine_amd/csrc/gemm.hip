@@ -761,8 +761,8 @@ static int gemm_compute_units() {
 }
 
 // The streaming kernel takes the product when K is a number of whole rounds of its 16 wavefronts
-// (1024 elements a round) that its registers hold, X has up to 16 rows, and W has more than one
-// tile of rows for every CU.
+// (1024 elements a round, 512 of float32) that its registers hold (up to 32 rows of X: fewer rounds
+// beyond 16), and W has more than one tile of rows for every CU.
 template <typename T, bool GATED, bool SCALED, typename TC>
 static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, int K,
                                  const NormFold& fold, hipStream_t stream) {
@@ -1076,7 +1076,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE) void gemm_skinny_f32_kernel(con
 }
 
 // X [M, K] and W [N, K] float32, contiguous; C [M, N] float32; 1 <= M <= 64; K a multiple of 4.
-// The streaming kernel takes what it holds a row of X of (K a multiple of 512 up to 4096; 2048 beyond 16 rows), as for
+// The streaming kernel takes what it holds a row of X of (K 512 times 1 to 6 or 8; up to 2048 beyond 16 rows), as for
 // bfloat16: at 8 rows 24576 x 4096 96.7 -> 83.6 us, 151936 x 4096 555 -> 457, 151936 x 1024 at 32 rows 240 -> 124.
 extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

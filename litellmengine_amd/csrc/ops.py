@@ -89,7 +89,7 @@ class HipOps:
         self._fn = {}
         self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta) ...
         self._forms_tuning = None  # ... with these numbers
-        self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives)
+        self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives, beyond the order of its sums)
 
     # -- plumbing ---------------------------------------------------------
     def _get(self, lib: str, name: str, argtypes):

@@ -1,4 +1,4 @@
-"""What was measured on one chip and decides WHICH kernel takes a product: never a result.
+"""What was measured on one chip and decides WHICH kernel takes a product: never a result, beyond the order of its sums.
 
 Every number here was found on an MI355X (256 CUs, HBM3E) with the weights of the Qwen3 sizes
 from 0.6B to 32B.  They sit in one object, `HipOps.tuning`, so that another chip or another family
