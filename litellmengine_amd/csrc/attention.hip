@@ -752,10 +752,13 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
     const int G = nq / nkv;
     if (FUSED && fused.order) {
         // More workgroups than CUs, which take one each and the next as they finish: with the longest requests first the
-        // last ones to start are short (all heads of a request before the next request).
-        const int id = blockIdx.y * gridDim.x + blockIdx.x;
-        s = fused.order[id / nkv];
-        kvh = id % nkv;
+        // last ones to start are short (all heads of a request before the next request).  Consecutive workgroups go to
+        // different dies: the heads turn from request to request, so that a die does not read the same head of every
+        // page, whose places repeat every 32 KB.  (64, 128 requests of 4096 keys, 8 key heads: 191, 351 us as they come; 191,
+        // 411 longest first, 180, 351 with turned heads.  32 of 16 key heads: 186, 232, 178.)
+        const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / nkv;
+        s = fused.order[rank];
+        kvh = (id + rank * min(nkv, 8) / 8) % nkv;
     }
     const int q_start = cu_tokens[s], q_end = cu_tokens[s + 1], kv_len = kv_lens[s], seq_slot = seq_slots[s];
     asm volatile("" ::"s"(q_start), "s"(q_end), "s"(kv_len), "s"(seq_slot));

@@ -50,3 +50,58 @@ def test_the_order_changes_no_result(nkv, group, lens):
     a, b = kv.clone(), kv.clone()
     plain, ordered = run(a, None), run(b, torch.argsort(kv_lens, descending=True, stable=True).to(torch.int32))
     assert torch.equal(plain, ordered) and torch.equal(a, b) and not torch.equal(a, kv) and bool(plain.float().isfinite().all())
+
+
+def step_of(nkv, group, lens):
+    """A decode step's arguments, and its attention over a pool in an order."""
+    o = ops()
+    d, P, S, nq = 128, 16, len(lens), nkv * group
+    g = torch.Generator(device="cuda").manual_seed(3)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    pages = [-(-n // P) for n in lens]
+    table = torch.full((S, max(pages)), -1, dtype=torch.int32)
+    first = 0
+    for s, n in enumerate(pages):
+        table[s, :n] = torch.arange(first, first + n, dtype=torch.int32)
+        first += n
+    slots = i32([int(table[s, (n - 1) // P]) * P + (n - 1) % P for s, n in enumerate(lens)])
+    table = table.cuda()
+    kv = torch.randn(first, 2, nkv, P, d, generator=g, device="cuda").bfloat16()
+    qkv = torch.randn(S, (nq + 2 * nkv) * d, generator=g, device="cuda").bfloat16()
+    w = torch.ones(d, device="cuda").bfloat16()
+    kv_lens, seqs, cu = i32(lens), i32(range(S)), i32(range(S + 1))
+    inv = (1e4 ** (-torch.arange(0, d, 2) / d)).float().cuda()
+    cs = o.rope_table((kv_lens - 1).contiguous(), inv)
+    run = lambda pool, order: o.qk_norm_rope_attention(qkv, slots, w, w, cs, 1e-6, pool, nq, nkv, d, True, table, seqs, cu, kv_lens, seqs, None,
+                                                       d ** -0.5, max(lens), order)
+    return kv, run, torch.argsort(kv_lens, descending=True, stable=True).to(torch.int32)
+
+
+@pytest.mark.parametrize("nkv,group,S", [(2, 3, 150), (4, 4, 70), (5, 2, 60), (12, 1, 23), (16, 2, 33), (16, 1, 3)])
+def test_every_head_of_every_request_is_taken_once(nkv, group, S):
+    """Numbers of key heads that divide the dies, or do not."""
+    kv, run, order = step_of(nkv, group, [1 + (37 * s) % 300 for s in range(S)])
+    a, b = kv.clone(), kv.clone()
+    plain, ordered = run(a, None), run(b, order)
+    assert torch.equal(plain, ordered) and torch.equal(a, b) and not torch.equal(a, kv) and bool(plain.float().isfinite().all())
+
+
+def milliseconds(run, kv, order):
+    best = float("inf")
+    for _ in range(6):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(4):
+            run(kv, order)
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end))
+    return best
+
+
+def test_requests_of_one_length_lose_nothing():
+    """32 requests of 4096 keys and 16 key heads took 186 us as they come and 232 in an order in which each die had its own heads."""
+    if ops().compute_units() != 256:
+        pytest.skip("measured with 256 CUs")
+    kv, run, order = step_of(16, 1, [4096] * 32)
+    assert milliseconds(run, kv, order) < 1.1 * milliseconds(run, kv, None)
