@@ -739,6 +739,12 @@ class HipOps:
                   kv_layer.stride(0), block_table.shape[1], win, float(scale), ns, _ptr(order))
         return out
 
+    # Keys that a workgroup of the decode kernel asks for at its start (two steps of 32 for each of four wavefronts): up to so many
+    # the longest request takes about as long as the shortest and an order is only one more thing to wait for.  (64 requests,
+    # 8 key heads, as they come / longest first: of 64 to 256 keys 19.0 / 19.5 us, of 96 to 384 23.9 / 23.0, of 256 to 1024
+    # 41.4 / 37.5; 96 of 2 key heads alike.)
+    DECODE_KEYS_AT_ONCE = 256
+
     def decode_order(self, kv_lens, num_kv_heads: int):
         """The requests of a decode step by falling length (int32 [S], on the device), for qk_norm_rope_attention; None where its
         workgroups, one for every request and key head, all start at once or there are over 1024 requests.  (A CU holds one

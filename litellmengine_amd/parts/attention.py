@@ -112,13 +112,15 @@ class PagedAttention(Mixer):
             if ops.can_fuse_rope_attention(qkv.dtype, self.d, rot, cache.kv.shape[3], self.nq // self.nkv,
                                            step.max_q_len, step.max_kv_len, step.seq_slots.shape[0]):
                 # a decode step: norm, rotation, cache write and attention in one launch
-                order_key = ("decode_order", self.nkv)
-                if order_key not in step.scratch:  # (once a step: every layer starts the requests in the same order)
-                    step.scratch[order_key] = ops.decode_order(step.kv_lens, self.nkv)
+                order, order_key = None, ("decode_order", self.nkv)
+                if min(step.max_kv_len, self.window or step.max_kv_len) > ops.DECODE_KEYS_AT_ONCE:
+                    if order_key not in step.scratch:  # (once a step: every layer starts the requests in the same order)
+                        step.scratch[order_key] = ops.decode_order(step.kv_lens, self.nkv)
+                    order = step.scratch[order_key]
                 a = ops.qk_norm_rope_attention(
                     qkv, group.slot_mapping, self.q_norm_w, self.k_norm_w, cos_sin, eps, cache.kv, self.nq,
                     self.nkv, self.d, cache.writes, group.block_table, step.seq_slots, step.cu_tokens,
-                    step.kv_lens, step.token_seq, self.window, self.scale, step.max_kv_len, step.scratch[order_key],
+                    step.kv_lens, step.token_seq, self.window, self.scale, step.max_kv_len, order,
                 )
                 return self.o.forward(a, fold=fold)
             q = ops.qk_norm_rope_write(

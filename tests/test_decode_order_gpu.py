@@ -105,3 +105,27 @@ def test_requests_of_one_length_lose_nothing():
         pytest.skip("measured with 256 CUs")
     kv, run, order = step_of(16, 1, [4096] * 32)
     assert milliseconds(run, kv, order) < 1.1 * milliseconds(run, kv, None)
+
+
+@pytest.mark.parametrize("keys,window,orders", [(256, None, False), (257, None, True), (4096, 256, False), (4096, 300, True)])
+def test_short_requests_come_as_they_are(monkeypatch, keys, window, orders):
+    """No order is made, nor waited for, where no layer's request has more keys than a workgroup asks for at its start."""
+    from types import SimpleNamespace
+
+    from litellmengine_amd.parts.attention import PagedAttention
+
+    o = ops()
+    made, given = [], []
+    monkeypatch.setattr(o, "decode_order", lambda lens, heads: made.append(heads) or "order")
+    monkeypatch.setattr(o, "can_fuse_rope_attention", lambda *a: True)
+    monkeypatch.setattr(o, "qk_norm_rope_attention", lambda *a: given.append(a[-1]))
+    part = SimpleNamespace(ctx=SimpleNamespace(ops=o), qkv=SimpleNamespace(forward=lambda x: x), o=SimpleNamespace(forward=lambda a, fold: a),
+                           position=SimpleNamespace(fused_rotary=lambda step: (None, 128)), qk_norm_eps=None, d=128, nq=8, nkv=8, q_norm_w=None,
+                           k_norm_w=None, window=window, scale=1.0)
+    lens = torch.full((64,), keys, dtype=torch.int32, device="cuda")
+    step = SimpleNamespace(max_q_len=1, max_kv_len=keys, seq_slots=lens, kv_lens=lens, cu_tokens=None, token_seq=None, scratch={})
+    cache = SimpleNamespace(kv=torch.empty(1, 2, 8, 16, 128), writes=True, group=SimpleNamespace(slot_mapping=None, block_table=None))
+    x = torch.empty(1, device="cuda", dtype=torch.bfloat16)
+    PagedAttention.forward(part, x, step, cache)
+    PagedAttention.forward(part, x, step, cache)
+    assert given == ["order" if orders else None] * 2 and len(made) == int(orders)
