@@ -837,7 +837,11 @@ class HipOps:
         half blocks of 128 rows per CU on (measured, 32 / 8 heads of 128: a 2048-token prompt 372 us, in
         one tile 481; a 1024-token one 184 and 126), and for portions with at least as much behind them,
         2048 keys or more, which key splits spread instead (300 tokens behind 4000: 239 us, in one tile
-        469; 512 behind 2048: 220 and 285; 128 behind 1000: 53 and 44).
+        469; 512 behind 2048: 220 and 285; 128 behind 1000: 53 and 44).  Splits fill two rounds where each has
+        14 steps of 16 keys left, else one where it has 10; with fewer, or where half of the second tiles
+        would be empty, one tile is faster: in one tile / two tiles and one round / two rounds 128 tokens behind
+        2000 71.5 / 62.0 / 70.9 us, 200 behind 2000 131 / 108 / 101, 64 behind 2000 43 / 43 / 51; of 8 / 1 heads
+        64 behind 4000 28.6 / 36.4 / 36.5, 128 behind 2000 28.9 / 30.1 / 40.4, 300 behind 2000 54 / 48 / 56.
         Between one and two blocks per CU all of them start at once and nothing evens out what the CUs
         got: the second one of a CU is the shortest left (a 2048-token prompt 480 -> 372 us, a 1024-token
         one 178 -> 126); otherwise the longest first (4096 tokens: 1386 us, paired 1584)."""
@@ -848,12 +852,15 @@ class HipOps:
         def blocks(tiles):  # (the rows of several requests share no block: a few more than this)
             return num_kv_heads * -(-N * group // (64 * tiles))
 
-        if not plain or d not in (64, 128):
-            tiles = 1
-        elif max_q_len * group > 64 and span >= max(2048, 2 * max_q_len) and 2 * blocks(2) < 3 * cus:
-            return 2, 0, 2
-        else:
-            tiles = 2 if 2 * blocks(2) >= 3 * cus else 1
+        tiles = 1
+        if plain and d in (64, 128):
+            if max_q_len * group > 64 and span >= max(2048, 2 * max_q_len) and 2 * blocks(2) < 3 * cus:
+                steps = (span + 15) // 16  # (of a split, once the splits fill `rounds` rounds)
+                for rounds, least in ((2, 14), (1, 10)):
+                    if 5 * blocks(2) <= 3 * blocks(1) and steps >= least * (rounds * cus // blocks(2)):
+                        return 2, 0, rounds
+            elif 2 * blocks(2) >= 3 * cus:
+                tiles = 2
         return tiles, int(cus < blocks(tiles) <= 2 * cus), 1
 
     def f32_attention_splits(self, num_seqs: int, num_kv_heads: int, row_blocks: int, max_q_len: int,

@@ -112,3 +112,19 @@ def test_rule():
     assert form(300, 32, 8, 128, True, 300, 4300) == (2, 0, 2)
     assert form(8, 32, 8, 128, True, 1, 4300) == (1, 0, 1)
     assert form(4096, 32, 8, 256, True, 4096, 4096)[0] == 1 and form(4096, 32, 8, 128, False, 4096, 4096)[0] == 1
+
+
+@pytest.mark.parametrize("nq,nkv,tokens,past,want", [(32, 8, 64, 2000, (1, 0, 1)), (32, 8, 128, 2000, (2, 0, 1)), (32, 8, 200, 2000, (2, 0, 2)),
+                                                     (32, 8, 300, 4000, (2, 0, 2)), (8, 1, 128, 2000, (1, 0, 1)), (8, 1, 64, 4000, (1, 0, 1)),
+                                                     (8, 1, 300, 2000, (2, 0, 1)), (16, 8, 96, 12000, (1, 0, 1)), (8, 2, 400, 12000, (2, 0, 2))])
+def test_splits_of_two_tiles_have_enough_keys(nq, nkv, tokens, past, want):
+    """Two tiles in splits of a few steps took up to 1.4 times as long as one tile (8 / 1 heads, 128 tokens behind 2000: 40.4 and 28.9 us)."""
+    o = default_ops()
+    if o.compute_units() != 256:
+        pytest.skip("the form follows the number of CUs")
+    assert o.f32_attention_form(tokens, nq, nkv, 128, True, tokens, past + tokens) == want
+    args = batch([tokens], [past], nq, nkv, 64)
+    got = run(o, args, [tokens], [past], None)
+    # a row's sums are chains of at most (12000 + 400) / 16 steps, rescaled and rounded, of weights that add to 1 over values up to 4
+    # (and the weights are off by the scores' roundings): under 1000 roundings of 4 * 2^-24
+    assert (got.cpu().double() - exact(args, [tokens], [past], nkv, None)).abs().max() < 1000 * 4 * 2**-24
