@@ -842,9 +842,11 @@ class HipOps:
         would be empty, one tile is faster: in one tile / two tiles and one round / two rounds 128 tokens behind
         2000 71.5 / 62.0 / 70.9 us, 200 behind 2000 131 / 108 / 101, 64 behind 2000 43 / 43 / 51; of 8 / 1 heads
         64 behind 4000 28.6 / 36.4 / 36.5, 128 behind 2000 28.9 / 30.1 / 40.4, 300 behind 2000 54 / 48 / 56.
-        Between one and two blocks per CU all of them start at once and nothing evens out what the CUs
+        Between four thirds and two blocks per CU all of them start at once and nothing evens out what the CUs
         got: the second one of a CU is the shortest left (a 2048-token prompt 480 -> 372 us, a 1024-token
-        one 178 -> 126); otherwise the longest first (4096 tokens: 1386 us, paired 1584)."""
+        one 178 -> 126); otherwise the longest first (4096 tokens: 1386 us, paired 1584; with 304 to 336 blocks
+        most CUs get no second one, and the pairs' first half has its longest there: 1300 tokens of 16 / 8 heads
+        173, paired 189, 600 and 60 tokens of 32 / 8 heads 80 and 99, under a window of 256 47 and 68)."""
         cus, group = self.compute_units(), nq // num_kv_heads
         if max_q_len * group <= 16:  # decoding: a block a request and key split
             return 1, 0, 1
@@ -861,7 +863,7 @@ class HipOps:
                         return 2, 0, rounds
             elif 2 * blocks(2) >= 3 * cus:
                 tiles = 2
-        return tiles, int(cus < blocks(tiles) <= 2 * cus), 1
+        return tiles, int(4 * cus <= 3 * blocks(tiles) <= 6 * cus), 1
 
     def f32_attention_splits(self, num_seqs: int, num_kv_heads: int, row_blocks: int, max_q_len: int,
                              max_kv_len: int, window: int, rounds: int = 1) -> int:

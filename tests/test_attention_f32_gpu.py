@@ -128,3 +128,16 @@ def test_splits_of_two_tiles_have_enough_keys(nq, nkv, tokens, past, want):
     # a row's sums are chains of at most (12000 + 400) / 16 steps, rescaled and rounded, of weights that add to 1 over values up to 4
     # (and the weights are off by the scores' roundings): under 1000 roundings of 4 * 2^-24
     assert (got.cpu().double() - exact(args, [tokens], [past], nkv, None)).abs().max() < 1000 * 4 * 2**-24
+
+
+def test_few_second_blocks_are_not_paired():
+    """Up to four thirds of a block a CU the longest go first (600 and 60 tokens of 32 / 8 heads, a window of 256: 47 us, paired 68)."""
+    o = default_ops()
+    if o.compute_units() != 256:
+        pytest.skip("the form follows the number of CUs")
+    form = lambda n, nq: o.f32_attention_form(n, nq, 8, 128, True, n, n)
+    assert form(660, 32) == form(1300, 16) == form(514, 32) == (1, 0, 1) and form(700, 32) == form(1024, 32) == (1, 1, 1)
+    lens, past = [600, 60], [0, 0]
+    args = batch(lens, past, 32, 8, 128)
+    got = run(o, args, lens, past, 256)
+    assert (got.cpu().double() - exact(args, lens, past, 8, 256)).abs().max() < 400 * 4 * 2**-24  # (as above)
