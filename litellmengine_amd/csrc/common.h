@@ -27,17 +27,59 @@ __device__ __forceinline__ float load_as_f32(const void* p, int64_t i, int dtype
     return dtype == LLE_F32 ? ((const float*)p)[i] : (float)((const bf16_t*)p)[i];
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = LLE_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, LLE_WAVE);
-    return v;
+// Lanes i and i ^ 32 (or i ^ 16) combined by `op`, in every lane: the two operands of the swap come out as the lower and the
+// upper halves (even and odd rows of 16) repeated.  All lanes of the wavefront must be active here and below.
+template <typename Op>
+__device__ __forceinline__ float combine_xor32(float v, Op op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+template <typename Op>
+__device__ __forceinline__ float combine_xor16(float v, Op op) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// the lane's own value and that of the lane N further on in its row of 16 (around its end)
+template <int N, typename Op>
+__device__ __forceinline__ float combine_row_ror(float v, Op op) {
+    return op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true)));
+}
+struct AddF32 {
+    __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct MaxF32 {
+    __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = LLE_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, LLE_WAVE));
-    return v;
+// All 64 lanes by the tree of i ^ 32, i ^ 16, i ^ 8, ... i ^ 1.  (Once lanes 8 apart hold the same, the lane 4 further on in the
+// row holds what lane i ^ 4 does, and so on.)  Ten instructions between registers instead of six trips through LDS of nine
+// each: a wavefront alone issues an instruction in four to eight cycles, so a decode step's short launches pay for every one.
+template <typename Op>
+__device__ __forceinline__ float combine_wave(float v, Op op) {
+    v = combine_xor32(v, op);
+    v = combine_xor16(v, op);
+    v = combine_row_ror<8>(v, op);
+    v = combine_row_ror<4>(v, op);
+    v = combine_row_ror<2>(v, op);
+    return combine_row_ror<1>(v, op);
 }
+__device__ __forceinline__ float wave_sum(float v) { return combine_wave(v, AddF32{}); }
+__device__ __forceinline__ float wave_max(float v) { return combine_wave(v, MaxF32{}); }
+// the lane's row of 16: i ^ 1, then i ^ 2, 4, 8.  (Once neighbours hold the same, the other pair of a quad is as good as lane
+// i ^ 2; then the mirrored half row as lane i ^ 4, and the mirrored row as lane i ^ 8.)
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row16_sum(float v) {
+    v = add_dpp<0xb1>(v);   // quad_perm 1 0 3 2
+    v = add_dpp<0x4e>(v);   // quad_perm 2 3 0 1
+    v = add_dpp<0x141>(v);  // row_half_mirror
+    return add_dpp<0x140>(v);  // row_mirror
+}
+// the four lanes i % 16 (a column of a matrix-core tile): i ^ 16, then i ^ 32
+__device__ __forceinline__ float column_sum(float v) { return combine_xor32(combine_xor16(v, AddF32{}), AddF32{}); }
+__device__ __forceinline__ float column_max(float v) { return combine_xor32(combine_xor16(v, MaxF32{}), MaxF32{}); }
 
 // Sum over a workgroup of up to 1024 threads; `smem` holds >= 16 floats.
 // Every thread gets the result; the order of the additions is fixed.

@@ -128,6 +128,13 @@ template <typename T, int WAVES = 16> struct SkShare {
     static constexpr int EXTENT = HALVES ? SECOND + WAVE : WAVE;  // from a wavefront's first element to behind its last of a round
 };
 
+// What such a launch is made of (in a HIP graph, one after the other): 1.7 us for a kernel that does nothing, 0.9 ns for every
+// instruction of a wavefront whose CU holds sixteen, a trip to memory; so reductions stay between registers (common.h), what a
+// launch will need is asked for at its start, and rounds that are left over go together.  With four, eight and sixteen
+// wavefronts a workgroup: 6144 x 1024 gated at 1 row 5.8, 4.9, 4.9 us, 4096 x 12288 at 8 rows 29.0, 23.3, 22.1.
+// Before / after these three (0.6B sizes): qkv at 1 / 32 rows 4.4 / 6.8 -> 4.1 / 6.1 us, gate_up 5.5 / 7.8 -> 4.9 / 7.1,
+// down_proj 4.8 / 9.9 -> 4.7 / 9.5.
+//
 // GATED: W holds gate rows [0, N/2) and then up rows [N/2, N); a workgroup takes 16 gate rows
 // and the 16 up rows that go with them (NT = 2) and writes silu(gate) * up, C is [M, N/2].
 //
@@ -170,8 +177,9 @@ __device__ __forceinline__ float gated_result(float g, float u, const NormFold& 
 
 template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL>
 // one tile of W and up to 16 rows of X: two workgroups of 16 wavefronts a CU (8 wavefronts a SIMD),
-// which 64 registers allow; the gated form measured faster with the registers it asks for
-__global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) void gemm_skinny_kernel(const T* __restrict__ X,
+// which 64 registers allow; the gated form measured faster with the registers it asks for, and the scaled one has no room in
+// 64 for the parts that it asks for at its start (three spilled registers cost a launch 0.9 us)
+__global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) ? 8 : 4) void gemm_skinny_kernel(const T* __restrict__ X,
                                                                          const T* __restrict__ W,
                                                                          TC* __restrict__ C, int M, int N, int K,
                                                                          int tile_rows, NormFold fold) {
@@ -195,15 +203,16 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                  "s"(fold.weight_dtype), "s"(fold.xw), "s"(fold.ss_out), "s"(fold.ss_in), "s"(fold.parts),
                  "s"(fold.eps));
     const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
-    // SCALED: wavefront w adds up the parts of the rows w, w + 16.  With one tile of rows the
-    // first parts are asked for now and added after the products.
-    static_assert(!SCALED || SK_WAVES == 16, "one wavefront per row of a tile of the norm");
-    constexpr int EARLY_PARTS = (GATED || MT > 1) ? 0 : 4;  // the gated form measured faster without them
-    float early[EARLY_PARTS + 1];
+    // SCALED: wavefront w adds up the parts of the rows w, w + SK_WAVES, ...  The first parts are asked for now and added after
+    // the products.
+    constexpr int EARLY_PARTS = 4, SUM_ROWS = (16 * MT + SK_WAVES - 1) / SK_WAVES;
+    float early[SUM_ROWS][EARLY_PARTS];
     if (SCALED) {
 #pragma unroll
-        for (int i = 0; i < EARLY_PARTS; ++i)  // past the parts: the last one again, dropped below
-            early[i] = fold.ss_in[(int64_t)wave * fold.parts + min(lane + LLE_WAVE * i, fold.parts - 1)];
+        for (int j = 0; j < SUM_ROWS; ++j)
+#pragma unroll
+            for (int i = 0; i < EARLY_PARTS; ++i)  // past the parts: the last one again, dropped below; past the rows likewise
+                early[j][i] = fold.ss_in[min(wave + SK_WAVES * j, M - 1) * fold.parts + min(lane + LLE_WAVE * i, fold.parts - 1)];
     }
     const int c = lane / 16, r16 = lane % 16;
     const int64_t n0 = (int64_t)blockIdx.x * ((GATED || NT == 1) ? tile_rows : 16 * NT);
@@ -245,11 +254,12 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
     const Vec zero = {};
 
     int kw = wave * Share::WAVE;
-    // UNROLL rounds at a time: all their loads are issued before the first product
-    for (; kw + (UNROLL - 1) * Share::ROUND + Share::EXTENT <= K; kw += UNROLL * Share::ROUND) {
-        Vec w0[UNROLL][NT], w1[UNROLL][NT], x0[UNROLL][MT], x1[UNROLL][MT];
+    // R rounds at a time: all their loads are issued before the first product
+    auto rounds = [&](auto rounds_c) {
+        constexpr int R = decltype(rounds_c)::value;
+        Vec w0[R][NT], w1[R][NT], x0[R][MT], x1[R][MT];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
+        for (int u = 0; u < R; ++u) {
             const int k0 = kw + u * Share::ROUND;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
@@ -262,8 +272,9 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                 x1[u][mt] = *(const Vec*)(xp[mt] + k0 + SECOND);
             }
         }
+        if (R < UNROLL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u)
+        for (int u = 0; u < R; ++u)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -271,9 +282,18 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                     acc[nt][mt] = SkOp<T>::mma(w0[u][nt], x0[u][mt], acc[nt][mt]);
                     acc[nt][mt] = SkOp<T>::mma(w1[u][nt], x1[u][mt], acc[nt][mt]);
                 }
+        kw += R * Share::ROUND;
+    };
+    auto whole = [&](int n) { return kw + (n - 1) * Share::ROUND + Share::EXTENT <= K; };
+    while (whole(UNROLL)) rounds(std::integral_constant<int, UNROLL>{});
+    // what is left of K: whole rounds together (one by one each would pay the way from memory), then a round that may be
+    // partial (K is a multiple of E); there both operands are zeroed beyond K so that nothing outside the matrices is read
+    if constexpr (UNROLL == 4 && MT <= 2) {  // (more rows of X leave no registers for it)
+        if (whole(3))
+            rounds(std::integral_constant<int, 3>{});
+        else if (whole(2))
+            rounds(std::integral_constant<int, 2>{});
     }
-    // what is left of K: single rounds; the last one may be partial (K is a multiple of E),
-    // and there both operands are zeroed beyond K so that nothing outside the matrices is read
     for (; kw < K; kw += Share::ROUND) {
         const int k0 = kw;
         const bool in0 = k0 + Share::LANE * c + E <= K, in1 = k0 + SECOND + Share::LANE * c + E <= K;
@@ -296,11 +316,12 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
     }
     if (SCALED) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int m = 16 * mt + wave;
+        for (int j = 0; j < SUM_ROWS; ++j) {
+            const int m = wave + SK_WAVES * j;
+            if (m >= M) break;  // (the same for the whole wavefront)
             float part = 0.f;
 #pragma unroll
-            for (int i = 0; i < EARLY_PARTS; ++i) part += lane + LLE_WAVE * i < fold.parts ? early[i] : 0.f;
+            for (int i = 0; i < EARLY_PARTS; ++i) part += lane + LLE_WAVE * i < fold.parts ? early[j][i] : 0.f;
             // what is left: four loads at a time (one after the other would each pay the way from memory)
             const float* in = fold.ss_in + (int64_t)m * fold.parts;
             for (int b = lane + LLE_WAVE * EARLY_PARTS; b < fold.parts; b += 4 * LLE_WAVE) {
@@ -359,8 +380,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED) ? 8 : 4) vo
                         (T)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid_w : resid_w << 16));
                     sq = h * h;
                 }
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, LLE_WAVE);
+                sq = row16_sum(sq);
                 if (n == 0) fold.ss_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
             }
         }

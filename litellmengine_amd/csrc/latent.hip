@@ -383,8 +383,7 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
                 sv[u][i] = (key >= lo[u] && key <= pos[u]) ? sacc[i] * sc2 : LAT_NEG_BIG;
                 mx = fmaxf(mx, sv[u][i]);
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, LLE_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, LLE_WAVE));
+            mx = column_max(mx);
             if (c == 0) s_max[buf][u][wave][r] = mx;
         }
         __syncthreads();
@@ -426,8 +425,7 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
     }
 #pragma unroll
     for (int u = 0; u < RT; ++u) {
-        l[u] += __shfl_xor(l[u], 16, LLE_WAVE);
-        l[u] += __shfl_xor(l[u], 32, LLE_WAVE);
+        l[u] = column_sum(l[u]);
         if (c == 0) s_l[u][wave][r] = l[u];
     }
     __syncthreads();

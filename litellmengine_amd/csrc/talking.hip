@@ -223,13 +223,11 @@ __global__ __launch_bounds__(256) void talking_scores_kernel(TalkArgs a, float* 
                 sc[i] = j < lo || j > pos ? NEG_BIG : fmaf(sc[i], a.scale * LOG2E, slope * (float)(j - pos));
                 top = fmaxf(top, sc[i]);
             }
-            top = fmaxf(top, __shfl_xor(top, 16, LLE_WAVE));
-            top = fmaxf(top, __shfl_xor(top, 32, LLE_WAVE));
+            top = column_max(top);
             float sum = 0.f;  // (every tile holds a key that the query sees: its maximum is a score)
 #pragma unroll
             for (int i = 0; i < 4; ++i) sum += __builtin_amdgcn_exp2f(sc[i] - top);
-            sum += __shfl_xor(sum, 16, LLE_WAVE);
-            sum += __shfl_xor(sum, 32, LLE_WAVE);
+            sum = column_sum(sum);
             if (exists) {
                 const int64_t row = (int64_t)s * a.H + h;
                 *(f32x4*)(ws_s + row * K + 16 * tile + 4 * c) = sc;
@@ -455,12 +453,10 @@ __global__ __launch_bounds__(TS_WAVES* LLE_WAVE) void talking_sums_kernel(TalkAr
         __syncthreads();  // (the round before has been read)
 #pragma unroll
         for (int i = 0; i < TS_HEADS; ++i) {
-            float top = fmaxf(m[i], __shfl_xor(m[i], 16, LLE_WAVE));
-            top = fmaxf(top, __shfl_xor(top, 32, LLE_WAVE));
+            const float top = column_max(m[i]);
             const float base = top <= NEG_BIG ? 0.f : top;
             float sum = l[i] * __builtin_amdgcn_exp2f(m[i] - base);
-            sum += __shfl_xor(sum, 16, LLE_WAVE);
-            sum += __shfl_xor(sum, 32, LLE_WAVE);
+            sum = column_sum(sum);
             if (c == 0) {
                 s_m[wave][i][r16] = top;
                 s_l[wave][i][r16] = sum;
