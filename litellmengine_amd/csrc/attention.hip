@@ -202,6 +202,7 @@ extern "C" int lle_paged_attention_generic(const void* q, const void* kv_layer, 
 typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
 typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define NEG_BIG (-1.0e30f)
 #define LAZY_MAX 8.0f  // a row's reference maximum may lag its true one by this much (base 2)
@@ -268,8 +269,8 @@ __device__ __forceinline__ void set_open_range(RowState<DK, RT>& st, const RowIn
     }
 }
 
-// LOAD_Q = false: the caller has filled st.qv itself
-template <int DK, int RT, bool LOAD_Q = true>
+// LOAD_Q = false: the caller has filled st.qv itself; FIND_OPEN = false: st.open_lo and st.open_hi, too
+template <int DK, int RT, bool LOAD_Q = true, bool FIND_OPEN = true>
 __device__ __forceinline__ void init_rows(RowState<DK, RT>& st, const RowInfo (&row)[RT]) {
     const int c = (threadIdx.x % LLE_WAVE) / 16;
 #pragma unroll
@@ -290,7 +291,7 @@ __device__ __forceinline__ void init_rows(RowState<DK, RT>& st, const RowInfo (&
         st.m[t] = NEG_BIG;
         st.l[t] = 0.f;
     }
-    set_open_range<DK, RT>(st, row);
+    if constexpr (FIND_OPEN) set_open_range<DK, RT>(st, row);
     // The rows of Q are waited for here, once.  Left pending, their first use lies inside the
     // key loop, where the wait for them also waits for the K/V loads just issued for a later
     // step: the loop would run at the latency of memory.
@@ -383,8 +384,7 @@ __device__ __forceinline__ void tile_step(RowState<DK, RT>& st, const RowInfo (&
 #pragma unroll
             for (int i = 0; i < 8; ++i) sc[i] = x[t][i] <= NEG_BIG ? NEG_BIG : s[t][i / 4][i % 4] * scale_log2;
             float tile_max = max_of_8(sc);
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, LLE_WAVE));
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, LLE_WAVE));
+            tile_max = column_max(tile_max);
             const float new_m = fmaxf(st.m[t], tile_max);
             // while the row has seen no key new_m is NEG_BIG as its masked scores are, and
             // exp2(0) = 1 would count them: shift such rows so that they give 0
@@ -424,10 +424,17 @@ template <int DK, int RT>
 __device__ __forceinline__ void finish_rows(RowState<DK, RT>& st) {
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-        st.l[t] += __shfl_xor(st.l[t], 16, LLE_WAVE);
-        st.l[t] += __shfl_xor(st.l[t], 32, LLE_WAVE);
+        st.l[t] = column_sum(st.l[t]);
     }
 }
+
+// Positions into pages: a shift for the usual powers of two (a division by a number known at run time is some thirty
+// instructions, and a decode launch makes half a dozen before its first load of a key)
+struct PageSize {
+    int P, log2;
+    __device__ __forceinline__ explicit PageSize(int P) : P(P), log2((P & (P - 1)) == 0 ? 31 - __clz(P) : -1) {}
+    __device__ __forceinline__ int of(int position) const { return log2 >= 0 ? position >> log2 : position / P; }
+};
 
 // The operands of one 32-key step as a wavefront loads them straight from the pages.
 template <int DK>
@@ -438,18 +445,18 @@ struct StepOperands {
 
 // The steps step_begin, step_begin + step_stride, ... < step_end with the operands loaded by
 // each wavefront straight from the pages, two steps ahead of their use: while one step is
-// multiplied the loads of the next two are on their way.  Nothing in the loop stands under a
-// condition (a load under a condition makes the compiler wait for every load where the paths
-// meet again): the loop runs an even number of steps, loads past the end go to a page that is
-// there, and the CALLER has limited the rows' `pos` to the last key of step_end - 1, so that a
-// step past the end is masked out whole.
+// multiplied the loads of the next two are on their way.  No load stands under a condition (a
+// load under a condition makes the compiler wait for every load where the paths meet again):
+// loads past the end go to a page that is there.  The loop is left as soon as its last step is
+// multiplied: a wavefront alone issues an instruction in four to eight cycles, so a step that
+// is masked out whole would be half a microsecond for nothing.
 // `before_keys()` runs when the first table lookup is on its way and no operand is asked for yet:
 // what the caller loads there travels beside the lookup, what it stores there is stored before
 // this wavefront reads any key.  `after_first_loads()` runs once the first two steps are asked for.
 // A second range of keys is walked by a call with FIRST = false (the rows' lo and pos are the range's
 // then, what the first call has summed up stays); all calls but the last have LAST = false.
-template <int DK, int RT, bool LOAD_Q = true, bool FIRST = true, bool LAST = true, bool CAP = false, typename BeforeKeys,
-          typename AfterFirstLoads>
+template <int DK, int RT, bool LOAD_Q = true, bool FIRST = true, bool LAST = true, bool CAP = false, bool FIND_OPEN = true,
+          typename BeforeKeys, typename AfterFirstLoads>
 __device__ __forceinline__ void attend_rows(RowState<DK, RT>& st, const RowInfo (&row)[RT],
                                             const bf16_t* kv_layer, const int32_t* __restrict__ table,
                                             int kvh, int nkv, int P, int64_t page_stride, int step_begin,
@@ -459,7 +466,7 @@ __device__ __forceinline__ void attend_rows(RowState<DK, RT>& st, const RowInfo 
     constexpr int D = DK * 32;
     const int lane = threadIdx.x % LLE_WAVE;
     const int c = lane / 16, r16 = lane % 16;
-    if constexpr (FIRST) init_rows<DK, RT, LOAD_Q>(st, row);
+    if constexpr (FIRST) init_rows<DK, RT, LOAD_Q, FIND_OPEN>(st, row);
     else set_open_range<DK, RT>(st, row);
     // the lane's keys of tile x lie in the 16-key half r16 / 8 of the step, its eight V keys in half c / 2
     const int k_half = r16 / 8, v_half = c / 2;
@@ -470,9 +477,10 @@ __device__ __forceinline__ void attend_rows(RowState<DK, RT>& st, const RowInfo 
     // out each time (the page size is no constant), and the table is read one load ahead.  A
     // half wholly outside [lo_min, hi] may lie in a page that is not there: the page index is
     // clamped to those of keys that are.
-    const int page_lo = lo_min / P, page_hi = hi / P;
-    const int adv_pages = (step_stride * KSTEP) / P, adv_off = (step_stride * KSTEP) % P;
-    int look_page = (step_begin * KSTEP) / P, look_off = (step_begin * KSTEP) % P;
+    const PageSize pages(P);
+    const int page_lo = pages.of(lo_min), page_hi = pages.of(hi);
+    const int adv_pages = pages.of(step_stride * KSTEP), adv_off = step_stride * KSTEP - adv_pages * P;
+    int look_page = pages.of(step_begin * KSTEP), look_off = step_begin * KSTEP - look_page * P;
     int page_id[2], page_off[2];
     auto lookup = [&]() {
         const bool next_page = look_off + 16 == P;  // pages hold a multiple of 16 keys
@@ -513,10 +521,13 @@ __device__ __forceinline__ void attend_rows(RowState<DK, RT>& st, const RowInfo 
     load(even);
     load(odd);
     after_first_loads();
-    for (int step = step_begin; step < step_end; step += 2 * step_stride) {
+    for (int step = step_begin; step < step_end; step += step_stride) {
         multiply(even, step);
+        step += step_stride;
+        if (step >= step_end) break;
         load(even);
-        multiply(odd, step + step_stride);
+        multiply(odd, step);
+        if (step + step_stride >= step_end) break;
         load(odd);
     }
     if constexpr (LAST) finish_rows<DK, RT>(st);
@@ -527,7 +538,7 @@ __device__ __forceinline__ RowInfo make_row(const bf16_t* q, int r, int nrows, i
                                             int kvh, int D, int window) {
     RowInfo info;
     if (r < nrows) {
-        const int t = r / G, g = r - t * G;
+        const int t = nrows == G ? 0 : r / G, g = r - t * G;
         info.q = q + ((int64_t)(q_start + t) * nq + kvh * G + g) * D;
         info.pos = past + t;
         info.lo = window > 0 ? max(0, info.pos - window + 1) : 0;
@@ -590,52 +601,60 @@ __device__ __forceinline__ float weight_as_f32(uint32_t raw, bool is_f32) {
 // partner D / 2 further on are both in this lane (DK is even).  Rounded to bfloat16 as the
 // separate kernel rounds q.  Everything is ASKED FOR in one go (load) and worked on later
 // (finish): a load that followed the arithmetic on another would cost the memory's latency again.
-template <int DK>
+// WEIGHTS: their type where the launch is made for it, -1 where only FusedQKV::weight_dtype knows.
+template <int DK, int WEIGHTS = -1>
 struct FusedQRow {
     static_assert(DK % 2 == 0, "rotation partners lie in one lane only for an even number of 32-element blocks");
+    typedef float4 Table[DK / 2][4];  // cos, sin of element 2 i, then of 2 i + 1
     bf16x8 raw[DK];
     RawWeights8 w[DK];
-    float4 tab[DK / 2][4];  // cos, sin of element 2 i, then of 2 i + 1
 
     // `src`: the head of a row that exists (lanes of rows that do not exist read another row's and drop it)
-    __device__ __forceinline__ void load(const bf16_t* src, const FusedQKV& f, int64_t tok) {
-        constexpr int D = DK * 32;
+    __device__ __forceinline__ void load(const bf16_t* src, const void* weight, int weight_dtype) {
         const int c = (threadIdx.x % LLE_WAVE) / 16;
 #pragma unroll
         for (int ks = 0; ks < DK; ++ks) raw[ks] = *(const bf16x8*)(src + 32 * ks + 8 * c);
+        if (weight) {
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks) load_raw_weights8(weight, 32 * ks + 8 * c, WEIGHTS < 0 ? weight_dtype : WEIGHTS, w[ks]);
+        }
+    }
+    static __device__ __forceinline__ void load_table(Table& tab, const FusedQKV& f, int64_t tok) {
+        constexpr int D = DK * 32;
+        const int c = (threadIdx.x % LLE_WAVE) / 16;
 #pragma unroll
         for (int ks = 0; ks < DK / 2; ++ks) {
             const float4* t = (const float4*)(f.cos_sin + (tok * (D / 2) + 32 * ks + 8 * c) * 2);
 #pragma unroll
             for (int i = 0; i < 4; ++i) tab[ks][i] = t[i];
         }
-        if (f.q_weight) {
-#pragma unroll
-            for (int ks = 0; ks < DK; ++ks) load_raw_weights8(f.q_weight, 32 * ks + 8 * c, f.weight_dtype, w[ks]);
-        }
     }
 
-    __device__ __forceinline__ void finish(bf16x8 (&qv)[DK], bool exists, const FusedQKV& f) const {
+    __device__ __forceinline__ void finish(bf16x8 (&qv)[DK], const Table& tab, const FusedQKV& f, bool normed) const {
         constexpr int D = DK * 32;
         float x[DK][8];
 #pragma unroll
         for (int ks = 0; ks < DK; ++ks)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) x[ks][i] = exists ? (float)raw[ks][i] : 0.f;
-        if (f.q_weight) {
+            for (int i = 0; i < 8; ++i) x[ks][i] = (float)raw[ks][i];
+        if (normed) {
             float ss = 0.f;
 #pragma unroll
             for (int ks = 0; ks < DK; ++ks)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) ss += x[ks][i] * x[ks][i];
-            ss += __shfl_xor(ss, 16, LLE_WAVE);
-            ss += __shfl_xor(ss, 32, LLE_WAVE);
+            ss = column_sum(ss);
             const float inv = 1.0f / sqrtf(ss / (float)D + f.eps);
-            const bool is_f32 = f.weight_dtype == LLE_F32;
+            auto weigh = [&](auto is_f32) {
 #pragma unroll
-            for (int ks = 0; ks < DK; ++ks)
+                for (int ks = 0; ks < DK; ++ks)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[ks][i] = x[ks][i] * inv * weights8_as_f32(w[ks], i, is_f32);
+                    for (int i = 0; i < 8; ++i) x[ks][i] = x[ks][i] * inv * weights8_as_f32(w[ks], i, decltype(is_f32)::value);
+            };
+            if (WEIGHTS < 0 ? f.weight_dtype == LLE_F32 : WEIGHTS == LLE_F32)  // (the same for the whole launch: a branch instead of 32 selects)
+                weigh(std::integral_constant<bool, true>{});
+            else
+                weigh(std::integral_constant<bool, false>{});
         }
 #pragma unroll
         for (int ks = 0; ks < DK / 2; ++ks) {
@@ -692,7 +711,7 @@ __device__ __forceinline__ void fused_kv_write(const FusedQKV& f, int64_t tok, i
         }
     }
     if (slot < 0) return;
-    const int page = slot / P, off = slot - page * P;
+    const int page = PageSize(P).of(slot), off = slot - page * P;
     bf16_t* page_base = kv_layer + (int64_t)page * page_stride;
     bf16_t* kdst = page_base + ((int64_t)kvh * P + off) * D;
     bf16_t* vdst = page_base + ((int64_t)nkv + kvh) * P * D + off;  // element e at vdst[e * P]
@@ -775,31 +794,37 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
     const int lo_min = window > 0 ? max(0, past - window + 1) : 0;
     const int hi = kv_len - 1;
     const int first = lo_min / KSTEP, last = hi / KSTEP;
-    const int per_split = (last - first + 1 + nsplit - 1) / nsplit;
+    const int per_split = nsplit == 1 ? last - first + 1 : (last - first + 1 + nsplit - 1) / nsplit;
     const int sb = first + split * per_split;
     const int se = min(last + 1, sb + per_split);
-    // keys of later splits are not this workgroup's: attend_rows may run a step past `se`
+    // keys of later splits are not this workgroup's
     row[0].pos = min(row[0].pos, se * KSTEP - 1);
-    // ... and asks for operands two steps ahead: past this split's last key those loads go to the
+    // attend_rows asks for operands two steps ahead: past this split's last key those loads go to the
     // split's own last page (which the caches hold) instead of the next split's pages, which would
     // travel from memory twice, once for each of the two workgroups
     const int hi_loads = max(lo_min, min(hi, se * KSTEP - 1));
 
     RowState<DK, 1> st;
+    if constexpr (!KEEP) {  // the request's tokens see from its last one's first key on, and up to its first one's own
+        st.open_lo[0] = window > 0 ? max(0, hi - window + 1) : 0;
+        st.open_hi[0] = min(past, se * KSTEP - 1);
+    }
     if constexpr (FUSED) {
         // The raw q row, its rotation table and the norm weights are asked for while the table
         // lookup is on its way.  A new token's K and V go into the pages by the hand of the
         // wavefront that multiplies the token's step (step sb + wave, + DEC_WAVES, ...): it
-        // stores them before it asks for any key, no other wavefront of this launch needs them
-        // (one that runs a step past its share masks that step out whole), and so no barrier
-        // stands between the write and the keys.
+        // stores them before it asks for any key, no other wavefront of this launch needs them,
+        // and so no barrier stands between the write and the keys.
         FusedQRow<DK> qrow;
+        typename FusedQRow<DK>::Table tab;
         const int rr = r16 < nrows ? r16 : 0;
-        const int64_t tok = (int64_t)q_start + rr / G;
-        attend_rows<DK, 1, false>(
+        const int t_row = nrows == G ? 0 : rr / G;
+        const int64_t tok = (int64_t)q_start + t_row;
+        attend_rows<DK, 1, false, true, true, false, false>(
             st, row, kv_layer, table, kvh, nkv, P, page_stride, sb + wave, se, DEC_WAVES, lo_min, hi_loads, scale_log2,
             [&]() {
-                qrow.load(fused.qkv + (tok * (nq + 2 * nkv) + kvh * G + rr % G) * D, fused, tok);
+                qrow.load(fused.qkv + (tok * (nq + 2 * nkv) + kvh * G + rr - t_row * G) * D, fused.q_weight, fused.weight_dtype);
+                FusedQRow<DK>::load_table(tab, fused, tok);
                 if (fused.write_kv) {
                     for (int t = 0; t < q_len; ++t) {
                         const int step_of = (past + t) / KSTEP;
@@ -813,7 +838,7 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
                     asm volatile("" ::: "memory");
                 }
             },
-            [&]() { qrow.finish(st.qv[0], r16 < nrows, fused); });
+            [&]() { qrow.finish(st.qv[0], tab, fused, fused.q_weight != nullptr); });
     } else if constexpr (KEEP) {
         // the kept first keys are the first split's work (few steps)
         init_rows<DK, 1, true>(st, row);
@@ -831,7 +856,7 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
             st, row, kv_layer, table, kvh, nkv, P, page_stride, sb + wave, se, DEC_WAVES, lo_min, hi_loads, scale_log2,
             []() {}, []() {});
     } else {
-        attend_rows<DK, 1, true, true, true, CAP>(
+        attend_rows<DK, 1, true, true, true, CAP, false>(
             st, row, kv_layer, table, kvh, nkv, P, page_stride, sb + wave, se, DEC_WAVES, lo_min, hi_loads, scale_log2,
             []() {}, []() {}, cap_log2);
     }
@@ -858,7 +883,7 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
             num += s_o[(w * 16 + r) * D + e] * f;
             den += s_l[w * 16 + r] * f;
         }
-        const int t = r / G, g = r - t * G;
+        const int t = nrows == G ? 0 : r / G, g = r - t * G;
         const int64_t head_row = (int64_t)(q_start + t) * nq + kvh * G + g;
         if (nsplit == 1) {
             if (sinks) den += exp2f(sinks[kvh * G + g] * 1.44269504088896340736f - big);  // (a sink: a place in the sum without a value)
@@ -870,6 +895,166 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
                 ws_ml[(head_row * ws_stride + split) * 2 + 1] = den;
             }
         }
+    }
+}
+
+// One new token a request, at most SHORT_WAVES * 32 keys: grid (requests, kv heads), a wavefront for every 32 keys and one for the
+// new token.  A launch of this size is bound by how many instructions stand in a row (a wavefront alone issues one in four to
+// eight cycles) and by trips to memory that wait for each other, not by bytes: no loop over keys, no running maximum, no carried
+// page numbers (a wavefront's keys lie at the same positions of every request), and the new token's key and value never pass
+// through the page: their wavefront scores and stores them while the others wait for theirs.  The wavefronts meet once, in LDS;
+// those without keys leave zeros there.
+// 0.6B sizes (16 q heads, 8 kv heads of 128) at 97 keys, 1 / 8 / 32 requests: 7.9 / 8.1 / 9.7 us in mfma_decode_kernel, whose
+// loop holds two steps and whose new token goes through the page, 6.1 / 6.5 / 8.0 here.
+#define SHORT_WAVES 8
+template <int DK, int WEIGHTS>
+__global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_kernel(
+    const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ seq_slots,
+    const int32_t* __restrict__ block_tables, int max_pages, int P, int window, int G, int nkv, bf16_t* kv_layer,
+    bf16_t* __restrict__ out, int64_t page_stride, float scale_log2, FusedQKV f) {
+    // The first sixteen words of the arguments come with the launch: the tables that everything waits for are among them, and what is
+    // known of the request is asked for before the other arguments.  Each of these statements has one trip to memory behind it:
+    // read where they are first used, the same loads are five in a row.  (Pointers that are read by scalar loads stay out of them.)
+    const int s = blockIdx.x, kvh = blockIdx.y;
+    const int tok = cu_tokens[s], tok_end = cu_tokens[s + 1], kv_len = kv_lens[s], seq_slot = seq_slots[s];
+    asm volatile("" ::"s"(tok), "s"(tok_end), "s"(kv_len), "s"(seq_slot), "s"(nkv), "s"(kv_layer), "s"(out), "s"(page_stride),
+                 "s"(scale_log2), "s"(f.qkv), "s"(f.q_weight), "s"(f.k_weight), "s"(f.cos_sin), "s"(f.eps), "s"(f.write_kv));
+    constexpr int D = DK * 32, WAVES = SHORT_WAVES + 1;
+    extern __shared__ float smem[];  // [waves][G][D] acc, then [waves][16] m, [waves][16] l
+    float* s_m = smem + WAVES * G * D;
+    float* s_l = s_m + WAVES * 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    const int c = lane / 16, r16 = lane % 16;
+    if (tok_end - tok != 1) return;  // (a request without a token has nothing to do)
+    const int last = kv_len - 1, lo = window > 0 ? max(0, kv_len - window) : 0;
+    const int j0 = wave * KSTEP;  // the wavefront's first key
+    // both halves' pages (a half outside what is seen reads the other half's page; a wavefront without keys the last key's)
+    const PageSize pages(P);
+    const int j0_kept = min(j0, last), j1 = j0_kept + 16 <= last ? j0_kept + 16 : j0_kept, j0_seen = j0_kept + 16 > lo ? j0_kept : j1;
+    const int p0 = pages.of(j0_seen), p1 = pages.of(j1);
+    const int32_t* table = block_tables + (int64_t)seq_slot * max_pages;
+    const int page0 = table[p0], page1 = table[p1], slot = f.slots[tok];
+    const bool fresh = f.write_kv && slot >= 0;  // (else the new token's place holds what the page does)
+    const bf16_t* qkv = f.qkv + (int64_t)tok * (nkv * (G + 2)) * D;
+    const bf16_t* q_head = qkv + (int64_t)(kvh * G + min(r16, G - 1)) * D;  // (rows past the group's: dropped at the end)
+    f32x4 o[2 * DK];
+    float top = NEG_BIG, l = 0.f;
+    if (wave < SHORT_WAVES && j0 <= last && j0 + KSTEP > lo) {
+        FusedQRow<DK, WEIGHTS> qrow;
+        typename FusedQRow<DK, WEIGHTS>::Table tab;
+        qrow.load(q_head, f.q_weight, f.weight_dtype);
+        FusedQRow<DK, WEIGHTS>::load_table(tab, f, tok);
+        const bool k_second = r16 / 8 != 0, v_second = c / 2 != 0;
+        const int64_t base0 = (int64_t)page0 * page_stride, base1 = (int64_t)page1 * page_stride;
+        const int off0 = j0_seen - p0 * P, off1 = j1 - p1 * P;
+        const bf16_t* kp = kv_layer + (k_second ? base1 : base0) + ((int64_t)kvh * P + (k_second ? off1 : off0)) * D + 8 * c;
+        const bf16_t* vp = kv_layer + (v_second ? base1 : base0) + ((int64_t)(nkv + kvh) * D + r16) * P +
+                           (v_second ? off1 : off0) + 8 * (c % 2);
+        StepOperands<DK> op;  // (laid out as KEY_OF_ROW says)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks) op.k[x][ks] = *(const bf16x8*)(kp + (KEY_OF_ROW(r16, x) % 16) * D + 32 * ks);
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n) op.v[n] = *(const bf16x8*)(vp + (int64_t)16 * n * P);
+        bf16x8 qv[DK];
+        qrow.finish(qv, tab, f, f.q_weight != nullptr);
+        f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks) sc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op.k[x][ks], qv[ks], sc[x], 0, 0, 0);
+        const int pos = fresh ? last - 1 : last;  // the last key that comes from the pages
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = sc[i / 4][i % 4] * scale_log2;
+        if (j0 < lo || j0 + KSTEP - 1 > pos) {  // (the same for the whole wavefront)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int j = j0 + 8 * c + i;
+                if (j < lo || j > pos) x[i] = NEG_BIG;
+            }
+        }
+        top = column_max(max_of_8(x));
+        const float base = top <= NEG_BIG ? 0.f : top;  // (no key is seen where the new token is the wavefront's first one)
+        bf16x8 pb;
+        float sum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float p = __builtin_amdgcn_exp2f(x[i] - base);
+            sum[i % 2] += p;
+            pb[i] = (bf16_t)p;
+        }
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n)
+            o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op.v[n], pb, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        l = column_sum(sum[0] + sum[1]);
+    } else if (wave == SHORT_WAVES && fresh) {
+        const bf16_t* k_head = qkv + (int64_t)(nkv * G + kvh) * D;
+        const bf16_t* v_head = k_head + (int64_t)nkv * D;
+        FusedQRow<DK, WEIGHTS> qrow, krow;
+        typename FusedQRow<DK, WEIGHTS>::Table tab;
+        krow.load(k_head, f.k_weight, f.weight_dtype);
+        FusedQRow<DK, WEIGHTS>::load_table(tab, f, tok);
+        qrow.load(q_head, f.q_weight, f.weight_dtype);
+        bf16x4 v[2 * DK];
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n) v[n] = *(const bf16x4*)(v_head + 16 * n + 4 * c);
+        bf16x8 kv[DK], qv[DK];
+        krow.finish(kv, tab, f, f.k_weight != nullptr);
+        const int page = pages.of(slot), off = slot - page * P;
+        bf16_t* base = kv_layer + (int64_t)page * page_stride;
+        if (r16 == 0) {
+            bf16_t* kdst = base + ((int64_t)kvh * P + off) * D + 8 * c;
+            bf16_t* vdst = base + ((int64_t)(nkv + kvh) * D + 4 * c) * P + off;
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks) *(bf16x8*)(kdst + 32 * ks) = kv[ks];
+#pragma unroll
+            for (int n = 0; n < 2 * DK; ++n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) vdst[(int64_t)(16 * n + i) * P] = v[n][i];
+        }
+        qrow.finish(qv, tab, f, f.q_weight != nullptr);
+        float dot[2] = {0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < DK; ++ks)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dot[i % 2] = fmaf((float)kv[ks][i], (float)qv[ks][i], dot[i % 2]);
+        top = column_sum(dot[0] + dot[1]) * scale_log2;
+        l = 1.f;
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[n][i] = (float)v[n][i];
+    } else {
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (r16 < G) {
+#pragma unroll
+        for (int n = 0; n < 2 * DK; ++n) *(f32x4*)(smem + (wave * G + r16) * D + 16 * n + 4 * c) = o[n];
+    }
+    if (c == 0) {
+        s_m[wave * 16 + r16] = top;
+        s_l[wave * 16 + r16] = l;
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < G * D; idx += WAVES * LLE_WAVE) {
+        const int r = idx / D;
+        float m[WAVES], big = NEG_BIG;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            m[w] = s_m[w * 16 + r];
+            big = fmaxf(big, m[w]);
+        }
+        float num = 0.f, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float e = __builtin_amdgcn_exp2f(m[w] - big);
+            num = fmaf(smem[w * G * D + idx], e, num);
+            den = fmaf(s_l[w * 16 + r], e, den);
+        }
+        out[((int64_t)tok * (nkv * G) + kvh * G) * D + idx] = (bf16_t)(num / den);
     }
 }
 
@@ -909,7 +1094,7 @@ __global__ __launch_bounds__(LLE_WAVE) void mfma_combine_kernel(const float* __r
     const int h = blockIdx.y;
     int nsplit = nsplit_decode;
     if (nsplit_decode != nsplit_prefill) {
-        const int s = token_seq[tok];
+        const int s = token_seq ? token_seq[tok] : (int)tok;
         if ((cu_tokens[s + 1] - cu_tokens[s]) * (nq / nkv) > 16) nsplit = nsplit_prefill;
     }
     if (nsplit <= 1) return;
@@ -1491,8 +1676,7 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
             x[e] = (j < lo[t] || j > pos[t]) ? NEG_BIG : score;
         }
         float top = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-        top = fmaxf(top, __shfl_xor(top, 16, LLE_WAVE));
-        top = fmaxf(top, __shfl_xor(top, 32, LLE_WAVE));
+        top = column_max(top);
         const float new_m = fmaxf(m[t], top);
         // while the row has seen no key new_m is NEG_BIG as its masked scores are, and
         // exp2(0) = 1 would count them: shift such rows so that they give 0
@@ -1567,8 +1751,7 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     }
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        l[t] += __shfl_xor(l[t], 16, LLE_WAVE);
-        l[t] += __shfl_xor(l[t], 32, LLE_WAVE);
+        l[t] = column_sum(l[t]);
     }
 
     if (!few) {  // every wavefront writes the rows of its own tiles
@@ -1744,6 +1927,17 @@ static int launch_decode(const bf16_t* q, bf16_t* kv_layer, const int32_t* block
         q, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, out, ws_o, ws_ml, ws_stride, nq, nkv, P,
         page_stride, max_pages, window, scale_log2, fused, sinks, keep_first, cap_log2);
     return 0;
+}
+
+template <int DK, int WEIGHTS>
+static int launch_short_decode(const FusedQKV& f, bf16_t* kv_layer, const int32_t* block_tables, const int32_t* seq_slots,
+                               const int32_t* cu_tokens, const int32_t* kv_lens, bf16_t* out, int S, int nq, int nkv, int P,
+                               int64_t page_stride, int max_pages, int window, float scale_log2, hipStream_t stream) {
+    const int G = nq / nkv;
+    const size_t smem = (size_t)(SHORT_WAVES + 1) * (G * DK * 32 + 2 * 16) * sizeof(float);
+    short_decode_kernel<DK, WEIGHTS><<<dim3(S, nkv), (SHORT_WAVES + 1) * LLE_WAVE, smem, stream>>>(
+        cu_tokens, kv_lens, seq_slots, block_tables, max_pages, P, window, G, nkv, kv_layer, out, page_stride, scale_log2, f);
+    LLE_RETURN_LAUNCH_STATUS();
 }
 
 // A second stream of this library's own (per device, made at first use, default priority) and the
@@ -1929,7 +2123,9 @@ extern "C" int lle_paged_attention_mfma(const void* q, const void* kv_layer, con
 // rotation over the whole head: the q/k norm, the rotation and the write of the new K and V
 // (write_kv != 0; slots [N], < 0: not written) happen inside the attention launch.  qkv is
 // [N, (nq + 2 nkv) * d] as the projection left it; q_weight / k_weight [d] or null; cos_sin
-// [N, d / 2, 2] float32.
+// [N, d / 2, 2] float32.  token_seq null: one token a request.  Then, with no more than SHORT_WAVES * 32 keys a request (`max_kv_len` > 0 is a
+// bound), heads of 64 or 128 and partial results that 64 KB of LDS hold (groups of up to 13 at 128): short_decode_kernel.
+// (`order` serves more keys.)
 extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* slots, const void* q_weight,
                                                  const void* k_weight, int weight_dtype, const void* cos_sin,
                                                  float eps, int write_kv, void* kv_layer, const void* block_tables,
@@ -1937,7 +2133,7 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
                                                  const void* token_seq, void* out, void* ws_o, void* ws_ml, int N,
                                                  int S, int nq, int nkv, int d, int page_size, int64_t page_stride,
                                                  int max_pages, int window, float scale, int nsplit_decode,
-                                                 const void* order, hipStream_t stream) {
+                                                 const void* order, int max_kv_len, hipStream_t stream) {
     if (!qkv || !cos_sin || !slots || d % 64 != 0) return (int)hipErrorInvalidValue;
     if ((q_weight == nullptr) != (k_weight == nullptr)) return (int)hipErrorInvalidValue;
     FusedQKV fused;
@@ -1950,6 +2146,17 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
     fused.eps = eps;
     fused.write_kv = write_kv;
     fused.order = (const int32_t*)order;
+    if (!token_seq && N == S && nsplit_decode == 1 && !order && max_kv_len > 0 && max_kv_len <= SHORT_WAVES * KSTEP && S > 0 && nkv > 0 && nq > 0 &&
+        nq % nkv == 0 && nq / nkv <= 16 && page_size > 0 && page_size % 16 == 0 && S <= 65535 &&
+        (size_t)(SHORT_WAVES + 1) * (nq / nkv * d + 2 * 16) * sizeof(float) <= 64 * 1024) {
+        const float scale_log2 = scale * 1.44269504088896340736f;
+        const bool f32 = weight_dtype == LLE_F32;
+        if (d == 64 || d == 128)
+            return (d == 64 ? (f32 ? launch_short_decode<2, LLE_F32> : launch_short_decode<2, LLE_BF16>)
+                            : (f32 ? launch_short_decode<4, LLE_F32> : launch_short_decode<4, LLE_BF16>))(
+                fused, (bf16_t*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
+                (const int32_t*)kv_lens, (bf16_t*)out, S, nq, nkv, page_size, page_stride, max_pages, window, scale_log2, stream);
+    }
     return paged_attention_mfma(nullptr, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, token_seq, out, ws_o,
                                 ws_ml, N, S, nq, nkv, d, page_size, page_stride, max_pages, window, scale, 1,
                                 nsplit_decode, 0, 1, 1, 0, fused, nullptr, 0, 0.f, stream);

@@ -696,18 +696,21 @@ class HipOps:
         """qk_norm_rope_write and paged_attention of a decode step in one launch (see
         can_fuse_rope_attention): the workgroup whose keys include a new token's position writes
         its K and V, every workgroup norms and rotates the q rows it multiplies.  `order` (int32 [S], or None):
-        the requests in the order in which they are started, see decode_order."""
+        the requests in the order in which they are started, see decode_order.  `max_kv_len`: a host-side bound; it chooses the
+        kernel and its key splits, never the result.  `token_seq` None: every request has one token."""
         _dev(qkv, "qkv", torch.bfloat16)
         _dev(kv_layer, "kv_layer", torch.bfloat16)
         _dev(cos_sin, "cos_sin", torch.float32)
         for t, name in ((slots, "slots"), (block_table, "block_table"), (seq_slots, "seq_slots"),
-                        (cu_tokens, "cu_tokens"), (kv_lens, "kv_lens"), (token_seq, "token_seq")):
+                        (cu_tokens, "cu_tokens"), (kv_lens, "kv_lens")):
             _dev(t, name, torch.int32)
+        if token_seq is not None:
+            _dev(token_seq, "token_seq", torch.int32)
         N = qkv.shape[0]
         page_size = kv_layer.shape[3]
         _need(qkv.shape[1] == (nq + 2 * nkv) * d, "qkv must be [N, (nq + 2 nkv) * d]")
         _need(tuple(kv_layer.shape[1:]) == (2, nkv, page_size, d), "kv_layer must be [pages, 2, nkv, page_size, d]")
-        _need(slots.shape == (N,) and token_seq.shape == (N,), "slots and token_seq must be [N]")
+        _need(slots.shape == (N,) and (token_seq is None or token_seq.shape == (N,)), "slots and token_seq must be [N]")
         _need(cos_sin.shape == (N, d // 2, 2), f"cos_sin must be [{N}, {d // 2}, 2]")
         _need((q_weight is None) == (k_weight is None), "q and k norm weights come together")
         wcode = 0
@@ -718,6 +721,7 @@ class HipOps:
             wcode = dtype_code(q_weight.dtype)
         S = seq_slots.shape[0]
         _need(cu_tokens.shape == (S + 1,) and kv_lens.shape == (S,), "cu_tokens [S + 1], kv_lens [S]")
+        _need(token_seq is not None or N == S, "without token_seq every request has one token")
         _need(nq % nkv == 0 and d % 64 == 0 and page_size % 16 == 0 and S <= 65535,
               "the fused decode attention does not take these sizes")
         if order is not None:
@@ -732,11 +736,11 @@ class HipOps:
             ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=qkv.device)
         self._run("attention", "lle_qk_norm_rope_attention_decode",
                   [_P, _P, _P, _P, _I, _P, _F, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I,
-                   _F, _I, _P, _P],
+                   _F, _I, _P, _I, _P],
                   _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wcode, _ptr(cos_sin), float(eps),
                   int(bool(write_kv)), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens),
                   _ptr(kv_lens), _ptr(token_seq), _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size,
-                  kv_layer.stride(0), block_table.shape[1], win, float(scale), ns, _ptr(order))
+                  kv_layer.stride(0), block_table.shape[1], win, float(scale), ns, _ptr(order), int(max_kv_len))
         return out
 
     # Keys that a workgroup of the decode kernel asks for at its start (two steps of 32 for each of four wavefronts): up to so many

@@ -120,7 +120,7 @@ class PagedAttention(Mixer):
                 a = ops.qk_norm_rope_attention(
                     qkv, group.slot_mapping, self.q_norm_w, self.k_norm_w, cos_sin, eps, cache.kv, self.nq,
                     self.nkv, self.d, cache.writes, group.block_table, step.seq_slots, step.cu_tokens,
-                    step.kv_lens, step.token_seq, self.window, self.scale, step.max_kv_len, order,
+                    step.kv_lens, None if step.max_q_len == 1 else step.token_seq, self.window, self.scale, step.max_kv_len, order,
                 )
                 return self.o.forward(a, fold=fold)
             q = ops.qk_norm_rope_write(

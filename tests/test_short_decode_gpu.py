@@ -1,0 +1,61 @@
+"""Decode steps of up to 256 keys a request: the launch with a wavefront for every 32 keys and one for the new token."""
+import pytest
+import torch
+
+from tests.test_kernels_gpu import attention_case, ops, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+# a request's first token, the edges of halves, steps and pages, the most keys that the launch takes; beyond them the general
+# one.  In each list one token's place is not written (slot -1): it attends to what the page holds.
+@pytest.mark.parametrize("lens", [[1, 2, 15, 16, 17], [31, 32, 33, 64, 97], [255, 256, 160, 1], [257, 40]])
+@pytest.mark.parametrize("nq,nkv,d,P,window", [(16, 8, 128, 16, None), (8, 8, 64, 48, None), (13, 1, 128, 32, 40), (14, 1, 128, 16, None),
+                                               (32, 2, 64, 16, 17), (4, 4, 128, 64, 1)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32, None])
+def test_short_decode_equals_its_two_halves(wdtype, nq, nkv, d, P, window, lens):
+    requests = [(n - 1, 1) for n in lens]
+    args, mq, mk = attention_case(torch.bfloat16, nq, nkv, d, P, window, requests,
+                                  pages=sum(-(-n // P) for n in lens) + 3, max_pages=-(-max(lens) // P) + 1)
+    _, kv, table, seq_slots, cu, kv_lens, token_seq, _, scale = args
+    S = len(lens)
+    qkv = rnd((S, (nq + 2 * nkv) * d), torch.bfloat16, 70, 1.5)
+    slots = torch.tensor([int(table[int(seq_slots[s]), (n - 1) // P]) * P + (n - 1) % P for s, n in enumerate(lens)], dtype=torch.int32)
+    slots[1] = -1
+    slots = slots.cuda()
+    inv = (1e6 ** (-(2.0 * torch.arange(d // 2, dtype=torch.float64)) / d)).float().cuda()
+    o = ops()
+    cs = o.rope_table((kv_lens - 1).int(), inv)
+    qw = kw = None
+    if wdtype is not None:
+        qw, kw = ((1 + 0.2 * rnd((d,), torch.float32, seed)).to(wdtype) for seed in (71, 72))
+    a, b = kv.clone(), kv.clone()
+    q = o.qk_norm_rope_write(qkv, slots, qw, kw, cs, d, 1e-5, a, nq, nkv, d, True)
+    want = o.paged_attention(q, a, table, seq_slots, cu, kv_lens, token_seq, window, scale, *mq, mk).double()
+    run = lambda pool, write: o.qk_norm_rope_attention(qkv, slots, qw, kw, cs, 1e-5, pool, nq, nkv, d, write, table, seq_slots, cu, kv_lens,
+                                                       None, window, scale, mk).double()
+    got = run(b, True)
+    # both round the same 32-bit results to bfloat16: a key may be one unit in the last place off where a product was fused differently
+    assert not torch.equal(b, kv) and (a.float() - b.float()).abs().max() <= 2.0 ** -7 * a.float().abs().max()
+    # weights in bfloat16 (2^-9 relative each) on values of size 4 at most, rounded once more
+    assert (got - want).abs().max() < 2e-2
+    c = a.clone()
+    assert (run(c, False) - want).abs().max() < 2e-2 and torch.equal(c, a)
+
+
+def test_a_request_without_a_token_is_left_alone():
+    """Three requests, the second with no token in this step: the others' rows are theirs."""
+    args, mq, mk = attention_case(torch.bfloat16, 4, 2, 64, 16, None, [(20, 1), (40, 1)])
+    _, kv, table, seq_slots, _, kv_lens, _, _, scale = args
+    o = ops()
+    qkv = rnd((2, 8 * 64), torch.bfloat16, 5)
+    cs = o.rope_table((kv_lens - 1).int(), torch.ones(32, device="cuda"))
+    slots = torch.full((2,), -1, dtype=torch.int32, device="cuda")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    run = lambda s, cu, lens, seq: o.qk_norm_rope_attention(qkv, slots, None, None, cs, 1e-5, kv, 4, 2, 64, True, table, s, cu, lens, seq, None, scale, mk)
+    want = run(seq_slots, i32([0, 1, 2]), kv_lens, None)
+    three = lambda x: torch.stack([x[0], x[0], x[1]])
+    got = run(three(seq_slots), i32([0, 1, 1, 2]), three(kv_lens), i32([0, 2]))
+    assert (got.double() - want.double()).abs().max() < 2e-2
+    with pytest.raises(Exception, match="one token"):
+        run(three(seq_slots), i32([0, 1, 1, 2]), three(kv_lens), None)
