@@ -33,6 +33,7 @@ LIBRARIES: Dict[str, List[str]] = {
     "gemm": ["gemm.hip"],
     "gemm_f32": ["gemm_f32.hip"],
     "gemm_tile": ["gemm_tile.hip"],
+    "gemm_wide": ["gemm_wide.hip"],
     "sampling": ["sampling.hip"],
     "recurrent": ["recurrent.hip"],
     "latent": ["latent.hip"],
@@ -54,6 +55,7 @@ OWN_HEADERS: Dict[str, List[str]] = {
     "gemm": ["lds.h"],
     "gemm_f32": ["lds.h"],
     "gemm_tile": ["lds.h"],
+    "gemm_wide": ["lds.h"],
 }
 # packed 32-bit float instructions are switched off on purpose (device flag); the first kernel
 # arguments come preloaded into scalar registers with the dispatch instead of being loaded by the
