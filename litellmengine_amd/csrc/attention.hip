@@ -563,6 +563,10 @@ struct FusedQKV {
     float eps;
     int write_kv;
     const int32_t* order;   // the requests, longest first (lle_decode_order), or nullptr: as they come
+    // short_decode_kernel, PAIRS: a row of qkv has `cols` columns (q, k, v, others), no norms; the first `rot` elements (a multiple
+    // of 8) of every q and k head turn in neighbouring pairs by cos_sin [N, rot / 2, 2].  CAP: see tile_step.
+    int cols, rot;
+    float cap_log2;
 };
 
 // Eight consecutive norm weights (float32 or bfloat16) as they lie in memory; what they mean is
@@ -627,6 +631,34 @@ struct FusedQRow {
             const float4* t = (const float4*)(f.cos_sin + (tok * (D / 2) + 32 * ks + 8 * c) * 2);
 #pragma unroll
             for (int i = 0; i < 4; ++i) tab[ks][i] = t[i];
+        }
+    }
+
+    // PAIRS: elements that turn come eight at a time (the others read what is there and are left as they are)
+    static __device__ __forceinline__ void load_pair_table(Table& tab, const FusedQKV& f, int64_t tok) {
+        const int c = (threadIdx.x % LLE_WAVE) / 16;
+        if (f.rot <= 0) return;  // (the same for the whole launch)
+#pragma unroll
+        for (int ks = 0; ks < DK; ++ks) {
+            const float4* t = (const float4*)(f.cos_sin + tok * f.rot + min(32 * ks + 8 * c, f.rot - 8));
+            tab[ks / 2][2 * (ks % 2)] = t[0];
+            tab[ks / 2][2 * (ks % 2) + 1] = t[1];
+        }
+    }
+    __device__ __forceinline__ void finish_pairs(bf16x8 (&qv)[DK], const Table& tab, const FusedQKV& f) const {
+        const int c = (threadIdx.x % LLE_WAVE) / 16;
+#pragma unroll
+        for (int ks = 0; ks < DK; ++ks) {
+            const float4 t0 = tab[ks / 2][2 * (ks % 2)], t1 = tab[ks / 2][2 * (ks % 2) + 1];
+            const float cs[4] = {t0.x, t0.z, t1.x, t1.z}, sn[4] = {t0.y, t0.w, t1.y, t1.w};
+            bf16x8 turned;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float a = (float)raw[ks][2 * i], b = (float)raw[ks][2 * i + 1];
+                turned[2 * i] = (bf16_t)(a * cs[i] - b * sn[i]);
+                turned[2 * i + 1] = (bf16_t)(b * cs[i] + a * sn[i]);
+            }
+            qv[ks] = 32 * ks + 8 * c < f.rot ? turned : raw[ks];
         }
     }
 
@@ -907,7 +939,15 @@ __global__ __launch_bounds__(DEC_WAVES* LLE_WAVE) void mfma_decode_kernel(
 // 0.6B sizes (16 q heads, 8 kv heads of 128) at 97 keys, 1 / 8 / 32 requests: 7.9 / 8.1 / 9.7 us in mfma_decode_kernel, whose
 // loop holds two steps and whose new token goes through the page, 6.1 / 6.5 / 8.0 here.
 #define SHORT_WAVES 8
-template <int DK, int WEIGHTS>
+// a score in the base-2 domain (CAP as in tile_step)
+template <bool CAP>
+__device__ __forceinline__ float short_score(float s, float scale_log2, float cap_log2) {
+    if constexpr (CAP) return fmaf(-2.f * cap_log2, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s * scale_log2)), cap_log2);
+    return s * scale_log2;
+}
+// PAIRS, CAP: what FusedQKV says.  Rorevik's attention (16 q heads, 4 kv heads of 128, capped scores) at 8 requests of 100 keys:
+// OLD_PAIRS us in two launches, NEW_PAIRS here.
+template <int DK, int WEIGHTS, bool PAIRS, bool CAP>
 __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_kernel(
     const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ seq_slots,
     const int32_t* __restrict__ block_tables, int max_pages, int P, int window, int G, int nkv, bf16_t* kv_layer,
@@ -935,15 +975,16 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
     const int32_t* table = block_tables + (int64_t)seq_slot * max_pages;
     const int page0 = table[p0], page1 = table[p1], slot = f.slots[tok];
     const bool fresh = f.write_kv && slot >= 0;  // (else the new token's place holds what the page does)
-    const bf16_t* qkv = f.qkv + (int64_t)tok * (nkv * (G + 2)) * D;
+    const bf16_t* qkv = f.qkv + (int64_t)tok * (PAIRS ? f.cols : nkv * (G + 2) * D);
     const bf16_t* q_head = qkv + (int64_t)(kvh * G + min(r16, G - 1)) * D;  // (rows past the group's: dropped at the end)
     f32x4 o[2 * DK];
     float top = NEG_BIG, l = 0.f;
     if (wave < SHORT_WAVES && j0 <= last && j0 + KSTEP > lo) {
         FusedQRow<DK, WEIGHTS> qrow;
         typename FusedQRow<DK, WEIGHTS>::Table tab;
-        qrow.load(q_head, f.q_weight, f.weight_dtype);
-        FusedQRow<DK, WEIGHTS>::load_table(tab, f, tok);
+        qrow.load(q_head, PAIRS ? nullptr : f.q_weight, f.weight_dtype);
+        if constexpr (PAIRS) qrow.load_pair_table(tab, f, tok);
+        else qrow.load_table(tab, f, tok);
         const bool k_second = r16 / 8 != 0, v_second = c / 2 != 0;
         const int64_t base0 = (int64_t)page0 * page_stride, base1 = (int64_t)page1 * page_stride;
         const int off0 = j0_seen - p0 * P, off1 = j1 - p1 * P;
@@ -958,7 +999,8 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
 #pragma unroll
         for (int n = 0; n < 2 * DK; ++n) op.v[n] = *(const bf16x8*)(vp + (int64_t)16 * n * P);
         bf16x8 qv[DK];
-        qrow.finish(qv, tab, f, f.q_weight != nullptr);
+        if constexpr (PAIRS) qrow.finish_pairs(qv, tab, f);
+        else qrow.finish(qv, tab, f, f.q_weight != nullptr);
         f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int x = 0; x < 2; ++x)
@@ -967,7 +1009,7 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
         const int pos = fresh ? last - 1 : last;  // the last key that comes from the pages
         float x[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = sc[i / 4][i % 4] * scale_log2;
+        for (int i = 0; i < 8; ++i) x[i] = short_score<CAP>(sc[i / 4][i % 4], scale_log2, f.cap_log2);
         if (j0 < lo || j0 + KSTEP - 1 > pos) {  // (the same for the whole wavefront)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -994,14 +1036,16 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
         const bf16_t* v_head = k_head + (int64_t)nkv * D;
         FusedQRow<DK, WEIGHTS> qrow, krow;
         typename FusedQRow<DK, WEIGHTS>::Table tab;
-        krow.load(k_head, f.k_weight, f.weight_dtype);
-        FusedQRow<DK, WEIGHTS>::load_table(tab, f, tok);
-        qrow.load(q_head, f.q_weight, f.weight_dtype);
+        krow.load(k_head, PAIRS ? nullptr : f.k_weight, f.weight_dtype);
+        if constexpr (PAIRS) krow.load_pair_table(tab, f, tok);
+        else krow.load_table(tab, f, tok);
+        qrow.load(q_head, PAIRS ? nullptr : f.q_weight, f.weight_dtype);
         bf16x4 v[2 * DK];
 #pragma unroll
         for (int n = 0; n < 2 * DK; ++n) v[n] = *(const bf16x4*)(v_head + 16 * n + 4 * c);
         bf16x8 kv[DK], qv[DK];
-        krow.finish(kv, tab, f, f.k_weight != nullptr);
+        if constexpr (PAIRS) krow.finish_pairs(kv, tab, f);
+        else krow.finish(kv, tab, f, f.k_weight != nullptr);
         const int page = pages.of(slot), off = slot - page * P;
         bf16_t* base = kv_layer + (int64_t)page * page_stride;
         if (r16 == 0) {
@@ -1014,13 +1058,14 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
 #pragma unroll
                 for (int i = 0; i < 4; ++i) vdst[(int64_t)(16 * n + i) * P] = v[n][i];
         }
-        qrow.finish(qv, tab, f, f.q_weight != nullptr);
+        if constexpr (PAIRS) qrow.finish_pairs(qv, tab, f);
+        else qrow.finish(qv, tab, f, f.q_weight != nullptr);
         float dot[2] = {0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < DK; ++ks)
 #pragma unroll
             for (int i = 0; i < 8; ++i) dot[i % 2] = fmaf((float)kv[ks][i], (float)qv[ks][i], dot[i % 2]);
-        top = column_sum(dot[0] + dot[1]) * scale_log2;
+        top = short_score<CAP>(column_sum(dot[0] + dot[1]), scale_log2, f.cap_log2);
         l = 1.f;
 #pragma unroll
         for (int n = 0; n < 2 * DK; ++n)
@@ -1929,13 +1974,13 @@ static int launch_decode(const bf16_t* q, bf16_t* kv_layer, const int32_t* block
     return 0;
 }
 
-template <int DK, int WEIGHTS>
+template <int DK, int WEIGHTS, bool PAIRS = false, bool CAP = false>
 static int launch_short_decode(const FusedQKV& f, bf16_t* kv_layer, const int32_t* block_tables, const int32_t* seq_slots,
                                const int32_t* cu_tokens, const int32_t* kv_lens, bf16_t* out, int S, int nq, int nkv, int P,
                                int64_t page_stride, int max_pages, int window, float scale_log2, hipStream_t stream) {
     const int G = nq / nkv;
     const size_t smem = (size_t)(SHORT_WAVES + 1) * (G * DK * 32 + 2 * 16) * sizeof(float);
-    short_decode_kernel<DK, WEIGHTS><<<dim3(S, nkv), (SHORT_WAVES + 1) * LLE_WAVE, smem, stream>>>(
+    short_decode_kernel<DK, WEIGHTS, PAIRS, CAP><<<dim3(S, nkv), (SHORT_WAVES + 1) * LLE_WAVE, smem, stream>>>(
         cu_tokens, kv_lens, seq_slots, block_tables, max_pages, P, window, G, nkv, kv_layer, out, page_stride, scale_log2, f);
     LLE_RETURN_LAUNCH_STATUS();
 }
@@ -2119,6 +2164,42 @@ extern "C" int lle_paged_attention_mfma(const void* q, const void* kv_layer, con
                                 (const float*)sinks, keep_first, softcap, stream);
 }
 
+// The most keys of a request, and the LDS, of short_decode_kernel.
+extern "C" int lle_short_decode_max_keys(void) { return SHORT_WAVES * KSTEP; }
+static bool short_decode_fits(int S, int nq, int nkv, int d, int page_size, int max_kv_len) {
+    return S > 0 && S <= 65535 && nkv > 0 && nkv <= 65535 && nq > 0 && nq % nkv == 0 && nq / nkv <= 16 && (d == 64 || d == 128) && page_size > 0 &&
+           page_size % 16 == 0 && max_kv_len > 0 && max_kv_len <= SHORT_WAVES * KSTEP &&
+           (size_t)(SHORT_WAVES + 1) * (nq / nkv * d + 2 * 16) * sizeof(float) <= 64 * 1024;
+}
+
+// One token a request (S of them): the rotation of q and k in neighbouring pairs, the write of K and V and the attention of
+// lle_pair_rope_write and lle_paged_attention_mfma in one launch, for heads of 64 or 128 of q, k and v alike without biases.  A row of u
+// has `cols` columns, a multiple of 8: q, k, v, then others.  rot: a multiple of 8 (0: nothing turns); softcap <= 0: none.
+extern "C" int lle_pair_rope_attention_decode(const void* u, int cols, const void* slots, const void* cos_sin, int rot, int write_kv,
+                                              void* kv_layer, const void* block_tables, const void* seq_slots, const void* cu_tokens,
+                                              const void* kv_lens, void* out, int S, int nq, int nkv, int d, int page_size,
+                                              int64_t page_stride, int max_pages, int window, float scale, float softcap, int max_kv_len,
+                                              hipStream_t stream) {
+    if (!short_decode_fits(S, nq, nkv, d, page_size, max_kv_len) || cols % 8 != 0 || cols < (nq + 2 * nkv) * d || rot < 0 || rot % 8 != 0 ||
+        rot > d || (rot > 0 && !cos_sin) || !u || !slots || ((uintptr_t)u & 15))
+        return (int)hipErrorInvalidValue;
+    FusedQKV f = {};
+    f.qkv = (const bf16_t*)u;
+    f.slots = (const int32_t*)slots;
+    f.cos_sin = (const float*)cos_sin;
+    f.write_kv = write_kv;
+    f.cols = cols;
+    f.rot = rot;
+    constexpr float LOG2E = 1.44269504088896340736f;
+    const bool cap = softcap > 0.f;
+    f.cap_log2 = cap ? softcap * LOG2E : 0.f;
+    const float scale_log2 = cap ? 2.f * LOG2E * scale / softcap : scale * LOG2E;
+    return (d == 64 ? (cap ? launch_short_decode<2, LLE_BF16, true, true> : launch_short_decode<2, LLE_BF16, true, false>)
+                    : (cap ? launch_short_decode<4, LLE_BF16, true, true> : launch_short_decode<4, LLE_BF16, true, false>))(
+        f, (bf16_t*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens, (const int32_t*)kv_lens,
+        (bf16_t*)out, S, nq, nkv, page_size, page_stride, max_pages, window, scale_log2, stream);
+}
+
 // Decode steps only (every request has at most 16 / group tokens), head_dim a multiple of 64, a
 // rotation over the whole head: the q/k norm, the rotation and the write of the new K and V
 // (write_kv != 0; slots [N], < 0: not written) happen inside the attention launch.  qkv is
@@ -2136,7 +2217,7 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
                                                  const void* order, int max_kv_len, hipStream_t stream) {
     if (!qkv || !cos_sin || !slots || d % 64 != 0) return (int)hipErrorInvalidValue;
     if ((q_weight == nullptr) != (k_weight == nullptr)) return (int)hipErrorInvalidValue;
-    FusedQKV fused;
+    FusedQKV fused = {};
     fused.qkv = (const bf16_t*)qkv;
     fused.slots = (const int32_t*)slots;
     fused.q_weight = q_weight;
@@ -2146,15 +2227,12 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
     fused.eps = eps;
     fused.write_kv = write_kv;
     fused.order = (const int32_t*)order;
-    if (!token_seq && N == S && nsplit_decode == 1 && !order && max_kv_len > 0 && max_kv_len <= SHORT_WAVES * KSTEP && S > 0 && nkv > 0 && nq > 0 &&
-        nq % nkv == 0 && nq / nkv <= 16 && page_size > 0 && page_size % 16 == 0 && S <= 65535 &&
-        (size_t)(SHORT_WAVES + 1) * (nq / nkv * d + 2 * 16) * sizeof(float) <= 64 * 1024) {
+    if (!token_seq && N == S && nsplit_decode == 1 && !order && short_decode_fits(S, nq, nkv, d, page_size, max_kv_len)) {
         const float scale_log2 = scale * 1.44269504088896340736f;
         const bool f32 = weight_dtype == LLE_F32;
-        if (d == 64 || d == 128)
-            return (d == 64 ? (f32 ? launch_short_decode<2, LLE_F32> : launch_short_decode<2, LLE_BF16>)
-                            : (f32 ? launch_short_decode<4, LLE_F32> : launch_short_decode<4, LLE_BF16>))(
-                fused, (bf16_t*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
+        return (d == 64 ? (f32 ? launch_short_decode<2, LLE_F32> : launch_short_decode<2, LLE_BF16>)
+                        : (f32 ? launch_short_decode<4, LLE_F32> : launch_short_decode<4, LLE_BF16>))(
+            fused, (bf16_t*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
                 (const int32_t*)kv_lens, (bf16_t*)out, S, nq, nkv, page_size, page_stride, max_pages, window, scale_log2, stream);
     }
     return paged_attention_mfma(nullptr, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, token_seq, out, ws_o,

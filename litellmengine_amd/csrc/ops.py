@@ -782,6 +782,48 @@ class HipOps:
                   kv_layer.stride(0), block_table.shape[1], win, float(scale), ns, _ptr(order), int(max_kv_len))
         return out
 
+    def can_fuse_pair_rope_attention(self, u, dim: int, vdim: int, rot: int, kv_layer, num_q_heads: int, max_q_len: int, max_kv_len: int,
+                                     num_seqs: int) -> bool:
+        """Whether pair_rope_attention takes this step: bfloat16, one token a request and few keys, heads of 64 or 128 of q, k, v
+        and cache alike."""
+        D, nkv, page_size = kv_layer.shape[4], kv_layer.shape[2], kv_layer.shape[3]
+        return (u.dtype == torch.bfloat16 and max_q_len == 1 and u.shape[0] == num_seqs and 0 < max_kv_len <= self.short_decode_max_keys()
+                and dim == vdim == D and D in (64, 128) and rot % 8 == 0 and u.shape[1] % 8 == 0 and u.data_ptr() % 16 == 0
+                and page_size % 16 == 0 and num_q_heads // nkv * D * 36 + 1152 <= 65536 and num_q_heads // nkv <= 16 and num_seqs <= 65535
+                and not self.force_generic_attention and not self.force_separate_rope)
+
+    def short_decode_max_keys(self) -> int:
+        return self._get("attention", "lle_short_decode_max_keys", [])()
+
+    def pair_rope_attention(self, u, slots, cos_sin, kv_layer, nq: int, nkv: int, d: int, write_kv: bool, block_table, seq_slots, cu_tokens,
+                            kv_lens, window: Optional[int], scale: float, max_kv_len: int, softcap: Optional[float] = None) -> torch.Tensor:
+        """pair_rope_write (without biases and value rotation) and paged_attention of a decode step in one launch, see
+        can_fuse_pair_rope_attention: u [S, cols] holds q, k, v and columns that are left alone -> [S, nq * d]."""
+        _dev(u, "u", torch.bfloat16)
+        _dev(kv_layer, "kv_layer", torch.bfloat16)
+        for t, name in ((slots, "slots"), (block_table, "block_table"), (seq_slots, "seq_slots"), (cu_tokens, "cu_tokens"),
+                        (kv_lens, "kv_lens")):
+            _dev(t, name, torch.int32)
+        S, cols = u.shape
+        page_size = kv_layer.shape[3]
+        _need(cols >= (nq + 2 * nkv) * d, "u has too few columns")
+        _need(tuple(kv_layer.shape[1:]) == (2, nkv, page_size, d), "kv_layer must be [pages, 2, nkv, page_size, d]")
+        _need(slots.shape == (S,) and seq_slots.shape == (S,) and cu_tokens.shape == (S + 1,) and kv_lens.shape == (S,),
+              "slots, seq_slots, kv_lens [S], cu_tokens [S + 1]")
+        _need(block_table.dim() == 2, "block_table must be [slots, pages]")
+        rot = 0
+        if cos_sin is not None:
+            _dev(cos_sin, "cos_sin", torch.float32)
+            rot = 2 * cos_sin.shape[1]
+            _need(cos_sin.shape == (S, rot // 2, 2) and rot <= d, "cos_sin must be [S, pairs, 2]")
+        out = torch.empty((S, nq * d), dtype=torch.bfloat16, device=u.device)
+        self._run("attention", "lle_pair_rope_attention_decode",
+                  [_P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _F, _I, _P],
+                  _ptr(u), cols, _ptr(slots), _ptr(cos_sin), rot, int(bool(write_kv)), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots),
+                  _ptr(cu_tokens), _ptr(kv_lens), _ptr(out), S, nq, nkv, d, page_size, kv_layer.stride(0), block_table.shape[1],
+                  int(window) if window else 0, float(scale), float(softcap) if softcap else 0.0, int(max_kv_len))
+        return out
+
     # Keys that a workgroup of the decode kernel asks for at its start (two steps of 32 for each of four wavefronts): up to so many
     # the longest request takes about as long as the shortest and an order is only one more thing to wait for.  (64 requests,
     # 8 key heads, as they come / longest first: of 64 to 256 keys 19.0 / 19.5 us, of 96 to 384 23.9 / 23.0, of 256 to 1024

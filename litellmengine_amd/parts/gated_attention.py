@@ -138,6 +138,14 @@ class GatedAttention(Mixer):
         u = self.qkvg.forward(x) if projected is None else projected[0]
         turn = None if self.rotation is None else self.rotation.table(step)
         value_turn = None if self.value_rotation is None else self.value_rotation.table(step)
+        fits = getattr(ops, "can_fuse_pair_rope_attention", None)  # (operations may go without that launch)
+        if (fits is not None and self.bias is None and value_turn is None and not self.talking and self.sinks is None
+                and not self.keep_first and fits(u, self.dim, self.vdim, 0 if turn is None else 2 * turn.shape[1], cache.kv, self.nq,
+                                                 step.max_q_len, step.max_kv_len, step.seq_slots.shape[0])):
+            a = ops.pair_rope_attention(u, group.slot_mapping, turn, cache.kv, self.nq, self.nkv, self.dim, cache.writes,
+                                        group.block_table, step.seq_slots, step.cu_tokens, step.kv_lens, self.window, self.scale,
+                                        step.max_kv_len, self.softcap)
+            return self._out(a, u, value_turn)
         q = ops.pair_rope_write(u, self.bias, group.slot_mapping, turn, value_turn, cache.kv, self.nq, self.nkv, self.dim,
                                 self.vdim, cache.writes)
         where = (cache.kv, group.block_table, step.seq_slots, step.cu_tokens, step.kv_lens, step.token_seq)
@@ -147,6 +155,10 @@ class GatedAttention(Mixer):
         else:
             a = ops.paged_attention(q, *where, self.window, self.scale, step.min_q_len, step.max_q_len, step.max_kv_len,
                                     sinks=self.sinks, keep_first=self.keep_first, softcap=self.softcap)
+        return self._out(a, u, value_turn)
+
+    def _out(self, a, u, value_turn):
+        ops = self.ctx.ops
         if not self.gated:  # heads of cache_dim elements, zeros past vdim, against zero columns of the weight
             return self.o.forward(a)
         return self.o.forward(ops.turn_back_gate(a, u, self.gate_col, self.nq, self.vdim, value_turn, self.out_scale))

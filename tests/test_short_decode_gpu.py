@@ -59,3 +59,32 @@ def test_a_request_without_a_token_is_left_alone():
     assert (got.double() - want.double()).abs().max() < 2e-2
     with pytest.raises(Exception, match="one token"):
         run(three(seq_slots), i32([0, 1, 1, 2]), three(kv_lens), None)
+
+
+@pytest.mark.parametrize("lens", [[1, 2, 15, 16, 17], [31, 32, 33, 64, 97], [255, 256, 160, 1]])
+@pytest.mark.parametrize("nq,nkv,d,P,window,rot,cap", [(16, 4, 128, 16, None, 64, 30.0), (8, 8, 64, 48, None, 64, None), (13, 1, 128, 32, 40, 8, None),
+                                                       (4, 2, 64, 16, 17, 0, 5.0), (4, 4, 128, 64, 1, 128, None)])
+def test_short_decode_with_pairs_equals_its_two_halves(lens, nq, nkv, d, P, window, rot, cap):
+    """The rotation of neighbouring pairs, capped scores, columns beside q, k and v."""
+    requests = [(n - 1, 1) for n in lens]
+    args, mq, mk = attention_case(torch.bfloat16, nq, nkv, d, P, window, requests,
+                                  pages=sum(-(-n // P) for n in lens) + 3, max_pages=-(-max(lens) // P) + 1)
+    _, kv, table, seq_slots, cu, kv_lens, token_seq, _, scale = args
+    S = len(lens)
+    u = rnd((S, (nq + 2 * nkv) * d + 24), torch.bfloat16, 70, 1.5)
+    slots = torch.tensor([int(table[int(seq_slots[s]), (n - 1) // P]) * P + (n - 1) % P for s, n in enumerate(lens)], dtype=torch.int32)
+    slots[1] = -1
+    slots = slots.cuda()
+    o = ops()
+    cs = o.rope_table((kv_lens - 1).int(), (1e4 ** (-torch.arange(rot // 2, dtype=torch.float64) / 32)).float().cuda()) if rot else None
+    a, b = kv.clone(), kv.clone()
+    q = o.pair_rope_write(u, None, slots, cs, None, a, nq, nkv, d, d, True)
+    want = o.paged_attention(q, a, table, seq_slots, cu, kv_lens, token_seq, window, scale, *mq, mk, softcap=cap).double()
+    assert o.can_fuse_pair_rope_attention(u, d, d, rot, kv, nq, 1, mk, S) and not o.can_fuse_pair_rope_attention(u, d, d, rot, kv, nq, 1, 257, S)
+    run = lambda pool, write: o.pair_rope_attention(u, slots, cs, pool, nq, nkv, d, write, table, seq_slots, cu, kv_lens, window, scale, mk, cap).double()
+    got = run(b, True)
+    # the same 32-bit rotation, rounded once: a unit in the last place where a product was fused differently
+    assert not torch.equal(b, kv) and (a.float() - b.float()).abs().max() <= 2.0 ** -7 * a.float().abs().max()
+    assert (got - want).abs().max() < 2e-2  # (as above)
+    c = a.clone()
+    assert (run(c, False) - want).abs().max() < 2e-2 and torch.equal(c, a)
