@@ -153,7 +153,8 @@ struct NormFold {
     bf16_t* xw;             // RESID: out, [M, N]
     float* ss_out;          // RESID: out, [16][workgroups]
     const float* ss_in;     // SCALED: [16][parts]
-    int parts;              // SCALED
+    int parts;              // SCALED, SPLIT
+    int part_rows;          // SPLIT: columns of a part, all of the tile's or half of them
     float eps;              // SCALED
     // GATED: biases [N] (or null) and with act_limit > 0 the clamped activation instead of silu
     const bf16_t* act_bias;
@@ -175,7 +176,8 @@ __device__ __forceinline__ float gated_result(float g, float u, const NormFold& 
     return g / (1.0f + expf(-g)) * u;
 }
 
-template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL>
+// SPLIT (RESID): the rows of X are dealt out sixteen a workgroup, see lle_gemm_skinny_resid_bf16.
+template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL, bool SPLIT = false>
 // one tile of W and up to 16 rows of X: two workgroups of 16 wavefronts a CU (8 wavefronts a SIMD),
 // which 64 registers allow; the gated form measured faster with the registers it asks for, and the scaled one has no room in
 // 64 for the parts that it asks for at its start (three spilled registers cost a launch 0.9 us)
@@ -203,6 +205,14 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
                  "s"(fold.weight_dtype), "s"(fold.xw), "s"(fold.ss_out), "s"(fold.ss_in), "s"(fold.parts),
                  "s"(fold.eps));
     const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
+    if (SPLIT && blockIdx.y > 0) {
+        const int before = 16 * blockIdx.y;
+        X += (int64_t)before * K;
+        M -= before;
+        fold.hidden += (int64_t)before * N;
+        fold.xw += (int64_t)before * N;
+        fold.ss_out += (int64_t)before * fold.parts;
+    }
     // SCALED: wavefront w adds up the parts of the rows w, w + SK_WAVES, ...  The first parts are asked for now and added after
     // the products.
     constexpr int EARLY_PARTS = 4, SUM_ROWS = (16 * MT + SK_WAVES - 1) / SK_WAVES;
@@ -380,8 +390,14 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
                         (T)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid_w : resid_w << 16));
                     sq = h * h;
                 }
-                sq = row16_sum(sq);
-                if (n == 0) fold.ss_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
+                if (!SPLIT || fold.part_rows == tile_rows) {  // (the same for the whole launch)
+                    sq = row16_sum(sq);
+                    if (n == 0) fold.ss_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
+                } else {
+                    const float first = row16_sum(n < fold.part_rows ? sq : 0.f), second = row16_sum(n < fold.part_rows ? 0.f : sq);
+                    const int part = 2 * blockIdx.x + n;
+                    if (n < 2 && part < fold.parts) fold.ss_out[(int64_t)m * fold.parts + part] = n == 0 ? first : second;
+                }
             }
         }
         return;
@@ -865,7 +881,7 @@ static int skinny_tile_rows(int rows) {
     return per_tile < 1 ? 1 : (per_tile > 16 ? 16 : per_tile);
 }
 
-// tiles of lle_gemm_skinny_resid_bf16 for a weight of N rows: the second size of its ss_part
+// tiles of lle_gemm_skinny_resid_bf16 for a weight of N rows at up to 16 rows of X: the second size of its ss_part
 extern "C" int lle_gemm_skinny_resid_parts(int N) {
     if (N <= 0) return 0;
     const int tr = skinny_tile_rows(N);
@@ -950,12 +966,17 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
     fold.weight_dtype = weight_dtype;
     fold.xw = (bf16_t*)xw;
     fold.ss_out = (float*)ss_part;
-    const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
+    // From 17 rows of X on a workgroup takes sixteen of them and, of a narrow model, tiles of W twice as high (two parts of the sums):
+    // with all 32 rows a workgroup of the 0.6B sizes reads eight times as much X as W, every CU all of X (1024 x 3072: 24 + 196 KB,
+    // so 48 + 98).  1024 x 2048 at 17 / 32 rows 5.9 / 7.2 -> 5.5 / 5.6 us, 1024 x 3072 7.3 / 9.5 -> 7.0 / 7.2.
+    fold.part_rows = skinny_tile_rows(N);
+    fold.parts = (N + fold.part_rows - 1) / fold.part_rows;
+    const int tr = M <= 16 || fold.part_rows > 8 ? fold.part_rows : 2 * fold.part_rows, blocks = (N + tr - 1) / tr;
     if (M <= 16)
         gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
             (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
     else
-        gemm_skinny_kernel<bf16_t, 2, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
+        gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4, true><<<dim3(blocks, 2), 16 * LLE_WAVE, 0, stream>>>(
             (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
     LLE_RETURN_LAUNCH_STATUS();
 }
