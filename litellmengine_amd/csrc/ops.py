@@ -89,7 +89,7 @@ class HipOps:
         self._fn = {}
         self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta) ...
         self._forms_tuning = None  # ... with these numbers
-        self._wide = {}  # by sizes: wide_tile_rows
+        self._wide = {}  # by sizes: wide_form
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives, beyond the order of its sums)
 
     # -- plumbing ---------------------------------------------------------
@@ -340,9 +340,9 @@ class HipOps:
                           _ptr(x), _ptr(weight), _ptr(out), M, N, K, dtype_code(out_dtype))
                 return out
             if out_dtype == torch.bfloat16:
-                tile_rows = self.wide_tile_rows(x, weight, gated=False)
-                if tile_rows:
-                    return self.linear_wide(x, weight, tile_rows)
+                form = self.wide_form(x, weight, gated=False)
+                if form >= 0:
+                    return self.linear_wide(x, weight, form)
             # the library product accumulates in 32-bit and can leave the result so
             return torch.mm(x, weight.t()) if out_dtype == torch.bfloat16 else torch.mm(x, weight.t(), out_dtype=out_dtype)
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
@@ -534,26 +534,28 @@ class HipOps:
             slices -= 1
         return slices if slices > 1 else 0
 
-    def wide_tile_rows(self, x, weight, gated: bool) -> int:
-        """The rows of the tiles in which the tiled product of many rows takes this one (linear_wide), or 0 where the library
-        stays: from the sizes alone, but for operands that do not begin at 16 bytes, which only the library takes."""
+    WIDE_FORMS = 11  # tiles of linear_wide (whole products: 0, 2 and 4 of them)
+
+    def wide_form(self, x, weight, gated: bool) -> int:
+        """In which tiles the tiled product of many rows takes this one (linear_wide), or -1 where the library stays: from the
+        sizes alone, but for operands that do not begin at 16 bytes, which only the library takes."""
         M, K = x.shape
         if M <= 128 or self.force_library_gemm:
-            return 0
+            return -1
         key = (M, weight.shape[0], K, gated)
-        rows = self._wide.get(key)
-        if rows is None:
-            fn = getattr(build.load_library("gemm_wide"), "lle_gemm_wide_tile_rows")
+        form = self._wide.get(key)
+        if form is None:
+            fn = getattr(build.load_library("gemm_wide"), "lle_gemm_wide_form")
             fn.argtypes, fn.restype = [_I, _I, _I, _I], _I
-            rows = int(fn(M, weight.shape[0], K, int(gated)))
+            form = int(fn(M, weight.shape[0], K, int(gated))) - 1
             if len(self._wide) >= 4096:
                 self._wide.clear()
-            self._wide[key] = rows
-        return rows if rows and (x.data_ptr() | weight.data_ptr()) % 16 == 0 else 0
+            self._wide[key] = form
+        return form if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else -1
 
-    def linear_wide(self, x, weight, tile_rows: int, activation: Optional[str] = None, bias=None, limit: float = 0.0) -> torch.Tensor:
-        """x [M, K] . weight [N, K]^T, bfloat16, in tiles of `tile_rows` (256, 192 or 128) rows: [M, N].  `activation`: weight is gate
-        rows and then up rows, the result [M, N / 2] is silu(gate) * up, or ("clamp") what gate_up_clamped says."""
+    def linear_wide(self, x, weight, form: int, activation: Optional[str] = None, bias=None, limit: float = 0.0) -> torch.Tensor:
+        """x [M, K] . weight [N, K]^T, bfloat16, in tiles of that form (see wide_form): [M, N].  `activation`: weight is gate rows
+        and then up rows, the result [M, N / 2] is silu(gate) * up, or ("clamp") what gate_up_clamped says."""
         _dev(x, "x", torch.bfloat16)
         _dev(weight, "weight", torch.bfloat16)
         M, K = x.shape
@@ -565,7 +567,7 @@ class HipOps:
             _need(bias.shape == (N,), "bias must cover the whole weight")
         out = torch.empty((M, N if activation is None else N // 2), dtype=torch.bfloat16, device=x.device)
         self._run("gemm_wide", "lle_gemm_wide_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
-                  float(limit), _ptr(out), M, N, K, (None, "silu", "clamp").index(activation), tile_rows)
+                  float(limit), _ptr(out), M, N, K, (None, "silu", "clamp").index(activation), form)
         return out
 
     def linear_slices(self, x, weight, slices: int) -> torch.Tensor:
@@ -995,7 +997,7 @@ class HipOps:
     def gate_up_silu(self, x, weight) -> torch.Tensor:
         """x [M, K], weight [2 I, K] (gate rows, then up rows) -> silu(x gate^T) * (x up^T), [M, I].
         Few rows run as ONE weight-streaming launch with the activation in its epilogue, many as one tiled launch where
-        wide_tile_rows says so; otherwise the product and silu_mul (in float32 also where _gated_f32_in_one says so)."""
+        wide_form says so; otherwise the product and silu_mul (in float32 also where _gated_f32_in_one says so)."""
         if isinstance(x, Prenormed):
             return self._linear_folded(x, weight, None, gated=True)
         _dev(x, "x")
@@ -1014,9 +1016,9 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
-        tile_rows = self.wide_tile_rows(x, weight, gated=True) if x.dtype == torch.bfloat16 else 0
-        if tile_rows:
-            return self.linear_wide(x, weight, tile_rows, "silu")
+        form = self.wide_form(x, weight, gated=True) if x.dtype == torch.bfloat16 else -1
+        if form >= 0:
+            return self.linear_wide(x, weight, form, "silu")
         return self.silu_mul(self.linear(x, weight))
 
     def _gated_f32_in_one(self, M: int, N2: int, K: int) -> bool:
@@ -1051,9 +1053,9 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_clamped_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(bias), float(limit), _ptr(out), M, N2, K)
             return out
-        tile_rows = self.wide_tile_rows(x, weight, gated=True) if x.dtype == torch.bfloat16 and limit > 0.0 else 0
-        if tile_rows and (bias is None or bias.data_ptr() % 8 == 0):
-            return self.linear_wide(x, weight, tile_rows, "clamp", bias, limit)
+        form = self.wide_form(x, weight, gated=True) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
+        if form >= 0 and (bias is None or bias.data_ptr() % 8 == 0):
+            return self.linear_wide(x, weight, form, "clamp", bias, limit)
         return self.bias_act(self.linear(x, weight), "clamp", True, bias=bias, limit=limit)
 
     # -- arrangements that norm a sublayer's output ------------------------------------
