@@ -946,7 +946,7 @@ __device__ __forceinline__ float short_score(float s, float scale_log2, float ca
     return s * scale_log2;
 }
 // PAIRS, CAP: what FusedQKV says.  Rorevik's attention (16 q heads, 4 kv heads of 128, capped scores) at 8 requests of 100 keys:
-// OLD_PAIRS us in two launches, NEW_PAIRS here.
+// 11.9 us in two launches (rotation and cache write 6.7, attention 5.2), 4.6 here.
 template <int DK, int WEIGHTS, bool PAIRS, bool CAP>
 __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_kernel(
     const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ seq_slots,
