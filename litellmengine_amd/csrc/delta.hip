@@ -283,105 +283,113 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const float* __restric
 
 template <int CTRL>
 __device__ __forceinline__ float delta_lanes(float x) {  // x of the lane that the pattern names
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
 
-// the sum over the 16 lanes of a row, in every one of them (each step adds the same two numbers in both lanes)
+// the sum over the 16 lanes of a column, in every one of them (each step adds the same two numbers in both lanes)
 __device__ __forceinline__ float delta_row_sum(float x) {
-    x += delta_lanes<0xB1>(x);   // neighbours: lanes 1 0 3 2 of every four
-    x += delta_lanes<0x4E>(x);   // lanes 2 3 0 1 of every four
+    x += delta_lanes<0x140>(x);  // the row of sixteen mirrored
     x += delta_lanes<0x141>(x);  // every eight mirrored
-    x += delta_lanes<0x140>(x);  // the sixteen mirrored
+    x += delta_lanes<0x4E>(x);   // lanes 2 3 0 1 of every four
+    x += delta_lanes<0xB1>(x);   // lanes 1 0 3 2 of every four
     return x;
 }
 
-// What a thread reads of one staged token: its share of k and q (CHANNEL: and of the channels' decays), and the
-// token's decay and beta.
+// The same sums for sixteen tokens at once, token t's in lane t: at every step a lane hands the half
+// of its sums that it does not end with to the lane that does, so 15 exchanges do for 16 tokens what 64 do one by one.
+template <int CTRL, int M>
+__device__ __forceinline__ void delta_fold(float (&r)[DELTA_TC], bool upper) {
+#pragma unroll
+    for (int t = 0; t < M; ++t) r[t] = (upper ? r[t + M] : r[t]) + delta_lanes<CTRL>(upper ? r[t] : r[t + M]);
+}
+__device__ __forceinline__ float delta_row_sums(float (&r)[DELTA_TC], int ig) {
+    delta_fold<0x140, 8>(r, ig & 8);
+    delta_fold<0x141, 4>(r, ig & 4);
+    delta_fold<0x4E, 2>(r, ig & 2);
+    delta_fold<0xB1, 1>(r, ig & 1);
+    return r[0];
+}
+
+// What a thread reads of one staged token: its share of k and q (CHANNEL: and of the channels' decays).
 template <int KI, bool CHANNEL>
 struct DeltaToken {
     float kk[KI], qq[KI], gg[CHANNEL ? KI : 1];
-    float g, beta;
 };
 
+template <int N, int STEP = 4>
+__device__ __forceinline__ void delta_copy(float* d, const float* __restrict__ p) {  // N aligned floats, four by four STEP apart
+    typedef float vec __attribute__((ext_vector_type(N < 4 ? N : 4)));
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+        const vec x = *(const vec*)(p + i / 4 * STEP);
+        if constexpr (N == 1) d[0] = ((const float*)p)[0];
+        else
+#pragma unroll
+            for (int e = 0; e < (N < 4 ? N : 4); ++e) d[i + e] = x[e];
+    }
+}
+
+// kt, qt, gt: where the lane's share begins (KI <= 2: q lies right behind k, one load for both)
 template <int KI, bool CHANNEL>
 __device__ __forceinline__ void delta_read(DeltaToken<KI, CHANNEL>& d, const float* __restrict__ kt, const float* __restrict__ qt,
-                                           const float* __restrict__ gt, const float2* __restrict__ par) {
-    if constexpr (CHANNEL) {
-        if (KI % 4 == 0) {
+                                           const float* __restrict__ gt) {
+    if constexpr (CHANNEL) delta_copy<KI, 4 * DELTA_IG>(d.gg, gt);
+    if constexpr (KI <= 2) {
+        float both[2 * KI];
+        delta_copy<2 * KI>(both, kt);
 #pragma unroll
-            for (int ii = 0; ii < KI; ii += 4) {
-                const float4 a = *(const float4*)(gt + ii);
-                d.gg[ii] = a.x, d.gg[ii + 1] = a.y, d.gg[ii + 2] = a.z, d.gg[ii + 3] = a.w;
-            }
-        } else {
-#pragma unroll
-            for (int ii = 0; ii < KI; ++ii) d.gg[ii] = gt[ii];
-        }
-    }
-    if (KI % 4 == 0) {
-#pragma unroll
-        for (int ii = 0; ii < KI; ii += 4) {
-            const float4 a = *(const float4*)(kt + ii), b = *(const float4*)(qt + ii);
-            d.kk[ii] = a.x, d.kk[ii + 1] = a.y, d.kk[ii + 2] = a.z, d.kk[ii + 3] = a.w;
-            d.qq[ii] = b.x, d.qq[ii + 1] = b.y, d.qq[ii + 2] = b.z, d.qq[ii + 3] = b.w;
-        }
+        for (int ii = 0; ii < KI; ++ii) d.kk[ii] = both[ii], d.qq[ii] = both[KI + ii];
     } else {
-#pragma unroll
-        for (int ii = 0; ii < KI; ++ii) {
-            d.kk[ii] = kt[ii];
-            d.qq[ii] = qt[ii];
-        }
+        delta_copy<KI, 4 * DELTA_IG>(d.kk, kt);
+        delta_copy<KI, 4 * DELTA_IG>(d.qq, qt);
     }
-    const float2 pr = *par;
-    d.g = pr.x, d.beta = pr.y;
 }
 
 // One token of the walk for this thread's share of column j: the sum over the key channels, the lanes' exchange, the
-// correction; returns the read-out, which the next token does not wait for.
+// correction; returns the thread's share of the read-out.
 template <int KI, bool CHANNEL>
-__device__ __forceinline__ float delta_token(float (&S)[KI], const DeltaToken<KI, CHANNEL>& d, float v) {
+__device__ __forceinline__ float delta_token(float (&S)[KI], const DeltaToken<KI, CHANNEL>& d, float g, float beta, float v) {
     float p = 0.f, r = 0.f;
-    if constexpr (CHANNEL) {  // the rows of S decay each at their own rate
 #pragma unroll
-        for (int ii = 0; ii < KI; ++ii) {
-            S[ii] *= d.gg[ii];
-            p = fmaf(S[ii], d.kk[ii], p);
-        }
-    } else {
-#pragma unroll
-        for (int ii = 0; ii < KI; ++ii) {
-            S[ii] *= d.g;
-            p = fmaf(S[ii], d.kk[ii], p);
-        }
+    for (int ii = 0; ii < KI; ++ii) {
+        S[ii] *= CHANNEL ? d.gg[ii] : g;  // (CHANNEL: the rows of S decay each at their own rate)
+        p = fmaf(S[ii], d.kk[ii], p);
     }
-    const float w = d.beta * (v - delta_row_sum(p));
+    const float w = beta * (v - delta_row_sum(p));
 #pragma unroll
     for (int ii = 0; ii < KI; ++ii) {
         S[ii] = fmaf(d.kk[ii], w, S[ii]);
         r = fmaf(S[ii], d.qq[ii], r);
     }
-    return delta_row_sum(r);
+    return r;
 }
 
-// grid = (requests, heads, blocks of DELTA_VB value channels).  Thread (jl, ig) = (tid / 16, tid % 16) owns the
-// key channels [ig KI, (ig + 1) KI) of column j = block DELTA_VB + jl.  The tokens pass through LDS DELTA_TC at a
-// time, in two buffers (one for heads over 128 channels): the next chunk goes to LDS and the one behind it is asked for
-// before the current chunk is walked, one barrier a chunk, and inside a chunk every token's operands leave LDS one token
-// ahead of their use.  The read-out is the lane's whose number the token has, so a chunk's leave from the registers.
-// Measured at 2048 tokens of 32 heads of 64 x 64, a decay per channel: 267 us with three barriers a chunk, k . q made
-// ahead of the walk (the read-out taken from the state before the correction, in the same pass) and the read-outs through
-// LDS; 239 us so.  Tried and not kept: all of a chunk's operands in registers before its first token.
+// grid = (requests, heads, blocks of DELTA_VB value channels).  Thread (jl, ig) = (tid / 16, tid % 16) owns KI key channels
+// of column j = block DELTA_VB + jl, four neighbours of every 64 (fewer than four: ig KI + 0 .. KI - 1), so that a wavefront's
+// 16-byte loads of k, q, decays and state lie one beside the other: no bank is asked twice, the state's lines are read whole.
+// The tokens pass through LDS DELTA_TC at a time, in two buffers (one for heads over 128 channels): the next chunk goes to LDS
+// and the one behind it is asked for before the current chunk is walked, one barrier a chunk, and inside a chunk every token's
+// operands leave LDS one token ahead of their use.  The read-outs of a chunk are added over the lanes together, at its end, and
+// leave from the registers, the lane's whose number the token has.
+// What bounds a long walk is the chain of a token (the four exchanges of S^T k and what stands around them, 101 ns) in the
+// two wavefronts that 32 heads of 64 x 64 leave a CU.  Measured with a decay per channel, 32 heads of 64 x 64: 2048 tokens
+// 237 -> 207 us, single tokens of 8 requests 5.0 -> 4.05, of 64 26.0 -> 21.6; one decay a head, 32 heads of 128 x 128: 2048
+// tokens 301 -> 285, single tokens of 8 requests 23.3 -> 10.8, of 32 83.5 -> 34.4; 16 of 256 x 128: 2048 tokens 586 -> 452,
+// single tokens of 32 requests 112 -> 32, against every read-out added up by itself and a thread's channels in one stretch.
+// Tried and not kept: three barriers a chunk and k . q made ahead of the walk; operands read two or three tokens ahead, or all
+// of them at a chunk's start; 32 lanes a column (heads of 64: 265 us, of 256: 381 us, but their single tokens 47).
 template <int KI, bool CHANNEL>
 __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) {
     constexpr int KD = KI * DELTA_IG;
     constexpr int PER = DELTA_TC * KD / DELTA_THREADS;  // elements of q (and of k) of a chunk that a thread fetches
     static_assert(DELTA_TC * KD % DELTA_THREADS == 0, "a chunk's q and k are dealt to the threads in equal shares");
+    static_assert(KI >= 4 || PER < 4, "heads whose k and q lie beside each other are staged one by one");
     static_assert(DELTA_TC == DELTA_IG, "every lane of a column takes one token's read-out");
-    constexpr int BUFS = KI <= 8 ? 2 : 1;
-    __shared__ __attribute__((aligned(16))) float s_q[BUFS][DELTA_TC][KD];
-    __shared__ __attribute__((aligned(16))) float s_k[BUFS][DELTA_TC][KD];
+    constexpr int BUFS = KD <= 128 ? 2 : 1;
+    constexpr bool BOTH = KI <= 2;  // k and q lie lane by lane beside each other
+    __shared__ __attribute__((aligned(16))) float s_kq[BUFS][DELTA_TC][2 * KD];
     __shared__ __attribute__((aligned(16))) float s_g[CHANNEL ? BUFS : 1][CHANNEL ? DELTA_TC : 1][CHANNEL ? KD : 4];
-    __shared__ float2 s_par[BUFS][DELTA_TC];  // (decay, beta) of every staged token
+    __shared__ __attribute__((aligned(16))) float s_par[BUFS][2][DELTA_TC];  // betas, decays of the staged tokens
     __shared__ __attribute__((aligned(16))) float s_v[BUFS][DELTA_VB][DELTA_TC + 4];
     const int s = blockIdx.x, h = blockIdx.y;
     const int tid = threadIdx.x, jl = tid / DELTA_IG, ig = tid % DELTA_IG;
@@ -391,11 +399,20 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
     [[maybe_unused]] const int HD = H * dim;
     const int q0 = a.cu_tokens[s], q1 = a.cu_tokens[s + 1];
     if (q1 <= q0) return;
-    float* col = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * vdim + j) * dim + ig * KI;
+    float* col = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * vdim + j) * dim;
     const bool live = j < vdim;
+    constexpr int AT = KI < 4 ? KI : 4, STEP = 4 * DELTA_IG;  // a thread's key channels are m STEP + ig AT + 0 .. AT - 1
+    const bool whole = KI >= 4 && dim == KD && a.state_stride % 4 == 0 && ((uintptr_t)a.state & 15) == 0;  // 16 bytes a load
     float S[KI];
+    if (whole && live) {
+        delta_copy<KI, STEP>(S, col + ig * AT);
+    } else {
 #pragma unroll
-    for (int ii = 0; ii < KI; ++ii) S[ii] = (live && ig * KI + ii < dim) ? col[ii] : 0.f;
+        for (int ii = 0; ii < KI; ++ii) {
+            const int i = ii / 4 * STEP + ig * AT + ii % 4;
+            S[ii] = (live && i < dim) ? col[i] : 0.f;
+        }
+    }
     const float decay_rate = CHANNEL ? 0.f : expf(a.a_log[h]), dt_bias = CHANNEL ? 0.f : a.dt_bias[h];
 
     float fq[PER], fk[PER], fg[CHANNEL ? PER : 1], fv = 0.f, fb = 0.f, fa = 0.f;  // the chunk that is on its way
@@ -450,16 +467,18 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
 #pragma unroll
             for (int r = 0; r + 3 < PER; r += 4) {
                 const int e = (tid + DELTA_THREADS * (r / 4)) * 4, t = e / KD, i = e - t * KD;
-                *(float4*)&s_q[buf][t][i] = float4{fq[r], fq[r + 1], fq[r + 2], fq[r + 3]};
-                *(float4*)&s_k[buf][t][i] = float4{fk[r], fk[r + 1], fk[r + 2], fk[r + 3]};
+                float* kq = s_kq[buf][t];
+                *(float4*)(kq + i) = float4{fk[r], fk[r + 1], fk[r + 2], fk[r + 3]};
+                *(float4*)(kq + KD + i) = float4{fq[r], fq[r + 1], fq[r + 2], fq[r + 3]};
                 if constexpr (CHANNEL) *(float4*)&s_g[buf][t][i] = float4{fg[r], fg[r + 1], fg[r + 2], fg[r + 3]};
             }
         } else {
 #pragma unroll
             for (int r = 0; r < PER; ++r) {
                 const int e = tid + DELTA_THREADS * r, t = e / KD, i = e - t * KD;
-                s_q[buf][t][i] = fq[r];
-                s_k[buf][t][i] = fk[r];
+                const int at = BOTH ? i / KI * 2 * KI + i % KI : i;
+                s_kq[buf][t][at] = fk[r];
+                s_kq[buf][t][at + (BOTH ? KI : KD)] = fq[r];
                 if constexpr (CHANNEL) s_g[buf][t][i] = fg[r];
             }
         }
@@ -474,7 +493,8 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
                 const float softplus = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
                 par = float2{expf(-decay_rate * softplus), 1.0f / (1.0f + expf(-fb))};
             }
-            s_par[buf][tid] = par;
+            s_par[buf][0][tid] = par.y;
+            s_par[buf][1][tid] = par.x;
         }
         s_v[buf][tid % DELTA_VB][tid / DELTA_VB] = fv;
     };
@@ -491,34 +511,36 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
             stage(buf ^ 1, count(c1));
             if (c2 < q1) fetch(c2, count(c2));
         }
-        float vv[DELTA_TC];
+        float vv[DELTA_TC], beta[DELTA_TC], g[DELTA_TC];
+        delta_copy<DELTA_TC>(vv, s_v[buf][jl]);
+        delta_copy<DELTA_TC>(beta, s_par[buf][0]);
+        if constexpr (!CHANNEL) delta_copy<DELTA_TC>(g, s_par[buf][1]);
+        else
 #pragma unroll
-        for (int t = 0; t < DELTA_TC; t += 4) {
-            const float4 x = *(const float4*)&s_v[buf][jl][t];
-            vv[t] = x.x, vv[t + 1] = x.y, vv[t + 2] = x.z, vv[t + 3] = x.w;
-        }
-        const float* kt = &s_k[buf][0][ig * KI];
-        const float* qt = &s_q[buf][0][ig * KI];
-        constexpr int GS = CHANNEL ? KD : 0;
-        const float* gt = CHANNEL ? &s_g[buf][0][ig * KI] : &s_g[0][0][0];
+            for (int t = 0; t < DELTA_TC; ++t) g[t] = 1.f;
+        const float* kt = &s_kq[buf][0][ig * AT * (BOTH ? 2 : 1)];
+        const float* qt = kt + KD;  // (not BOTH)
+        constexpr int GS = CHANNEL ? KD : 0, KS = 2 * KD;
+        const float* gt = CHANNEL ? &s_g[buf][0][ig * AT] : &s_g[0][0][0];
         float out = 0.f;  // of token ig
         if (nt == DELTA_TC) {  // a whole chunk: nothing under a condition, every token's operands read a token ahead
             DeltaToken<KI, CHANNEL> cur, nxt;
-            delta_read<KI, CHANNEL>(cur, kt, qt, gt, &s_par[buf][0]);
+            float r[DELTA_TC];
+            delta_read<KI, CHANNEL>(cur, kt, qt, gt);
 #pragma unroll
             for (int t = 0; t < DELTA_TC; ++t) {
-                if (t + 1 < DELTA_TC) delta_read<KI, CHANNEL>(nxt, kt + (t + 1) * KD, qt + (t + 1) * KD, gt + (t + 1) * GS, &s_par[buf][t + 1]);
-                const float o = delta_token<KI, CHANNEL>(S, cur, vv[t]);
-                out = ig == t ? o : out;
+                if (t + 1 < DELTA_TC) delta_read<KI, CHANNEL>(nxt, kt + (t + 1) * KS, qt + (t + 1) * KS, gt + (t + 1) * GS);
+                r[t] = delta_token<KI, CHANNEL>(S, cur, g[t], beta[t], vv[t]);
                 cur = nxt;
             }
+            out = delta_row_sums(r, ig);
         } else {
 #pragma unroll
             for (int t = 0; t < DELTA_TC; ++t) {
                 if (t < nt) {
                     DeltaToken<KI, CHANNEL> cur;
-                    delta_read<KI, CHANNEL>(cur, kt + t * KD, qt + t * KD, gt + t * GS, &s_par[buf][t]);
-                    const float o = delta_token<KI, CHANNEL>(S, cur, vv[t]);
+                    delta_read<KI, CHANNEL>(cur, kt + t * KS, qt + t * KS, gt + t * GS);
+                    const float o = delta_row_sum(delta_token<KI, CHANNEL>(S, cur, g[t], beta[t], vv[t]));
                     out = ig == t ? o : out;
                 }
             }
@@ -533,14 +555,20 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
             __syncthreads();
         }
     }
-    if (live) {
+    if (whole && live) {
 #pragma unroll
-        for (int ii = 0; ii < KI; ++ii)
-            if (ig * KI + ii < dim) col[ii] = S[ii];
+        for (int ii = 0; ii + 3 < KI; ii += 4) *(float4*)(col + ii / 4 * STEP + ig * AT) = float4{S[ii], S[ii + 1], S[ii + 2], S[ii + 3]};
+    } else if (live) {
+#pragma unroll
+        for (int ii = 0; ii < KI; ++ii) {
+            const int i = ii / 4 * STEP + ig * AT + ii % 4;
+            if (i < dim) col[i] = S[ii];
+        }
     }
 }
 
-extern "C" int lle_delta_max_dim(void) { return 16 * DELTA_IG; }
+#define DELTA_MAX_DIM (16 * DELTA_IG)
+extern "C" int lle_delta_max_dim(void) { return DELTA_MAX_DIM; }
 
 // q, k float32 [N, G dim] (unit vectors, q scaled), v float32 [N, H vdim], ba float32 [N, 2 H], a_log and dt_bias
 // float32 [H]; state float32 rows of `state_stride` floats whose first H vdim dim hold the heads' states transposed;
@@ -552,7 +580,7 @@ extern "C" int lle_delta_scan(const void* q, const void* k, const void* v, const
                               const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, void* gates, int N,
                               hipStream_t stream) {
     if (S <= 0 || H <= 0) return 0;
-    if (G <= 0 || H % G || dim <= 0 || dim > 16 * DELTA_IG || vdim <= 0 || H > 65535 || (vdim + DELTA_VB - 1) / DELTA_VB > 65535)
+    if (G <= 0 || H % G || dim <= 0 || dim > DELTA_MAX_DIM || vdim <= 0 || H > 65535 || (vdim + DELTA_VB - 1) / DELTA_VB > 65535)
         return (int)hipErrorInvalidValue;
     if (ba_cols < (decay ? H : 2 * H)) return (int)hipErrorInvalidValue;
     DeltaArgs a{(const float*)q, (const float*)k, (const float*)v, (const float*)ba, ba_cols, (const float*)a_log,
