@@ -247,9 +247,12 @@ __device__ __forceinline__ float ssd_row_sum(float x) {
 }
 
 // Requests of at most SSD_WALK tokens.  grid = (requests, heads, blocks of 16 value channels), 256 threads: thread
-// (jl, ig) = (tid / 16, tid % 16) owns the state channels [ig KI, (ig + 1) KI) of column j = block 16 + jl; the sixteen
+// (jl, ig) = (tid / 16, tid % 16) owns KI state channels of column j = block 16 + jl, four neighbours of every 64 (fewer than
+// four: ig KI + 0 .. KI - 1), so that a wavefront's loads lie one beside the other in memory and in LDS; the sixteen
 // threads of a column are neighbours in a wavefront and add their shares of S^T C up through the lanes' cross-bar.  The
-// tokens pass through LDS SSD_TC at a time.
+// tokens pass through LDS SSD_TC at a time.  What bounds it: the states, read and written once.  Single tokens of Rorevik's
+// mid sizes (64 heads of 64 x 128): 1 request 3.6 -> 3.15 us, 8 8.3 -> 7.1, 32 26.7 -> 24.2, 128 104 -> 92 (5.8 TB/s),
+// against a thread's channels in one stretch and LDS filled up with zeros past the chunk's last token.
 #define SSD_TC 8
 template <int KI>
 __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
@@ -261,26 +264,28 @@ __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
     const int q0 = a.cu_tokens[s], q1 = a.cu_tokens[s + 1];
     if (q1 <= q0 || q1 - q0 > SSD_WALK) return;
     const int grp = h / (a.H / a.G), inner = a.H * vdim;
-    float* col = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * vdim + j) * n + ig * KI;
+    float* col = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * vdim + j) * n;
     const bool live = j < vdim;
+    constexpr int AT = KI < 4 ? KI : 4;
+    auto channel = [&](int i) { return i / 4 * 64 + ig * AT + i % 4; };
     float S[KI];
     if (KI % 4 == 0 && n == KN && a.state_wide) {  // (rows of a multiple of 64 channels: 16 bytes a load)
 #pragma unroll
         for (int i = 0; i + 3 < KI; i += 4) {
-            const float4 v = live ? *(const float4*)(col + i) : float4{0.f, 0.f, 0.f, 0.f};
+            const float4 v = live ? *(const float4*)(col + channel(i)) : float4{0.f, 0.f, 0.f, 0.f};
             S[i] = v.x, S[i + 1] = v.y, S[i + 2] = v.z, S[i + 3] = v.w;
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < KI; ++i) S[i] = (live && ig * KI + i < n) ? col[i] : 0.f;
+        for (int i = 0; i < KI; ++i) S[i] = (live && channel(i) < n) ? col[channel(i)] : 0.f;
     }
     const float rate = expf(a.a_log[h]), dt_bias = a.dt_bias[h], D = a.D[h];
     for (int c0 = q0; c0 < q1; c0 += SSD_TC) {
         const int nt = min(SSD_TC, q1 - c0);
         if (c0 > q0) __syncthreads();  // (the chunk before has been read)
-        for (int e = tid; e < SSD_TC * KN; e += 256) {
+        for (int e = tid; e < nt * KN; e += 256) {
             const int t = e / KN, i = e - t * KN;
-            const bool there = t < nt && i < n;
+            const bool there = i < n;
             const float* row = a.c + (int64_t)(c0 + t) * a.CC + inner + grp * n + i;
             s_B[t][i] = there ? row[0] : 0.f;
             s_C[t][i] = there ? row[a.G * n] : 0.f;
@@ -298,12 +303,11 @@ __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
         for (int t = 0; t < SSD_TC; ++t) {
             if (t < nt) {
                 const float g = s_g[t], x = s_x[t][jl], xdt = x * s_dt[t];
-                const float *B = &s_B[t][ig * KI], *C = &s_C[t][ig * KI];
                 float o = 0.f;
 #pragma unroll
                 for (int i = 0; i < KI; ++i) {
-                    S[i] = fmaf(B[i], xdt, g * S[i]);
-                    o = fmaf(S[i], C[i], o);
+                    S[i] = fmaf(s_B[t][channel(i)], xdt, g * S[i]);
+                    o = fmaf(S[i], s_C[t][channel(i)], o);
                 }
                 o = ssd_row_sum(o);
                 if (ig == 0 && live) a.y[(int64_t)(c0 + t) * inner + h * vdim + j] = fmaf(D, x, o);
@@ -313,11 +317,11 @@ __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
     if (!live) return;
     if (KI % 4 == 0 && n == KN && a.state_wide) {
 #pragma unroll
-        for (int i = 0; i + 3 < KI; i += 4) *(float4*)(col + i) = float4{S[i], S[i + 1], S[i + 2], S[i + 3]};
+        for (int i = 0; i + 3 < KI; i += 4) *(float4*)(col + channel(i)) = float4{S[i], S[i + 1], S[i + 2], S[i + 3]};
     } else {
 #pragma unroll
         for (int i = 0; i < KI; ++i)
-            if (ig * KI + i < n) col[i] = S[i];
+            if (channel(i) < n) col[channel(i)] = S[i];
     }
 }
 
