@@ -1858,6 +1858,224 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     }
 }
 
+// A q or k head of a raw float32 projection in mfma_f32_attention_kernel's layout: lane (c, r) holds elements 16 i + 4 c .. + 3,
+// element e and its partner of the rotation, D / 2 further on, in one lane.  load asks for everything, finish works on it.
+template <int DQ, int WEIGHTS>
+struct F32Head {
+    f32x4 x[DQ], w[DQ];
+    typedef f32x4 Table[DQ / 2][2];  // cos, sin of two elements each
+    __device__ __forceinline__ void load(const float* src, const void* weight, int c) {
+#pragma unroll
+        for (int i = 0; i < DQ; ++i) x[i] = *(const f32x4*)(src + 16 * i + 4 * c);
+        if (!weight) return;  // (the same for the whole launch)
+#pragma unroll
+        for (int i = 0; i < DQ; ++i) {
+            if constexpr (WEIGHTS == LLE_F32) {
+                w[i] = *(const f32x4*)((const float*)weight + 16 * i + 4 * c);
+            } else {
+                const bf16x4 b = *(const bf16x4*)((const bf16_t*)weight + 16 * i + 4 * c);
+                w[i] = f32x4{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
+            }
+        }
+    }
+    static __device__ __forceinline__ void load_table(Table& tab, const float* cos_sin, int tok, int c) {
+#pragma unroll
+        for (int i = 0; i < DQ / 2; ++i) {
+            const f32x4* t = (const f32x4*)(cos_sin + ((int64_t)tok * (8 * DQ) + 16 * i + 4 * c) * 2);
+            tab[i][0] = t[0];
+            tab[i][1] = t[1];
+        }
+    }
+    __device__ __forceinline__ void norm(float eps) {
+        f32x4 ss = x[0] * x[0];
+#pragma unroll
+        for (int i = 1; i < DQ; ++i) ss += x[i] * x[i];
+        const float inv = 1.0f / sqrtf(column_sum((ss[0] + ss[1]) + (ss[2] + ss[3])) / (float)(16 * DQ) + eps);
+#pragma unroll
+        for (int i = 0; i < DQ; ++i) x[i] = x[i] * inv * w[i];
+    }
+    __device__ __forceinline__ void turn(const Table& tab) {
+#pragma unroll
+        for (int i = 0; i < DQ / 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float cs = tab[i][e / 2][e % 2 * 2], sn = tab[i][e / 2][e % 2 * 2 + 1], a = x[i][e], b = x[i + DQ / 2][e];
+                x[i][e] = a * cs - b * sn;
+                x[i + DQ / 2][e] = b * cs + a * sn;
+            }
+    }
+};
+
+// short_decode_kernel in float32: one new token a request, at most SHORT_F32_KEYS keys, a wavefront for every 16 of them (past 176:
+// a second 16) and one for the new token; products on the float32 matrix instruction as in mfma_f32_attention_kernel (1024 cycles for the scores of
+// 16 keys of 128, as many for the values: V flies under the scores).  Twelve wavefronts leave a lane the 168 registers that a
+// head, its weights, its rotation and K need side by side.  0.6B sizes (16 q heads, 8 kv heads of 128) at 97 keys, 1 / 8 / 32
+// requests: 9.0 / 10.0 / 12.0 us in two launches (rotation and cache write, attention), 7.0 / 7.7 / 9.1 here; 32 requests at 200 keys
+// 19.2 and 15.7, 8 at 256 11.4 and 12.5 (there the two launches' key splits reach CUs that this one leaves idle; which of them
+// takes a step is can_fuse_rope_attention's to say).  Tried and not kept: the second step's K asked for before the first's values.
+#define SHORT_F32_WAVES 11
+#define SHORT_F32_KEYS 256
+static_assert(SHORT_F32_KEYS <= 2 * SHORT_F32_WAVES * F32_KEYS, "two steps a wavefront");
+template <int DQ, int WEIGHTS>
+__global__ __launch_bounds__((SHORT_F32_WAVES + 1) * LLE_WAVE) void short_decode_f32_kernel(
+    const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ seq_slots,
+    const int32_t* __restrict__ block_tables, int max_pages, int P, int window, int G, int nkv, float* kv_layer,
+    float* __restrict__ out, int64_t page_stride, float scale_log2, FusedQKV f) {
+    const int s = blockIdx.x, kvh = blockIdx.y;
+    const int tok = cu_tokens[s], tok_end = cu_tokens[s + 1], kv_len = kv_lens[s], seq_slot = seq_slots[s];
+    asm volatile("" ::"s"(tok), "s"(tok_end), "s"(kv_len), "s"(seq_slot), "s"(nkv), "s"(kv_layer), "s"(out), "s"(page_stride),
+                 "s"(scale_log2), "s"(f.qkv), "s"(f.q_weight), "s"(f.k_weight), "s"(f.cos_sin), "s"(f.eps), "s"(f.write_kv));
+    constexpr int D = DQ * 16, WAVES = SHORT_F32_WAVES + 1;
+    extern __shared__ float smem[];  // [waves][G][D] acc, then [waves][16] m, [waves][16] l
+    float* s_m = smem + WAVES * G * D;
+    float* s_l = s_m + WAVES * 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    const int c = lane / 16, r16 = lane % 16;
+    if (tok_end - tok != 1) return;  // (a request without a token has nothing to do)
+    const int last = kv_len - 1, lo = window > 0 ? max(0, kv_len - window) : 0;
+    // the wavefront's steps of 16 keys: its own number and, past SHORT_F32_WAVES steps, the one that many further on
+    int j0 = wave * F32_KEYS;
+    constexpr int ROUND = SHORT_F32_WAVES * F32_KEYS;
+    if (j0 + F32_KEYS <= lo) j0 += ROUND;
+    const PageSize pages(P);
+    const int32_t* table = block_tables + (int64_t)seq_slot * max_pages;
+    int at = min(j0, max(last, 0)), lp = pages.of(at);  // (16 keys of a step lie in one page)
+    int page = table[lp];
+    const int slot = f.slots[tok];
+    const bool fresh = f.write_kv && slot >= 0;  // (else the new token's place holds what the page does)
+    const float* qkv = (const float*)f.qkv + (int64_t)tok * (nkv * (G + 2) * D);
+    const float* q_head = qkv + (int64_t)(kvh * G + min(r16, G - 1)) * D;  // (rows past the group's: dropped at the end)
+    f32x4 o[DQ];
+#pragma unroll
+    for (int n = 0; n < DQ; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float top = NEG_BIG, l = 0.f;
+    if (wave < SHORT_F32_WAVES && j0 <= last && j0 + F32_KEYS > lo) {
+        F32Head<DQ, WEIGHTS> q;
+        typename F32Head<DQ, WEIGHTS>::Table tab;
+        q.load(q_head, f.q_weight, c);
+        q.load_table(tab, f.cos_sin, tok, c);
+        f32x4 k[DQ], v[DQ];
+        auto load_k = [&] {
+            const float* kp = kv_layer + (int64_t)page * page_stride + ((int64_t)kvh * P + (at - lp * P) + r16) * D + 4 * c;
+#pragma unroll
+            for (int i = 0; i < DQ; ++i) k[i] = *(const f32x4*)(kp + 16 * i);
+        };
+        load_k();
+        if (f.q_weight) q.norm(f.eps);
+        q.turn(tab);
+        const int pos = fresh ? last - 1 : last;  // the last key that comes from the pages
+        for (;;) {
+            const float* vp = kv_layer + (int64_t)page * page_stride + ((int64_t)(nkv + kvh) * D + r16) * P + (at - lp * P) + 4 * c;
+#pragma unroll
+            for (int n = 0; n < DQ; ++n) v[n] = *(const f32x4*)(vp + (int64_t)16 * n * P);
+            f32x4 sc = {0.f, 0.f, 0.f, 0.f}, sc2 = sc;  // (two chains)
+#pragma unroll
+            for (int i = 0; i < DQ; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    sc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][e], q.x[i][e], sc, 0, 0, 0);
+                    sc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][e + 1], q.x[i][e + 1], sc2, 0, 0, 0);
+                }
+            sc += sc2;
+            f32x4 x = sc * scale_log2;
+            if (j0 < lo || j0 + F32_KEYS - 1 > pos) {  // (the same for the whole wavefront) places without a key: whatever lies there
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int key = j0 + 4 * c + e;
+                    const bool out_of = key < lo || key > pos;
+                    if (out_of) x[e] = NEG_BIG;
+#pragma unroll
+                    for (int n = 0; n < DQ; ++n) v[n][e] = out_of ? 0.f : v[n][e];
+                }
+            }
+            const float before = top;
+            top = fmaxf(top, column_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
+            const float base = top <= NEG_BIG ? 0.f : top;  // (no key is seen where the new token is the step's first one)
+            f32x4 p;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[e] = exp2f(x[e] - base);
+            const float sum = (p[0] + p[1]) + (p[2] + p[3]);
+            if (j0 >= ROUND && before > NEG_BIG) {  // a second step
+                const float alpha = exp2f(before - base);
+                l = fmaf(l, alpha, sum);
+#pragma unroll
+                for (int n = 0; n < DQ; ++n) o[n] *= alpha;
+            } else {
+                l = sum;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int n = 0; n < DQ; ++n) o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][e], p[e], o[n], 0, 0, 0);
+            j0 += ROUND;
+            if (j0 > last) break;
+            at = j0, lp = pages.of(at), page = table[lp];
+            load_k();
+        }
+        l = column_sum(l);
+    } else if (wave == SHORT_F32_WAVES && fresh) {
+        const float* k_head = qkv + (int64_t)(nkv * G + kvh) * D;
+        const float* v_head = k_head + (int64_t)nkv * D;
+        F32Head<DQ, WEIGHTS> k, q;
+        typename F32Head<DQ, WEIGHTS>::Table tab;
+        k.load(k_head, f.k_weight, c);
+        k.load_table(tab, f.cos_sin, tok, c);
+        if (f.k_weight) k.norm(f.eps);
+        q.load(q_head, f.q_weight, c);
+        k.turn(tab);
+        const int own = pages.of(slot), off = slot - own * P;
+        float* base = kv_layer + (int64_t)own * page_stride;
+        if (r16 == 0) {
+            float* kdst = base + ((int64_t)kvh * P + off) * D + 4 * c;
+#pragma unroll
+            for (int i = 0; i < DQ; ++i) *(f32x4*)(kdst + 16 * i) = k.x[i];
+        }
+        if (f.q_weight) q.norm(f.eps);
+        // (v only now, where the weights' registers are free)
+#pragma unroll
+        for (int n = 0; n < DQ; ++n) o[n] = *(const f32x4*)(v_head + 16 * n + 4 * c);
+        q.turn(tab);
+        f32x4 dot = k.x[0] * q.x[0];
+#pragma unroll
+        for (int i = 1; i < DQ; ++i) dot += k.x[i] * q.x[i];
+        top = column_sum((dot[0] + dot[1]) + (dot[2] + dot[3])) * scale_log2;
+        l = 1.f;
+        if (r16 == 0) {
+            float* vdst = base + ((int64_t)(nkv + kvh) * D + 4 * c) * P + off;
+#pragma unroll
+            for (int n = 0; n < DQ; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vdst[(int64_t)(16 * n + e) * P] = o[n][e];
+        }
+    }
+    if (r16 < G) {
+#pragma unroll
+        for (int n = 0; n < DQ; ++n) *(f32x4*)(smem + (wave * G + r16) * D + 16 * n + 4 * c) = o[n];
+    }
+    if (c == 0) {
+        s_m[wave * 16 + r16] = top;
+        s_l[wave * 16 + r16] = l;
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < G * D; idx += WAVES * LLE_WAVE) {
+        const int r = idx / D;
+        float m[WAVES], big = NEG_BIG;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            m[w] = s_m[w * 16 + r];
+            big = fmaxf(big, m[w]);
+        }
+        float num = 0.f, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float e = exp2f(m[w] - big);
+            num = fmaf(smem[w * G * D + idx], e, num);
+            den = fmaf(s_l[w * 16 + r], e, den);
+        }
+        out[((int64_t)tok * (nkv * G) + kvh * G) * D + idx] = num / den;
+    }
+}
+
 // merges the key splits of the kernel above: grid = (tokens, q heads), one wavefront each
 __global__ __launch_bounds__(LLE_WAVE) void f32_combine_kernel(const float* __restrict__ ws_o,
                                                                const float* __restrict__ ws_ml, int nsplit,
@@ -2198,6 +2416,42 @@ extern "C" int lle_pair_rope_attention_decode(const void* u, int cols, const voi
                     : (cap ? launch_short_decode<4, LLE_BF16, true, true> : launch_short_decode<4, LLE_BF16, true, false>))(
         f, (bf16_t*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens, (const int32_t*)kv_lens,
         (bf16_t*)out, S, nq, nkv, page_size, page_stride, max_pages, window, scale_log2, stream);
+}
+
+// The most keys of a request of short_decode_f32_kernel.
+extern "C" int lle_short_decode_max_keys_f32(void) { return SHORT_F32_KEYS; }
+
+// One token a request (S of them), float32 throughout (norm weights: weight_dtype, or none): q/k norm, rotation over the whole
+// head, the write of K and V and the attention in one launch, for heads of 64 or 128 and at most SHORT_F32_KEYS keys.  Else as
+// lle_qk_norm_rope_attention_decode below.
+extern "C" int lle_qk_norm_rope_attention_decode_f32(const void* qkv, const void* slots, const void* q_weight, const void* k_weight,
+                                                     int weight_dtype, const void* cos_sin, float eps, int write_kv, void* kv_layer,
+                                                     const void* block_tables, const void* seq_slots, const void* cu_tokens,
+                                                     const void* kv_lens, void* out, int S, int nq, int nkv, int d, int page_size,
+                                                     int64_t page_stride, int max_pages, int window, float scale, int max_kv_len,
+                                                     hipStream_t stream) {
+    if (S <= 0) return 0;
+    if (!qkv || !cos_sin || !slots || (q_weight == nullptr) != (k_weight == nullptr) || S > 65535 || nkv <= 0 || nkv > 65535 || nq <= 0 ||
+        nq % nkv != 0 || nq / nkv > 16 || (d != 64 && d != 128) || page_size <= 0 || page_size % 16 != 0 || max_kv_len <= 0 ||
+        max_kv_len > SHORT_F32_KEYS || (((uintptr_t)qkv | (uintptr_t)cos_sin | (uintptr_t)kv_layer) & 15) || page_stride % 4 != 0)
+        return (int)hipErrorInvalidValue;
+    const size_t smem = (size_t)(SHORT_F32_WAVES + 1) * (nq / nkv * d + 2 * 16) * sizeof(float);
+    if (smem > 64 * 1024) return (int)hipErrorInvalidValue;
+    FusedQKV f = {};
+    f.qkv = (const bf16_t*)qkv;
+    f.slots = (const int32_t*)slots;
+    f.q_weight = q_weight;
+    f.k_weight = k_weight;
+    f.cos_sin = (const float*)cos_sin;
+    f.eps = eps;
+    f.write_kv = write_kv;
+    const bool f32 = weight_dtype == LLE_F32;
+    auto kernel = d == 64 ? (f32 ? short_decode_f32_kernel<4, LLE_F32> : short_decode_f32_kernel<4, LLE_BF16>)
+                          : (f32 ? short_decode_f32_kernel<8, LLE_F32> : short_decode_f32_kernel<8, LLE_BF16>);
+    kernel<<<dim3(S, nkv), (SHORT_F32_WAVES + 1) * LLE_WAVE, smem, stream>>>(
+        (const int32_t*)cu_tokens, (const int32_t*)kv_lens, (const int32_t*)seq_slots, (const int32_t*)block_tables, max_pages, page_size,
+        window, nq / nkv, nkv, (float*)kv_layer, (float*)out, page_stride, scale * 1.44269504088896340736f, f);
+    LLE_RETURN_LAUNCH_STATUS();
 }
 
 // Decode steps only (every request has at most 16 / group tokens), head_dim a multiple of 64, a

@@ -723,9 +723,20 @@ class HipOps:
         return out
 
     def can_fuse_rope_attention(self, dtype, head_dim: int, rotary_dim: int, page_size: int, group: int,
-                                max_q_len: int, max_kv_len: int, num_seqs: int) -> bool:
+                                max_q_len: int, max_kv_len: int, num_seqs: int, kv_heads: int = 0) -> bool:
         """Whether qk_norm_rope_attention takes this step: bfloat16, a rotation over the whole head
-        of a multiple of 64 elements, and only requests of at most 16 / group tokens (decode steps)."""
+        of a multiple of 64 elements, and only requests of at most 16 / group tokens (decode steps); float32: one token and few
+        keys a request, heads of 64 or 128."""
+        if dtype == torch.float32:
+            # past 176 keys a wavefront has two steps: then only where a workgroup a request and kv head reach as many CUs as the key
+            # splits of the two launches do (256 keys, 8 kv heads: 8 requests 11.4 us in two launches and 12.5 in one, 12 14.0 and
+            # 12.5, 16 16.4 and 12.9; 140 keys, 8 requests: 12.9 and 9.3)
+            if max_kv_len > 176 and num_seqs * kv_heads < 96:
+                return False
+            return (head_dim in (64, 128) and rotary_dim == head_dim and page_size % 16 == 0 and max_q_len == 1 and group <= 16
+                    and 0 < max_kv_len <= self._get("attention", "lle_short_decode_max_keys_f32", [])()
+                    and 48 * group * head_dim + 1536 <= 65536 and num_seqs <= 65535 and not self.force_generic_attention
+                    and not self.force_separate_rope)
         return (dtype == torch.bfloat16 and head_dim % 64 == 0 and head_dim <= self.MAX_HEAD_DIM
                 and rotary_dim == head_dim and page_size % 16 == 0 and 0 < max_q_len and max_q_len * group <= 16
                 and max_kv_len > 0 and num_seqs <= 65535 and not self.force_generic_attention
@@ -739,8 +750,9 @@ class HipOps:
         its K and V, every workgroup norms and rotates the q rows it multiplies.  `order` (int32 [S], or None):
         the requests in the order in which they are started, see decode_order.  `max_kv_len`: a host-side bound; it chooses the
         kernel and its key splits, never the result.  `token_seq` None: every request has one token."""
-        _dev(qkv, "qkv", torch.bfloat16)
-        _dev(kv_layer, "kv_layer", torch.bfloat16)
+        f32 = qkv.dtype == torch.float32
+        _dev(qkv, "qkv", torch.float32 if f32 else torch.bfloat16)
+        _dev(kv_layer, "kv_layer", qkv.dtype)
         _dev(cos_sin, "cos_sin", torch.float32)
         for t, name in ((slots, "slots"), (block_table, "block_table"), (seq_slots, "seq_slots"),
                         (cu_tokens, "cu_tokens"), (kv_lens, "kv_lens")):
@@ -769,6 +781,15 @@ class HipOps:
             _dev(order, "order", torch.int32)
             _need(order.shape == (S,), "order must be [S]")
         win = int(window) if window else 0
+        if f32:
+            _need(token_seq is None and order is None and d in (64, 128), "in float32 every request has one token and heads are of 64 or 128")
+            out = torch.empty((N, nq * d), dtype=torch.float32, device=qkv.device)
+            self._run("attention", "lle_qk_norm_rope_attention_decode_f32",
+                      [_P, _P, _P, _P, _I, _P, _F, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _I, _P],
+                      _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wcode, _ptr(cos_sin), float(eps), int(bool(write_kv)),
+                      _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens), _ptr(out), S, nq, nkv, d,
+                      page_size, kv_layer.stride(0), block_table.shape[1], win, float(scale), int(max_kv_len))
+            return out
         ns = self.decode_splits(S, nkv, max_kv_len, win)
         out = torch.empty((N, nq * d), dtype=torch.bfloat16, device=qkv.device)
         ws_o = ws_ml = None

@@ -110,7 +110,7 @@ class PagedAttention(Mixer):
         if fused is not None:
             cos_sin, rot = fused
             if ops.can_fuse_rope_attention(qkv.dtype, self.d, rot, cache.kv.shape[3], self.nq // self.nkv,
-                                           step.max_q_len, step.max_kv_len, step.seq_slots.shape[0]):
+                                           step.max_q_len, step.max_kv_len, step.seq_slots.shape[0], self.nkv):
                 # a decode step: norm, rotation, cache write and attention in one launch
                 order, order_key = None, ("decode_order", self.nkv)
                 if min(step.max_kv_len, self.window or step.max_kv_len) > ops.DECODE_KEYS_AT_ONCE:

@@ -88,3 +88,44 @@ def test_short_decode_with_pairs_equals_its_two_halves(lens, nq, nkv, d, P, wind
     assert (got - want).abs().max() < 2e-2  # (as above)
     c = a.clone()
     assert (run(c, False) - want).abs().max() < 2e-2 and torch.equal(c, a)
+
+
+# float32: the edges of its steps of 16 keys, of a wavefront's second step (176), the most keys that the launch takes
+@pytest.mark.parametrize("lens", [[1, 2, 15, 16, 17], [31, 32, 33, 64, 97], [175, 176, 177, 178], [255, 256, 240, 193]])
+@pytest.mark.parametrize("nq,nkv,d,P,window", [(16, 8, 128, 16, None), (8, 8, 64, 48, None), (10, 1, 128, 32, 40), (32, 2, 64, 16, 17), (4, 4, 128, 64, 1)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32, None])
+def test_short_decode_in_float32_equals_its_two_halves(wdtype, nq, nkv, d, P, window, lens):
+    requests = [(n - 1, 1) for n in lens]
+    args, mq, mk = attention_case(torch.float32, nq, nkv, d, P, window, requests,
+                                  pages=sum(-(-n // P) for n in lens) + 3, max_pages=-(-max(lens) // P) + 1)
+    _, kv, table, seq_slots, cu, kv_lens, token_seq, _, scale = args
+    S = len(lens)
+    o = ops()
+    fits = lambda keys, group=nq // nkv, rot=d, heads=96: o.can_fuse_rope_attention(torch.float32, d, rot, P, group, 1, keys, S, heads)
+    assert fits(mk) and not fits(257) and not fits(mk, 17) and not fits(mk, rot=d // 2) and fits(176, heads=1) and not fits(177, heads=1)
+    qkv = rnd((S, (nq + 2 * nkv) * d), torch.float32, 70, 1.5)
+    slots = torch.tensor([int(table[int(seq_slots[s]), (n - 1) // P]) * P + (n - 1) % P for s, n in enumerate(lens)], dtype=torch.int32)
+    slots[1] = -1
+    for s, n in enumerate(lens):  # what lies behind a request's last key in its page is nobody's
+        page, off = int(table[int(seq_slots[s]), (n - 1) // P]), (n - 1) % P
+        kv[page, 0, :, off + 1:] = float("nan")
+        kv[page, 1].view(nkv, d, P)[:, :, off + 1:] = float("nan")
+    slots = slots.cuda()
+    inv = (1e6 ** (-(2.0 * torch.arange(d // 2, dtype=torch.float64)) / d)).float().cuda()
+    cs = o.rope_table((kv_lens - 1).int(), inv)
+    qw = kw = None
+    if wdtype is not None:
+        qw, kw = ((1 + 0.2 * rnd((d,), torch.float32, seed)).to(wdtype) for seed in (71, 72))
+    a, b = kv.clone(), kv.clone()
+    q = o.qk_norm_rope_write(qkv, slots, qw, kw, cs, d, 1e-5, a, nq, nkv, d, True)
+    a.nan_to_num_(0.0)
+    want = o.paged_attention(q, a, table, seq_slots, cu, kv_lens, token_seq, window, scale, *mq, mk).double()
+    run = lambda pool, write: o.qk_norm_rope_attention(qkv, slots, qw, kw, cs, 1e-5, pool, nq, nkv, d, write, table, seq_slots, cu, kv_lens,
+                                                       None, window, scale, mk).double()
+    got = run(b, True)
+    # sums of 128 products in 32 bits, in another order: 128 x 2^-24 = 8e-6 of values of size 4 and of scores of size 10
+    assert (got - want).abs().max() < 1e-4
+    written = b.nan_to_num(0.0)
+    assert not torch.equal(written, kv.nan_to_num(0.0)) and (a - written).abs().max() < 1e-5
+    c = a.clone()
+    assert (run(c, False) - want).abs().max() < 1e-4 and torch.equal(c, a)
