@@ -1468,8 +1468,8 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
                 const bf16_t* vb = page + v_head + off;
                 const unsigned kdst = lds_base + 2 * (buf * TILE + first_piece * 8);
                 const unsigned vdst = kdst + 2 * KSTEP * D;
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kdst), "v"(kd_lane[i]), "s"(kb) : "memory", "m0");
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(vdst), "v"(vd_lane[i]), "s"(vb) : "memory", "m0");
+                load_into_lds(kdst, kd_lane[i], kb);
+                load_into_lds(vdst, vd_lane[i], vb);
             }
             if constexpr (LOADS == 1) {
                 own_page += own_adv_pages;

@@ -81,6 +81,13 @@ __device__ __forceinline__ float row16_sum(float v) {
 __device__ __forceinline__ float column_sum(float v) { return combine_xor32(combine_xor16(v, AddF32{}), AddF32{}); }
 __device__ __forceinline__ float column_max(float v) { return combine_xor32(combine_xor16(v, MaxF32{}), MaxF32{}); }
 
+// 16 bytes a lane from `base` and its byte offset straight into LDS, the lanes' one behind the other from byte `at` on (both
+// the same for the wavefront).  The load takes its address in LDS from M0 and wants a wait state behind a write of it, which the
+// compiler cannot put into an asm.  Nothing waits for the load here: vmcnt counts it.
+__device__ __forceinline__ void load_into_lds(unsigned at, unsigned offset, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+}
+
 // Sum over a workgroup of up to 1024 threads; `smem` holds >= 16 floats.
 // Every thread gets the result; the order of the additions is fixed.
 __device__ __forceinline__ float block_sum(float v, float* smem) {

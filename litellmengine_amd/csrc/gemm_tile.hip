@@ -64,8 +64,7 @@ __global__ __launch_bounds__(WM* WN* LLE_WAVE, 2) void gemm_tile_kernel(const bf
         for (int i = 0; i < LOADS; ++i) {
             const int g = wave + WAVES * i;
             const bf16_t* base = (g < BM / RPL ? xb : wb) + step * BK;
-            const unsigned dst = lds_base + buf * STAGE + g * 1024;
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offset[i]), "s"(base) : "memory", "m0");
+            load_into_lds(lds_base + buf * STAGE + g * 1024, offset[i], base);
         }
     };
     const int wm = wave / WN * (32 * TM), wn = wave % WN * (32 * TN);

@@ -88,9 +88,7 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
     using Half0 = std::integral_constant<int, 0>;
     using Half1 = std::integral_constant<int, 1>;
     const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) void*)wide_lds;
-    auto dma = [&](unsigned at_lds, unsigned offset, const bf16_t* base) {
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base + at_lds), "v"(offset), "s"(base) : "memory", "m0");
-    };
+    auto dma = [&](unsigned at_lds, unsigned offset, const bf16_t* base) { load_into_lds(lds_base + at_lds, offset, base); };
     auto issue_x = [&](int step, auto half) {
         constexpr int h = decltype(half)::value;
 #pragma unroll

@@ -2,6 +2,7 @@
 import glob
 import os
 import re
+import shutil
 import subprocess
 
 import pytest
@@ -59,3 +60,22 @@ int main() {
                     f"-I{os.path.dirname(build.__file__)}", str(source), "-o", str(program)], check=True)
     assert subprocess.run([str(program)]).returncode == 0
     assert not [p for p in SOURCES if re.search(r"static bool \w+ =", open(p).read())]  # (asked for once a process)
+
+
+@pytest.mark.parametrize("name", [n for n, files in build.LIBRARIES.items()
+                                  if any("load_into_lds(" in open(os.path.join(os.path.dirname(build.__file__), f)).read() for f in files)])
+def test_loads_into_lds_wait_for_their_address(name, tmp_path):
+    """Between a scalar write of M0 and a load whose target is LDS stands another instruction: the load may take the M0 before
+    otherwise, and nothing in the processor sees to it (the compiler does, for what it writes itself)."""
+    objdump = os.path.join(os.path.dirname(os.path.dirname(build._hipcc())), "llvm", "bin", "llvm-objdump")
+    if not os.path.isfile(objdump):
+        pytest.skip("no llvm-objdump")
+    library = shutil.copy(build._find_built(name) or build.compile_library(name), tmp_path)
+    subprocess.run([objdump, "--offloading", library], check=True, cwd=tmp_path, capture_output=True)
+    code, = glob.glob(f"{library}*{build.ARCH}")
+    text = subprocess.run([objdump, "-d", f"--mcpu={build.ARCH}", code], check=True, capture_output=True, text=True).stdout
+    code = [line.split("//")[0].split() for line in text.splitlines() if line.startswith("\t")]
+    loads = [i for i, words in enumerate(code) if "_load_lds_" in words[0]]
+    assert loads
+    early = [code[i - 1 : i + 1] for i in loads if code[i - 1][1:2] == ["m0,"]]
+    assert not early, (len(early), early[:3])
