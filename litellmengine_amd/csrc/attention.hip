@@ -317,15 +317,30 @@ __device__ __forceinline__ float max_of_8(const float (&x)[8]) {
     return max3(max3(x[6], x[7], a), b, b);
 }
 
+// The values of keys outside [lo, hi] become zeros; v[n][i] belongs to key `first` + i.  Their weight is 0, which drops whatever
+// lies there but an infinity or a NaN (pages are handed on as they are).
+template <int N>
+__device__ __forceinline__ void drop_values(bf16x8 (&v)[N], int first, int lo, int hi) {
+    u32x4 keep;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int j = first + 2 * i;
+        keep[i] = (j >= lo && j <= hi ? 0xffffu : 0u) | (j + 1 >= lo && j + 1 <= hi ? 0xffff0000u : 0u);
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v[n]) & keep);
+}
+
 // One 32-key step for RT tiles of 16 rows.  load_k(x, ks): for lane (c, r16) key
 // KEY_OF_ROW(r16, x) of the step, elements 32 ks + 8 c .. + 7.  load_v(n): value element
 // 16 n + r16, keys 8c..8c+7 of the step.  Each operand is fetched once and used by all row tiles.
+// No row sees a key outside [seen_lo, seen_hi].
 // CAP: the scores pass through cap * tanh(score / cap).  In the base-2 domain that is C (1 - 2 / (1 + 2^(s k))) with
 // C = cap log2 e (`cap_log2`) and k = 2 log2 e scale / cap, which the caller hands in for the scale; either end of the
 // exponential's range gives the right limit.
 template <int DK, int RT, bool CAP, typename LoadK, typename LoadV>
 __device__ __forceinline__ void tile_step(RowState<DK, RT>& st, const RowInfo (&row)[RT], LoadK load_k,
-                                          LoadV load_v, int j0, float scale_log2, float cap_log2) {
+                                          LoadV load_v, int j0, int seen_lo, int seen_hi, float scale_log2, float cap_log2) {
     const int c = (threadIdx.x % LLE_WAVE) / 16;
     f32x4 s[RT][2];
 #pragma unroll
@@ -373,6 +388,7 @@ __device__ __forceinline__ void tile_step(RowState<DK, RT>& st, const RowInfo (&
                 const int j = j0 + 8 * c + i;  // score i of the lane: tile i / 4, row 4 c + i % 4
                 if (j < row[t].lo || j > row[t].pos) x[t][i] = NEG_BIG;
             }
+            if (t == 0 && (j0 < seen_lo || j0 + KSTEP - 1 > seen_hi)) drop_values(vv, j0 + 8 * c, seen_lo, seen_hi);
         }
         raise = raise || max_of_8(x[t]) > LAZY_MAX;
     }
@@ -513,7 +529,7 @@ __device__ __forceinline__ void attend_rows(RowState<DK, RT>& st, const RowInfo 
     auto multiply = [&](const StepOperands<DK>& op, int step) {
         tile_step<DK, RT, CAP>(
             st, row, [&](int x, int ks) { return op.k[x][ks]; }, [&](int n) { return op.v[n]; }, step * KSTEP,
-            scale_log2, cap_log2);
+            lo_min, hi, scale_log2, cap_log2);
     };
     StepOperands<DK> even, odd;
     lookup();
@@ -1016,6 +1032,8 @@ __global__ __launch_bounds__((SHORT_WAVES + 1) * LLE_WAVE) void short_decode_ker
                 const int j = j0 + 8 * c + i;
                 if (j < lo || j > pos) x[i] = NEG_BIG;
             }
+            // (the new token's place among them, which its wavefront may be writing just now)
+            drop_values(op.v, j0 + 8 * c, lo, pos);
         }
         top = column_max(max_of_8(x));
         const float base = top <= NEG_BIG ? 0.f : top;  // (no key is seen where the new token is the wavefront's first one)
@@ -1378,7 +1396,7 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
                 st, row,
                 [&](int x, int ks) { return *(const bf16x8*)(kt + kx[x] * D + (((4 * ks + c) ^ ksw[x]) * 8)); },
                 [&](int n) { return *(const bf16x8*)(vt + (16 * n + r16) * KSTEP + ((c ^ vsw) * 8)); },
-                step * KSTEP, scale_log2, cap_log2);
+                step * KSTEP, lo_min, hi, scale_log2, cap_log2);
         }
         stash(buf ^ 1, set_c);
         __syncthreads();
@@ -1499,8 +1517,8 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
             if (step >= my_first && step < my_end) {
                 tile_step<DK, PRE_RT, CAP>(
                     st, row, [&](int x, int ks) { return kreg[x][ks]; },
-                    [&](int n) { return *(const bf16x8*)(vt + v_read + n * 256); }, step * KSTEP, scale_log2,
-                    cap_log2);
+                    [&](int n) { return *(const bf16x8*)(vt + v_read + n * 256); }, step * KSTEP, lo_min, hi,
+                    scale_log2, cap_log2);
             }
             // the loads just issued may stay in flight; the tile before them has landed, and this one has been read (its
             // buffer is the next one to be filled)
@@ -1649,7 +1667,8 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     // the keys that each tile's rows see, in steps of 16, and the wavefront's share of them
     int step_begin = 0, step_end = 0, step_stride = 1;
     int first[TILES], end[TILES];
-    [[maybe_unused]] int kept_end = 0;  // steps of the kept first keys, which are the first split's work
+    [[maybe_unused]] int kept = 0, kept_end = 0;  // the kept first keys and their steps, which are the first split's work
+    int seen_lo = 0, seen_hi = -1;  // the keys that any of its rows sees
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         const int r0 = row0 + 16 * t;
@@ -1660,8 +1679,15 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
         first[t] = lo_tile / F32_KEYS;
         end[t] = hi / F32_KEYS + 1;
         step_end = end[t];  // (a later tile's rows see no less far)
-        if (KEEP && split == 0) kept_end = (min(keep_first, max(0, hi - window + 1)) + F32_KEYS - 1) / F32_KEYS;
+        seen_hi = hi;
+        if (t == 0) seen_lo = lo_tile;
+        if (KEEP && split == 0) {
+            kept = min(keep_first, max(0, hi - window + 1));
+            kept_end = (kept + F32_KEYS - 1) / F32_KEYS;
+        }
     }
+    seen_lo = __builtin_amdgcn_readfirstlane(seen_lo);
+    seen_hi = __builtin_amdgcn_readfirstlane(seen_hi);
     if (wave_has_rows) {
         const int per_split = (step_end - first[0] + nsplit - 1) / nsplit;
         step_begin = first[0] + split * per_split;
@@ -1736,8 +1762,17 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
         }
         l[t] = l[t] * alpha + psum;
     };
-    auto values = [&](auto from, auto to, const f32x4* p, const float* alpha) {
+    auto values = [&](auto from, auto to, int step, const f32x4* p, const float* alpha) {
         constexpr int T0 = decltype(from)::value, T1 = decltype(to)::value;
+        if (step * F32_KEYS < seen_lo || step * F32_KEYS + F32_KEYS - 1 > seen_hi) {  // as drop_values
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = step * F32_KEYS + 4 * c + e;
+                const bool out_of = j < seen_lo || j > seen_hi;
+#pragma unroll
+                for (int n = 0; n < DQ; ++n) vf[n][e] = out_of ? 0.f : vf[n][e];
+            }
+        }
 #pragma unroll
         for (int n = 0; n < DQ; ++n) {
 #pragma unroll
@@ -1752,13 +1787,15 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     using None = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
     using All = std::integral_constant<int, TILES>;
-    [[maybe_unused]] const int w_pos = pos[0], w_lo = lo[0], w_begin = step_begin, w_end = step_end;
+    [[maybe_unused]] const int w_pos = pos[0], w_lo = lo[0], w_begin = step_begin, w_end = step_end, w_seen_lo = seen_lo, w_seen_hi = seen_hi;
     for (int range = KEEP && kept_end > 0 ? 0 : 1; range < 2; ++range) {
     if constexpr (KEEP) {
         pos[0] = range == 0 ? (exists[0] ? min(keep_first, w_lo) - 1 : -1) : w_pos;
         lo[0] = range == 0 ? 0 : w_lo;
         step_begin = range == 0 ? (few ? wave : 0) : w_begin;
         step_end = range == 0 ? kept_end : w_end;
+        seen_lo = range == 0 ? 0 : w_seen_lo;
+        seen_hi = __builtin_amdgcn_readfirstlane(range == 0 ? kept - 1 : w_seen_hi);
     }
     if (step_begin >= step_end) continue;
     // K of the next step is asked for before the values of this one are multiplied, V of it before
@@ -1778,17 +1815,17 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
             if (next < step_end) load_k(next);
 #pragma unroll
             for (int t = 0; t < TILES; ++t) weigh(t, step, sc[t], p[t], alpha[t]);
-            values(None{}, All{}, p, alpha);
+            values(None{}, All{}, step, p, alpha);
         } else {
             if (first_in) scores(None{}, One{}, sc);
             else if (second_in) scores(One{}, All{}, sc);
             if (next < step_end) load_k(next);
             if (first_in) {
                 weigh(0, step, sc[0], p[0], alpha[0]);
-                values(None{}, One{}, p, alpha);
+                values(None{}, One{}, step, p, alpha);
             } else if (second_in) {
                 weigh(TILES - 1, step, sc[TILES - 1], p[TILES - 1], alpha[TILES - 1]);
-                values(One{}, All{}, p, alpha);
+                values(One{}, All{}, step, p, alpha);
             }
         }
         if (next < step_end) load_v(next);
