@@ -18,6 +18,7 @@
 // All exponents are at most zero.  The sums l are kept as two floats, so that the difference of two neighbours deep in
 // a chunk is as exact as if it had been added up on its own.  The products are taken on the 32-bit matrix instruction.
 #include "common.h"
+#include <type_traits>
 
 LLE_DEFINE_ERROR_STRING()
 
@@ -251,8 +252,8 @@ __device__ __forceinline__ float ssd_row_sum(float x) {
 // four: ig KI + 0 .. KI - 1), so that a wavefront's loads lie one beside the other in memory and in LDS; the sixteen
 // threads of a column are neighbours in a wavefront and add their shares of S^T C up through the lanes' cross-bar.  The
 // tokens pass through LDS SSD_TC at a time.  What bounds it: the states, read and written once.  Single tokens of Rorevik's
-// mid sizes (64 heads of 64 x 128): 1 request 3.6 -> 3.15 us, 8 8.3 -> 7.1, 32 26.7 -> 24.2, 128 104 -> 92 (5.8 TB/s),
-// against a thread's channels in one stretch and LDS filled up with zeros past the chunk's last token.
+// mid sizes (64 heads of 64 x 128): 1 request 4.0 -> 3.7 us, 8 8.9 -> 7.9, 32 27.5 -> 25.6, 128 105 -> 102 (in a graph), against a
+// thread's channels in one stretch.
 #define SSD_TC 8
 template <int KI>
 __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
@@ -283,13 +284,27 @@ __global__ __launch_bounds__(256) void ssd_walk_kernel(SsdArgs a) {
     for (int c0 = q0; c0 < q1; c0 += SSD_TC) {
         const int nt = min(SSD_TC, q1 - c0);
         if (c0 > q0) __syncthreads();  // (the chunk before has been read)
-        for (int e = tid; e < nt * KN; e += 256) {
-            const int t = e / KN, i = e - t * KN;
-            const bool there = i < n;
-            const float* row = a.c + (int64_t)(c0 + t) * a.CC + inner + grp * n + i;
-            s_B[t][i] = there ? row[0] : 0.f;
-            s_C[t][i] = there ? row[a.G * n] : 0.f;
-        }
+        // R times 256 places, asked for together (in a loop each would wait for the one before) and without a condition: past the
+        // last token that one's again, which nobody reads, past the last channel zeros.  Portions of 8 / 16 / 32 tokens of one
+        // request of 64 heads of 64 x 128: 6.2 / 9.1 / 15.0 us in a loop, 5.4 / 7.4 / 11.7 so.
+        auto stage = [&](auto rounds) {
+            constexpr int R = decltype(rounds)::value;
+            float vb[R], vc[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int e = tid + 256 * r, t = e / KN, i = e - t * KN;
+                const float* row = a.c + (int64_t)(c0 + min(t, nt - 1)) * a.CC + inner + grp * n + min(i, n - 1);
+                vb[r] = row[0];
+                vc[r] = row[a.G * n];
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int e = tid + 256 * r, t = e / KN, i = e - t * KN;
+                if (SSD_TC * KN >= 256 || e < SSD_TC * KN) s_B[t][i] = i < n ? vb[r] : 0.f, s_C[t][i] = i < n ? vc[r] : 0.f;
+            }
+        };
+        if (nt * KN <= 256) stage(std::integral_constant<int, 1>{});
+        else stage(std::integral_constant<int, (SSD_TC * KN + 255) / 256>{});
         if (tid < SSD_TC * 16) {
             const int t = tid / 16, e = tid % 16;
             s_x[t][e] = (t < nt && j0 + e < vdim) ? a.c[(int64_t)(c0 + t) * a.CC + h * vdim + j0 + e] : 0.f;
