@@ -2427,6 +2427,13 @@ static bool short_decode_fits(int S, int nq, int nkv, int d, int page_size, int 
            (size_t)(SHORT_WAVES + 1) * (nq / nkv * d + 2 * 16) * sizeof(float) <= 64 * 1024;
 }
 
+// Whether it takes a step of S requests in place of mfma_decode_kernel, of which twice as many workgroups fit a CU where heads
+// are of 64: only while all of its own are at work at once.  Heads of 64 in groups of 1 to 8 at 512 workgroups and 24 / 97 / 160
+// / 256 keys: 8.8 / 9.7 / 9.6 / 10.3 -> 7.1 / 7.9 / 8.8 / 10.1 us, at 768 10.1 / 12.3 / 12.5 / 14.4 -> 9.6 / 10.8 / 12.3 / 16.1, at 2048
+// 21 / 27 / 28 / 29 -> 22 / 27 / 31 / 35; groups of 16 at 256: 8.3 / 8.5 / 8.5 / 8.5 -> 5.3 / 5.8 / 6.2 / 6.9, at 320 10.6 -> 11.6
+// with 256 keys.  (Heads of 128: 0.95 of the time at 2048 workgroups of 256 keys, less at fewer.)
+static bool short_decode_pays(int S, int G, int nkv, int d) { return d != 64 || (int64_t)S * nkv <= (G > 8 ? 256 : 512); }
+
 // One token a request (S of them): the rotation of q and k in neighbouring pairs, the write of K and V and the attention of
 // lle_pair_rope_write and lle_paged_attention_mfma in one launch, for heads of 64 or 128 of q, k and v alike without biases.  A row of u
 // has `cols` columns, a multiple of 8: q, k, v, then others.  rot: a multiple of 8 (0: nothing turns); softcap <= 0: none.
@@ -2496,7 +2503,8 @@ extern "C" int lle_qk_norm_rope_attention_decode_f32(const void* qkv, const void
 // (write_kv != 0; slots [N], < 0: not written) happen inside the attention launch.  qkv is
 // [N, (nq + 2 nkv) * d] as the projection left it; q_weight / k_weight [d] or null; cos_sin
 // [N, d / 2, 2] float32.  token_seq null: one token a request.  Then, with no more than SHORT_WAVES * 32 keys a request (`max_kv_len` > 0 is a
-// bound), heads of 64 or 128 and partial results that 64 KB of LDS hold (groups of up to 13 at 128): short_decode_kernel.
+// bound), heads of 64 or 128 and partial results that 64 KB of LDS hold (groups of up to 13 at 128): short_decode_kernel, where
+// short_decode_pays.
 // (`order` serves more keys.)
 extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* slots, const void* q_weight,
                                                  const void* k_weight, int weight_dtype, const void* cos_sin,
@@ -2518,7 +2526,8 @@ extern "C" int lle_qk_norm_rope_attention_decode(const void* qkv, const void* sl
     fused.eps = eps;
     fused.write_kv = write_kv;
     fused.order = (const int32_t*)order;
-    if (!token_seq && N == S && nsplit_decode == 1 && !order && short_decode_fits(S, nq, nkv, d, page_size, max_kv_len)) {
+    if (!token_seq && N == S && nsplit_decode == 1 && !order && short_decode_fits(S, nq, nkv, d, page_size, max_kv_len) &&
+        short_decode_pays(S, nq / nkv, nkv, d)) {
         const float scale_log2 = scale * 1.44269504088896340736f;
         const bool f32 = weight_dtype == LLE_F32;
         return (d == 64 ? (f32 ? launch_short_decode<2, LLE_F32> : launch_short_decode<2, LLE_BF16>)

@@ -731,7 +731,13 @@ class HipOps:
             # past 176 keys a wavefront has two steps: then only where a workgroup a request and kv head reach as many CUs as the key
             # splits of the two launches do (256 keys, 8 kv heads: 8 requests 11.4 us in two launches and 12.5 in one, 12 14.0 and
             # 12.5, 16 16.4 and 12.9; 140 keys, 8 requests: 12.9 and 9.3)
-            if max_kv_len > 176 and num_seqs * kv_heads < 96:
+            workgroups, units = num_seqs * kv_heads, self.compute_units()
+            if max_kv_len > 176 and workgroups < 96:
+                return False
+            # one workgroup fits a CU: two rounds of them, or nearly three (8 kv heads, 97 / 256 keys: 64 requests 19.6 / 29.6 us in
+            # two launches and 17.5 / 28.5 in one, 80 24.4 / 36.5 and 23.0 / 37.8, 96 27.2 / 43.2 and 24.4 / 40.4, 128 30.7 / 50.5
+            # and 31.3 / 53.7, 256 52 / 118 and 58 / 130)
+            if not (workgroups <= 2 * units or 2.75 * units <= workgroups <= 3 * units):
                 return False
             return (head_dim in (64, 128) and rotary_dim == head_dim and page_size % 16 == 0 and max_q_len == 1 and group <= 16
                     and 0 < max_kv_len <= self._get("attention", "lle_short_decode_max_keys_f32", [])()

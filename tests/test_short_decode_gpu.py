@@ -129,3 +129,28 @@ def test_short_decode_in_float32_equals_its_two_halves(wdtype, nq, nkv, d, P, wi
     assert not torch.equal(written, kv.nan_to_num(0.0)) and (a - written).abs().max() < 1e-5
     c = a.clone()
     assert (run(c, False) - want).abs().max() < 1e-4 and torch.equal(c, a)
+
+
+# as many workgroups as the launch takes and one request more, which the general launches take
+@pytest.mark.parametrize("dtype,nq,nkv,d,S", [(torch.bfloat16, 8, 8, 64, 64), (torch.bfloat16, 32, 2, 64, 128), (torch.float32, 4, 8, 64, 64),
+                                              (torch.float32, 16, 8, 64, 96)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_many_requests(dtype, nq, nkv, d, S, more):
+    nq, P, n, S = max(nq, nkv), 16, 33, S + more
+    o, i32 = ops(), lambda x: torch.as_tensor(x, dtype=torch.int32).cuda()
+    kv, qkv = rnd((3 * S, 2, nkv, P, d), dtype, 1), rnd((S, (nq + 2 * nkv) * d), dtype, 2, 1.5)
+    table = i32(torch.randperm(3 * S, generator=torch.Generator().manual_seed(3)).view(S, 3))
+    slots, seqs, cu, lens = (table[:, 2] * P).int(), i32(range(S)), i32(range(S + 1)), i32([n] * S)
+    cs = o.rope_table((lens - 1).int(), torch.ones(d // 2, device="cuda"))
+    a, b = kv.clone(), kv.clone()
+    q = o.qk_norm_rope_write(qkv, slots, None, None, cs, d, 1e-6, a, nq, nkv, d, True)
+    want = o.paged_attention(q, a, table, seqs, cu, lens, seqs, None, d ** -0.5, 1, 1, n).double()
+    fits = lambda S, kv_heads: o.can_fuse_rope_attention(dtype, d, d, P, nq // nkv, 1, n, S, kv_heads)
+    if dtype == torch.float32:
+        if o.compute_units() == 256:
+            assert [S for S in (64, 65, 87, 88, 96, 97, 256) if fits(S, 8)] == [64, 88, 96] and fits(256, 2) and not fits(257, 2)
+        if not fits(S, nkv):
+            return
+    got = o.qk_norm_rope_attention(qkv, slots, None, None, cs, 1e-6, b, nq, nkv, d, True, table, seqs, cu, lens, None, None, d ** -0.5, n).double()
+    assert (got - want).abs().max() < (2e-2 if dtype == torch.bfloat16 else 1e-4)  # (as above)
+    assert (a.float() - b.float()).abs().max() <= (2.0 ** -7 * 8 if dtype == torch.bfloat16 else 1e-5)
