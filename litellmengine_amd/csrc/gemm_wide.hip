@@ -1,5 +1,5 @@
-// bfloat16 products X[M, K] . W[N, K]^T of many rows, whole: as they are, or gate and up with the activation between them
-// (W holds gate rows and then up rows, the result is act(gate) . up).
+// bfloat16 products X[M, K] . W[N, K]^T of many rows, gate and up with the activation between them (W holds gate rows and
+// then up rows, the result is act(gate) . up).
 //
 // Tiles of 128 to 288 rows of X by 256 or 128 of W (half of them gate rows, half the up rows that go with them: a lane then holds the
 // sums of both for the same places), stages of 64 columns straight into LDS, eight wavefronts in two groups of four that take
@@ -12,7 +12,8 @@
 //   24576 x 4096 gated, 262 / 700 / 1024 / 2048 / 2111 rows: 77 / 159 / 184 / 306 / 369 -> 69 / 128 / 166 / 275 / 322
 //   51200 x 5120 gated, 512 / 1024 / 2048 / 2111 rows: 280 / 510 / 895 / 1021 -> 234 / 443 / 780 / 827
 //   16384 x 2048 gated, 300 / 2048 rows: 34 / 121 -> 27 / 106; 6144 x 1024 gated, 600 / 2048 rows: 19 / 35 -> 13 / 27
-//   5120 x 8192, 5120 x 25600 at 2111 rows: 150, 452 -> 138, 424
+// Whole products in such tiles are the library's: it does between 0.65 and 1.5 PFLOP/s, by no rule that sizes tell (these tiles
+// 1.1 to 1.3), and where a model of both took the tiles, 38 of 63 measured products were slower by up to 16 %.
 // Tried: all W of a stage read in the first turn, two buffers of everything (24576 x 4096 gated at 1500 rows 236 -> 222, tiles
 // of 128 rows 51 -> 46 us a round); 32 x 32 matrix instructions (+10 %); a ring of all 160 KB with loads asked for half a
 // stage earlier (+15 %: its bookkeeping stands between the turns).
@@ -33,38 +34,37 @@ typedef float wf32x4 __attribute__((ext_vector_type(4)));
 // them over all banks
 #define WIDE_SWIZZLE(r) ((((r) >> 1) & 7) ^ ((((r) >> 3) ^ ((r) >> 2)) & 1))
 
-enum WideOut { WIDE_WHOLE, WIDE_SILU, WIDE_CLAMPED };
+enum WideOut { WIDE_SILU = 1, WIDE_CLAMPED };
 
-// A tile is 32 I0 + 32 I1 rows, its two halves, by 2 x 64 J columns.  bias [N] (or null) and limit: WIDE_CLAMPED.
+// A tile is 32 I0 + 32 I1 rows, its two halves, by 64 J gate rows and 64 J up rows of W.  bias [N] (or null) and limit: WIDE_CLAMPED.
 template <int OUT, int I0, int I1, int J>
 __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                            bf16_t* __restrict__ C, int M, int N, int K, int m_tiles, int n_tiles,
                                                            const bf16_t* __restrict__ bias, float limit) {
-    constexpr bool GATED = OUT != WIDE_WHOLE;
     constexpr int ROWS0 = 32 * I0, BM = ROWS0 + 32 * I1;
     extern __shared__ __attribute__((aligned(16))) unsigned char wide_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
     // Consecutive workgroups go to different dies.  A die takes an eighth of all tiles, neighbours in an order that walks bands of up
     // to eight rows of tiles column by column: what its CUs read at a time are about as many rows as columns, and no die has more
-    // than its share (5120 x 8192 at 2111 rows, 220 tiles: with whole columns for a die 33 tiles for some dies' 32 CUs).
+    // than its share (220 tiles in 20 columns: with whole columns for a die 33 tiles for some dies' 32 CUs).
     const int tiles = m_tiles * n_tiles, share = (tiles + 7) / 8, at = blockIdx.x / 8;
     const int id = blockIdx.x % 8 * share + at;
     if (at >= share || id >= tiles) return;
     const int bands = (m_tiles + 7) / 8, band = (m_tiles + bands - 1) / bands;
     const int b = id / (band * n_tiles), in_band = id - b * band * n_tiles;
     const int height = min(band, m_tiles - b * band), nt = in_band / height, mt = b * band + in_band - nt * height;
-    const int rows = GATED ? N / 2 : N;  // of a result
-    const int m0 = mt * BM, n0 = nt * (GATED ? 64 * J : 128 * J);
+    const int rows = N / 2;  // of a result
+    const int m0 = mt * BM, n0 = nt * (64 * J);
     const int steps = K / WIDE_BK;
     const bf16_t* xb = X + (int64_t)m0 * K;
     const bf16_t* wb0 = W + (int64_t)n0 * K;
-    const bf16_t* wb1 = GATED ? wb0 + (int64_t)rows * K : wb0;
+    const bf16_t* wb1 = wb0 + (int64_t)rows * K;
     // a load brings eight rows of 128 bytes, the eight wavefronts' 64; lane -> row lane / 8, physical piece lane % 8, the logical
     // piece that belongs there (rows behind the last read it again and are dropped).  Of 32 rows that are left of a half two
     // wavefronts bring the same eight, so that all have as many loads on their way.
     constexpr int LX0 = (I0 + 1) / 2, LX1 = (I1 + 1) / 2;  // a wavefront's loads of the halves
     auto group_of = [&](int rows32, int i) { return wave + 8 * i < 4 * rows32 ? wave + 8 * i : wave + 8 * i - 4; };
-    unsigned xo0[LX0], xo1[LX1], wo[2][J];
+    unsigned xo0[LX0], xo1[LX1], wo[J];
 #pragma unroll
     for (int i = 0; i < LX0; ++i) {
         const int r = 8 * group_of(I0, i) + lane / 8;
@@ -76,12 +76,10 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
         xo1[i] = (unsigned)min(ROWS0 + r, M - 1 - m0) * (unsigned)(K * 2) + ((lane % 8) ^ WIDE_SWIZZLE(r % 16)) * 16;
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < J; ++i) {
-            const int r = 8 * (wave + 8 * i) + lane / 8;
-            wo[h][i] = (unsigned)min((GATED ? 0 : 64 * J * h) + r, rows - 1 - n0) * (unsigned)(K * 2) + ((lane % 8) ^ WIDE_SWIZZLE(r % 16)) * 16;
-        }
+    for (int i = 0; i < J; ++i) {
+        const int r = 8 * (wave + 8 * i) + lane / 8;
+        wo[i] = (unsigned)min(r, rows - 1 - n0) * (unsigned)(K * 2) + ((lane % 8) ^ WIDE_SWIZZLE(r % 16)) * 16;
+    }
     // LDS: two buffers of the first half of X, of the second and of the second half of W; three of the first half of W
     constexpr int X0_BYTES = I0 * 4096, X1_BYTES = I1 * 4096, W_BYTES = J * 8192;
     constexpr int AT_X0 = 0, AT_X1 = 2 * X0_BYTES, AT_W1 = AT_X1 + 2 * X1_BYTES, AT_W0 = AT_W1 + 2 * W_BYTES;
@@ -99,7 +97,7 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
     auto issue_w = [&](int step, int at_lds, auto half) {
         constexpr int h = decltype(half)::value;
 #pragma unroll
-        for (int i = 0; i < J; ++i) dma(at_lds + (wave + 8 * i) * 1024, wo[h][i], (h ? wb1 : wb0) + step * WIDE_BK);
+        for (int i = 0; i < J; ++i) dma(at_lds + (wave + 8 * i) * 1024, wo[i], (h ? wb1 : wb0) + step * WIDE_BK);
     };
     const int group = wave / 4, wn = wave % 4;
     const int c = lane / 16, r16 = lane % 16;
@@ -205,28 +203,23 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
     auto put = [&](int m, int n, wf32x4 v, wf32x4 u) {  // (n: of the result's columns; u: the up rows' sums)
         if (m >= M || n >= rows) return;
         wbf16x4 out;
-        if constexpr (OUT == WIDE_WHOLE) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) out[e] = (bf16_t)v[e];
-        } else {
-            if (OUT == WIDE_CLAMPED && bias) {
-                const wbf16x4 bg = *(const wbf16x4*)(bias + n), bu = *(const wbf16x4*)(bias + rows + n);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] += (float)bg[e];
-                    u[e] += (float)bu[e];
-                }
-            }
-            // (the hardware's exponential and reciprocal, each good to a unit in the last place of 32 bits: what follows is rounded to 16)
+        if (OUT == WIDE_CLAMPED && bias) {
+            const wbf16x4 bg = *(const wbf16x4*)(bias + n), bu = *(const wbf16x4*)(bias + rows + n);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                constexpr float LOG2E = 1.44269504088896340736f;
-                if constexpr (OUT == WIDE_CLAMPED) {
-                    const float g = fminf(v[e], limit), w = fminf(fmaxf(u[e], -limit), limit);
-                    out[e] = (bf16_t)(g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.702f * LOG2E))) * (w + 1.0f));
-                } else {
-                    out[e] = (bf16_t)(v[e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * -LOG2E)) * u[e]);
-                }
+                v[e] += (float)bg[e];
+                u[e] += (float)bu[e];
+            }
+        }
+        // (the hardware's exponential and reciprocal, each good to a unit in the last place of 32 bits: what follows is rounded to 16)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            constexpr float LOG2E = 1.44269504088896340736f;
+            if constexpr (OUT == WIDE_CLAMPED) {
+                const float g = fminf(v[e], limit), w = fminf(fmaxf(u[e], -limit), limit);
+                out[e] = (bf16_t)(g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.702f * LOG2E))) * (w + 1.0f));
+            } else {
+                out[e] = (bf16_t)(v[e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * -LOG2E)) * u[e]);
             }
         }
         *(wbf16x4*)(C + (int64_t)m * rows + n) = out;
@@ -239,15 +232,14 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
             for (int j = 0; j < J; ++j) {
                 const int m = m0 + ROWS0 * a + 16 * (a ? I1 : I0) * group + 16 * i + r16, n = n0 + 16 * J * wn + 16 * j + 4 * c;
                 put(m, n, acc[a][0][i][j], acc[a][1][i][j]);
-                if constexpr (!GATED) put(m, n + 64 * J, acc[a][1][i][j], acc[a][1][i][j]);
             }
 }
 
 template <int OUT, int I0, int I1, int J>
 static int launch_wide(const void* X, const void* W, const void* bias, float limit, void* C, int M, int N, int K, hipStream_t stream) {
-    constexpr int BM = 32 * (I0 + I1), BN = OUT == WIDE_WHOLE ? 128 * J : 64 * J, LDS = 8192 * (I0 + I1) + 5 * 8192 * J;
+    constexpr int BM = 32 * (I0 + I1), BN = 64 * J, LDS = 8192 * (I0 + I1) + 5 * 8192 * J;
     static_assert(LDS <= 160 * 1024, "the LDS of a CU");
-    const int rows = OUT == WIDE_WHOLE ? N : N / 2, m_tiles = (M + BM - 1) / BM, n_tiles = (rows + BN - 1) / BN;
+    const int m_tiles = (M + BM - 1) / BM, n_tiles = (N / 2 + BN - 1) / BN;
     const int64_t blocks = ((int64_t)m_tiles * n_tiles + 7) / 8 * 8;
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
     auto kernel = gemm_wide_kernel<OUT, I0, I1, J>;
@@ -270,9 +262,6 @@ static const WideForm wide_forms[11] = {
     {256, 256, 6.5f, 0.97f, 0.36f}, {224, 256, 6.3f, 0.96f, 0.25f}, {192, 256, 4.2f, 0.98f, 0.14f}, {160, 256, 4.1f, 0.93f, 0.07f},
     {128, 256, 3.7f, 0.79f, 0.09f}, {288, 128, 4.4f, 0.84f, 0.10f}, {256, 128, 4.6f, 0.72f, 0.13f}, {224, 128, 5.1f, 0.70f, 0.09f},
     {192, 128, 4.4f, 0.68f, 0.07f}, {160, 128, 2.8f, 0.72f, -0.13f}, {128, 128, 2.1f, 0.67f, -0.16f}};
-// ... and of whole products (K up to 25600, fewer forms)
-static const WideForm whole_forms[3] = {{256, 256, 11.f, 0.87f, 0.40f}, {192, 256, 9.f, 0.77f, 0.30f}, {128, 256, 7.f, 0.63f, 0.20f}};
-static const int whole_form[3] = {0, 2, 4};  // ... which of wide_forms they are
 
 template <int OUT>
 static int launch_wide_form(const void* X, const void* W, const void* bias, float limit, void* C, int M, int N, int K, int form,
@@ -280,53 +269,44 @@ static int launch_wide_form(const void* X, const void* W, const void* bias, floa
 #define WIDE_CASE(F, I0, I1, J) \
     case F: return launch_wide<OUT, I0, I1, J>(X, W, bias, limit, C, M, N, K, stream);
     switch (form) {
-        WIDE_CASE(0, 4, 4, 2) WIDE_CASE(2, 3, 3, 2) WIDE_CASE(4, 2, 2, 2)
-    }
-    if constexpr (OUT != WIDE_WHOLE) {
-        switch (form) {
-            WIDE_CASE(1, 4, 3, 2) WIDE_CASE(3, 3, 2, 2) WIDE_CASE(5, 5, 4, 1) WIDE_CASE(6, 4, 4, 1)
-            WIDE_CASE(7, 4, 3, 1) WIDE_CASE(8, 3, 3, 1) WIDE_CASE(9, 3, 2, 1) WIDE_CASE(10, 2, 2, 1)
-        }
+        WIDE_CASE(0, 4, 4, 2) WIDE_CASE(1, 4, 3, 2) WIDE_CASE(2, 3, 3, 2) WIDE_CASE(3, 3, 2, 2)
+        WIDE_CASE(4, 2, 2, 2) WIDE_CASE(5, 5, 4, 1) WIDE_CASE(6, 4, 4, 1) WIDE_CASE(7, 4, 3, 1)
+        WIDE_CASE(8, 3, 3, 1) WIDE_CASE(9, 3, 2, 1) WIDE_CASE(10, 2, 2, 1)
     }
 #undef WIDE_CASE
     return (int)hipErrorInvalidValue;
 }
 
-// The form in which the product takes the least time (which of wide_forms, and one), or 0 where the library's product, with the
-// pass of its own that the activation takes, is expected to be as fast: gated 1.0 PFLOP/s or W at 6 TB/s, 9 us, and the activation's
-// 4.8 TB/s (slower than the library is at its best, and than this kernel nearly everywhere: of 102 measured sizes from 129 rows on
-// two of those that are taken are up to 1 % slower, the others 2 to 36 % faster, 14 % on average); whole 1.25 PFLOP/s and 5 us, where
-// less than 3 % slower (5120 x 25600 at 2111 rows 450 -> 430 us, 10240 x 5120 at 1500 rows 123 -> 115; the library reaches 0.8 to
-// 1.45 PFLOP/s, so products that it is slow at are left to it now and then).
-extern "C" int lle_gemm_wide_form(int M, int N, int K, int gated) {
-    if (M <= 128 || N <= 0 || K <= 0 || K % WIDE_BK != 0 || N % (gated ? 8 : 4) != 0 || (int64_t)320 * K * 2 > 0x7fffffff) return 0;
+// The form in which the product takes the least time (which of wide_forms, and one), or 0 where the library's product with the
+// pass of its own that the activation takes is expected to be as fast: 1.0 PFLOP/s or W at 6 TB/s, 9 us, and the activation's
+// 4.8 TB/s (slower than the library is at its best, and than this kernel nearly everywhere).
+extern "C" int lle_gemm_wide_form(int M, int N, int K) {
+    if (M <= 128 || N <= 0 || K <= 0 || K % WIDE_BK != 0 || N % 8 != 0 || (int64_t)320 * K * 2 > 0x7fffffff) return 0;
     const float stages = (float)(K / WIDE_BK), gflop = 2e-9f * M * N * K;
     float best = 0.f;
     int choice = 0;
-    for (int i = 0; i < (gated ? 11 : 3); ++i) {
-        const WideForm& v = gated ? wide_forms[i] : whole_forms[i];
+    for (int i = 0; i < 11; ++i) {
+        const WideForm& v = wide_forms[i];
         const int64_t tiles = (int64_t)((M + v.rows - 1) / v.rows) * ((N + v.columns - 1) / v.columns), whole = tiles / 256;
         const float rest = (float)(tiles - whole * 256) / 256.f;
         const float us = whole * (v.start + stages * (v.stage + v.full)) + (rest > 0.f ? v.start + stages * (v.stage + v.full * rest) : 0.f);
-        if (choice == 0 || us < best) best = us, choice = (gated ? i : whole_form[i]) + 1;
+        if (choice == 0 || us < best) best = us, choice = i + 1;
     }
-    const float library = gated ? 1.02f * (fmaxf(gflop, (float)N * K / 3e6f) + 9.f + (float)M * N / 1.6e6f) : 0.97f * (gflop / 1.25f + 5.f);
+    const float library = 1.02f * (fmaxf(gflop, (float)N * K / 3e6f) + 9.f + (float)M * N / 1.6e6f);
     return best < library ? choice : 0;
 }
 
-// X [M, K] and W [N, K] bfloat16, contiguous, 16-byte aligned; K a multiple of 64.  gated 0: C [M, N], N a multiple of 4.  gated 1: W
-// is gate rows and then up rows, C [M, N / 2] = silu(gate) . up, N a multiple of 8; gated 2: with bias [N] (or null) and limit,
-// g = min(gate + b, limit), u = clamp(up + b, -limit, limit), C = g sigmoid(1.702 g) (u + 1).  form: which of wide_forms (gated 0: 0, 2
-// or 4).
+// X [M, K] and W [N, K] bfloat16, contiguous, 16-byte aligned; K a multiple of 64, N of 8; W is gate rows and then up rows, C [M, N / 2].
+// gated 1: silu(gate) . up; gated 2: with bias [N] (or null) and limit, g = min(gate + b, limit), u = clamp(up + b, -limit, limit),
+// C = g sigmoid(1.702 g) (u + 1).  form: which of wide_forms.
 extern "C" int lle_gemm_wide_bf16(const void* X, const void* W, const void* bias, float limit, void* C, int M, int N, int K, int gated,
                                   int form, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K <= 0 || K % WIDE_BK != 0 || (int64_t)320 * K * 2 > 0x7fffffff || N % (gated ? 8 : 4) != 0) return (int)hipErrorInvalidValue;
+    if (K <= 0 || K % WIDE_BK != 0 || (int64_t)320 * K * 2 > 0x7fffffff || N % 8 != 0) return (int)hipErrorInvalidValue;
     if ((((uintptr_t)X | (uintptr_t)W) & 15) || (((uintptr_t)bias | (uintptr_t)C) & 7)) return (int)hipErrorInvalidValue;
     switch (gated) {
-        case 0: return launch_wide_form<WIDE_WHOLE>(X, W, nullptr, 0.f, C, M, N, K, form, stream);
-        case 1: return launch_wide_form<WIDE_SILU>(X, W, nullptr, 0.f, C, M, N, K, form, stream);
-        case 2:
+        case WIDE_SILU: return launch_wide_form<WIDE_SILU>(X, W, nullptr, 0.f, C, M, N, K, form, stream);
+        case WIDE_CLAMPED:
             if (!(limit > 0.f)) return (int)hipErrorInvalidValue;
             return launch_wide_form<WIDE_CLAMPED>(X, W, bias, limit, C, M, N, K, form, stream);
         default: return (int)hipErrorInvalidValue;

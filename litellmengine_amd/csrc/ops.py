@@ -339,10 +339,6 @@ class HipOps:
                 self._run("gemm", "lle_gemm_skinny_bf16", [_P, _P, _P, _I, _I, _I, _I, _P],
                           _ptr(x), _ptr(weight), _ptr(out), M, N, K, dtype_code(out_dtype))
                 return out
-            if out_dtype == torch.bfloat16:
-                form = self.wide_form(x, weight, gated=False)
-                if form >= 0:
-                    return self.linear_wide(x, weight, form)
             # the library product accumulates in 32-bit and can leave the result so
             return torch.mm(x, weight.t()) if out_dtype == torch.bfloat16 else torch.mm(x, weight.t(), out_dtype=out_dtype)
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
@@ -534,40 +530,39 @@ class HipOps:
             slices -= 1
         return slices if slices > 1 else 0
 
-    WIDE_FORMS = 11  # tiles of linear_wide (whole products: 0, 2 and 4 of them)
-
-    def wide_form(self, x, weight, gated: bool) -> int:
-        """In which tiles the tiled product of many rows takes this one (linear_wide), or -1 where the library stays: from the
-        sizes alone, but for operands that do not begin at 16 bytes, which only the library takes."""
+    def wide_form(self, x, weight) -> int:
+        """In which tiles (one of eleven) the tiled product of many rows takes gate and up (gated_wide), or -1 where the library and a
+        pass for the activation stay: from the sizes alone, but for operands that do not begin at 16 bytes, which only the
+        library takes."""
         M, K = x.shape
         if M <= 128 or self.force_library_gemm:
             return -1
-        key = (M, weight.shape[0], K, gated)
+        key = (M, weight.shape[0], K)
         form = self._wide.get(key)
         if form is None:
             fn = getattr(build.load_library("gemm_wide"), "lle_gemm_wide_form")
-            fn.argtypes, fn.restype = [_I, _I, _I, _I], _I
-            form = int(fn(M, weight.shape[0], K, int(gated))) - 1
+            fn.argtypes, fn.restype = [_I, _I, _I], _I
+            form = int(fn(M, weight.shape[0], K)) - 1
             if len(self._wide) >= 4096:
                 self._wide.clear()
             self._wide[key] = form
         return form if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else -1
 
-    def linear_wide(self, x, weight, form: int, activation: Optional[str] = None, bias=None, limit: float = 0.0) -> torch.Tensor:
-        """x [M, K] . weight [N, K]^T, bfloat16, in tiles of that form (see wide_form): [M, N].  `activation`: weight is gate rows
-        and then up rows, the result [M, N / 2] is silu(gate) * up, or ("clamp") what gate_up_clamped says."""
+    def gated_wide(self, x, weight, form: int, activation: str, bias=None, limit: float = 0.0) -> torch.Tensor:
+        """x [M, K], weight [N, K] (gate rows, then up rows), bfloat16, in tiles of that form (see wide_form) -> [M, N / 2]:
+        silu(gate) * up, or ("clamp") what gate_up_clamped says."""
         _dev(x, "x", torch.bfloat16)
         _dev(weight, "weight", torch.bfloat16)
         M, K = x.shape
         N = weight.shape[0]
         _need(weight.shape[1] == K and K % 64 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
-        _need(activation in (None, "silu", "clamp"), f"unknown activation {activation!r}")
+        _need(activation in ("silu", "clamp"), f"unknown activation {activation!r}")
         if bias is not None:
             _dev(bias, "bias", torch.bfloat16)
             _need(bias.shape == (N,), "bias must cover the whole weight")
-        out = torch.empty((M, N if activation is None else N // 2), dtype=torch.bfloat16, device=x.device)
+        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
         self._run("gemm_wide", "lle_gemm_wide_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
-                  float(limit), _ptr(out), M, N, K, (None, "silu", "clamp").index(activation), form)
+                  float(limit), _ptr(out), M, N, K, 1 + ("silu", "clamp").index(activation), form)
         return out
 
     def linear_slices(self, x, weight, slices: int) -> torch.Tensor:
@@ -1043,9 +1038,9 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
-        form = self.wide_form(x, weight, gated=True) if x.dtype == torch.bfloat16 else -1
+        form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 else -1
         if form >= 0:
-            return self.linear_wide(x, weight, form, "silu")
+            return self.gated_wide(x, weight, form, "silu")
         return self.silu_mul(self.linear(x, weight))
 
     def _gated_f32_in_one(self, M: int, N2: int, K: int) -> bool:
@@ -1080,9 +1075,9 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_clamped_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(bias), float(limit), _ptr(out), M, N2, K)
             return out
-        form = self.wide_form(x, weight, gated=True) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
+        form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
         if form >= 0 and (bias is None or bias.data_ptr() % 8 == 0):
-            return self.linear_wide(x, weight, form, "clamp", bias, limit)
+            return self.gated_wide(x, weight, form, "clamp", bias, limit)
         return self.bias_act(self.linear(x, weight), "clamp", True, bias=bias, limit=limit)
 
     # -- arrangements that norm a sublayer's output ------------------------------------
