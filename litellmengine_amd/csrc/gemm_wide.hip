@@ -277,22 +277,24 @@ static int launch_wide_form(const void* X, const void* W, const void* bias, floa
     return (int)hipErrorInvalidValue;
 }
 
-// The form in which the product takes the least time (which of wide_forms, and one), or 0 where the library's product with the
-// pass of its own that the activation takes is expected to be as fast: 1.0 PFLOP/s or W at 6 TB/s, 9 us, and the activation's
-// 4.8 TB/s (slower than the library is at its best, and than this kernel nearly everywhere).
-extern "C" int lle_gemm_wide_form(int M, int N, int K) {
-    if (M <= 128 || N <= 0 || K <= 0 || K % WIDE_BK != 0 || N % 8 != 0 || (int64_t)320 * K * 2 > 0x7fffffff) return 0;
+// The form in which the product takes the least time (which of wide_forms, and one) on a chip of `units` CUs, or 0 where the library's
+// product with the pass of its own that the activation takes is expected to be as fast: 1.0 PFLOP/s (256 CUs) or W at 6 TB/s, 9 us, and
+// the activation's 4.8 TB/s; slower than the library is at its best and than this kernel nearly everywhere.  481 sizes of 129 to
+// 8192 rows, 120 of them random: of the 429 that are taken 417 are not slower, 12 by 1 to 8 % (36864 x 4608 at 256 and 576 rows, 51200 x
+// 5120 at 300 to 384 and 576: the library's tiles happen to fit), all together 0.82 of the library's time.
+extern "C" int lle_gemm_wide_form(int M, int N, int K, int units) {
+    if (M <= 128 || N <= 0 || K <= 0 || units <= 0 || K % WIDE_BK != 0 || N % 8 != 0 || (int64_t)320 * K * 2 > 0x7fffffff) return 0;
     const float stages = (float)(K / WIDE_BK), gflop = 2e-9f * M * N * K;
     float best = 0.f;
     int choice = 0;
     for (int i = 0; i < 11; ++i) {
         const WideForm& v = wide_forms[i];
-        const int64_t tiles = (int64_t)((M + v.rows - 1) / v.rows) * ((N + v.columns - 1) / v.columns), whole = tiles / 256;
-        const float rest = (float)(tiles - whole * 256) / 256.f;
+        const int64_t tiles = (int64_t)((M + v.rows - 1) / v.rows) * ((N + v.columns - 1) / v.columns), whole = tiles / units;
+        const float rest = (float)(tiles - whole * units) / units;
         const float us = whole * (v.start + stages * (v.stage + v.full)) + (rest > 0.f ? v.start + stages * (v.stage + v.full * rest) : 0.f);
         if (choice == 0 || us < best) best = us, choice = i + 1;
     }
-    const float library = 1.02f * (fmaxf(gflop, (float)N * K / 3e6f) + 9.f + (float)M * N / 1.6e6f);
+    const float library = 0.97f * (fmaxf(gflop * 256.f / units, (float)N * K / 3e6f) + 9.f + (float)M * N / 1.6e6f);
     return best < library ? choice : 0;
 }
 

@@ -537,12 +537,12 @@ class HipOps:
         M, K = x.shape
         if M <= 128 or self.force_library_gemm:
             return -1
-        key = (M, weight.shape[0], K)
+        key = (M, weight.shape[0], K, self.compute_units())
         form = self._wide.get(key)
         if form is None:
             fn = getattr(build.load_library("gemm_wide"), "lle_gemm_wide_form")
-            fn.argtypes, fn.restype = [_I, _I, _I], _I
-            form = int(fn(M, weight.shape[0], K)) - 1
+            fn.argtypes, fn.restype = [_I, _I, _I, _I], _I
+            form = int(fn(*key)) - 1
             if len(self._wide) >= 4096:
                 self._wide.clear()
             self._wide[key] = form

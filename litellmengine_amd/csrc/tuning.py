@@ -3,7 +3,8 @@
 Every number here was found on an MI355X (256 CUs, HBM3E) with the weights of the Qwen3 sizes
 from 0.6B to 32B.  They sit in one object, `HipOps.tuning`, so that another chip or another family
 of widths replaces the numbers and not the code that reads them; `HipOps(tuning=...)` takes
-another set."""
+another set.  Models that are fitted to one kernel's own forms sit beside it: the tiles of gate and
+up (gemm_wide.hip), the float32 tiles and slices (gemm_f32.hip), the sums of slices (gemm_tile.hip)."""
 from __future__ import annotations
 
 import dataclasses

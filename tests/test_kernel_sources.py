@@ -1,4 +1,5 @@
 """What the kernels' sources promise and no run shows reliably."""
+import ctypes
 import glob
 import os
 import re
@@ -79,3 +80,12 @@ def test_loads_into_lds_wait_for_their_address(name, tmp_path):
     assert loads
     early = [code[i - 1 : i + 1] for i in loads if code[i - 1][1:2] == ["m0,"]]
     assert not early, (len(early), early[:3])
+
+
+def test_tiles_of_gate_and_up_follow_the_units_of_the_chip():
+    """Which tiles take a product is a matter of rounds, so of how many CUs there are; sizes that the kernel refuses are never taken."""
+    form = build.load_library("gemm_wide").lle_gemm_wide_form
+    form.argtypes = [ctypes.c_int] * 4
+    assert form(2048, 24576, 4096, 256) == 1 and form(262, 16384, 2048, 256) == 10 and form(262, 16384, 2048, 128) == 6
+    assert [form(m, 6144, 1024, 256) for m in (129, 144, 160)] == [0, 0, 0]  # (8 % slower there)
+    assert form(128, 24576, 4096, 256) == form(2048, 24576, 4090, 256) == form(2048, 24572, 4096, 256) == form(2048, 24576, 4096, 0) == 0
