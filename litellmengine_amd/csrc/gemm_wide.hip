@@ -211,7 +211,10 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(const bf16_t* __restr
                 u[e] += (float)bu[e];
             }
         }
-        // (the hardware's exponential and reciprocal, each good to a unit in the last place of 32 bits: what follows is rounded to 16)
+        // (The hardware's exponential and reciprocal, each good to a unit in the last place of 32 bits, and the exponent's rounding, 1e-7 of
+        // every unit of the gate: what follows is rounded to 16.  A reciprocal below the least normal number comes out as 0, so gates
+        // below -87.3 give 0; silu_mul gives the 1e-36 that is due down to -88.7.  Adding up a quarter of the sum keeps those too; it
+        // changes the last bits of everything else and measured 0.3 % slower.)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             constexpr float LOG2E = 1.44269504088896340736f;
