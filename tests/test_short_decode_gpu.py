@@ -154,3 +154,33 @@ def test_many_requests(dtype, nq, nkv, d, S, more):
     got = o.qk_norm_rope_attention(qkv, slots, None, None, cs, 1e-6, b, nq, nkv, d, True, table, seqs, cu, lens, None, None, d ** -0.5, n).double()
     assert (got - want).abs().max() < (2e-2 if dtype == torch.bfloat16 else 1e-4)  # (as above)
     assert (a.float() - b.float()).abs().max() <= (2.0 ** -7 * 8 if dtype == torch.bfloat16 else 1e-5)
+
+
+def test_which_float32_steps_of_a_runner_take_the_short_launch(monkeypatch):
+    """A decode step runs as a graph whose bound on the keys is 256 at least: with 8 kv heads the short launch is for 12 requests and
+    more, whatever their length.  Steps without graphs know how few keys there are."""
+    from litellmengine_amd.cache import CacheManager
+    from litellmengine_amd.config import Qwen3Config
+    from litellmengine_amd.engine import ModelRunner, StepEntry
+    from litellmengine_amd.models.build import random_model
+
+    config = Qwen3Config.from_dict(dict(architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=1, hidden_size=64,
+                                        num_attention_heads=8, num_key_value_heads=8, head_dim=64, intermediate_size=64, vocab_size=128,
+                                        rope_theta=1e4, rms_norm_eps=1e-6, tie_word_embeddings=True))
+    model = random_model(config, 3, "float32")
+    o, taken = model.ctx.ops, []
+    launch = o.qk_norm_rope_attention
+    monkeypatch.setattr(o, "qk_norm_rope_attention", lambda qkv, *a: taken.append(qkv.shape[0]) or launch(qkv, *a))
+    if o.compute_units() != 256:
+        pytest.skip("the rule counts workgroups for 256 CUs")
+    for graphs, want in ((True, [(1, False), (8, False), (12, True), (64, True), (100, False)]), (False, [(1, True), (8, True), (64, True), (100, False)])):
+        cache = CacheManager(model, page_size=16, num_pages=200, max_requests=128, dtype=torch.float32, device=model.ctx.device)
+        runner = ModelRunner(model, cache, use_graphs=graphs)
+        for n, short in want:
+            slots = [runner.admit() for _ in range(n)]
+            runner.step([StepEntry(s, [1, 2, 3], [2]) for s in slots])
+            taken.clear()
+            runner.step([StepEntry(s, [4], [0]) for s in slots])
+            assert bool(taken) == short, (graphs, n)
+            for s in slots:
+                runner.release(s)
