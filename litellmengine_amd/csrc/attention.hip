@@ -202,7 +202,6 @@ extern "C" int lle_paged_attention_generic(const void* q, const void* kv_layer, 
 typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
 typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define NEG_BIG (-1.0e30f)
 #define LAZY_MAX 8.0f  // a row's reference maximum may lag its true one by this much (base 2)
@@ -315,20 +314,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 __device__ __forceinline__ float max_of_8(const float (&x)[8]) {
     const float a = max3(x[0], x[1], x[2]), b = max3(x[3], x[4], x[5]);
     return max3(max3(x[6], x[7], a), b, b);
-}
-
-// The values of keys outside [lo, hi] become zeros; v[n][i] belongs to key `first` + i.  Their weight is 0, which drops whatever
-// lies there but an infinity or a NaN (pages are handed on as they are).
-template <int N>
-__device__ __forceinline__ void drop_values(bf16x8 (&v)[N], int first, int lo, int hi) {
-    u32x4 keep;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int j = first + 2 * i;
-        keep[i] = (j >= lo && j <= hi ? 0xffffu : 0u) | (j + 1 >= lo && j + 1 <= hi ? 0xffff0000u : 0u);
-    }
-#pragma unroll
-    for (int n = 0; n < N; ++n) v[n] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v[n]) & keep);
 }
 
 // One 32-key step for RT tiles of 16 rows.  load_k(x, ks): for lane (c, r16) key

@@ -88,6 +88,22 @@ __device__ __forceinline__ void load_into_lds(unsigned at, unsigned offset, cons
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
 }
 
+// The values of keys outside [lo, hi] become zeros; v[n][i], of eight 16-bit numbers, belongs to key `first` + i.  Their weight is
+// 0, which drops whatever lies there but an infinity or a NaN (pages are handed on as they are).
+template <typename Vec, int N>
+__device__ __forceinline__ void drop_values(Vec (&v)[N], int first, int lo, int hi) {
+    typedef uint32_t quad __attribute__((ext_vector_type(4)));
+    static_assert(sizeof(Vec) == sizeof(quad), "eight 16-bit numbers");
+    quad keep;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int j = first + 2 * i;
+        keep[i] = (j >= lo && j <= hi ? 0xffffu : 0u) | (j + 1 >= lo && j + 1 <= hi ? 0xffff0000u : 0u);
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] = __builtin_bit_cast(Vec, __builtin_bit_cast(quad, v[n]) & keep);
+}
+
 // Sum over a workgroup of up to 1024 threads; `smem` holds >= 16 floats.
 // Every thread gets the result; the order of the additions is fixed.
 __device__ __forceinline__ float block_sum(float v, float* smem) {

@@ -244,7 +244,7 @@ extern "C" int lle_latent_attention_generic(const void* q_lat, int q_lat_dtype, 
 // RK = 32-element steps over the latent (rank <= 32 RK, padded with zeros), RR the same for k_rot.
 // PAD: rank < 32 RK or rot < 32 RR, and the operands' tails are filled with zeros under a condition.
 // Without it every load is unconditional (a key outside the tile's range is read from the nearest one
-// inside it and masked afterwards; the pages hold finite numbers everywhere).
+// inside it and masked afterwards, its latents as a value cleared).
 // ---------------------------------------------------------------------------------------------
 typedef bf16_t lbf16x8 __attribute__((ext_vector_type(8)));
 typedef bf16_t lbf16x4 __attribute__((ext_vector_type(4)));
@@ -407,6 +407,10 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
             *(lbf16x4*)&s_p[buf][u][r][16 * wave + 4 * c] = pw;
         }
         __syncthreads();
+        if (j0 < lo_min || j0 + LAT_STEP - 1 > kmax) {  // (the same for the whole workgroup)
+            drop_values(va[0], j0 + 8 * c, lo_min, kmax);
+            drop_values(va[1], j0 + 32 + 8 * c, lo_min, kmax);
+        }
 #pragma unroll
         for (int u = 0; u < RT; ++u) {
             if (__any(alpha[u] != 1.0f)) {

@@ -306,10 +306,15 @@ __global__ __launch_bounds__(1024) void talking_values_kernel(TalkArgs a, const 
 #pragma unroll
             for (int i = 0; i < CNT; ++i) s_w[i * TV_ROW + threadIdx.x] = (bf16_t)w[i];
             __syncthreads();
+            const int j0 = __builtin_amdgcn_readfirstlane(lo16 + b0 + 256 * part);
 #pragma unroll
             for (int st = 0; st < 8; ++st) {
+                const int k0 = j0 + 32 * st;
+                if (k0 > pos) continue;  // (the same for the whole wavefront, and so is what follows)
+                bf16x8 v[1] = {vv[st]};
+                if (k0 < lo || k0 + 31 > pos) drop_values(v, k0 + 8 * c, lo, pos);
                 const bf16x8 p = *(const bf16x8*)(s_w + (r16 % CNT) * TV_ROW + 256 * part + 32 * st + 8 * c);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv[st], p, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[0], p, acc, 0, 0, 0);
             }
         }
         __syncthreads();
@@ -671,6 +676,8 @@ __global__ __launch_bounds__(512) void talking_prefill_kernel(TalkArgs a, const 
             bf16x8 w[BH];
 #pragma unroll
             for (int n = 0; n < BH; ++n) w[n] = *(const bf16x8*)(from + talk_w_at(r16, oh_local + n, c));
+            const int j0 = 32 * (first_step + i - 2);
+            if (j0 < key_lo || j0 + 31 > key_hi) drop_values(vreg, j0 + 8 * c, key_lo, key_hi);
 #pragma unroll
             for (int n = 0; n < BH; ++n)
 #pragma unroll

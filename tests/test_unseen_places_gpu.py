@@ -80,3 +80,48 @@ def test_the_new_tokens_place_and_those_behind_it(nq, nkv, d, P, window, lens, w
         want, got = (o.pair_rope_attention(qkv, slots, cs, p, nq, nkv, d, write, table, seq_slots, cu, kv_lens, window, scale, mk, 30.0)
                      for p in (pool, spoilt))
         assert want.isfinite().all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("P,rank,rot,H,lens,pasts,window", [(16, 96, 8, 5, [7, 1, 1], [0, 40, 300], None), (32, 512, 64, 16, [40, 1, 1], [100, 1900, 333], None),
+                                                            (16, 64, 32, 8, [1, 1, 1, 1], [0, 31, 32, 700], 50), (16, 128, 32, 4, [90, 1], [0, 70], 33)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_latents_that_no_row_sees(dtype, P, rank, rot, H, lens, pasts, window):
+    from tests.test_birelix_kernels_gpu import latent_case
+
+    c = latent_case(dtype, P, rank, rot, H, lens, pasts, 21, pages_total=160)
+    q_lat, q_rot = rnd((H, c["N"], rank), dtype, 24, 0.3).transpose(0, 1), rnd((c["N"], H, rot), torch.float32, 23)
+    pages = c["pages"].shape[0]
+    seen = torch.zeros((pages, P), dtype=torch.bool)
+    for s, (past, n) in enumerate(zip(pasts, lens)):
+        for j in range(max(0, past - window + 1) if window else 0, past + n):
+            seen[int(c["table"][int(c["seq_slots"][s]), j // P]), j % P] = True
+    bad, nobodys = c["pages"].clone().view(pages, -1), (~seen).cuda()  # a page: latents by key, latents by element, rotated keys
+    for part, by_key, width in ((0, True, rank), (P * rank, False, rank), (2 * P * rank, True, rot)):
+        view = bad[:, part : part + P * width].view(pages, P, width) if by_key else bad[:, part : part + P * width].view(pages, width, P).transpose(1, 2)
+        view.masked_fill_(nobodys[:, :, None], NAN)
+    assert bad.isnan().any()
+    run = lambda p: ops().latent_attention(q_lat, q_rot, p.view(c["pages"].shape), P, rank, rot, c["table"], c["seq_slots"], c["cu"], c["kv_lens"],
+                                           c["token_seq"], None, window, 0.11, max(lens), max(c["kv_lens"].tolist()), dtype)
+    want = run(c["pages"])
+    assert want.isfinite().all() and torch.equal(run(bad), want)
+
+
+@pytest.mark.parametrize("H,G,D,P", [(8, 4, 64, 16), (6, 2, 32, 16), (16, 2, 128, 16), (20, 5, 64, 48), (32, 8, 128, 16), (5, 1, 48, 8)])
+@pytest.mark.parametrize("chunk", [None, 24, 100])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_places_that_no_row_sees_with_heads_mixed(dtype, H, G, D, P, chunk):
+    from tests.test_telulorn_kernels_gpu import talking_case
+
+    for lens, pasts in (([1, 37, 2, 1, 61, 1], [100, 0, 47, 99, 130, 0]), ([1, 1, 1, 1], [190, 23, 24, 1500])):
+        args, most, slopes, talk = talking_case(dtype, lens, pasts, H, G, D, P)
+        _, kv, table, slots = args[:4]
+        seen = torch.zeros((kv.shape[0], P), dtype=torch.bool)
+        for s, (past, n) in enumerate(zip(pasts, lens)):
+            for j in range(past // chunk * chunk if chunk else 0, past + n):
+                seen[int(table[int(slots[s]), j // P]), j % P] = True
+        bad, nobodys = kv.clone(), (~seen).to(kv.device)
+        bad[:, 0].masked_fill_(nobodys[:, None, :, None], NAN)
+        bad[:, 1].view(kv.shape[0], G, D, P).masked_fill_(nobodys[:, None, None, :], NAN)
+        assert bad.isnan().any()
+        want, got = (ops().talking_attention(args[0], p, *args[2:], chunk, 0.2, slopes, talk, min(lens), max(lens), most) for p in (kv, bad))
+        assert want.isfinite().all() and torch.equal(got, want)
