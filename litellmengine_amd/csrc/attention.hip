@@ -1931,10 +1931,12 @@ struct F32Head {
 // short_decode_kernel in float32: one new token a request, at most SHORT_F32_KEYS keys, a wavefront for every 16 of them (past 176:
 // a second 16) and one for the new token; products on the float32 matrix instruction as in mfma_f32_attention_kernel (1024 cycles for the scores of
 // 16 keys of 128, as many for the values: V flies under the scores).  Twelve wavefronts leave a lane the 168 registers that a
-// head, its weights, its rotation and K need side by side.  0.6B sizes (16 q heads, 8 kv heads of 128) at 97 keys, 1 / 8 / 32
-// requests: 9.0 / 10.0 / 12.0 us in two launches (rotation and cache write, attention), 7.0 / 7.7 / 9.1 here; 32 requests at 200 keys
-// 19.2 and 15.7, 8 at 256 11.4 and 12.5 (there the two launches' key splits reach CUs that this one leaves idle; which of them
-// takes a step is can_fuse_rope_attention's to say).  Tried and not kept: the second step's K asked for before the first's values.
+// head, its weights, its rotation and K need side by side.  0.6B sizes (16 q heads, 8 kv heads of 128) at 97 keys, 32 requests:
+// 12.0 us in two launches (rotation and cache write, attention), 9.1 here; at 200 keys 19.2 and 15.7.  1 / 8 requests 9.0 / 10.0 and
+// 7.0 / 7.7, at 256 keys 8 requests 11.4 and 12.5 (the two launches' key splits reach CUs that this one leaves idle).  Which of
+// them takes a step is can_fuse_rope_attention's to say, from the bound on the keys that it is given: a step that runs as a graph
+// has a bound of 256 at least, so there 1 to 11 requests of 8 kv heads are the two launches' whatever their length.  Tried and
+// not kept: the second step's K asked for before the first's values.
 #define SHORT_F32_WAVES 11
 #define SHORT_F32_KEYS 256
 static_assert(SHORT_F32_KEYS <= 2 * SHORT_F32_WAVES * F32_KEYS, "two steps a wavefront");

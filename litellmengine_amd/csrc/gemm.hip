@@ -143,16 +143,16 @@ template <typename T, int WAVES = 16> struct SkShare {
 // the factor r[m] commutes with the product that follows, so
 //   RESID (the product before the norm): its result is the delta of the residual stream; the
 //     epilogue forms h = hidden + delta in 32-bit, writes it back, writes xw = h * w as the
-//     next product's input, and leaves the sum of h^2 over its 16 columns per row in
-//     ss_part[16 MT][workgroups];
+//     next product's input, and leaves the sums of h^2 over its columns per row in ss_part[16 or 32 rows][parts] (a part a
+//     workgroup, or two);
 //   SCALED (the product after the norm): adds up the parts, and multiplies its rows by r[m].
 struct NormFold {
     float* hidden;          // RESID: residual stream [M, N], read and written
     const void* weight;     // RESID: norm weight [N]
     int weight_dtype;
     bf16_t* xw;             // RESID: out, [M, N]
-    float* ss_out;          // RESID: out, [16][workgroups]
-    const float* ss_in;     // SCALED: [16][parts]
+    float* ss_out;          // RESID: out, [16][parts]; SPLIT: [32][parts]
+    const float* ss_in;     // SCALED: the same
     int parts;              // SCALED, SPLIT
     int part_rows;          // SPLIT: columns of a part, all of the tile's or half of them
     float eps;              // SCALED
@@ -882,7 +882,8 @@ static int skinny_tile_rows(int rows) {
     return per_tile < 1 ? 1 : (per_tile > 16 ? 16 : per_tile);
 }
 
-// tiles of lle_gemm_skinny_resid_bf16 for a weight of N rows at up to 16 rows of X: the second size of its ss_part
+// parts of lle_gemm_skinny_resid_bf16's sums of squares for a weight of N rows (its tiles at up to 16 rows of X): the second size of
+// its ss_part
 extern "C" int lle_gemm_skinny_resid_parts(int N) {
     if (N <= 0) return 0;
     const int tr = skinny_tile_rows(N);
@@ -954,7 +955,7 @@ extern "C" int lle_gemm_skinny_clamped_bf16(const void* X, const void* W, const 
 
 // The product BEFORE a folded norm: delta = X W^T [M, N] is added into `hidden` (float32 [M, N],
 // in place), xw = hidden * norm_weight goes to `xw` (bfloat16 [M, N]) and the sums of squares of
-// the new hidden over each workgroup's columns to ss_part [16 or 32][lle_gemm_skinny_resid_parts(N)]
+// the new hidden over each part's columns to ss_part [16 or 32][lle_gemm_skinny_resid_parts(N)]
 // (32 rows when M > 16).  1 <= M <= 32.
 extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hidden, const void* norm_weight,
                                           int weight_dtype, void* xw, void* ss_part, int M, int N, int K,

@@ -749,8 +749,9 @@ class HipOps:
         """qk_norm_rope_write and paged_attention of a decode step in one launch (see
         can_fuse_rope_attention): the workgroup whose keys include a new token's position writes
         its K and V, every workgroup norms and rotates the q rows it multiplies.  `order` (int32 [S], or None):
-        the requests in the order in which they are started, see decode_order.  `max_kv_len`: a host-side bound; it chooses the
-        kernel and its key splits, never the result.  `token_seq` None: every request has one token."""
+        the requests in the order in which they are started, see decode_order.  `max_kv_len`: a bound on kv_lens; it chooses the
+        kernel and its key splits, never the result (a request longer than it says may lose keys).  `token_seq` None: every
+        request has one token; with few keys then, and always in float32, it is the launch of a wavefront for every few keys."""
         f32 = qkv.dtype == torch.float32
         _dev(qkv, "qkv", torch.float32 if f32 else torch.bfloat16)
         _dev(kv_layer, "kv_layer", qkv.dtype)
