@@ -78,7 +78,8 @@ extern "C" int lle_gemm_nt_simt(const void* A, const void* B, void* C, int M, in
 
 // ---------------------------------------------------------------------------------
 // Skinny product for decoding: M <= 64 rows of activations against a weight
-// matrix that is read exactly once.  bfloat16 in, 32-bit accumulate, bfloat16 or
+// matrix that is read exactly once (gemm_lines_kernel takes what it can of it, see there; this one float32 and
+// what has no whole lines, few columns, odd addresses or more rows).  bfloat16 in, 32-bit accumulate, bfloat16 or
 // 32-bit out.  HBM-bound: the kernel is shaped to keep whole 128-byte lines of W
 // in flight from all CUs.
 //   workgroup = 16 rows of W (one matrix-core tile), 16 wavefronts split K:
@@ -176,6 +177,115 @@ __device__ __forceinline__ float gated_result(float g, float u, const NormFold& 
     return g / (1.0f + expf(-g)) * u;
 }
 
+// What the kernels around a folded norm ask for at their start, and what they do behind their products.
+//
+// RESID: thread (m, n) of the first 256 owns element [m][n0 + n] of every 16 rows.  What it needs of the residual stream and of the
+// norm weight has arrived by the epilogue (all threads ask, for places that are there; the bits of the weight are read as
+// they lie and interpreted in the epilogue).
+template <int MT>
+struct ResidRows {
+    float h[MT];
+    uint32_t w;
+    __device__ __forceinline__ void load(const NormFold& fold, int64_t n0, int tile_rows, int M, int N) {
+        const int64_t col = min(n0 + min((int)(threadIdx.x % 16), tile_rows - 1), (int64_t)N - 1);
+        if (fold.weight_dtype == LLE_F32)
+            w = ((const uint32_t*)fold.weight)[col];
+        else
+            w = ((const uint16_t*)fold.weight)[col];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) h[mt] = fold.hidden[(int64_t)min(16 * mt + (int)(threadIdx.x / 16) % 16, M - 1) * N + col];
+    }
+};
+// SCALED: wavefront w adds up the parts of the rows w, w + WAVES, ...  The first parts are asked for at the start and added after the
+// products.
+template <int MT, int WAVES>
+struct NormParts {
+    static constexpr int EARLY = 4, ROWS = (16 * MT + WAVES - 1) / WAVES;
+    float early[ROWS][EARLY];
+    __device__ __forceinline__ void load(const NormFold& fold, int wave, int lane, int M) {
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+#pragma unroll
+            for (int i = 0; i < EARLY; ++i)  // past the parts: the last one again, dropped below; past the rows likewise
+                early[j][i] = fold.ss_in[min(wave + WAVES * j, M - 1) * fold.parts + min(lane + LLE_WAVE * i, fold.parts - 1)];
+    }
+    __device__ __forceinline__ void finish(const NormFold& fold, int wave, int lane, int M, int K, float* s_inv) const {
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) {
+            const int m = wave + WAVES * j;
+            if (m >= M) break;  // (the same for the whole wavefront)
+            float part = 0.f;
+#pragma unroll
+            for (int i = 0; i < EARLY; ++i) part += lane + LLE_WAVE * i < fold.parts ? early[j][i] : 0.f;
+            // what is left: four loads at a time (one after the other would each pay the way from memory)
+            const float* in = fold.ss_in + (int64_t)m * fold.parts;
+            for (int b = lane + LLE_WAVE * EARLY; b < fold.parts; b += 4 * LLE_WAVE) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = in[min(b + i * LLE_WAVE, fold.parts - 1)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part += b + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
+            }
+            part = wave_sum(part);
+            if (lane == 0) s_inv[m] = 1.0f / sqrtf(part / (float)K + fold.eps);
+        }
+    }
+};
+// The epilogue: total(nt, mt, n, m) adds up the wavefronts' partial sums in their order.
+template <int WAVES, int MT, int NT, bool GATED, bool RESID, bool SCALED, bool SPLIT, typename T, typename TC, typename Total>
+__device__ __forceinline__ void finish_skinny(const Total& total, TC* C, int M, int N, int64_t n0, int tile_rows, const NormFold& fold,
+                                              const ResidRows<MT>& resid, const float* s_inv) {
+    if (GATED) {
+        for (int idx = threadIdx.x; idx < MT * 256; idx += WAVES * LLE_WAVE) {
+            const int mt = idx / 256, m = (idx / 16) % 16, n = idx % 16;
+            const int64_t row = 16 * mt + m, col = n0 + n;
+            if (row >= M || col >= N / 2 || n >= tile_rows) continue;
+            float g = total(0, mt, n, m), u = total(NT - 1, mt, n, m);
+            if (SCALED) {
+                g *= s_inv[16 * mt + m];
+                u *= s_inv[16 * mt + m];
+            }
+            C[row * (N / 2) + col] = from_f32<TC>(gated_result(g, u, fold, col, N / 2));
+        }
+        return;
+    }
+    if (RESID) {  // NT = 1
+        if (threadIdx.x < 256) {
+            const int n = threadIdx.x % 16;
+            const int64_t col = n0 + n;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int m16 = threadIdx.x / 16, m = 16 * mt + m16;
+                float sq = 0.f;
+                if (m < M && col < N && n < tile_rows) {
+                    const float h = resid.h[mt] + total(0, mt, n, m16);
+                    fold.hidden[(int64_t)m * N + col] = h;
+                    ((T*)fold.xw)[(int64_t)m * N + col] =
+                        (T)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid.w : resid.w << 16));
+                    sq = h * h;
+                }
+                if (!SPLIT || fold.part_rows == tile_rows) {  // (the same for the whole launch)
+                    sq = row16_sum(sq);
+                    if (n == 0) fold.ss_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
+                } else {
+                    const float first = row16_sum(n < fold.part_rows ? sq : 0.f), second = row16_sum(n < fold.part_rows ? 0.f : sq);
+                    const int part = 2 * blockIdx.x + n;
+                    if (n < 2 && part < fold.parts) fold.ss_out[(int64_t)m * fold.parts + part] = n == 0 ? first : second;
+                }
+            }
+        }
+        return;
+    }
+    for (int idx = threadIdx.x; idx < NT * MT * 256; idx += WAVES * LLE_WAVE) {
+        const int nt = idx / (MT * 256), mt = (idx / 256) % MT, m = (idx / 16) % 16, n = idx % 16;
+        const int64_t row = 16 * mt + m, col = n0 + 16 * nt + n;
+        if (row >= M || col >= N || (NT == 1 && n >= tile_rows)) continue;
+        float sum = total(nt, mt, n, m);
+        if (SCALED) sum *= s_inv[16 * mt + m];
+        C[row * N + col] = from_f32<TC>(sum);
+    }
+}
+
 // SPLIT (RESID): the rows of X are dealt out sixteen a workgroup, see lle_gemm_skinny_resid_bf16.
 template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int SK_WAVES, int UNROLL, bool SPLIT = false>
 // one tile of W and up to 16 rows of X: two workgroups of 16 wavefronts a CU (8 wavefronts a SIMD),
@@ -213,37 +323,12 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
         fold.xw += (int64_t)before * N;
         fold.ss_out += (int64_t)before * fold.parts;
     }
-    // SCALED: wavefront w adds up the parts of the rows w, w + SK_WAVES, ...  The first parts are asked for now and added after
-    // the products.
-    constexpr int EARLY_PARTS = 4, SUM_ROWS = (16 * MT + SK_WAVES - 1) / SK_WAVES;
-    float early[SUM_ROWS][EARLY_PARTS];
-    if (SCALED) {
-#pragma unroll
-        for (int j = 0; j < SUM_ROWS; ++j)
-#pragma unroll
-            for (int i = 0; i < EARLY_PARTS; ++i)  // past the parts: the last one again, dropped below; past the rows likewise
-                early[j][i] = fold.ss_in[min(wave + SK_WAVES * j, M - 1) * fold.parts + min(lane + LLE_WAVE * i, fold.parts - 1)];
-    }
+    NormParts<MT, SK_WAVES> parts;
+    if (SCALED) parts.load(fold, wave, lane, M);
     const int c = lane / 16, r16 = lane % 16;
     const int64_t n0 = (int64_t)blockIdx.x * ((GATED || NT == 1) ? tile_rows : 16 * NT);
-    // RESID: thread (m, n) of the first 256 owns element [m][n0 + n]; what it needs of the
-    // residual stream and of the norm weight is asked for now and has arrived by the epilogue
-    // (all threads ask, for places that are there; the bits of the weight are read as they lie
-    // and interpreted in the epilogue)
-    float resid_h[MT];
-    uint32_t resid_w = 0;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) resid_h[mt] = 0.f;
-    if (RESID) {
-        const int64_t col = min(n0 + min((int)(threadIdx.x % 16), tile_rows - 1), (int64_t)N - 1);
-        if (fold.weight_dtype == LLE_F32)
-            resid_w = ((const uint32_t*)fold.weight)[col];
-        else
-            resid_w = ((const uint16_t*)fold.weight)[col];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-            resid_h[mt] = fold.hidden[(int64_t)min(16 * mt + (int)(threadIdx.x / 16) % 16, M - 1) * N + col];
-    }
+    ResidRows<MT> resid;
+    if (RESID) resid.load(fold, n0, tile_rows, M, N);
     const T* wp[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -325,27 +410,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
             }
         }
     }
-    if (SCALED) {
-#pragma unroll
-        for (int j = 0; j < SUM_ROWS; ++j) {
-            const int m = wave + SK_WAVES * j;
-            if (m >= M) break;  // (the same for the whole wavefront)
-            float part = 0.f;
-#pragma unroll
-            for (int i = 0; i < EARLY_PARTS; ++i) part += lane + LLE_WAVE * i < fold.parts ? early[j][i] : 0.f;
-            // what is left: four loads at a time (one after the other would each pay the way from memory)
-            const float* in = fold.ss_in + (int64_t)m * fold.parts;
-            for (int b = lane + LLE_WAVE * EARLY_PARTS; b < fold.parts; b += 4 * LLE_WAVE) {
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = in[min(b + i * LLE_WAVE, fold.parts - 1)];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) part += b + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
-            }
-            part = wave_sum(part);
-            if (lane == 0) s_inv[m] = 1.0f / sqrtf(part / (float)K + fold.eps);
-        }
-    }
+    if (SCALED) parts.finish(fold, wave, lane, M, K, s_inv);
     // lane holds C^T[n = 4c + i][m = r16]
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -354,65 +419,13 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
 #pragma unroll
             for (int i = 0; i < 4; ++i) s_acc[wave][nt][mt][4 * c + i][r16] = acc[nt][mt][i];
     __syncthreads();
-    if (GATED) {
-        for (int idx = threadIdx.x; idx < MT * 256; idx += blockDim.x) {
-            const int mt = idx / 256, m = (idx / 16) % 16, n = idx % 16;
-            const int64_t row = 16 * mt + m, col = n0 + n;
-            if (row >= M || col >= N / 2 || n >= tile_rows) continue;
-            float g = 0.f, u = 0.f;
-#pragma unroll
-            for (int w = 0; w < SK_WAVES; ++w) {
-                g += s_acc[w][0][mt][n][m];
-                u += s_acc[w][NT - 1][mt][n][m];
-            }
-            if (SCALED) {
-                g *= s_inv[16 * mt + m];
-                u *= s_inv[16 * mt + m];
-            }
-            C[row * (N / 2) + col] = from_f32<TC>(gated_result(g, u, fold, col, N / 2));
-        }
-        return;
-    }
-    if (RESID) {  // NT = 1
-        if (threadIdx.x < 256) {
-            const int n = threadIdx.x % 16;
-            const int64_t col = n0 + n;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int m16 = threadIdx.x / 16, m = 16 * mt + m16;
-                float sq = 0.f;
-                if (m < M && col < N && n < tile_rows) {
-                    float sum = 0.f;
-#pragma unroll
-                    for (int w = 0; w < SK_WAVES; ++w) sum += s_acc[w][0][mt][n][m16];
-                    const float h = resid_h[mt] + sum;
-                    fold.hidden[(int64_t)m * N + col] = h;
-                    ((T*)fold.xw)[(int64_t)m * N + col] =
-                        (T)(h * __uint_as_float(fold.weight_dtype == LLE_F32 ? resid_w : resid_w << 16));
-                    sq = h * h;
-                }
-                if (!SPLIT || fold.part_rows == tile_rows) {  // (the same for the whole launch)
-                    sq = row16_sum(sq);
-                    if (n == 0) fold.ss_out[(int64_t)m * gridDim.x + blockIdx.x] = sq;
-                } else {
-                    const float first = row16_sum(n < fold.part_rows ? sq : 0.f), second = row16_sum(n < fold.part_rows ? 0.f : sq);
-                    const int part = 2 * blockIdx.x + n;
-                    if (n < 2 && part < fold.parts) fold.ss_out[(int64_t)m * fold.parts + part] = n == 0 ? first : second;
-                }
-            }
-        }
-        return;
-    }
-    for (int idx = threadIdx.x; idx < NT * MT * 256; idx += blockDim.x) {
-        const int nt = idx / (MT * 256), mt = (idx / 256) % MT, m = (idx / 16) % 16, n = idx % 16;
-        const int64_t row = 16 * mt + m, col = n0 + 16 * nt + n;
-        if (row >= M || col >= N || (NT == 1 && n >= tile_rows)) continue;
+    auto total = [&](int nt, int mt, int n, int m) {
         float sum = 0.f;
 #pragma unroll
         for (int w = 0; w < SK_WAVES; ++w) sum += s_acc[w][nt][mt][n][m];
-        if (SCALED) sum *= s_inv[16 * mt + m];
-        C[row * N + col] = from_f32<TC>(sum);
-    }
+        return sum;
+    };
+    finish_skinny<SK_WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
 }
 
 // ---------------------------------------------------------------------------------
@@ -882,6 +895,195 @@ static int skinny_tile_rows(int rows) {
     return per_tile < 1 ? 1 : (per_tile > 16 ? 16 : per_tile);
 }
 
+
+// ---------------------------------------------------------------------------------
+// The same by way of LDS: bfloat16, up to 32 rows of X, K a multiple of 64 from 1024 on.  The same products and sums in the same order,
+// bit for bit; only the operands' way is another one.
+// What bounds gemm_skinny_kernel is a CU's vector cache: a load to registers costs it four cycles for every line of 128 bytes that it
+// touches, and loads as the matrix instruction wants its operands touch sixteen lines for half of each (16 bytes a cycle, 38 B/ns
+// a CU, for W and for X; whole lines 75), while loads straight into LDS, here eight whole lines at a time, bring 85 to 118
+// B/ns.  So every wavefront copies its 64 columns of a step of the tile's rows and of X's into LDS of its own and multiplies
+// from there: no barrier, it waits for its own loads.  It has up to DEPTH steps on their way, as many as 160 KB hold; a step's
+// buffer takes the next load when it has been read.  The wavefronts' sums take the place of their operands.
+// WH, XH: loads of eight rows for a tile of W and for sixteen rows of X (one where there are no more than eight).
+// Launches in a HIP graph, weights from memory, gemm_skinny_kernel -> this one in us at 1 / 8 / 16 / 32 rows of X (norm folded as in
+// a model): 4096 x 1024 4.3 / 4.5 / 4.9 / 6.3 -> 3.7 / 3.8 / 4.4 / 5.5; 6144 x 1024 gated 5.0 / 5.3 / 6.0 / 7.2 -> 4.7 / 4.9 / 5.2 /
+// 6.3; 1024 x 2048 3.9 / 4.6 / 5.4 / 5.7 -> 3.5 / 3.6 / 3.8 / 3.9; 1024 x 3072 5.1 / 5.8 / 6.9 / 7.3 -> 4.1 / 4.3 / 5.1 / 5.4; 2048 x
+// 8192 at up to 16 rows 11.1 / 11.9 / 14.7 -> 7.7 / 7.9 / 10.2; 4096 x 4096 8.4 / 9.5 / 12.1 -> 8.2 / 8.3 / 8.8; 4096 x 12288 20.2 / 22.5 /
+// 28.8 -> 18.9 / 18.9 / 21.8 (5.3 TB/s); 5120 x 25600 54.8 / 64.8 / 81.3 -> 48.2 / 50.9 / 65.5.
+// ---------------------------------------------------------------------------------
+// where piece p (16 bytes) of row r lies in its 128 bytes of LDS: p ^ this.  A 16-byte read serves sixteen lanes a cycle, rows with
+// r / 4 in {0, 3} at piece 2 c + e and the others at that of the next c (or the other way round): they meet every bank once.
+#define LINES_SWIZZLE(r) ((((r) >> 1) & 7) ^ (((((r) >> 3) ^ ((r) >> 2)) & 1) << 1))
+#define LINES_LDS (160 * 1024 - 256)  // (of a CU, less what the row factors take)
+
+// bytes of LDS of a wavefront
+static constexpr int lines_bytes(int loads, int depth, int tiles) {
+    const int operands = depth * loads * 1024, sums = tiles * 16 * 17 * 4;
+    return operands > sums ? operands : (sums + 1023) / 1024 * 1024;
+}
+
+template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, int DEPTH, bool SPLIT>
+__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                   TC* __restrict__ C, int M, int N, int K, int tile_rows, NormFold fold) {
+    constexpr int WAVES = 16, LOADS = NT * WH + MT * XH, STEP = LOADS * 1024, OWN = lines_bytes(LOADS, DEPTH, NT * MT);
+    static_assert(NT == (GATED ? 2 : 1) && WAVES * OWN <= LINES_LDS, "a tile of W, and of the up rows; the LDS of a CU");
+    extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
+    __shared__ float s_inv[16 * MT];
+    if constexpr (RESID || SCALED)  // (all arguments in one go, as gemm_skinny_kernel)
+        asm volatile("" ::"s"(X), "s"(W), "s"(C), "s"(M), "s"(N), "s"(K), "s"(tile_rows), "s"(fold.hidden), "s"(fold.weight),
+                     "s"(fold.weight_dtype), "s"(fold.xw), "s"(fold.ss_out), "s"(fold.ss_in), "s"(fold.parts),
+                     "s"(fold.eps));
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    if (SPLIT && blockIdx.y > 0) {
+        const int before = 16 * blockIdx.y;
+        X += (int64_t)before * K;
+        M -= before;
+        fold.hidden += (int64_t)before * N;
+        fold.xw += (int64_t)before * N;
+        fold.ss_out += (int64_t)before * fold.parts;
+    }
+    const int64_t n0 = (int64_t)blockIdx.x * tile_rows;
+    const int rows = GATED ? N / 2 : N;
+    // a load: lane -> row lane / 8, physical piece lane % 8, the logical piece that belongs there; rows behind the tile's and X's last
+    // one read it again and are dropped
+    unsigned wo[WH], xo[MT][XH];
+#pragma unroll
+    for (int h = 0; h < WH; ++h) {
+        const int r = 8 * h + lane / 8;
+        wo[h] = (unsigned)min(min(r, tile_rows - 1), rows - 1 - (int)n0) * (unsigned)(K * 2) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int h = 0; h < XH; ++h) {
+            const int r = 8 * h + lane / 8;
+            xo[mt][h] = (unsigned)min(16 * mt + r, M - 1) * (unsigned)(K * 2) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
+        }
+    unsigned char* own = lines_lds + wave * OWN;
+    const unsigned own_at = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lines_lds + wave * OWN;
+    const bf16_t *wb = W + n0 * K + wave * SK_KSTEP, *xb = X + wave * SK_KSTEP;
+    auto issue = [&](int step, int buf) {
+        const int64_t k = (int64_t)step * (SK_KSTEP * WAVES);
+        const unsigned at = own_at + buf * STEP;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int h = 0; h < WH; ++h) load_into_lds(at + (nt * WH + h) * 1024, wo[h], wb + k + (nt ? (int64_t)rows * K : 0));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int h = 0; h < XH; ++h) load_into_lds(at + (NT * WH + mt * XH + h) * 1024, xo[mt][h], xb + k);
+    };
+    NormParts<MT, WAVES> parts;
+    if (SCALED) parts.load(fold, wave, lane, M);
+    ResidRows<MT> resid;
+    if (RESID) resid.load(fold, n0, tile_rows, M, N);
+    const int steps = (K / SK_KSTEP - wave + WAVES - 1) / WAVES;  // of this wavefront: DEPTH or more
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) issue(d, d);
+    // lane (c, r) reads pieces 2 c and 2 c + 1 of row r (of eight rows: each twice)
+    const int c = lane / 16, r16 = lane % 16;
+    int w_at[2], x_at[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int wr = WH == 1 ? r16 % 8 : r16, xr = XH == 1 ? r16 % 8 : r16;
+        w_at[e] = wr * 128 + ((2 * c + e) ^ LINES_SWIZZLE(wr)) * 16;
+        x_at[e] = xr * 128 + ((2 * c + e) ^ LINES_SWIZZLE(xr)) * 16;
+    }
+    gf32x4 acc[NT][MT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
+    int buf = 0;
+    // the next step: `behind` steps have been asked for after it
+    auto multiply = [&](auto behind) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(behind)::value * LOADS) : "memory");
+        const unsigned char* at = own + buf * STEP;
+        gbf16x8 w[NT][2], x[MT][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) w[nt][e] = *(const gbf16x8*)(at + nt * WH * 1024 + w_at[e]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) x[mt][e] = *(const gbf16x8*)(at + (NT * WH + mt * XH) * 1024 + x_at[e]);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) acc[nt][mt] = SkOp<bf16_t>::mma(w[nt][e], x[mt][e], acc[nt][mt]);
+    };
+    auto next = [&]() { buf = buf == DEPTH - 1 ? 0 : buf + 1; };
+    for (int step = 0; step + DEPTH < steps; ++step, next()) {
+        multiply(std::integral_constant<int, DEPTH - 1>{});
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the buffer has been read
+        issue(step + DEPTH, buf);
+    }
+    if constexpr (DEPTH >= 5) multiply(std::integral_constant<int, 4>{}), next();
+    if constexpr (DEPTH >= 4) multiply(std::integral_constant<int, 3>{}), next();
+    if constexpr (DEPTH >= 3) multiply(std::integral_constant<int, 2>{}), next();
+    if constexpr (DEPTH >= 2) multiply(std::integral_constant<int, 1>{}), next();
+    multiply(std::integral_constant<int, 0>{});
+    if (SCALED) parts.finish(fold, wave, lane, M, K, s_inv);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // lane holds C^T[n = 4c + i][m = r16]
+    float* mine = (float*)own;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mine[((nt * MT + mt) * 16 + 4 * c + i) * 17 + r16] = acc[nt][mt][i];
+    __syncthreads();
+    auto total = [&](int nt, int mt, int n, int m) {
+        const unsigned char* at = lines_lds + (((nt * MT + mt) * 16 + n) * 17 + m) * 4;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += *(const float*)(at + w * OWN);
+        return sum;
+    };
+    finish_skinny<WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, bf16_t>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
+}
+
+// DEPTH: the most steps that LDS holds, up to 5, and up to what the wavefront with the fewest has.
+template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, bool SPLIT, int DEPTH>
+static hipError_t launch_lines_depth(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
+                                     hipStream_t stream) {
+    constexpr int LDS = 16 * lines_bytes(NT * WH + MT * XH, DEPTH, NT * MT);
+    if constexpr (LDS > LINES_LDS) {
+        return launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
+    } else if (DEPTH > 1 && K / (16 * SK_KSTEP) < DEPTH) {
+        return launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH == 1 ? 1 : DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
+    } else {
+        auto kernel = gemm_lines_kernel<MT, NT, GATED, RESID, SCALED, TC, WH, XH, DEPTH, SPLIT>;
+        static std::atomic<uint64_t> granted{0};
+        const hipError_t e = lle_grant_lds((const void*)kernel, LDS, granted);
+        if (e != hipSuccess) return e;
+        kernel<<<dim3(blocks, SPLIT ? 2 : 1), 16 * LLE_WAVE, LDS, stream>>>(X, W, C, M, N, K, tile_rows, fold);
+        return hipGetLastError();
+    }
+}
+
+// Whether gemm_lines_kernel takes a product of up to 32 rows: whole lines, all wavefronts with a step, operands that a load
+// into LDS can take (16 bytes).
+static bool lines_fit(const void* X, const void* W, int M, int K) {
+    return M <= 32 && K % SK_KSTEP == 0 && K >= 16 * SK_KSTEP && (int64_t)32 * K * 2 <= 0x7fffffff && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+}
+template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, bool SPLIT = false>
+static int launch_lines(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
+                        hipStream_t stream) {
+    if constexpr (MT == 1 && !SPLIT) {
+        if (M <= 8)
+            return (int)(tile_rows <= 8 ? launch_lines_depth<1, NT, GATED, RESID, SCALED, TC, 1, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
+                                        : launch_lines_depth<1, NT, GATED, RESID, SCALED, TC, 2, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
+    }
+    return (int)(tile_rows <= 8 ? launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, 1, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
+                                : launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, 2, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
+}
+
 // parts of lle_gemm_skinny_resid_bf16's sums of squares for a weight of N rows (its tiles at up to 16 rows of X): the second size of
 // its ss_part
 extern "C" int lle_gemm_skinny_resid_parts(int N) {
@@ -898,6 +1100,10 @@ static int launch_skinny(const T* X, const T* W, TC* C, int M, int N, int K, hip
     const int per_block = (GATED || NT == 1) ? tile_rows : 16 * NT;
     const int blocks = (rows + per_block - 1) / per_block;
     const int mt = (M + 15) / 16;
+    if constexpr (std::is_same<T, bf16_t>::value && (GATED || NT == 1))
+        if (lines_fit(X, W, M, K))
+            return mt == 1 ? launch_lines<1, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream)
+                           : launch_lines<2, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream);
     switch (mt) {
         case 1: gemm_skinny_kernel<T, 1, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
         case 2: gemm_skinny_kernel<T, 2, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
@@ -974,12 +1180,16 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
     fold.part_rows = skinny_tile_rows(N);
     fold.parts = (N + fold.part_rows - 1) / fold.part_rows;
     const int tr = M <= 16 || fold.part_rows > 8 ? fold.part_rows : 2 * fold.part_rows, blocks = (N + tr - 1) / tr;
+    const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
+    if (lines_fit(X, W, M, K))
+        return M <= 16 ? launch_lines<1, 1, false, true, false>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream)
+                       : launch_lines<1, 1, false, true, false, bf16_t, true>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream);
     if (M <= 16)
         gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
-            (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
+            x, w, (bf16_t*)nullptr, M, N, K, tr, fold);
     else
         gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4, true><<<dim3(blocks, 2), 16 * LLE_WAVE, 0, stream>>>(
-            (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, tr, fold);
+            x, w, (bf16_t*)nullptr, M, N, K, tr, fold);
     LLE_RETURN_LAUNCH_STATUS();
 }
 
@@ -991,11 +1201,14 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
 #define SCALED_TILES_AT_32_ROWS 4
 #endif
 template <typename TC>
-static void launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M, int N, int K, const NormFold& fold,
+static int launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M, int N, int K, const NormFold& fold,
                                  hipStream_t stream) {
-    if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream)) return;
+    if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream)) return (int)hipGetLastError();
     const int threads = 16 * LLE_WAVE;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
+    if (lines_fit(x, w, M, K) && (M <= 16 || N < 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()))
+        return M <= 16 ? launch_lines<1, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream)
+                       : launch_lines<2, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
     if (M <= 16) {
         gemm_skinny_kernel<bf16_t, 1, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
     } else if (N >= 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()) {
@@ -1008,6 +1221,7 @@ static void launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M,
     } else {
         gemm_skinny_kernel<bf16_t, 2, 1, false, false, true, TC, 16, 4><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
     }
+    return (int)hipGetLastError();
 }
 
 extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C, const void* ss_part, int parts,
@@ -1026,13 +1240,15 @@ extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C
     const int threads = 16 * LLE_WAVE;
     if (!gated) {
         if (out_dtype == LLE_F32)
-            launch_skinny_scaled<float>(x, w, (float*)C, M, N, K, fold, stream);
-        else
-            launch_skinny_scaled<bf16_t>(x, w, c, M, N, K, fold, stream);
+            return launch_skinny_scaled<float>(x, w, (float*)C, M, N, K, fold, stream);
+        return launch_skinny_scaled<bf16_t>(x, w, c, M, N, K, fold, stream);
     } else if (launch_skinny_stream<bf16_t, true, true, bf16_t>(x, w, c, M, N, K, fold, stream)) {
     } else {
         const int rows = N / 2;
         const int tr = skinny_tile_rows(rows), blocks = (rows + tr - 1) / tr;
+        if (lines_fit(X, W, M, K))
+            return M <= 16 ? launch_lines<1, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream)
+                           : launch_lines<2, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
         if (M <= 16)
             gemm_skinny_kernel<bf16_t, 1, 2, true, false, true, bf16_t, 16, 2><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold);
         else

@@ -1,0 +1,131 @@
+"""The weight-streaming product by way of LDS (bfloat16, up to 32 rows of X, K a multiple of 64 from 1024 on) against the same
+product with operands in registers, which operands that do not begin at 16 bytes still take: the same products and sums in the
+same order, so the same bits."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+_PLAIN = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 + [ctypes.c_void_p]
+_GATED = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+
+# few rows of X in one load of eight (1, 7, 8), two (9, 16), two tiles (17, 31, 32)
+ROWS = [1, 7, 8, 9, 16, 17, 31, 32]
+# tiles of four rows and of eight, of sixteen and a last one of a few; steps: one for every wavefront, two for some, more than LDS holds
+SIZES = [(1024, 1024), (1030, 1088), (2048, 1600), (1024, 3072), (4100, 2048), (1500, 4160), (528, 8192)]
+
+
+def ops():
+    from litellmengine_amd.csrc.ops import default_ops
+
+    return default_ops()
+
+
+def operands(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(1000 * seed + M + 7 * N + 13 * K)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    return x, (torch.randn(N, K, generator=g, device="cuda") * 0.05).bfloat16()
+
+
+def off_lines(x):
+    """The same rows, at an address that no load into LDS takes."""
+    t = torch.empty(x.numel() + 8, dtype=x.dtype, device=x.device)
+    view = t[4: 4 + x.numel()].view(x.shape)
+    assert view.data_ptr() % 16 == 8
+    return view.copy_(x)
+
+
+def close(got, want, K):
+    """Sums of exact products in 32 bits, a rounding to 16 at the end."""
+    scale = want.abs().max()
+    assert float((got.double() - want).abs().max() / scale) <= 2.0 ** -8 + K * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("N,K", SIZES)
+def test_plain(M, N, K):
+    o = ops()
+    x, w = operands(M, N, K)
+    run = lambda t, out: o._run("gemm", "lle_gemm_skinny_bf16", _PLAIN, t.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K,
+                                0 if out.dtype == torch.float32 else 1)
+    for dtype in (torch.bfloat16, torch.float32):
+        a, b = (torch.full((M, N), math.nan, dtype=dtype, device="cuda") for _ in range(2))
+        run(x, a)
+        run(off_lines(x), b)
+        close(a, x.double() @ w.double().T, K)
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("N,K", SIZES)
+def test_gated(M, N, K):
+    """Also a result whose rows of W are odd in number: 515 gate rows."""
+    o = ops()
+    x, w = operands(M, N, K, seed=1)
+    gate, up = (x.double() @ w.double().T).chunk(2, dim=1)
+    outs = []
+    for t in (x, off_lines(x)):
+        out = torch.full((M, N // 2), math.nan, dtype=torch.bfloat16, device="cuda")
+        o._run("gemm", "lle_gemm_skinny_gated_bf16", _GATED, t.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K)
+        outs.append(out)
+    close(outs[0], torch.nn.functional.silu(gate) * up, K)
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("N,K", SIZES)
+def test_around_a_folded_norm(M, N, K):
+    """A product into the residual stream (its rows, the norm's input and sums), and products that apply the row factors."""
+    from litellmengine_amd.parts import Prenormed
+    from litellmengine_amd.parts.base import NormFold
+
+    o = ops()
+    x, w = operands(M, N, K, seed=2)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    hidden = torch.randn(M, N, generator=g, device="cuda")
+    norm = torch.randn(N, generator=g, device="cuda").bfloat16()
+    got = []
+    for t in (x, off_lines(x)):
+        h = hidden.clone()
+        if o.can_fold_norm(M, N, x.dtype):
+            pre = o.linear(t, w, fold=NormFold(h, norm, 1e-6))
+            got.append((h, pre.xw, pre.sums[:M]))
+    if got:
+        want = hidden.double() + x.double() @ w.double().T
+        close(got[0][0], want, K)
+        close(got[0][1], got[0][0].double() * norm.double(), 1)
+        assert torch.allclose(got[0][2].double().sum(1), (got[0][0].double() ** 2).sum(1), rtol=1e-5)
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
+    if not o.can_fold_norm(M, K, x.dtype):
+        return
+    sums = torch.rand(16 if M <= 16 else 32, o.norm_sum_parts(K), generator=g, device="cuda")
+    factors = torch.rsqrt(sums[:M].double().sum(1) / K + 1e-6)[:, None]
+    product = x.double() @ w.double().T * factors
+    plain = [o.linear(Prenormed(t, sums, 1e-6), w) for t in (x, off_lines(x))]
+    close(plain[0], product, K)
+    assert torch.equal(*plain)
+    gated = [o.gate_up_silu(Prenormed(t, sums, 1e-6), w) for t in (x, off_lines(x))]
+    gate, up = product.chunk(2, dim=1)
+    close(gated[0], torch.nn.functional.silu(gate) * up, K)
+    assert torch.equal(*gated)
+
+
+def test_replayed_in_a_graph():
+    """One launch and nothing kept between them: every replay gives the eager bits."""
+    o = ops()
+    x, w = operands(5, 1024, 2048, seed=3)
+    want = o.linear(x, w)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = o.linear(x, w)
+    for _ in range(3):
+        out.fill_(math.nan)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        o.linear(x, w)
