@@ -88,6 +88,11 @@ __device__ __forceinline__ void load_into_lds(unsigned at, unsigned offset, cons
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
 }
 
+// the same with 4 bytes a lane
+__device__ __forceinline__ void load_word_into_lds(unsigned at, unsigned offset, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+}
+
 // The values of keys outside [lo, hi] become zeros; v[n][i], of eight 16-bit numbers, belongs to key `first` + i.  Their weight is
 // 0, which drops whatever lies there but an infinity or a NaN (pages are handed on as they are).
 template <typename Vec, int N>

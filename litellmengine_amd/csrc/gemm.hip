@@ -810,72 +810,6 @@ static int gemm_compute_units() {
     return cached[dev];
 }
 
-// The streaming kernel takes the product when K is a number of whole rounds of its 16 wavefronts
-// (1024 elements a round, 512 of float32) that its registers hold (up to 32 rows of X: fewer rounds
-// beyond 16), and W has more than one tile of rows for every CU.
-template <typename T, bool GATED, bool SCALED, typename TC>
-static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, int K,
-                                 const NormFold& fold, hipStream_t stream) {
-    constexpr int ROUND = SkShare<T>::ROUND;
-    if (M > 32 || K % ROUND != 0) return false;
-    const int rows = GATED ? N / 2 : N;
-    const int units = gemm_compute_units();
-    const int share = (rows + units - 1) / units;
-    if (share <= 16) return false;
-    // a float32 row of X in the registers costs a start that few rows of W and of X do not repay (6144 x 4096 at 1 row: 24.7
-    // against 21.2 us, at 8 rows 26.6 against 27.9; 24576 x 4096 at 8 rows 83.6 against 96.7)
-    if (std::is_same<T, float>::value && share <= 32 && M <= 4) return false;
-    const int blocks = (rows + share - 1) / share;
-    if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
-        if (K == ROUND) {
-            gemm_skinny_stream_kernel<T, GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-            return true;
-        }
-        if (K == 2 * ROUND) {
-            gemm_skinny_stream_kernel<T, GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-            return true;
-        }
-        if constexpr (!GATED) {
-            if (K == 3 * ROUND) {
-                gemm_skinny_stream_kernel<T, GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-                return true;
-            }
-            if (K == 4 * ROUND) {
-                gemm_skinny_stream_kernel<T, GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-                return true;
-            }
-        }
-        return false;
-    }
-#define LLE_STREAM_CASE(XSV)                                                                                          \
-    case XSV:                                                                                                         \
-        gemm_skinny_stream_kernel<T, GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
-                                                                                               fold);                \
-        return true;
-    switch (K / ROUND) {
-        LLE_STREAM_CASE(1)
-        LLE_STREAM_CASE(2)
-        LLE_STREAM_CASE(3)
-        LLE_STREAM_CASE(4)
-        LLE_STREAM_CASE(5)
-        case 6:
-        case 8:
-            if constexpr (!GATED) {  // the gated form's two tiles leave no registers for this much of X
-                if (K / ROUND == 6) {
-                    gemm_skinny_stream_kernel<T, GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
-                                                                                                          share, fold);
-                } else {
-                    gemm_skinny_stream_kernel<T, GATED, SCALED, 8, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
-                                                                                                          share, fold);
-                }
-                return true;
-            }
-            return false;
-    }
-#undef LLE_STREAM_CASE
-    return false;
-}
-
 // Rows of W per tile of the one-tile-per-workgroup kernel: as many as give every CU the same share.
 // More 16-row tiles than CUs: as many rows as make the last round full (with 320 tiles of 16 rows on
 // 256 CUs a quarter of the CUs reads twice what the others read and the launch lasts as long as two
@@ -1084,6 +1018,311 @@ static int launch_lines(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, i
                                 : launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, 2, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
 }
 
+// ---------------------------------------------------------------------------------
+// The product as a STREAM by way of LDS, for K = 64 * 16 * XS (XS steps a wavefront, all of X that it needs held in registers)
+// and up to 16 rows of X, or 32 (MT = 2); plain or gated, with or without the row factors of a folded norm.
+// The chip reads fastest when every CU has the same share of W.  There is one workgroup per CU, and it takes `share` rows of W
+// (share = rows / CUs, rounded up) in tiles of 16, the last of which may be lower: tile t of all workgroups together is one
+// block of consecutive rows (the memory channels see what they see of a plain sweep over W), of which workgroup b takes the
+// b-th piece.  The lanes of a tile that is not full read its last row again, which costs no traffic.
+// A wavefront's loads are pieces of sixteen rows of 128 bytes, two loads of whole lines into LDS of its own (gemm_lines_kernel says
+// why), DEPTH pieces on their way: first its part of X, which goes to registers, then its parts of the tiles one after the other, also
+// across the end of a tile, where the partial tiles are added up in LDS between barriers that wait for no load.
+// In a HIP graph, weights from memory, with operand-shaped loads to registers -> so, at 1 / 8 / 16 / 32 rows of X (us): 6144 x 4096
+// 12.5 / 12.7 / 14.8 -> 11.3 / 11.3 / 11.9 (norm folded); 24576 x 4096 gated 35.1 / 36.5 / 38.2 -> 35.7 / 35.7 / 36.0, plain at 32 rows
+// 41.6 -> 37.8; 51200 x 5120 gated 101 / 104 / 109 -> 91 / 92 / 95 (5.7 TB/s); 8768 x 2048 8.9 / 9.2 / 10.3 / 12.6 -> 9.0 / 9.0 / 9.5 /
+// 10.6; 12288 x 2048 gated 11.9 / 12.5 / 13.6 / 16.6 -> 11.8 / 11.9 / 12.0 / 13.9; 151936 x 1024 59.7 / 64.4 / 63.1 / 69.0 -> 54.7 / 57.8 /
+// 60.9 / 65.2.  What is left is the launch, 2 us, and memory.
+// ---------------------------------------------------------------------------------
+template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT, int DEPTH>
+__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_stream_kernel(const T* __restrict__ X, const T* __restrict__ W, TC* __restrict__ C, int M,
+                                                                          int N, int share, NormFold fold) {
+    using Vec = typename SkOp<T>::vec;
+    constexpr int WAVES = 16, NT = GATED ? 2 : 1, E = SkOp<T>::E, COLUMNS = 8 * E, K = XS * WAVES * COLUMNS, PIECE = 2048;
+    constexpr int ACC = NT * MT * 16 * 17 * 4, OWN = DEPTH * PIECE + ACC;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
+    __shared__ float s_inv[16 * MT];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    const int c = lane / 16, r16 = lane % 16;
+    const int rows = GATED ? N / 2 : N;
+    const int tiles = (share + 15) / 16;
+    // rows [tile_begin(t), tile_end(t)) of this workgroup's tile t; none where W ends before them
+    auto tile_begin = [&](int t) { return (int)gridDim.x * 16 * t + (int)blockIdx.x * min(16, share - 16 * t); };
+    auto tile_end = [&](int t) { return min(rows, tile_begin(t) + min(16, share - 16 * t)); };
+    // wavefront's LDS: the pieces [DEPTH][16 rows][128 bytes], and its sums (all wavefronts' sums one behind the other)
+    unsigned char* pieces = lines_lds + wave * (DEPTH * PIECE);
+    const unsigned pieces_at = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lines_lds + wave * (DEPTH * PIECE);
+    float* sums = (float*)(lines_lds + WAVES * DEPTH * PIECE);  // [wavefronts][NT][MT][16 n][17]
+    float* mine = sums + wave * (ACC / 4);
+    // a load: eight rows of 128 bytes; lane -> row lane / 8, physical piece lane % 8, the logical piece that belongs there
+    const unsigned in_row = (unsigned)(lane % 8) * 16, at_wave = (unsigned)wave * 128;
+    auto offset = [&](int row, int r) { return (unsigned)row * (unsigned)(K * sizeof(T)) + (in_row ^ (LINES_SWIZZLE(r) * 16)); };
+    const int lr0 = lane / 8, lr1 = 8 + lane / 8;
+    int fill = 0;  // the buffer that is asked for next
+    auto ask = [&](unsigned o0, unsigned o1, const void* base) {
+        load_into_lds(pieces_at + fill * PIECE, o0, base);
+        load_into_lds(pieces_at + fill * PIECE + 1024, o1, base);
+        fill = fill == DEPTH - 1 ? 0 : fill + 1;
+    };
+    // the cursor over W's pieces: tile, step, and gate or up rows
+    int load_tile = 0, load_step = 0, load_up = 0;
+    unsigned wo0, wo1;
+    const unsigned char* wb;
+    auto aim = [&]() {
+        const int first = tile_begin(load_tile), last = max(0, tile_end(load_tile) - 1 - first);  // (a tile without rows reads rows that are there)
+        wo0 = offset(min(lr0, last), lr0), wo1 = offset(min(lr1, last), lr1);
+        wb = (const unsigned char*)(W + (int64_t)min(first, rows - 1) * K) + at_wave;
+    };
+    auto ask_w = [&]() {
+        ask(wo0, wo1, wb + load_step * (WAVES * 128) + (GATED && load_up ? (int64_t)rows * K * sizeof(T) : 0));
+        if (GATED && !load_up) {
+            load_up = 1;
+            return;
+        }
+        load_up = 0;
+        if (++load_step == XS) {
+            load_step = 0;
+            if (++load_tile < tiles) aim();
+        }
+    };
+    // SCALED: the parts of the norm's sums of rows wave and 16 + wave, four bytes a lane, where the wavefront's sums will be
+    if constexpr (SCALED) {
+        const unsigned at = (unsigned)(size_t)(__attribute__((address_space(3))) void*)mine;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                load_word_into_lds(at + (mt * 4 + i) * 256, (unsigned)min(lane + i * LLE_WAVE, fold.parts - 1) * 4,
+                                   fold.ss_in + (int64_t)min(16 * mt + wave, M - 1) * fold.parts);
+    }
+    constexpr int XP = XS * MT;  // pieces of X
+    auto ask_x = [&](int q) {
+        const int mt = q / XS, step = q % XS;
+        ask(offset(min(16 * mt + lr0, M - 1), lr0), offset(min(16 * mt + lr1, M - 1), lr1),
+            (const unsigned char*)X + at_wave + step * (WAVES * 128));
+    };
+    aim();
+    auto ask_next = [&](int q) {  // piece q, X's first
+        if (q < XP) ask_x(q);
+        else ask_w();
+    };
+#pragma unroll
+    for (int q = 0; q < DEPTH; ++q) ask_next(q);  // (W has DEPTH pieces or more)
+    // lane (c, r) reads pieces 2 c and 2 c + 1 of row r
+    const int at0 = r16 * 128 + ((2 * c) ^ LINES_SWIZZLE(r16)) * 16, at1 = r16 * 128 + ((2 * c + 1) ^ LINES_SWIZZLE(r16)) * 16;
+    int buf = 0;
+    auto take = [&](Vec& v0, Vec& v1) {
+        const unsigned char* at = pieces + buf * PIECE;
+        v0 = *(const Vec*)(at + at0);
+        v1 = *(const Vec*)(at + at1);
+        buf = buf == DEPTH - 1 ? 0 : buf + 1;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the buffer has been read
+    };
+    auto landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * 2) : "memory"); };
+    Vec x0[MT][XS], x1[MT][XS];
+#pragma unroll
+    for (int q = 0; q < XP; ++q) {
+        landed();
+        take(x0[q / XS][q % XS], x1[q / XS][q % XS]);
+        ask_next(q + DEPTH);
+    }
+    if constexpr (SCALED) {  // (older than the pieces: landed with the first)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            float v[4], part = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = mine[(mt * 4 + i) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part += lane + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
+            const float* in = fold.ss_in + (int64_t)min(16 * mt + wave, M - 1) * fold.parts;
+            for (int b = lane + 4 * LLE_WAVE; b < fold.parts; b += 4 * LLE_WAVE) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = in[min(b + i * LLE_WAVE, fold.parts - 1)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part += b + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
+            }
+            part = wave_sum(part);
+            if (lane == 0) s_inv[16 * mt + wave] = 1.0f / sqrtf(part / (float)K + fold.eps);
+        }
+    }
+    int left = tiles * XS * NT - DEPTH;  // pieces that have not been asked for
+    for (int tile = 0; tile < tiles; ++tile) {
+        gf32x4 acc[NT][MT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < XS; ++j)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                if (left >= 0)
+                    landed();
+                else
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                Vec w0, w1;
+                take(w0, w1);
+                if (left > 0) ask_w();
+                --left;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    acc[nt][mt] = SkOp<T>::mma(w0, x0[mt][j], acc[nt][mt]);
+                    acc[nt][mt] = SkOp<T>::mma(w1, x1[mt][j], acc[nt][mt]);
+                }
+            }
+        // the tile's sums: nobody adds up the last tile's any more (barriers that wait for no load)
+        if (tile > 0) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mine[((nt * MT + mt) * 16 + 4 * c + i) * 17 + r16] = acc[nt][mt][i];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (threadIdx.x < 256 * MT) {
+            const int m = threadIdx.x / 16, n = threadIdx.x % 16;
+            const int64_t col = (int64_t)tile_begin(tile) + n;
+            if (m < M && col < tile_end(tile)) {
+                float g = 0.f, u = 0.f;
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) {
+                    g += sums[w * (ACC / 4) + ((m / 16) * 16 + n) * 17 + m % 16];
+                    if (GATED) u += sums[w * (ACC / 4) + ((MT + m / 16) * 16 + n) * 17 + m % 16];
+                }
+                if (SCALED) {
+                    g *= s_inv[m];
+                    u *= s_inv[m];
+                }
+                C[(int64_t)m * rows + col] = from_f32<TC>(GATED ? gated_result(g, u, fold, col, rows) : g);
+            }
+        }
+    }
+}
+
+// TILES: as many as every workgroup has at least.
+template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT, int TILES>
+static int launch_lines_stream_depth(const T* X, const T* W, TC* C, int M, int N, int share, int blocks, const NormFold& fold, hipStream_t stream) {
+    constexpr int NT = GATED ? 2 : 1, ACC = NT * MT * 16 * 17 * 4, MOST = (LINES_LDS / 16 - ACC) / 2048;
+    constexpr int DEPTH = MOST < TILES * XS * NT ? MOST : TILES * XS * NT, LDS = 16 * (DEPTH * 2048 + ACC);
+    auto kernel = gemm_lines_stream_kernel<T, GATED, SCALED, XS, TC, MT, DEPTH>;
+    static std::atomic<uint64_t> granted{0};
+    const hipError_t e = lle_grant_lds((const void*)kernel, LDS, granted);
+    if (e != hipSuccess) return (int)e;
+    kernel<<<blocks, 16 * LLE_WAVE, LDS, stream>>>(X, W, C, M, N, share, fold);
+    return (int)hipGetLastError();
+}
+template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT>
+static int launch_lines_stream(const T* X, const T* W, TC* C, int M, int N, int share, int blocks, const NormFold& fold, hipStream_t stream) {
+    if (XS == 1 && !GATED && share > 48)  // (short rows, an output head: 151936 x 1024 at 8 rows 61.1 us with two pieces on their way, 57.8 with four)
+        return launch_lines_stream_depth<T, GATED, SCALED, XS, TC, MT, XS == 1 && !GATED ? 4 : 2>(X, W, C, M, N, share, blocks, fold, stream);
+    return launch_lines_stream_depth<T, GATED, SCALED, XS, TC, MT, 2>(X, W, C, M, N, share, blocks, fold, stream);  // (a share is more than a tile)
+}
+
+// The streaming kernel takes the product when K is a number of whole rounds of its 16 wavefronts
+// (1024 elements a round, 512 of float32) that its registers hold (up to 32 rows of X: fewer rounds
+// beyond 16), and W has more than one tile of rows for every CU.
+template <typename T, bool GATED, bool SCALED, typename TC>
+static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, int K, const NormFold& fold, hipStream_t stream, hipError_t& e) {
+    e = hipSuccess;
+    constexpr int ROUND = SkShare<T>::ROUND;
+    if (M > 32 || K % ROUND != 0) return false;
+    const int rows = GATED ? N / 2 : N;
+    const int units = gemm_compute_units();
+    const int share = (rows + units - 1) / units;
+    if (share <= 16) return false;
+    // a float32 row of X in the registers costs a start that few rows of W and of X do not repay (6144 x 4096 at 1 row: 24.7
+    // against 21.2 us, at 8 rows 26.6 against 27.9; 24576 x 4096 at 8 rows 83.6 against 96.7)
+    if (std::is_same<T, float>::value && share <= 32 && M <= 4) return false;
+    const int blocks = (rows + share - 1) / share;
+    if constexpr (std::is_same<T, bf16_t>::value) {
+        if (((uintptr_t)X | (uintptr_t)W) & 15) return false;  // (what no load into LDS takes is gemm_skinny_kernel's)
+#define LLE_STREAM_CASE(XSV, MTV)                                                                                                 \
+    case XSV:                                                                                                                     \
+        e = (hipError_t)launch_lines_stream<T, GATED, SCALED, XSV, TC, MTV>(X, W, C, M, N, share, blocks, fold, stream);          \
+        return true;
+        if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
+            switch (K / ROUND) {
+                LLE_STREAM_CASE(1, 2)
+                LLE_STREAM_CASE(2, 2)
+            }
+            if constexpr (!GATED) switch (K / ROUND) {
+                LLE_STREAM_CASE(3, 2)
+                LLE_STREAM_CASE(4, 2)
+            }
+            return false;
+        }
+        switch (K / ROUND) {
+            LLE_STREAM_CASE(1, 1)
+            LLE_STREAM_CASE(2, 1)
+            LLE_STREAM_CASE(3, 1)
+            LLE_STREAM_CASE(4, 1)
+            LLE_STREAM_CASE(5, 1)
+        }
+        if constexpr (!GATED) switch (K / ROUND) {
+            LLE_STREAM_CASE(6, 1)
+            LLE_STREAM_CASE(8, 1)
+        }
+        return false;
+#undef LLE_STREAM_CASE
+    } else {
+    if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
+        if (K == ROUND) {
+            gemm_skinny_stream_kernel<T, GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+            return true;
+        }
+        if (K == 2 * ROUND) {
+            gemm_skinny_stream_kernel<T, GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+            return true;
+        }
+        if constexpr (!GATED) {
+            if (K == 3 * ROUND) {
+                gemm_skinny_stream_kernel<T, GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+                return true;
+            }
+            if (K == 4 * ROUND) {
+                gemm_skinny_stream_kernel<T, GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
+                return true;
+            }
+        }
+        return false;
+    }
+#define LLE_STREAM_CASE(XSV)                                                                                          \
+    case XSV:                                                                                                         \
+        gemm_skinny_stream_kernel<T, GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
+                                                                                               fold);                \
+        return true;
+    switch (K / ROUND) {
+        LLE_STREAM_CASE(1)
+        LLE_STREAM_CASE(2)
+        LLE_STREAM_CASE(3)
+        LLE_STREAM_CASE(4)
+        LLE_STREAM_CASE(5)
+        case 6:
+        case 8:
+            if constexpr (!GATED) {  // the gated form's two tiles leave no registers for this much of X
+                if (K / ROUND == 6) {
+                    gemm_skinny_stream_kernel<T, GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
+                                                                                                          share, fold);
+                } else {
+                    gemm_skinny_stream_kernel<T, GATED, SCALED, 8, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
+                                                                                                          share, fold);
+                }
+                return true;
+            }
+            return false;
+    }
+#undef LLE_STREAM_CASE
+    return false;
+    }
+}
+
+
 // parts of lle_gemm_skinny_resid_bf16's sums of squares for a weight of N rows (its tiles at up to 16 rows of X): the second size of
 // its ss_part
 extern "C" int lle_gemm_skinny_resid_parts(int N) {
@@ -1121,14 +1360,15 @@ extern "C" int lle_gemm_skinny_bf16(const void* X, const void* W, void* C, int M
     if (M > 64 || K % 8 != 0 || K <= 0) return (int)hipErrorInvalidValue;
     const bf16_t* x = (const bf16_t*)X;
     const bf16_t* w = (const bf16_t*)W;
+    hipError_t e;
     // one tile of W rows per workgroup measured best up to 16 rows of X (two tiles share the X
     // operands but halve the number of workgroups; they only pay off from 16 rows on)
     if (out_dtype == LLE_F32) {
-        if (launch_skinny_stream<bf16_t, false, false, float>(x, w, (float*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+        if (launch_skinny_stream<bf16_t, false, false, float>(x, w, (float*)C, M, N, K, NormFold{}, stream, e)) return (int)e;
         return launch_skinny<bf16_t, float, 1, false>(x, w, (float*)C, M, N, K, stream);
     }
     if (out_dtype == LLE_BF16) {
-        if (launch_skinny_stream<bf16_t, false, false, bf16_t>(x, w, (bf16_t*)C, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+        if (launch_skinny_stream<bf16_t, false, false, bf16_t>(x, w, (bf16_t*)C, M, N, K, NormFold{}, stream, e)) return (int)e;
         return launch_skinny<bf16_t, bf16_t, 1, false>(x, w, (bf16_t*)C, M, N, K, stream);
     }
     return (int)hipErrorInvalidValue;
@@ -1140,8 +1380,9 @@ extern "C" int lle_gemm_skinny_gated_bf16(const void* X, const void* W, void* C,
                                           hipStream_t stream) {
     if (M <= 0 || N2 <= 0) return 0;
     if (M > 32 || K % 8 != 0 || K <= 0 || N2 % 2 != 0) return (int)hipErrorInvalidValue;
-    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, NormFold{}, stream))
-        LLE_RETURN_LAUNCH_STATUS();
+    hipError_t e;
+    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, NormFold{}, stream, e))
+        return (int)e;
     return launch_skinny<bf16_t, bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream);
 }
 
@@ -1154,8 +1395,9 @@ extern "C" int lle_gemm_skinny_clamped_bf16(const void* X, const void* W, const 
     NormFold fold = {};
     fold.act_bias = (const bf16_t*)bias;
     fold.act_limit = limit;
-    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, fold, stream))
-        LLE_RETURN_LAUNCH_STATUS();
+    hipError_t e;
+    if (launch_skinny_stream<bf16_t, true, false, bf16_t>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, fold, stream, e))
+        return (int)e;
     return launch_skinny<bf16_t, bf16_t, 2, true>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)C, M, N2, K, stream, fold);
 }
 
@@ -1203,7 +1445,8 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
 template <typename TC>
 static int launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M, int N, int K, const NormFold& fold,
                                  hipStream_t stream) {
-    if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream)) return (int)hipGetLastError();
+    hipError_t e;
+    if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream, e)) return (int)e;
     const int threads = 16 * LLE_WAVE;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     if (lines_fit(x, w, M, K) && (M <= 16 || N < 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()))
@@ -1238,11 +1481,13 @@ extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C
     const bf16_t* w = (const bf16_t*)W;
     bf16_t* c = (bf16_t*)C;
     const int threads = 16 * LLE_WAVE;
+    hipError_t e;
     if (!gated) {
         if (out_dtype == LLE_F32)
             return launch_skinny_scaled<float>(x, w, (float*)C, M, N, K, fold, stream);
         return launch_skinny_scaled<bf16_t>(x, w, c, M, N, K, fold, stream);
-    } else if (launch_skinny_stream<bf16_t, true, true, bf16_t>(x, w, c, M, N, K, fold, stream)) {
+    } else if (launch_skinny_stream<bf16_t, true, true, bf16_t>(x, w, c, M, N, K, fold, stream, e)) {
+        return (int)e;
     } else {
         const int rows = N / 2;
         const int tr = skinny_tile_rows(rows), blocks = (rows + tr - 1) / tr;
@@ -1343,7 +1588,8 @@ extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M,
     const float* x = (const float*)X;
     const float* w = (const float*)W;
     float* c = (float*)C;
-    if (launch_skinny_stream<float, false, false, float>(x, w, c, M, N, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+    hipError_t e;
+    if (launch_skinny_stream<float, false, false, float>(x, w, c, M, N, K, NormFold{}, stream, e)) return (int)e;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
     switch ((M + 15) / 16) {
         case 1: gemm_skinny_f32_kernel<1, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;
@@ -1359,6 +1605,7 @@ extern "C" int lle_gemm_skinny_gated_f32(const void* X, const void* W, void* C, 
     if (M <= 0 || N2 <= 0) return 0;
     if (M > 32 || K % 4 != 0 || K <= 0 || N2 % 2 != 0) return (int)hipErrorInvalidValue;
     const float *x = (const float*)X, *w = (const float*)W;
-    if (launch_skinny_stream<float, true, false, float>(x, w, (float*)C, M, N2, K, NormFold{}, stream)) LLE_RETURN_LAUNCH_STATUS();
+    hipError_t e;
+    if (launch_skinny_stream<float, true, false, float>(x, w, (float*)C, M, N2, K, NormFold{}, stream, e)) return (int)e;
     return launch_skinny<float, float, 2, true>(x, w, (float*)C, M, N2, K, stream);
 }

@@ -15,7 +15,10 @@ _GATED = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
 # few rows of X in one load of eight (1, 7, 8), two (9, 16), two tiles (17, 31, 32)
 ROWS = [1, 7, 8, 9, 16, 17, 31, 32]
 # tiles of four rows and of eight, of sixteen and a last one of a few; steps: one for every wavefront, two for some, more than LDS holds
-SIZES = [(1024, 1024), (1030, 1088), (2048, 1600), (1024, 3072), (4100, 2048), (1500, 4160), (528, 8192)]
+SIZES = [(1024, 1024), (1030, 1088), (2048, 1600), (1024, 3072), (1500, 4160), (528, 8192)]
+# more than a tile of sixteen rows for every CU (of 256), of the plain product or of the gated one too: as a stream; shares of 17, 33 and 51
+# rows, the last workgroup's of one row
+SIZES += [(4100, 2048), (4098, 3072), (4200, 6144), (4354, 8192), (8450, 1024), (12802, 1024), (8196, 4096), (8710, 5120)]
 
 
 def ops():
@@ -62,7 +65,7 @@ def test_plain(M, N, K):
 @pytest.mark.parametrize("M", ROWS)
 @pytest.mark.parametrize("N,K", SIZES)
 def test_gated(M, N, K):
-    """Also a result whose rows of W are odd in number: 515 gate rows."""
+    """Also gate rows that are odd in number (515)."""
     o = ops()
     x, w = operands(M, N, K, seed=1)
     gate, up = (x.double() @ w.double().T).chunk(2, dim=1)
