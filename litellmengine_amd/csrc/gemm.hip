@@ -116,9 +116,8 @@ template <> struct SkOp<float> {
 // How the wavefronts share the columns of a row, in rounds of 128 bytes a wavefront, each lane two pieces of 16 bytes a round:
 // bfloat16 wavefronts take 128 bytes in a row, a lane's pieces side by side; float32 ones 64 bytes of each half of the round,
 // as gemm_skinny_f32_kernel does: which of the float32 kernels takes a product follows the number of rows, and a row's sums must
-// not.  (The other way round that kernel is slower with few rows: 6144 x 4096 at 1 row 21 us, with 128 bytes in a row 26.
-// The streaming kernel, 128 bytes in a row against so: 24576 x 4096 at 1 / 16 rows 79 / 83 against 75 / 81 us, gated 6144 x 1024
-// at 32 rows 11.0 against 10.3, gated 12288 x 2048 at 8 rows 22.5 against 24.7, 151936 x 1024 at 32 rows 123 against 138.)
+// not.  (The other way round that kernel is slower with few rows: 6144 x 4096 at 1 row 21 us, with 128 bytes in a row 26.  The
+// products that go by way of LDS, by K, take 128 bytes in a row whatever the number of rows.)
 template <typename T, int WAVES = 16> struct SkShare {
     static constexpr bool HALVES = std::is_same<T, float>::value;
     static constexpr int E = SkOp<T>::E;
@@ -593,210 +592,6 @@ extern "C" int lle_gemm_mid_slices_bf16(const void* X, const void* W, void* out,
     LLE_RETURN_LAUNCH_STATUS();
 }
 
-// ---------------------------------------------------------------------------------
-// The product as a STREAM, for K = 64 * 16 * XS (XS steps per wavefront, all of X that a
-// wavefront needs held in registers) and up to 16 rows of X; plain or gated, with or
-// without the row factors of a folded norm.
-// How fast a CU reads is bounded by the loads it can have on their way, so the chip is
-// fastest when every CU has the same share of W.  There is one workgroup per CU, and it
-// takes `share` rows of W (share = rows / CUs, rounded up) in tiles of 16, the last of
-// which may be lower: tile t of all workgroups together is one block of consecutive rows
-// (the memory channels see what they see of a plain sweep over W), of which workgroup b
-// takes the b-th piece.  The lanes of a tile that is not full read its last row again,
-// which costs no traffic.  A wavefront keeps two sets of W operands (two steps each where
-// XS is even and small, one step otherwise): while one is multiplied the loads of the next are on
-// their way, also across the end of a tile, where the partial tiles are added up in LDS
-// and written out.  X is read once per workgroup instead of once per tile, and the sums of
-// the folded norm are added up once.
-// ---------------------------------------------------------------------------------
-// MT = 2: up to 32 rows of X (two tiles of matrix-core columns), where all of X that a wavefront
-// needs still fits its registers (XS <= 2: narrow models, the only ones whose norms are folded at
-// more than 16 rows);
-// the head of the 0.6B sizes (151936 x 1024) at 32 rows: 73.6 us, against 112.1 for the
-// one-tile-per-workgroup kernel with four tiles a workgroup and 66.8 at 16 rows.
-template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT = 1>
-__global__ __launch_bounds__(16 * LLE_WAVE, 4) void gemm_skinny_stream_kernel(const T* __restrict__ X,
-                                                                              const T* __restrict__ W,
-                                                                              TC* __restrict__ C, int M, int N, int K,
-                                                                              int share, NormFold fold) {
-    using Vec = typename SkOp<T>::vec;
-    constexpr int WAVES = 16;
-    using Share = SkShare<T, WAVES>;
-    constexpr int NT = GATED ? 2 : 1;
-    constexpr int SS = (XS % 2 == 0 && XS <= 6) ? 2 : 1;  // steps of a set (one where X takes most of the registers)
-    // sets of W operands: one is multiplied, the others are on their way (single steps of float32: four)
-    constexpr int SETS = std::is_same<T, float>::value && !GATED && SS == 1 && XS % 4 == 0 ? 4 : 2;
-    constexpr int SPT = XS / SS;             // sets of a tile
-    static_assert(MT == 1 || (MT == 2 && (XS <= 2 || (!GATED && XS <= 4))), "two tiles of X rows only while X fits the registers");
-    __shared__ float s_acc[2][WAVES][NT][MT][16][17];  // tiles take the two halves in turn: one barrier a tile
-    __shared__ float s_inv[16 * MT];
-    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
-    const int c = lane / 16, r16 = lane % 16;
-    const int rows = GATED ? N / 2 : N;
-    const int tiles = (share + 15) / 16;
-    // rows [tile_begin(t), tile_end(t)) of this workgroup's tile t; none where W ends before them
-    auto tile_begin = [&](int t) { return (int)gridDim.x * 16 * t + (int)blockIdx.x * min(16, share - 16 * t); };
-    auto tile_end = [&](int t) { return min(rows, tile_begin(t) + min(16, share - 16 * t)); };
-
-    // a set: SS steps of the tile (and of the up tile that goes with a gate tile)
-    struct Set {
-        Vec g0[SS], g1[SS], u0[SS], u1[SS];
-    };
-    // the load cursor: tile and step of the set that is asked for next
-    int load_tile = 0, load_step = 0;
-    const T* wp = nullptr;
-    auto aim = [&]() {
-        const int t = min(load_tile, tiles - 1);
-        const int row = max(0, min(tile_begin(t) + r16, tile_end(t) - 1));  // a tile without rows reads rows that are there
-        wp = W + (int64_t)row * K + Share::LANE * c + wave * Share::WAVE;
-    };
-    auto load = [&](Set& set) {
-#pragma unroll
-        for (int i = 0; i < SS; ++i) {
-            const T* g = wp + (load_step + i) * Share::ROUND;
-            set.g0[i] = *(const Vec*)g;
-            set.g1[i] = *(const Vec*)(g + Share::SECOND);
-            if (GATED) {
-                const T* u = g + (int64_t)rows * K;
-                set.u0[i] = *(const Vec*)u;
-                set.u1[i] = *(const Vec*)(u + Share::SECOND);
-            }
-        }
-        load_step += SS;
-        if (load_step == XS) {
-            load_step = 0;
-            ++load_tile;
-            aim();
-        }
-    };
-    Set sets[SETS];
-    aim();
-#pragma unroll
-    for (int i = 0; i < SETS - 1; ++i) load(sets[i]);
-    // rows of X beyond M are never written back, so their lanes may read any valid row
-    Vec x0[MT][XS], x1[MT][XS];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const T* xp = X + (int64_t)min(16 * mt + r16, M - 1) * K + Share::LANE * c + wave * Share::WAVE;
-#pragma unroll
-        for (int j = 0; j < XS; ++j) {
-            x0[mt][j] = *(const Vec*)(xp + j * Share::ROUND);
-            x1[mt][j] = *(const Vec*)(xp + j * Share::ROUND + Share::SECOND);
-        }
-    }
-    if (SCALED) {
-        // the row factors of the folded norm: wavefront w adds up the parts of row w (and of row
-        // 16 + w), four loads at a time
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const float* in = fold.ss_in + (int64_t)(16 * mt + wave) * fold.parts;
-            float part = 0.f;
-            for (int p0 = lane; p0 < fold.parts; p0 += 4 * LLE_WAVE) {
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = in[min(p0 + i * LLE_WAVE, fold.parts - 1)];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) part += p0 + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
-            }
-            part = wave_sum(part);
-            if (lane == 0) s_inv[16 * mt + wave] = 1.0f / sqrtf(part / (float)K + fold.eps);
-        }
-    }
-    gf32x4 acc_g[MT], acc_u[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc_g[mt] = acc_u[mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const Set& set, int j) {
-#pragma unroll
-        for (int i = 0; i < SS; ++i)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                acc_g[mt] = SkOp<T>::mma(set.g0[i], x0[mt][j + i], acc_g[mt]);
-                acc_g[mt] = SkOp<T>::mma(set.g1[i], x1[mt][j + i], acc_g[mt]);
-                if (GATED) {
-                    acc_u[mt] = SkOp<T>::mma(set.u0[i], x0[mt][j + i], acc_u[mt]);
-                    acc_u[mt] = SkOp<T>::mma(set.u1[i], x1[mt][j + i], acc_u[mt]);
-                }
-            }
-    };
-    int half = 0;
-    auto finish_tile = [&](int tile) {
-        // lane holds C^T[n = 4c + i][m = 16 mt + r16]
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                s_acc[half][wave][0][mt][4 * c + i][r16] = acc_g[mt][i];
-                if (GATED) s_acc[half][wave][NT - 1][mt][4 * c + i][r16] = acc_u[mt][i];
-            }
-            acc_g[mt] = acc_u[mt] = gf32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        __syncthreads();
-        if (threadIdx.x < 256 * MT) {
-            const int m = threadIdx.x / 16, n = threadIdx.x % 16;
-            const int64_t col = (int64_t)tile_begin(tile) + n;
-            if (m < M && col < tile_end(tile)) {
-                float g = 0.f, u = 0.f;
-#pragma unroll
-                for (int w = 0; w < WAVES; ++w) {
-                    g += s_acc[half][w][0][m / 16][n][m % 16];
-                    if (GATED) u += s_acc[half][w][NT - 1][m / 16][n][m % 16];
-                }
-                if (SCALED) {
-                    g *= s_inv[m];
-                    u *= s_inv[m];
-                }
-                C[(int64_t)m * rows + col] = from_f32<TC>(GATED ? gated_result(g, u, fold, col, rows) : g);
-            }
-        }
-        // The other half is written next; this one again only after the next tile's barrier,
-        // which the threads that are still adding here have then passed.
-        half ^= 1;
-    };
-    // One tile: its sets in turn, the one after each asked for before it is multiplied (also the
-    // first of the next tile; the share's last tile asks for nothing beyond itself).  `first` is
-    // the buffer that holds the tile's first set: the sets alternate between the two buffers
-    // across tiles, so with an odd number of sets a tile every other tile starts in buffer 1.
-    auto run_tile = [&](int tile, auto first_c, bool last) {
-        constexpr int first = decltype(first_c)::value;
-#pragma unroll
-        for (int s = 0; s < SPT; ++s) {
-            if (!(last && s == SPT - 1)) load(sets[(first + s + 1) % 2]);
-            multiply(sets[(first + s) % 2], s * SS);
-        }
-        finish_tile(tile);
-    };
-    using Buf0 = std::integral_constant<int, 0>;
-    using Buf1 = std::integral_constant<int, 1>;
-    int tile = 0;
-    if constexpr (SETS > 2) {
-        auto run = [&](bool last) {
-#pragma unroll
-            for (int s = 0; s < SPT; ++s) {
-                if (!(last && s + SETS - 1 >= SPT)) load(sets[(s + SETS - 1) % SETS]);
-                multiply(sets[s % SETS], s * SS);
-            }
-            finish_tile(tile);
-        };
-        static_assert(SPT % SETS == 0, "a tile's sets go around the buffers in whole rounds");
-        for (; tile + 1 < tiles; ++tile) run(false);
-        run(true);
-    } else if constexpr (SPT % 2 == 0) {
-        for (; tile + 1 < tiles; ++tile) run_tile(tile, Buf0{}, false);
-        run_tile(tile, Buf0{}, true);
-    } else {
-        for (; tile + 2 < tiles; tile += 2) {
-            run_tile(tile, Buf0{}, false);
-            run_tile(tile + 1, Buf1{}, false);
-        }
-        if (tile + 1 < tiles) {
-            run_tile(tile, Buf0{}, false);
-            run_tile(tile + 1, Buf1{}, true);
-        } else {
-            run_tile(tile, Buf0{}, true);
-        }
-    }
-}
-
 // CUs of the current device (asked once per device)
 static int gemm_compute_units() {
     static int cached[64] = {0};
@@ -831,8 +626,8 @@ static int skinny_tile_rows(int rows) {
 
 
 // ---------------------------------------------------------------------------------
-// The same by way of LDS: bfloat16, up to 32 rows of X, K a multiple of 64 from 1024 on.  The same products and sums in the same order,
-// bit for bit; only the operands' way is another one.
+// The same by way of LDS: up to 32 rows of X, K a multiple of 64 from 1024 on; float32, plain up to 64 rows, of 32 from 512 on.  In bfloat16 the
+// same products and sums in the same order, bit for bit; only the operands' way is another one.
 // What bounds gemm_skinny_kernel is a CU's vector cache: a load to registers costs it four cycles for every line of 128 bytes that it
 // touches, and loads as the matrix instruction wants its operands touch sixteen lines for half of each (16 bytes a cycle, 38 B/ns
 // a CU, for W and for X; whole lines 75), while loads straight into LDS, here eight whole lines at a time, bring 85 to 118
@@ -849,7 +644,7 @@ static int skinny_tile_rows(int rows) {
 // where piece p (16 bytes) of row r lies in its 128 bytes of LDS: p ^ this.  A 16-byte read serves sixteen lanes a cycle, rows with
 // r / 4 in {0, 3} at piece 2 c + e and the others at that of the next c (or the other way round): they meet every bank once.
 #define LINES_SWIZZLE(r) ((((r) >> 1) & 7) ^ (((((r) >> 3) ^ ((r) >> 2)) & 1) << 1))
-#define LINES_LDS (160 * 1024 - 256)  // (of a CU, less what the row factors take)
+#define LINES_LDS(scaled) (160 * 1024 - ((scaled) ? 256 : 0))  // (of a CU, less what the row factors take)
 
 // bytes of LDS of a wavefront
 static constexpr int lines_bytes(int loads, int depth, int tiles) {
@@ -857,11 +652,13 @@ static constexpr int lines_bytes(int loads, int depth, int tiles) {
     return operands > sums ? operands : (sums + 1023) / 1024 * 1024;
 }
 
-template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, int DEPTH, bool SPLIT>
-__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, int DEPTH, bool SPLIT>
+__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                                    TC* __restrict__ C, int M, int N, int K, int tile_rows, NormFold fold) {
+    using Vec = typename SkOp<T>::vec;
+    constexpr int COLUMNS = 8 * SkOp<T>::E;  // of a wavefront's part of a step: 128 bytes
     constexpr int WAVES = 16, LOADS = NT * WH + MT * XH, STEP = LOADS * 1024, OWN = lines_bytes(LOADS, DEPTH, NT * MT);
-    static_assert(NT == (GATED ? 2 : 1) && WAVES * OWN <= LINES_LDS, "a tile of W, and of the up rows; the LDS of a CU");
+    static_assert(NT == (GATED ? 2 : 1) && WAVES * OWN <= LINES_LDS(SCALED), "a tile of W, and of the up rows; the LDS of a CU");
     extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
     __shared__ float s_inv[16 * MT];
     if constexpr (RESID || SCALED)  // (all arguments in one go, as gemm_skinny_kernel)
@@ -885,20 +682,20 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t*
 #pragma unroll
     for (int h = 0; h < WH; ++h) {
         const int r = 8 * h + lane / 8;
-        wo[h] = (unsigned)min(min(r, tile_rows - 1), rows - 1 - (int)n0) * (unsigned)(K * 2) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
+        wo[h] = (unsigned)min(min(r, tile_rows - 1), rows - 1 - (int)n0) * (unsigned)(K * sizeof(T)) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int h = 0; h < XH; ++h) {
             const int r = 8 * h + lane / 8;
-            xo[mt][h] = (unsigned)min(16 * mt + r, M - 1) * (unsigned)(K * 2) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
+            xo[mt][h] = (unsigned)min(16 * mt + r, M - 1) * (unsigned)(K * sizeof(T)) + ((lane % 8) ^ LINES_SWIZZLE(r)) * 16;
         }
     unsigned char* own = lines_lds + wave * OWN;
     const unsigned own_at = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lines_lds + wave * OWN;
-    const bf16_t *wb = W + n0 * K + wave * SK_KSTEP, *xb = X + wave * SK_KSTEP;
+    const T *wb = W + n0 * K + wave * COLUMNS, *xb = X + wave * COLUMNS;
     auto issue = [&](int step, int buf) {
-        const int64_t k = (int64_t)step * (SK_KSTEP * WAVES);
+        const int64_t k = (int64_t)step * (COLUMNS * WAVES);
         const unsigned at = own_at + buf * STEP;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
@@ -913,7 +710,7 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t*
     if (SCALED) parts.load(fold, wave, lane, M);
     ResidRows<MT> resid;
     if (RESID) resid.load(fold, n0, tile_rows, M, N);
-    const int steps = (K / SK_KSTEP - wave + WAVES - 1) / WAVES;  // of this wavefront: DEPTH or more
+    const int steps = (K / COLUMNS - wave + WAVES - 1) / WAVES;  // of this wavefront: DEPTH or more
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) issue(d, d);
     // lane (c, r) reads pieces 2 c and 2 c + 1 of row r (of eight rows: each twice)
@@ -935,20 +732,20 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t*
     auto multiply = [&](auto behind) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(behind)::value * LOADS) : "memory");
         const unsigned char* at = own + buf * STEP;
-        gbf16x8 w[NT][2], x[MT][2];
+        Vec w[NT][2], x[MT][2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) w[nt][e] = *(const gbf16x8*)(at + nt * WH * 1024 + w_at[e]);
+            for (int nt = 0; nt < NT; ++nt) w[nt][e] = *(const Vec*)(at + nt * WH * 1024 + w_at[e]);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) x[mt][e] = *(const gbf16x8*)(at + (NT * WH + mt * XH) * 1024 + x_at[e]);
+            for (int mt = 0; mt < MT; ++mt) x[mt][e] = *(const Vec*)(at + (NT * WH + mt * XH) * 1024 + x_at[e]);
         }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                for (int e = 0; e < 2; ++e) acc[nt][mt] = SkOp<bf16_t>::mma(w[nt][e], x[mt][e], acc[nt][mt]);
+                for (int e = 0; e < 2; ++e) acc[nt][mt] = SkOp<T>::mma(w[nt][e], x[mt][e], acc[nt][mt]);
     };
     auto next = [&]() { buf = buf == DEPTH - 1 ? 0 : buf + 1; };
     for (int step = 0; step + DEPTH < steps; ++step, next()) {
@@ -979,20 +776,20 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const bf16_t*
         for (int w = 0; w < WAVES; ++w) sum += *(const float*)(at + w * OWN);
         return sum;
     };
-    finish_skinny<WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, bf16_t>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
+    finish_skinny<WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
 }
 
 // DEPTH: the most steps that LDS holds, up to 5, and up to what the wavefront with the fewest has.
-template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, bool SPLIT, int DEPTH>
-static hipError_t launch_lines_depth(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
+template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, int WH, int XH, bool SPLIT, int DEPTH>
+static hipError_t launch_lines_depth(const T* X, const T* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
                                      hipStream_t stream) {
     constexpr int LDS = 16 * lines_bytes(NT * WH + MT * XH, DEPTH, NT * MT);
-    if constexpr (LDS > LINES_LDS) {
-        return launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
-    } else if (DEPTH > 1 && K / (16 * SK_KSTEP) < DEPTH) {
-        return launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH == 1 ? 1 : DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
+    if constexpr (LDS > LINES_LDS(SCALED)) {
+        return launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
+    } else if (DEPTH > 1 && K / (16 * 8 * SkOp<T>::E) < DEPTH) {
+        return launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH == 1 ? 1 : DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
     } else {
-        auto kernel = gemm_lines_kernel<MT, NT, GATED, RESID, SCALED, TC, WH, XH, DEPTH, SPLIT>;
+        auto kernel = gemm_lines_kernel<T, MT, NT, GATED, RESID, SCALED, TC, WH, XH, DEPTH, SPLIT>;
         static std::atomic<uint64_t> granted{0};
         const hipError_t e = lle_grant_lds((const void*)kernel, LDS, granted);
         if (e != hipSuccess) return e;
@@ -1001,21 +798,22 @@ static hipError_t launch_lines_depth(const bf16_t* X, const bf16_t* W, TC* C, in
     }
 }
 
-// Whether gemm_lines_kernel takes a product of up to 32 rows: whole lines, all wavefronts with a step, operands that a load
-// into LDS can take (16 bytes).
-static bool lines_fit(const void* X, const void* W, int M, int K) {
-    return M <= 32 && K % SK_KSTEP == 0 && K >= 16 * SK_KSTEP && (int64_t)32 * K * 2 <= 0x7fffffff && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+// Whether gemm_lines_kernel takes a product of up to 32 rows (a plain one of float32 64): whole lines, all wavefronts with a step, operands
+// that a load into LDS can take (16 bytes).
+template <typename T>
+static bool lines_fit(const T* X, const T* W, int K) {
+    return K % (8 * SkOp<T>::E) == 0 && K >= 16 * 8 * SkOp<T>::E && (int64_t)64 * K * sizeof(T) <= 0x7fffffff && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
 }
-template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, bool SPLIT = false>
-static int launch_lines(const bf16_t* X, const bf16_t* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
+template <int MT, int NT, bool GATED, bool RESID, bool SCALED, typename TC, bool SPLIT = false, typename T>
+static int launch_lines(const T* X, const T* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
                         hipStream_t stream) {
     if constexpr (MT == 1 && !SPLIT) {
         if (M <= 8)
-            return (int)(tile_rows <= 8 ? launch_lines_depth<1, NT, GATED, RESID, SCALED, TC, 1, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
-                                        : launch_lines_depth<1, NT, GATED, RESID, SCALED, TC, 2, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
+            return (int)(tile_rows <= 8 ? launch_lines_depth<T, 1, NT, GATED, RESID, SCALED, TC, 1, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
+                                        : launch_lines_depth<T, 1, NT, GATED, RESID, SCALED, TC, 2, 1, false, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
     }
-    return (int)(tile_rows <= 8 ? launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, 1, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
-                                : launch_lines_depth<MT, NT, GATED, RESID, SCALED, TC, 2, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
+    return (int)(tile_rows <= 8 ? launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, 1, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream)
+                                : launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, 2, 2, SPLIT, 5>(X, W, C, M, N, K, tile_rows, fold, blocks, stream));
 }
 
 // ---------------------------------------------------------------------------------
@@ -1208,7 +1006,7 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_stream_kernel(const 
 // TILES: as many as every workgroup has at least.
 template <typename T, bool GATED, bool SCALED, int XS, typename TC, int MT, int TILES>
 static int launch_lines_stream_depth(const T* X, const T* W, TC* C, int M, int N, int share, int blocks, const NormFold& fold, hipStream_t stream) {
-    constexpr int NT = GATED ? 2 : 1, ACC = NT * MT * 16 * 17 * 4, MOST = (LINES_LDS / 16 - ACC) / 2048;
+    constexpr int NT = GATED ? 2 : 1, ACC = NT * MT * 16 * 17 * 4, MOST = (LINES_LDS(true) / 16 - ACC) / 2048;
     constexpr int DEPTH = MOST < TILES * XS * NT ? MOST : TILES * XS * NT, LDS = 16 * (DEPTH * 2048 + ACC);
     auto kernel = gemm_lines_stream_kernel<T, GATED, SCALED, XS, TC, MT, DEPTH>;
     static std::atomic<uint64_t> granted{0};
@@ -1236,90 +1034,36 @@ static bool launch_skinny_stream(const T* X, const T* W, TC* C, int M, int N, in
     const int units = gemm_compute_units();
     const int share = (rows + units - 1) / units;
     if (share <= 16) return false;
-    // a float32 row of X in the registers costs a start that few rows of W and of X do not repay (6144 x 4096 at 1 row: 24.7
-    // against 21.2 us, at 8 rows 26.6 against 27.9; 24576 x 4096 at 8 rows 83.6 against 96.7)
-    if (std::is_same<T, float>::value && share <= 32 && M <= 4) return false;
     const int blocks = (rows + share - 1) / share;
-    if constexpr (std::is_same<T, bf16_t>::value) {
-        if (((uintptr_t)X | (uintptr_t)W) & 15) return false;  // (what no load into LDS takes is gemm_skinny_kernel's)
+    if (((uintptr_t)X | (uintptr_t)W) & 15) return false;  // (what no load into LDS takes is gemm_skinny_kernel's)
 #define LLE_STREAM_CASE(XSV, MTV)                                                                                                 \
     case XSV:                                                                                                                     \
         e = (hipError_t)launch_lines_stream<T, GATED, SCALED, XSV, TC, MTV>(X, W, C, M, N, share, blocks, fold, stream);          \
         return true;
-        if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
-            switch (K / ROUND) {
-                LLE_STREAM_CASE(1, 2)
-                LLE_STREAM_CASE(2, 2)
-            }
-            if constexpr (!GATED) switch (K / ROUND) {
-                LLE_STREAM_CASE(3, 2)
-                LLE_STREAM_CASE(4, 2)
-            }
-            return false;
-        }
+    if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
         switch (K / ROUND) {
-            LLE_STREAM_CASE(1, 1)
-            LLE_STREAM_CASE(2, 1)
-            LLE_STREAM_CASE(3, 1)
-            LLE_STREAM_CASE(4, 1)
-            LLE_STREAM_CASE(5, 1)
+            LLE_STREAM_CASE(1, 2)
+            LLE_STREAM_CASE(2, 2)
         }
         if constexpr (!GATED) switch (K / ROUND) {
-            LLE_STREAM_CASE(6, 1)
-            LLE_STREAM_CASE(8, 1)
-        }
-        return false;
-#undef LLE_STREAM_CASE
-    } else {
-    if (M > 16) {  // two tiles of X rows: while all of X that a wavefront needs fits its registers
-        if (K == ROUND) {
-            gemm_skinny_stream_kernel<T, GATED, SCALED, 1, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-            return true;
-        }
-        if (K == 2 * ROUND) {
-            gemm_skinny_stream_kernel<T, GATED, SCALED, 2, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-            return true;
-        }
-        if constexpr (!GATED) {
-            if (K == 3 * ROUND) {
-                gemm_skinny_stream_kernel<T, GATED, SCALED, 3, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-                return true;
-            }
-            if (K == 4 * ROUND) {
-                gemm_skinny_stream_kernel<T, GATED, SCALED, 4, TC, 2><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, fold);
-                return true;
-            }
+            LLE_STREAM_CASE(3, 2)
+            LLE_STREAM_CASE(4, 2)
         }
         return false;
     }
-#define LLE_STREAM_CASE(XSV)                                                                                          \
-    case XSV:                                                                                                         \
-        gemm_skinny_stream_kernel<T, GATED, SCALED, XSV, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, share, \
-                                                                                               fold);                \
-        return true;
     switch (K / ROUND) {
-        LLE_STREAM_CASE(1)
-        LLE_STREAM_CASE(2)
-        LLE_STREAM_CASE(3)
-        LLE_STREAM_CASE(4)
-        LLE_STREAM_CASE(5)
-        case 6:
-        case 8:
-            if constexpr (!GATED) {  // the gated form's two tiles leave no registers for this much of X
-                if (K / ROUND == 6) {
-                    gemm_skinny_stream_kernel<T, GATED, SCALED, 6, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
-                                                                                                          share, fold);
-                } else {
-                    gemm_skinny_stream_kernel<T, GATED, SCALED, 8, TC><<<blocks, 16 * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K,
-                                                                                                          share, fold);
-                }
-                return true;
-            }
-            return false;
+        LLE_STREAM_CASE(1, 1)
+        LLE_STREAM_CASE(2, 1)
+        LLE_STREAM_CASE(3, 1)
+        LLE_STREAM_CASE(4, 1)
+        LLE_STREAM_CASE(5, 1)
     }
-#undef LLE_STREAM_CASE
+    if constexpr (!GATED) switch (K / ROUND) {
+        LLE_STREAM_CASE(6, 1)
+        LLE_STREAM_CASE(8, 1)
+    }
     return false;
-    }
+#undef LLE_STREAM_CASE
 }
 
 
@@ -1335,14 +1079,12 @@ template <typename T, typename TC, int NT, bool GATED>
 static int launch_skinny(const T* X, const T* W, TC* C, int M, int N, int K, hipStream_t stream, const NormFold& none = {}) {
     constexpr int WAVES = 16, UNROLL = 4 / NT;
     const int rows = GATED ? N / 2 : N;
-    const int tile_rows = (GATED || NT == 1) ? skinny_tile_rows(rows) : 16;
-    const int per_block = (GATED || NT == 1) ? tile_rows : 16 * NT;
-    const int blocks = (rows + per_block - 1) / per_block;
+    const int tile_rows = skinny_tile_rows(rows), blocks = (rows + tile_rows - 1) / tile_rows;
     const int mt = (M + 15) / 16;
-    if constexpr (std::is_same<T, bf16_t>::value && (GATED || NT == 1))
-        if (lines_fit(X, W, M, K))
-            return mt == 1 ? launch_lines<1, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream)
-                           : launch_lines<2, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream);
+    if (lines_fit(X, W, K)) {
+        if (mt == 1) return launch_lines<1, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream);
+        if (mt == 2) return launch_lines<2, NT, GATED, false, false>(X, W, C, M, N, K, tile_rows, none, blocks, stream);
+    }
     switch (mt) {
         case 1: gemm_skinny_kernel<T, 1, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
         case 2: gemm_skinny_kernel<T, 2, NT, GATED, false, false, TC, WAVES, UNROLL><<<blocks, WAVES * LLE_WAVE, 0, stream>>>(X, W, C, M, N, K, tile_rows, none); break;
@@ -1423,7 +1165,7 @@ extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hi
     fold.parts = (N + fold.part_rows - 1) / fold.part_rows;
     const int tr = M <= 16 || fold.part_rows > 8 ? fold.part_rows : 2 * fold.part_rows, blocks = (N + tr - 1) / tr;
     const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
-    if (lines_fit(X, W, M, K))
+    if (lines_fit((const bf16_t*)X, (const bf16_t*)W, K))
         return M <= 16 ? launch_lines<1, 1, false, true, false>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream)
                        : launch_lines<1, 1, false, true, false, bf16_t, true>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream);
     if (M <= 16)
@@ -1449,7 +1191,7 @@ static int launch_skinny_scaled(const bf16_t* x, const bf16_t* w, TC* c, int M, 
     if (launch_skinny_stream<bf16_t, false, true, TC>(x, w, c, M, N, K, fold, stream, e)) return (int)e;
     const int threads = 16 * LLE_WAVE;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
-    if (lines_fit(x, w, M, K) && (M <= 16 || N < 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()))
+    if (lines_fit(x, w, K) && (M <= 16 || N < 16 * SCALED_TILES_AT_32_ROWS * gemm_compute_units()))
         return M <= 16 ? launch_lines<1, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream)
                        : launch_lines<2, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
     if (M <= 16) {
@@ -1491,7 +1233,7 @@ extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C
     } else {
         const int rows = N / 2;
         const int tr = skinny_tile_rows(rows), blocks = (rows + tr - 1) / tr;
-        if (lines_fit(X, W, M, K))
+        if (lines_fit((const bf16_t*)X, (const bf16_t*)W, K))
             return M <= 16 ? launch_lines<1, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream)
                            : launch_lines<2, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
         if (M <= 16)
@@ -1503,7 +1245,7 @@ extern "C" int lle_gemm_skinny_scaled_bf16(const void* X, const void* W, void* C
 }
 
 // ---------------------------------------------------------------------------------
-// The same for float32 operands: decoding in 32-bit where the streaming kernel does not take the product.  W is read once;
+// The same for float32 operands that do not go by way of LDS (few columns, no whole lines, odd addresses).  W is read once;
 // v_mfma_f32_16x16x4_f32 multiplies and adds in float32 (no reduced-precision mode).
 // Lane (c, r) loads 16 contiguous bytes W[n0 + r][k0 + 4c .. + 3]; its four values are the
 // k slot c of four instructions, and the X operand is laid out the same way.
@@ -1580,8 +1322,11 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE) void gemm_skinny_f32_kernel(con
 }
 
 // X [M, K] and W [N, K] float32, contiguous; C [M, N] float32; 1 <= M <= 64; K a multiple of 4.
-// The streaming kernel takes what it holds a row of X of (K 512 times 1 to 6 or 8; up to 2048 beyond 16 rows), as for
-// bfloat16: at 8 rows 24576 x 4096 96.7 -> 83.6 us, 151936 x 4096 555 -> 457, 151936 x 1024 at 32 rows 240 -> 124.
+// K a multiple of 32 from 512 on goes by way of LDS whatever the number of rows (one of them decides the order of a row's sums, so K has to),
+// as bfloat16 does; in a HIP graph, before -> so, at 1 / 8 / 17 / 32 / 64 rows (us): 4096 x 1024 5.6 / 6.7 / 8.0 / 9.2 / 13.6 -> 5.0 / 5.3 /
+// 6.3 / 7.2 / 9.6; 6144 x 4096 22.4 / 28.5 / 37.4 / 48.2 / 80.2 -> 21.9 / 21.9 / 26.5 / 31.4 / 46.5; 24576 x 4096 gated 80.2 / 83.2 / 107 / 121 /
+// 255 -> 75.2 / 75.1 / 82.7 / 84.6 / 148; 151936 x 4096 444 / 450 / 725 / 933 / 1540 -> 413 / 424 / 529 / 615 / 860.  The errors against 64 bits are
+// the same (1.6e-7 at K = 1024, 3.0e-7 at 4096).
 extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (M > 64 || K % 4 != 0 || K <= 0) return (int)hipErrorInvalidValue;
@@ -1591,6 +1336,12 @@ extern "C" int lle_gemm_skinny_f32(const void* X, const void* W, void* C, int M,
     hipError_t e;
     if (launch_skinny_stream<float, false, false, float>(x, w, c, M, N, K, NormFold{}, stream, e)) return (int)e;
     const int tr = skinny_tile_rows(N), blocks = (N + tr - 1) / tr;
+    if (lines_fit(x, w, K)) switch ((M + 15) / 16) {
+        case 1: return launch_lines<1, 1, false, false, false>(x, w, c, M, N, K, tr, NormFold{}, blocks, stream);
+        case 2: return launch_lines<2, 1, false, false, false>(x, w, c, M, N, K, tr, NormFold{}, blocks, stream);
+        case 3: return launch_lines<3, 1, false, false, false>(x, w, c, M, N, K, tr, NormFold{}, blocks, stream);
+        default: return launch_lines<4, 1, false, false, false>(x, w, c, M, N, K, tr, NormFold{}, blocks, stream);
+    }
     switch ((M + 15) / 16) {
         case 1: gemm_skinny_f32_kernel<1, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;
         case 2: gemm_skinny_f32_kernel<2, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, c, M, N, K, tr); break;

@@ -1,6 +1,6 @@
 """The weight-streaming product by way of LDS (bfloat16, up to 32 rows of X, K a multiple of 64 from 1024 on) against the same
 product with operands in registers, which operands that do not begin at 16 bytes still take: the same products and sums in the
-same order, so the same bits."""
+same order, so the same bits.  (test_gemm_f32_gpu.py has the float32 twins at these edges.)"""
 import ctypes
 import math
 
@@ -132,3 +132,22 @@ def test_replayed_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         o.linear(x, w)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(1024, 512), (1030, 544), (2000, 1600), (4100, 2048), (4354, 4096), (8450, 1024), (12802, 512)])
+def test_float32(M, N, K):
+    """Tiles and steps as above, three and four tiles of X's rows; sums of K float32 products: 2^-24 (K + 16) of their sizes at most.
+    The last row alone gives the bits that it has among the others."""
+    o = ops()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda")
+    out = torch.full((M, N), math.nan, device="cuda")
+    run = lambda t, y: o._run("gemm", "lle_gemm_skinny_f32", _GATED, t.data_ptr(), w.data_ptr(), y.data_ptr(), t.shape[0], N, K)
+    run(x, out)
+    size = x.double().abs() @ w.double().abs().T
+    assert bool(((out.double() - x.double() @ w.double().T).abs() <= 2.0 ** -24 * (K + 16) * size).all())
+    last = torch.full((1, N), math.nan, device="cuda")
+    run(x[-1:].contiguous(), last)
+    assert torch.equal(last, out[-1:])
