@@ -280,7 +280,7 @@ extern "C" int lle_gemm_nt_f32(const void* A, const void* B, void* C, int M, int
 // reads M / 16 times as many bytes of A as of B.  So a workgroup takes 64 rows of B and a slice of K: four wavefronts (one for
 // every 16 rows) read the same pieces of A, which the CU's vector cache hands out; four such groups take every fourth step of
 // 32 columns; their sums meet in LDS.  Two sets of operands: the next is on its way while one is multiplied (float32 matrix
-// instruction).  Against all of K in one workgroup: 1024 x 3072 at 32 rows 15.4 -> 7.6 us, at 1 row 7.6 -> 4.8;
+// instruction).  (Rows of whole lines go by way of LDS, below.)  Against all of K in one workgroup: 1024 x 3072 at 32 rows 15.4 -> 7.6 us, at 1 row 7.6 -> 4.8;
 // 4096 x 12288 at 8 rows 52.0 -> 43.0, at 32 rows 84.6 -> 68.5; 4096 x 4096 at 8 rows 18.7 -> 16.1.
 // ---------------------------------------------------------------------------------
 #define FS_ROWS 64
@@ -375,6 +375,207 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_slices_f32_kernel(const fl
     }
 }
 
+// The same by way of LDS where rows are whole lines of 128 bytes (K a multiple of 32): the same products and sums in the same order, bit
+// for bit.  Loads of operands as the matrix instruction wants them touch sixteen lines for half of each, four cycles of the CU's
+// vector cache for every one of them; here a load brings eight whole lines straight into LDS.
+// From 17 rows on where a slice is long the rows of X that four wavefronts share come once (gemm_slices_lines_f32_kernel: a stage is a
+// step for each of the FS_KW groups, a barrier a stage, as many stages as LDS holds).  Up to 16 rows, and up to 32 in short
+// slices, every wavefront brings what it multiplies itself and waits for nobody (gemm_slices_own_f32_kernel): X comes four times, but
+// in stages 4096 x 12288 takes 44.9 us at 8 rows against 40.3, 1024 x 2048 in ten slices 6.4 at 32 rows against 5.5 (in long
+// slices at 32 rows 48.2 against 53.6).
+// In a HIP graph at 1 / 8 / 16 / 32 / 64 rows, operand-shaped -> so (us): 1024 x 2048 4.4 / 5.1 / 5.7 / 7.6 / 10.9 -> 3.9 / 4.1 / 4.4 / 5.5 / 8.1;
+// 1024 x 3072 4.8 / 5.4 / 6.3 / 8.1 / 10.9 -> 4.6 / 4.7 / 4.9 / 5.8 / 8.6; 4096 x 4096 15.7 / 16.9 / 19.1 / 25.3 / 41.2 -> 15.1 / 15.3 / 15.9 / 18.5 /
+// 24.4; 4096 x 12288 40.5 / 47.0 / 52.8 / 71.0 / 117 -> 39.3 / 40.3 (5.0 TB/s) / 43.0 / 47.4 / 68.3; 5120 x 25600 97 / 114 / 136 / 185 / 313 -> 93 / 94 /
+// 104 / 108 / 157.
+// LDS of a stage: [step][8 groups of 8 rows of B, then 2 MT groups of X][1 KB]; where piece p of row r lies: p ^ swizzle
+#define FS_SWIZZLE(r) ((((r) >> 1) & 7) ^ (((((r) >> 3) ^ ((r) >> 2)) & 1) << 1))
+template <int MT, int STAGES>
+__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_slices_lines_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                                              float* __restrict__ out, int M, int N, int K, int slice_steps) {
+    constexpr int GROUPS = 8 + 2 * MT, STEP = GROUPS * 1024, STAGE = FS_KW * STEP;
+    constexpr int XL = (FS_KW * 2 * MT + 15) / 16, LOADS = 2 + XL;  // a wavefront's loads of a stage: two of B, and of X
+    static_assert(STAGES * STAGE <= 160 * 1024 && 16 * MT * 16 * 17 * 4 <= STAGES * STAGE, "the LDS of a CU, and the sums in its place");
+    extern __shared__ __attribute__((aligned(16))) unsigned char fs_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    const int c = lane / 16, r16 = lane % 16;
+    const int tile = wave % 4, kw = wave / 4;
+    const int n0 = blockIdx.x * FS_ROWS;
+    const int first = blockIdx.y * slice_steps, last = min(K / FS_STEP, first + slice_steps);
+    // the wavefront's loads: the 16 rows of B that it multiplies, at its own step; group g of X's of the stage, at step g / (2 MT)
+    unsigned offset[LOADS], at[LOADS];
+    int step_of[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int g = i < 2 ? 0 : (wave + 16 * (i - 2)) % (FS_KW * 2 * MT), u = i < 2 ? kw : g / (2 * MT);
+        const int r = i < 2 ? 16 * tile + 8 * i + lane / 8 : 8 * (g % (2 * MT)) + lane / 8;
+        const int row = i < 2 ? min(r, N - 1 - n0) : min(r, M - 1);
+        offset[i] = (unsigned)row * (unsigned)(K * 4) + ((lane % 8) ^ FS_SWIZZLE(r % 16)) * 16;
+        at[i] = u * STEP + (i < 2 ? 2 * tile + i : 8 + g % (2 * MT)) * 1024;
+        step_of[i] = u;
+    }
+    const float* b = B + (int64_t)n0 * K;
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) void*)fs_lds;
+    auto issue = [&](int step, int buf) {  // (past the slice: its last step again)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            load_into_lds(lds_base + buf * STAGE + at[i], offset[i], (i < 2 ? b : A) + min(step + step_of[i], last - 1) * FS_STEP);
+    };
+    const int at0 = r16 * 128 + ((2 * c) ^ FS_SWIZZLE(r16)) * 16, at1 = r16 * 128 + ((2 * c + 1) ^ FS_SWIZZLE(r16)) * 16;
+    sf32x4 acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = sf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+        if (first + s * FS_KW < last) issue(first + s * FS_KW, s);
+    int buf = 0;
+    for (int step = first; step < last; step += FS_KW) {
+        // this stage has landed for every wavefront, and nobody reads the buffer any more that the next load takes
+        if (step + (STAGES - 2) * FS_KW < last)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (step + (STAGES - 1) * FS_KW < last) issue(step + (STAGES - 1) * FS_KW, buf == 0 ? STAGES - 1 : buf - 1);
+        if (step + kw < last) {
+            const unsigned char* from = fs_lds + buf * STAGE + kw * STEP;
+            const sf32x4 b0 = *(const sf32x4*)(from + 2 * tile * 1024 + at0), b1 = *(const sf32x4*)(from + 2 * tile * 1024 + at1);
+            sf32x4 a0[MT], a1[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a0[mt] = *(const sf32x4*)(from + (8 + 2 * mt) * 1024 + at0), a1[mt] = *(const sf32x4*)(from + (8 + 2 * mt) * 1024 + at1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(h ? b1[e] : b0[e], h ? a1[mt][e] : a0[mt][e], acc[mt], 0, 0, 0);
+        }
+        buf = buf == STAGES - 1 ? 0 : buf + 1;
+    }
+    __syncthreads();  // the sums take the operands' place
+    // lane holds C^T[n = 4 c + i][m = r16]
+    float* red = (float*)fs_lds;  // [16 wavefronts][MT][16 n][17]
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[((wave * MT + mt) * 16 + 4 * c + i) * 17 + r16] = acc[mt][i];
+    __syncthreads();
+    float* dst = out + (int64_t)blockIdx.y * M * N;
+    for (int idx = threadIdx.x; idx < MT * 16 * FS_ROWS; idx += 16 * LLE_WAVE) {
+        const int n = idx % FS_ROWS, m = idx / FS_ROWS;  // consecutive threads: consecutive columns
+        const int col = n0 + n;
+        if (m >= M || col >= N) continue;
+        float sum = 0.f;
+#pragma unroll
+        for (int g = 0; g < FS_KW; ++g) sum += red[(((4 * g + n / 16) * MT + m / 16) * 16 + n % 16) * 17 + m % 16];
+        dst[(int64_t)m * N + col] = sum;
+    }
+}
+
+// Up to 16 rows: a wavefront brings its rows of B and X (8 XH of them) itself, into LDS of its own, DEPTH steps ahead, and waits for
+// its own loads alone, without a barrier.
+template <int XH>
+__global__ __launch_bounds__(16 * LLE_WAVE) void gemm_slices_own_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                                            float* __restrict__ out, int M, int N, int K, int slice_steps) {
+    constexpr int MT = (XH + 1) / 2, LOADS = 2 + XH, STEP = LOADS * 1024, DEPTH = 10 / LOADS, OWN = DEPTH * STEP;
+    extern __shared__ __attribute__((aligned(16))) unsigned char fs_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE;
+    const int c = lane / 16, r16 = lane % 16;
+    const int tile = wave % 4, kw = wave / 4;
+    const int n0 = blockIdx.x * FS_ROWS;
+    const int first = blockIdx.y * slice_steps + kw, last = min(K / FS_STEP, (int)(blockIdx.y + 1) * slice_steps);
+    const int steps = (last - first + FS_KW - 1) / FS_KW;  // of this wavefront (none: zero or less)
+    unsigned offset[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int r = (i < 2 ? 16 * tile + 8 * i : 8 * (i - 2)) + lane / 8;
+        offset[i] = (unsigned)min(r, i < 2 ? N - 1 - n0 : M - 1) * (unsigned)(K * 4) + ((lane % 8) ^ FS_SWIZZLE(r % 16)) * 16;
+    }
+    const float *b = B + (int64_t)n0 * K + first * FS_STEP, *a = A + first * FS_STEP;
+    const unsigned own_at = (unsigned)(size_t)(__attribute__((address_space(3))) void*)fs_lds + wave * OWN;
+    const unsigned char* own = fs_lds + wave * OWN;
+    auto issue = [&](int step, int buf) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) load_into_lds(own_at + buf * STEP + i * 1024, offset[i], (i < 2 ? b : a) + step * (FS_KW * FS_STEP));
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+        if (d < steps) issue(d, d);
+    const int xr = XH == 1 ? r16 % 8 : r16;  // (of eight rows: each twice)
+    int b_at[2], a_at[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        b_at[e] = r16 * 128 + ((2 * c + e) ^ FS_SWIZZLE(r16)) * 16;
+        a_at[e] = 2048 + xr * 128 + ((2 * c + e) ^ FS_SWIZZLE(xr)) * 16;
+    }
+    sf32x4 acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = sf32x4{0.f, 0.f, 0.f, 0.f};
+    int buf = 0;
+    for (int step = 0; step < steps; ++step) {
+        if (step + DEPTH <= steps)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * LOADS) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        sf32x4 bv[2], av[MT][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            bv[e] = *(const sf32x4*)(own + buf * STEP + b_at[e]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) av[mt][e] = *(const sf32x4*)(own + buf * STEP + mt * 2048 + a_at[e]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the buffer has been read
+        if (step + DEPTH < steps) issue(step + DEPTH, buf);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[h][e], av[mt][h][e], acc[mt], 0, 0, 0);
+        buf = buf == DEPTH - 1 ? 0 : buf + 1;
+    }
+    // lane holds C^T[n = 4 c + i][m = r16]; a wavefront's sums take the place of its operands
+    float* mine = (float*)(fs_lds + wave * OWN);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mine[(mt * 16 + 4 * c + i) * 17 + r16] = acc[mt][i];
+    __syncthreads();
+    float* dst = out + (int64_t)blockIdx.y * M * N;
+    const int n = threadIdx.x % FS_ROWS, col = n0 + n;  // consecutive threads: consecutive columns
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m16 = threadIdx.x / FS_ROWS, m = 16 * mt + m16;
+        if (m >= M || col >= N) return;
+        float sum = 0.f;
+#pragma unroll
+        for (int g = 0; g < FS_KW; ++g) sum += *(const float*)(fs_lds + (4 * g + n / 16) * OWN + ((mt * 16 + n % 16) * 17 + m16) * 4);
+        dst[(int64_t)m * N + col] = sum;
+    }
+}
+
+template <int XH>
+static int launch_slices_own(const float* A, const float* B, float* out, int M, int N, int K, int each, dim3 grid, hipStream_t stream) {
+    constexpr int LDS = 16 * (10 / (2 + XH)) * (2 + XH) * 1024;
+    static std::atomic<uint64_t> granted{0};
+    const hipError_t e = lle_grant_lds((const void*)gemm_slices_own_f32_kernel<XH>, LDS, granted);
+    if (e != hipSuccess) return (int)e;
+    gemm_slices_own_f32_kernel<XH><<<grid, 16 * LLE_WAVE, LDS, stream>>>(A, B, out, M, N, K, each);
+    LLE_RETURN_LAUNCH_STATUS();
+}
+
+template <int MT>
+static int launch_slices_lines(const float* A, const float* B, float* out, int M, int N, int K, int each, dim3 grid, hipStream_t stream) {
+    constexpr int STAGE = FS_KW * (8 + 2 * MT) * 1024, STAGES = 160 * 1024 / STAGE;
+    auto kernel = gemm_slices_lines_f32_kernel<MT, STAGES>;
+    static std::atomic<uint64_t> granted{0};
+    const hipError_t e = lle_grant_lds((const void*)kernel, STAGES * STAGE, granted);
+    if (e != hipSuccess) return (int)e;
+    kernel<<<grid, 16 * LLE_WAVE, STAGES * STAGE, stream>>>(A, B, out, M, N, K, each);
+    LLE_RETURN_LAUNCH_STATUS();
+}
+
 // In how many slices of K the product of up to 64 rows is taken: as many workgroups of 64 rows of B as there are CUs, six steps
 // for the four wavefronts of a row group at least; 1 where the rows of B alone occupy the CUs, and where K is so short that the
 // sums' way to the norm and back costs what the slices gain.  Product and norm, whole / in slices of four steps / so, at 1, 8
@@ -399,6 +600,13 @@ extern "C" int lle_gemm_slices_f32(const void* A, const void* B, void* out, int 
     const dim3 grid((N + FS_ROWS - 1) / FS_ROWS, slices);
     const float *a = (const float*)A, *b = (const float*)B;
     float* o = (float*)out;
+    // (by K and the operands' addresses, not by M; a tile's rows in 32-bit offsets)
+    if (K % FS_STEP == 0 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && (int64_t)FS_ROWS * K * 4 <= 0x7fffffff) switch ((M + 15) / 16) {
+        case 1: return M <= 8 ? launch_slices_own<1>(a, b, o, M, N, K, each, grid, stream) : launch_slices_own<2>(a, b, o, M, N, K, each, grid, stream);
+        case 2: return each <= 16 ? launch_slices_own<4>(a, b, o, M, N, K, each, grid, stream) : launch_slices_lines<2>(a, b, o, M, N, K, each, grid, stream);
+        case 3: return launch_slices_lines<3>(a, b, o, M, N, K, each, grid, stream);
+        default: return launch_slices_lines<4>(a, b, o, M, N, K, each, grid, stream);
+    }
     switch ((M + 15) / 16) {
         case 1: gemm_slices_f32_kernel<1><<<grid, 16 * LLE_WAVE, 0, stream>>>(a, b, o, M, N, K, each); break;
         case 2: gemm_slices_f32_kernel<2><<<grid, 16 * LLE_WAVE, 0, stream>>>(a, b, o, M, N, K, each); break;

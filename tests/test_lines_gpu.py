@@ -36,7 +36,7 @@ def operands(M, N, K, seed=0):
 def off_lines(x):
     """The same rows, at an address that no load into LDS takes."""
     t = torch.empty(x.numel() + 8, dtype=x.dtype, device=x.device)
-    view = t[4: 4 + x.numel()].view(x.shape)
+    view = t[8 // x.element_size():][: x.numel()].view(x.shape)
     assert view.data_ptr() % 16 == 8
     return view.copy_(x)
 
@@ -151,3 +151,17 @@ def test_float32(M, N, K):
     last = torch.full((1, N), math.nan, device="cuda")
     run(x[-1:].contiguous(), last)
     assert torch.equal(last, out[-1:])
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 48, 64])
+@pytest.mark.parametrize("N,K,slices", [(64, 32, 1), (100, 96, 3), (1024, 2048, 10), (72, 2080, 5), (130, 3072, 4), (64, 4160, 2)])
+def test_float32_slices(M, N, K, slices):
+    """One step for one of four wavefronts and none for the others, slices of 16 steps and of 17, the last one shorter, columns that fill no
+    group of 64: the bits of operand-shaped loads, which an address that is no multiple of 16 still takes."""
+    o = ops()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    got = o.linear_f32_slices(x, w, slices)
+    size = x.double().abs() @ w.double().abs().T
+    assert bool(((got.double().sum(0) - x.double() @ w.double().T).abs() <= 2.0 ** -24 * (K + 16) * size).all())
+    assert torch.equal(got, o.linear_f32_slices(off_lines(x), w, slices))
