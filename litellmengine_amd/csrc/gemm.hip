@@ -150,8 +150,8 @@ struct NormFold {
     float* hidden;          // RESID: residual stream [M, N], read and written
     const void* weight;     // RESID: norm weight [N]
     int weight_dtype;
-    bf16_t* xw;             // RESID: out, [M, N]
-    float* ss_out;          // RESID: out, [16][parts]; SPLIT: [32][parts]
+    void* xw;               // RESID: out, [M, N], of X's type
+    float* ss_out;          // RESID: out, [16][parts]; SPLIT: [32][parts] or more
     const float* ss_in;     // SCALED: the same
     int parts;              // SCALED, SPLIT
     int part_rows;          // SPLIT: columns of a part, all of the tile's or half of them
@@ -208,7 +208,8 @@ struct NormParts {
             for (int i = 0; i < EARLY; ++i)  // past the parts: the last one again, dropped below; past the rows likewise
                 early[j][i] = fold.ss_in[min(wave + WAVES * j, M - 1) * fold.parts + min(lane + LLE_WAVE * i, fold.parts - 1)];
     }
-    __device__ __forceinline__ void finish(const NormFold& fold, int wave, int lane, int M, int K, float* s_inv) const {
+    template <typename Inv>
+    __device__ __forceinline__ void finish(const NormFold& fold, int wave, int lane, int M, int K, const Inv& inv) const {
 #pragma unroll
         for (int j = 0; j < ROWS; ++j) {
             const int m = wave + WAVES * j;
@@ -226,14 +227,14 @@ struct NormParts {
                 for (int i = 0; i < 4; ++i) part += b + i * LLE_WAVE < fold.parts ? v[i] : 0.f;
             }
             part = wave_sum(part);
-            if (lane == 0) s_inv[m] = 1.0f / sqrtf(part / (float)K + fold.eps);
+            if (lane == 0) inv(m) = 1.0f / sqrtf(part / (float)K + fold.eps);
         }
     }
 };
-// The epilogue: total(nt, mt, n, m) adds up the wavefronts' partial sums in their order.
-template <int WAVES, int MT, int NT, bool GATED, bool RESID, bool SCALED, bool SPLIT, typename T, typename TC, typename Total>
+// The epilogue: total(nt, mt, n, m) adds up the wavefronts' partial sums in their order; inv(m) is row m's factor.
+template <int WAVES, int MT, int NT, bool GATED, bool RESID, bool SCALED, bool SPLIT, typename T, typename TC, typename Total, typename Inv>
 __device__ __forceinline__ void finish_skinny(const Total& total, TC* C, int M, int N, int64_t n0, int tile_rows, const NormFold& fold,
-                                              const ResidRows<MT>& resid, const float* s_inv) {
+                                              const ResidRows<MT>& resid, const Inv& inv) {
     if (GATED) {
         for (int idx = threadIdx.x; idx < MT * 256; idx += WAVES * LLE_WAVE) {
             const int mt = idx / 256, m = (idx / 16) % 16, n = idx % 16;
@@ -241,8 +242,8 @@ __device__ __forceinline__ void finish_skinny(const Total& total, TC* C, int M, 
             if (row >= M || col >= N / 2 || n >= tile_rows) continue;
             float g = total(0, mt, n, m), u = total(NT - 1, mt, n, m);
             if (SCALED) {
-                g *= s_inv[16 * mt + m];
-                u *= s_inv[16 * mt + m];
+                g *= inv(16 * mt + m);
+                u *= inv(16 * mt + m);
             }
             C[row * (N / 2) + col] = from_f32<TC>(gated_result(g, u, fold, col, N / 2));
         }
@@ -280,7 +281,7 @@ __device__ __forceinline__ void finish_skinny(const Total& total, TC* C, int M, 
         const int64_t row = 16 * mt + m, col = n0 + 16 * nt + n;
         if (row >= M || col >= N || (NT == 1 && n >= tile_rows)) continue;
         float sum = total(nt, mt, n, m);
-        if (SCALED) sum *= s_inv[16 * mt + m];
+        if (SCALED) sum *= inv(16 * mt + m);
         C[row * N + col] = from_f32<TC>(sum);
     }
 }
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
     using Vec = typename SkOp<T>::vec;
     using Share = SkShare<T, SK_WAVES>;
     constexpr int E = SkOp<T>::E, SECOND = Share::SECOND;
-    static_assert(!(RESID || SCALED) || MT <= 2, "the norm is folded for up to 32 rows");
+    static_assert(!(RESID || SCALED) || MT <= (std::is_same<T, float>::value ? 4 : 2), "the norm is folded for up to 32 rows, float32 64");
     // `tile_rows` (at most 16) rows of W per tile: fewer than 16 where that makes the number of tiles a
     // multiple of the number of CUs (see skinny_tile_rows); the lanes past them read the tile's last
     // row again, which costs no traffic, and write nothing.  Forms with several tiles of W per
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
         X += (int64_t)before * K;
         M -= before;
         fold.hidden += (int64_t)before * N;
-        fold.xw += (int64_t)before * N;
+        fold.xw = (T*)fold.xw + (int64_t)before * N;
         fold.ss_out += (int64_t)before * fold.parts;
     }
     NormParts<MT, SK_WAVES> parts;
@@ -409,7 +410,8 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
             }
         }
     }
-    if (SCALED) parts.finish(fold, wave, lane, M, K, s_inv);
+    auto inv = [&](int m) -> float& { return s_inv[m]; };
+    if (SCALED) parts.finish(fold, wave, lane, M, K, inv);
     // lane holds C^T[n = 4c + i][m = r16]
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -424,7 +426,7 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE, (MT == 1 && !GATED && !SCALED) 
         for (int w = 0; w < SK_WAVES; ++w) sum += s_acc[w][nt][mt][n][m];
         return sum;
     };
-    finish_skinny<SK_WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
+    finish_skinny<SK_WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, inv);
 }
 
 // ---------------------------------------------------------------------------------
@@ -658,9 +660,9 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const T* __re
     using Vec = typename SkOp<T>::vec;
     constexpr int COLUMNS = 8 * SkOp<T>::E;  // of a wavefront's part of a step: 128 bytes
     constexpr int WAVES = 16, LOADS = NT * WH + MT * XH, STEP = LOADS * 1024, OWN = lines_bytes(LOADS, DEPTH, NT * MT);
-    static_assert(NT == (GATED ? 2 : 1) && WAVES * OWN <= LINES_LDS(SCALED), "a tile of W, and of the up rows; the LDS of a CU");
+    static_assert(NT == (GATED ? 2 : 1) && WAVES * OWN <= LINES_LDS(SCALED && MT <= 2) && (MT <= 2 || OWN >= NT * MT * 16 * 17 * 4 + 16), "a tile of W, and of the up rows; the LDS of a CU");
     extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
-    __shared__ float s_inv[16 * MT];
+    __shared__ float s_inv[MT <= 2 ? 16 * MT : 1];
     if constexpr (RESID || SCALED)  // (all arguments in one go, as gemm_skinny_kernel)
         asm volatile("" ::"s"(X), "s"(W), "s"(C), "s"(M), "s"(N), "s"(K), "s"(tile_rows), "s"(fold.hidden), "s"(fold.weight),
                      "s"(fold.weight_dtype), "s"(fold.xw), "s"(fold.ss_out), "s"(fold.ss_in), "s"(fold.parts),
@@ -671,7 +673,7 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const T* __re
         X += (int64_t)before * K;
         M -= before;
         fold.hidden += (int64_t)before * N;
-        fold.xw += (int64_t)before * N;
+        fold.xw = (T*)fold.xw + (int64_t)before * N;
         fold.ss_out += (int64_t)before * fold.parts;
     }
     const int64_t n0 = (int64_t)blockIdx.x * tile_rows;
@@ -758,7 +760,12 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const T* __re
     if constexpr (DEPTH >= 3) multiply(std::integral_constant<int, 2>{}), next();
     if constexpr (DEPTH >= 2) multiply(std::integral_constant<int, 1>{}), next();
     multiply(std::integral_constant<int, 0>{});
-    if (SCALED) parts.finish(fold, wave, lane, M, K, s_inv);
+    // (three and four tiles of X's rows take all of LDS: a wavefront keeps its rows' factors behind what its sums will take)
+    auto inv = [&](int m) -> float& {
+        if constexpr (MT <= 2) return s_inv[m];
+        else return *(float*)(lines_lds + m % 16 * OWN + OWN - 16 + m / 16 * 4);
+    };
+    if (SCALED) parts.finish(fold, wave, lane, M, K, inv);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     // lane holds C^T[n = 4c + i][m = r16]
     float* mine = (float*)own;
@@ -776,7 +783,7 @@ __global__ __launch_bounds__(16 * LLE_WAVE) void gemm_lines_kernel(const T* __re
         for (int w = 0; w < WAVES; ++w) sum += *(const float*)(at + w * OWN);
         return sum;
     };
-    finish_skinny<WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, s_inv);
+    finish_skinny<WAVES, MT, NT, GATED, RESID, SCALED, SPLIT, T>(total, C, M, N, n0, tile_rows, fold, resid, inv);
 }
 
 // DEPTH: the most steps that LDS holds, up to 5, and up to what the wavefront with the fewest has.
@@ -784,7 +791,7 @@ template <typename T, int MT, int NT, bool GATED, bool RESID, bool SCALED, typen
 static hipError_t launch_lines_depth(const T* X, const T* W, TC* C, int M, int N, int K, int tile_rows, const NormFold& fold, int blocks,
                                      hipStream_t stream) {
     constexpr int LDS = 16 * lines_bytes(NT * WH + MT * XH, DEPTH, NT * MT);
-    if constexpr (LDS > LINES_LDS(SCALED)) {
+    if constexpr (LDS > LINES_LDS(SCALED && MT <= 2)) {
         return launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
     } else if (DEPTH > 1 && K / (16 * 8 * SkOp<T>::E) < DEPTH) {
         return launch_lines_depth<T, MT, NT, GATED, RESID, SCALED, TC, WH, XH, SPLIT, DEPTH == 1 ? 1 : DEPTH - 1>(X, W, C, M, N, K, tile_rows, fold, blocks, stream);
@@ -793,7 +800,7 @@ static hipError_t launch_lines_depth(const T* X, const T* W, TC* C, int M, int N
         static std::atomic<uint64_t> granted{0};
         const hipError_t e = lle_grant_lds((const void*)kernel, LDS, granted);
         if (e != hipSuccess) return e;
-        kernel<<<dim3(blocks, SPLIT ? 2 : 1), 16 * LLE_WAVE, LDS, stream>>>(X, W, C, M, N, K, tile_rows, fold);
+        kernel<<<dim3(blocks, SPLIT ? (M + 15) / 16 : 1), 16 * LLE_WAVE, LDS, stream>>>(X, W, C, M, N, K, tile_rows, fold);
         return hipGetLastError();
     }
 }
@@ -1147,34 +1154,46 @@ extern "C" int lle_gemm_skinny_clamped_bf16(const void* X, const void* W, const 
 // in place), xw = hidden * norm_weight goes to `xw` (bfloat16 [M, N]) and the sums of squares of
 // the new hidden over each part's columns to ss_part [16 or 32][lle_gemm_skinny_resid_parts(N)]
 // (32 rows when M > 16).  1 <= M <= 32.
+template <typename T>
+static int launch_resid(const T* x, const T* w, void* hidden, const void* norm_weight, int weight_dtype, void* xw, void* ss_part, int M, int N, int K,
+                        hipStream_t stream) {
+    NormFold fold = {};
+    fold.hidden = (float*)hidden;
+    fold.weight = norm_weight;
+    fold.weight_dtype = weight_dtype;
+    fold.xw = xw;
+    fold.ss_out = (float*)ss_part;
+    // From 17 rows of X on a workgroup takes sixteen of them and, of a narrow model, tiles of W twice as high (two parts of the sums):
+    // with all 32 rows a workgroup of the 0.6B sizes reads eight times as much X as W, every CU all of X (1024 x 3072: 24 + 196 KB,
+    // so 48 + 98).  1024 x 2048 at 17 / 32 rows 5.9 / 7.2 -> 5.5 / 5.6 us, 1024 x 3072 7.3 / 9.5 -> 7.0 / 7.2.
+    // (float32: only where both parts are added up in the same tree, so that a row's sums are the same whatever the number of rows)
+    fold.part_rows = skinny_tile_rows(N);
+    fold.parts = (N + fold.part_rows - 1) / fold.part_rows;
+    const bool high = fold.part_rows <= 8 && (std::is_same<T, bf16_t>::value || (fold.part_rows & (fold.part_rows - 1)) == 0);
+    const int tr = M <= 16 || !high ? fold.part_rows : 2 * fold.part_rows, blocks = (N + tr - 1) / tr;
+    T* none = nullptr;
+    if (lines_fit(x, w, K))
+        return M <= 16 ? launch_lines<1, 1, false, true, false>(x, w, none, M, N, K, tr, fold, blocks, stream)
+                       : launch_lines<1, 1, false, true, false, T, true>(x, w, none, M, N, K, tr, fold, blocks, stream);
+    if (M <= 16)
+        gemm_skinny_kernel<T, 1, 1, false, true, false, T, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(x, w, none, M, N, K, tr, fold);
+    else
+        gemm_skinny_kernel<T, 1, 1, false, true, false, T, 16, 4, true><<<dim3(blocks, (M + 15) / 16), 16 * LLE_WAVE, 0, stream>>>(x, w, none, M, N, K, tr, fold);
+    LLE_RETURN_LAUNCH_STATUS();
+}
 extern "C" int lle_gemm_skinny_resid_bf16(const void* X, const void* W, void* hidden, const void* norm_weight,
                                           int weight_dtype, void* xw, void* ss_part, int M, int N, int K,
                                           hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (M > 32 || K % 8 != 0 || K <= 0) return (int)hipErrorInvalidValue;
-    NormFold fold = {};
-    fold.hidden = (float*)hidden;
-    fold.weight = norm_weight;
-    fold.weight_dtype = weight_dtype;
-    fold.xw = (bf16_t*)xw;
-    fold.ss_out = (float*)ss_part;
-    // From 17 rows of X on a workgroup takes sixteen of them and, of a narrow model, tiles of W twice as high (two parts of the sums):
-    // with all 32 rows a workgroup of the 0.6B sizes reads eight times as much X as W, every CU all of X (1024 x 3072: 24 + 196 KB,
-    // so 48 + 98).  1024 x 2048 at 17 / 32 rows 5.9 / 7.2 -> 5.5 / 5.6 us, 1024 x 3072 7.3 / 9.5 -> 7.0 / 7.2.
-    fold.part_rows = skinny_tile_rows(N);
-    fold.parts = (N + fold.part_rows - 1) / fold.part_rows;
-    const int tr = M <= 16 || fold.part_rows > 8 ? fold.part_rows : 2 * fold.part_rows, blocks = (N + tr - 1) / tr;
-    const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
-    if (lines_fit((const bf16_t*)X, (const bf16_t*)W, K))
-        return M <= 16 ? launch_lines<1, 1, false, true, false>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream)
-                       : launch_lines<1, 1, false, true, false, bf16_t, true>(x, w, (bf16_t*)nullptr, M, N, K, tr, fold, blocks, stream);
-    if (M <= 16)
-        gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4><<<blocks, 16 * LLE_WAVE, 0, stream>>>(
-            x, w, (bf16_t*)nullptr, M, N, K, tr, fold);
-    else
-        gemm_skinny_kernel<bf16_t, 1, 1, false, true, false, bf16_t, 16, 4, true><<<dim3(blocks, 2), 16 * LLE_WAVE, 0, stream>>>(
-            x, w, (bf16_t*)nullptr, M, N, K, tr, fold);
-    LLE_RETURN_LAUNCH_STATUS();
+    return launch_resid((const bf16_t*)X, (const bf16_t*)W, hidden, norm_weight, weight_dtype, xw, ss_part, M, N, K, stream);
+}
+// The same in float32 (xw too), up to 64 rows (ss_part: whole sixteens of them), K a multiple of 4.
+extern "C" int lle_gemm_skinny_resid_f32(const void* X, const void* W, void* hidden, const void* norm_weight, int weight_dtype, void* xw,
+                                         void* ss_part, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 64 || K % 4 != 0 || K <= 0) return (int)hipErrorInvalidValue;
+    return launch_resid((const float*)X, (const float*)W, hidden, norm_weight, weight_dtype, xw, ss_part, M, N, K, stream);
 }
 
 // The product AFTER a folded norm: X is the xw of lle_gemm_skinny_resid_bf16 and ss_part its
@@ -1318,6 +1337,49 @@ __global__ __launch_bounds__(SK_WAVES* LLE_WAVE) void gemm_skinny_f32_kernel(con
 #pragma unroll
         for (int w = 0; w < SK_WAVES; ++w) sum += s_acc[w][mt][n][m];
         C[row * N + col] = sum;
+    }
+}
+
+// The product after a folded norm in float32 (lle_gemm_skinny_resid_f32): up to 64 rows, gated up to 32; K a multiple of 4.  By way of LDS
+// where K and the operands' addresses let it (then the sums are those of lle_gemm_skinny_f32 and its gated form).
+extern "C" int lle_gemm_skinny_scaled_f32(const void* X, const void* W, void* C, const void* ss_part, int parts, float eps, int M, int N, int K,
+                                          int gated, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    const float *x = (const float*)X, *w = (const float*)W;
+    float* c = (float*)C;
+    if (M > (gated ? 32 : 64) || K <= 0 || parts <= 0 || (gated && N % 2 != 0) || K % 4 != 0) return (int)hipErrorInvalidValue;
+    NormFold fold = {};
+    fold.ss_in = (const float*)ss_part;
+    fold.parts = parts;
+    fold.eps = eps;
+    const int rows = gated ? N / 2 : N, tr = skinny_tile_rows(rows), blocks = (rows + tr - 1) / tr;
+    const int mt = (M + 15) / 16, threads = 16 * LLE_WAVE;
+    hipError_t e;
+    if (!lines_fit(x, w, K)) {
+#define LLE_SCALED_F32(MT, NT, G, U) gemm_skinny_kernel<float, MT, NT, G, false, true, float, 16, U><<<blocks, threads, 0, stream>>>(x, w, c, M, N, K, tr, fold)
+        if (gated) {
+            if (mt == 1) LLE_SCALED_F32(1, 2, true, 2);
+            else LLE_SCALED_F32(2, 2, true, 2);
+        } else switch (mt) {
+            case 1: LLE_SCALED_F32(1, 1, false, 4); break;
+            case 2: LLE_SCALED_F32(2, 1, false, 4); break;
+            case 3: LLE_SCALED_F32(3, 1, false, 2); break;
+            default: LLE_SCALED_F32(4, 1, false, 2); break;
+        }
+#undef LLE_SCALED_F32
+        LLE_RETURN_LAUNCH_STATUS();
+    }
+    if (gated) {
+        if (launch_skinny_stream<float, true, true, float>(x, w, c, M, N, K, fold, stream, e)) return (int)e;
+        return mt == 1 ? launch_lines<1, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream)
+                       : launch_lines<2, 2, true, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
+    }
+    if (launch_skinny_stream<float, false, true, float>(x, w, c, M, N, K, fold, stream, e)) return (int)e;
+    switch (mt) {
+        case 1: return launch_lines<1, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
+        case 2: return launch_lines<2, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
+        case 3: return launch_lines<3, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
+        default: return launch_lines<4, 1, false, false, true>(x, w, c, M, N, K, tr, fold, blocks, stream);
     }
 }
 

@@ -251,6 +251,13 @@ class HipOps:
         most = 32 if width <= self.tuning.skinny_small_width else self.tuning.skinny_max_rows
         return dtype == torch.bfloat16 and 0 < rows <= most and width % 8 == 0 and not self.force_library_gemm
 
+    def can_fold_norm_f32(self, rows: int, width: int) -> bool:
+        """The same for a float32 model: as many rows as the weight-streaming products take (which of two ways a row's norm goes
+        follows the width alone, so its bits do not depend on the number of rows among those), where the products after it go by way
+        of LDS."""
+        return (0 < rows <= self.tuning.skinny_f32_max_rows and width % 32 == 0 and width >= 512
+                and not self.force_library_gemm and not self.force_simt_gemm)
+
     def norm_sum_parts(self, width: int) -> int:
         """Into how many column ranges the product before a folded norm over `width` splits the
         sums of squares (one per tile of its launch; the kernel library decides the tiles)."""
@@ -297,6 +304,39 @@ class HipOps:
                   _ptr(xw), _ptr(sums), M, N, K)
         return Prenormed(xw, sums, fold.eps)
 
+    def _linear_folded_f32(self, x, weight, fold, gated: bool):
+        """_linear_folded of float32 operands (up to 64 rows).  A gated product of more rows than its kernel takes, and where two launches
+        are faster, is the plain one and silu_mul: the same bits."""
+        pre = x if isinstance(x, Prenormed) else None
+        xin = pre.xw if pre is not None else x
+        _dev(xin, "x", torch.float32)
+        _dev(weight, "weight", torch.float32)
+        M, K = xin.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 4 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        _need(pre is None or fold is None, "a product takes a Prenormed or makes one, not both")
+        if pre is not None:
+            _need(self.can_fold_norm_f32(M, K), f"a norm over {K} cannot be folded for {M} rows")
+            _dev(pre.sums, "sums", torch.float32)
+            parts = pre.sums.shape[1]
+            _need(pre.sums.shape[0] == -(-M // 16) * 16, "sums of squares do not fit")
+            _need(not gated or N % 2 == 0, "a gated weight has an even number of rows")
+            in_one = gated and self._gated_f32_in_one(M, N, K)
+            out = torch.empty((M, N // 2 if in_one else N), dtype=torch.float32, device=xin.device)
+            self._run("gemm", "lle_gemm_skinny_scaled_f32", [_P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _P], _ptr(xin), _ptr(weight),
+                      _ptr(out), _ptr(pre.sums), parts, float(pre.eps), M, N, K, int(in_one))
+            return self.silu_mul(out) if gated and not in_one else out
+        _dev(fold.hidden, "hidden", torch.float32)
+        _dev(fold.weight, "norm weight")
+        _need(not gated and fold.hidden.shape == (M, N) and fold.weight.shape == (N,),
+              f"residual stream {list(fold.hidden.shape)} does not fit a product [{M}, {N}]")
+        _need(self.can_fold_norm_f32(M, N), f"a norm over {N} cannot be folded for {M} rows")
+        xw = torch.empty((M, N), dtype=torch.float32, device=xin.device)
+        sums = torch.empty((-(-M // 16) * 16, self.norm_sum_parts(N)), dtype=torch.float32, device=xin.device)
+        self._run("gemm", "lle_gemm_skinny_resid_f32", [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P], _ptr(xin), _ptr(weight),
+                  _ptr(fold.hidden), _ptr(fold.weight), dtype_code(fold.weight.dtype), _ptr(xw), _ptr(sums), M, N, K)
+        return Prenormed(xw, sums, fold.eps)
+
     def linear(self, x, weight, out_dtype=None, fold=None, sums_ok=False):
         """x [M, K] . weight [N, K]^T -> [M, N].  With `sums_ok` the caller takes the result also as
         PartialSums (float32 [slices, M, N], what add_rmsnorm adds into the residual stream).  float32 operands take a
@@ -306,6 +346,9 @@ class HipOps:
         accumulate in 32-bit and write either result type.  `x` a Prenormed or `fold`
         a NormFold: see _linear_folded."""
         if fold is not None or isinstance(x, Prenormed):
+            if weight.dtype == torch.float32:
+                _need(out_dtype in (None, torch.float32), "a float32 product has a float32 result")
+                return self._linear_folded_f32(x, weight, fold, gated=False)
             _need(out_dtype in (None, torch.bfloat16) or (fold is None and out_dtype == torch.float32),
                   "a product that makes a folded norm's input writes bfloat16")
             return self._linear_folded(x, weight, fold, gated=False, out_dtype=out_dtype or torch.bfloat16)
@@ -1022,7 +1065,8 @@ class HipOps:
         Few rows run as ONE weight-streaming launch with the activation in its epilogue, many as one tiled launch where
         wide_form says so; otherwise the product and silu_mul (in float32 also where _gated_f32_in_one says so)."""
         if isinstance(x, Prenormed):
-            return self._linear_folded(x, weight, None, gated=True)
+            folded = self._linear_folded_f32 if weight.dtype == torch.float32 else self._linear_folded
+            return folded(x, weight, None, gated=True)
         _dev(x, "x")
         _dev(weight, "weight", x.dtype)
         M, K = x.shape

@@ -62,6 +62,8 @@ class RMSNorm(Norm):
     def fold(self, hidden) -> Optional[NormFold]:
         if self.one_plus:
             return None
-        if not self.ctx.ops.can_fold_norm(hidden.shape[0], self.size, self.ctx.dtype):
+        ops, rows = self.ctx.ops, hidden.shape[0]
+        in_f32 = getattr(ops, "can_fold_norm_f32", None) if self.ctx.dtype == torch.float32 else None
+        if not (in_f32(rows, self.size) if in_f32 else ops.can_fold_norm(rows, self.size, self.ctx.dtype)):
             return None
         return NormFold(hidden, self.weight, self.eps)

@@ -165,3 +165,44 @@ def test_float32_slices(M, N, K, slices):
     size = x.double().abs() @ w.double().abs().T
     assert bool(((got.double().sum(0) - x.double() @ w.double().T).abs() <= 2.0 ** -24 * (K + 16) * size).all())
     assert torch.equal(got, o.linear_f32_slices(off_lines(x), w, slices))
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K,N2", [(1024, 2048, 1000), (1536, 512, 4100), (520, 1300, 700), (2048, 72, 8450), (4096, 4160, 516)])
+def test_a_float32_norm_folded_into_products(M, N, K, N2):
+    """The residual rows, the norm's input and sums behind a product, and the products after the norm, plain and gated, in float64; the last
+    row alone has the bits that it has among the others (also where a tile holds two parts of the sums); operands at odd
+    addresses are taken."""
+    from litellmengine_amd.parts import NormFold
+
+    o = ops()
+    if not o.can_fold_norm_f32(M, N):
+        assert N % 32 != 0
+        return
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 0.05
+    hidden, norm = torch.randn(M, N, generator=g, device="cuda"), 1 + 0.3 * torch.randn(N, generator=g, device="cuda")
+    hidden[:, N - 3] += 20.0
+    w2 = torch.randn(N2, N, generator=g, device="cuda") * 0.1
+    want = hidden.double() + x.double() @ w.double().T
+    normed = want * torch.rsqrt((want ** 2).mean(1, keepdim=True) + 1e-6) * norm.double()
+    y = normed @ w2.double().T
+    gate, up = y.chunk(2, dim=1)
+
+    def run(x, hidden, w, w2):
+        h = hidden.clone()
+        pre = o.linear(x, w, fold=NormFold(h, norm, 1e-6))
+        return h, pre.xw, pre.sums[: x.shape[0]], o.linear(pre, w2), o.gate_up_silu(pre, w2)
+
+    got = run(x, hidden, w, w2)
+    # a row's products of K and N float32 numbers: a rounding for each, and for their sums', of their sizes; the gate's slope is below 1.1
+    size = (x.double().abs() @ w.double().abs().T + hidden.double().abs()) * 2.0 ** -24 * (K + 16)
+    assert bool(((got[0].double() - want).abs() <= size).all())
+    assert torch.allclose(got[1].double(), got[0].double() * norm.double(), rtol=2.0 ** -23, atol=0)
+    assert torch.allclose(got[2].double().sum(1), (got[0].double() ** 2).sum(1), rtol=1e-5)
+    for mine, exact in ((got[3], y), (got[4], torch.nn.functional.silu(gate) * up)):
+        assert float((mine.double() - exact).norm() / exact.norm()) <= 2.0 ** -24 * 40
+    for a, b in zip(got, run(x[-1:].contiguous(), hidden[-1:].contiguous(), w, w2)):
+        assert torch.equal(a[-1:], b)
+    odd = run(off_lines(x), hidden, off_lines(w), off_lines(w2))
+    assert float((odd[4].double() - got[4].double()).norm() / got[4].double().norm()) <= 2.0 ** -24 * 40
