@@ -34,6 +34,7 @@ LIBRARIES: Dict[str, List[str]] = {
     "gemm_f32": ["gemm_f32.hip"],
     "gemm_tile": ["gemm_tile.hip"],
     "gemm_wide": ["gemm_wide.hip"],
+    "gemm_rows": ["gemm_rows.hip"],
     "sampling": ["sampling.hip"],
     "recurrent": ["recurrent.hip"],
     "latent": ["latent.hip"],
@@ -56,6 +57,7 @@ OWN_HEADERS: Dict[str, List[str]] = {
     "gemm_f32": ["lds.h"],
     "gemm_tile": ["lds.h"],
     "gemm_wide": ["lds.h"],
+    "gemm_rows": ["lds.h"],
 }
 # packed 32-bit float instructions are switched off on purpose (device flag); the first kernel
 # arguments come preloaded into scalar registers with the dispatch instead of being loaded by the

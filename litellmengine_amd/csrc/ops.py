@@ -90,6 +90,7 @@ class HipOps:
         self._forms = {}  # by sizes: the form in which a delta of the residual stream is taken (_form_of_delta) ...
         self._forms_tuning = None  # ... with these numbers
         self._wide = {}  # by sizes: wide_form
+        self._rows = {}  # by sizes: rows_tile
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives, beyond the order of its sums)
 
     # -- plumbing ---------------------------------------------------------
@@ -382,6 +383,9 @@ class HipOps:
                 self._run("gemm", "lle_gemm_skinny_bf16", [_P, _P, _P, _I, _I, _I, _I, _P],
                           _ptr(x), _ptr(weight), _ptr(out), M, N, K, dtype_code(out_dtype))
                 return out
+            tile = self.rows_tile(x, weight, gated=False) if out_dtype == torch.bfloat16 else 0
+            if tile:
+                return self.linear_rows(x, weight, tile)
             # the library product accumulates in 32-bit and can leave the result so
             return torch.mm(x, weight.t()) if out_dtype == torch.bfloat16 else torch.mm(x, weight.t(), out_dtype=out_dtype)
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
@@ -590,6 +594,40 @@ class HipOps:
                 self._wide.clear()
             self._wide[key] = form
         return form if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else -1
+
+    def rows_tile(self, x, weight, gated: bool) -> int:
+        """How many rows of the weight a workgroup takes where a product of 33 to 192 rows is linear_rows' (the kernel library says which
+        are, from the sizes), or 0 where it is not; operands that do not begin at 16 bytes are never."""
+        M, K = x.shape
+        if not 32 < M <= 192 or self.force_library_gemm:
+            return 0
+        key = (M, weight.shape[0], K, int(gated), self.compute_units())
+        tile = self._rows.get(key)
+        if tile is None:
+            fn = getattr(build.load_library("gemm_rows"), "lle_gemm_rows_tile")
+            fn.argtypes, fn.restype = [_I] * 5, _I
+            tile = int(fn(*key))
+            if len(self._rows) >= 4096:
+                self._rows.clear()
+            self._rows[key] = tile
+        return tile if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else 0
+
+    def linear_rows(self, x, weight, tile: int, activation: Optional[str] = None, bias=None, limit: float = 0.0) -> torch.Tensor:
+        """x [M, K], weight [N, K], bfloat16, up to 192 rows, `tile` rows of the weight (or gate rows) a workgroup: x weight^T [M, N], or with
+        `activation` what gated_wide gives, [M, N / 2]."""
+        _dev(x, "x", torch.bfloat16)
+        _dev(weight, "weight", torch.bfloat16)
+        M, K = x.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 256 == 0 and M <= 192, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        _need(activation in (None, "silu", "clamp"), f"unknown activation {activation!r}")
+        if bias is not None:
+            _dev(bias, "bias", torch.bfloat16)
+            _need(activation == "clamp" and bias.shape == (N,), "bias must cover the whole weight of a clamped product")
+        out = torch.empty((M, N // 2 if activation else N), dtype=torch.bfloat16, device=x.device)
+        self._run("gemm_rows", "lle_gemm_rows_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
+                  float(limit), _ptr(out), M, N, K, (None, "silu", "clamp").index(activation), tile)
+        return out
 
     def gated_wide(self, x, weight, form: int, activation: str, bias=None, limit: float = 0.0) -> torch.Tensor:
         """x [M, K], weight [N, K] (gate rows, then up rows), bfloat16, in tiles of that form (see wide_form) -> [M, N / 2]:
@@ -1083,6 +1121,9 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
+        tile = self.rows_tile(x, weight, gated=True) if x.dtype == torch.bfloat16 else 0
+        if tile:
+            return self.linear_rows(x, weight, tile, "silu")
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 else -1
         if form >= 0:
             return self.gated_wide(x, weight, form, "silu")
@@ -1120,8 +1161,12 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_clamped_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(bias), float(limit), _ptr(out), M, N2, K)
             return out
+        aligned = bias is None or bias.data_ptr() % 8 == 0
+        tile = self.rows_tile(x, weight, gated=True) if x.dtype == torch.bfloat16 and limit > 0.0 and aligned else 0
+        if tile:
+            return self.linear_rows(x, weight, tile, "clamp", bias, limit)
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
-        if form >= 0 and (bias is None or bias.data_ptr() % 8 == 0):
+        if form >= 0 and aligned:
             return self.gated_wide(x, weight, form, "clamp", bias, limit)
         return self.bias_act(self.linear(x, weight), "clamp", True, bias=bias, limit=limit)
 
