@@ -59,6 +59,23 @@ __device__ __forceinline__ float4 load_weight4(const void* w, int64_t i, int dty
     return dtype == LLE_F32 ? Quad<float>::load((const float*)w + i) : Quad<bf16_t>::load((const bf16_t*)w + i);
 }
 
+static int units_of_device() {
+    static int units[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (units[dev] == 0 && hipDeviceGetAttribute(&units[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) units[dev] = 256;
+    return units[dev];
+}
+// Threads a row: as many as make four elements each (up to 1024) where the rows are no more than the CUs (`most` times as many), else 256.
+// A wavefront alone issues an instruction in four to eight cycles, so few rows take as long as a thread's part of one: 4096 wide at 1 / 64
+// rows with 256 / with 1024 threads 3.9 / 4.3 -> 2.7 / 3.1 us, in four slices 4.1 / 4.6 -> 3.0 / 3.4, two scaled summands 4.3 / 4.7 -> 2.8 /
+// 3.2; 2048 wide with 512 2.8 / 3.1 -> 2.2 / 2.6; at 2048 rows 16.5 -> 16.6, 18.5 -> 20.3.  (The sum's order follows: bfloat16 rows only, a
+// float32 row's sums are the same whatever else is in the step.)
+static int norm_threads(int R, int H, int most = 1) {
+    if (R > most * units_of_device() || H <= 1024) return 256;
+    return H <= 2048 ? 512 : 1024;
+}
+
 // The same sums in one pass for rows of up to 256 * 4 * NORM_CHUNKS elements (a multiple of 4):
 // every thread keeps its part of the row in registers between the sum and the scaling.
 #define NORM_CHUNKS 8
@@ -67,8 +84,8 @@ __device__ __forceinline__ float4 load_weight4(const void* w, int64_t i, int dty
 // CHUNKS: 1024-element pieces of a row that a thread holds four elements of each; as few as the row needs, so that more
 // rows fit a CU and several slices' loads are on their way at a time (bfloat16, against eight pieces whatever the row: 32 rows of 1024
 // in 16 slices 4.0 against 7.7 us, 2048 rows of 1024 in 4 slices 11.7 against 19.3, 2048 rows of 4096 in 2 slices 32.2 against 34.5).
-template <typename T, typename TD, bool SLICED, int CHUNKS>
-__global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ hidden, const TD* __restrict__ delta,
+template <typename T, typename TD, bool SLICED, int CHUNKS, int THREADS = 256>
+__global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restrict__ hidden, const TD* __restrict__ delta,
                                                               const int32_t* __restrict__ rows,
                                                               const void* __restrict__ weight, int weight_dtype,
                                                               T* __restrict__ out, int H, float eps, int slices,
@@ -82,7 +99,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < CHUNKS; ++k) {  // the weights do not wait for the sum
-        const int i = (k * 256 + threadIdx.x) * 4;
+        const int i = (k * THREADS + threadIdx.x) * 4;
         if (i < H) wv[k] = load_weight4(weight, i, weight_dtype);
     }
     if constexpr (SLICED) {
@@ -91,7 +108,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
         float4 d[CHUNKS];
     #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            const int i = (k * 256 + threadIdx.x) * 4;
+            const int i = (k * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 v[k] = *(const float4*)(h + i);
                 if (dl) d[k] = Quad<TD>::load(dl + i);
@@ -106,7 +123,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
                 for (int b = 0; b < COUNT; ++b)
 #pragma unroll
                     for (int k = 0; k < CHUNKS; ++k) {
-                        const int i = (k * 256 + threadIdx.x) * 4;
+                        const int i = (k * THREADS + threadIdx.x) * 4;
                         if (i < H) e[b][k] = Quad<TD>::load(dl + min(sl + b, slices - 1) * slice_stride + i);  // (past the end: the last once more)
                     }
 #pragma unroll
@@ -127,7 +144,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
         }
     #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            const int i = (k * 256 + threadIdx.x) * 4;
+            const int i = (k * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 float4 x = v[k];
                 if (dl) {
@@ -144,7 +161,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
     } else {
 #pragma unroll
         for (int k = 0; k < CHUNKS; ++k) {
-            const int i = (k * 256 + threadIdx.x) * 4;
+            const int i = (k * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 float4 x = *(const float4*)(h + i);
                 if (dl) {
@@ -165,7 +182,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
     T* o = out + r * H;
 #pragma unroll
     for (int k = 0; k < CHUNKS; ++k) {
-        const int i = (k * 256 + threadIdx.x) * 4;
+        const int i = (k * THREADS + threadIdx.x) * 4;
         if (i < H) {
             const float4 w = wv[k];
             Quad<T>::store(o + i, make_float4(v[k].x * inv * w.x, v[k].y * inv * w.y, v[k].z * inv * w.z,
@@ -269,10 +286,16 @@ extern "C" int lle_embedding_rmsnorm(const void* ids, const void* table, void* h
 template <typename T, typename TD, bool SLICED>
 static void launch_add_rmsnorm(void* hidden, const void* delta, const void* rows, const void* weight, int weight_dtype, void* out, int R,
                                int H, float eps, int slices, int64_t slice_stride, hipStream_t stream) {
-    auto launch = [&](auto kernel) {
-        kernel<<<R, 256, 0, stream>>>((float*)hidden, (const TD*)delta, (const int32_t*)rows, weight, weight_dtype, (T*)out, H, eps, slices,
+    auto launch = [&](auto kernel, int threads = 256) {
+        kernel<<<R, threads, 0, stream>>>((float*)hidden, (const TD*)delta, (const int32_t*)rows, weight, weight_dtype, (T*)out, H, eps, slices,
                                       slice_stride);
     };
+    if constexpr (std::is_same<T, bf16_t>::value) {
+        const int threads = norm_threads(R, H, H <= 4096 ? 2 : 1);  // (5120 wide in four slices at 262 rows 7.1 -> 7.4 us, 4096 wide 5.7 -> 5.0)
+        if (threads == 512) return launch(add_rmsnorm_vec_kernel<T, TD, SLICED, 1, 512>, 512);
+        if (threads == 1024 && H <= 4096) return launch(add_rmsnorm_vec_kernel<T, TD, SLICED, 1, 1024>, 1024);
+        if (threads == 1024) return launch(add_rmsnorm_vec_kernel<T, TD, SLICED, 2, 1024>, 1024);
+    }
     if (H <= 1024)
         launch(add_rmsnorm_vec_kernel<T, TD, SLICED, 1>);
     else if (H <= 2048)
@@ -408,8 +431,8 @@ extern "C" int lle_rmsnorm_add(void* hidden, const void* y, int y_dtype, const v
 // rows[r] gives out[r], and `hidden` is left alone.  The new row waits in registers between the sum of
 // squares and the scaling (rows up to 256 x 4 x SA_CHUNKS wide and a multiple of 4; a plain loop otherwise).
 #define SA_CHUNKS 8
-template <typename TO>
-__global__ __launch_bounds__(256) void scaled_add_rmsnorm_kernel(float* __restrict__ hidden, const void* __restrict__ a,
+template <typename TO, int THREADS = 256>
+__global__ __launch_bounds__(THREADS) void scaled_add_rmsnorm_kernel(float* __restrict__ hidden, const void* __restrict__ a,
                                                                   int a_dtype, const void* __restrict__ b, int b_dtype,
                                                                   float mult_a, float mult_b, const int32_t* __restrict__ rows,
                                                                   const void* __restrict__ weight, int weight_dtype,
@@ -418,11 +441,12 @@ __global__ __launch_bounds__(256) void scaled_add_rmsnorm_kernel(float* __restri
     const int64_t r = rows ? rows[blockIdx.x] : blockIdx.x;
     const int64_t at = r * H, to = (int64_t)blockIdx.x * H;
     float ss = 0.f;
-    if (H % 4 == 0 && H <= 256 * 4 * SA_CHUNKS) {
-        float4 keep[SA_CHUNKS];
+    constexpr int CHUNKS = 256 * SA_CHUNKS / THREADS;
+    if (H % 4 == 0 && H <= 4 * THREADS * CHUNKS) {
+        float4 keep[CHUNKS];
 #pragma unroll
-        for (int c = 0; c < SA_CHUNKS; ++c) {
-            const int i = (c * 256 + threadIdx.x) * 4;
+        for (int c = 0; c < CHUNKS; ++c) {
+            const int i = (c * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 float4 v = *(const float4*)(hidden + at + i);
                 const float4 x = load_weight4(a, at + i, a_dtype);
@@ -440,8 +464,8 @@ __global__ __launch_bounds__(256) void scaled_add_rmsnorm_kernel(float* __restri
         ss = block_sum(ss, red);
         const float inv = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
-        for (int c = 0; c < SA_CHUNKS; ++c) {
-            const int i = (c * 256 + threadIdx.x) * 4;
+        for (int c = 0; c < CHUNKS; ++c) {
+            const int i = (c * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 const float4 w = load_weight4(weight, i, weight_dtype);
                 Quad<TO>::store(out + to + i, make_float4(keep[c].x * inv * w.x, keep[c].y * inv * w.y, keep[c].z * inv * w.z,
@@ -475,10 +499,11 @@ extern "C" int lle_scaled_add_rmsnorm(void* hidden, const void* a, int a_dtype, 
     if (out_dtype == LLE_F32)
         scaled_add_rmsnorm_kernel<float><<<R, 256, 0, stream>>>((float*)hidden, a, a_dtype, b, b_dtype, mult_a, mult_b,
                                                                  (const int32_t*)rows, weight, weight_dtype, (float*)out, H, eps);
-    else
-        scaled_add_rmsnorm_kernel<bf16_t><<<R, 256, 0, stream>>>((float*)hidden, a, a_dtype, b, b_dtype, mult_a, mult_b,
-                                                                  (const int32_t*)rows, weight, weight_dtype, (bf16_t*)out, H,
-                                                                  eps);
+    else {
+        const int threads = norm_threads(R, H, 2);
+        (threads == 256 ? scaled_add_rmsnorm_kernel<bf16_t> : threads == 512 ? scaled_add_rmsnorm_kernel<bf16_t, 512> : scaled_add_rmsnorm_kernel<bf16_t, 1024>)
+            <<<R, threads, 0, stream>>>((float*)hidden, a, a_dtype, b, b_dtype, mult_a, mult_b, (const int32_t*)rows, weight, weight_dtype, (bf16_t*)out, H, eps);
+    }
     LLE_RETURN_LAUNCH_STATUS();
 }
 
@@ -604,8 +629,8 @@ __device__ __forceinline__ void add_quad(float4& v, float4 d) {
     v.w += d.w;
 }
 
-template <typename TO>
-__global__ __launch_bounds__(256) void inject_rmsnorm_kernel(InjectArgs x) {
+template <typename TO, int THREADS = 256>
+__global__ __launch_bounds__(THREADS) void inject_rmsnorm_kernel(InjectArgs x) {
     __shared__ float red[16];
     const int64_t n = x.rows ? x.rows[blockIdx.x] : blockIdx.x, at = n * x.H, to = (int64_t)blockIdx.x * x.H;
     const int H = x.H;
@@ -617,11 +642,12 @@ __global__ __launch_bounds__(256) void inject_rmsnorm_kernel(InjectArgs x) {
     }
     TO* out = (TO*)x.out;
     float ss = 0.f;
-    if (H % 4 == 0 && H <= 256 * 4 * NORM_CHUNKS) {
-        float4 keep[NORM_CHUNKS], wv[NORM_CHUNKS];
+    constexpr int CHUNKS = 256 * NORM_CHUNKS / THREADS;
+    if (H % 4 == 0 && H <= 4 * THREADS * CHUNKS) {
+        float4 keep[CHUNKS], wv[CHUNKS];
 #pragma unroll
-        for (int k = 0; k < NORM_CHUNKS; ++k) {
-            const int i = (k * 256 + threadIdx.x) * 4;
+        for (int k = 0; k < CHUNKS; ++k) {
+            const int i = (k * THREADS + threadIdx.x) * 4;
             if (i < H) {
                 wv[k] = load_weight4(x.weight, i, x.weight_dtype);
                 float4 v = *(const float4*)(x.hidden + at + i);
@@ -644,8 +670,8 @@ __global__ __launch_bounds__(256) void inject_rmsnorm_kernel(InjectArgs x) {
         ss = block_sum(ss, red);
         const float inv = 1.0f / sqrtf(ss / (float)H + x.eps);
 #pragma unroll
-        for (int k = 0; k < NORM_CHUNKS; ++k) {
-            const int i = (k * 256 + threadIdx.x) * 4;
+        for (int k = 0; k < CHUNKS; ++k) {
+            const int i = (k * THREADS + threadIdx.x) * 4;
             if (i < H)
                 Quad<TO>::store(out + to + i, make_float4(keep[k].x * inv * wv[k].x, keep[k].y * inv * wv[k].y,
                                                           keep[k].z * inv * wv[k].z, keep[k].w * inv * wv[k].w));
@@ -690,7 +716,11 @@ extern "C" int lle_inject_rmsnorm(void* hidden, const void* a, int a_dtype, int 
                        table, table_dtype, scale, (const int32_t*)feedback, (const int32_t*)token_seq,
                        (const int32_t*)seq_slots, (const int32_t*)rows, weight, weight_dtype, out, H, eps};
     if (out_dtype == LLE_F32) inject_rmsnorm_kernel<float><<<N, 256, 0, stream>>>(x);
-    else inject_rmsnorm_kernel<bf16_t><<<N, 256, 0, stream>>>(x);
+    else {
+        const int threads = norm_threads(N, H);
+        (threads == 256 ? inject_rmsnorm_kernel<bf16_t> : threads == 512 ? inject_rmsnorm_kernel<bf16_t, 512> : inject_rmsnorm_kernel<bf16_t, 1024>)
+            <<<N, threads, 0, stream>>>(x);
+    }
     LLE_RETURN_LAUNCH_STATUS();
 }
 
