@@ -41,11 +41,19 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& p1, uint32_t&
 // their power leaves: 1800 us, 229 TFLOP/s of float32 product (1.37 PFLOP/s of the instruction); the float32 instruction, in
 // 64 x 64 tiles, took 4160 us.  2048 x 4096 x 12288: 965 us against 1774; 2048 x 4096 x 4096: 321 against 590.  The error
 // against 64 bits is a tenth smaller (1.0e-6 against 1.1e-6 at K = 4096): fewer, exact products per rounding of a sum.
-template <int TM, int TN, int PER_SIMD>
+//
+// SPLIT_SILU, SPLIT_CLAMPED: B holds gate rows and then up rows, N of each, and C [M, N] is act(gate) . up.  Of a wavefront's 64 rows of B
+// the first 32 are gate rows and the others the up rows that go with them, so a lane holds both sums of a place; the same sums and
+// the same bits as the whole product and the activation's pass, without the way of 2 N floats a row to memory and back.
+enum SplitOut { SPLIT_PLAIN = 0, SPLIT_SILU, SPLIT_CLAMPED };
+
+template <int OUT, int TM, int TN, int PER_SIMD>
 __global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const float* __restrict__ A, const float* __restrict__ B,
                                                                       float* __restrict__ C, int M, int N, int K, int64_t lda,
-                                                                      int64_t ldb, int64_t ldc, int m_tiles, int n_tiles, int slice) {
-    constexpr int BM = 64 * TM, BN = 64 * TN;
+                                                                      int64_t ldb, int64_t ldc, int m_tiles, int n_tiles, int slice,
+                                                                      const float* __restrict__ bias, float limit) {
+    constexpr int BM = 64 * TM, BN = 64 * TN, COLUMNS = OUT == SPLIT_PLAIN ? BN : BN / 2;
+    static_assert(OUT == SPLIT_PLAIN || TN == 2, "a gate tile and an up tile for every wavefront");
     extern __shared__ __attribute__((aligned(16))) unsigned char sg_lds[];
     unsigned char* as = sg_lds;                            // [3 parts][BM][4 pieces of 16 bytes]
     unsigned char* bs = sg_lds + 3 * BM * SG_BK * 2;       // [3 parts][BN][4 pieces]
@@ -55,7 +63,7 @@ __global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const floa
     const int die = blockIdx.x % 8, at = blockIdx.x / 8;
     const int nt = die + 8 * (at / m_tiles), mt = at % m_tiles;
     if (nt >= n_tiles) return;
-    const int m0 = mt * BM, n0 = nt * BN;
+    const int m0 = mt * BM, n0 = nt * COLUMNS;
     const int k_begin = blockIdx.y * slice, k_end = min(K, k_begin + slice);  // (a slice is a whole number of steps)
     C += (int64_t)blockIdx.y * M * N;
     // the copy: thread -> (row of 64, piece)
@@ -64,7 +72,12 @@ __global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const floa
 #pragma unroll
     for (int i = 0; i < TM; ++i) ap[i] = A + (int64_t)min(m0 + 64 * i + lr, M - 1) * lda;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) bp[j] = B + (int64_t)min(n0 + 64 * j + lr, N - 1) * ldb;
+    for (int j = 0; j < TN; ++j) {
+        if constexpr (OUT == SPLIT_PLAIN)
+            bp[j] = B + (int64_t)min(n0 + 64 * j + lr, N - 1) * ldb;
+        else
+            bp[j] = B + ((int64_t)min(n0 + 32 * j + lr % 32, N - 1) + (lr < 32 ? 0 : N)) * ldb;
+    }
     const int dst = lr * (SG_BK * 2) + ((lp ^ ((lr >> 3) & 3)) * 16);
     sf32x4 ar[TM][2], br[TN][2];
     auto issue = [&](int k0) {
@@ -146,30 +159,9 @@ __global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const floa
         __builtin_amdgcn_s_barrier();  // nobody reads this step any more
     }
     // lane holds C[m = 8 (e / 4) + 4 (lane / 32) + e % 4][n = lane % 32] of every 32 x 32 tile
-    uint32_t again = 0;  // the tiles with a result that is not finite, the same in all lanes
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            bool odd = false;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
-                const float v = acc[i][j][e];
-                odd |= (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u;
-                if (m < M && n < N) C[m * ldc + n] = v;
-            }
-            if (__any(odd)) again |= 1u << (i * TN + j);
-        }
-    // An infinity has no parts (inf - inf is no number), and numbers within 2^-9 of the largest one round to infinity: such a tile
-    // is made again with the float32 instruction, straight from memory.  (A request whose rows are no numbers any more has this
-    // in every product of every layer, beside requests that are in order.  2048 x 24576 x 4096, 1.8 ms: with one such row 2.9,
-    // with 64 of them 3.7, 72 with a loop over K for every element; with all 2048 rows 8.3.)
-    while (again) {
-        const int t = __builtin_ctz(again), i = t / TN, j = t % TN;
-        again &= again - 1;
-        const float* a_row = A + (int64_t)min(m0 + wm + 32 * i + fr, M - 1) * lda;
-        const float* b_row = B + (int64_t)min(n0 + wn + 32 * j + fr, N - 1) * ldb;
+    auto not_finite = [](float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u; };
+    // the sums of a 32 x 32 tile by the float32 instruction, straight from memory; a_row, b_row: the lane's row of either
+    auto plain_sums = [&](const float* a_row, const float* b_row) {
         sf32x16 sum;
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[e] = 0.f;
@@ -181,29 +173,85 @@ __global__ __launch_bounds__(256, PER_SIMD) void gemm_nt_split_kernel(const floa
 #pragma unroll
             for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[e], sum, 0, 0, 0);
         }
+        return sum;
+    };
+    if constexpr (OUT != SPLIT_PLAIN) {
+        const int n = n0 + wn / 2 + fr, nb = min(n, N - 1);
+        const float b_gate = OUT == SPLIT_CLAMPED && bias ? bias[nb] : 0.f, b_up = OUT == SPLIT_CLAMPED && bias ? bias[N + nb] : 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {  // (what is not finite is made again, as below)
+                bool odd = false;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) odd |= not_finite(acc[i][j][e]);
+                if (__any(odd)) {
+                    const sf32x16 sum = plain_sums(A + (int64_t)min(m0 + wm + 32 * i + fr, M - 1) * lda, B + ((int64_t)nb + (j ? N : 0)) * ldb);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] = not_finite(acc[i][j][e]) ? sum[e] : acc[i][j][e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4;
+                float g = acc[i][0][e], u = acc[i][1][e];
+                if constexpr (OUT == SPLIT_CLAMPED) {
+                    g = fminf(g + b_gate, limit), u = fminf(fmaxf(u + b_up, -limit), limit);
+                    g = g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
+                } else {
+                    g = g / (1.0f + expf(-g)) * u;
+                }
+                if (m < M && n < N) C[m * ldc + n] = g;
+            }
+        }
+        return;
+    }
+    uint32_t again = 0;  // the tiles with a result that is not finite, the same in all lanes
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            bool odd = false;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
+                const float v = acc[i][j][e];
+                odd |= not_finite(v);
+                if (m < M && n < N) C[m * ldc + n] = v;
+            }
+            if (__any(odd)) again |= 1u << (i * TN + j);
+        }
+    // An infinity has no parts (inf - inf is no number), and numbers within 2^-9 of the largest one round to infinity: such a tile
+    // is made again with the float32 instruction, straight from memory.  (A request whose rows are no numbers any more has this
+    // in every product of every layer, beside requests that are in order.  2048 x 24576 x 4096, 1.8 ms: with one such row 2.9,
+    // with 64 of them 3.7, 72 with a loop over K for every element; with all 2048 rows 8.3.)
+    while (again) {
+        const int t = __builtin_ctz(again), i = t / TN, j = t % TN;
+        again &= again - 1;
+        const sf32x16 sum = plain_sums(A + (int64_t)min(m0 + wm + 32 * i + fr, M - 1) * lda, B + (int64_t)min(n0 + wn + 32 * j + fr, N - 1) * ldb);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * fh + e % 4, n = n0 + wn + 32 * j + fr;
             if (m >= M || n >= N) continue;
             float* at = C + m * ldc + n;  // (what is finite stays: a row's bits do not depend on its neighbours)
-            if ((__builtin_bit_cast(uint32_t, *at) & 0x7f800000u) == 0x7f800000u) *at = sum[e];
+            if (not_finite(*at)) *at = sum[e];
         }
     }
 }
 
-template <int TM, int TN, int PER_SIMD>
+template <int OUT, int TM, int TN, int PER_SIMD>
 static int launch_split(const float* A, const float* B, float* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                        int slices, hipStream_t stream) {
-    constexpr int lds = 3 * 64 * (TM + TN) * SG_BK * 2;
-    const int m_tiles = (M + 64 * TM - 1) / (64 * TM), n_tiles = (N + 64 * TN - 1) / (64 * TN);
+                        int slices, hipStream_t stream, const float* bias = nullptr, float limit = 0.f) {
+    constexpr int lds = 3 * 64 * (TM + TN) * SG_BK * 2, columns = OUT == SPLIT_PLAIN ? 64 * TN : 32 * TN;
+    const int m_tiles = (M + 64 * TM - 1) / (64 * TM), n_tiles = (N + columns - 1) / columns;
     static std::atomic<uint64_t> granted{0};
-    const hipError_t e = lle_grant_lds((const void*)gemm_nt_split_kernel<TM, TN, PER_SIMD>, lds, granted);
+    const hipError_t e = lle_grant_lds((const void*)gemm_nt_split_kernel<OUT, TM, TN, PER_SIMD>, lds, granted);
     if (e != hipSuccess) return (int)e;
     const int64_t blocks = (int64_t)8 * m_tiles * ((n_tiles + 7) / 8);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
     const int steps = (K + SG_BK - 1) / SG_BK, slice = (steps + slices - 1) / slices * SG_BK;
-    gemm_nt_split_kernel<TM, TN, PER_SIMD><<<dim3((int)blocks, slices), 256, lds, stream>>>(A, B, C, M, N, K, lda, ldb, ldc, m_tiles,
-                                                                                         n_tiles, slice);
+    gemm_nt_split_kernel<OUT, TM, TN, PER_SIMD><<<dim3((int)blocks, slices), 256, lds, stream>>>(A, B, C, M, N, K, lda, ldb, ldc, m_tiles,
+                                                                                              n_tiles, slice, bias, limit);
     LLE_RETURN_LAUNCH_STATUS();
 }
 
@@ -266,12 +314,52 @@ extern "C" int lle_gemm_nt_f32(const void* A, const void* B, void* C, int M, int
     const float *a = (const float*)A, *b = (const float*)B;
     float* c = (float*)C;
     switch (tiles) {
-        case 0: return launch_split<4, 2, 2>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
-        case 1: return launch_split<2, 2, 3>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
-        case 2: return launch_split<2, 1, 4>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
-        case 3: return launch_split<1, 1, 6>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 0: return launch_split<SPLIT_PLAIN, 4, 2, 2>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 1: return launch_split<SPLIT_PLAIN, 2, 2, 3>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 2: return launch_split<SPLIT_PLAIN, 2, 1, 4>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
+        case 3: return launch_split<SPLIT_PLAIN, 1, 1, 6>(a, b, c, M, N, K, lda, ldb, ldc, slices, stream);
         default: return (int)hipErrorInvalidValue;
     }
+}
+
+// In which tiles (0 or 1 of split_tiles, and one) gate and up, N rows of B together, are taken with their activation, or 0 where the product
+// and a pass for the activation, which may take the other tiles, are expected to be faster: by the times above, 4 us for the launch,
+// and the pass' bytes and half of the product's result at 4.8 TB/s; and where the tiles are one for a CU at most, whose long end nothing covers
+// then.  In a HIP graph, product and pass -> one launch (us; where it is not taken: / one launch):
+//   24576 x 4096 at 262 / 512 / 1024 / 2048 rows 431 / 449, 525 -> 508, 1070 -> 959, 1830 -> 1774; 16384 x 2048 at 300 / 512 / 2048 rows 147 / 143,
+//   178 -> 167, 629 -> 602; 6144 x 1024 at 512 / 1024 / 2048 rows 52 / 60, 85 -> 75, 145 -> 130; 8192 x 1024 at 400 / 700 / 2048 rows 57 / 62,
+//   85 -> 75, 177 -> 159; 51200 x 5120 at 100 / 262 / 700 rows 382 -> 383, 994 -> 959, 2088 -> 1977
+extern "C" int lle_gemm_nt_gated_f32_tiles(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || N % 2 != 0 || K <= 0 || K % 4 != 0) return 0;
+    const int units = units_of_device(), steps = (K + SG_BK - 1) / SG_BK;
+    const float pass = 4.f + (float)M * N * 8 / 4.8e6f;
+    float best = 0.f;
+    int choice = 0;
+    for (int t = 0; t < 4; ++t) {
+        const SplitTile& v = split_tiles[t];
+        const int64_t count = (int64_t)((M + 64 * v.tm - 1) / (64 * v.tm)) * ((N + 64 * v.tn - 1) / (64 * v.tn));
+        const bool in_one = t < 2 && count > units;
+        const float us = (float)steps * fmaxf(v.alone, (float)((count + units - 1) / units) * v.shared) + (in_one ? 0.f : pass);
+        if (t == 0 || us < best) best = us, choice = in_one ? t + 1 : 0;
+    }
+    return choice;
+}
+
+// A [M, K], B [N, K] (gate rows, then up rows), C [M, N / 2], contiguous; N even, K a multiple of 4.  gated 1: silu(gate) . up; gated 2: with bias
+// [N] (or null) and limit, g = min(gate + b, limit), u = clamp(up + b, -limit, limit), C = g sigmoid(1.702 g) (u + 1).  tiles: 0 or 1.
+extern "C" int lle_gemm_nt_gated_f32(const void* A, const void* B, const void* bias, float limit, void* C, int M, int N, int K, int gated,
+                                     int tiles, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || K % 4 != 0 || N % 2 != 0 || (tiles != 0 && tiles != 1)) return (int)hipErrorInvalidValue;
+    const float *a = (const float*)A, *b = (const float*)B;
+    float* c = (float*)C;
+    const int half = N / 2;
+    if (gated == SPLIT_SILU)
+        return tiles == 0 ? launch_split<SPLIT_SILU, 4, 2, 2>(a, b, c, M, half, K, K, K, half, 1, stream)
+                          : launch_split<SPLIT_SILU, 2, 2, 3>(a, b, c, M, half, K, K, K, half, 1, stream);
+    if (gated != SPLIT_CLAMPED || !(limit > 0.f)) return (int)hipErrorInvalidValue;
+    return tiles == 0 ? launch_split<SPLIT_CLAMPED, 4, 2, 2>(a, b, c, M, half, K, K, K, half, 1, stream, (const float*)bias, limit)
+                      : launch_split<SPLIT_CLAMPED, 2, 2, 3>(a, b, c, M, half, K, K, K, half, 1, stream, (const float*)bias, limit);
 }
 
 // ---------------------------------------------------------------------------------

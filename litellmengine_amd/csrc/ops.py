@@ -91,6 +91,7 @@ class HipOps:
         self._forms_tuning = None  # ... with these numbers
         self._wide = {}  # by sizes: wide_form
         self._rows = {}  # by sizes: rows_tile
+        self._gated_f32 = {}  # by sizes: gated_f32_tiles
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives, beyond the order of its sums)
 
     # -- plumbing ---------------------------------------------------------
@@ -472,6 +473,40 @@ class HipOps:
         out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
         self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, slices,
                   tiles)
+        return out
+
+    def gated_f32_tiles(self, x, weight) -> int:
+        """In which tiles (0 or 1) a float32 product of gate and up of more rows than stream the weight takes the activation with it, or -1
+        where the product and a pass for the activation stay (the same bits): the kernel library says, from the sizes."""
+        M, K = x.shape
+        if M <= self.tuning.skinny_f32_max_rows or K % 4 != 0 or self.force_library_gemm or self.force_simt_gemm:
+            return -1
+        key = (M, weight.shape[0], K, self.compute_units())
+        tiles = self._gated_f32.get(key)
+        if tiles is None:
+            fn = getattr(build.load_library("gemm_f32"), "lle_gemm_nt_gated_f32_tiles")
+            fn.argtypes, fn.restype = [_I, _I, _I], _I
+            tiles = int(fn(*key[:3])) - 1
+            if len(self._gated_f32) >= 4096:
+                self._gated_f32.clear()
+            self._gated_f32[key] = tiles
+        return tiles
+
+    def gated_f32(self, x, weight, tiles: int, activation: str, bias=None, limit: float = 0.0) -> torch.Tensor:
+        """x [M, K], weight [N, K] (gate rows, then up rows), float32, in those tiles (see gated_f32_tiles) -> [M, N / 2]:
+        silu(gate) * up, or ("clamp") what gate_up_clamped says."""
+        _dev(x, "x", torch.float32)
+        _dev(weight, "weight", torch.float32)
+        M, K = x.shape
+        N = weight.shape[0]
+        _need(weight.shape[1] == K and K % 4 == 0 and N % 2 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        _need(activation in ("silu", "clamp"), f"unknown activation {activation!r}")
+        if bias is not None:
+            _dev(bias, "bias", torch.float32)
+            _need(activation == "clamp" and bias.shape == (N,), "bias must cover the whole weight of a clamped product")
+        out = torch.empty((M, N // 2), dtype=torch.float32, device=x.device)
+        self._run("gemm_f32", "lle_gemm_nt_gated_f32", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
+                  float(limit), _ptr(out), M, N, K, ("silu", "clamp").index(activation) + 1, tiles)
         return out
 
     SLICED_MIN_ROWS, SLICED_MAX_ROWS = 17, 128  # (lle_gemm_mid_slices_max_rows)
@@ -1127,6 +1162,9 @@ class HipOps:
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 else -1
         if form >= 0:
             return self.gated_wide(x, weight, form, "silu")
+        tiles = self.gated_f32_tiles(x, weight) if x.dtype == torch.float32 else -1
+        if tiles >= 0:
+            return self.gated_f32(x, weight, tiles, "silu")
         return self.silu_mul(self.linear(x, weight))
 
     def _gated_f32_in_one(self, M: int, N2: int, K: int) -> bool:
@@ -1168,6 +1206,9 @@ class HipOps:
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
         if form >= 0 and aligned:
             return self.gated_wide(x, weight, form, "clamp", bias, limit)
+        tiles = self.gated_f32_tiles(x, weight) if x.dtype == torch.float32 and limit > 0.0 else -1
+        if tiles >= 0:
+            return self.gated_f32(x, weight, tiles, "clamp", bias, limit)
         return self.bias_act(self.linear(x, weight), "clamp", True, bias=bias, limit=limit)
 
     # -- arrangements that norm a sublayer's output ------------------------------------
