@@ -1,4 +1,4 @@
-// bfloat16 products X[M, K] . W[N, K]^T of 33 to 192 rows against weights of up to 48 rows for every CU: gate and up with the activation
+// bfloat16 products X[M, K] . W[N, K]^T of 33 to 192 rows (gate and up: 256) against weights of up to 48 rows for every CU: gate and up with the activation
 // between them (W holds gate rows and then up rows), and whole products.
 //
 // A workgroup takes all rows of X and `tile_rows` rows of W (or as many gate rows, and the up rows that go with them), so that the
@@ -10,6 +10,8 @@
 //   24576 x 4096 gated 50.0 / 53.8 / 63.0 -> 45.3 / 49.7 / 54.5; 16384 x 2048 gated 19.9 / 23.0 / 25.3 -> 16.1 / 18.5 / 24.2; 6144 x 1024 gated 14.1 / 15.0 /
 //   16.2 -> 6.2 / 8.3 / 10.5; 10240 x 5120 30.5 / 37.1 -> 27.1 / 36.1; 6144 x 4096 17.8 / 25.3 -> 16.9 / 23.8; 8768 x 2048 15.2 / 18.1 -> 12.2 / 16.0;
 //   4096 x 2048 12.3 / 14.8 -> 8.7 / 12.2; 4096 x 1024 8.7 / 9.3 -> 4.5 / 6.3
+// In tiles of gemm_wide, or the library's product and the pass -> this kernel at 193 / 224 / 256 rows, gated: 24576 x 4096 65.3 / 65.1 / 66.7 -> 57.5 / 60.8 / 61.9;
+//   19456 x 2560 43.7 / 45.8 / 50.7 -> 37.5 / 39.3 / 42.2; 6144 x 1024 16.5 / 14.1 / 14.2 -> 11.2 / 11.9 / 12.5; at 262 rows (288 a workgroup) 70.4 -> 68.7, not built
 // Whole products of more than 128 rows are the library's, and weights of more than one round (51200 x 5120 gated at 64 rows 104 -> 107).
 #include "common.h"
 #include "lds.h"
@@ -160,7 +162,7 @@ static int launch_rows(const void* X, const void* W, const void* bias, float lim
     LLE_RETURN_LAUNCH_STATUS();
 }
 
-// Tiles of up to 16, 32 or 48 rows by up to 64, 128 or 192 of X; the shapes of the wavefronts and stages are those that took the least
+// Tiles of up to 16, 32 or 48 rows by up to 64, 128, 192 or (gated, 16 and 48) 256 of X; the shapes of the wavefronts and stages are those that took the least
 // time (24576 x 4096 gated at 64 rows, tiles of 48: stages of 64 / 128 columns 46.7 / 45.0 us, at 128 rows 49.8 / 58.5; 6144 x 1024 gated at 64
 // rows, tiles of 16: 64 / 128 / 256 columns 6.8 / 6.6 / 6.2).
 template <int OUT>
@@ -176,6 +178,10 @@ static int launch_rows_form(const void* X, const void* W, const void* bias, floa
     ROWS_CASE(12, 4, 1, 1, 1)
     ROWS_CASE(12, 4, 2, 2, 1)
     ROWS_CASE(12, 4, 3, 3, 1)
+    if constexpr (OUT != ROWS_PLAIN) {  // (whole products of so many rows are the library's)
+        ROWS_CASE(16, 8, 1, 1, 1)
+        ROWS_CASE(16, 4, 3, 3, 1)
+    }
 #undef ROWS_CASE
     return (int)hipErrorInvalidValue;
 }
@@ -183,12 +189,14 @@ static int launch_rows_form(const void* X, const void* W, const void* bias, floa
 // How many rows of W a workgroup takes (gated: gate rows) where this kernel takes the product on a chip of `units` CUs, 0 where it does not: as
 // many, in eights, as make the weight one round of the CUs.  Not where X, which every CU reads whole, is many times the CU's share of W, unless
 // the product is short (us, library / so: 2048 x 2048 at 64 / 128 rows 8.9, 8.4 / 6.7, 9.7; 2048 x 4096 at 128 rows 12.7 / 19.5; 4096 x 8192 at 64
-// rows 24.0 / 25.3; 7168 x 5120 at 64 / 96 rows 22.4, 28.7 / 24.8, 30.6; 6144 x 4096 17.8, 22.9 / 16.9, 22.5; 10240 x 5120 30.5, 34.1 / 27.1, 32.6).
+// rows 24.0 / 25.3; gated beyond 192 rows the wide tiles are as fast in between, 16384 x 2048 at 208 / 256 26.0, 26.4 / 26.3, 27.3, 12288 x 1536 20.1, 20.6 / 20.4,
+// 21.6, 8192 x 2048 19.8, 27.6 / 20.4, 22.3; 7168 x 5120 at 64 / 96 rows 22.4, 28.7 / 24.8, 30.6; 6144 x 4096 17.8, 22.9 / 16.9, 22.5; 10240 x 5120 30.5, 34.1 / 27.1, 32.6).
 extern "C" int lle_gemm_rows_tile(int M, int N, int K, int gated, int units) {
-    if (M <= 32 || M > (gated ? 192 : 128) || N <= 0 || units <= 0 || K < 1024 || K % 256 != 0 || (int64_t)192 * K * 2 > 0x7fffffff) return 0;
+    if (M <= 32 || M > (gated ? 256 : 128) || N <= 0 || units <= 0 || K < 1024 || K % 256 != 0 || (int64_t)256 * K * 2 > 0x7fffffff) return 0;
     if (N % (gated ? 8 : 4) != 0) return 0;
     const int rows = gated ? N / 2 : N, share = (rows + units - 1) / units;
     if (share > 48 || K > std::max(M <= 64 ? 4096 : 1024, 176 * share * (gated ? 2 : 1))) return 0;
+    if (M > 192 && share <= 32 && (share > 16 || K > 1024)) return 0;
     return (share + 7) / 8 * 8;
 }
 
@@ -197,7 +205,7 @@ extern "C" int lle_gemm_rows_tile(int M, int N, int K, int gated, int units) {
 extern "C" int lle_gemm_rows_bf16(const void* X, const void* W, const void* bias, float limit, void* C, int M, int N, int K, int gated, int tile_rows,
                                   hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 192 || K <= 0 || K % 256 != 0 || (int64_t)192 * K * 2 > 0x7fffffff || N % (gated ? 8 : 4) != 0) return (int)hipErrorInvalidValue;
+    if (M > (gated ? 256 : 192) || K <= 0 || K % 256 != 0 || (int64_t)256 * K * 2 > 0x7fffffff || N % (gated ? 8 : 4) != 0) return (int)hipErrorInvalidValue;
     if (tile_rows <= 0 || tile_rows > 48 || tile_rows % 4 != 0) return (int)hipErrorInvalidValue;
     if ((((uintptr_t)X | (uintptr_t)W) & 15) || (((uintptr_t)bias | (uintptr_t)C) & 7)) return (int)hipErrorInvalidValue;
     switch (gated) {

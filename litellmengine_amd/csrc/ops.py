@@ -384,7 +384,7 @@ class HipOps:
                 self._run("gemm", "lle_gemm_skinny_bf16", [_P, _P, _P, _I, _I, _I, _I, _P],
                           _ptr(x), _ptr(weight), _ptr(out), M, N, K, dtype_code(out_dtype))
                 return out
-            tile = self.rows_tile(x, weight, gated=False) if out_dtype == torch.bfloat16 else 0
+            tile = self.rows_tile(x, weight, gated=False) if 32 < M <= 192 and out_dtype == torch.bfloat16 else 0
             if tile:
                 return self.linear_rows(x, weight, tile)
             # the library product accumulates in 32-bit and can leave the result so
@@ -631,10 +631,10 @@ class HipOps:
         return form if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else -1
 
     def rows_tile(self, x, weight, gated: bool) -> int:
-        """How many rows of the weight a workgroup takes where a product of 33 to 192 rows is linear_rows' (the kernel library says which
+        """How many rows of the weight a workgroup takes where a product of 33 to 256 rows is linear_rows' (the kernel library says which
         are, from the sizes), or 0 where it is not; operands that do not begin at 16 bytes are never."""
         M, K = x.shape
-        if not 32 < M <= 192 or self.force_library_gemm:
+        if not 32 < M <= 256 or self.force_library_gemm:
             return 0
         key = (M, weight.shape[0], K, int(gated), self.compute_units())
         tile = self._rows.get(key)
@@ -648,13 +648,13 @@ class HipOps:
         return tile if (x.data_ptr() | weight.data_ptr()) % 16 == 0 else 0
 
     def linear_rows(self, x, weight, tile: int, activation: Optional[str] = None, bias=None, limit: float = 0.0) -> torch.Tensor:
-        """x [M, K], weight [N, K], bfloat16, up to 192 rows, `tile` rows of the weight (or gate rows) a workgroup: x weight^T [M, N], or with
+        """x [M, K], weight [N, K], bfloat16, up to 192 rows (with `activation` 256), `tile` rows of the weight (or gate rows) a workgroup: x weight^T [M, N], or with
         `activation` what gated_wide gives, [M, N / 2]."""
         _dev(x, "x", torch.bfloat16)
         _dev(weight, "weight", torch.bfloat16)
         M, K = x.shape
         N = weight.shape[0]
-        _need(weight.shape[1] == K and K % 256 == 0 and M <= 192, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
+        _need(weight.shape[1] == K and K % 256 == 0 and M <= (256 if activation else 192), f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
         _need(activation in (None, "silu", "clamp"), f"unknown activation {activation!r}")
         if bias is not None:
             _dev(bias, "bias", torch.bfloat16)
@@ -1156,7 +1156,7 @@ class HipOps:
             self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
-        tile = self.rows_tile(x, weight, gated=True) if x.dtype == torch.bfloat16 else 0
+        tile = self.rows_tile(x, weight, gated=True) if 32 < M <= 256 and x.dtype == torch.bfloat16 else 0
         if tile:
             return self.linear_rows(x, weight, tile, "silu")
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 else -1
@@ -1200,7 +1200,7 @@ class HipOps:
                       _ptr(x), _ptr(weight), _ptr(bias), float(limit), _ptr(out), M, N2, K)
             return out
         aligned = bias is None or bias.data_ptr() % 8 == 0
-        tile = self.rows_tile(x, weight, gated=True) if x.dtype == torch.bfloat16 and limit > 0.0 and aligned else 0
+        tile = self.rows_tile(x, weight, gated=True) if 32 < M <= 256 and x.dtype == torch.bfloat16 and limit > 0.0 and aligned else 0
         if tile:
             return self.linear_rows(x, weight, tile, "clamp", bias, limit)
         form = self.wide_form(x, weight) if x.dtype == torch.bfloat16 and limit > 0.0 else -1
