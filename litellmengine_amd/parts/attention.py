@@ -91,6 +91,8 @@ class PagedAttention(Mixer):
 
     def bind(self, weights, ctx: BuildContext) -> None:
         self.ctx = ctx
+        if ctx.dtype == torch.float32 and self.nq * self.d % 4 != 0:
+            self.folds_norm = False  # (the float32 products that do a folded norm's work read four columns at a time)
         self.qkv.bind(weights, ctx)
         self.o.bind(weights, ctx)
         self.position.bind(weights, ctx)
