@@ -1169,15 +1169,19 @@ class HipOps:
 
     def _gated_f32_in_one(self, M: int, N2: int, K: int) -> bool:
         """Whether the float32 product of gate and up and its activation are one launch (the same sums either way).  Not
-        * over 32 rows, and up to 16 rows with more than 2560 columns, which the streaming kernel's gated form does not hold
-          (24576 x 4096 at 8 rows 83.6 + 5 against 93.4 us in one launch, at 32 rows 153 + 5 against 122);
+        * over 32 rows, and up to 16 rows with more than 2560 columns but where the streaming kernel's gated form takes them: 3072 and
+          4096 columns, more than 16 gate rows for every CU in tiles of 16, the last of them at least half full (in two launches / in one at 8
+          rows, shares of 20, 24, 28, 32, 33, 35, 40, 48, 49, 52 and 65 gate rows: 4096 columns 37.0 / 38.2, 41.2 / 40.4, 48.5 / 44.2, 52.8 / 49.9, 57.8 / 59.1,
+          59.0 / 59.5, 64.7 / 63.6, 75.8 / 73.2, 81.7 / 84.7, 84.0 / 85.9, 104.9 / 108.3 us; 3072 columns 27.9 / 28.6, 30.3 / 28.9, 35.1 / 32.7,
+          39.1 / 36.9, 42.1 / 43.1, 42.9 / 43.5, 47.1 / 45.3, 57.3 / 55.5, 61.4 / 59.8, 60.6 / 60.8, 78.9 / 79.8);
         * where the plain product's tiles of 16 rows are one for a CU at most: a gated one is two of them, so half of the CUs have
           work or all of them low tiles, which costs more than a launch saves but for short rows and 9 to 16 rows of x (in two
           launches / in one at 1, 8, 16 and 17 rows: 4096 x 1024 7.9, 8.4, 8.9, 9.5 / 6.4, 6.6, 7.3, 9.2 us; 2048 x 1536 7.9, 8.3,
           9.4, 10.7 / 8.3, 8.9, 9.0, 12.5; 4096 x 2560 13.9, 15.8, 18.1, 19.2 / 15.0, 15.1, 17.3, 21.4; 4096 x 4096 at 17 rows
           26.0 / 30.4; 5120 x 1536, over one round of tiles, 13.1, 13.4, 15.1, 18.0 / 10.3, 10.8, 11.8, 14.6)."""
         if M > 32 or (M <= 16 and not 16 < K <= 2560):
-            return False
+            share = -(-(N2 // 2) // self.compute_units())
+            return M <= 16 and K in (3072, 4096) and share > 16 and (share - 1) % 16 >= 7
         return K <= 1024 or N2 > 16 * self.compute_units() or 8 < M <= 16
 
     def gate_up_clamped(self, x, weight, bias, limit: float) -> torch.Tensor:

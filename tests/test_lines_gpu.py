@@ -206,3 +206,23 @@ def test_a_float32_norm_folded_into_products(M, N, K, N2):
         assert torch.equal(a[-1:], b)
     odd = run(off_lines(x), hidden, off_lines(w), off_lines(w2))
     assert float((odd[4].double() - got[4].double()).norm() / got[4].double().norm()) <= 2.0 ** -24 * 40
+
+
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(12290, 4096), (12800, 3072), (24576, 4096), (20996, 3072)])
+def test_float32_gated_streams_of_long_rows(M, N, K):
+    """Shares of 25, 25, 48 and 42 gate rows, the last workgroup's whole or of a few: one launch, plain and behind a folded norm, to the last bit what
+    the product and silu_mul give."""
+    from litellmengine_amd.parts import Prenormed
+
+    o = ops()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 0.05
+    sums = torch.rand(16, o.norm_sum_parts(K), generator=g, device="cuda") * K
+    if o.compute_units() == 256:
+        assert o._gated_f32_in_one(M, N, K) and not any(o._gated_f32_in_one(M, n, K) for n in (8192, 8704, 16896))
+    gate, up = (x.double() @ w.double().T).chunk(2, dim=1)
+    got, want = o.gate_up_silu(x, w), torch.nn.functional.silu(gate) * up
+    assert float((got.double() - want).norm() / want.norm()) <= 2.0 ** -24 * 40
+    assert torch.equal(got, o.silu_mul(o.linear(x, w)))
+    assert torch.equal(o.gate_up_silu(Prenormed(x, sums, 1e-6), w), o.silu_mul(o.linear(Prenormed(x, sums, 1e-6), w)))
