@@ -264,7 +264,20 @@ struct DeltaArgs {
     int H, G, dim, vdim;
     const float* gates;    // [N, 2 H]: decay and beta of every token and head, made ahead (or null: made in the walk)
     const float* decay;    // [N, H dim]: the decays of every key channel (or null: one per head, as above)
+    int S;
+    int most, few;         // requests of more than `most` tokens go in chunks where there are no more than `few` of them
 };
+
+// Whether request s of a step goes in chunks (few: not at all), the same for every wavefront that asks
+__device__ __forceinline__ bool delta_in_chunks(const DeltaArgs& a, int tokens) {
+    if (tokens <= a.most || a.few <= 0) return false;
+    int count = 0;
+    for (int s0 = 0; s0 < a.S; s0 += LLE_WAVE) {
+        const int s = min(s0 + (int)threadIdx.x % LLE_WAVE, a.S - 1);
+        count += __popcll(__ballot(s0 + (int)threadIdx.x % LLE_WAVE < a.S && a.cu_tokens[s + 1] - a.cu_tokens[s] > a.most));
+    }
+    return count <= a.few;
+}
 
 // decay and beta of every token and head, for the walks of long portions: in the walk itself the exponentials and the
 // logarithm of a chunk's sixteen tokens are one wavefront's work while the other three wait (a ninth of the walk's time)
@@ -364,14 +377,15 @@ __device__ __forceinline__ float delta_token(float (&S)[KI], const DeltaToken<KI
     return r;
 }
 
-// grid = (requests, heads, blocks of DELTA_VB value channels).  Thread (jl, ig) = (tid / 16, tid % 16) owns KI key channels
+// grid = (blocks of DELTA_VB value channels, heads, requests): neighbouring workgroups, which go to the dies in turn, are one request's (with the
+// requests in front, one of 256 tokens behind 31 single ones had all its workgroups on one die and took 172 us instead of 42).  Thread (jl, ig) = (tid / 16, tid % 16) owns KI key channels
 // of column j = block DELTA_VB + jl, four neighbours of every 64 (fewer than four: ig KI + 0 .. KI - 1), so that a wavefront's
 // 16-byte loads of k, q, decays and state lie one beside the other: no bank is asked twice, the state's lines are read whole.
 // The tokens pass through LDS DELTA_TC at a time, in two buffers (one for heads over 128 channels): the next chunk goes to LDS
 // and the one behind it is asked for before the current chunk is walked, one barrier a chunk, and inside a chunk every token's
 // operands leave LDS one token ahead of their use.  The read-outs of a chunk are added over the lanes together, at its end, and
 // leave from the registers, the lane's whose number the token has.
-// What bounds a long walk is the chain of a token (the four exchanges of S^T k and what stands around them, 101 ns) in the
+// Long requests go in chunks instead where they are few (below).  What bounds a long walk is the chain of a token (the four exchanges of S^T k and what stands around them, 101 ns) in the
 // two wavefronts that 32 heads of 64 x 64 leave a CU.  Measured with a decay per channel, 32 heads of 64 x 64: 2048 tokens
 // 237 -> 207 us, single tokens of 8 requests 5.0 -> 4.05, of 64 26.0 -> 21.6; one decay a head, 32 heads of 128 x 128: 2048
 // tokens 301 -> 285, single tokens of 8 requests 23.3 -> 10.8, of 32 83.5 -> 34.4; 16 of 256 x 128: 2048 tokens 586 -> 452,
@@ -391,14 +405,14 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
     __shared__ __attribute__((aligned(16))) float s_g[CHANNEL ? BUFS : 1][CHANNEL ? DELTA_TC : 1][CHANNEL ? KD : 4];
     __shared__ __attribute__((aligned(16))) float s_par[BUFS][2][DELTA_TC];  // betas, decays of the staged tokens
     __shared__ __attribute__((aligned(16))) float s_v[BUFS][DELTA_VB][DELTA_TC + 4];
-    const int s = blockIdx.x, h = blockIdx.y;
+    const int s = blockIdx.z, h = blockIdx.y;
     const int tid = threadIdx.x, jl = tid / DELTA_IG, ig = tid % DELTA_IG;
-    const int j0 = blockIdx.z * DELTA_VB, j = j0 + jl;
+    const int j0 = blockIdx.x * DELTA_VB, j = j0 + jl;
     const int dim = a.dim, vdim = a.vdim, H = a.H;
     const int hk = h / (H / a.G), GD = a.G * dim, HV = H * vdim;
     [[maybe_unused]] const int HD = H * dim;
     const int q0 = a.cu_tokens[s], q1 = a.cu_tokens[s + 1];
-    if (q1 <= q0) return;
+    if (q1 <= q0 || delta_in_chunks(a, q1 - q0)) return;
     float* col = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * vdim + j) * dim;
     const bool live = j < vdim;
     constexpr int AT = KI < 4 ? KI : 4, STEP = 4 * DELTA_IG;  // a thread's key channels are m STEP + ig AT + 0 .. AT - 1
@@ -573,25 +587,26 @@ extern "C" int lle_delta_max_dim(void) { return DELTA_MAX_DIM; }
 // q, k float32 [N, G dim] (unit vectors, q scaled), v float32 [N, H vdim], ba float32 [N, 2 H], a_log and dt_bias
 // float32 [H]; state float32 rows of `state_stride` floats whose first H vdim dim hold the heads' states transposed;
 // out float32 [N, H vdim]; `gates` (or null) scratch float32 [N, 2 H] for the decays and betas made ahead of the walk.
+// Where there are `few` requests of more than `most` tokens or fewer, they are left alone: lle_delta_chunks takes them (few = 0: it is not called).
 // `decay` float32 [N, H dim] (or null): the decays of every key channel; then ba (rows of ba_cols floats) holds beta's
 // inputs alone, and a_log, dt_bias and gates are not used.
 extern "C" int lle_delta_scan(const void* q, const void* k, const void* v, const void* ba, int ba_cols, const void* decay,
                               const void* a_log, const void* dt_bias, void* state, int64_t state_stride, const void* seq_slots,
-                              const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, void* gates, int N,
+                              const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, void* gates, int N, int most, int few,
                               hipStream_t stream) {
     if (S <= 0 || H <= 0) return 0;
-    if (G <= 0 || H % G || dim <= 0 || dim > DELTA_MAX_DIM || vdim <= 0 || H > 65535 || (vdim + DELTA_VB - 1) / DELTA_VB > 65535)
+    if (G <= 0 || H % G || dim <= 0 || dim > DELTA_MAX_DIM || vdim <= 0 || H > 65535 || S > 65535)
         return (int)hipErrorInvalidValue;
     if (ba_cols < (decay ? H : 2 * H)) return (int)hipErrorInvalidValue;
     DeltaArgs a{(const float*)q, (const float*)k, (const float*)v, (const float*)ba, ba_cols, (const float*)a_log,
                 (const float*)dt_bias, (float*)state, state_stride, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
-                (float*)out, H, G, dim, vdim, (const float*)gates, (const float*)decay};
+                (float*)out, H, G, dim, vdim, (const float*)gates, (const float*)decay, S, most, few};
     if (gates != nullptr && decay == nullptr) {  // scratch float32 [N, 2 H], given for steps with long portions
         const int64_t total = (int64_t)N * H;
         delta_gates_kernel<<<(int)((total + 255) / 256), 256, 0, stream>>>((const float*)ba, ba_cols, (const float*)a_log,
                                                                             (const float*)dt_bias, (float*)gates, total, H);
     }
-    const dim3 grid(S, H, (vdim + DELTA_VB - 1) / DELTA_VB);
+    const dim3 grid((vdim + DELTA_VB - 1) / DELTA_VB, H, S);
 #define DELTA_CASE(KI)                                                      \
     if (dim <= KI * DELTA_IG) {                                             \
         if (decay) delta_scan_kernel<KI, true><<<grid, DELTA_THREADS, 0, stream>>>(a);   \
@@ -605,6 +620,301 @@ extern "C" int lle_delta_scan(const void* q, const void* k, const void* v, const
     DELTA_CASE(16)
 #undef DELTA_CASE
     return (int)hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------------
+// Long portions: the same recurrence in chunks of sixteen tokens.  With c_t the product of a chunk's decays up to token t (per key
+// channel), S the state before the chunk and r(t, j) = g_{j+1} ... g_t,
+//   L[t][j] = k_t . (r(t, j) k_j)  (j < t),   A[t][j] = q_t . (r(t, j) k_j)  (j <= t)
+//   w_t = beta_t (v_t - (c_t k_t)^T S - sum_{j < t} L[t][j] w_j)
+//   o_t = (c_t q_t)^T S + sum_{j <= t} A[t][j] w_j,   S <- diag(c_16) S + sum_j (r(16, j) k_j) w_j^T
+// The w_t are linear in S, so everything that does not need S is made by one launch for all chunks at once
+// (delta_chunk_kernel): X and U with w = U - X S, row t of both by the forward substitution of the line for w_t.  What is
+// left to walk is a chunk at a time, three small products (delta_chunk_walk_kernel).  Products of decays are taken as they are, never as
+// quotients: a decay of 0 is as good as any.  All of it in 32 bits, the products on the float32 matrix instruction.
+//
+// A chunk's unit in `work`, float32: X [16][dim], c q [16][dim], r(16, j) k_j [dim][16], A [16][16], c_16 [dim], U [columns][16] (whole
+// sixteens of value channels).  Request s has the chunks cu_tokens[s] / 16 + s and on, so that every request's are found without
+// a table.
+// ---------------------------------------------------------------------------------
+typedef float delta_vec4 __attribute__((ext_vector_type(4)));
+
+static constexpr int delta_unit_floats(int dim, int vdim) { return 3 * DELTA_TC * dim + DELTA_TC * DELTA_TC + dim + DELTA_TC * ((vdim + 15) / 16 * 16); }
+
+// grid = (chunks, heads).  Thread (j, ig) = (tid / 16, tid % 16) follows r(t, j) k_j over its 4 KT channels through the chunk's tokens; its
+// shares of L[., j] and A[., j] are added over the row of sixteen lanes in one go.  Then a thread a column of X and of U.
+template <int KT, bool CHANNEL>
+__global__ __launch_bounds__(DELTA_THREADS) void delta_chunk_kernel(DeltaArgs a, int chunks, float* __restrict__ work) {
+    constexpr int KD = 64 * KT, TC = DELTA_TC;
+    __shared__ __attribute__((aligned(16))) float s_k[TC][KD], s_q[TC][KD], s_g[CHANNEL ? TC : 1][CHANNEL ? KD : TC];
+    __shared__ __attribute__((aligned(16))) float s_l[TC][TC], s_beta[TC], s_kd[KD][TC + 1];
+    const int h = blockIdx.y, tid = threadIdx.x;
+    int s = 0;  // the last request whose chunks begin here or before
+    for (int high = a.S - 1; s < high;) {
+        const int mid = (s + high + 1) / 2;
+        if (a.cu_tokens[mid] / TC + mid <= (int)blockIdx.x) s = mid;
+        else high = mid - 1;
+    }
+    const int q0 = a.cu_tokens[s], q1 = a.cu_tokens[s + 1], c0 = q0 + ((int)blockIdx.x - q0 / TC - s) * TC;
+    if (c0 >= q1 || !delta_in_chunks(a, q1 - q0)) return;
+    const int nt = min(TC, q1 - c0), hk = h / (a.H / a.G), GD = a.G * KD, HV = a.H * a.vdim;
+    // behind the last token: k, q and beta 0, decays 1
+#pragma unroll
+    for (int r = 0; r < KT; ++r) {
+        const int e = (tid + DELTA_THREADS * r) * 4, t = e / KD, i = e - t * KD;
+        float4 x = float4{0.f, 0.f, 0.f, 0.f}, y = x, z = float4{1.f, 1.f, 1.f, 1.f};
+        if (t < nt) {
+            const int64_t at = (int64_t)(c0 + t) * GD + hk * KD + i;
+            x = *(const float4*)(a.q + at);
+            y = *(const float4*)(a.k + at);
+            if constexpr (CHANNEL) z = *(const float4*)(a.decay + (int64_t)(c0 + t) * a.H * KD + h * KD + i);
+        }
+        *(float4*)&s_q[t][i] = x;
+        *(float4*)&s_k[t][i] = y;
+        if constexpr (CHANNEL) *(float4*)&s_g[t][i] = z;
+    }
+    if (tid < TC) {
+        const float* ba = a.ba + (int64_t)(c0 + min(tid, nt - 1)) * a.ba_cols;
+        s_beta[tid] = tid < nt ? 1.0f / (1.0f + expf(-ba[h])) : 0.f;
+        if constexpr (!CHANNEL) {
+            const float x = ba[a.H + h] + a.dt_bias[h], softplus = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
+            s_g[0][tid] = tid < nt ? expf(-expf(a.a_log[h]) * softplus) : 1.f;
+        }
+    }
+    // from here on thread c makes column c of X (c < KD) or column c - KD of U, which begins with v: asked for ahead of everything
+    const int column = __builtin_amdgcn_readfirstlane(tid / LLE_WAVE) * LLE_WAVE < KD ? tid : tid - KD;
+    const bool of_x = __builtin_amdgcn_readfirstlane(tid / LLE_WAVE) * LLE_WAVE < KD, of_u = !of_x && column < (a.vdim + 15) / 16 * 16;
+    float y[TC];
+    if (of_u) {
+        const float* v = a.v + (int64_t)c0 * HV + h * a.vdim + min(column, a.vdim - 1);
+#pragma unroll
+        for (int t = 0; t < TC; ++t) y[t] = v[(int64_t)min(t, nt - 1) * HV];
+    }
+    float* unit = work + ((int64_t)h * chunks + blockIdx.x) * delta_unit_floats(KD, a.vdim);
+    float *out_x = unit, *out_q = unit + TC * KD, *out_k = unit + 2 * TC * KD, *out_a = unit + 3 * TC * KD, *out_c = out_a + TC * TC, *out_u = out_c + KD;
+    __syncthreads();
+    {
+        const int j = tid / TC, ig = tid % TC;
+        delta_vec4 r[KT];
+        float l[TC], p[TC];
+#pragma unroll
+        for (int m = 0; m < KT; ++m) r[m] = *(const delta_vec4*)&s_k[j][64 * m + 4 * ig];
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {
+            l[t] = p[t] = 0.f;
+            if (t < tid / LLE_WAVE * 4) continue;  // (the wavefront's four j come later)
+            float dl = 0.f, dp = 0.f;
+#pragma unroll
+            for (int m = 0; m < KT; ++m) {
+                const delta_vec4 k = *(const delta_vec4*)&s_k[t][64 * m + 4 * ig], q = *(const delta_vec4*)&s_q[t][64 * m + 4 * ig];
+                delta_vec4 g;
+                if constexpr (CHANNEL) g = *(const delta_vec4*)&s_g[t][64 * m + 4 * ig];
+                else g = delta_vec4{s_g[0][t], s_g[0][t], s_g[0][t], s_g[0][t]};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    r[m][e] *= t > j ? g[e] : 1.f;
+                    dl = fmaf(r[m][e], k[e], dl);
+                    dp = fmaf(r[m][e], q[e], dp);
+                }
+            }
+            l[t] = t > j ? dl : 0.f;
+            p[t] = t >= j ? dp : 0.f;
+        }
+        s_l[ig][j] = delta_row_sums(l, ig);
+        out_a[ig * TC + j] = delta_row_sums(p, ig);
+#pragma unroll
+        for (int m = 0; m < KT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s_kd[64 * m + 4 * ig + e][j] = r[m][e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4 * KT; ++r) {
+        const int e = tid + DELTA_THREADS * r;
+        out_k[e] = s_kd[e / TC][e % TC];
+    }
+    auto substitute = [&]() {
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {
+            float sum = y[t];
+#pragma unroll
+            for (int i = 0; i < t; ++i) sum = fmaf(-s_l[t][i], y[i], sum);
+            y[t] = s_beta[t] * sum;
+        }
+    };
+    if (of_x) {
+        float cum = 1.f;
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {
+            if constexpr (CHANNEL) cum *= s_g[t][column];
+            else cum *= s_g[0][t];
+            y[t] = cum * s_k[t][column];
+            out_q[t * KD + column] = cum * s_q[t][column];
+        }
+        out_c[column] = cum;
+        substitute();
+#pragma unroll
+        for (int t = 0; t < TC; ++t) out_x[t * KD + column] = y[t];
+    } else if (of_u) {
+#pragma unroll
+        for (int t = 0; t < TC; ++t) y[t] = t < nt && column < a.vdim ? y[t] : 0.f;
+        substitute();
+#pragma unroll
+        for (int t = 0; t < TC; t += 4) *(float4*)(out_u + column * TC + t) = float4{y[t], y[t + 1], y[t + 2], y[t + 3]};
+    }
+}
+
+// grid = (sixteens of value channels, heads, requests).  The first NW wavefronts carry the state, one for every sixteen key channels: it keeps
+// its tile of S, rows 4 c + e and column r in lane (c, r), element e, which is the operand of a product over the key channels as it
+// lies; so are the w_t for one over the tokens.  Their shares of X S meet in LDS (two buffers, one barrier a chunk), AHEAD chunks of operands are
+// on their way.  The other NW wavefronts take the read-outs of every NW-th chunk each, a tile of S in the time of a chunk: a wavefront issues
+// in order, so what is not on the chain S -> X S -> LDS -> w -> S is not in the chain's wavefronts.
+// What bounds it is that chain, 0.48 us a chunk (16 of the float32 matrix instruction's 32 cycles, a barrier, the trip through LDS): with
+// every wavefront taking its share of the read-outs 0.53, with a barrier that waits for loads 0.74; operands that are never
+// further than L2 change nothing.  32 heads of 64 x 64 with a decay per channel: the chunks' launch 28 us and this one 55 for 2048 tokens, walked 207.
+template <int NW, int AHEAD>
+__global__ __launch_bounds__(2 * NW * LLE_WAVE, NW / 2) void delta_chunk_walk_kernel(DeltaArgs a, int chunks, const float* __restrict__ work) {
+    constexpr int KD = 16 * NW, TC = DELTA_TC;
+    __shared__ __attribute__((aligned(16))) float s_p[2][NW][256], s_s[2][NW][256];  // X S of every sixteen key channels, S
+    const int s = blockIdx.z, h = blockIdx.y;
+    const int q0 = a.cu_tokens[s], q1 = a.cu_tokens[s + 1];
+    if (!delta_in_chunks(a, q1 - q0)) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE, c = lane / 16, r = lane % 16;
+    const int j = blockIdx.x * 16 + r;
+    const int unit = delta_unit_floats(KD, a.vdim), n = (q1 - q0 + TC - 1) / TC;
+    // (a buffer's address and the chunk's offset are the wavefront's, so that a load takes no additions of 64 bits)
+    const __amdgpu_buffer_rsrc_t units =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(work + ((int64_t)h * chunks + q0 / TC + s) * unit), 0, 4 * unit * n, 0x00020000);
+    auto load = [&](int i, unsigned at) {  // (behind the last chunk: the last one again)
+        return __builtin_bit_cast(delta_vec4, __builtin_amdgcn_raw_buffer_load_b128(units, 4 * at, 4 * unit * min(i, n - 1), 0));
+    };
+    const unsigned in_row = r * KD + 4 * c, in_k = 2 * TC * KD + (16 * wave + r) * TC + 4 * c, in_a = 3 * TC * KD + r * TC + 4 * c;
+    const unsigned in_g = 3 * TC * KD + TC * TC + 16 * wave + 4 * c, in_u = 3 * TC * KD + TC * TC + KD + j * TC + 4 * c;
+    auto meet = [&]() {  // (waits for no load on its way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto corrections = [&](const delta_vec4& u, int i) {  // w of chunk i
+        delta_vec4 part[NW];
+#pragma unroll
+        for (int v = 0; v < NW; ++v) part[v] = *(const delta_vec4*)&s_p[i & 1][v][lane * 4];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) part[0] += part[v];
+        return u - part[0];
+    };
+    if (wave < NW) {
+        const bool live = j < a.vdim;
+        float* at = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * a.vdim + min(j, a.vdim - 1)) * KD + 16 * wave + 4 * c;
+        delta_vec4 St;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) St[e] = at[e];
+        struct Operands {
+            delta_vec4 x, k, u, g;
+        } ops[AHEAD];
+        auto ask = [&](Operands& o, int i) {
+            o.x = load(i, in_row + 16 * wave);
+            o.u = load(i, in_u);
+            o.g = load(i, in_g);
+            o.k = load(i, in_k);
+        };
+        auto chunk = [&](Operands& now, int i) {
+            delta_vec4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p = __builtin_amdgcn_mfma_f32_16x16x4f32(now.x[e], St[e], p, 0, 0, 0);
+            *(delta_vec4*)&s_s[i & 1][wave][lane * 4] = St;
+            St *= now.g;
+            *(delta_vec4*)&s_p[i & 1][wave][lane * 4] = p;
+            meet();
+            const delta_vec4 w = corrections(now.u, i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) St = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[e], w[e], St, 0, 0, 0);
+            ask(now, i + AHEAD);
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) ask(ops[i], i);
+        int i0 = 0;
+        for (; i0 + AHEAD <= n; i0 += AHEAD)
+#pragma unroll
+            for (int b = 0; b < AHEAD; ++b) chunk(ops[b], i0 + b);
+#pragma unroll
+        for (int b = 0; b < AHEAD - 1; ++b)
+            if (i0 + b < n) chunk(ops[b], i0 + b);
+        if (live)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) at[e] = St[e];
+        return;
+    }
+    const int mine = wave - NW;
+    const int64_t HV = (int64_t)a.H * a.vdim;
+    float* to = a.out + (q0 + mine * TC + 4 * c) * HV + h * a.vdim + j;
+    for (int i = 0; i < min(mine, n); ++i) meet();
+    for (int i = mine; i < n; i += NW) {
+        delta_vec4 q[NW], S[NW];
+#pragma unroll
+        for (int v = 0; v < NW; ++v) q[v] = load(i, TC * KD + in_row + 16 * v);
+        const delta_vec4 t = load(i, in_a), u = load(i, in_u);
+        meet();
+#pragma unroll
+        for (int v = 0; v < NW; ++v) S[v] = *(const delta_vec4*)&s_s[i & 1][v][lane * 4];
+        const delta_vec4 w = corrections(u, i);
+        delta_vec4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            if (v > 0 && i + v < n) meet();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[v][e], S[v][e], o, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(t[e], w[e], o, 0, 0, 0);
+        const int left = q1 - (q0 + i * TC + 4 * c);
+        if (j < a.vdim) {
+            if (i < n - 1) {  // (the same for the wavefront: a whole chunk)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) to[e * HV] = o[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (e < left) to[e * HV] = o[e];
+            }
+        }
+        to += NW * TC * HV;
+    }
+}
+
+// Floats of `work` for a step of N tokens of S requests, or 0 where no chunks are made of such heads or of so many tokens.
+extern "C" int lle_delta_chunk_floats(int N, int S, int H, int dim, int vdim) {
+    if (N <= 0 || S <= 0 || H <= 0 || H > 65535 || vdim <= 0 || (dim != 64 && dim != 128) || dim + vdim > DELTA_THREADS) return 0;
+    const int64_t floats = (int64_t)(N / DELTA_TC + S) * H * delta_unit_floats(dim, vdim);
+    return floats <= 0x7fffffff ? (int)floats : 0;
+}
+
+// The requests of more than `most` tokens of lle_delta_scan (its arguments), where they are `few` or fewer; `work` float32 of lle_delta_chunk_floats, q, k, decay
+// and work at 16 bytes.
+extern "C" int lle_delta_chunks(const void* q, const void* k, const void* v, const void* ba, int ba_cols, const void* decay,
+                                const void* a_log, const void* dt_bias, void* state, int64_t state_stride, const void* seq_slots,
+                                const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, int N, int most, int few, void* work,
+                                hipStream_t stream) {
+    if (S <= 0 || H <= 0 || N <= 0) return 0;
+    if (lle_delta_chunk_floats(N, S, H, dim, vdim) == 0 || G <= 0 || H % G || S > 65535 || ba_cols < (decay ? H : 2 * H) || most < 0 ||
+        (((uintptr_t)q | (uintptr_t)k | (uintptr_t)decay | (uintptr_t)work) & 15))
+        return (int)hipErrorInvalidValue;
+    const DeltaArgs a{(const float*)q, (const float*)k, (const float*)v, (const float*)ba, ba_cols, (const float*)a_log,
+                      (const float*)dt_bias, (float*)state, state_stride, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
+                      (float*)out, H, G, dim, vdim, nullptr, (const float*)decay, S, most, few};
+    const int chunks = N / DELTA_TC + S;
+    const dim3 all(chunks, H), walk((vdim + 15) / 16, H, S);
+    float* w = (float*)work;
+    if (dim == 64) {
+        if (decay) delta_chunk_kernel<1, true><<<all, DELTA_THREADS, 0, stream>>>(a, chunks, w);
+        else delta_chunk_kernel<1, false><<<all, DELTA_THREADS, 0, stream>>>(a, chunks, w);
+        delta_chunk_walk_kernel<4, 4><<<walk, 8 * LLE_WAVE, 0, stream>>>(a, chunks, w);
+    } else {
+        if (decay) delta_chunk_kernel<2, true><<<all, DELTA_THREADS, 0, stream>>>(a, chunks, w);
+        else delta_chunk_kernel<2, false><<<all, DELTA_THREADS, 0, stream>>>(a, chunks, w);
+        delta_chunk_walk_kernel<8, 4><<<walk, 16 * LLE_WAVE, 0, stream>>>(a, chunks, w);
+    }
+    LLE_RETURN_LAUNCH_STATUS();
 }
 
 // ---------------------------------------------------------------------------------

@@ -2077,6 +2077,14 @@ class HipOps:
 
     DELTA_GATES_AHEAD = 64  # tokens of a step from which decays and betas are made by a launch of their own
 
+    # Long requests of heads of 64 or 128 key channels go in chunks where their workgroups (one for a head and sixteen value channels) are no
+    # more than the CUs: the walk's wavefronts, which share their SIMDs with one another well, are as fast or faster from there on (32
+    # heads of 64 x 64, chunks / walk in us: one request of 128, 256, 2048 tokens 15 / 17, 21 / 29, 83 / 209; two of 192, 1024 23 / 23,
+    # 64 / 108; four of 256, 1024 41 / 38, 134 / 129; 32 heads of 128 x 128: one of 128, 192, 2048 25 / 25, 29 / 33, 162 / 291; two of 512
+    # 95 / 96, four 194 / 175).
+    DELTA_WALK = 160  # most tokens of a request that are always walked
+    DELTA_CHUNK_FLOATS = 1 << 28  # of what the chunks of a step keep, 1 GiB (59000 tokens of 32 heads of 64 x 64); steps of more tokens are walked
+
     def delta_scan(self, q, k, v, ba, a_log, dt_bias, state, heads: int, kv_heads: int, dim: int, vdim: int, seq_slots,
                    cu_tokens, decay=None) -> torch.Tensor:
         """Per head h, with the matrix state S [dim, vdim] of the request (float32; `state[slot]` holds the heads'
@@ -2111,10 +2119,24 @@ class HipOps:
         out = torch.empty((N, H * vdim), dtype=torch.float32, device=v.device)
         # steps with portions: the exponentials of decay and beta leave the walk (a step of single tokens keeps them there:
         # one launch less).  The number of tokens is known on the host and fixed inside a graph.
+        args = (_ptr(q), _ptr(k), _ptr(v), _ptr(ba), ba.shape[1], _ptr(decay), _ptr(a_log), _ptr(dt_bias), _ptr(state), state.stride(0),
+                _ptr(seq_slots), _ptr(cu_tokens), _ptr(out), S, H, G, dim, vdim)
+        types = [_P, _P, _P, _P, _I, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I]
+        few = 0  # requests that may go in chunks
+        if N - S + 1 > self.DELTA_WALK * (1 if S == 1 else 4):  # (so many tokens may be one request's)
+            few = self.compute_units(v.device) // (H * -(-int(vdim) // 16))
+            if S > few and N > S * self.DELTA_WALK:  # (about all of them are long)
+                few = 0
+            floats = self._get("delta", "lle_delta_chunk_floats", [_I, _I, _I, _I, _I])(N, S, H, dim, vdim) if few > 0 else 0
+            if 0 < floats <= self.DELTA_CHUNK_FLOATS and not any(t is not None and t.data_ptr() % 16 for t in (q, k, decay)):
+                work = torch.empty((floats,), dtype=torch.float32, device=v.device)
+                self._run("delta", "lle_delta_chunks", types + [_I, _I, _I, _P, _P], *args, N, self.DELTA_WALK, few, _ptr(work))
+                if S == 1:
+                    return out
+            else:
+                few = 0
         gates = torch.empty((N, 2 * H), dtype=torch.float32, device=v.device) if decay is None and N >= max(self.DELTA_GATES_AHEAD, 2 * S) else None
-        self._run("delta", "lle_delta_scan", [_P, _P, _P, _P, _I, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P],
-                  _ptr(q), _ptr(k), _ptr(v), _ptr(ba), ba.shape[1], _ptr(decay), _ptr(a_log), _ptr(dt_bias), _ptr(state), state.stride(0),
-                  _ptr(seq_slots), _ptr(cu_tokens), _ptr(out), S, H, G, dim, vdim, _ptr(gates), N)
+        self._run("delta", "lle_delta_scan", types + [_P, _I, _I, _I, _P], *args, _ptr(gates), N, self.DELTA_WALK, few)
         return out
 
     def delta_out_norm(self, o, gate, norm_w, eps: float, heads: int, vdim: int, act: str = "silu", out_dtype=None) -> torch.Tensor:

@@ -1,0 +1,45 @@
+"""The delta rule in chunks of sixteen tokens (long requests where they are few) against the plain recurrence: the shortest request that goes in
+chunks and the longest that is walked, last chunks of one and of fifteen tokens, value channels that are no sixteens, one decay
+a head and one a channel, decays of zero and of one, more long requests than go in chunks."""
+import pytest
+import torch
+
+from .torch_ops import TorchOps
+
+pytestmark = pytest.mark.gpu
+REF = TorchOps()
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("dim,vdim,H,G,lens", [(64, 64, 2, 1, [161]), (64, 64, 4, 2, [1, 700, 160, 161, 3]), (64, 17, 3, 3, [223]), (64, 192, 2, 1, [176]),
+                                               (128, 128, 2, 2, [175]), (128, 16, 2, 1, [5, 1, 650]), (64, 16, 130, 1, [165, 170, 400])])
+def test_long_requests_in_chunks(dim, vdim, H, G, lens, channel):
+    from litellmengine_amd.csrc.ops import HipOps
+
+    o = HipOps()
+    N, S, rand = sum(lens), len(lens), torch.Generator().manual_seed(dim + vdim)
+    f = lambda *shape: torch.randn(shape, generator=rand).cuda()
+    unit = lambda t: torch.nn.functional.normalize(t.view(N, G, dim), dim=-1).reshape(N, G * dim).contiguous()
+    q, k, v, ba = unit(f(N, G * dim)), unit(f(N, G * dim)), f(N, H * vdim), f(N, 2 * H)
+    k[N // 2] = k[N // 2 - 1]  # a key written twice
+    a_log, dt_bias = (None, None) if channel else (f(H), f(H))
+    decay = torch.sigmoid(3.0 * f(N, H * dim)) if channel else None
+    if channel:
+        decay[:, ::7], decay[:, 1::7] = 1.0, 0.0  # some channels never forget, some at once
+        decay[::5] = 1.0
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    cu, slots = ints([sum(lens[:i]) for i in range(S + 1)]), ints(list(range(S, 0, -1)))
+    start = 0.3 * f(S + 2, H * vdim * dim + 5)
+    a, b = start.clone(), start.clone()
+    want = REF.delta_scan(q, k, v, ba, a_log, dt_bias, a, H, G, dim, vdim, slots, cu, decay=decay)
+    got = o.delta_scan(q, k, v, ba, a_log, dt_bias, b, H, G, dim, vdim, slots, cu, decay=decay)
+    # values stay of the order of |v| + |S_0|, up to about 5 (unit keys, decays and betas up to one).  Where channels never forget an error
+    # of a token stays, too: 700 tokens, each with sums of up to 144 products in 32 bits, sqrt(700 x 144) x 2^-24 x 5 = 1e-4, and twice that for
+    # the largest of 10^5 elements
+    assert (got.double() - want.double()).abs().max() < 2e-4
+    assert (a.double() - b.double()).abs().max() < 2e-4
+    assert torch.equal(b[:, H * vdim * dim:], start[:, H * vdim * dim:]) and torch.equal(b[0], start[0]) and torch.equal(b[S + 1], start[S + 1])
+    if S == 1:  # walked one by one, the same recurrence in another order
+        o.DELTA_WALK, c = N, start.clone()
+        walked = o.delta_scan(q, k, v, ba, a_log, dt_bias, c, H, G, dim, vdim, slots, cu, decay=decay)
+        assert (got - walked).abs().max() < 2e-4 and not torch.equal(got, walked)
