@@ -6,12 +6,14 @@ CPU path: without a GPU or without the compiled libraries these raise.
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import Optional
 
 import torch
 
 from ..parts.base import Injected, PartialSums, Prenormed, ScaledSum
 from . import build
+from .record import LaunchRecord
 from .tuning import ProductTuning
 from .limits import (MAX_DELTA_HEAD_DIM, MAX_GLA_HEAD_DIM, MAX_HEAD_DIM, MAX_SSD_DIM, MAX_SUMMED_NORM_WIDTH,
                      MAX_WKV_HEAD_DIM)
@@ -21,10 +23,36 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _L = ctypes.c_int64
 _F = ctypes.c_float
+_TYPES = {"P": _P, "I": _I, "L": _L, "F": _F}
 
 
 class KernelError(RuntimeError):
     pass
+
+
+class _Recording(threading.local):
+    to: Optional[LaunchRecord] = None  # the record that this thread's launches go into (record.py)
+
+
+_recording = _Recording()
+_of_kind = {}  # (dtype, device) -> a tensor of no elements: its new_empty() takes the host 0.25 us less than torch.empty() with a type and a device
+
+
+def _made(shape, dtype, device) -> torch.Tensor:
+    kind = _of_kind.get((dtype, device))
+    if kind is None:
+        kind = _of_kind[dtype, device] = torch.empty((0,), dtype=dtype, device=device)
+    t = kind.new_empty(shape)
+    if _recording.to is not None:
+        _recording.to.made.append(t)
+    return t
+
+
+def _made_like(x: torch.Tensor) -> torch.Tensor:
+    t = torch.empty_like(x)
+    if _recording.to is not None:
+        _recording.to.made.append(t)
+    return t
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -78,6 +106,10 @@ def _stream_handle() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _library_product(x, weight, out):
+    torch.mm(x, weight.t(), out=out)
+
+
 class HipOps:
     """The operations a model part may call.  One instance per process is enough."""
 
@@ -96,21 +128,62 @@ class HipOps:
 
     # -- plumbing ---------------------------------------------------------
     def _get(self, lib: str, name: str, argtypes):
+        """`argtypes`: ctypes' types, or a letter for each (a text is no list that every launch makes anew)."""
         key = (lib, name)
         fn = self._fn.get(key)
         if fn is None:
             fn = getattr(build.load_library(lib), name)
-            fn.argtypes = argtypes
+            fn.argtypes = [_TYPES[t] for t in argtypes] if isinstance(argtypes, str) else argtypes
             fn.restype = ctypes.c_int
             self._fn[key] = fn
         return fn
 
     def _run(self, lib: str, name: str, argtypes, *args):
-        fn = self._get(lib, name, argtypes)
-        code = fn(*args, _stream_handle())
+        fn = self._fn.get((lib, name)) or self._get(lib, name, argtypes)
+        stream = _raw_stream(_raw_device()) if _raw_stream is not None and _raw_device is not None else _stream_handle()
+        code = fn(*args, stream)
         if code != 0:
-            msg = build.load_library(lib).lle_error_string(code).decode()
-            raise KernelError(f"{name} failed to launch: {msg} (hip error {code})")
+            self._failed(lib, name, code)
+        if _recording.to is not None:
+            _recording.to.launch(fn, lib, name, args, stream)
+
+    @staticmethod
+    def _failed(lib: str, name: str, code: int):
+        msg = build.load_library(lib).lle_error_string(code).decode()
+        raise KernelError(f"{name} failed to launch: {msg} (hip error {code})")
+
+    # -- the launches of a layer for the layers that are alike (record.py) ------------------
+    def may_record(self) -> bool:
+        """Whether what this object launches may be launched again for another layer: not where a caller has put a method of
+        its own in the place of one, which would not be called then."""
+        return type(self) is HipOps and not any(callable(v) for v in vars(self).values()) and _recording.to is None
+
+    def record(self) -> LaunchRecord:
+        """From here until end_record() this thread's launches are kept."""
+        _recording.to = LaunchRecord(_stream_handle())
+        return _recording.to
+
+    @staticmethod
+    def end_record() -> None:
+        _recording.to = None
+
+    def replay(self, replay, operands, addresses) -> None:
+        failed = replay.run(operands, addresses)
+        if failed is not None:
+            self._failed(*failed)
+
+    @staticmethod
+    def _library(take, x, weight, result):
+        record = _recording.to
+        if record is not None:
+            record.product(take, x, weight, result)
+        return result
+
+    @staticmethod
+    def _not_recorded() -> None:
+        record = _recording.to
+        if record is not None:
+            record.whole = False
 
     # -- embedding -----------------------------------------------------------
     def embedding(self, ids: torch.Tensor, table: torch.Tensor, feedback=None, token_seq=None,
@@ -127,8 +200,8 @@ class HipOps:
                 _need(t is not None, "feedback, token_seq and seq_slots come together")
                 _dev(t, name, torch.int32)
             _need(token_seq.shape == (N,), "token_seq must be [N]")
-        out = torch.empty((N, H), dtype=torch.float32, device=table.device)
-        self._run("elementwise", "lle_embedding_scaled", [_P, _P, _P, _I, _I, _I, _P, _P, _P, _F, _P],
+        out = _made((N, H), dtype=torch.float32, device=table.device)
+        self._run("elementwise", "lle_embedding_scaled", "PPPIIIPPPFP",
                   _ptr(ids), _ptr(table), _ptr(out), N, H, dtype_code(table.dtype), _ptr(feedback),
                   _ptr(token_seq) if feedback is not None else None, _ptr(seq_slots) if feedback is not None else None,
                   float(scale))
@@ -148,9 +221,9 @@ class HipOps:
                 _need(t is not None, "feedback, token_seq and seq_slots come together")
                 _dev(t, name, torch.int32)
             _need(token_seq.shape == (N,), "token_seq must be [N]")
-        hidden = torch.empty((N, H), dtype=torch.float32, device=table.device)
-        out = torch.empty((N, H), dtype=table.dtype, device=table.device)
-        self._run("norm", "lle_embedding_rmsnorm", [_P, _P, _P, _P, _I, _P, _I, _I, _F, _I, _P, _P, _P, _P],
+        hidden = _made((N, H), dtype=torch.float32, device=table.device)
+        out = _made((N, H), dtype=table.dtype, device=table.device)
+        self._run("norm", "lle_embedding_rmsnorm", "PPPPIPIIFIPPPP",
                   _ptr(ids), _ptr(table), _ptr(hidden), _ptr(weight), dtype_code(weight.dtype), _ptr(out), N, H,
                   float(eps), dtype_code(table.dtype), _ptr(feedback),
                   _ptr(token_seq) if feedback is not None else None, _ptr(seq_slots) if feedback is not None else None)
@@ -180,11 +253,11 @@ class HipOps:
                 _need(t is not None, "feedback, token_seq and seq_slots come together")
                 _dev(t, name, torch.int32)
             _need(token_seq.shape == (N,), "token_seq must be [N]")
-        hidden = torch.empty((N, H), dtype=torch.float32, device=table.device)
-        out = torch.empty((N, H), dtype=out_dtype, device=table.device) if next_weight is not None else None
+        hidden = _made((N, H), dtype=torch.float32, device=table.device)
+        out = _made((N, H), dtype=out_dtype, device=table.device) if next_weight is not None else None
         code = lambda t: F32 if t is None else dtype_code(t.dtype)
         self._run("norm", "lle_embedding_norm",
-                  [_P, _P, _I, _F, _P, _P, _P, _P, _I, _I, _P, _P, _I, _F, _P, _P, _I, _F, _P, _I, _I, _I, _P],
+                  "PPIFPPPPIIPPIFPPIFPIIIP",
                   _ptr(ids), _ptr(table), dtype_code(table.dtype), float(scale), _ptr(feedback),
                   _ptr(token_seq) if feedback is not None else None, _ptr(seq_slots) if feedback is not None else None,
                   _ptr(pos_table), code(pos_table), pos_table.shape[0] if pos_table is not None else 0,
@@ -217,13 +290,13 @@ class HipOps:
             R = rows.shape[0]
         else:
             R = N
-        out = torch.empty((R, H), dtype=out_dtype, device=hidden.device)
+        out = _made((R, H), dtype=out_dtype, device=hidden.device)
         if sums:
-            self._run("norm", "lle_add_rmsnorm_sums", [_P, _P, _I, _L, _P, _P, _I, _P, _I, _I, _F, _I, _P],
+            self._run("norm", "lle_add_rmsnorm_sums", "PPILPPIPIIFIP",
                       _ptr(hidden), _ptr(delta), delta.shape[0], delta.stride(0), _ptr(rows), _ptr(weight),
                       dtype_code(weight.dtype), _ptr(out), R, H, float(eps), dtype_code(out_dtype))
             return out
-        self._run("norm", "lle_add_rmsnorm", [_P, _P, _P, _P, _I, _P, _I, _I, _F, _I, _P],
+        self._run("norm", "lle_add_rmsnorm", "PPPPIPIIFIP",
                   _ptr(hidden), _ptr(delta), _ptr(rows), _ptr(weight), dtype_code(weight.dtype), _ptr(out),
                   R, H, float(eps), dtype_code(out_dtype))
         return out
@@ -237,12 +310,12 @@ class HipOps:
         _need(weight.shape == (H,), f"norm weight must be [{H}], is {list(weight.shape)}")
         if out_dtype is not None and out_dtype != x.dtype:
             _need(x.dtype == torch.float32 and out_dtype == torch.bfloat16, "a norm hands float32 rows on as they are or in bfloat16")
-            out = torch.empty((R, H), dtype=out_dtype, device=x.device)
-            self._run("norm", "lle_rmsnorm_f32_to_bf16", [_P, _P, _I, _P, _I, _I, _F, _P],
+            out = _made((R, H), dtype=out_dtype, device=x.device)
+            self._run("norm", "lle_rmsnorm_f32_to_bf16", "PPIPIIFP",
                       _ptr(x), _ptr(weight), dtype_code(weight.dtype), _ptr(out), R, H, float(eps))
             return out
-        out = torch.empty_like(x)
-        self._run("norm", "lle_rmsnorm", [_P, _P, _I, _P, _I, _I, _F, _I, _P],
+        out = _made_like(x)
+        self._run("norm", "lle_rmsnorm", "PPIPIIFIP",
                   _ptr(x), _ptr(weight), dtype_code(weight.dtype), _ptr(out), R, H, float(eps), dtype_code(x.dtype))
         return out
 
@@ -263,9 +336,7 @@ class HipOps:
     def norm_sum_parts(self, width: int) -> int:
         """Into how many column ranges the product before a folded norm over `width` splits the
         sums of squares (one per tile of its launch; the kernel library decides the tiles)."""
-        fn = getattr(build.load_library("gemm"), "lle_gemm_skinny_resid_parts")
-        fn.argtypes, fn.restype = [_I], _I
-        return int(fn(int(width)))
+        return self._get("gemm", "lle_gemm_skinny_resid_parts", "I")(int(width))
 
     def _linear_folded(self, x, weight, fold, gated: bool, out_dtype=torch.bfloat16):
         """The forms of the weight-streaming product around a folded norm: `x` a Prenormed
@@ -289,8 +360,8 @@ class HipOps:
             _need(not gated or N % 2 == 0, "a gated weight has an even number of rows")
             _need(out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and not gated),
                   "the product after a folded norm writes bfloat16, or float32 where it is not gated")
-            out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=xin.device)
-            self._run("gemm", "lle_gemm_skinny_scaled_bf16", [_P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _I, _P],
+            out = _made((M, N // 2 if gated else N), dtype=out_dtype, device=xin.device)
+            self._run("gemm", "lle_gemm_skinny_scaled_bf16", "PPPPIFIIIIIP",
                       _ptr(xin), _ptr(weight), _ptr(out), _ptr(pre.sums), parts, float(pre.eps), M, N, K, int(gated),
                       dtype_code(out_dtype))
             return out
@@ -299,9 +370,9 @@ class HipOps:
         _need(not gated and fold.hidden.shape == (M, N) and fold.weight.shape == (N,),
               f"residual stream {list(fold.hidden.shape)} does not fit a product [{M}, {N}]")
         _need(self.can_fold_norm(M, N, xin.dtype), f"a norm over {N} cannot be folded for {M} rows")
-        xw = torch.empty((M, N), dtype=torch.bfloat16, device=xin.device)
-        sums = torch.empty((16 if M <= 16 else 32, self.norm_sum_parts(N)), dtype=torch.float32, device=xin.device)
-        self._run("gemm", "lle_gemm_skinny_resid_bf16", [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P],
+        xw = _made((M, N), dtype=torch.bfloat16, device=xin.device)
+        sums = _made((16 if M <= 16 else 32, self.norm_sum_parts(N)), dtype=torch.float32, device=xin.device)
+        self._run("gemm", "lle_gemm_skinny_resid_bf16", "PPPPIPPIIIP",
                   _ptr(xin), _ptr(weight), _ptr(fold.hidden), _ptr(fold.weight), dtype_code(fold.weight.dtype),
                   _ptr(xw), _ptr(sums), M, N, K)
         return Prenormed(xw, sums, fold.eps)
@@ -324,8 +395,8 @@ class HipOps:
             _need(pre.sums.shape[0] == -(-M // 16) * 16, "sums of squares do not fit")
             _need(not gated or N % 2 == 0, "a gated weight has an even number of rows")
             in_one = gated and self._gated_f32_in_one(M, N, K)
-            out = torch.empty((M, N // 2 if in_one else N), dtype=torch.float32, device=xin.device)
-            self._run("gemm", "lle_gemm_skinny_scaled_f32", [_P, _P, _P, _P, _I, _F, _I, _I, _I, _I, _P], _ptr(xin), _ptr(weight),
+            out = _made((M, N // 2 if in_one else N), dtype=torch.float32, device=xin.device)
+            self._run("gemm", "lle_gemm_skinny_scaled_f32", "PPPPIFIIIIP", _ptr(xin), _ptr(weight),
                       _ptr(out), _ptr(pre.sums), parts, float(pre.eps), M, N, K, int(in_one))
             return self.silu_mul(out) if gated and not in_one else out
         _dev(fold.hidden, "hidden", torch.float32)
@@ -333,9 +404,9 @@ class HipOps:
         _need(not gated and fold.hidden.shape == (M, N) and fold.weight.shape == (N,),
               f"residual stream {list(fold.hidden.shape)} does not fit a product [{M}, {N}]")
         _need(self.can_fold_norm_f32(M, N), f"a norm over {N} cannot be folded for {M} rows")
-        xw = torch.empty((M, N), dtype=torch.float32, device=xin.device)
-        sums = torch.empty((-(-M // 16) * 16, self.norm_sum_parts(N)), dtype=torch.float32, device=xin.device)
-        self._run("gemm", "lle_gemm_skinny_resid_f32", [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P], _ptr(xin), _ptr(weight),
+        xw = _made((M, N), dtype=torch.float32, device=xin.device)
+        sums = _made((-(-M // 16) * 16, self.norm_sum_parts(N)), dtype=torch.float32, device=xin.device)
+        self._run("gemm", "lle_gemm_skinny_resid_f32", "PPPPIPPIIIP", _ptr(xin), _ptr(weight),
                   _ptr(fold.hidden), _ptr(fold.weight), dtype_code(fold.weight.dtype), _ptr(xw), _ptr(sums), M, N, K)
         return Prenormed(xw, sums, fold.eps)
 
@@ -369,9 +440,12 @@ class HipOps:
                     return PartialSums(self.linear_slices(x, weight, slices))
                 if form == "library":
                     # one batched library product over the slices of K, partial sums left in 32-bit
-                    xs = x.view(M, slices, K // slices).permute(1, 0, 2)
-                    ws = weight.view(N, slices, K // slices).permute(1, 2, 0)
-                    return PartialSums(torch.bmm(xs, ws, out_dtype=torch.float32))
+                    def take(x, weight, out=None):
+                        xs = x.view(M, slices, K // slices).permute(1, 0, 2)
+                        ws = weight.view(N, slices, K // slices).permute(1, 2, 0)
+                        return torch.bmm(xs, ws, out_dtype=torch.float32) if out is None else torch.bmm(xs, ws, out_dtype=torch.float32, out=out)
+
+                    return PartialSums(self._library(take, x, weight, take(x, weight)))
             t = self.tuning
             skinny = K % 8 == 0 and not self.force_library_gemm and (
                 M <= t.skinny_max_rows
@@ -380,15 +454,18 @@ class HipOps:
                 # tiles of X rows in its registers (K a multiple of 1024 up to 4096)
                 or (M <= 32 and K % 1024 == 0 and K <= 4096 and N >= t.stream_32_rows_min_share * self.compute_units()))
             if skinny:
-                out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-                self._run("gemm", "lle_gemm_skinny_bf16", [_P, _P, _P, _I, _I, _I, _I, _P],
+                out = _made((M, N), dtype=out_dtype, device=x.device)
+                self._run("gemm", "lle_gemm_skinny_bf16", "PPPIIIIP",
                           _ptr(x), _ptr(weight), _ptr(out), M, N, K, dtype_code(out_dtype))
                 return out
             tile = self.rows_tile(x, weight, gated=False) if 32 < M <= 128 and out_dtype == torch.bfloat16 else 0
             if tile:
                 return self.linear_rows(x, weight, tile)
             # the library product accumulates in 32-bit and can leave the result so
-            return torch.mm(x, weight.t()) if out_dtype == torch.bfloat16 else torch.mm(x, weight.t(), out_dtype=out_dtype)
+            if out_dtype == torch.bfloat16:
+                return self._library(_library_product, x, weight, torch.mm(x, weight.t()))
+            self._not_recorded()
+            return torch.mm(x, weight.t(), out_dtype=out_dtype)
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
         # (up to 16 columns are one step of one of the weight-streaming kernel's sixteen wavefronts: nothing to stream, and in
         # the tiles' kernel a row's result does not depend on how many rows there are)
@@ -396,17 +473,17 @@ class HipOps:
             slices = self._form_of_delta(x.dtype, M, N, K)[1] if sums_ok else 1
             if slices > 1:
                 return PartialSums(self.linear_f32_slices(x, weight, slices))
-            out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+            out = _made((M, N), dtype=out_dtype, device=x.device)
             # few rows: W streamed once, float32 matrix instruction
-            self._run("gemm", "lle_gemm_skinny_f32", [_P, _P, _P, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
+            self._run("gemm", "lle_gemm_skinny_f32", "PPPIIIP", _ptr(x), _ptr(weight), _ptr(out),
                       M, N, K)
             return out
         if K % 4 == 0 and not self.force_simt_gemm:
             slices = self._form_of_delta(x.dtype, M, N, K)[1] if sums_ok else 1
             out = self.linear_f32_tiles(x, weight, slices)
             return PartialSums(out) if slices > 1 else out[0]
-        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
+        out = _made((M, N), dtype=out_dtype, device=x.device)
+        self._run("gemm", "lle_gemm_nt_simt", "PPPIIILLLIIP",
                   _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, dtype_code(x.dtype), dtype_code(out_dtype))
         return out
 
@@ -432,7 +509,7 @@ class HipOps:
             self._forms[key] = form
         return form
 
-    _F32_TILES = [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P]
+    _F32_TILES = "PPPIIILLLIIP"
 
     def f32_slices_for(self, M: int, N: int, K: int) -> int:
         """In how many slices of K a float32 product is cut whose reader adds up partial sums, so that the CUs have work and no
@@ -457,8 +534,8 @@ class HipOps:
         M, K = x.shape
         N = weight.shape[0]
         _need(weight.shape[1] == K and K % 4 == 0 and M <= 64, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
-        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
-        self._run("gemm_f32", "lle_gemm_slices_f32", [_P, _P, _P, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out), M, N, K,
+        out = _made((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm_f32", "lle_gemm_slices_f32", "PPPIIIIP", _ptr(x), _ptr(weight), _ptr(out), M, N, K,
                   slices)
         return out
 
@@ -470,7 +547,7 @@ class HipOps:
         M, K = x.shape
         N = weight.shape[0]
         _need(weight.shape[1] == K and K % 4 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
-        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        out = _made((slices, M, N), dtype=torch.float32, device=x.device)
         self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, _ptr(x), _ptr(weight), _ptr(out), M, N, K, K, K, N, slices,
                   tiles)
         return out
@@ -504,8 +581,8 @@ class HipOps:
         if bias is not None:
             _dev(bias, "bias", torch.float32)
             _need(activation == "clamp" and bias.shape == (N,), "bias must cover the whole weight of a clamped product")
-        out = torch.empty((M, N // 2), dtype=torch.float32, device=x.device)
-        self._run("gemm_f32", "lle_gemm_nt_gated_f32", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
+        out = _made((M, N // 2), dtype=torch.float32, device=x.device)
+        self._run("gemm_f32", "lle_gemm_nt_gated_f32", "PPPFPIIIIIP", _ptr(x), _ptr(weight), _ptr(bias),
                   float(limit), _ptr(out), M, N, K, ("silu", "clamp").index(activation) + 1, tiles)
         return out
 
@@ -588,8 +665,8 @@ class HipOps:
         M, K = x.shape
         N = weight.shape[0]
         _need(weight.shape[1] == K and K % 64 == 0, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
-        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
-        self._run("gemm_tile", "lle_gemm_tile_sums_bf16", [_P, _P, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
+        out = _made((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm_tile", "lle_gemm_tile_sums_bf16", "PPPIIIIIP", _ptr(x), _ptr(weight), _ptr(out),
                   M, N, K, slices, tiles)
         return out
 
@@ -659,8 +736,8 @@ class HipOps:
         if bias is not None:
             _dev(bias, "bias", torch.bfloat16)
             _need(activation == "clamp" and bias.shape == (N,), "bias must cover the whole weight of a clamped product")
-        out = torch.empty((M, N // 2 if activation else N), dtype=torch.bfloat16, device=x.device)
-        self._run("gemm_rows", "lle_gemm_rows_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
+        out = _made((M, N // 2 if activation else N), dtype=torch.bfloat16, device=x.device)
+        self._run("gemm_rows", "lle_gemm_rows_bf16", "PPPFPIIIIIP", _ptr(x), _ptr(weight), _ptr(bias),
                   float(limit), _ptr(out), M, N, K, (None, "silu", "clamp").index(activation), tile)
         return out
 
@@ -676,8 +753,8 @@ class HipOps:
         if bias is not None:
             _dev(bias, "bias", torch.bfloat16)
             _need(bias.shape == (N,), "bias must cover the whole weight")
-        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-        self._run("gemm_wide", "lle_gemm_wide_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(bias),
+        out = _made((M, N // 2), dtype=torch.bfloat16, device=x.device)
+        self._run("gemm_wide", "lle_gemm_wide_bf16", "PPPFPIIIIIP", _ptr(x), _ptr(weight), _ptr(bias),
                   float(limit), _ptr(out), M, N, K, 1 + ("silu", "clamp").index(activation), form)
         return out
 
@@ -691,8 +768,8 @@ class HipOps:
         _need(weight.shape[1] == K, f"weight [{N}, {weight.shape[1]}] does not fit x [{M}, {K}]")
         _need(0 < M <= self.SLICED_MAX_ROWS and N % 64 == 0 and slices > 0 and K % (self.SLICED_UNIT * slices) == 0,
               f"no product in {slices} slices for [{M}, {K}] x [{N}, {K}]")
-        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
-        self._run("gemm", "lle_gemm_mid_slices_bf16", [_P, _P, _P, _I, _I, _I, _I, _P], _ptr(x), _ptr(weight), _ptr(out),
+        out = _made((slices, M, N), dtype=torch.float32, device=x.device)
+        self._run("gemm", "lle_gemm_mid_slices_bf16", "PPPIIIIP", _ptr(x), _ptr(weight), _ptr(out),
                   M, N, K, slices)
         return out
 
@@ -707,8 +784,8 @@ class HipOps:
         _dev(positions, "positions", torch.int32)
         _dev(inv_freq, "inv_freq", torch.float32)
         N, half = positions.shape[0], inv_freq.shape[0]
-        out = torch.empty((N, half, 2), dtype=torch.float32, device=positions.device)
-        self._run("rope_kv", "lle_rope_table", [_P, _P, _P, _I, _I, _P], _ptr(positions), _ptr(inv_freq), _ptr(out),
+        out = _made((N, half, 2), dtype=torch.float32, device=positions.device)
+        self._run("rope_kv", "lle_rope_table", "PPPIIP", _ptr(positions), _ptr(inv_freq), _ptr(out),
                   N, half)
         return out
 
@@ -739,9 +816,9 @@ class HipOps:
             _dev(cos_sin, "cos_sin", torch.float32)
             _need(cos_sin.shape == (N, rotary_dim // 2, 2), "cos_sin must be [N, rotary_dim / 2, 2]")
         page_size = kv_layer.shape[3]
-        q_out = torch.empty((N, nq, d), dtype=qkv.dtype, device=qkv.device)
+        q_out = _made((N, nq, d), dtype=qkv.dtype, device=qkv.device)
         self._run("rope_kv", "lle_qk_norm_rope_write",
-                  [_P, _P, _P, _P, _I, _P, _I, _F, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _P],
+                  "PPPPIPIFPPIIIIILIIP",
                   _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wd,
                   _ptr(cos_sin) if rotary_dim > 0 else None, rotary_dim, float(eps), _ptr(q_out), _ptr(kv_layer),
                   N, nq, nkv, d, page_size, kv_layer.stride(0), 1 if write_kv else 0, dtype_code(qkv.dtype))
@@ -776,7 +853,7 @@ class HipOps:
         if sinks is not None:
             _dev(sinks, "sinks", torch.float32)
             _need(sinks.shape == (nq,), "sinks must be [nq]")
-        out = torch.empty((N, nq * d), dtype=q.dtype, device=q.device)
+        out = _made((N, nq * d), dtype=q.dtype, device=q.device)
         win = int(window) if window else 0
         keep = int(keep_first) if win else 0
         _need(keep >= 0, "keep_first must not be negative")
@@ -796,18 +873,17 @@ class HipOps:
             ns = self.f32_attention_splits(S, nkv, row_blocks, max_q_len, max_kv_len, win, rounds)
             ws_o = ws_ml = None
             if ns > 1:
-                ws_o = torch.empty((N * nq * ns * d,), dtype=torch.float32, device=q.device)
-                ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=q.device)
+                ws_o = _made((N * nq * ns * d,), dtype=torch.float32, device=q.device)
+                ws_ml = _made((N * nq * ns * 2,), dtype=torch.float32, device=q.device)
             self._run("attention", "lle_paged_attention_mfma_f32",
-                      [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I, _I, _F, _I, _I, _I, _I, _P, _F,
-                       _P],
+                      "PPPPPPPPPIIIIIILIIIFIIIIPFP",
                       _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens),
                       _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size, kv_layer.stride(0),
                       block_table.shape[1], win, keep, float(scale), row_blocks, tiles, paired, ns, _ptr(sinks), cap)
             return out
         if not mfma:
             self._run("attention", "lle_paged_attention_generic",
-                      [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _I, _F, _I, _P, _F, _P],
+                      "PPPPPPPPIIIIILIIIFIPFP",
                       _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens),
                       _ptr(token_seq), _ptr(out), N, nq, nkv, d, page_size, kv_layer.stride(0), block_table.shape[1],
                       win, keep, float(scale), dtype_code(q.dtype), _ptr(sinks), cap)
@@ -822,11 +898,10 @@ class HipOps:
         ns = max(ns_decode, ns_prefill)
         ws_o = ws_ml = None
         if ns > 1:
-            ws_o = torch.empty((N * nq * ns * d,), dtype=torch.float32, device=q.device)
-            ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=q.device)
+            ws_o = _made((N * nq * ns * d,), dtype=torch.float32, device=q.device)
+            ws_ml = _made((N * nq * ns * 2,), dtype=torch.float32, device=q.device)
         self._run("attention", "lle_paged_attention_mfma",
-                  [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I, _F, _I, _I, _I, _I, _I, _I,
-                   _P, _I, _F, _P],
+                  "PPPPPPPPPPIIIIIILIIFIIIIIIPIFP",
                   _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens),
                   _ptr(token_seq), _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size,
                   kv_layer.stride(0), block_table.shape[1], win, float(scale), int(run_decode), ns_decode,
@@ -901,22 +976,21 @@ class HipOps:
         win = int(window) if window else 0
         if f32:
             _need(token_seq is None and order is None and d in (64, 128), "in float32 every request has one token and heads are of 64 or 128")
-            out = torch.empty((N, nq * d), dtype=torch.float32, device=qkv.device)
+            out = _made((N, nq * d), dtype=torch.float32, device=qkv.device)
             self._run("attention", "lle_qk_norm_rope_attention_decode_f32",
-                      [_P, _P, _P, _P, _I, _P, _F, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _I, _P],
+                      "PPPPIPFIPPPPPPIIIIILIIFIP",
                       _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wcode, _ptr(cos_sin), float(eps), int(bool(write_kv)),
                       _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens), _ptr(out), S, nq, nkv, d,
                       page_size, kv_layer.stride(0), block_table.shape[1], win, float(scale), int(max_kv_len))
             return out
         ns = self.decode_splits(S, nkv, max_kv_len, win)
-        out = torch.empty((N, nq * d), dtype=torch.bfloat16, device=qkv.device)
+        out = _made((N, nq * d), dtype=torch.bfloat16, device=qkv.device)
         ws_o = ws_ml = None
         if ns > 1:
-            ws_o = torch.empty((N * nq * ns * d,), dtype=torch.float32, device=qkv.device)
-            ws_ml = torch.empty((N * nq * ns * 2,), dtype=torch.float32, device=qkv.device)
+            ws_o = _made((N * nq * ns * d,), dtype=torch.float32, device=qkv.device)
+            ws_ml = _made((N * nq * ns * 2,), dtype=torch.float32, device=qkv.device)
         self._run("attention", "lle_qk_norm_rope_attention_decode",
-                  [_P, _P, _P, _P, _I, _P, _F, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _I, _I,
-                   _F, _I, _P, _I, _P],
+                  "PPPPIPFIPPPPPPPPPIIIIIILIIFIPIP",
                   _ptr(qkv), _ptr(slots), _ptr(q_weight), _ptr(k_weight), wcode, _ptr(cos_sin), float(eps),
                   int(bool(write_kv)), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens),
                   _ptr(kv_lens), _ptr(token_seq), _ptr(out), _ptr(ws_o), _ptr(ws_ml), N, S, nq, nkv, d, page_size,
@@ -957,9 +1031,9 @@ class HipOps:
             _dev(cos_sin, "cos_sin", torch.float32)
             rot = 2 * cos_sin.shape[1]
             _need(cos_sin.shape == (S, rot // 2, 2) and rot <= d, "cos_sin must be [S, pairs, 2]")
-        out = torch.empty((S, nq * d), dtype=torch.bfloat16, device=u.device)
+        out = _made((S, nq * d), dtype=torch.bfloat16, device=u.device)
         self._run("attention", "lle_pair_rope_attention_decode",
-                  [_P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _F, _I, _P],
+                  "PIPPIIPPPPPPIIIIILIIFFIP",
                   _ptr(u), cols, _ptr(slots), _ptr(cos_sin), rot, int(bool(write_kv)), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots),
                   _ptr(cu_tokens), _ptr(kv_lens), _ptr(out), S, nq, nkv, d, page_size, kv_layer.stride(0), block_table.shape[1],
                   int(window) if window else 0, float(scale), float(softcap) if softcap else 0.0, int(max_kv_len))
@@ -979,8 +1053,8 @@ class HipOps:
         S = kv_lens.shape[0]
         if S > 1024 or S * num_kv_heads <= self.compute_units():
             return None
-        order = torch.empty((S,), dtype=torch.int32, device=kv_lens.device)
-        self._run("attention", "lle_decode_order", [_P, _P, _I, _P], _ptr(kv_lens), _ptr(order), S)
+        order = _made((S,), dtype=torch.int32, device=kv_lens.device)
+        self._run("attention", "lle_decode_order", "PPIP", _ptr(kv_lens), _ptr(order), S)
         return order
 
     force_generic_attention = False  # tests flip this to compare the two families of kernels
@@ -1118,7 +1192,7 @@ class HipOps:
         _dev(x, "x")
         _dev(bias, "bias")
         _need(x.dim() == 2 and bias.shape == (x.shape[1],), f"bias {list(bias.shape)} does not fit x {list(x.shape)}")
-        self._run("elementwise", "lle_add_bias", [_P, _P, _I, _I, _I, _I, _P], _ptr(x), _ptr(bias), x.shape[0],
+        self._run("elementwise", "lle_add_bias", "PPIIIIP", _ptr(x), _ptr(bias), x.shape[0],
                   x.shape[1], dtype_code(x.dtype), dtype_code(bias.dtype))
         return x
 
@@ -1128,8 +1202,8 @@ class HipOps:
         _dev(gate_up, "gate_up")
         N, two_i = gate_up.shape
         _need(two_i % 2 == 0, "gate_up must have an even width")
-        out = torch.empty((N, two_i // 2), dtype=gate_up.dtype, device=gate_up.device)
-        self._run("elementwise", "lle_silu_mul", [_P, _P, _I, _I, _I, _P],
+        out = _made((N, two_i // 2), dtype=gate_up.dtype, device=gate_up.device)
+        self._run("elementwise", "lle_silu_mul", "PPIIIP",
                   _ptr(gate_up), _ptr(out), N, two_i // 2, dtype_code(gate_up.dtype))
         return out
 
@@ -1147,13 +1221,13 @@ class HipOps:
         _need(weight.shape[1] == K and N2 % 2 == 0, f"weight {list(weight.shape)} does not fit x [{M}, {K}]")
         few = M <= self.tuning.skinny_max_rows or (M <= 32 and N2 * K <= self.tuning.skinny_small_weight)
         if x.dtype == torch.bfloat16 and few and K % 8 == 0 and not self.force_library_gemm:
-            out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
-            self._run("gemm", "lle_gemm_skinny_gated_bf16", [_P, _P, _P, _I, _I, _I, _P],
+            out = _made((M, N2 // 2), dtype=x.dtype, device=x.device)
+            self._run("gemm", "lle_gemm_skinny_gated_bf16", "PPPIIIP",
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
         if x.dtype == torch.float32 and K % 4 == 0 and self._gated_f32_in_one(M, N2, K) and not self.force_library_gemm:
-            out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
-            self._run("gemm", "lle_gemm_skinny_gated_f32", [_P, _P, _P, _I, _I, _I, _P],
+            out = _made((M, N2 // 2), dtype=x.dtype, device=x.device)
+            self._run("gemm", "lle_gemm_skinny_gated_f32", "PPPIIIP",
                       _ptr(x), _ptr(weight), _ptr(out), M, N2, K)
             return out
         tile = self.rows_tile(x, weight, gated=True) if 32 < M <= 256 and x.dtype == torch.bfloat16 else 0
@@ -1200,8 +1274,8 @@ class HipOps:
         few = M <= self.tuning.skinny_max_rows or (M <= 32 and N2 * K <= self.tuning.skinny_small_weight)
         if x.dtype == torch.bfloat16 and few and K % 8 == 0 and not self.force_library_gemm:
             _need(limit > 0.0, "a clamped activation has a positive limit")
-            out = torch.empty((M, N2 // 2), dtype=x.dtype, device=x.device)
-            self._run("gemm", "lle_gemm_skinny_clamped_bf16", [_P, _P, _P, _F, _P, _I, _I, _I, _P],
+            out = _made((M, N2 // 2), dtype=x.dtype, device=x.device)
+            self._run("gemm", "lle_gemm_skinny_clamped_bf16", "PPPFPIIIP",
                       _ptr(x), _ptr(weight), _ptr(bias), float(limit), _ptr(out), M, N2, K)
             return out
         aligned = bias is None or bias.data_ptr() % 8 == 0
@@ -1222,15 +1296,15 @@ class HipOps:
         if x.dtype == dtype:
             return x
         _dev(x, "x")
-        out = torch.empty(x.shape, dtype=dtype, device=x.device)
-        self._run("elementwise", "lle_cast", [_P, _P, _L, _I, _I, _P], _ptr(x), _ptr(out), x.numel(),
+        out = _made(x.shape, dtype=dtype, device=x.device)
+        self._run("elementwise", "lle_cast", "PPLIIP", _ptr(x), _ptr(out), x.numel(),
                   dtype_code(x.dtype), dtype_code(dtype))
         return out
 
     def scale_(self, x, factor: float) -> torch.Tensor:
         """float32 x *= factor, in place."""
         _dev(x, "x", torch.float32)
-        self._run("elementwise", "lle_scale", [_P, _L, _F, _P], _ptr(x), x.numel(), float(factor))
+        self._run("elementwise", "lle_scale", "PLFP", _ptr(x), x.numel(), float(factor))
         return x
 
     def rmsnorm_add(self, hidden, y, weight, eps: float, out_dtype, extra=None) -> torch.Tensor:
@@ -1244,8 +1318,8 @@ class HipOps:
             if t is not None:
                 _dev(t, name)
                 _need(t.shape == hidden.shape, f"{name} must have the shape of hidden")
-        out = None if out_dtype == torch.float32 else torch.empty((N, H), dtype=out_dtype, device=hidden.device)
-        self._run("norm", "lle_rmsnorm_add", [_P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _F, _I, _P],
+        out = None if out_dtype == torch.float32 else _made((N, H), dtype=out_dtype, device=hidden.device)
+        self._run("norm", "lle_rmsnorm_add", "PPIPIPIPIIFIP",
                   _ptr(hidden), _ptr(y), dtype_code(y.dtype), _ptr(extra), dtype_code(extra.dtype) if extra is not None else 0,
                   _ptr(weight), dtype_code(weight.dtype), _ptr(out), N, H, float(eps), dtype_code(out_dtype))
         return hidden if out is None else out
@@ -1269,10 +1343,10 @@ class HipOps:
         _need(zxg.shape == (N, 3 * W) and x_bias.shape == (W,), "zxg must be [N, 3 W] and the biases [W]")
         _need(state.dim() == 2 and state.shape[1] == W, "state must be [slots, W]")
         _need(cu_tokens.shape == (S + 1,), "cu_tokens must be [S + 1]")
-        out = torch.empty((N, W), dtype=out_dtype, device=zxg.device)
+        out = _made((N, W), dtype=out_dtype, device=zxg.device)
         pieces = max(1, min(1024, -(-max(1, max_q_len) // self.MINGRU_PIECE)))
-        part = torch.empty((S * pieces * 3 * W,), dtype=torch.float32, device=zxg.device) if pieces > 1 else None
-        self._run("recurrent", "lle_mingru_scan", [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P],
+        part = _made((S * pieces * 3 * W,), dtype=torch.float32, device=zxg.device) if pieces > 1 else None
+        self._run("recurrent", "lle_mingru_scan", "PIPPPPPPIPIIIP",
                   _ptr(zxg), dtype_code(zxg.dtype), _ptr(z_bias), _ptr(x_bias), _ptr(state), _ptr(seq_slots),
                   _ptr(cu_tokens), _ptr(out), dtype_code(out_dtype), _ptr(part), S, W, pieces)
         return out
@@ -1294,7 +1368,7 @@ class HipOps:
         if rot_dims:
             _dev(cos_sin, "cos_sin", torch.float32)
             _need(cos_sin.shape == (N, rot_dims // 2, 2), "cos_sin must be [N, rot_dims / 2, 2]")
-        self._run("latent", "lle_latent_kv_write", [_P, _P, _I, _F, _P, _I, _P, _P, _L, _I, _I, _I, _I, _I, _P],
+        self._run("latent", "lle_latent_kv_write", "PPIFPIPPLIIIIIP",
                   _ptr(dkv), _ptr(norm_w), dtype_code(norm_w.dtype), float(eps), _ptr(cos_sin) if rot_dims else None,
                   int(rot_dims), _ptr(slots), _ptr(pages), pages.stride(0), int(page_size), N, rank, rot,
                   dtype_code(dkv.dtype))
@@ -1307,8 +1381,8 @@ class HipOps:
         if rot_dims:
             _dev(cos_sin, "cos_sin", torch.float32)
             _need(cos_sin.shape == (N, rot_dims // 2, 2), "cos_sin must be [N, rot_dims / 2, 2]")
-        out = torch.empty((N, heads, rot), dtype=torch.float32, device=q.device)
-        self._run("latent", "lle_latent_q_rope", [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P],
+        out = _made((N, heads, rot), dtype=torch.float32, device=q.device)
+        self._run("latent", "lle_latent_q_rope", "PPIPIIIIIP",
                   _ptr(q), _ptr(cos_sin) if rot_dims else None, int(rot_dims), _ptr(out), N, heads, dim, rot,
                   dtype_code(q.dtype))
         return out
@@ -1326,10 +1400,11 @@ class HipOps:
         if x.dtype == torch.bfloat16:
             a = x3[:, :, col0 : col0 + K].transpose(0, 1)  # [heads, N, K]
             b = weight.transpose(1, 2)  # [heads, K, out]
+            self._not_recorded()
             y = torch.bmm(a, b) if out_dtype == torch.bfloat16 else torch.bmm(a, b, out_dtype=out_dtype)
             return y.transpose(0, 1)  # [N, heads, out], strided
         _need(out_dtype == torch.float32, "a float32 product has a float32 result")
-        out = torch.empty((N, heads, O), dtype=torch.float32, device=x.device)
+        out = _made((N, heads, O), dtype=torch.float32, device=x.device)
         quick = K % 4 == 0 and xw % 4 == 0 and col0 % 4 == 0 and not self.force_simt_gemm
         for h in range(heads):
             a_ptr = x.data_ptr() + 4 * (h * xw + col0)
@@ -1339,7 +1414,7 @@ class HipOps:
                 self._run("gemm_f32", "lle_gemm_nt_f32", self._F32_TILES, a_ptr, b_ptr, c_ptr, N, O, K, heads * xw, K,
                           heads * O, 1, -1)
             else:
-                self._run("gemm", "lle_gemm_nt_simt", [_P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _I, _P],
+                self._run("gemm", "lle_gemm_nt_simt", "PPPIIILLLIIP",
                           a_ptr, b_ptr, c_ptr, N, O, K, heads * xw, K, heads * O, F32, F32)
         return out
 
@@ -1395,7 +1470,7 @@ class HipOps:
         _need(token_seq.shape == (N,) and cu_tokens.shape == (S + 1,) and kv_lens.shape == (S,), "the step's arrays")
         _need(block_table.dim() == 2, "block_table must be [slots, pages]")
         _need(rank <= 1024, f"a latent of {rank} elements is wider than the attention kernels take (1024)")
-        out = torch.empty((N, H, rank), dtype=out_dtype, device=pages.device)
+        out = _made((N, H, rank), dtype=out_dtype, device=pages.device)
         win = int(window) if window else 0
         if (q_lat.dtype == torch.bfloat16 and self.latent_query_dtype(pages.dtype, page_size, rank, rot) == torch.bfloat16
                 and q_lat.stride(0) % 8 == 0 and q_lat.stride(1) % 8 == 0 and pages.stride(0) % 8 == 0
@@ -1405,11 +1480,10 @@ class HipOps:
             self.last_latent_kernel = ("matrix cores", ns)
             ws_o = ws_ml = None
             if ns > 1:
-                ws_o = torch.empty((N * H * ns * rank,), dtype=torch.float32, device=pages.device)
-                ws_ml = torch.empty((N * H * ns * 2,), dtype=torch.float32, device=pages.device)
+                ws_o = _made((N * H * ns * rank,), dtype=torch.float32, device=pages.device)
+                ws_ml = _made((N * H * ns * 2,), dtype=torch.float32, device=pages.device)
             self._run("latent", "lle_latent_attention_mfma",
-                      [_P, _L, _L, _P, _P, _L, _I, _I, _I, _P, _I, _P, _P, _P, _P, _I, _F, _P, _P, _P, _I, _I, _I, _I, _I, _I,
-                       _P],
+                      "PLLPPLIIIPIPPPPIFPPPIIIIIIP",
                       _ptr(q_lat), q_lat.stride(0), q_lat.stride(1), _ptr(q_rot), _ptr(pages), pages.stride(0),
                       int(page_size), rank, rot, _ptr(block_table), block_table.shape[1], _ptr(seq_slots),
                       _ptr(cu_tokens), _ptr(kv_lens), _ptr(sink), win, float(scale), _ptr(out), _ptr(ws_o), _ptr(ws_ml),
@@ -1417,7 +1491,7 @@ class HipOps:
             return out
         self.last_latent_kernel = ("generic", 1)
         self._run("latent", "lle_latent_attention_generic",
-                  [_P, _I, _L, _L, _P, _P, _L, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _I, _F, _P, _I, _I, _I, _P],
+                  "PILLPPLIIIPIPPPPPIFPIIIP",
                   _ptr(q_lat), dtype_code(q_lat.dtype), q_lat.stride(0), q_lat.stride(1), _ptr(q_rot), _ptr(pages),
                   pages.stride(0), int(page_size), rank, rot, _ptr(block_table), block_table.shape[1], _ptr(seq_slots),
                   _ptr(cu_tokens), _ptr(kv_lens), _ptr(token_seq), _ptr(sink), int(window) if window else 0,
@@ -1438,9 +1512,9 @@ class HipOps:
         if bias is not None:
             _dev(bias, "router bias", torch.float32)
             _need(bias.shape == (E,), "the router's bias must be [E]")
-        ids = torch.empty((N, top), dtype=torch.int32, device=logits.device)
-        gains = torch.empty((N, top), dtype=torch.float32, device=logits.device)
-        self._run("moe", "lle_moe_route", [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P], _ptr(logits), _ptr(bias), _ptr(ids),
+        ids = _made((N, top), dtype=torch.int32, device=logits.device)
+        gains = _made((N, top), dtype=torch.float32, device=logits.device)
+        self._run("moe", "lle_moe_route", "PPPPIIIIIP", _ptr(logits), _ptr(bias), _ptr(ids),
                   _ptr(gains), N, E, top, cols, 1 if score == "sigmoid" else 0)
         return ids, gains
 
@@ -1461,9 +1535,9 @@ class HipOps:
         _need(groups > 0 and E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups),
               "the experts form equal groups, and the kept groups hold at least `top` experts")
         _need(2 * E + groups <= 4096, "the router's kernel keeps its scores in LDS: at most about 2000 experts")
-        ids = torch.empty((N, top), dtype=torch.int32, device=logits.device)
-        gains = torch.empty((N, top), dtype=torch.float32, device=logits.device)
-        self._run("moe", "lle_moe_route_grouped", [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P], _ptr(logits),
+        ids = _made((N, top), dtype=torch.int32, device=logits.device)
+        gains = _made((N, top), dtype=torch.float32, device=logits.device)
+        self._run("moe", "lle_moe_route_grouped", "PPPPIIIIIIIP", _ptr(logits),
                   _ptr(correction), _ptr(ids), _ptr(gains), N, E, top, int(groups), int(keep),
                   1 if score == "sigmoid" else 0, int(group_top))
         return ids, gains
@@ -1498,20 +1572,20 @@ class HipOps:
         F = F2 if plain else F2 // 2
         _need(ids.shape == (N, top) and gains.shape == (N, top), "ids and gains must be [N, top]")
         _need(gate_up.shape == (E, F2, K) and (plain or F2 % 2 == 0) and down.shape == (E, H, F), "expert weights do not fit")
-        act = torch.empty((N * top, F), dtype=x.dtype, device=x.device)
-        out = torch.empty((N, H), dtype=torch.float32, device=x.device)
+        act = _made((N * top, F), dtype=x.dtype, device=x.device)
+        out = _made((N, H), dtype=torch.float32, device=x.device)
         code, on_input = self.EXPERT_FORMS[form], (1 if gain_on_input else 0)
         if (x.dtype == torch.bfloat16 and N * top >= self.MOE_TILED_MIN_PAIRS and E <= 256 and K % 8 == 0 and F % 8 == 0
                 and H % 4 == 0):
-            plan = torch.empty((4 * E + 1,), dtype=torch.int32, device=x.device)
-            order = torch.empty((2, N * top), dtype=torch.int32, device=x.device)
-            y = torch.empty((N * top, H), dtype=torch.float32, device=x.device)
+            plan = _made((4 * E + 1,), dtype=torch.int32, device=x.device)
+            order = _made((2, N * top), dtype=torch.int32, device=x.device)
+            y = _made((N * top, H), dtype=torch.float32, device=x.device)
             self._run("moe", "lle_moe_experts_tiled",
-                      [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+                      "PPPPPPPPPPPIIIIIIIIFP",
                       _ptr(x), _ptr(ids), _ptr(gains), _ptr(gate_up), _ptr(down), _ptr(plan), order[0].data_ptr(),
                       order[1].data_ptr(), _ptr(act), _ptr(y), _ptr(out), N, top, E, F, K, H, code, on_input, float(limit))
             return out
-        self._run("moe", "lle_moe_experts", [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+        self._run("moe", "lle_moe_experts", "PPPPPPPIIIIIIIIIFP",
                   _ptr(x), _ptr(ids), _ptr(gains), _ptr(gate_up), _ptr(down), _ptr(act), _ptr(out), N, top, E, F,
                   K, H, dtype_code(x.dtype), code, on_input, float(limit))
         return out
@@ -1553,9 +1627,9 @@ class HipOps:
         if rotary_dim > 0:
             _dev(cos_sin, "cos_sin", torch.float32)
             _need(cos_sin.shape == (N, rotary_dim // 2, 2), "cos_sin must be [N, rotary_dim / 2, 2]")
-        q_out = torch.empty((N, nq, D), dtype=qkv.dtype, device=qkv.device)
+        q_out = _made((N, nq, D), dtype=qkv.dtype, device=qkv.device)
         self._run("rope_kv", "lle_proj_norm_rope_write",
-                  [_P, _I, _P, _P, _P, _P, _I, _P, _I, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I, _L, _I, _I, _I, _I, _P],
+                  "PIPPPPIPIFPPIIIIIIILIIIIP",
                   _ptr(qkv), cols, _ptr(bias), _ptr(slots), _ptr(q_weight), _ptr(k_weight) if has_kv else None,
                   dtype_code(q_weight.dtype) if q_weight is not None else F32, _ptr(cos_sin) if rotary_dim > 0 else None,
                   rotary_dim, float(eps), _ptr(q_out), _ptr(kv_layer), N, nq, nkv, dim, vdim, D, page_size,
@@ -1571,15 +1645,15 @@ class HipOps:
         N = a.shape[0]
         _need(a.dim() == 2 and a.shape[1] % heads == 0 and a.shape[1] // heads >= vdim, "a must be [N, heads * D], D >= vdim")
         _need(gates.dim() == 2 and gates.shape[0] == N and 0 <= col0 and col0 + heads <= gates.shape[1], "gates [N, >= col0 + heads]")
-        out = torch.empty((N, heads * vdim), dtype=a.dtype, device=a.device)
-        self._run("elementwise", "lle_head_gate", [_P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _P], _ptr(a), _ptr(gates),
+        out = _made((N, heads * vdim), dtype=a.dtype, device=a.device)
+        self._run("elementwise", "lle_head_gate", "PPIIPIIIIIP", _ptr(a), _ptr(gates),
                   gates.shape[1], int(col0), _ptr(out), N, heads, a.shape[1] // heads, vdim, dtype_code(a.dtype))
         return out
 
     def tanh_(self, x) -> torch.Tensor:
         """x = tanh(x), in place."""
         _dev(x, "x")
-        self._run("elementwise", "lle_tanh", [_P, _L, _I, _P], _ptr(x), x.numel(), dtype_code(x.dtype))
+        self._run("elementwise", "lle_tanh", "PLIP", _ptr(x), x.numel(), dtype_code(x.dtype))
         return x
 
     def scaled_add_rmsnorm(self, hidden, a, b, mult: float, weight, eps: float, out_dtype, rows=None,
@@ -1599,8 +1673,8 @@ class HipOps:
         if rows is not None:
             _dev(rows, "rows", torch.int32)
             R = rows.shape[0]
-        out = torch.empty((R, H), dtype=out_dtype, device=hidden.device)
-        self._run("norm", "lle_scaled_add_rmsnorm", [_P, _P, _I, _P, _I, _F, _F, _P, _P, _I, _P, _I, _I, _F, _I, _P],
+        out = _made((R, H), dtype=out_dtype, device=hidden.device)
+        self._run("norm", "lle_scaled_add_rmsnorm", "PPIPIFFPPIPIIFIP",
                   _ptr(hidden), _ptr(a), dtype_code(a.dtype), _ptr(b), dtype_code(b.dtype) if b is not None else 0,
                   float(mult), float(mult if mult_b is None else mult_b), _ptr(rows), _ptr(weight), dtype_code(weight.dtype), _ptr(out), R, H, float(eps),
                   dtype_code(out_dtype))
@@ -1619,8 +1693,8 @@ class HipOps:
         N, W = x.shape
         M = mu.shape[0]
         _need(mu.shape == (M, W) and state.dim() == 2 and prev_offset + W <= state.shape[1], "mu [M, W]; the state row holds W saved elements")
-        out = torch.empty((M, N, W), dtype=x.dtype, device=x.device)
-        self._run("wkv", "lle_shift_mix", [_P, _P, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P], _ptr(x), _ptr(state),
+        out = _made((M, N, W), dtype=x.dtype, device=x.device)
+        self._run("wkv", "lle_shift_mix", "PPLIPPPPPIIIIP", _ptr(x), _ptr(state),
                   state.stride(0), int(prev_offset), _ptr(mu), _ptr(token_seq), _ptr(cu_tokens), _ptr(seq_slots), _ptr(out),
                   N, W, M, dtype_code(x.dtype))
         return out
@@ -1653,16 +1727,16 @@ class HipOps:
         _need(w0.shape == (HD,) and u.shape == (HD,) and norm_w.shape == (HD,), "w0, u and the norm weight must be [heads * dim]")
         _need(state.dim() == 2 and state.shape[1] >= HD * dim + W, "a state row holds heads * dim * dim + W floats")
         _need(cu_tokens.shape == (S + 1,), "cu_tokens must be [S + 1]")
-        out = torch.empty((N, HD), dtype=out_dtype, device=x.device)
+        out = _made((N, HD), dtype=out_dtype, device=x.device)
         piece = self.WKV_PIECE
         pieces = -(-max_q_len // piece) if max_q_len > 2 * piece else 1
         part = None
         if pieces > 1:
-            part = torch.empty((S * pieces * heads * (dim * dim + dim),), dtype=torch.float32, device=x.device)
+            part = _made((S * pieces * heads * (dim * dim + dim),), dtype=torch.float32, device=x.device)
         else:
             piece = 1 << 30
         self._run("wkv", "lle_wkv_scan",
-                  [_P, _P, _P, _P, _P, _P, _P, _P, _I, _F, _P, _P, _L, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P],
+                  "PPPPPPPPIFPPLIPPPIIIIIIPIP",
                   _ptr(r), _ptr(k), _ptr(v), _ptr(wraw), _ptr(w0), _ptr(u), _ptr(g), _ptr(norm_w),
                   dtype_code(norm_w.dtype), float(eps), _ptr(x), _ptr(state), state.stride(0), HD * dim, _ptr(seq_slots),
                   _ptr(cu_tokens), _ptr(out), S, heads, dim, W, pieces, piece, _ptr(part), dtype_code(out_dtype))
@@ -1716,10 +1790,10 @@ class HipOps:
         if rows is not None:
             _dev(rows, "rows", torch.int32)
             R = rows.shape[0]
-        out = torch.empty((R, H), dtype=out_dtype, device=hidden.device)
+        out = _made((R, H), dtype=out_dtype, device=hidden.device)
         code = lambda t: 0 if t is None else dtype_code(t.dtype)
         self._run("norm", "lle_inject_rmsnorm",
-                  [_P, _P, _I, _I, _L, _P, _I, _P, _P, _P, _I, _F, _P, _P, _P, _P, _P, _I, _P, _I, _I, _F, _I, _P],
+                  "PPIILPIPPPIFPPPPPIPIIFIP",
                   _ptr(hidden), _ptr(a), code(a), slices, stride, _ptr(b), code(b), _ptr(vector), _ptr(ids), _ptr(table),
                   code(table), scale, _ptr(feedback), _ptr(token_seq) if feedback is not None else None,
                   _ptr(seq_slots) if feedback is not None else None, _ptr(rows), _ptr(weight), dtype_code(weight.dtype),
@@ -1756,9 +1830,9 @@ class HipOps:
         if cos_sin is not None:
             rot = 2 * cos_sin.shape[1]
         _need(v_cos_sin is None or 2 * v_cos_sin.shape[1] == vdim, "v_cos_sin must cover the whole value")
-        q_out = torch.empty((N, nq, D), dtype=u.dtype, device=u.device)
+        q_out = _made((N, nq, D), dtype=u.dtype, device=u.device)
         self._run("rope_kv", "lle_pair_rope_write",
-                  [_P, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _L, _I, _I, _P],
+                  "PIPPPIPPPIIIIIIILIIP",
                   _ptr(u), cols, _ptr(bias), _ptr(slots), _ptr(cos_sin), rot, _ptr(v_cos_sin), _ptr(q_out), _ptr(kv_layer), N,
                   nq, nkv, dim, vdim, D, page_size, kv_layer.stride(0), 1 if write_kv else 0, dtype_code(u.dtype))
         return q_out
@@ -1775,8 +1849,8 @@ class HipOps:
         if v_cos_sin is not None:
             _dev(v_cos_sin, "v_cos_sin", torch.float32)
             _need(v_cos_sin.shape == (N, vdim // 2, 2) and vdim % 2 == 0, "v_cos_sin must cover the whole value")
-        out = torch.empty((N, heads * vdim), dtype=a.dtype, device=a.device)
-        self._run("rope_kv", "lle_turn_back_gate", [_P, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F, _I, _P], _ptr(a), _ptr(u),
+        out = _made((N, heads * vdim), dtype=a.dtype, device=a.device)
+        self._run("rope_kv", "lle_turn_back_gate", "PPIIPPIIIIFIP", _ptr(a), _ptr(u),
                   u.shape[1], int(gate_col), _ptr(v_cos_sin), _ptr(out), N, heads, a.shape[1] // heads, vdim, float(out_scale),
                   dtype_code(a.dtype))
         return out
@@ -1808,7 +1882,7 @@ class HipOps:
         if slopes is not None:
             _dev(slopes, "slopes", torch.float32)
             _need(slopes.shape == (H,), "slopes must be [H]")
-        out = torch.empty((N, H * D), dtype=q.dtype, device=q.device)
+        out = _made((N, H * D), dtype=q.dtype, device=q.device)
         run_decode, run_prefill = min_q_len <= 1, max_q_len > 1
         if (q.dtype == torch.bfloat16 and D % 32 == 0 and D <= 128 and P % 16 == 0 and max_q_len > 0 and max_kv_len > 0
                 and S <= 65535 and (H <= 32 if run_prefill else H <= 128) and not self.force_generic_attention):
@@ -1819,21 +1893,20 @@ class HipOps:
                 K = -(-(seen + 15) // 16) * 16
                 # a wavefront should have a tile of 16 keys or two, and the workgroups fill the CUs once or twice
                 splits = int(max(1, min(-(-K // 64), 2 * self.compute_units() // max(1, S * G))))
-                ws_s = torch.empty((S * H * K,), dtype=torch.float32, device=q.device)
-                ws_ml = torch.empty((S * H * (K // 16) * 2,), dtype=torch.float32, device=q.device)
-            ws_sums = torch.empty((N * H,), dtype=torch.float32, device=q.device) if run_prefill else None
+                ws_s = _made((S * H * K,), dtype=torch.float32, device=q.device)
+                ws_ml = _made((S * H * (K // 16) * 2,), dtype=torch.float32, device=q.device)
+            ws_sums = _made((N * H,), dtype=torch.float32, device=q.device) if run_prefill else None
             # one output head a wavefront: twice the workgroups, which make all scores again; where the tiles leave CUs idle
             out_heads = 1 if -(-max_q_len // 16) * S * 2 <= self.compute_units() else 2
             self._run("talking", "lle_talking_mfma",
-                      [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _P, _P, _I, _I, _I, _P, _P, _I, _I, _I,
-                       _P, _P],
+                      "PPPPPPPPIIIIILIIFPPIIIPPIIIPP",
                       _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens),
                       _ptr(token_seq), _ptr(out), S, H, G, D, P, kv_layer.stride(0), block_table.shape[1], int(chunk or 0),
                       float(scale), _ptr(slopes), _ptr(talk), int(run_decode), splits, K, _ptr(ws_s), _ptr(ws_ml),
                       int(run_prefill), max_q_len, out_heads, _ptr(ws_sums))
             return out
         self._run("talking", "lle_talking_generic",
-                  [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _F, _P, _P, _I, _P],
+                  "PPPPPPPPIIIIILIIFPPIP",
                   _ptr(q), _ptr(kv_layer), _ptr(block_table), _ptr(seq_slots), _ptr(cu_tokens), _ptr(kv_lens), _ptr(token_seq),
                   _ptr(out), N, H, G, D, P, kv_layer.stride(0), block_table.shape[1], int(chunk or 0), float(scale),
                   _ptr(slopes), _ptr(talk), dtype_code(q.dtype))
@@ -1849,8 +1922,8 @@ class HipOps:
         N, R = low.shape
         C = bias.shape[0]
         _need(a2.shape == (R, C), "a2 must be [R, C]")
-        out = torch.empty((N, C), dtype=torch.float32, device=low.device)
-        self._run("gla", "lle_gla_decay", [_P, _P, _P, _P, _I, _I, _I, _F, _P], _ptr(low), _ptr(a2), _ptr(bias), _ptr(out), N, R,
+        out = _made((N, C), dtype=torch.float32, device=low.device)
+        self._run("gla", "lle_gla_decay", "PPPPIIIFP", _ptr(low), _ptr(a2), _ptr(bias), _ptr(out), N, R,
                   C, float(tau))
         return out
 
@@ -1875,16 +1948,16 @@ class HipOps:
         _need(norm_w.shape == (vdim,), "the norm weight must be [vdim]")
         _need(state.dim() == 2 and state.shape[1] >= heads * dim * vdim, "a state row holds heads * dim * vdim floats")
         _need(cu_tokens.shape == (S + 1,), "cu_tokens must be [S + 1]")
-        out = torch.empty((N, heads * vdim), dtype=u.dtype, device=u.device)
+        out = _made((N, heads * vdim), dtype=u.dtype, device=u.device)
         piece = self.GLA_PIECE
         pieces = -(-max_q_len // piece) if max_q_len > 2 * piece else 1
         part = None
         if pieces > 1:
-            part = torch.empty((S * pieces * heads * (dim * vdim + dim),), dtype=torch.float32, device=u.device)
+            part = _made((S * pieces * heads * (dim * vdim + dim),), dtype=torch.float32, device=u.device)
         else:
             piece = 1 << 30
         self._run("gla", "lle_gla_scan",
-                  [_P, _I, _P, _F, _P, _F, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P],
+                  "PIPFPFPLPPPIIIIIIPIP",
                   _ptr(u), cols, _ptr(decay), float(q_scale), _ptr(norm_w), float(eps), _ptr(state), state.stride(0),
                   _ptr(seq_slots), _ptr(cu_tokens), _ptr(out), S, heads, dim, vdim, pieces, piece, _ptr(part),
                   dtype_code(u.dtype))
@@ -1913,8 +1986,8 @@ class HipOps:
             _dev(gate_t, "row gate", torch.float32)
             _need(gate_t.dim() == 2 and gate_t.shape[0] == N and 0 <= col < gate_t.shape[1], "row gate [N, > col]")
             stride = gate_t.shape[1]
-        out = torch.empty((N, F), dtype=z.dtype, device=z.device)
-        self._run("elementwise", "lle_bias_act", [_P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _F, _I, _P], _ptr(z), _ptr(bias),
+        out = _made((N, F), dtype=z.dtype, device=z.device)
+        self._run("elementwise", "lle_bias_act", "PPPIIPIIIIFIP", _ptr(z), _ptr(bias),
                   _ptr(gate_t), stride, int(col), _ptr(out), N, F, 1 if gated else 0, self.ACT_CODES[kind],
                   float(limit), dtype_code(z.dtype))
         return out
@@ -1923,7 +1996,7 @@ class HipOps:
         """float32 x = cap * tanh(x / cap), in place."""
         _dev(x, "x", torch.float32)
         _need(cap > 0.0, "a cap must be positive")
-        self._run("elementwise", "lle_softcap", [_P, _L, _F, _P], _ptr(x), x.numel(), float(cap))
+        self._run("elementwise", "lle_softcap", "PLFP", _ptr(x), x.numel(), float(cap))
         return x
 
     def rmsnorm_add_rmsnorm(self, hidden, y, weight, eps: float, next_weight, next_eps: float, out_dtype,
@@ -1940,8 +2013,8 @@ class HipOps:
             if t is not None:
                 _dev(t, name)
                 _need(t.shape == hidden.shape, f"{name} must have the shape of hidden")
-        out = torch.empty((N, H), dtype=out_dtype, device=hidden.device)
-        self._run("norm", "lle_rmsnorm_add_rmsnorm", [_P, _P, _I, _P, _I, _P, _P, _I, _P, _I, _I, _F, _F, _I, _P],
+        out = _made((N, H), dtype=out_dtype, device=hidden.device)
+        self._run("norm", "lle_rmsnorm_add_rmsnorm", "PPIPIPPIPIIFFIP",
                   _ptr(hidden), _ptr(y), dtype_code(y.dtype), _ptr(extra), dtype_code(extra.dtype) if extra is not None else 0,
                   _ptr(weight), _ptr(next_weight), dtype_code(weight.dtype), _ptr(out), N, H, float(eps), float(next_eps),
                   dtype_code(out_dtype))
@@ -1987,9 +2060,9 @@ class HipOps:
         if rotary_dim > 0:
             _dev(cos_sin, "cos_sin", torch.float32)
             _need(cos_sin.shape == (N, rotary_dim // 2, 2), "cos_sin must be [N, rotary_dim / 2, 2]")
-        q_out = torch.empty((N, nq, D), dtype=u.dtype, device=u.device)
+        q_out = _made((N, nq, D), dtype=u.dtype, device=u.device)
         self._run("rope_kv", "lle_conv_norm_rope_write",
-                  [_P, _I, _P, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I, _L, _I, _I, _P],
+                  "PIPIPLPPPPPPPIFPPIIIIIIILIIP",
                   _ptr(u), cols, _ptr(taps), J, _ptr(state) if J > 1 else None, state.stride(0) if J > 1 else 0,
                   _ptr(token_seq), _ptr(cu_tokens), _ptr(seq_slots), _ptr(slots), _ptr(q_weight), _ptr(k_weight),
                   _ptr(cos_sin) if rotary_dim > 0 else None, rotary_dim, float(eps), _ptr(q_out), _ptr(kv_layer), N, nq, nkv,
@@ -2006,7 +2079,7 @@ class HipOps:
         N, cols = u.shape
         S = seq_slots.shape[0]
         _need(kept > 0 and state.shape[1] >= kept * cols and cu_tokens.shape == (S + 1,), "a state row holds `kept` rows of u")
-        self._run("rope_kv", "lle_conv_state_update", [_P, _I, _P, _L, _I, _P, _P, _I, _I, _P], _ptr(u), cols, _ptr(state),
+        self._run("rope_kv", "lle_conv_state_update", "PIPLIPPIIP", _ptr(u), cols, _ptr(state),
                   state.stride(0), int(kept), _ptr(cu_tokens), _ptr(seq_slots), S, dtype_code(u.dtype))
 
     # -- the gated delta rule --------------------------------------------------------------
@@ -2039,11 +2112,11 @@ class HipOps:
             _need(state is not None, "a convolution of several taps needs the requests' state rows")
             _rows(state, "state", torch.float32)
             _need(state.shape[1] >= (J - 1) * cols, "a state row holds J - 1 rows of u")
-        q = torch.empty((N, G * dim), dtype=torch.float32, device=u.device)
-        k = torch.empty((N, G * dim), dtype=torch.float32, device=u.device)
-        v = torch.empty((N, H * vdim), dtype=torch.float32, device=u.device)
+        q = _made((N, G * dim), dtype=torch.float32, device=u.device)
+        k = _made((N, G * dim), dtype=torch.float32, device=u.device)
+        v = _made((N, H * vdim), dtype=torch.float32, device=u.device)
         _need(not advance or (1 < J <= self.DELTA_MAX_ADVANCE and N == S), "the state moves on in this launch for single tokens")
-        self._run("delta", "lle_delta_conv", [_P, _I, _P, _I, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _I, _I, _P],
+        self._run("delta", "lle_delta_conv", "PIPIPLPPPPPPIIIIIFFIIP",
                   _ptr(u), cols, _ptr(taps), J, _ptr(state) if J > 1 else None, state.stride(0) if J > 1 else 0,
                   _ptr(token_seq), _ptr(cu_tokens), _ptr(seq_slots), _ptr(q), _ptr(k), _ptr(v), N, G, dim, H, vdim,
                   float(unit_eps), float(q_scale), int(advance), dtype_code(u.dtype))
@@ -2068,9 +2141,9 @@ class HipOps:
         _need(CA % dim == 0 and a_log.shape == (CA // dim,) and dt_bias.shape == (CA,), "a2 [heads * dim, R], a_log [heads], dt_bias [heads * dim]")
         _need(RA % 16 == 0 and RG % 16 == 0 and cols % 4 == 0 and a_col % 4 == 0 and g_col % 4 == 0, "ranks are multiples of 16, columns start at multiples of 4")
         _need(0 <= a_col and a_col + RA <= cols and 0 <= g_col and g_col + RG <= cols, "low has too few columns")
-        decay = torch.empty((N, CA), dtype=torch.float32, device=low.device)
-        gate = torch.empty((N, CG), dtype=torch.float32, device=low.device) if g2 is not None else None
-        self._run("delta", "lle_low_rank_gates", [_P, _I, _I, _I, _P, _I, _I, _P, _I, _I, _P, _P, _I, _P, _P, _I, _P],
+        decay = _made((N, CA), dtype=torch.float32, device=low.device)
+        gate = _made((N, CG), dtype=torch.float32, device=low.device) if g2 is not None else None
+        self._run("delta", "lle_low_rank_gates", "PIIIPIIPIIPPIPPIP",
                   _ptr(low), cols, int(a_col), int(g_col), _ptr(a2), RA, CA, _ptr(g2), RG, CG, _ptr(a_log), _ptr(dt_bias), int(dim),
                   _ptr(decay), _ptr(gate), N)
         return decay, gate
@@ -2116,27 +2189,27 @@ class HipOps:
                   "ba [N, >= heads]; decay [N, heads dim]")
         _need(state.shape[1] >= H * vdim * dim, "a state row holds heads * vdim * dim floats")
         _need(cu_tokens.shape == (S + 1,), "cu_tokens must be [S + 1]")
-        out = torch.empty((N, H * vdim), dtype=torch.float32, device=v.device)
+        out = _made((N, H * vdim), dtype=torch.float32, device=v.device)
         # steps with portions: the exponentials of decay and beta leave the walk (a step of single tokens keeps them there:
         # one launch less).  The number of tokens is known on the host and fixed inside a graph.
         args = (_ptr(q), _ptr(k), _ptr(v), _ptr(ba), ba.shape[1], _ptr(decay), _ptr(a_log), _ptr(dt_bias), _ptr(state), state.stride(0),
                 _ptr(seq_slots), _ptr(cu_tokens), _ptr(out), S, H, G, dim, vdim)
-        types = [_P, _P, _P, _P, _I, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I]
+        types = "PPPPIPPPPLPPPIIIII"
         few = 0  # requests that may go in chunks
         if N - S + 1 > self.DELTA_WALK * (1 if S == 1 else 4):  # (so many tokens may be one request's)
             few = self.compute_units(v.device) // (H * -(-int(vdim) // 16))
             if S > few and N > S * self.DELTA_WALK:  # (about all of them are long)
                 few = 0
-            floats = self._get("delta", "lle_delta_chunk_floats", [_I, _I, _I, _I, _I])(N, S, H, dim, vdim) if few > 0 else 0
+            floats = self._get("delta", "lle_delta_chunk_floats", "IIIII")(N, S, H, dim, vdim) if few > 0 else 0
             if 0 < floats <= self.DELTA_CHUNK_FLOATS and not any(t is not None and t.data_ptr() % 16 for t in (q, k, decay)):
-                work = torch.empty((floats,), dtype=torch.float32, device=v.device)
-                self._run("delta", "lle_delta_chunks", types + [_I, _I, _I, _P, _P], *args, N, self.DELTA_WALK, few, _ptr(work))
+                work = _made((floats,), dtype=torch.float32, device=v.device)
+                self._run("delta", "lle_delta_chunks", types + "IIIPP", *args, N, self.DELTA_WALK, few, _ptr(work))
                 if S == 1:
                     return out
             else:
                 few = 0
-        gates = torch.empty((N, 2 * H), dtype=torch.float32, device=v.device) if decay is None and N >= max(self.DELTA_GATES_AHEAD, 2 * S) else None
-        self._run("delta", "lle_delta_scan", types + [_P, _I, _I, _I, _P], *args, _ptr(gates), N, self.DELTA_WALK, few)
+        gates = _made((N, 2 * H), dtype=torch.float32, device=v.device) if decay is None and N >= max(self.DELTA_GATES_AHEAD, 2 * S) else None
+        self._run("delta", "lle_delta_scan", types + "PIIIP", *args, _ptr(gates), N, self.DELTA_WALK, few)
         return out
 
     def delta_out_norm(self, o, gate, norm_w, eps: float, heads: int, vdim: int, act: str = "silu", out_dtype=None) -> torch.Tensor:
@@ -2150,9 +2223,9 @@ class HipOps:
         N = o.shape[0]
         _need(o.shape == (N, heads * vdim) and gate.shape == o.shape and norm_w.shape == (vdim,),
               "o and gate [N, heads vdim]; norm weight [vdim]")
-        out = torch.empty(o.shape, dtype=out_dtype or gate.dtype, device=o.device)
+        out = _made(o.shape, dtype=out_dtype or gate.dtype, device=o.device)
         _need(gate.dtype in (torch.float32, out.dtype), "the gate is float32 or of the result's type")
-        self._run("delta", "lle_delta_out_norm", [_P, _P, _I, _I, _P, _I, _F, _P, _I, _I, _I, _I, _P], _ptr(o), _ptr(gate),
+        self._run("delta", "lle_delta_out_norm", "PPIIPIFPIIIIP", _ptr(o), _ptr(gate),
                   dtype_code(gate.dtype), 1 if act == "sigmoid" else 0, _ptr(norm_w), dtype_code(norm_w.dtype), float(eps),
                   _ptr(out), N, int(heads), int(vdim), dtype_code(out.dtype))
         return out
@@ -2188,16 +2261,16 @@ class HipOps:
             _need(state is not None, "a convolution of several taps needs the requests' state rows")
             _rows(state, "state", torch.float32)
             _need(state.shape[1] >= (J - 1) * C, "a state row holds J - 1 inputs")
-        out = torch.empty((N, C), dtype=torch.float32, device=u.device)
+        out = _made((N, C), dtype=torch.float32, device=u.device)
         dt, K, H = None, 0, 0
         if x is not None:
             _dev(x, "x", u.dtype)
             _dev(dt_w, "dt_w", u.dtype)
             K, H = x.shape[1], dt_w.shape[0]
             _need(x.shape[0] == N and dt_w.shape == (H, K), "x must be [N, K], dt_w [H, K]")
-            dt = torch.empty((N, H), dtype=torch.float32, device=u.device)
+            dt = _made((N, H), dtype=torch.float32, device=u.device)
         self._run("ssd", "lle_ssd_conv",
-                  [_P, _I, _I, _P, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P],
+                  "PIIPIPPLPPPPIIIIPPPIIIP",
                   _ptr(u), cols, int(col0), _ptr(taps), J, _ptr(bias), _ptr(state) if J > 1 else None,
                   state.stride(0) if J > 1 else 0, _ptr(token_seq), _ptr(cu_tokens), _ptr(seq_slots), _ptr(out), N, S, C,
                   1 if single else 0, _ptr(x), _ptr(dt_w), _ptr(dt), K, H, dtype_code(u.dtype))
@@ -2233,16 +2306,16 @@ class HipOps:
         _need(state.shape[1] >= H * vdim * n and cu_tokens.shape == (S + 1,), "a state row holds heads * vdim * n floats")
         longest = min(max_q_len or N, N)
         pieces = -(-longest // self.SSD_CHUNK) if longest > self.SSD_WALK else 0
-        y = torch.empty((N, H * vdim), dtype=torch.float32, device=c.device)
+        y = _made((N, H * vdim), dtype=torch.float32, device=c.device)
         part = part_decay = None
         together = 1
         if pieces:
             slots = N // self.SSD_CHUNK + S
-            part = torch.empty((slots * H * vdim * n,), dtype=torch.float32, device=c.device)
-            part_decay = torch.empty((slots * H,), dtype=torch.float32, device=c.device)
+            part = _made((slots * H * vdim * n,), dtype=torch.float32, device=c.device)
+            part_decay = _made((slots * H,), dtype=torch.float32, device=c.device)
             together = self.ssd_heads_a_group(H, G, -(-N // self.SSD_CHUNK))
         self._run("ssd", "lle_ssd_scan",
-                  [_P, _I, _P, _I, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
+                  "PIPIPPPPLPPPIIIIIIIIPPP",
                   _ptr(c), CC, _ptr(dt_in), dt_in.shape[1], _ptr(dt_bias), _ptr(a_log), _ptr(D), _ptr(state), state.stride(0),
                   _ptr(seq_slots), _ptr(cu_tokens), _ptr(y), S, H, G, int(vdim), int(n),
                   1 if (min_q_len or 1) <= self.SSD_WALK else 0, pieces, together, _ptr(part), _ptr(part_decay))
@@ -2257,8 +2330,8 @@ class HipOps:
         N, inner = y.shape
         _need(u.shape[0] == N and 0 <= z_col and z_col + inner <= u.shape[1], "u has too few columns")
         _need(norm_w.shape == (inner,) and groups > 0 and inner % groups == 0, "the norm weight must be [inner], cut into equal parts")
-        out = torch.empty((N, inner), dtype=u.dtype, device=u.device)
-        self._run("ssd", "lle_ssd_gate_norm", [_P, _P, _I, _I, _P, _F, _P, _I, _I, _I, _I, _P], _ptr(y), _ptr(u), u.shape[1],
+        out = _made((N, inner), dtype=u.dtype, device=u.device)
+        self._run("ssd", "lle_ssd_gate_norm", "PPIIPFPIIIIP", _ptr(y), _ptr(u), u.shape[1],
                   int(z_col), _ptr(norm_w), float(eps), _ptr(out), N, inner, int(groups), dtype_code(u.dtype))
         return out
 
@@ -2268,17 +2341,17 @@ class HipOps:
         the pick of row r is also written to dst[index[r]] (the host has made sure that index is in range)."""
         _dev(logits, "logits", torch.float32)
         R, V = logits.shape
-        out = torch.empty((R,), dtype=torch.int32, device=logits.device)
+        out = _made((R,), dtype=torch.int32, device=logits.device)
         chunks = max(1, min(64, V // 2048))  # enough workgroups to stream a long row from all CUs
-        part_val = torch.empty((R * chunks,), dtype=torch.float32, device=logits.device)
-        part_idx = torch.empty((R * chunks,), dtype=torch.int32, device=logits.device)
+        part_val = _made((R * chunks,), dtype=torch.float32, device=logits.device)
+        part_idx = _made((R * chunks,), dtype=torch.int32, device=logits.device)
         dst = index = None
         if scatter is not None:
             dst, index = scatter
             _dev(dst, "scatter destination", torch.int32)
             _dev(index, "scatter index", torch.int32)
             _need(index.shape == (R,), "one scatter index for every row")
-        self._run("sampling", "lle_argmax_rows_scatter", [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P],
+        self._run("sampling", "lle_argmax_rows_scatter", "PPPPIIIPPP",
                   _ptr(logits), _ptr(out), _ptr(part_val), _ptr(part_idx), R, V, chunks, _ptr(dst), _ptr(index))
         return out
 
@@ -2289,8 +2362,8 @@ class HipOps:
         _dev(uniform, "uniform", torch.float32)
         R, V = logits.shape
         _need(temperature.shape == (R,) and uniform.shape == (R,), "temperature and uniform must be [R]")
-        out = torch.empty((R,), dtype=torch.int32, device=logits.device)
-        self._run("sampling", "lle_sample_rows", [_P, _P, _P, _P, _I, _I, _P],
+        out = _made((R,), dtype=torch.int32, device=logits.device)
+        self._run("sampling", "lle_sample_rows", "PPPPIIP",
                   _ptr(logits), _ptr(temperature), _ptr(uniform), _ptr(out), R, V)
         return out
 
@@ -2301,11 +2374,11 @@ class HipOps:
         _dev(data, "data")
         nbytes = data.numel() * data.element_size()
         _need(nbytes % 16 == 0 and nbytes > 0, "the read probe takes a multiple of 16 bytes")
-        self._run("probe", "lle_probe_read_stream", [_P, _L, _I, _P, _P], _ptr(data), nbytes, int(blocks), None)
+        self._run("probe", "lle_probe_read_stream", "PLIPP", _ptr(data), nbytes, int(blocks), None)
 
     def probe_mfma(self, dtype, blocks: int, iters: int) -> float:
         """Launch a kernel of nothing but matrix instructions on registers; returns its flops."""
-        self._run("probe", "lle_probe_mfma", [_I, _I, _I, _P, _P], dtype_code(dtype), int(blocks), int(iters), None)
+        self._run("probe", "lle_probe_mfma", "IIIPP", dtype_code(dtype), int(blocks), int(iters), None)
         per_instruction = 2.0 * 16 * 16 * (32 if dtype == torch.bfloat16 else 4)
         return per_instruction * 16 * iters * 4 * blocks
 

@@ -16,7 +16,8 @@ from typing import Dict, List, Optional, Sequence
 
 import torch
 
-from ..parts.base import Block, BuildContext, Carried, Injected, Norm, Normed, Prenormed
+from ..csrc.record import Replay, addresses_of, operand_kinds
+from ..parts.base import Block, BuildContext, Carried, Injected, Norm, Normed, PartialSums, Prenormed
 from ..parts.embedding import Embedding
 from ..parts.injection import PassVectors
 from ..parts.linear import Linear
@@ -55,6 +56,17 @@ def looped_plan(blocks: int, start: int, stop: int, times: int, inject: bool = T
     for t in range(times):
         plan += [PlanEntry(i, inject=Inject(t, t > 0) if inject and i == start else None) for i in range(start, stop)]
     return plan + [PlanEntry(i) for i in range(stop, blocks)]
+
+
+def _tensors(delta):
+    """The tensors of what a block leaves to be added, where it is one of these; else None."""
+    if isinstance(delta, torch.Tensor):
+        return (delta,)
+    if type(delta) is PartialSums:
+        return (delta.sums,)
+    if type(delta) is Prenormed:
+        return delta.xw, delta.sums
+    return None
 
 
 class DecoderLM:
@@ -152,6 +164,86 @@ class DecoderLM:
         return Injected(delta, None if inject.vector is None else self.pass_vectors.row(inject.vector),
                         self.embedding.again(step) if inject.embedding else None, self.ctx.ops)
 
+    def _run_layer(self, i: int, hidden, delta, step, caches):
+        """Plan entry i: what the block leaves to be added."""
+        e, last = self.plan[i], len(self.plan) - 1
+        # the norm that the next block starts with, if the products around it may do its work
+        if i < last and self.plan[i + 1].inject is not None:
+            next_norm = None  # something enters the stream first
+        elif i < last:
+            follower = self.blocks[self.plan[i + 1].block]
+            next_norm = follower.entry_norm()
+            if next_norm is None and self.blocks[e.block].chained_norm() is not None:
+                next_norm = follower.chained_norm()  # (between two blocks that chain their norms)
+        else:  # the final norm, where the head's product can take its place (every row goes to the head) ...
+            next_norm = self.final_norm if step.every_row_wanted and not self.head.has_bias else None
+            # ... but not in float32, whose rows' sums do not follow what else the step brings: folded, they run in another order
+            if self.ctx.dtype == torch.float32 and self.blocks[e.block].chained_norm() is None:
+                next_norm = None
+        if e.inject is not None:
+            delta = self._injected(e.inject, delta, step)
+        return self.blocks[e.block].forward(hidden, delta, step, caches.layer(i), next_norm=next_norm)
+
+    # Layers that are alike (csrc/record.py): worth it from two layers launched again on, the host's checks of all layers being about a
+    # layer's launches again (28 layers: 0.2 ms).  Steps of more tokens keep the device busy for longer than the host needs, and what a layer made would
+    # be held for longer than before.
+    ALIKE_LAYERS, ALIKE_TOKENS = 6, 2048
+
+    def _alike_layers(self, step, caches):
+        """(first entry to record, end, [(operands, their addresses)] of the entries from the first on): the entries first - 1 ..
+        end - 1 have blocks that launch alike; None without such a stretch."""
+        ops, plan = self.ctx.ops, self.plan
+        if (len(plan) < self.ALIKE_LAYERS or step.token_ids.shape[0] > self.ALIKE_TOKENS
+                or not getattr(ops, "may_record", lambda: False)()):
+            return None
+        best, start, seen, settings, kinds, like = None, 0, [], None, None, None  # the stretch: first entry, (tensors, addresses), what its blocks share
+        for i, e in enumerate(plan):
+            made = self.blocks[e.block].launches() if e.inject is None else None
+            cache = caches.layer(i)
+            if made is None or cache.kv is None or cache.state is not None:
+                settings = None
+                continue
+            tensors = made[1] + (cache.kv,)
+            if settings is not None and made[0] == settings and cache.group is like.group and cache.writes == like.writes:
+                at = addresses_of(tensors, kinds)
+                if at is not None:
+                    seen.append((tensors, at))
+                    continue
+            start, settings, like, kinds = i, made[0], cache, operand_kinds(tensors)
+            seen = [(tensors, addresses_of(tensors, kinds))]
+            if seen[0][1] is None:
+                settings = None
+            elif best is None or len(best[1]) < self.ALIKE_LAYERS:
+                best = (start, seen)
+        if best is None or len(best[1]) < self.ALIKE_LAYERS:
+            return None
+        start, seen = best
+        # the last product of a layer may do the work of the norm that its follower starts with
+        out = []
+        for k in range(1, len(seen) - 1):
+            w = self.blocks[plan[start + k + 1].block].input_norm().weight
+            out.append((seen[k][0] + (w,), seen[k][1] + [w.data_ptr()]))
+        return start + 1, start + len(seen), out
+
+    def _run_alike(self, stretch, hidden, delta, step, caches):
+        """The recorded entry and those behind it but for the stretch's last, whose follower is another: (what the last of them
+        leaves, the entry that comes next)."""
+        first, end, operands = stretch
+        ops, given = self.ctx.ops, _tensors(delta)
+        record = ops.record()
+        try:
+            left = self._run_layer(first, hidden, delta, step, caches)
+        finally:
+            ops.end_record()
+        if given is None or type(left) is not type(delta) or getattr(left, "eps", None) != getattr(delta, "eps", None):
+            return left, first + 1
+        replay = Replay(record, operands[0][0], given, _tensors(left))
+        if not replay.ok:
+            return left, first + 1
+        for tensors, addresses in operands[1:]:
+            ops.replay(replay, tensors, addresses)
+        return left, end - 1
+
     def forward(self, step, caches) -> torch.Tensor:
         """Run the tokens of `step` (engine.batch.StepState) through the plan and
         return float32 logits [len(step.logit_rows), vocab]."""
@@ -163,24 +255,13 @@ class DecoderLM:
             hidden, delta = self.embedding.forward(step.token_ids, step, norm=first_norm)
         else:
             hidden, delta = self.embedding.forward(step.token_ids, step), None
-        last = len(self.plan) - 1
-        for i, e in enumerate(self.plan):
-            # the norm that the next block starts with, if the products around it may do its work
-            if i < last and self.plan[i + 1].inject is not None:
-                next_norm = None  # something enters the stream first
-            elif i < last:
-                follower = self.blocks[self.plan[i + 1].block]
-                next_norm = follower.entry_norm()
-                if next_norm is None and self.blocks[e.block].chained_norm() is not None:
-                    next_norm = follower.chained_norm()  # (between two blocks that chain their norms)
-            else:  # the final norm, where the head's product can take its place (every row goes to the head) ...
-                next_norm = self.final_norm if step.every_row_wanted and not self.head.has_bias else None
-                # ... but not in float32, whose rows' sums do not follow what else the step brings: folded, they run in another order
-                if self.ctx.dtype == torch.float32 and self.blocks[e.block].chained_norm() is None:
-                    next_norm = None
-            if e.inject is not None:
-                delta = self._injected(e.inject, delta, step)
-            delta = self.blocks[e.block].forward(hidden, delta, step, caches.layer(i), next_norm=next_norm)
+        stretch = self._alike_layers(step, caches)
+        i = 0
+        while i < len(self.plan):
+            if stretch is not None and i == stretch[0]:
+                delta, i = self._run_alike(stretch, hidden, delta, step, caches)
+            else:
+                delta, i = self._run_layer(i, hidden, delta, step, caches), i + 1
         if step.logit_rows.shape[0] == 0:
             return torch.empty((0, self.vocab_size), dtype=torch.float32, device=hidden.device)
         if isinstance(delta, Carried):  # the last block has added everything into the stream itself

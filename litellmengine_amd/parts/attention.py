@@ -103,6 +103,14 @@ class PagedAttention(Mixer):
                 qw, kw = qw.float(), kw.float()
             self.q_norm_w, self.k_norm_w = qw.contiguous(), kw.contiguous()
 
+    def launches(self):
+        qkv, o, position = self.qkv.launches(), self.o.launches(), self.position.launches()
+        if not (self._as_made(PagedAttention) and qkv and o and position):
+            return None
+        settings = (self.nq, self.nkv, self.d, self.qk_norm_eps, self.window, self.scale, self.folds_norm, qkv[0], o[0], position[0])
+        norms = () if self.qk_norm_eps is None else (self.q_norm_w, self.k_norm_w)
+        return settings, qkv[1] + o[1] + norms
+
     def forward(self, x, step, cache, fold=None):
         ops = self.ctx.ops
         qkv = self.qkv.forward(x)

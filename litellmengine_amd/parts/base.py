@@ -127,6 +127,16 @@ class Part:
         """Take the tensors named by `tensor_specs` out of `weights`."""
         self.ctx = ctx
 
+    def launches(self) -> Optional[Tuple[tuple, tuple]]:
+        """(settings, tensors) of a part that launches through `ctx.ops` alone, and what follows from the settings, the step and
+        the tensors' sizes, types and alignment: of two such parts with equal settings and such tensors the second's launches are
+        the first's with its own tensors in their places.  None where that is not promised (a subclass, an instance with a
+        method of its own)."""
+        return None
+
+    def _as_made(self, cls) -> bool:
+        return type(self) is cls and "forward" not in vars(self)
+
 
 @dataclasses.dataclass
 class NormFold:

@@ -43,6 +43,14 @@ class PreNormBlock(Block):
         kernel that takes it adds the two."""
         return ScaledSum(y[0], y[1], 1.0) if isinstance(y, tuple) else y
 
+    def launches(self):
+        if not self._as_made(PreNormBlock) or self.feed_forward is None:
+            return None
+        a, b, c, d = self.norm_in.launches(), self.mixer.launches(), self.norm_post.launches(), self.feed_forward.launches()
+        if a is None or b is None or c is None or d is None:
+            return None
+        return (a[0], b[0], c[0], d[0]), a[1] + b[1] + c[1] + d[1]
+
     def entry_norm(self):
         return self.norm_in if self.mixer.folds_norm else None
 

@@ -57,6 +57,12 @@ class GatedMLP(FeedForward):
         if self.late_bias_name:
             self.late_bias = weights[self.late_bias_name].float().reshape(-1).contiguous()
 
+    def launches(self):
+        a, b = self.gate_up.launches(), self.down.launches()
+        if not (self._as_made(GatedMLP) and self.fused and self.late_bias is None and a and b):
+            return None
+        return (self.folds_norm, a[0], b[0]), a[1] + b[1]
+
     def forward(self, x, fold=None):
         ops = self.ctx.ops
         if self.fused:

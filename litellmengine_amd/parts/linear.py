@@ -56,6 +56,9 @@ class Linear(Part):
         self.ctx = ctx
         self.weight = tensor
 
+    def launches(self):
+        return ((self.to_residual,), (self.weight,)) if self._as_made(Linear) and self.bias is None else None
+
     def forward(self, x, out_dtype=None, fold=None):
         """`x` may be a parts.base.Prenormed; with `fold` (a parts.base.NormFold) the result
         is added into the residual stream and comes back as the Prenormed of that norm."""

@@ -33,6 +33,9 @@ class RMSNorm(Norm):
             w = 1.0 + w.float()
         self.weight = (w.reshape(1).expand(self.size) if self.scalar else w).contiguous()
 
+    def launches(self):
+        return ((self.size, self.eps, self.one_plus), (self.weight,)) if self._as_made(RMSNorm) else None
+
     def add_normed(self, hidden, y, extra=None, then=None) -> torch.Tensor:
         ops = self.ctx.ops
         if then is None:

@@ -20,7 +20,6 @@ results: the allocator's own order by stream is enough.
 """
 from __future__ import annotations
 
-import dataclasses
 from typing import Dict, Optional
 
 import torch
@@ -93,7 +92,7 @@ class SideBySideMixer(Mixer):
     def _share(self, cache, which: int):
         columns = self._columns[which]
         state = None if columns is None else cache.state[:, columns[0] : columns[0] + columns[1]]
-        return dataclasses.replace(cache, state=state)
+        return type(cache)(cache.group, cache.kv, cache.writes, state, cache.pages)  # (dataclasses.replace: 3 us more)
 
     def forward(self, x, step, cache):
         """-> (left's result, right's result): a pair that a norm's kernel adds up; with factors a ScaledSum."""
