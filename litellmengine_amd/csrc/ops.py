@@ -2282,6 +2282,14 @@ class HipOps:
         most, share = max(1, heads * chunks // (2 * self.compute_units())), heads // groups
         return max(k for k in range(1, share + 1) if share % k == 0 and (k <= most or k == 1))
 
+    def ssd_streams(self, num_tokens: int, num_seqs: int, heads: int, vdim: int, n: int, longest: int) -> bool:
+        """Whether the chunks of long requests go one after the other, the state in registers (ssd_stream_kernel): up to 512 tokens, and beyond
+        where the long requests' workgroups (a head and sixteen value channels each) are as many as the CUs.  With fewer the chain of the chunks
+        is what takes the time: 32 heads of 64 x 128, chunks side by side / one after the other, one request of 256, 512, 1024, 2048 tokens
+        34 / 24, 39 / 36, 54 / 59, 76 / 101 us; two of 1024 77 / 64; 64 heads, one request of 1024, 2048, 4096 tokens 76 / 63, 120 / 107, 224 / 189."""
+        few = max(1, (num_tokens - num_seqs) // max(1, longest)) * heads * (vdim // 16) < self.compute_units()
+        return n == 128 and vdim % 16 == 0 and longest < 1 << 15 and (longest <= 512 or not few)
+
     def ssd_scan(self, c, dt_in, dt_bias, a_log, D, state, heads: int, groups: int, vdim: int, n: int, seq_slots, cu_tokens,
                  min_q_len: int = 0, max_q_len: int = 0) -> torch.Tensor:
         """Per head h, with the matrix state S [n, vdim] of the request (float32; `state[slot]` begins with the heads'
@@ -2308,17 +2316,21 @@ class HipOps:
         pieces = -(-longest // self.SSD_CHUNK) if longest > self.SSD_WALK else 0
         y = _made((N, H * vdim), dtype=torch.float32, device=c.device)
         part = part_decay = None
-        together = 1
+        together, stream_floats = 1, 0
         if pieces:
             slots = N // self.SSD_CHUNK + S
-            part = _made((slots * H * vdim * n,), dtype=torch.float32, device=c.device)
-            part_decay = _made((slots * H,), dtype=torch.float32, device=c.device)
-            together = self.ssd_heads_a_group(H, G, -(-N // self.SSD_CHUNK))
+            if S <= 65535 and self.ssd_streams(N, S, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
+                stream_floats = slots * (G * (2 * self.SSD_CHUNK * 128 + 2560) + H * 5 * self.SSD_CHUNK)  # (lle_ssd_stream_floats)
+                part = _made((stream_floats,), dtype=torch.float32, device=c.device)
+            else:
+                part = _made((slots * H * vdim * n,), dtype=torch.float32, device=c.device)
+                part_decay = _made((slots * H,), dtype=torch.float32, device=c.device)
+                together = self.ssd_heads_a_group(H, G, -(-N // self.SSD_CHUNK))
         self._run("ssd", "lle_ssd_scan",
-                  "PIPIPPPPLPPPIIIIIIIIPPP",
+                  "PIPIPPPPLPPPIIIIIIIIPPILP",
                   _ptr(c), CC, _ptr(dt_in), dt_in.shape[1], _ptr(dt_bias), _ptr(a_log), _ptr(D), _ptr(state), state.stride(0),
                   _ptr(seq_slots), _ptr(cu_tokens), _ptr(y), S, H, G, int(vdim), int(n),
-                  1 if (min_q_len or 1) <= self.SSD_WALK else 0, pieces, together, _ptr(part), _ptr(part_decay))
+                  1 if (min_q_len or 1) <= self.SSD_WALK else 0, pieces, together, _ptr(part), _ptr(part_decay), N, stream_floats)
         return y
 
     def ssd_gate_norm(self, y, u, z_col: int, norm_w, eps: float, groups: int) -> torch.Tensor:

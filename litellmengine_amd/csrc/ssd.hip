@@ -658,22 +658,276 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------
+// States of 128 channels and value channels in sixteens: the chunks one after the other, the state in registers, so that no chunk's
+// contribution or entry state goes through memory (written twice and read twice, 32 KB a chunk and head of 64 x 128 each time).
+//   ssd_pairs_kernel  for every chunk at once: the step sizes and the sums l of its heads, C, B and the products C_t . B_s of its groups in the
+//     order in which the other kernel's lanes take them
+//   ssd_stream_kernel grid = (sixteens of value channels, heads, requests), four wavefronts.  Wavefront w keeps the state channels 32 w .. 32 w + 31:
+//     two tiles, lane (c, r), element e: channel 32 w + 8 c + 2 e + tile of value channel r, which is the operand of the products with C as
+//     it lies.  A chunk: the wavefront's share of C S for all 64 tokens and its tiles of the products of tokens within the chunk meet
+//     the others' in LDS (two buffers, one barrier a chunk), S moves on by the chunk's B x.  Every operand of the next chunk is asked
+//     for as soon as its place is free.
+// 64 heads of 64 x 128, a chunk's three passes through memory -> so, in us: one request of 64, 512, 2048 tokens 33 -> 17, 54 -> 41, 120 -> 107; 8 of 64,
+// 256, 512 tokens 82 -> 44, 134 -> 95, 234 -> 160.  A workgroup's chunk takes a CU 2.5 us: 1.0 of the float32 matrix instruction, 0.8 of loads (74 KB,
+// shared by four workgroups and 32 heads only in L2), the rest a wavefront or two a SIMD that nothing covers.  With eight wavefronts of 16 channels
+// each one request of 2048 tokens takes 100, eight of 64 55; with loads from the rows themselves, sixteen lines each, 112 and 49.
+// ---------------------------------------------------------------------------------
+#define SSD_N 128
+#define SSD_OF_B (SSD_CHUNK * SSD_N)
+#define SSD_OF_PAIRS (2 * SSD_CHUNK * SSD_N)
+#define SSD_OPERANDS (2 * SSD_CHUNK * SSD_N + 10 * 256)
+struct SsdStream {
+    float* operands;  // [chunk slots][G]: C, B and the ten tiles of C_t . B_s, s <= t, all lane by lane (SSD_OPERANDS floats)
+    float* steps;  // [chunk slots][H][5][64]: dt, l's two floats, exp(l_last - l) dt, exp(l)
+};
+
+// grid = (chunk slots, groups + ceil(heads / 4)), 256 threads
+__global__ __launch_bounds__(256) void ssd_pairs_kernel(SsdArgs a, SsdStream p, int S) {
+    int s = 0;  // the last request whose chunks begin here or before
+    for (int high = S - 1; s < high;) {
+        const int mid = (s + high + 1) / 2;
+        if (ssd_slot(a.cu_tokens[mid], mid) <= (int64_t)blockIdx.x) s = mid;
+        else high = mid - 1;
+    }
+    const int q0 = a.cu_tokens[s], len = a.cu_tokens[s + 1] - q0, piece = (int)(blockIdx.x - ssd_slot(q0, s));
+    if (len <= SSD_WALK || piece * SSD_CHUNK >= len) return;
+    const int t0 = q0 + piece * SSD_CHUNK, nt = min(SSD_CHUNK, len - piece * SSD_CHUNK);
+    const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE, c = lane / 16, r = lane % 16;
+    if ((int)blockIdx.y >= a.G) {  // a wavefront a head
+        const int h = ((int)blockIdx.y - a.G) * 4 + wave;
+        if (h >= a.H) return;
+        float dt, hi, lo;
+        ssd_chunk_steps(a, h, t0, nt, dt, hi, lo);
+        const float hi_last = __shfl(hi, LLE_WAVE - 1, LLE_WAVE), lo_last = __shfl(lo, LLE_WAVE - 1, LLE_WAVE);
+        float* out = p.steps + ((int64_t)blockIdx.x * a.H + h) * 5 * SSD_CHUNK + lane;
+        out[0] = dt;
+        out[SSD_CHUNK] = hi;
+        out[2 * SSD_CHUNK] = lo;
+        out[3 * SSD_CHUNK] = expf((hi_last - hi) + (lo_last - lo)) * dt;
+        out[4 * SSD_CHUNK] = expf(hi);
+        return;
+    }
+    // wavefront w: tokens 16 w .. 16 w + 15 with all keys up to them
+    const int inner = a.H * a.vdim, g = blockIdx.y, tok = wave * 16 + r;
+    const float* rows = a.c + (int64_t)t0 * a.CC + inner + g * SSD_N;
+    const float* crow = rows + (int64_t)min(tok, nt - 1) * a.CC + a.G * SSD_N;
+    float* out = p.operands + ((int64_t)blockIdx.x * a.G + g) * SSD_OPERANDS;
+    ssd_f32x4 C[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) C[q] = *(const ssd_f32x4*)(crow + 16 * q + 4 * c);
+    for (int st = 0; st <= wave; ++st) {
+        const float* brow = rows + (int64_t)min(st * 16 + r, nt - 1) * a.CC;
+        ssd_f32x4 B[8], acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) B[q] = *(const ssd_f32x4*)(brow + 16 * q + 4 * c);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(B[q][e], C[q][e], acc, 0, 0, 0);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(B[q][e + 1], C[q][e + 1], acc2, 0, 0, 0);
+            }
+        *(ssd_f32x4*)(out + SSD_OF_PAIRS + (wave * (wave + 1) / 2 + st) * 256 + lane * 4) = acc + acc2;
+    }
+    // C and B as ssd_stream_kernel's wavefront w takes them, zeros behind the last token: C of token 16 tt + r and channels 32 w + 8 c + 4 half,
+    // B of the tokens 4 k + c, k = 2 m and 2 m + 1, and channels 32 w + 2 r
+    const float* brows = rows + 32 * wave + 2 * r;
+    const float* crows = rows + a.G * SSD_N + 32 * wave + 8 * c;
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const ssd_f32x4 v = *(const ssd_f32x4*)(crows + (int64_t)min(16 * tt + r, nt - 1) * a.CC + 4 * half);
+            *(ssd_f32x4*)(out + ((wave * 4 + tt) * 2 + half) * 256 + lane * 4) = 16 * tt + r < nt ? v : ssd_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        ssd_f32x4 v;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int t = 4 * (2 * m + k) + c;
+            const float* row = brows + (int64_t)min(t, nt - 1) * a.CC;
+            v[2 * k] = t < nt ? row[0] : 0.f;
+            v[2 * k + 1] = t < nt ? row[1] : 0.f;
+        }
+        *(ssd_f32x4*)(out + SSD_OF_B + (wave * 8 + m) * 256 + lane * 4) = v;
+    }
+}
+
+// e^x for x <= 0 to about an ulp (expf's way to large and odd arguments is half of a tile's instructions): x log2 e in two floats
+__device__ __forceinline__ float ssd_exp(float x) {
+    const float p = x * 1.44269502162933349609f;
+    const float rest = fmaf(x, 1.92596302e-8f, fmaf(x, 1.44269502162933349609f, -p));
+    const float y = __builtin_amdgcn_exp2f(p);
+    return fmaf(y * 0.69314718f, rest, y);
+}
+
+__global__ __launch_bounds__(256, 2) void ssd_stream_kernel(SsdArgs a, SsdStream p) {
+    constexpr int XS = 20;  // words of a row of x in LDS: four rows apart meet every bank once
+    __shared__ __attribute__((aligned(16))) float s_x[2][SSD_CHUNK][XS], s_xf[2][SSD_CHUNK][XS];  // x, x times its factor
+    __shared__ __attribute__((aligned(16))) float s_y[2][4][4][256];                                // [wavefront][tile of tokens]
+    __shared__ __attribute__((aligned(16))) float s_step[2][4][SSD_CHUNK];                          // dt, l's two floats, exp(l)
+    const int s = blockIdx.z, h = blockIdx.y, j0 = blockIdx.x * 16;
+    const int q0 = a.cu_tokens[s], len = a.cu_tokens[s + 1] - q0;
+    if (len <= SSD_WALK) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / LLE_WAVE), lane = tid % LLE_WAVE, c = lane / 16, r = lane % 16;
+    const int grp = h / (a.H / a.G), inner = a.H * a.vdim, live = (len + SSD_CHUNK - 1) / SSD_CHUNK;
+    const int64_t slot0 = ssd_slot(q0, s);
+    const float* rows = a.c + (int64_t)q0 * a.CC;
+    const float D = a.D[h];
+    float* own = a.state + (int64_t)a.seq_slots[s] * a.state_stride + ((int64_t)h * a.vdim + j0 + r) * SSD_N + 32 * wave + 8 * c;
+    ssd_f32x4 S[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[0][e] = own[2 * e], S[1][e] = own[2 * e + 1];
+    // The operands that are on their way: C, B and the products C . B of the wavefront's tiles as the lanes take them, four x of token tid / 4,
+    // the steps of token tid.
+    ssd_f32x4 B[8], C[4][2], cb[3], x;
+    float step = 0.f, f = 0.f;
+    const int first[4] = {0, 1, 3, 5}, second[4] = {6, 2, 4, 9}, third[4] = {7, 8, 0, 0};
+    const int tile_at[3] = {first[wave], second[wave], third[wave]};  // the wavefront's tiles, of the ten
+    const int of_lane = 16 * lane, of_x = 4 * (tid / 4 * a.CC + h * a.vdim + j0 + 4 * (tid % 4));
+    auto four = [&](__amdgpu_buffer_rsrc_t unit, int floats) {
+        return __builtin_bit_cast(ssd_f32x4, __builtin_amdgcn_raw_buffer_load_b128(unit, of_lane, 4 * floats, 0));
+    };
+    auto unit_of = [&](int i) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(p.operands + ((slot0 + min(i, live - 1)) * a.G + grp) * SSD_OPERANDS), 0, 4 * SSD_OPERANDS, 0x00020000);
+    };
+    auto ask_b = [&](int i) {
+        const auto unit = unit_of(i);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) B[m] = four(unit, SSD_OF_B + (wave * 8 + m) * 256);
+    };
+    auto ask_c = [&](int i) {
+        const auto unit = unit_of(i);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) C[tt][half] = four(unit, ((wave * 4 + tt) * 2 + half) * 256);
+    };
+    auto ask_cb = [&](int i) {
+        const auto unit = unit_of(i);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) cb[n] = four(unit, SSD_OF_PAIRS + tile_at[n] * 256);
+    };
+    auto ask_x = [&](int i) {
+        // (a buffer that ends with the request's last token: tokens past it are zeros)
+        const auto chunk = __builtin_amdgcn_make_buffer_rsrc((void*)(rows + (int64_t)min(i, live - 1) * SSD_CHUNK * a.CC), 0,
+                                                             i < live ? (len - i * SSD_CHUNK) * a.CC * 4 : 0, 0x00020000);
+        x = __builtin_bit_cast(ssd_f32x4, __builtin_amdgcn_raw_buffer_load_b128(chunk, of_x, 0, 0));
+        const auto steps = __builtin_amdgcn_make_buffer_rsrc((void*)(p.steps + ((slot0 + min(i, live - 1)) * a.H + h) * (5 * SSD_CHUNK)), 0, 20 * SSD_CHUNK, 0x00020000);
+        auto word = [&](int at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(steps, 4 * at, 0, 0)); };
+        f = word(3 * SSD_CHUNK + tid / 4);
+        step = word((wave == 3 ? 4 : wave) * SSD_CHUNK + lane);  // (a wavefront an array)
+    };
+    auto stage = [&](int i) {
+        const int b = i & 1;
+        *(ssd_f32x4*)&s_x[b][tid / 4][4 * (tid % 4)] = x;
+        *(ssd_f32x4*)&s_xf[b][tid / 4][4 * (tid % 4)] = x * f;
+        s_step[b][wave][lane] = step;
+    };
+    auto meet = [&]() {  // (waits for no load on its way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    ask_x(0);
+    ask_c(0);
+    ask_cb(0);
+    ask_b(0);
+    stage(0);
+    ask_x(1);
+    meet();
+    for (int i = 0; i < live; ++i) {
+        const int b = i & 1;
+        ssd_f32x4 y[4];
+        // every token's share of C S, times exp(l_t)
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) y[tt] = ssd_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) y[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(C[tt][e / 4][e % 4], S[e % 2][e / 2], y[tt], 0, 0, 0);
+        ask_c(i + 1);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) y[tt] *= *(const ssd_f32x4*)&s_step[b][3][16 * tt + 4 * c];
+        // the chunk's tokens among each other
+        auto among = [&](auto tt_, auto st_, const ssd_f32x4& v) {
+            constexpr int tt = decltype(tt_)::value, st = decltype(st_)::value;
+            const float hi_t = s_step[b][1][16 * tt + r], lo_t = s_step[b][2][16 * tt + r];
+            const ssd_f32x4 dt_s = *(const ssd_f32x4*)&s_step[b][0][16 * st + 4 * c], hi_s = *(const ssd_f32x4*)&s_step[b][1][16 * st + 4 * c],
+                            lo_s = *(const ssd_f32x4*)&s_step[b][2][16 * st + 4 * c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                // (later keys weigh nothing; their exponent would be above zero)
+                const float m = tt > st || 4 * c + e <= r ? v[e] * ssd_exp((hi_t - hi_s[e]) + (lo_t - lo_s[e])) * dt_s[e] : 0.f;
+                y[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(m, s_x[b][16 * st + 4 * c + e][r], y[tt], 0, 0, 0);
+            }
+        };
+        using T0 = std::integral_constant<int, 0>;
+        using T1 = std::integral_constant<int, 1>;
+        using T2 = std::integral_constant<int, 2>;
+        using T3 = std::integral_constant<int, 3>;
+        switch (wave) {  // three, three, two and two of the ten tiles (tile_at)
+            case 0: among(T0{}, T0{}, cb[0]), among(T3{}, T0{}, cb[1]), among(T3{}, T1{}, cb[2]); break;
+            case 1: among(T1{}, T0{}, cb[0]), among(T1{}, T1{}, cb[1]), among(T3{}, T2{}, cb[2]); break;
+            case 2: among(T2{}, T0{}, cb[0]), among(T2{}, T1{}, cb[1]); break;
+            default: among(T2{}, T2{}, cb[0]), among(T3{}, T3{}, cb[1]); break;
+        }
+        ask_cb(i + 1);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) *(ssd_f32x4*)&s_y[b][wave][tt][lane * 4] = y[tt];
+        // the state behind the chunk
+        const float keep = s_step[b][3][SSD_CHUNK - 1];
+        S[0] *= keep;
+        S[1] *= keep;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const float xf = s_xf[b][4 * k + c][r];
+            S[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(B[k / 2][k % 2 * 2], xf, S[0], 0, 0, 0);
+            S[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(B[k / 2][k % 2 * 2 + 1], xf, S[1], 0, 0, 0);
+        }
+        ask_b(i + 1);
+        stage(i + 1);
+        ask_x(i + 2);
+        meet();
+        // four value channels of token tid / 4
+        const int t = tid / 4, tok = i * SSD_CHUNK + t;
+        ssd_f32x4 sum;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int at = (t % 16 / 4 * 16 + 4 * (tid % 4) + e) * 4 + t % 4;
+            sum[e] = ((s_y[b][0][t / 16][at] + s_y[b][1][t / 16][at]) + s_y[b][2][t / 16][at]) + s_y[b][3][t / 16][at];
+        }
+        const ssd_f32x4 xt = *(const ssd_f32x4*)&s_x[b][t][4 * (tid % 4)];
+        if (tok < len) *(ssd_f32x4*)(a.y + (int64_t)(q0 + tok) * inner + h * a.vdim + j0 + 4 * (tid % 4)) = xt * D + sum;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) own[2 * e] = S[0][e], own[2 * e + 1] = S[1][e];
+}
+
 extern "C" int lle_ssd_max_dim(void) { return 256; }
 extern "C" int lle_ssd_chunk(void) { return SSD_CHUNK; }
 extern "C" int lle_ssd_walk(void) { return SSD_WALK; }
+
+// Floats of `part` where the chunks go one after the other (ssd_stream_kernel), for a step of N tokens of S requests
+extern "C" int64_t lle_ssd_stream_floats(int N, int S, int H, int G) {
+    return (int64_t)(N / SSD_CHUNK + S) * (G * SSD_OPERANDS + H * 5 * SSD_CHUNK);
+}
 
 // c float32 [N, CC], CC = H vdim + 2 G n; dt_in float32 rows of dt_cols; dt_bias, a_log, D float32 [H]; state rows of
 // state_stride floats that begin with [H][vdim][n]; y float32 [N, H vdim].  `walk`: some request has at most SSD_WALK
 // tokens; `pieces` > 0: chunks of the longest request (0: no request has more), with `part` float32
 // [(N / SSD_CHUNK + S) H vdim n] and `part_decay` [(N / SSD_CHUNK + S) H].  heads_a_group divides H / G.
+// stream_floats > 0: requests of more tokens go chunk after chunk; `part` holds so many floats (lle_ssd_stream_floats), part_decay nothing.
 extern "C" int lle_ssd_scan(const void* c, int CC, const void* dt_in, int dt_cols, const void* dt_bias, const void* a_log,
                             const void* D, void* state, int64_t state_stride, const void* seq_slots, const void* cu_tokens, void* y,
                             int S, int H, int G, int vdim, int n, int walk, int pieces, int heads_a_group, void* part,
-                            void* part_decay, hipStream_t stream) {
+                            void* part_decay, int N, int64_t stream_floats, hipStream_t stream) {
     if (S <= 0 || H <= 0) return 0;
     if (G <= 0 || H % G || vdim <= 0 || vdim > 256 || n <= 0 || n > 256 || H > 65535 || CC != H * vdim + 2 * G * n || dt_cols < H ||
         pieces < 0 || heads_a_group <= 0 || (H / G) % heads_a_group || (int64_t)S * (pieces > 0 ? pieces : 1) > 0x7fffffff ||
-        (pieces > 0 && (!part || !part_decay)))
+        (pieces > 0 && (!part || (!part_decay && stream_floats == 0))))
         return (int)hipErrorInvalidValue;
     // LDS holds the step sizes of a workgroup's heads: at most SSD_HEADS of them
     for (int k = SSD_HEADS; heads_a_group > SSD_HEADS; --k)
@@ -692,6 +946,15 @@ extern "C" int lle_ssd_scan(const void* c, int CC, const void* dt_in, int dt_col
         if (e != hipSuccess || pieces == 0) return (int)e;
     }
     if (pieces == 0) return 0;
+    if (stream_floats > 0) {
+        const int chunks = N / SSD_CHUNK + S;
+        if (n != SSD_N || vdim % 16 != 0 || S > 65535 || stream_floats < lle_ssd_stream_floats(N, S, H, G) || (((uintptr_t)c | (uintptr_t)y | (uintptr_t)part) & 15))
+            return (int)hipErrorInvalidValue;
+        const SsdStream p{(float*)part, (float*)part + (int64_t)chunks * G * SSD_OPERANDS};
+        ssd_pairs_kernel<<<dim3(chunks, G + (H + 3) / 4), 256, 0, stream>>>(a, p, S);
+        ssd_stream_kernel<<<dim3(vdim / 16, H, S), 256, 0, stream>>>(a, p);
+        LLE_RETURN_LAUNCH_STATUS();
+    }
     const bool wide = n % 4 == 0 && vdim % 4 == 0;  // (then CC and every column offset are multiples of 4 too)
     const dim3 grid(S * pieces, H / heads_a_group);
     auto go = [&](auto kernel, size_t lds) {

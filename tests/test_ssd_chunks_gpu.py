@@ -32,3 +32,46 @@ def test_heads_of_a_workgroup(together, H, G, vdim, n, monkeypatch):
     # sums of at most 64 tokens and n <= 132 channels, in 32 bits: under 64 roundings of the largest result
     close(got[together][0], want, 64 * 2**-24 * max(1.0, float(want.abs().max())))
     close(got[together][1], state, 64 * 2**-24 * max(1.0, float(state.abs().max())))
+
+
+@pytest.mark.parametrize("H,G,vdim,q_lens", [(2, 1, 16, [33]), (3, 3, 48, [64]), (4, 2, 64, [65, 1, 127]), (4, 1, 80, [128, 32, 129, 7]), (6, 2, 32, [400]),
+                                             (64, 2, 64, [1, 193])])
+def test_chunks_one_after_the_other(H, G, vdim, q_lens, monkeypatch):
+    """States of 128 channels kept in registers: the shortest request of one chunk, whole last chunks and ones of one token, beside
+    requests that are walked; the oracle's rows and states, and those of the chunks side by side."""
+    o = ops()
+    c, dt_in, dt_bias, a_log, D, wide, seq_slots, cu = ssd_case(H, G, vdim, 128, q_lens)
+    args, got = (c, dt_in, dt_bias, a_log, D), {}
+    for streams in (True, False):
+        monkeypatch.setattr(o, "ssd_streams", lambda *a, s=streams: s)
+        state = wide.clone()
+        got[streams] = o.ssd_scan(*args, state, H, G, vdim, 128, seq_slots, cu, min(q_lens), max(q_lens)), state
+    state = wide.clone()
+    want = REF.ssd_scan(*args, state, H, G, vdim, 128, seq_slots, cu)
+    # sums of at most 64 tokens and 128 channels, in 32 bits: under 64 roundings of the largest result
+    for rows, states in got.values():
+        close(rows, want, 64 * 2**-24 * max(1.0, float(want.abs().max())))
+        close(states, state, 64 * 2**-24 * max(1.0, float(state.abs().max())))
+    behind = H * vdim * 128
+    assert torch.equal(got[True][1][:, behind:], wide[:, behind:])  # what lies behind the matrices stays
+    untouched = [i for i in range(wide.shape[0]) if i not in seq_slots.tolist()]
+    assert torch.equal(got[True][1][untouched], wide[untouched])
+
+
+def test_a_steep_drop_inside_a_chunk():
+    """Decays that end a state at once, and none at all: later tokens' exponents never rise above zero, what is forgotten is gone."""
+    o = ops()
+    H, G, vdim, N = 2, 1, 16, 150
+    c = torch.randn((N, H * vdim + 2 * 128), generator=torch.Generator().manual_seed(2)).cuda()
+    dt_in = torch.zeros((N, H)).cuda()
+    dt_in[70, 0] = 2000.0  # head 0: the decay of token 70 is exp(-2000)
+    dt_in[:, 1] = -60.0  # head 1: no step at all
+    zeros, D = torch.zeros(H).cuda(), torch.zeros(H).cuda()
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    state = torch.ones((2, H * vdim * 128)).cuda()
+    got = o.ssd_scan(c, dt_in, zeros, zeros, D, state, H, G, vdim, 128, ints([1]), ints([0, N]), N, N)
+    want_state = torch.ones((2, H * vdim * 128)).cuda()
+    want = REF.ssd_scan(c, dt_in, zeros, zeros, D, want_state, H, G, vdim, 128, ints([1]), ints([0, N]))
+    scale = float(want.abs().max())
+    assert torch.isfinite(got).all() and (got - want).abs().max() < 128 * 2**-24 * scale
+    assert (state - want_state).abs().max() < 64 * 2**-24 * float(want_state.abs().max())
