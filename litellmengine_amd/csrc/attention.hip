@@ -31,6 +31,8 @@
 //    all keys up to each row's own position; the four wavefronts of a workgroup
 //    share the K/V tiles through LDS, two workgroups share a CU.
 #include "common.h"
+#include "lds.h"
+#include "parts.h"
 #include <type_traits>
 #include <mutex>
 
@@ -1575,6 +1577,7 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
 //     wavefronts take every fourth 16-key step and are merged through LDS (decoding);
 //   * any other: a workgroup takes 64 rows, each wavefront a tile of 16 of them and all keys
 //     that its rows see; or (TILES == 2, heads of 64 and 128) 128 rows, two tiles a wavefront.
+//     (Many rows of heads of 128: split_f32_attention_kernel.)
 // What bounds it: the matrix instruction (32 cycles for 1024 products) where the loads keep up.
 // Every wavefront loads K and V for itself, 16 KB a step of 16 keys of 128 elements, and one tile
 // multiplies them in 2048 cycles; two tiles halve the bytes and leave two independent chains of
@@ -1594,17 +1597,20 @@ __global__ __launch_bounds__(PRE_WAVES* LLE_WAVE, DK <= 6 ? 2 : 1) void mfma_pre
 // ---------------------------------------------------------------------------------
 #define F32_WAVES 4
 #define F32_KEYS 16
+// split, yb: which of the key splits, which of the request's row blocks.  given_end >= 0: the rows of a request with more than 16 take the 16-key
+// steps given_begin .. given_end - 1 in the place of the split's; `skip`, of each lane: its row of tile t stays as it is in `out` and the
+// workspaces.
 template <int DQ, int TILES, bool KEEP, bool CAP>
-__global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES == 2 ? 2 : 3) void mfma_f32_attention_kernel(
+__device__ __forceinline__ void f32_attention_rows(
     const float* __restrict__ q, const float* __restrict__ kv_layer, const int32_t* __restrict__ block_tables,
     const int32_t* __restrict__ seq_slots, const int32_t* __restrict__ cu_tokens,
     const int32_t* __restrict__ kv_lens, float* __restrict__ out, float* __restrict__ ws_o,
-    float* __restrict__ ws_ml, int nsplit, int nq, int nkv, int P, int64_t page_stride, int max_pages, int window,
-    int keep_first, float scale_log2, const float* __restrict__ sinks, float cap_log2, int paired) {
+    float* __restrict__ ws_ml, int nsplit, int parts, int nq, int nkv, int P, int64_t page_stride, int max_pages, int window,
+    int keep_first, float scale_log2, const float* __restrict__ sinks, float cap_log2, int paired, float* smem, int split, int yb, int given_begin,
+    int given_end, uint32_t skip) {
     static_assert(TILES == 1 || !KEEP, "kept first keys: one tile");
     constexpr int D = 16 * DQ, ROWS = 16 * TILES;
-    extern __shared__ float smem[];  // [waves][16][D] acc, then [waves][16] m, [waves][16] l
-    float* s_o = smem;
+    float* s_o = smem;  // [waves][16][D] acc, then [waves][16] m, [waves][16] l
     float* s_m = smem + F32_WAVES * 16 * D;
     float* s_l = s_m + F32_WAVES * 16;
     const int s = blockIdx.z, kvh = blockIdx.x;
@@ -1615,9 +1621,6 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     if (nrows <= 0) return;
     const int kv_len = kv_lens[s];
     const int past = kv_len - q_len;
-    const int row_blocks = gridDim.y / nsplit;
-    const int split = blockIdx.y / row_blocks;
-    int yb = blockIdx.y % row_blocks;
     const bool few = nrows <= 16;  // the same for the whole workgroup
     const int wave = threadIdx.x / LLE_WAVE, lane = threadIdx.x % LLE_WAVE;
     const int c = lane / 16, r16 = lane % 16;
@@ -1680,6 +1683,9 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
         if (few) {
             step_begin += wave;
             step_stride = F32_WAVES;
+        } else if (given_end >= 0) {
+            step_begin = max(first[0], given_begin);
+            step_end = min(TILES == 2 && end[TILES - 1] > 0 ? end[TILES - 1] : end[0], given_end);
         }
     }
     f32x4 o[TILES][DQ];
@@ -1824,8 +1830,8 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
     if (!few) {  // every wavefront writes the rows of its own tiles
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            if (!exists[t]) continue;
-            if (nsplit > 1) {
+            if (!exists[t] || (skip >> t & 1)) continue;
+            if (parts > 1) {
                 float* po = ws_o + (head_row[t] * nsplit + split) * D;
 #pragma unroll
                 for (int n = 0; n < DQ; ++n) *(f32x4*)(po + 16 * n + 4 * c) = o[t][n];
@@ -1878,6 +1884,378 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
             }
         }
     }
+}
+
+template <int DQ, int TILES, bool KEEP, bool CAP>
+__global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES == 2 ? 2 : 3) void mfma_f32_attention_kernel(
+    const float* __restrict__ q, const float* __restrict__ kv_layer, const int32_t* __restrict__ block_tables,
+    const int32_t* __restrict__ seq_slots, const int32_t* __restrict__ cu_tokens,
+    const int32_t* __restrict__ kv_lens, float* __restrict__ out, float* __restrict__ ws_o,
+    float* __restrict__ ws_ml, int nsplit, int nq, int nkv, int P, int64_t page_stride, int max_pages, int window,
+    int keep_first, float scale_log2, const float* __restrict__ sinks, float cap_log2, int paired) {
+    extern __shared__ float smem[];
+    const int row_blocks = gridDim.y / nsplit;
+    f32_attention_rows<DQ, TILES, KEEP, CAP>(q, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, out, ws_o, ws_ml, nsplit, nsplit, nq, nkv, P, page_stride, max_pages, window,
+                                             keep_first, scale_log2, sinks, cap_log2, paired, smem, blockIdx.y / row_blocks, blockIdx.y % row_blocks, 0, -1, 0);
+}
+
+// ---------------------------------------------------------------------------------
+// float32 attention of many rows on the bfloat16 matrix cores without losing a bit of an operand: q, K, V and the probabilities as three bfloat16
+// parts each (parts.h), both products in six of the bfloat16 instruction (gemm_f32.hip says what that keeps), scores, maxima and sums in
+// float32.  The float32 instruction bounds mfma_f32_attention_kernel (8192 cycles for 32 rows and 32 keys of 128 elements, 3072 here).
+// A workgroup takes 128 rows of a request, a wavefront 32, whose first two parts of q stay in its registers and the third in its own piece of LDS.
+// 32 keys a step: K and V^T are loaded once a workgroup, split once and laid out in LDS as three planes each in the layouts of
+// mfma_prefill_kernel; K of the next step is on its way while this one's scores are made, V of it under the product with the values.  80 KB
+// and 256 registers a lane: two workgroups a CU.  Requests of at most 16 rows, and rows that come out not finite (an infinity has no parts),
+// are f32_attention_rows'.
+// What bounds it: matrix cores busy 0.53 of the time and the other vector instructions, half of them splitting, most of the rest (4096 tokens; they
+// hardly run beside each other, whatever the priorities: matrix instructions first made it 720 us); below two workgroups a CU a wavefront's
+// own chain, 3.7 us a step.  32 / 8 heads of 128, the other kernel -> this one: a prompt of 512 / 1024 / 2048 / 4096 tokens 55 -> 40, 116 -> 78,
+// 385 -> 246, 1375 -> 700 us; 300 tokens behind 4000 231 -> 131, 1000 behind 5000 914 -> 477, 512 behind 2048 beside 20 decoded tokens
+// 468 -> 183.  Error against 64 bits (1024 tokens) 3.9e-7 -> 2.7e-7: fewer roundings of a sum.
+// Tried: two sums in turn in place of four (2048 tokens + 15 us), all of q in registers (nothing can be asked of LDS ahead; + 4 %), whole
+// blocks that fill the chip in parts (2048 tokens 252 to 265).
+// ---------------------------------------------------------------------------------
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#define SA_KEYS 32
+#define SA_PLANE 8192  // bytes of a part of a step's K or V
+#define SA_LDS (10 * SA_PLANE)  // three of each, and the third parts of q
+__global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_kernel(
+    const float* __restrict__ q, const float* __restrict__ kv_layer, const int32_t* __restrict__ block_tables,
+    const int32_t* __restrict__ seq_slots, const int32_t* __restrict__ cu_tokens,
+    const int32_t* __restrict__ kv_lens, float* __restrict__ out, float* __restrict__ ws_o,
+    float* __restrict__ ws_ml, int nsplit, int nq, int nkv, int P, int64_t page_stride, int max_pages, int window,
+    float scale_log2, const float* __restrict__ sinks, int part_steps) {
+    constexpr int D = 128, KS = D / 32, N = D / 16, TILES = 2, ROWS = 32 * F32_WAVES;
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    unsigned char* lds = (unsigned char*)smem;
+    const int s = blockIdx.z, kvh = blockIdx.x, G = nq / nkv;
+    const int q_start = cu_tokens[s], q_len = cu_tokens[s + 1] - q_start, nrows = q_len * G;
+    if (nrows <= 0) return;
+    const bool few = nrows <= 16;
+    int split = blockIdx.y, place = blockIdx.y, parts = nsplit;  // (of few rows: a part each)
+    if (few && split >= nsplit) return;
+    int given_begin = 0, given_end = -1;
+    uint32_t skip = 0;
+    if (!few) {
+        const int own = (nrows + ROWS - 1) / ROWS;
+        const int past = kv_lens[s] - q_len;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE), lane = threadIdx.x % LLE_WAVE, c = lane / 16, r16 = lane % 16;
+        // the keys that a block of rows sees: place 0 is the last block, whose rows see the most
+        auto keys_of = [&](int at_place, int& lo, int& hi) {
+            const int r0 = (own - 1 - at_place) * ROWS;
+            hi = past + (min(nrows, r0 + ROWS) - 1) / G, lo = window > 0 ? max(0, past + r0 / G - window + 1) : 0;
+            return hi / SA_KEYS + 1 - lo / SA_KEYS;  // steps
+        };
+        int hi, lo;
+        if (nsplit == 1) {
+            if (place >= own) return;
+            parts = 1;
+            split = 0;
+        } else {
+            // Which block's part this workgroup is: of the blocks with as many parts as there can be the one with the longest, of those with a part less
+            // the one with the longest, and so on, then the second of each kind (rows of one prompt: as many blocks of each), so that the parts
+            // come by falling length, and a workgroup without work behind all others: the dies deal workgroups out to their engines in turn,
+            // and with an idle one after every other half of the engines had nothing to do (4096 tokens of 32 / 8 heads 720 -> 1830 us).
+            const int kind = (own + nsplit - 1) / nsplit;
+            int before = 0, found = -1;
+            for (int i0 = 0; i0 < kind * nsplit && found < 0; i0 += LLE_WAVE) {
+                const int i = i0 + lane, p = i % nsplit * kind + i / nsplit;
+                const bool there = i < kind * nsplit && p < own;
+                const int n = there ? min(nsplit, (keys_of(p, lo, hi) + part_steps - 1) / part_steps) : 0;
+                int sum = n;
+#pragma unroll
+                for (int d = 1; d < LLE_WAVE; d *= 2) {
+                    const int up = __shfl_up(sum, d);
+                    if (lane >= d) sum += up;
+                }
+                const uint64_t past_it = __ballot(before + sum > (int)blockIdx.y);
+                if (past_it) {
+                    const int at = __builtin_ctzll(past_it);
+                    found = __builtin_amdgcn_readlane(p, at), parts = __builtin_amdgcn_readlane(n, at);
+                    split = (int)blockIdx.y - before - (__builtin_amdgcn_readlane(sum, at) - parts);
+                }
+                before += __builtin_amdgcn_readlane(sum, LLE_WAVE - 1);
+            }
+            if (found < 0) return;
+            place = found;
+        }
+        const int steps = keys_of(place, lo, hi);
+        const int block0 = (own - 1 - place) * ROWS, row0 = block0 + 32 * wave;
+        const int32_t* table = block_tables + (int64_t)seq_slots[s] * max_pages;
+        // A block of few steps is in fewer parts than there can be: its first part says so of the others, and a part that is all writes the result.
+        if (split == 0 && parts < nsplit) {
+            for (int i = threadIdx.x; i < ROWS * nsplit; i += F32_WAVES * LLE_WAVE) {
+                const int row = block0 + i / nsplit, k = i % nsplit;
+                if (row >= nrows || (k < parts && parts > 1)) continue;
+                float* ml = ws_ml + (((int64_t)(q_start + row / G) * nq + kvh * G + row % G) * nsplit + k) * 2;
+                ml[0] = NEG_BIG;
+                ml[1] = k < parts ? -1.f : 0.f;  // (below zero: the row is in `out`)
+            }
+        }
+        const int first = lo / SA_KEYS;
+        const int per_part = (steps + parts - 1) / parts, begin = first + split * per_part, end = min(first + steps, begin + per_part);
+        given_begin = 2 * begin, given_end = max(0, 2 * end);
+        // those that the wavefront's rows see, and those that all of them see
+        const bool has_rows = row0 < nrows;
+        const int w_hi = has_rows ? past + (min(nrows, row0 + 32) - 1) / G : -1, w_lo = window > 0 ? max(0, past + row0 / G - window + 1) : 0;
+        const int all_hi = past + row0 / G, all_lo = window > 0 ? max(0, w_hi - window + 1) : 0;
+        bool exists[TILES];
+        int pos[TILES], low[TILES];
+        int64_t head_row[TILES];
+        u32x4 qp[TILES][KS][2];
+        unsigned char* third = lds + 6 * SA_PLANE + (wave * LLE_WAVE + lane) * 16;  // each lane's own, [tile][32 elements of q]
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const int row = row0 + 16 * t + r16;
+            exists[t] = row < nrows;
+            const int tok = exists[t] ? row / G : 0, g = exists[t] ? row - tok * G : 0;
+            head_row[t] = (int64_t)(q_start + tok) * nq + kvh * G + g;
+            pos[t] = exists[t] ? past + tok : -1;
+            low[t] = exists[t] && window > 0 ? max(0, pos[t] - window + 1) : 0;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const float* at = q + head_row[t] * D + 32 * ks + 8 * c;
+                const f32x4 a = *(const f32x4*)at, b = *(const f32x4*)(at + 4);
+                u32x4 last;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    uint32_t p1, p2, p3;
+                    split2(h < 2 ? a[2 * h] : b[2 * h - 4], h < 2 ? a[2 * h + 1] : b[2 * h - 3], p1, p2, p3);
+                    qp[t][ks][0][h] = p1, qp[t][ks][1][h] = p2, last[h] = p3;
+                }
+                *(u32x4*)(third + (t * KS + ks) * (F32_WAVES * LLE_WAVE * 16)) = last;
+            }
+        }
+        // the copies: of K a thread takes pieces of eight elements of one key, of V^T pieces of eight keys of one element
+        const PageSize pages(P);
+        const int kr = threadIdx.x / 8, kp = threadIdx.x % 8, ve = threadIdx.x / 4, vp = threadIdx.x % 4;
+        auto place_of = [&](int step, int half, int& off) {  // (of a half that no row sees, whose page may be gone: the other half's)
+            int j = step * SA_KEYS + 16 * half;
+            j = j > hi ? j - 16 : j + 15 < lo ? j + 16 : j;
+            const int p = pages.of(j);
+            off = j - p * P;
+            return kv_layer + (int64_t)table[p] * page_stride;
+        };
+        f32x4 kreg[2][2], vreg[2][2];
+        auto load_k = [&](int step) {
+            int off;
+            const float* at = place_of(step, wave / 2, off);
+            at += ((int64_t)kvh * P + off + kr % 16) * D + 8 * kp;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) kreg[i][0] = *(const f32x4*)(at + 64 * i), kreg[i][1] = *(const f32x4*)(at + 64 * i + 4);
+        };
+        auto load_v = [&](int step) {
+            int off0, off1;
+            const float *at0 = place_of(step, 0, off0), *at1 = place_of(step, 1, off1);
+            const float* at = (vp < 2 ? at0 + off0 : at1 + off1) + (((int64_t)nkv + kvh) * D + ve) * P + 8 * (vp % 2);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) vreg[i][0] = *(const f32x4*)(at + (int64_t)64 * i * P), vreg[i][1] = *(const f32x4*)(at + (int64_t)64 * i * P + 4);
+        };
+        auto put = [&](unsigned char* at, const f32x4 (&v)[2]) {
+            u32x4 part[3];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                uint32_t p1, p2, p3;
+                split2(v[h / 2][2 * (h % 2)], v[h / 2][2 * (h % 2) + 1], p1, p2, p3);
+                part[0][h] = p1, part[1][h] = p2, part[2][h] = p3;
+            }
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *(u32x4*)(at + p * SA_PLANE) = part[p];
+        };
+        auto store_k = [&]() {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) put(lds + kr * 256 + ((kp + 8 * i) ^ K_SWIZZLE(kr, 4)) * 16, kreg[i]);
+        };
+        auto store_v = [&](int step) {
+            const int j0 = step * SA_KEYS + 8 * vp;
+            if (step * SA_KEYS < lo || step * SA_KEYS + SA_KEYS - 1 > hi) {  // as drop_values
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) vreg[i][e / 4][e % 4] = j0 + e < lo || j0 + e > hi ? 0.f : vreg[i][e / 4][e % 4];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) put(lds + 3 * SA_PLANE + (ve + 64 * i) * 64 + (vp ^ V_SWIZZLE(ve)) * 16, vreg[i]);
+        };
+        auto meet = [&]() {  // what every wavefront has put into LDS is there, and what it has asked of it has come
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        f32x4 o[TILES][N];
+        float m[TILES], l[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int n = 0; n < N; ++n) o[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+            m[t] = NEG_BIG;
+            l[t] = 0.f;
+        }
+        constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};  // the smallest products first
+        const int key[2] = {KEY_OF_ROW(r16, 0), KEY_OF_ROW(r16, 1)};
+        const int ksw[2] = {K_SWIZZLE(key[0], 4), K_SWIZZLE(key[1], 4)};
+        const unsigned char* v_at = lds + 3 * SA_PLANE + r16 * 64 + (c ^ V_SWIZZLE(r16)) * 16;
+        if (begin < end) {
+            load_k(begin);
+            load_v(begin);
+            store_k();
+        }
+        for (int step = begin; step < end; ++step) {
+            const bool active = step * SA_KEYS <= w_hi && step * SA_KEYS + SA_KEYS > w_lo;
+            meet();  // K of this step is there, V of the one before has been read
+            store_v(step);
+            if (step + 1 < end) load_k(step + 1);
+            u32x4 pp[TILES][3];
+            float alpha[TILES];
+            if (active) {
+                f32x4 sc[TILES][2];
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) sc[t][0] = sc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                bf16x8 a[2][2][3], q3[2][TILES];
+                auto read_k = [&](int ks, auto set) {
+                    constexpr int b = decltype(set)::value;
+#pragma unroll
+                    for (int x = 0; x < 2; ++x)
+#pragma unroll
+                        for (int p = 0; p < 3; ++p) a[b][x][p] = *(const bf16x8*)(lds + p * SA_PLANE + key[x] * 256 + ((4 * ks + c) ^ ksw[x]) * 16);
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t) q3[b][t] = *(const bf16x8*)(third + (t * KS + ks) * (F32_WAVES * LLE_WAVE * 16));
+                };
+                auto score_k = [&](int ks, auto set) {
+                    constexpr int b = decltype(set)::value;
+#pragma unroll
+                    for (int i = 0; i < 6; ++i)  // (four sums in turn: one after the other they wait for each other)
+#pragma unroll
+                        for (int x = 0; x < 2; ++x)
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t)
+                                sc[t][x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b][x][pa[i]], pb[i] == 2 ? q3[b][t] : __builtin_bit_cast(bf16x8, qp[t][ks][pb[i] == 2 ? 0 : pb[i]]), sc[t][x], 0, 0, 0);
+                };
+                using Set0 = std::integral_constant<int, 0>;
+                using Set1 = std::integral_constant<int, 1>;
+                read_k(0, Set0{});
+                read_k(1, Set1{});
+                score_k(0, Set0{});
+                __builtin_amdgcn_sched_barrier(0);
+                read_k(2, Set0{});
+                score_k(1, Set1{});
+                __builtin_amdgcn_sched_barrier(0);
+                read_k(3, Set1{});
+                score_k(2, Set0{});
+                __builtin_amdgcn_sched_barrier(0);
+                score_k(3, Set1{});
+                const bool masked = step * SA_KEYS + SA_KEYS - 1 > all_hi || step * SA_KEYS < all_lo;  // (the same for the whole wavefront)
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    float x[8];  // of keys 8 c + i
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] = sc[t][i / 4][i % 4] * scale_log2;
+                    if (masked) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const int j = step * SA_KEYS + 8 * c + i;
+                            x[i] = j < low[t] || j > pos[t] ? NEG_BIG : x[i];
+                        }
+                    }
+                    float top = x[0];
+#pragma unroll
+                    for (int i = 1; i < 8; ++i) top = fmaxf(top, x[i]);
+                    const float new_m = fmaxf(m[t], column_max(top));
+                    const float base = new_m <= NEG_BIG ? 0.f : new_m;  // (a row that has seen no key: as in f32_attention_rows)
+                    alpha[t] = exp2f(m[t] - base);
+                    m[t] = new_m;
+                    float sum[2] = {0.f, 0.f};
+#pragma unroll
+                    for (int h = 0; h < 4; ++h) {
+                        const float a = __builtin_amdgcn_exp2f(x[2 * h] - base), b = __builtin_amdgcn_exp2f(x[2 * h + 1] - base);
+                        sum[0] += a, sum[1] += b;
+                        uint32_t p1, p2, p3;
+                        split2(a, b, p1, p2, p3);
+                        pp[t][0][h] = p1, pp[t][1][h] = p2, pp[t][2][h] = p3;
+                    }
+                    l[t] = l[t] * alpha[t] + (sum[0] + sum[1]);
+                }
+            }
+            meet();  // V of this step is there, K has been read
+            if (step + 1 < end) {
+                store_k();
+                load_v(step + 1);
+            }
+            if (active) {
+                if (!__all(alpha[0] == 1.f && alpha[1] == 1.f)) {
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                        for (int n = 0; n < N; ++n) o[t][n] *= alpha[t];
+                }
+                bf16x8 a[2][2][3];
+                auto read_v = [&](int n, auto set) {
+                    constexpr int b = decltype(set)::value;
+#pragma unroll
+                    for (int x = 0; x < 2; ++x)
+#pragma unroll
+                        for (int p = 0; p < 3; ++p) a[b][x][p] = *(const bf16x8*)(v_at + p * SA_PLANE + (n + x) * 1024);
+                };
+                auto add_v = [&](auto at, auto set) {
+                    constexpr int n = decltype(at)::value, b = decltype(set)::value;
+#pragma unroll
+                    for (int i = 0; i < 6; ++i)
+#pragma unroll
+                        for (int x = 0; x < 2; ++x)
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t)
+                                o[t][n + x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b][x][pa[i]], __builtin_bit_cast(bf16x8, pp[t][pb[i]]), o[t][n + x], 0, 0, 0);
+                };
+                using Set0 = std::integral_constant<int, 0>;
+                using Set1 = std::integral_constant<int, 1>;
+                read_v(0, Set0{});
+                read_v(2, Set1{});
+                add_v(std::integral_constant<int, 0>{}, Set0{});
+                __builtin_amdgcn_sched_barrier(0);
+                read_v(4, Set0{});
+                add_v(std::integral_constant<int, 2>{}, Set1{});
+                __builtin_amdgcn_sched_barrier(0);
+                read_v(6, Set1{});
+                add_v(std::integral_constant<int, 4>{}, Set0{});
+                __builtin_amdgcn_sched_barrier(0);
+                add_v(std::integral_constant<int, 6>{}, Set1{});
+            }
+        }
+        bool again = false;  // a row of the wavefront is not finite
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            l[t] = column_sum(l[t]);
+            float sizes = fabsf(l[t]);
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sizes = fmaxf(sizes, o[t][n][e] == o[t][n][e] ? fabsf(o[t][n][e]) : INFINITY);
+            const uint64_t odd = __ballot(exists[t] && !(sizes < INFINITY && l[t] == l[t]));  // (a row is four lanes)
+            const bool row_odd = (odd >> r16 | odd >> (r16 + 16) | odd >> (r16 + 32) | odd >> (r16 + 48)) & 1;
+            again = again || odd != 0;
+            if (!exists[t] || row_odd) continue;
+            skip |= 1u << t;
+            if (parts > 1) {
+                float* po = ws_o + (head_row[t] * nsplit + split) * D;
+#pragma unroll
+                for (int n = 0; n < N; ++n) *(f32x4*)(po + 16 * n + 4 * c) = o[t][n];
+                if (c == 0) {
+                    ws_ml[(head_row[t] * nsplit + split) * 2] = m[t];
+                    ws_ml[(head_row[t] * nsplit + split) * 2 + 1] = l[t];
+                }
+                continue;
+            }
+            // (a sink: a place in the sum without a value)
+            const float sum = sinks ? l[t] + exp2f(sinks[head_row[t] % nq] * 1.44269504088896340736f - m[t]) : l[t];
+            const float inv = 1.0f / sum;
+#pragma unroll
+            for (int n = 0; n < N; ++n) *(f32x4*)(out + head_row[t] * D + 16 * n + 4 * c) = o[t][n] * inv;
+        }
+        if (!again) return;
+    }
+    f32_attention_rows<8, 2, false, false>(q, kv_layer, block_tables, seq_slots, cu_tokens, kv_lens, out, ws_o, ws_ml, nsplit, parts, nq, nkv, P, page_stride,
+                                           max_pages, window, 0, scale_log2, sinks, 0.f, 0, smem, split, few ? 0 : place, given_begin, given_end, skip);
 }
 
 // A q or k head of a raw float32 projection in mfma_f32_attention_kernel's layout: lane (c, r) holds elements 16 i + 4 c .. + 3,
@@ -2100,7 +2478,8 @@ __global__ __launch_bounds__((SHORT_F32_WAVES + 1) * LLE_WAVE) void short_decode
     }
 }
 
-// merges the key splits of the kernel above: grid = (tokens, q heads), one wavefront each
+// merges the key splits of the kernels above: grid = (tokens, q heads), one wavefront each.  PARTS: split_f32_attention_kernel's, whose rows may
+// have fewer parts than nsplit, or none.
 __global__ __launch_bounds__(LLE_WAVE) void f32_combine_kernel(const float* __restrict__ ws_o,
                                                                const float* __restrict__ ws_ml, int nsplit,
                                                                float* __restrict__ out, int nq, int D,
@@ -2124,10 +2503,42 @@ __global__ __launch_bounds__(LLE_WAVE) void f32_combine_kernel(const float* __re
     }
 }
 
+// The same of split_f32_attention_kernel, whose rows may have fewer parts than nsplit, or be in `out` already: rows of 128, one a wavefront, two
+// neighbouring elements a lane.
+__global__ __launch_bounds__(256) void split_f32_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, int nsplit,
+                                                                float* __restrict__ out, int64_t rows, int nq, const float* __restrict__ sinks) {
+    const int64_t head_row = (int64_t)blockIdx.x * 4 + threadIdx.x / LLE_WAVE;
+    const int lane = threadIdx.x % LLE_WAVE;
+    if (head_row >= rows) return;
+    const float2 ml = *(const float2*)(ws_ml + (head_row * nsplit + min(lane, nsplit - 1)) * 2);
+    const float m = lane < nsplit ? ml.x : NEG_BIG, l = lane < nsplit ? ml.y : 0.f;
+    const uint64_t some = __ballot(l != 0.f);  // (behind the last of them there may be nothing written)
+    if (some == 0 || (__ballot(l < 0.f) & 1)) return;
+    const int held = 64 - __builtin_clzll(some);
+    const float big = wave_max(m);
+    const float f = exp2f(m - big);
+    float den = wave_sum(l * f);
+    if (sinks) den += exp2f(sinks[head_row % nq] * 1.44269504088896340736f - big);
+    const float* o = ws_o + head_row * nsplit * 128 + 2 * lane;
+    float2 num = {0.f, 0.f};
+    for (int k0 = 0; k0 < held; k0 += 4) {
+        float2 part[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[j] = *(const float2*)(o + (int64_t)min(k0 + j, held - 1) * 128);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float fk = __shfl(f, k0 + j);
+            if (k0 + j < held) num.x += part[j].x * fk, num.y += part[j].y * fk;
+        }
+    }
+    *(float2*)(out + head_row * 128 + 2 * lane) = float2{num.x / den, num.y / den};
+}
+
 // float32, head_dim a multiple of 16 (<= 256), page size a multiple of 16.  `row_blocks`: the
 // most 64-row blocks that a request of this batch has (1 when every request has at most 16
 // rows); with nsplit > 1 the workspaces ws_o [N * nq * nsplit * d] and ws_ml [N * nq * nsplit * 2]
-// floats are needed (nsplit <= 64).
+// floats are needed (nsplit <= 64).  tiles 3: split_f32_attention_kernel, heads of 128; `row_blocks` then the workgroups for the parts of a request's
+// blocks, `paired` the most steps of 32 keys of a part, nsplit the most parts of a block.
 extern "C" int lle_paged_attention_mfma_f32(const void* q, const void* kv_layer, const void* block_tables,
                                             const void* seq_slots, const void* cu_tokens, const void* kv_lens,
                                             void* out, void* ws_o, void* ws_ml, int N, int S, int nq, int nkv, int d,
@@ -2135,18 +2546,19 @@ extern "C" int lle_paged_attention_mfma_f32(const void* q, const void* kv_layer,
                                             int keep_first, float scale, int row_blocks, int tiles, int paired, int nsplit,
                                             const void* sinks, float softcap, hipStream_t stream) {
     if (N <= 0) return 0;
-    if (tiles < 1 || tiles > 2 || (tiles == 2 && ((d != 64 && d != 128) || keep_first > 0 || softcap > 0.f))) return (int)hipErrorInvalidValue;
-    if (d % 16 != 0 || d > 256 || d <= 0 || page_size % 16 != 0 || nq % nkv != 0) return (int)hipErrorInvalidValue;
-    if (S > 65535 || nkv <= 0 || row_blocks < 1 || nsplit < 1 || nsplit > 64 || (int64_t)row_blocks * nsplit > 65535)
+    if (tiles < 1 || tiles > 3 || (tiles > 1 && ((d != 64 && d != 128) || keep_first > 0 || softcap > 0.f)) || (tiles == 3 && (d != 128 || paired < 1)))
         return (int)hipErrorInvalidValue;
+    if (d % 16 != 0 || d > 256 || d <= 0 || page_size % 16 != 0 || nq % nkv != 0) return (int)hipErrorInvalidValue;
+    const int64_t grid_y = tiles == 3 ? row_blocks : (int64_t)row_blocks * nsplit;
+    if (S > 65535 || nkv <= 0 || row_blocks < 1 || nsplit < 1 || nsplit > 64 || grid_y > 65535) return (int)hipErrorInvalidValue;
     if (nsplit > 1 && (!ws_o || !ws_ml)) return (int)hipErrorInvalidValue;
     if (keep_first < 0 || (keep_first > 0 && window <= 0)) return (int)hipErrorInvalidValue;
     if (softcap < 0.f || (softcap > 0.f && keep_first > 0)) return (int)hipErrorInvalidValue;
     // with a cap: the factor that tanh's argument gets, and the cap in the base-2 domain
     const float scale_log2 = softcap > 0.f ? scale / softcap : scale * 1.44269504088896340736f;
     const float cap_log2 = softcap * 1.44269504088896340736f;
-    const dim3 grid(nkv, row_blocks * nsplit, S);
-    const size_t smem = (size_t)(F32_WAVES * 16 * d + 2 * F32_WAVES * 16) * sizeof(float);
+    const dim3 grid(nkv, (int)grid_y, S);
+    const size_t smem = tiles == 3 ? SA_LDS : (size_t)(F32_WAVES * 16 * d + 2 * F32_WAVES * 16) * sizeof(float);
     auto launch = [&](auto kernel) {
         if (smem > 64 * 1024) {
             const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -2171,14 +2583,27 @@ extern "C" int lle_paged_attention_mfma_f32(const void* q, const void* kv_layer,
                    : softcap > 0.f ? launch(mfma_f32_attention_kernel<DQV, 1, false, true>)   \
                                    : launch(mfma_f32_attention_kernel<DQV, 1, false, false>); \
         break;
-    switch (d / 16) {
+    if (tiles == 3) {
+        static std::atomic<uint64_t> granted{0};
+        const hipError_t e = lle_grant_lds((const void*)split_f32_attention_kernel, SA_LDS, granted);
+        if (e != hipSuccess) return (int)e;
+        split_f32_attention_kernel<<<grid, F32_WAVES * LLE_WAVE, smem, stream>>>(
+            (const float*)q, (const float*)kv_layer, (const int32_t*)block_tables, (const int32_t*)seq_slots, (const int32_t*)cu_tokens,
+            (const int32_t*)kv_lens, (float*)out, (float*)ws_o, (float*)ws_ml, nsplit, nq, nkv, page_size, page_stride, max_pages, window,
+            scale_log2, (const float*)sinks, paired);
+        launched = hipGetLastError();
+    } else switch (d / 16) {
         LLE_F32_CASE(1) LLE_F32_CASE(2) LLE_F32_CASE(3) LLE_F32_CASE(4) LLE_F32_CASE(5) LLE_F32_CASE(6)
         LLE_F32_CASE(7) LLE_F32_CASE(8) LLE_F32_CASE(9) LLE_F32_CASE(10) LLE_F32_CASE(11) LLE_F32_CASE(12)
         LLE_F32_CASE(13) LLE_F32_CASE(14) LLE_F32_CASE(15) LLE_F32_CASE(16)
     }
 #undef LLE_F32_CASE
     if (launched != hipSuccess) return (int)launched;
-    if (nsplit > 1)
+    const int64_t out_rows = (int64_t)N * nq;
+    if (nsplit > 1 && tiles == 3)
+        split_f32_combine_kernel<<<(int)((out_rows + 3) / 4), 256, 0, stream>>>((const float*)ws_o, (const float*)ws_ml, nsplit, (float*)out, out_rows,
+                                                                                nq, (const float*)sinks);
+    else if (nsplit > 1)
         f32_combine_kernel<<<dim3(N, nq), LLE_WAVE, 0, stream>>>((const float*)ws_o, (const float*)ws_ml, nsplit,
                                                                  (float*)out, nq, d, (const float*)sinks);
     return (int)hipGetLastError();

@@ -54,7 +54,8 @@ HEADERS = ["common.h"]
 OWN_HEADERS: Dict[str, List[str]] = {
     "sampling": ["sampling.h"],
     "gemm": ["lds.h"],
-    "gemm_f32": ["lds.h"],
+    "gemm_f32": ["lds.h", "parts.h"],
+    "attention": ["lds.h", "parts.h"],
     "gemm_tile": ["lds.h"],
     "gemm_wide": ["lds.h"],
     "gemm_rows": ["lds.h"],

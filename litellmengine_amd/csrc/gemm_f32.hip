@@ -6,6 +6,7 @@
 // rounding of a b.  The float32 matrix instruction does 157 TFLOP/s, the bfloat16 one 2500, a sixth of which is 417.
 #include "common.h"
 #include "lds.h"
+#include "parts.h"
 #include <math.h>
 
 LLE_DEFINE_ERROR_STRING()
@@ -17,20 +18,6 @@ typedef uint32_t su32x4 __attribute__((ext_vector_type(4)));
 
 #define SG_BK 32      // columns of K per step
 #define SG_PIECES 4   // 8-element pieces of a row of a step
-
-// two numbers as their three bfloat16 parts, packed
-__device__ __forceinline__ void split2(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
-    typedef bf16_t pair __attribute__((ext_vector_type(2)));
-    typedef float fpair __attribute__((ext_vector_type(2)));
-    auto pack = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(fpair{x, y}, pair)); };
-    p1 = pack(a, b);
-    a -= __builtin_bit_cast(float, p1 << 16);
-    b -= __builtin_bit_cast(float, p1 & 0xffff0000u);
-    p2 = pack(a, b);
-    a -= __builtin_bit_cast(float, p2 << 16);
-    b -= __builtin_bit_cast(float, p2 & 0xffff0000u);
-    p3 = pack(a, b);
-}
 
 // Tiles of 64 TM rows of A x 64 TN rows of B, four wavefronts of 32 TM x 32 TN.  A step of 32 columns is asked for while the
 // one before is multiplied, split in registers on its way to LDS (one buffer; two or more workgroups a CU fill each other's

@@ -865,12 +865,17 @@ class HipOps:
         group = nq // nkv
         if (q.dtype == torch.float32 and d % 16 == 0 and page_size % 16 == 0 and max_q_len > 0 and max_kv_len > 0
                 and S <= 65535 and not both and not self.force_generic_attention):
-            # float32 on the matrix cores (float32 operands, products and sums)
+            # float32 on the matrix cores (float32 operands, products and sums; many rows of 128: operands in three bfloat16 parts)
             rows = max_q_len * group
             span = min(max_kv_len, win + max_q_len) if win else max_kv_len
             tiles, paired, rounds = self.f32_attention_form(N, nq, nkv, d, keep == 0 and cap == 0.0, max_q_len, span)
-            row_blocks = 1 if rows <= 16 else -(-rows // (64 * tiles))
-            ns = self.f32_attention_splits(S, nkv, row_blocks, max_q_len, max_kv_len, win, rounds)
+            part_steps = self.f32_attention_part_steps(N, S, nq, nkv, d, keep == 0 and cap == 0.0, max_q_len, span)
+            if part_steps:
+                ns, row_blocks = self.f32_attention_parts(part_steps, rows, group, max_kv_len, span)
+                tiles, paired = 3, part_steps
+            else:
+                row_blocks = 1 if rows <= 16 else -(-rows // (64 * tiles))
+                ns = self.f32_attention_splits(S, nkv, row_blocks, max_q_len, max_kv_len, win, rounds)
             ws_o = ws_ml = None
             if ns > 1:
                 ws_o = _made((N * nq * ns * d,), dtype=torch.float32, device=q.device)
@@ -1128,6 +1133,36 @@ class HipOps:
             units = resident // 2
             return 1 if low <= units or (low <= resident and max_kv_len <= max_q_len and num_seqs <= 1) else 3
         return 1 if low <= resident else 2
+
+    def f32_attention_part_steps(self, N: int, S: int, nq: int, num_kv_heads: int, d: int, plain: bool, max_q_len: int, span: int) -> int:
+        """The most steps of 32 keys that a workgroup of the float32 kernel of many rows (operands in three bfloat16 parts, blocks of 128
+        rows, heads of 128) takes, or 0 where the float32 instruction's kernel stays.  Two workgroups a CU: as many steps as make one
+        round of all blocks' parts, each block having half a part less than whole ones on average, and a tenth more; whole blocks
+        where there are two a CU.  At 32 / 8 heads, the other kernel -> this one: prompts of 512 / 1024 / 2048 / 4096 tokens 55 -> 40, 116 -> 78,
+        385 -> 246, 1375 -> 700 us, 300 tokens behind 4000 231 -> 131, 1000 behind 5000 914 -> 477, 512 behind 2048 beside 20 decoded
+        tokens 468 -> 183.  Below two steps for every one of those workgroups, counted in whole blocks, a launch is the chain of one
+        workgroup, which is longer here: 200 tokens 23 / 28, eight prompts of 100 23 / 24, 16 tokens behind 6000 34 / 39; 64 behind 2000,
+        at the line, 40 / 38."""
+        group = nq // num_kv_heads
+        if not plain or d != 128 or max_q_len * group <= 16:
+            return 0
+        slots, length = 2 * self.compute_units(), (span - min(span, max_q_len) / 2) / 32
+        if num_kv_heads * (N - S) * group / 128 * length < 1.9 * slots:  # (a token of each request left out: those that decode have no more)
+            return 0
+        blocks = num_kv_heads * max(S, -(-N * group // 128))
+        if blocks >= slots:
+            return 1 << 20
+        return max(4, int(1.1 * blocks * length / (slots - blocks / 2)))
+
+    @staticmethod
+    def f32_attention_parts(part_steps: int, rows: int, group: int, max_kv_len: int, span: int) -> tuple:
+        """(the most parts of a block of 128 rows, workgroups enough for the parts of all blocks of any request) in parts of at most `part_steps`
+        steps of 32 keys (of equal parts where that makes more than 64).  A block's keys lie in one step more than they fill at most, and without a
+        window block j from the end sees at least j - 1 blocks' tokens less than the last one; every block may have a part that is not whole."""
+        steps, blocks = -(-min(span, max_kv_len) // 32) + 1, -(-rows // 128)
+        most = min(64, -(-steps // part_steps))
+        fewer = (128 // group) / 32 * (blocks - 1) * (blocks - 2) / 2 if span >= max_kv_len else 0.0
+        return most, max(1, min(blocks * most, int((blocks * (steps + 1) - fewer) / part_steps) + blocks + 1))
 
     def f32_attention_form(self, N: int, nq: int, num_kv_heads: int, d: int, plain: bool, max_q_len: int,
                            span: int) -> tuple:
