@@ -178,19 +178,23 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
 // writes one value element of 8 tokens, as one 16-byte store when those tokens sit in
 // consecutive slots of one page starting at a multiple of 8 (prompt portions do), else one by one.
 #define VW_TOKENS 16
-__device__ __forceinline__ void v_write_transposed_block(const bf16_t* __restrict__ qkv,
+#define VW_ROW(T, d) ((d) + (sizeof(T) == 2 ? 2 : 1))
+template <typename T>
+__device__ __forceinline__ void v_write_transposed_block(const T* __restrict__ qkv,
                                                          const int32_t* __restrict__ slots,
-                                                         bf16_t* __restrict__ kv_layer, int N, int nq, int nkv, int d,
+                                                         T* __restrict__ kv_layer, int N, int nq, int nkv, int d,
                                                          int page_size, int64_t page_stride, int t0, int kvh,
-                                                         bf16_t* tile /* [VW_TOKENS][d + 2] */, int* s_slot) {
+                                                         T* tile /* [VW_TOKENS][VW_ROW(T, d)] */, int* s_slot) {
+    constexpr int E = 16 / sizeof(T);  // elements of a load
+    typedef T vec __attribute__((ext_vector_type(E)));
     const int width = (nq + 2 * nkv) * d;
-    const int row = d + 2;
-    for (int idx = threadIdx.x; idx < VW_TOKENS * (d / 8); idx += blockDim.x) {
-        const int t = idx / (d / 8), ch = idx % (d / 8);
+    const int row = VW_ROW(T, d);
+    for (int idx = threadIdx.x; idx < VW_TOKENS * (d / E); idx += blockDim.x) {
+        const int t = idx / (d / E), ch = idx % (d / E);
         if (t0 + t < N) {
-            const rbf16x8 v = *(const rbf16x8*)(qkv + (int64_t)(t0 + t) * width + (int64_t)(nq + nkv + kvh) * d + 8 * ch);
+            const vec v = *(const vec*)(qkv + (int64_t)(t0 + t) * width + (int64_t)(nq + nkv + kvh) * d + E * ch);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) tile[t * row + 8 * ch + i] = v[i];
+            for (int i = 0; i < E; ++i) tile[t * row + E * ch + i] = v[i];
         }
     }
     if (threadIdx.x < VW_TOKENS) s_slot[threadIdx.x] = t0 + threadIdx.x < N ? slots[t0 + threadIdx.x] : -1;
@@ -204,10 +208,14 @@ __device__ __forceinline__ void v_write_transposed_block(const bf16_t* __restric
         if (run) {
             const int64_t page = first / page_size;
             const int off = first - (int)page * page_size;
-            rbf16x8 y;
+            T* dst = kv_layer + page * page_stride + ((int64_t)nkv + kvh) * page_size * d + (int64_t)e * page_size + off;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = tile[(8 * g + i) * row + e];
-            *(rbf16x8*)(kv_layer + page * page_stride + ((int64_t)nkv + kvh) * page_size * d + (int64_t)e * page_size + off) = y;
+            for (int h = 0; h < 8; h += E) {
+                vec y;
+#pragma unroll
+                for (int i = 0; i < E; ++i) y[i] = tile[(8 * g + h + i) * row + e];
+                *(vec*)(dst + h) = y;
+            }
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -337,6 +345,67 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_pair_kernel(
     }
 }
 
+// The first kernel's arithmetic, to the last bit, for float32 heads of 128 rotated whole and many tokens: a wavefront takes four heads of a
+// token at once, lane i elements i and i + 64, and behind them workgroups take the V heads as above.  A wavefront for every head was bound by
+// workgroups of one wavefront and by values stored one by one, 64 bytes apart: 2048 tokens of 16 / 8 heads 32.0 ->
+// 16.1 us, of 32 / 8 40.8 -> 20.8 (4.8 TB/s).
+#define QK_HEADS 4
+__global__ __launch_bounds__(256) void qk_norm_rope_write_f32_kernel(
+    const float* __restrict__ qkv, const int32_t* __restrict__ slots, const void* __restrict__ q_weight,
+    const void* __restrict__ k_weight, int weight_dtype, const float* __restrict__ cos_sin, float eps,
+    float* __restrict__ q_out, float* __restrict__ kv_layer, int nq, int nkv, int page_size, int64_t page_stride,
+    int write_kv, int head_groups, int64_t total_groups, int64_t head_blocks, int N) {
+    constexpr int d = 128, half = 64;
+    if ((int64_t)blockIdx.x >= head_blocks) {
+        __shared__ float tile[VW_TOKENS * VW_ROW(float, d)];
+        __shared__ int s_slot[VW_TOKENS];
+        const int vb = (int)(blockIdx.x - head_blocks);
+        v_write_transposed_block<float>(qkv, slots, kv_layer, N, nq, nkv, d, page_size, page_stride, (vb / nkv) * VW_TOKENS, vb % nkv, tile, s_slot);
+        return;
+    }
+    const int lane = threadIdx.x % LLE_WAVE;
+    const int64_t group = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / LLE_WAVE);
+    if (group >= total_groups) return;
+    const int64_t n = group / head_groups;
+    const int head0 = (int)(group - n * head_groups) * QK_HEADS, heads = nq + (write_kv ? nkv : 0);
+    const float* src = qkv + n * (nq + 2 * nkv) * d + lane;
+    const float2 cs = ((const float2*)cos_sin)[n * half + lane];
+    const int slot = write_kv ? slots[n] : -1;
+    float lo[QK_HEADS], hi[QK_HEADS];
+#pragma unroll
+    for (int h = 0; h < QK_HEADS; ++h) {
+        const int head = min(head0 + h, heads - 1);
+        lo[h] = src[(int64_t)head * d], hi[h] = src[(int64_t)head * d + half];
+    }
+#pragma unroll
+    for (int h = 0; h < QK_HEADS; ++h) {
+        const int head = head0 + h;
+        if (head >= heads) break;
+        const bool is_q = head < nq;
+        if (!is_q && slot < 0) break;
+        const void* w = is_q ? q_weight : k_weight;
+        float inv = 1.0f;
+        if (w) {
+            const float ss = wave_sum(fmaf(hi[h], hi[h], lo[h] * lo[h]));  // (what is fused to what is the first kernel's here and below)
+            inv = 1.0f / sqrtf(ss / (float)d + eps);
+        }
+        float x1 = lo[h] * inv, x2 = hi[h] * inv;
+        if (w) {
+            x1 *= load_as_f32(w, lane, weight_dtype);
+            x2 *= load_as_f32(w, lane + half, weight_dtype);
+        }
+        float* dst;
+        if (is_q) {
+            dst = q_out + (n * nq + head) * d + lane;
+        } else {
+            const int page = slot / page_size;
+            dst = kv_layer + page * page_stride + ((int64_t)(head - nq) * page_size + (slot - page * page_size)) * d + lane;
+        }
+        dst[0] = fmaf(x1, cs.x, -(x2 * cs.y));
+        dst[half] = fmaf(x2, cs.x, x1 * cs.y);
+    }
+}
+
 // cos and sin of float(pos) * inv_freq[i] for every token of the step: out [N][half][2]
 __global__ __launch_bounds__(256) void rope_table_kernel(const int32_t* __restrict__ positions,
                                                           const float* __restrict__ inv_freq,
@@ -398,6 +467,20 @@ extern "C" int lle_qk_norm_rope_write(const void* qkv, const void* slots,
                                         VW_TOKENS * (d + 2) * sizeof(bf16_t), stream>>>(
                 (const bf16_t*)qkv, (const int32_t*)slots, (bf16_t*)kv_layer, N, nq, nkv, d, page_size, page_stride);
         LLE_RETURN_LAUNCH_STATUS();
+    }
+    // (us, a wavefront a head / four: 64 tokens of 16 / 8 heads 3.7 / 3.9, of 8 / 1 3.0 / 3.5, 100 of 8 / 1 3.1 / 3.5; 64 of 32 / 8 4.1 / 4.0, 100 of 16 / 8
+    // 4.4 / 4.0, 300 of 8 / 1 4.0 / 3.7)
+    if (dtype == LLE_F32 && d == 128 && rot == d && (int64_t)N * (nq + 2 * nkv) >= 3000 && page_size % 8 == 0 && page_stride % 4 == 0 &&
+        (((uintptr_t)qkv | (uintptr_t)kv_layer) & 15) == 0) {
+        const int heads = nq + (write_kv ? nkv : 0), head_groups = (heads + QK_HEADS - 1) / QK_HEADS;
+        const int64_t groups = (int64_t)N * head_groups, head_blocks = (groups + 3) / 4;
+        const int64_t v_blocks = write_kv ? (int64_t)((N + VW_TOKENS - 1) / VW_TOKENS) * nkv : 0;
+        if (head_blocks + v_blocks <= 0x7fffffff) {
+            qk_norm_rope_write_f32_kernel<<<(unsigned)(head_blocks + v_blocks), 256, 0, stream>>>(
+                (const float*)qkv, (const int32_t*)slots, q_weight, k_weight, weight_dtype, (const float*)cos_sin, eps, (float*)q_out,
+                (float*)kv_layer, nq, nkv, page_size, page_stride, write_kv, head_groups, groups, head_blocks, N);
+            LLE_RETURN_LAUNCH_STATUS();
+        }
     }
     dim3 grid(N, nq + 2 * nkv);
     if (dtype == LLE_F32)
