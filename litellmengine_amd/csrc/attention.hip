@@ -2478,8 +2478,7 @@ __global__ __launch_bounds__((SHORT_F32_WAVES + 1) * LLE_WAVE) void short_decode
     }
 }
 
-// merges the key splits of the kernels above: grid = (tokens, q heads), one wavefront each.  PARTS: split_f32_attention_kernel's, whose rows may
-// have fewer parts than nsplit, or none.
+// merges the key splits of mfma_f32_attention_kernel: grid = (tokens, q heads), one wavefront each
 __global__ __launch_bounds__(LLE_WAVE) void f32_combine_kernel(const float* __restrict__ ws_o,
                                                                const float* __restrict__ ws_ml, int nsplit,
                                                                float* __restrict__ out, int nq, int D,
@@ -2513,8 +2512,9 @@ __global__ __launch_bounds__(256) void split_f32_combine_kernel(const float* __r
     const float2 ml = *(const float2*)(ws_ml + (head_row * nsplit + min(lane, nsplit - 1)) * 2);
     const float m = lane < nsplit ? ml.x : NEG_BIG, l = lane < nsplit ? ml.y : 0.f;
     const uint64_t some = __ballot(l != 0.f);  // (behind the last of them there may be nothing written)
-    if (some == 0 || (__ballot(l < 0.f) & 1)) return;
-    const int held = 64 - __builtin_clzll(some);
+    if (__ballot(l < 0.f) & 1) return;
+    // (none: every score is -inf or as good as, and the row 0 / 0 as in f32_combine_kernel, or 0 beside a sink)
+    const int held = some ? 64 - __builtin_clzll(some) : 0;
     const float big = wave_max(m);
     const float f = exp2f(m - big);
     float den = wave_sum(l * f);

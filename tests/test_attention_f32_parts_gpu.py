@@ -84,6 +84,35 @@ def test_what_is_not_finite(steps, value, monkeypatch):
     assert torch.equal(got[:128], clean[:128])  # (blocks of 32 tokens: a block whose rows see none of them)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps", [1, 3, 1 << 20])
+@pytest.mark.parametrize("value", [math.inf, 3e17])
+@pytest.mark.parametrize("sink", [False, True])
+def test_a_row_that_nothing_weighs_in(steps, value, sink, monkeypatch):
+    """Every score of a row -inf, or finite and too low to count: NaN as from the float32 instruction in splits, 0 beside a sink, and never what the
+    result's memory held before."""
+    from litellmengine_amd.csrc import ops
+
+    o, (nq, nkv) = ops.default_ops(), (8, 2)
+    q, kv, *rest = batch([200], [50], nq, nkv, 128)
+    kv[:, 0, 0, :, 3] = -1e16  # one channel of the first head's keys, all of one sign
+    q[:, :4, 3] = 0.0
+    q[190, 2] = 0.0
+    q[190, 2, 3] = value
+    sinks = torch.linspace(-2.0, 6.0, nq, device="cuda") if sink else None
+    monkeypatch.setattr(ops, "_made", lambda shape, dtype, device: torch.full(shape, 5.0, dtype=dtype, device=device))
+    call = lambda: o.paged_attention(q, kv, *rest, window=None, scale=128**-0.5, min_q_len=200, max_q_len=200, max_kv_len=250, sinks=sinks)
+    in_parts(o, monkeypatch, steps)
+    got = call()
+    in_parts(o, monkeypatch, 0)
+    monkeypatch.setattr(o, "f32_attention_splits", lambda *a: 3)
+    want = call()
+    row = got[190, 2 * 128 : 3 * 128]
+    assert bool((row == 0.0).all()) if sink else bool(row.isnan().all())
+    assert torch.equal(got.isnan(), want.isnan())
+    assert (got - want)[want.isfinite()].abs().max() < 400 * 4 * 2**-24 * 2
+
+
 @pytest.mark.parametrize("group", [1, 2, 3, 4, 5, 8, 40])
 @pytest.mark.parametrize("window", [0, 16, 500])
 def test_every_part_has_a_workgroup(group, window):
