@@ -2321,7 +2321,8 @@ class HipOps:
         """Whether the chunks of long requests go one after the other, the state in registers (ssd_stream_kernel): up to 512 tokens, and beyond
         where the long requests' workgroups (a head and sixteen value channels each) are as many as the CUs.  With fewer the chain of the chunks
         is what takes the time: 32 heads of 64 x 128, chunks side by side / one after the other, one request of 256, 512, 1024, 2048 tokens
-        34 / 24, 39 / 36, 54 / 59, 76 / 101 us; two of 1024 77 / 64; 64 heads, one request of 1024, 2048, 4096 tokens 76 / 63, 120 / 107, 224 / 189."""
+        34 / 24, 39 / 36, 54 / 59, 76 / 101 us; two of 1024 77 / 64; 64 heads, one request of 1024, 2048, 4096 tokens 76 / 63, 120 / 107, 224 / 189.
+        Requests of 32768 tokens and more have not been measured and stay as they were."""
         few = max(1, (num_tokens - num_seqs) // max(1, longest)) * heads * (vdim // 16) < self.compute_units()
         return n == 128 and vdim % 16 == 0 and longest < 1 << 15 and (longest <= 512 or not few)
 
@@ -2354,7 +2355,8 @@ class HipOps:
         together, stream_floats = 1, 0
         if pieces:
             slots = N // self.SSD_CHUNK + S
-            if S <= 65535 and self.ssd_streams(N, S, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
+            # (a chunk's bytes of c are counted in 32 bits there)
+            if S <= 65535 and CC < 1 << 23 and self.ssd_streams(N, S, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
                 stream_floats = slots * (G * (2 * self.SSD_CHUNK * 128 + 2560) + H * 5 * self.SSD_CHUNK)  # (lle_ssd_stream_floats)
                 part = _made((stream_floats,), dtype=torch.float32, device=c.device)
             else:

@@ -677,6 +677,7 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdArgs a) {
 #define SSD_OF_B (SSD_CHUNK * SSD_N)
 #define SSD_OF_PAIRS (2 * SSD_CHUNK * SSD_N)
 #define SSD_OPERANDS (2 * SSD_CHUNK * SSD_N + 10 * 256)
+#define SSD_STREAM_CC (0x7fffffff / (4 * SSD_CHUNK))  // widest row of c: a chunk's bytes are counted in 32 bits
 struct SsdStream {
     float* operands;  // [chunk slots][G]: C, B and the ten tiles of C_t . B_s, s <= t, all lane by lane (SSD_OPERANDS floats)
     float* steps;  // [chunk slots][H][5][64]: dt, l's two floats, exp(l_last - l) dt, exp(l)
@@ -811,9 +812,9 @@ __global__ __launch_bounds__(256, 2) void ssd_stream_kernel(SsdArgs a, SsdStream
         for (int n = 0; n < 3; ++n) cb[n] = four(unit, SSD_OF_PAIRS + tile_at[n] * 256);
     };
     auto ask_x = [&](int i) {
-        // (a buffer that ends with the request's last token: tokens past it are zeros)
+        // (a buffer that ends with the chunk's last token: tokens past it are zeros; a chunk's bytes fit 32 bits, a long request's of wide rows do not)
         const auto chunk = __builtin_amdgcn_make_buffer_rsrc((void*)(rows + (int64_t)min(i, live - 1) * SSD_CHUNK * a.CC), 0,
-                                                             i < live ? (len - i * SSD_CHUNK) * a.CC * 4 : 0, 0x00020000);
+                                                             i < live ? min(SSD_CHUNK, len - i * SSD_CHUNK) * a.CC * 4 : 0, 0x00020000);
         x = __builtin_bit_cast(ssd_f32x4, __builtin_amdgcn_raw_buffer_load_b128(chunk, of_x, 0, 0));
         const auto steps = __builtin_amdgcn_make_buffer_rsrc((void*)(p.steps + ((slot0 + min(i, live - 1)) * a.H + h) * (5 * SSD_CHUNK)), 0, 20 * SSD_CHUNK, 0x00020000);
         auto word = [&](int at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(steps, 4 * at, 0, 0)); };
@@ -948,7 +949,7 @@ extern "C" int lle_ssd_scan(const void* c, int CC, const void* dt_in, int dt_col
     if (pieces == 0) return 0;
     if (stream_floats > 0) {
         const int chunks = N / SSD_CHUNK + S;
-        if (n != SSD_N || vdim % 16 != 0 || S > 65535 || stream_floats < lle_ssd_stream_floats(N, S, H, G) || (((uintptr_t)c | (uintptr_t)y | (uintptr_t)part) & 15))
+        if (n != SSD_N || vdim % 16 != 0 || S > 65535 || CC > SSD_STREAM_CC || stream_floats < lle_ssd_stream_floats(N, S, H, G) || (((uintptr_t)c | (uintptr_t)y | (uintptr_t)part) & 15))
             return (int)hipErrorInvalidValue;
         const SsdStream p{(float*)part, (float*)part + (int64_t)chunks * G * SSD_OPERANDS};
         ssd_pairs_kernel<<<dim3(chunks, G + (H + 3) / 4), 256, 0, stream>>>(a, p, S);

@@ -75,3 +75,26 @@ def test_a_steep_drop_inside_a_chunk():
     scale = float(want.abs().max())
     assert torch.isfinite(got).all() and (got - want).abs().max() < 128 * 2**-24 * scale
     assert (state - want_state).abs().max() < 64 * 2**-24 * float(want_state.abs().max())
+
+
+def test_a_long_request_of_wide_rows(monkeypatch):
+    """32767 tokens of 512 heads: the rest of the request behind a chunk is over 4 GiB, so that a count of its bytes in 32 bits is too small for the first
+    chunks.  Rows and states are those of the chunks side by side."""
+    o = ops()
+    H, G, vdim, n, N = 512, 1, 64, 128, 32767
+    assert o.ssd_streams(N, 1, H, vdim, n, N) and 4 * N * (H * vdim + 2 * G * n) > 1 << 32
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    c = torch.zeros((N, H * vdim + 2 * G * n), device="cuda")
+    c[:512], c[-100:] = rand(512, c.shape[1]), rand(100, c.shape[1])
+    dt_in, dt_bias, a_log, D = rand(N, H), rand(H), rand(H) - 8.0, rand(H)  # (decays of a thousandth a token: the first chunks are still seen)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    got = {}
+    for streams in (True, False):
+        monkeypatch.setattr(o, "ssd_streams", lambda *a, s=streams: s)
+        state = torch.zeros((1, H * vdim * n), device="cuda")
+        y = o.ssd_scan(c, dt_in, dt_bias, a_log, D, state, H, G, vdim, n, ints([0]), ints([0, N]), N, N)
+        got[streams] = y[:1024].clone(), y[-200:].clone(), state
+        del y
+    for a, b in zip(got[True], got[False]):  # sums of at most 64 tokens and 128 channels, in 32 bits: under 64 roundings of the largest result
+        close(a, b, 64 * 2**-24 * max(1.0, float(b.abs().max())))
