@@ -865,8 +865,23 @@ __global__ __launch_bounds__(2 * NW * LLE_WAVE, NW / 2) void delta_chunk_walk_ke
 #pragma unroll
             for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[v][e], S[v][e], o, 0, 0, 0);
         }
+        bool odd = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(t[e], w[e], o, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(w[e]) < INFINITY);
+        if (!__any(odd)) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(t[e], w[e], o, 0, 0, 0);
+        } else {  // 0 times a later token's infinity would be NaN: row after row, without what the row does not see
+            const delta_vec4 before = o;
+#pragma unroll 1
+            for (int row = 0; row < TC; ++row) {
+                delta_vec4 all = before;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) all = __builtin_amdgcn_mfma_f32_16x16x4f32(t[e], 4 * c + e <= row ? w[e] : 0.f, all, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = 4 * c + e == row ? all[e] : o[e];
+            }
+        }
         const int left = q1 - (q0 + i * TC + 4 * c);
         if (j < a.vdim) {
             if (i < n - 1) {  // (the same for the wavefront: a whole chunk)

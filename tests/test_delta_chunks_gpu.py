@@ -1,6 +1,8 @@
 """The delta rule in chunks of sixteen tokens (long requests where they are few) against the plain recurrence: the shortest request that goes in
 chunks and the longest that is walked, last chunks of one and of fifteen tokens, value channels that are no sixteens, one decay
-a head and one a channel, decays of zero and of one, more long requests than go in chunks."""
+a head and one a channel, decays of zero and of one, more long requests than go in chunks; what is not finite."""
+import math
+
 import pytest
 import torch
 
@@ -43,3 +45,35 @@ def test_long_requests_in_chunks(dim, vdim, H, G, lens, channel):
         o.DELTA_WALK, c = N, start.clone()
         walked = o.delta_scan(q, k, v, ba, a_log, dt_bias, c, H, G, dim, vdim, slots, cu, decay=decay)
         assert (got - walked).abs().max() < 2e-4 and not torch.equal(got, walked)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "decay", "state"])
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_what_is_not_finite_stays_behind_its_token(what, value, dim):
+    """Token 24, inside a chunk, brings something that is not finite: rows before it are what they were, and in all others and in the states
+    nothing else is finite or not than where the tokens are walked."""
+    from litellmengine_amd.csrc.ops import HipOps
+
+    o, H, vdim, N, token = HipOps(), 2, 64, 200, 24
+    rand = torch.Generator().manual_seed(1)
+    f = lambda *shape: torch.randn(shape, generator=rand).cuda()
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    q, k, v, beta, decay, state = unit(f(N, dim)), unit(f(N, dim)), f(N, H * vdim), f(N, H), torch.sigmoid(3.0 * f(N, H * dim)), 0.3 * f(1, H * vdim * dim)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+
+    def run(own):
+        return o.delta_scan(q, k, v, beta, None, None, own, H, 1, dim, vdim, ints([0]), ints([0, N]), decay=decay)
+
+    clean = run(state.clone())
+    operand = {"q": q, "k": k, "v": v, "beta": beta, "decay": decay}.get(what, state)
+    operand[0 if what == "state" else token, 1] = value
+    chunks, walked = state.clone(), state.clone()
+    got = run(chunks)
+    o.DELTA_WALK = N
+    want = run(walked)
+    assert torch.equal(got.isfinite(), want.isfinite()) and torch.equal(chunks.isfinite(), walked.isfinite())
+    fine = want.isfinite()
+    assert (got - want)[fine].abs().max() < 2e-4 if fine.any() else what == "state"  # (as above)
+    if what != "state":
+        assert torch.equal(got[:token], clean[:token])
