@@ -2238,7 +2238,8 @@ class HipOps:
             floats = self._get("delta", "lle_delta_chunk_floats", "IIIII")(N, S, H, dim, vdim) if few > 0 else 0
             if 0 < floats <= self.DELTA_CHUNK_FLOATS and not any(t is not None and t.data_ptr() % 16 for t in (q, k, decay)):
                 work = _made((floats,), dtype=torch.float32, device=v.device)
-                self._run("delta", "lle_delta_chunks", types + "IIIPP", *args, N, self.DELTA_WALK, few, _ptr(work))
+                # (a single request goes in chunks whatever cu_tokens says it has of the N tokens: nothing else is launched for it)
+                self._run("delta", "lle_delta_chunks", types + "IIIPP", *args, N, self.DELTA_WALK if S > 1 else 0, few, _ptr(work))
                 if S == 1:
                     return out
             else:

@@ -77,3 +77,22 @@ def test_what_is_not_finite_stays_behind_its_token(what, value, dim):
     assert (got - want)[fine].abs().max() < 2e-4 if fine.any() else what == "state"  # (as above)
     if what != "state":
         assert torch.equal(got[:token], clean[:token])
+
+
+@pytest.mark.parametrize("tokens", [0, 3, 150, 161])
+def test_a_single_request_of_fewer_tokens_than_rows(tokens):
+    """Rows behind the request's last token belong to nobody; whether it is long is seen on the device, not by the rows."""
+    from litellmengine_amd.csrc.ops import HipOps
+
+    o, H, dim, N = HipOps(), 2, 64, 200
+    rand = torch.Generator().manual_seed(1)
+    f = lambda *shape: torch.randn(shape, generator=rand).cuda()
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    q, k, v, ba, a_log, dt_bias, state = unit(f(N, dim)), unit(f(N, dim)), f(N, H * dim), f(N, 2 * H), f(H), f(H), 0.3 * f(1, H * dim * dim)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    a, b = state.clone(), state.clone()
+    head = [t[:tokens] for t in (q, k, v, ba)]
+    want = REF.delta_scan(*head, a_log, dt_bias, a, H, 1, dim, dim, ints([0]), ints([0, tokens])) if tokens else v[:0]
+    got = o.delta_scan(q, k, v, ba, a_log, dt_bias, b, H, 1, dim, dim, ints([0]), ints([0, tokens]))
+    assert torch.equal(got[:0], want) if tokens == 0 else (got[:tokens] - want).abs().max() < 2e-4  # (as above)
+    assert (a - b).abs().max() < 2e-4
