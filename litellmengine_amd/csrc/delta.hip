@@ -582,6 +582,7 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_scan_kernel(DeltaArgs a) 
 }
 
 #define DELTA_MAX_DIM (16 * DELTA_IG)
+#define DELTA_GRID_Z 65535  // most requests of a launch
 extern "C" int lle_delta_max_dim(void) { return DELTA_MAX_DIM; }
 
 // q, k float32 [N, G dim] (unit vectors, q scaled), v float32 [N, H vdim], ba float32 [N, 2 H], a_log and dt_bias
@@ -595,7 +596,7 @@ extern "C" int lle_delta_scan(const void* q, const void* k, const void* v, const
                               const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, void* gates, int N, int most, int few,
                               hipStream_t stream) {
     if (S <= 0 || H <= 0) return 0;
-    if (G <= 0 || H % G || dim <= 0 || dim > DELTA_MAX_DIM || vdim <= 0 || H > 65535 || S > 65535)
+    if (G <= 0 || H % G || dim <= 0 || dim > DELTA_MAX_DIM || vdim <= 0 || H > 65535 || (few > 0 && S > DELTA_GRID_Z))
         return (int)hipErrorInvalidValue;
     if (ba_cols < (decay ? H : 2 * H)) return (int)hipErrorInvalidValue;
     DeltaArgs a{(const float*)q, (const float*)k, (const float*)v, (const float*)ba, ba_cols, (const float*)a_log,
@@ -606,13 +607,17 @@ extern "C" int lle_delta_scan(const void* q, const void* k, const void* v, const
         delta_gates_kernel<<<(int)((total + 255) / 256), 256, 0, stream>>>((const float*)ba, ba_cols, (const float*)a_log,
                                                                             (const float*)dt_bias, (float*)gates, total, H);
     }
-    const dim3 grid((vdim + DELTA_VB - 1) / DELTA_VB, H, S);
-#define DELTA_CASE(KI)                                                      \
-    if (dim <= KI * DELTA_IG) {                                             \
-        if (decay) delta_scan_kernel<KI, true><<<grid, DELTA_THREADS, 0, stream>>>(a);   \
-        else delta_scan_kernel<KI, false><<<grid, DELTA_THREADS, 0, stream>>>(a);        \
-        LLE_RETURN_LAUNCH_STATUS();                                         \
-    }
+    auto launch = [&](auto kernel) {  // (more requests than the grid's third dimension holds: one launch after the other)
+        for (int s0 = 0; s0 < S; s0 += DELTA_GRID_Z) {
+            a.seq_slots = (const int32_t*)seq_slots + s0;
+            a.cu_tokens = (const int32_t*)cu_tokens + s0;
+            a.S = min(DELTA_GRID_Z, S - s0);
+            kernel<<<dim3((vdim + DELTA_VB - 1) / DELTA_VB, H, a.S), DELTA_THREADS, 0, stream>>>(a);
+        }
+        LLE_RETURN_LAUNCH_STATUS();
+    };
+#define DELTA_CASE(KI) \
+    if (dim <= KI * DELTA_IG) return decay ? launch(delta_scan_kernel<KI, true>) : launch(delta_scan_kernel<KI, false>);
     DELTA_CASE(1)
     DELTA_CASE(2)
     DELTA_CASE(4)
@@ -899,7 +904,7 @@ __global__ __launch_bounds__(2 * NW * LLE_WAVE, NW / 2) void delta_chunk_walk_ke
 
 // Floats of `work` for a step of N tokens of S requests, or 0 where no chunks are made of such heads or of so many tokens.
 extern "C" int lle_delta_chunk_floats(int N, int S, int H, int dim, int vdim) {
-    if (N <= 0 || S <= 0 || H <= 0 || H > 65535 || vdim <= 0 || (dim != 64 && dim != 128) || dim + vdim > DELTA_THREADS) return 0;
+    if (N <= 0 || S <= 0 || S > DELTA_GRID_Z || H <= 0 || H > 65535 || vdim <= 0 || (dim != 64 && dim != 128) || dim + vdim > DELTA_THREADS) return 0;
     const int64_t floats = (int64_t)(N / DELTA_TC + S) * H * delta_unit_floats(dim, vdim);
     return floats <= 0x7fffffff ? (int)floats : 0;
 }
@@ -911,7 +916,7 @@ extern "C" int lle_delta_chunks(const void* q, const void* k, const void* v, con
                                 const void* cu_tokens, void* out, int S, int H, int G, int dim, int vdim, int N, int most, int few, void* work,
                                 hipStream_t stream) {
     if (S <= 0 || H <= 0 || N <= 0) return 0;
-    if (lle_delta_chunk_floats(N, S, H, dim, vdim) == 0 || G <= 0 || H % G || S > 65535 || ba_cols < (decay ? H : 2 * H) || most < 0 ||
+    if (lle_delta_chunk_floats(N, S, H, dim, vdim) == 0 || G <= 0 || H % G || ba_cols < (decay ? H : 2 * H) || most < 0 ||
         (((uintptr_t)q | (uintptr_t)k | (uintptr_t)decay | (uintptr_t)work) & 15))
         return (int)hipErrorInvalidValue;
     const DeltaArgs a{(const float*)q, (const float*)k, (const float*)v, (const float*)ba, ba_cols, (const float*)a_log,

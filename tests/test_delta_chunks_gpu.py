@@ -96,3 +96,21 @@ def test_a_single_request_of_fewer_tokens_than_rows(tokens):
     got = o.delta_scan(q, k, v, ba, a_log, dt_bias, b, H, 1, dim, dim, ints([0]), ints([0, tokens]))
     assert torch.equal(got[:0], want) if tokens == 0 else (got[:tokens] - want).abs().max() < 2e-4  # (as above)
     assert (a - b).abs().max() < 2e-4
+
+
+def test_more_requests_than_a_grid_holds():
+    """65600 requests of one token: the ones at the edges of the launches that they are cut into."""
+    from litellmengine_amd.csrc.ops import HipOps
+
+    S, dim = 65600, 16
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    f = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    q, k, v, ba, a_log, dt_bias, state = f(S, dim), f(S, dim), f(S, dim), f(S, 2), f(1), f(1), f(S, dim * dim)
+    slots, cu = torch.arange(S, dtype=torch.int32, device="cuda"), torch.arange(S + 1, dtype=torch.int32, device="cuda")
+    at = torch.tensor([0, 1, 65534, 65535, 65536, S - 1], device="cuda")
+    want_state = state[at].clone()
+    want = REF.delta_scan(q[at], k[at], v[at], ba[at], a_log, dt_bias, want_state, 1, 1, dim, dim, slots[:6], cu[:7])
+    got = HipOps().delta_scan(q, k, v, ba, a_log, dt_bias, state, 1, 1, dim, dim, slots, cu)
+    # (keys that are no unit vectors: values of |k| |q| |S|, some hundreds, with sums of 16 products in 32 bits)
+    scale = float(want.abs().max())
+    assert (got[at] - want).abs().max() < 32 * 2**-24 * max(1.0, scale) and (state[at] - want_state).abs().max() < 32 * 2**-24 * max(1.0, scale)
