@@ -756,8 +756,10 @@ __global__ __launch_bounds__(256) void ssd_pairs_kernel(SsdArgs a, SsdStream p, 
     }
 }
 
-// e^x for x <= 0 to about an ulp (expf's way to large and odd arguments is half of a tile's instructions): x log2 e in two floats
+// e^x for x <= 0 to two ulps, as x log2 e in two floats (expf's way to large and odd arguments is half of a tile's instructions).  Results below
+// 2^-126 are 0; so are those of what is below -1000, whose product with log2 e may be an infinity; NaN stays.
 __device__ __forceinline__ float ssd_exp(float x) {
+    x = x < -1000.f ? -1000.f : x;
     const float p = x * 1.44269502162933349609f;
     const float rest = fmaf(x, 1.92596302e-8f, fmaf(x, 1.44269502162933349609f, -p));
     const float y = __builtin_amdgcn_exp2f(p);

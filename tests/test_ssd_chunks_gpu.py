@@ -77,6 +77,48 @@ def test_a_steep_drop_inside_a_chunk():
     assert (state - want_state).abs().max() < 64 * 2**-24 * float(want_state.abs().max())
 
 
+def test_a_drop_further_than_its_exponent():
+    """A decay of exp(-3e38), finite as it is: what was before is gone, what comes after is not touched."""
+    o = ops()
+    H, G, vdim, N = 2, 1, 16, 150
+    c = torch.randn((N, H * vdim + 2 * 128), generator=torch.Generator().manual_seed(2)).cuda()
+    dt_in = torch.full((N, H), -200.0).cuda()  # (exp(69) would end the state with any other step of head 0)
+    dt_in[70, 0] = 3.0e8
+    a_log = torch.tensor([69.0, 0.0]).cuda()  # exp(69) 3e8 = 2.8e38
+    zeros, D = torch.zeros(H).cuda(), torch.zeros(H).cuda()
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    state, want_state = torch.ones((2, H * vdim * 128)).cuda(), torch.ones((2, H * vdim * 128)).cuda()
+    got = o.ssd_scan(c, dt_in, zeros, a_log, D, state, H, G, vdim, 128, ints([1]), ints([0, N]), N, N)
+    want = REF.ssd_scan(c, dt_in, zeros, a_log, D, want_state, H, G, vdim, 128, ints([1]), ints([0, N]))
+    assert torch.isfinite(got).all()
+    for part in (slice(0, 70), slice(70, N)):  # (from token 70 on rows of head 0 are of the order of 3e8)
+        assert (got[part] - want[part]).abs().max() < 128 * 2**-24 * float(want[part].abs().max())
+    assert (state - want_state).abs().max() < 64 * 2**-24 * float(want_state.abs().max())
+
+
+@pytest.mark.parametrize("a_log", [-8.0, -4.0, -2.0, 0.0])
+def test_decays_inside_a_chunk_to_two_ulps(a_log):
+    """y of the token behind x = 1 is 32 exp(-exp(a_log) dt), dt from 32 to 95 and exact in 32 bits; arguments from -0.01 to -95."""
+    o = ops()
+    H, vdim, N = 64, 16, 40
+    c = torch.zeros((N, H * vdim + 2 * 128))
+    c[0, : H * vdim] = 1.0  # x of token 0 alone
+    c[:, H * vdim], c[:, H * vdim + 128] = 1.0, 1.0  # B and C of channel 0
+    dt_in = torch.full((N, H), -200.0)  # (steps of 1e-87: none)
+    dt_in[0] = 32.0
+    dt_in[1] = 32.0 + torch.arange(H)
+    zeros, state = torch.zeros(H).cuda(), torch.zeros((1, H * vdim * 128)).cuda()
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    y = o.ssd_scan(c.cuda(), dt_in.cuda(), zeros, zeros + a_log, zeros, state, H, 1, vdim, 128, ints([0]), ints([0, N]), N, N)
+    arg = -torch.exp(torch.tensor(a_log, dtype=torch.float64)) * dt_in[1].double()
+    want = 32.0 * torch.exp(arg)
+    got = y[1].view(H, vdim)[:, 0].cpu().double()
+    # the argument is off by an ulp of exp(a_log) and half a one of its product: |arg| 1.5 ulps; the exponential and two products: four; results below
+    # 2^-126 are gone
+    assert ((got - want).abs() < (1.5 * arg.abs() + 4) * 2**-23 * want + 32 * 2**-126).all()
+    assert torch.equal(y[2:].view(-1, H, vdim)[:, :, 0].cpu().double(), got.expand(N - 2, H))  # (nothing happens any more)
+
+
 def test_a_long_request_of_wide_rows(monkeypatch):
     """32767 tokens of 512 heads: the rest of the request behind a chunk is over 4 GiB, so that a count of its bytes in 32 bits is too small for the first
     chunks.  Rows and states are those of the chunks side by side."""
