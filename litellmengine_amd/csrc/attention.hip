@@ -1900,14 +1900,16 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, DQ > 12 ? 1 : DQ >= 8 || TILES
 }
 
 // ---------------------------------------------------------------------------------
-// float32 attention of many rows on the bfloat16 matrix cores without losing a bit of an operand: q, K, V and the probabilities as three bfloat16
-// parts each (parts.h), both products in six of the bfloat16 instruction (gemm_f32.hip says what that keeps), scores, maxima and sums in
+// float32 attention of many rows on the bfloat16 matrix cores: q, K, V and the probabilities as three bfloat16 parts each, which hold all bits of what
+// is not too small (parts.h), both products in six of the nine of the bfloat16 instruction (gemm_f32.hip says what that keeps), scores, maxima and sums in
 // float32.  The float32 instruction bounds mfma_f32_attention_kernel (8192 cycles for 32 rows and 32 keys of 128 elements, 3072 here).
 // A workgroup takes 128 rows of a request, a wavefront 32, whose first two parts of q stay in its registers and the third in its own piece of LDS.
 // 32 keys a step: K and V^T are loaded once a workgroup, split once and laid out in LDS as three planes each in the layouts of
 // mfma_prefill_kernel; K of the next step is on its way while this one's scores are made, V of it under the product with the values.  80 KB
-// and 256 registers a lane: two workgroups a CU.  Requests of at most 16 rows, and rows that come out not finite (an infinity has no parts),
-// are f32_attention_rows'.
+// and 256 registers a lane: two workgroups a CU.  Requests of at most 16 rows are f32_attention_rows', and rows that come out not finite (an infinity
+// has no parts) or whose parts may have run out of exponent (the last one ends at 2^-133): elements of q below SA_SMALL, or above SA_LARGE, where keys
+// below SA_SMALL matter, and results below SA_SMALL, whose values are as small.  (Left: probabilities below SA_SMALL, which only values 2^80 times the rest
+// bring back.)  V of 1e-36: error 2.7e-5 without, 4.1e-7 so.
 // What bounds it: matrix cores busy 0.53 of the time and the other vector instructions, half of them splitting, most of the rest (4096 tokens; they
 // hardly run beside each other, whatever the priorities: matrix instructions first made it 720 us); below two workgroups a CU a wavefront's
 // own chain, 3.7 us a step.  32 / 8 heads of 128, the other kernel -> this one: a prompt of 512 / 1024 / 2048 / 4096 tokens 55 -> 40, 116 -> 78,
@@ -1920,6 +1922,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define SA_KEYS 32
 #define SA_PLANE 8192  // bytes of a part of a step's K or V
 #define SA_LDS (10 * SA_PLANE)  // three of each, and the third parts of q
+#define SA_SMALL 0x1p-105f
+#define SA_LARGE 0x1p100f
 __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_kernel(
     const float* __restrict__ q, const float* __restrict__ kv_layer, const int32_t* __restrict__ block_tables,
     const int32_t* __restrict__ seq_slots, const int32_t* __restrict__ cu_tokens,
@@ -2004,6 +2008,8 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_ke
         int pos[TILES], low[TILES];
         int64_t head_row[TILES];
         u32x4 qp[TILES][KS][2];
+        // (the bits of a size are in its order; 0 comes out as the largest)
+        auto size_less_one = [](float x) { return __builtin_bit_cast(uint32_t, fabsf(x)) - 1u; };
         unsigned char* third = lds + 6 * SA_PLANE + (wave * LLE_WAVE + lane) * 16;  // each lane's own, [tile][32 elements of q]
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
@@ -2013,6 +2019,7 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_ke
             head_row[t] = (int64_t)(q_start + tok) * nq + kvh * G + g;
             pos[t] = exists[t] ? past + tok : -1;
             low[t] = exists[t] && window > 0 ? max(0, pos[t] - window + 1) : 0;
+            uint32_t least = ~0u, most = 0;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 const float* at = q + head_row[t] * D + 32 * ks + 8 * c;
@@ -2023,9 +2030,11 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_ke
                     uint32_t p1, p2, p3;
                     split2(h < 2 ? a[2 * h] : b[2 * h - 4], h < 2 ? a[2 * h + 1] : b[2 * h - 3], p1, p2, p3);
                     qp[t][ks][0][h] = p1, qp[t][ks][1][h] = p2, last[h] = p3;
+                    least = min(least, min(size_less_one(a[h]), size_less_one(b[h]))), most = max(most, max(size_less_one(a[h]) + 1, size_less_one(b[h]) + 1));
                 }
                 *(u32x4*)(third + (t * KS + ks) * (F32_WAVES * LLE_WAVE * 16)) = last;
             }
+            if (least < size_less_one(SA_SMALL) || most > size_less_one(SA_LARGE)) qp[t][0][0][0] = 0x7fc07fc0u;  // (NaN: the row comes out not finite)
         }
         // the copies: of K a thread takes pieces of eight elements of one key, of V^T pieces of eight keys of one element
         const PageSize pages(P);
@@ -2222,16 +2231,21 @@ __global__ __launch_bounds__(F32_WAVES* LLE_WAVE, 2) void split_f32_attention_ke
                 add_v(std::integral_constant<int, 6>{}, Set1{});
             }
         }
-        bool again = false;  // a row of the wavefront is not finite
+        bool again = false;  // a row of the wavefront is not finite, or too small for parts
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             l[t] = column_sum(l[t]);
             float sizes = fabsf(l[t]);
+            uint32_t least = ~0u;
 #pragma unroll
             for (int n = 0; n < N; ++n)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sizes = fmaxf(sizes, o[t][n][e] == o[t][n][e] ? fabsf(o[t][n][e]) : INFINITY);
-            const uint64_t odd = __ballot(exists[t] && !(sizes < INFINITY && l[t] == l[t]));  // (a row is four lanes)
+                for (int e = 0; e < 4; ++e) {
+                    sizes = fmaxf(sizes, o[t][n][e] == o[t][n][e] ? fabsf(o[t][n][e]) : INFINITY);
+                    least = min(least, size_less_one(o[t][n][e]));
+                }
+            const bool held = sizes < INFINITY && l[t] == l[t] && least >= size_less_one(l[t] * SA_SMALL);
+            const uint64_t odd = __ballot(exists[t] && !held);  // (a row is four lanes)
             const bool row_odd = (odd >> r16 | odd >> (r16 + 16) | odd >> (r16 + 32) | odd >> (r16 + 48)) & 1;
             again = again || odd != 0;
             if (!exists[t] || row_odd) continue;

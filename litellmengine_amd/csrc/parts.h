@@ -3,7 +3,7 @@
 #include "common.h"
 
 // Two numbers as their three bfloat16 parts, packed: x1 = x rounded, x2 = what is left rounded, x3 = the rest (3 x 8 significand bits and
-// two signs hold 24).
+// two signs hold 24, down to 2^-133, where bfloat16 ends: of numbers below 2^-109 the last bits are lost).
 __device__ __forceinline__ void split2(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
     typedef bf16_t pair __attribute__((ext_vector_type(2)));
     typedef float fpair __attribute__((ext_vector_type(2)));

@@ -85,6 +85,32 @@ def test_what_is_not_finite(steps, value, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("steps", [3, 1 << 20])
+@pytest.mark.parametrize("q_size", [1.0, 1e-36, 1e-34, 1e-32, 1e30, 1e34, 1e36])
+@pytest.mark.parametrize("v_size", [1.0, 1e-28, 1e-31, 1e-34, 1e-36])
+def test_small_numbers(steps, q_size, v_size, monkeypatch):
+    """Numbers whose last parts are below what bfloat16 has: no further off than with the float32 instruction, which takes such rows; keys are as
+    small as q is large.  Some elements are 0, which is no small number."""
+    from litellmengine_amd.csrc.ops import default_ops
+
+    o, lens, past = default_ops(), [200], [50]
+    q, kv, *rest = batch(lens, past, 8, 2, 128)
+    q *= q_size
+    kv[:, 0] /= q_size
+    kv[:, 1] *= v_size
+    q[:, :, 5], kv[:, 1].view(-1, 2, 128, 32)[:, :, 9] = 0.0, 0.0
+    args = (q, kv, *rest)
+    want = exact(args, lens, past, 2, None)
+    monkeypatch.setattr(o, "f32_attention_splits", lambda *a: 1)
+    in_parts(o, monkeypatch, 0)
+    before = run(o, args, lens, past, None)
+    in_parts(o, monkeypatch, steps)
+    got = run(o, args, lens, past, None)
+    off = lambda x: (x.cpu().double() - want).norm()
+    assert off(got) <= 1.05 * off(before)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("steps", [1, 3, 1 << 20])
 @pytest.mark.parametrize("value", [math.inf, 3e17])
 @pytest.mark.parametrize("sink", [False, True])
