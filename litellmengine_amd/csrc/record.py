@@ -49,7 +49,7 @@ class Replay:
         over = {t.data_ptr(): u.data_ptr() for t, u in zip(given, left)}
         if len(over) != len(given) or any(p in places for p in over) or any(u in places or u in over for u in over.values()):
             return
-        spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in operands)
+        spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in (*operands, *given))
         starts = [a for a, _ in spans]
         written = set(over.values())
         self.calls, last_given, first_left = [], -1, len(record.calls)
@@ -77,7 +77,7 @@ class Replay:
                 else:
                     at = bisect.bisect_right(starts, p) - 1
                     if at >= 0 and p < spans[at][1]:
-                        return  # (inside an operand)
+                        return  # (inside an operand, or inside what was taken over)
             self.calls.append((fn, name, args + [record.stream], tuple(patches), None))
         # what a layer takes over has been read before the same memory is written for the next one
         self.ok = last_given < first_left
