@@ -11,7 +11,7 @@ from typing import Optional
 
 import torch
 
-from ..parts.base import Injected, PartialSums, Prenormed, ScaledSum
+from ..parts.base import Injected, PartialSums, Prenormed, ScaledSum, Written, is_own_function
 from . import build
 from .record import LaunchRecord
 from .tuning import ProductTuning
@@ -156,7 +156,8 @@ class HipOps:
     def may_record(self) -> bool:
         """Whether what this object launches may be launched again for another layer: not where a caller has put a method of
         its own in the place of one, which would not be called then."""
-        return type(self) is HipOps and not any(callable(v) for v in vars(self).values()) and _recording.to is None
+        return (type(self) is HipOps and _recording.to is None and _written.unchanged()
+                and all(is_own_function(self, k, v) for k, v in vars(self).items() if callable(v)))
 
     def record(self) -> LaunchRecord:
         """From here until end_record() this thread's launches are kept."""
@@ -2433,6 +2434,7 @@ class HipOps:
         return per_instruction * 16 * iters * 4 * blocks
 
 
+_written = Written(HipOps, free=("record", "end_record", "replay"))  # (these launch nothing of a layer's own)
 _default: Optional[HipOps] = None
 
 

@@ -17,7 +17,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 
 from ..csrc.record import Replay, addresses_of, operand_kinds
-from ..parts.base import Block, BuildContext, Carried, Injected, Norm, Normed, PartialSums, Prenormed
+from ..parts.base import Block, BuildContext, Carried, Injected, Norm, Normed, PartialSums, Prenormed, parts_as_written
 from ..parts.embedding import Embedding
 from ..parts.injection import PassVectors
 from ..parts.linear import Linear
@@ -194,7 +194,7 @@ class DecoderLM:
         end - 1 have blocks that launch alike; None without such a stretch."""
         ops, plan = self.ctx.ops, self.plan
         if (len(plan) < self.ALIKE_LAYERS or step.token_ids.shape[0] > self.ALIKE_TOKENS
-                or not getattr(ops, "may_record", lambda: False)()):
+                or not getattr(ops, "may_record", lambda: False)() or not parts_as_written()):
             return None
         best, start, seen, settings, kinds, like = None, 0, [], None, None, None  # the stretch: first entry, (tensors, addresses), what its blocks share
         for i, e in enumerate(plan):

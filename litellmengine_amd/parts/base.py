@@ -12,6 +12,7 @@ concrete classes.
 from __future__ import annotations
 
 import dataclasses
+import functools
 from typing import Any, Dict, Optional, Tuple
 
 import torch
@@ -118,7 +119,46 @@ class StateSpec:
     dtype: torch.dtype = torch.float32
 
 
+class Written:
+    """A class's functions as they are now; `unchanged()`: whether they still are, but for those named in `free`."""
+
+    def __init__(self, cls, free=()):
+        self.cls, self.free = cls, free
+        self.everything, self.functions = dict(vars(cls)), self._functions()
+
+    def _functions(self) -> dict:
+        return {k: v for k, v in vars(self.cls).items()
+                if k not in self.free and (callable(v) or isinstance(v, (staticmethod, classmethod, property)))}
+
+    def unchanged(self) -> bool:
+        return vars(self.cls) == self.everything or self._functions() == self.functions  # (the first: no list made, 0.5 us)
+
+
+def is_own_function(owner, name: str, value) -> bool:
+    """Whether `value`, put on an instance, is what the instance has under this name anyway."""
+    made = getattr(type(owner), name, None)
+    return made is not None and getattr(value, "__func__", value) is made and getattr(value, "__self__", owner) is owner
+
+
 class Part:
+    _written: Dict[type, Written] = {}  # every kind of part
+    _replaced: frozenset = frozenset()  # of an instance: its class's functions in whose place it has others
+
+    def __init_subclass__(cls, **kwargs):
+        super().__init_subclass__(**kwargs)
+        Part._written[cls] = Written(cls)
+
+    def __setattr__(self, name, value):
+        if callable(getattr(type(self), name, None)):
+            others = self._replaced - {name} if is_own_function(self, name, value) else self._replaced | {name}
+            object.__setattr__(self, "_replaced", others)
+        object.__setattr__(self, name, value)
+
+    def __delattr__(self, name):
+        object.__delattr__(self, name)
+        if name in self._replaced:
+            object.__setattr__(self, "_replaced", self._replaced - {name})
+
     def tensor_specs(self) -> Dict[str, TensorSpec]:
         """Checkpoint tensors of this part, by full name."""
         return {}
@@ -135,7 +175,21 @@ class Part:
         return None
 
     def _as_made(self, cls) -> bool:
-        return type(self) is cls and "forward" not in vars(self)
+        return type(self) is cls and not self._replaced
+
+
+Part._written[Part] = Written(Part)
+
+
+def parts_as_written() -> bool:
+    """Whether no function of the parts that say what they launch (Part.launches), or of their bases, has been replaced."""
+    return all(written.unchanged() for written in _that_launch(len(Part._written)))
+
+
+@functools.lru_cache(maxsize=1)
+def _that_launch(kinds: int) -> list:
+    named = {base for cls, written in Part._written.items() if "launches" in written.functions for base in cls.__mro__}
+    return [written for cls, written in Part._written.items() if cls in named]
 
 
 @dataclasses.dataclass

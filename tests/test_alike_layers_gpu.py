@@ -10,6 +10,8 @@ from litellmengine_amd.engine.batch import StepEntry
 from litellmengine_amd.engine.runner import ModelRunner
 from litellmengine_amd.models import make_context
 from litellmengine_amd.models.decoder import DecoderLM
+from litellmengine_amd.parts import PagedAttention
+from litellmengine_amd.parts.norm import RMSNorm
 
 pytestmark = pytest.mark.gpu
 LAYERS = 8
@@ -125,3 +127,15 @@ def test_layers_that_differ_or_are_watched_run_by_themselves(replays):
     del replays[:]
     steps(runner, [60])
     assert not replays
+
+
+@pytest.mark.parametrize("cls,name,a_layer", [(HipOps, "linear", 3), (HipOps, "paged_attention", 1), (PagedAttention, "forward", 1), (RMSNorm, "forward", 2)])
+def test_a_function_replaced_on_its_class_is_called_for_every_layer(monkeypatch, replays, cls, name, a_layer):
+    runner = made("bfloat16")
+    steps(runner, [60])
+    assert replays
+    del replays[:]
+    calls, plain = [], getattr(cls, name)
+    monkeypatch.setattr(cls, name, lambda *a, **kw: (calls.append(1), plain(*a, **kw))[1])
+    steps(runner, [60])
+    assert not replays and len(calls) >= 2 * LAYERS * a_layer

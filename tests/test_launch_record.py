@@ -1,10 +1,14 @@
-"""What may be launched again for another layer: launches whose operands are whole tensors."""
+"""What may be launched again for another layer: launches whose operands are whole tensors, parts and operations that are as they were written."""
 import ctypes
 
 import pytest
 import torch
 
+from litellmengine_amd.config import Qwen3Config, get_architecture
 from litellmengine_amd.csrc.record import LaunchRecord, Replay
+from litellmengine_amd.parts import PagedAttention
+from litellmengine_amd.parts.base import Norm, parts_as_written
+from litellmengine_amd.parts.norm import RMSNorm
 
 
 def replay_of(pointer):
@@ -36,3 +40,43 @@ def test_a_launch_that_reads_what_was_taken_over():
 def test_a_launch_that_points_inside_a_tensor_is_not_launched_again(pointer):
     """Inside an operand, or inside what the layer before has left: the other layer's place is not known."""
     assert not replay_of(pointer)[0].ok
+
+
+def blocks():
+    config = Qwen3Config.from_dict({
+        "architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "num_hidden_layers": 2, "hidden_size": 64, "num_attention_heads": 2,
+        "num_key_value_heads": 1, "head_dim": 32, "intermediate_size": 96, "vocab_size": 100, "rope_theta": 1e6, "rms_norm_eps": 1e-6})
+    return get_architecture(config.architecture).build(config).blocks
+
+
+PARTS = [lambda b: b, lambda b: b.mixer, lambda b: b.norm_in, lambda b: b.norm_post, lambda b: b.feed_forward, lambda b: b.mixer.qkv, lambda b: b.mixer.o,
+         lambda b: b.feed_forward.down, lambda b: b.mixer.position]
+
+
+@pytest.mark.parametrize("part", PARTS)
+def test_a_part_with_a_function_of_its_own(part):
+    """Whichever of its functions a caller has replaced on a part, its block says no launches; until it has its own again."""
+    block, other = blocks()
+    assert block.launches() is not None
+    p = part(block)
+    for name in ("forward", "bind", "fold" if hasattr(p, "fold") else "tensor_specs"):
+        plain = getattr(p, name, None)
+        if plain is None:
+            continue
+        setattr(p, name, lambda *a, **kw: plain(*a, **kw))
+        assert block.launches() is None and other.launches() is not None
+        delattr(p, name)
+        assert block.launches() is not None
+        setattr(p, name, lambda *a, **kw: plain(*a, **kw))
+        setattr(p, name, plain)  # (as a patch that is undone leaves it)
+        assert block.launches() is not None
+
+
+@pytest.mark.parametrize("cls,name", [(PagedAttention, "forward"), (RMSNorm, "forward"), (PagedAttention, "entry"), (Norm, "fold")])
+def test_a_class_with_another_function(cls, name, monkeypatch):
+    """Replaced, added over a base's, or replaced on a base."""
+    assert parts_as_written()
+    monkeypatch.setattr(cls, name, lambda self, *a: None, raising=False)
+    assert not parts_as_written()
+    monkeypatch.undo()
+    assert parts_as_written()
