@@ -240,8 +240,9 @@ class DecoderLM:
         replay = Replay(record, operands[0][0], given, _tensors(left))
         if not replay.ok:
             return left, first + 1
-        for tensors, addresses in operands[1:]:
-            ops.replay(replay, tensors, addresses)
+        with torch.no_grad():  # (a product into a tensor that is there has no gradient, whatever its weight asks for)
+            for tensors, addresses in operands[1:]:
+                ops.replay(replay, tensors, addresses)
         return left, end - 1
 
     def forward(self, step, caches) -> torch.Tensor:

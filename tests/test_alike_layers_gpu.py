@@ -139,3 +139,19 @@ def test_a_function_replaced_on_its_class_is_called_for_every_layer(monkeypatch,
     monkeypatch.setattr(cls, name, lambda *a, **kw: (calls.append(1), plain(*a, **kw))[1])
     steps(runner, [60])
     assert not replays and len(calls) >= 2 * LAYERS * a_layer
+
+
+def test_weights_that_ask_for_gradients(monkeypatch, replays):
+    """Products of the library's go into tensors that are there, which torch refuses where a gradient is asked for."""
+    def run():
+        runner = made("bfloat16")
+        for block in runner.model.blocks:
+            for linear in (block.mixer.qkv, block.mixer.o, block.feed_forward.gate_up, block.feed_forward.down):
+                linear.weight.requires_grad_(True)
+        return steps(runner, [300, 200])
+
+    got = run()
+    assert replays
+    monkeypatch.setattr(DecoderLM, "ALIKE_LAYERS", 10 ** 6)
+    for a, b in zip(got, run()):
+        assert torch.equal(a, b)
