@@ -41,7 +41,9 @@ _of_kind = {}  # (dtype, device) -> a tensor of no elements: its new_empty() tak
 def _made(shape, dtype, device) -> torch.Tensor:
     kind = _of_kind.get((dtype, device))
     if kind is None:
-        kind = _of_kind[dtype, device] = torch.empty((0,), dtype=dtype, device=device)
+        kind = torch.empty((0,), dtype=dtype, device=device)
+        if type(kind) is torch.Tensor:  # (a tracing mode's own kind would be found long after the mode)
+            _of_kind[dtype, device] = kind
     t = kind.new_empty(shape)
     if _recording.to is not None:
         _recording.to.made.append(t)

@@ -80,3 +80,18 @@ def test_a_class_with_another_function(cls, name, monkeypatch):
     assert not parts_as_written()
     monkeypatch.undo()
     assert parts_as_written()
+
+
+def test_results_made_after_a_tracing_mode():
+    """What a mode of fake tensors has made is not what later results are made like."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from litellmengine_amd.csrc import ops
+
+    kind, cpu = torch.float64, torch.device("cpu")
+    with FakeTensorMode():
+        ops._made((2,), dtype=kind, device=cpu)
+    try:
+        assert type(ops._made((2,), dtype=kind, device=cpu)) is torch.Tensor
+    finally:
+        ops._of_kind.pop((kind, cpu), None)
