@@ -2321,14 +2321,19 @@ class HipOps:
         most, share = max(1, heads * chunks // (2 * self.compute_units())), heads // groups
         return max(k for k in range(1, share + 1) if share % k == 0 and (k <= most or k == 1))
 
-    def ssd_streams(self, num_tokens: int, num_seqs: int, heads: int, vdim: int, n: int, longest: int) -> bool:
+    def ssd_streams(self, num_tokens: int, heads: int, vdim: int, n: int, longest: int) -> bool:
         """Whether the chunks of long requests go one after the other, the state in registers (ssd_stream_kernel): up to 512 tokens, and beyond
         where the long requests' workgroups (a head and sixteen value channels each) are as many as the CUs.  With fewer the chain of the chunks
         is what takes the time: 32 heads of 64 x 128, chunks side by side / one after the other, one request of 256, 512, 1024, 2048 tokens
         34 / 24, 39 / 36, 54 / 59, 76 / 101 us; two of 1024 77 / 64; 64 heads, one request of 1024, 2048, 4096 tokens 76 / 63, 120 / 107, 224 / 189.
+        Where those workgroups are fewer than 128 the chunks side by side catch up earlier, the more so the smaller a head (one request of 256, 320, 448, 512
+        tokens, side by side / one after the other: 4 heads of 16 23 / 23, 23 / 25, 23 / 30, 23 / 33; 32 of 32 in 16 groups 27 / 29, 29 / 33, 30 / 39, 30 / 41;
+        8 of 64 30 / 23, 30 / 26, 31 / 31, 32 / 34; 64 of 16 25 / 23, 30 / 26, 31 / 31, 31 / 34).  Heads that share no group read four times as much and gain
+        less: 64 heads of 64 in 64 groups, four requests of 256, 512 tokens 109 / 101, 194 / 204.
         Requests of 32768 tokens and more have not been measured and stay as they were."""
-        few = max(1, (num_tokens - num_seqs) // max(1, longest)) * heads * (vdim // 16) < self.compute_units()
-        return n == 128 and vdim % 16 == 0 and longest < 1 << 15 and (longest <= 512 or not few)
+        workgroups = max(1, num_tokens // max(1, longest)) * heads * (vdim // 16)  # (of as many long requests as there can be)
+        few = 512 if workgroups >= 128 else 448 if vdim >= 64 else 256
+        return n == 128 and vdim % 16 == 0 and longest < 1 << 15 and (longest <= few or workgroups >= self.compute_units())
 
     def ssd_scan(self, c, dt_in, dt_bias, a_log, D, state, heads: int, groups: int, vdim: int, n: int, seq_slots, cu_tokens,
                  min_q_len: int = 0, max_q_len: int = 0) -> torch.Tensor:
@@ -2360,7 +2365,7 @@ class HipOps:
         if pieces:
             slots = N // self.SSD_CHUNK + S
             # (a chunk's bytes of c are counted in 32 bits there)
-            if S <= 65535 and CC < 1 << 23 and self.ssd_streams(N, S, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
+            if S <= 65535 and CC < 1 << 23 and self.ssd_streams(N, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
                 stream_floats = slots * (G * (2 * self.SSD_CHUNK * 128 + 2560) + H * 5 * self.SSD_CHUNK)  # (lle_ssd_stream_floats)
                 part = _made((stream_floats,), dtype=torch.float32, device=c.device)
             else:

@@ -124,7 +124,7 @@ def test_a_long_request_of_wide_rows(monkeypatch):
     chunks.  Rows and states are those of the chunks side by side."""
     o = ops()
     H, G, vdim, n, N = 512, 1, 64, 128, 32767
-    assert o.ssd_streams(N, 1, H, vdim, n, N) and 4 * N * (H * vdim + 2 * G * n) > 1 << 32
+    assert o.ssd_streams(N, H, vdim, n, N) and 4 * N * (H * vdim + 2 * G * n) > 1 << 32
     gen = torch.Generator(device="cuda").manual_seed(3)
     rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
     c = torch.zeros((N, H * vdim + 2 * G * n), device="cuda")
