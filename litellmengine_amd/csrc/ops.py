@@ -129,14 +129,14 @@ class HipOps:
         self.tuning = tuning or ProductTuning()  # which kernel takes a product (never what it gives, beyond the order of its sums)
 
     # -- plumbing ---------------------------------------------------------
-    def _get(self, lib: str, name: str, argtypes):
+    def _get(self, lib: str, name: str, argtypes, restype=_I):
         """`argtypes`: ctypes' types, or a letter for each (a text is no list that every launch makes anew)."""
         key = (lib, name)
         fn = self._fn.get(key)
         if fn is None:
             fn = getattr(build.load_library(lib), name)
             fn.argtypes = [_TYPES[t] for t in argtypes] if isinstance(argtypes, str) else argtypes
-            fn.restype = ctypes.c_int
+            fn.restype = restype
             self._fn[key] = fn
         return fn
 
@@ -2194,7 +2194,7 @@ class HipOps:
     # 64 / 108; four of 256, 1024 41 / 38, 134 / 129; 32 heads of 128 x 128: one of 128, 192, 2048 25 / 25, 29 / 33, 162 / 291; two of 512
     # 95 / 96, four 194 / 175).
     DELTA_WALK = 160  # most tokens of a request that are always walked
-    DELTA_CHUNK_FLOATS = 1 << 28  # of what the chunks of a step keep, 1 GiB (59000 tokens of 32 heads of 64 x 64); steps of more tokens are walked
+    DELTA_CHUNK_FLOATS = 1 << 28  # of what the chunks of a step keep, 1 GiB (30000 tokens of 32 heads of 64 x 64); steps of more tokens are walked
 
     def delta_scan(self, q, k, v, ba, a_log, dt_bias, state, heads: int, kv_heads: int, dim: int, vdim: int, seq_slots,
                    cu_tokens, decay=None) -> torch.Tensor:
@@ -2366,7 +2366,7 @@ class HipOps:
             slots = N // self.SSD_CHUNK + S
             # (a chunk's bytes of c are counted in 32 bits there)
             if S <= 65535 and CC < 1 << 23 and self.ssd_streams(N, H, int(vdim), int(n), longest) and (c.data_ptr() | y.data_ptr()) % 16 == 0:
-                stream_floats = slots * (G * (2 * self.SSD_CHUNK * 128 + 2560) + H * 5 * self.SSD_CHUNK)  # (lle_ssd_stream_floats)
+                stream_floats = self._get("ssd", "lle_ssd_stream_floats", "IIII", _L)(N, S, H, G)
                 part = _made((stream_floats,), dtype=torch.float32, device=c.device)
             else:
                 part = _made((slots * H * vdim * n,), dtype=torch.float32, device=c.device)
