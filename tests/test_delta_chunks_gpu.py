@@ -1,6 +1,6 @@
 """The delta rule in chunks of sixteen tokens (long requests where they are few) against the plain recurrence: the shortest request that goes in
 chunks and the longest that is walked, last chunks of one and of fifteen tokens, value channels that are no sixteens, one decay
-a head and one a channel, decays of zero and of one, more long requests than go in chunks; what is not finite."""
+a head and one a channel, decays of zero and of one; more long requests than go in chunks; what is not finite."""
 import math
 
 import pytest
@@ -45,6 +45,31 @@ def test_long_requests_in_chunks(dim, vdim, H, G, lens, channel):
         o.DELTA_WALK, c = N, start.clone()
         walked = o.delta_scan(q, k, v, ba, a_log, dt_bias, c, H, G, dim, vdim, slots, cu, decay=decay)
         assert (got - walked).abs().max() < 2e-4 and not torch.equal(got, walked)
+
+
+@pytest.mark.parametrize("H,vdim,lens,chunks", [(130, 16, [350, 350, 1, 1, 1], False), (130, 16, [1] * 5 + [700], True), (2, 64, [1] * 70 + [700], True),
+                                                (32, 64, [250] * 2 + [1] * 66 + [250], False), (32, 64, [250] + [1] * 66 + [450], True)])
+def test_which_requests_go_in_chunks_is_seen_on_the_device(H, vdim, lens, chunks, monkeypatch):
+    """The host launches both; the requests go in chunks where the long ones are few enough, wherever among over 64 requests they are, else they are
+    walked, and never both."""
+    from litellmengine_amd.csrc.ops import HipOps
+
+    o, dim, N, S, rand = HipOps(), 64, sum(lens), len(lens), torch.Generator().manual_seed(H)
+    f = lambda *shape: torch.randn(shape, generator=rand).cuda()
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    q, k, v, ba, a_log, dt_bias = unit(f(N, dim)), unit(f(N, dim)), f(N, H * vdim), f(N, 2 * H), f(H), f(H)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    cu, slots = ints([sum(lens[:i]) for i in range(S + 1)]), ints(list(range(S)))
+    start, names, run = 0.3 * f(S, H * vdim * dim), [], o._run
+    monkeypatch.setattr(o, "_run", lambda lib, name, *a: (names.append(name), run(lib, name, *a))[1])
+    a, b, c = start.clone(), start.clone(), start.clone()
+    want = REF.delta_scan(q, k, v, ba, a_log, dt_bias, a, H, 1, dim, vdim, slots, cu)
+    got = o.delta_scan(q, k, v, ba, a_log, dt_bias, b, H, 1, dim, vdim, slots, cu)
+    assert names == ["lle_delta_chunks", "lle_delta_scan"]
+    assert (got - want).abs().max() < 2e-4 and (a - b).abs().max() < 2e-4  # (as above)
+    o.DELTA_WALK = N
+    walked = o.delta_scan(q, k, v, ba, a_log, dt_bias, c, H, 1, dim, vdim, slots, cu)
+    assert torch.equal(got, walked) != chunks and torch.equal(b, c) != chunks
 
 
 @pytest.mark.parametrize("dim", [64, 128])

@@ -119,6 +119,35 @@ def test_decays_inside_a_chunk_to_two_ulps(a_log):
     assert torch.equal(y[2:].view(-1, H, vdim)[:, :, 0].cpu().double(), got.expand(N - 2, H))  # (nothing happens any more)
 
 
+@pytest.mark.parametrize("what", ["x", "B", "C", "dt", "state"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_what_is_not_finite(what, value, monkeypatch):
+    """In the chunks one after the other nothing is lost that the chunks side by side keep: no row before the token's tile of sixteen, no other state (and
+    no row before the token where its step size is what is not finite, which there is a factor of what an earlier row takes 0 times)."""
+    o = ops()
+    H, G, vdim, N, token = 4, 2, 32, 150, 88
+    c, dt_in, dt_bias, a_log, D, wide, seq_slots, cu = ssd_case(H, G, vdim, 128, [N])
+    inner, slot = H * vdim, int(seq_slots[0])
+    if what == "state":
+        wide[slot, 3 * vdim * 128 + 7] = value
+    elif what == "dt":
+        dt_in[token, 1] = value
+    else:
+        c[token, {"x": vdim + 3, "B": inner + 5, "C": inner + G * 128 + 5}[what]] = value
+    got = {}
+    for streams in (True, False):
+        monkeypatch.setattr(o, "ssd_streams", lambda *a, s=streams: s)
+        state = wide.clone()
+        got[streams] = o.ssd_scan(c, dt_in, dt_bias, a_log, D, state, H, G, vdim, 128, seq_slots, cu, N, N), state
+    assert torch.equal(got[True][1].isfinite(), got[False][1].isfinite())
+    for a, b in zip(got[True], got[False]):
+        fine = b.isfinite()  # (tolerance as above)
+        assert a[fine].isfinite().all()
+        assert (a - b)[fine].abs().max() < 2 * 64 * 2**-24 * max(1.0, float(b[fine].abs().max()))
+    if what != "state":
+        assert got[True][0][: token if what == "dt" else token // 16 * 16].isfinite().all() and not got[True][0][token].isfinite().all()
+
+
 def test_a_long_request_of_wide_rows(monkeypatch):
     """32767 tokens of 512 heads: the rest of the request behind a chunk is over 4 GiB, so that a count of its bytes in 32 bits is too small for the first
     chunks.  Rows and states are those of the chunks side by side."""
