@@ -142,22 +142,10 @@ def is_own_function(owner, name: str, value) -> bool:
 
 class Part:
     _written: Dict[type, Written] = {}  # every kind of part
-    _replaced: frozenset = frozenset()  # of an instance: its class's functions in whose place it has others
 
     def __init_subclass__(cls, **kwargs):
         super().__init_subclass__(**kwargs)
         Part._written[cls] = Written(cls)
-
-    def __setattr__(self, name, value):
-        if callable(getattr(type(self), name, None)):
-            others = self._replaced - {name} if is_own_function(self, name, value) else self._replaced | {name}
-            object.__setattr__(self, "_replaced", others)
-        object.__setattr__(self, name, value)
-
-    def __delattr__(self, name):
-        object.__delattr__(self, name)
-        if name in self._replaced:
-            object.__setattr__(self, "_replaced", self._replaced - {name})
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
         """Checkpoint tensors of this part, by full name."""
@@ -175,7 +163,8 @@ class Part:
         return None
 
     def _as_made(self, cls) -> bool:
-        return type(self) is cls and not self._replaced
+        """Whether this is a `cls` and no other kind, with the class's own forward."""
+        return type(self) is cls and "forward" not in self.__dict__
 
 
 Part._written[Part] = Written(Part)

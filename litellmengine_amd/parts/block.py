@@ -44,7 +44,9 @@ class PreNormBlock(Block):
         return ScaledSum(y[0], y[1], 1.0) if isinstance(y, tuple) else y
 
     def launches(self):
-        if not self._as_made(PreNormBlock) or self.feed_forward is None:
+        own = self.__dict__
+        if (not self._as_made(PreNormBlock) or self.feed_forward is None or "entry_norm" in own or "chained_norm" in own or "input_norm" in own
+                or "_sum" in own):
             return None
         a, b, c, d = self.norm_in.launches(), self.mixer.launches(), self.norm_post.launches(), self.feed_forward.launches()
         if a is None or b is None or c is None or d is None:

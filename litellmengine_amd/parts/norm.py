@@ -34,7 +34,7 @@ class RMSNorm(Norm):
         self.weight = (w.reshape(1).expand(self.size) if self.scalar else w).contiguous()
 
     def launches(self):
-        return ((self.size, self.eps, self.one_plus), (self.weight,)) if self._as_made(RMSNorm) else None
+        return ((self.size, self.eps, self.one_plus), (self.weight,)) if self._as_made(RMSNorm) and "fold" not in self.__dict__ else None
 
     def add_normed(self, hidden, y, extra=None, then=None) -> torch.Tensor:
         ops = self.ctx.ops

@@ -55,7 +55,7 @@ class RotaryHalfSplit(PositionEncoding):
         return None if s is None else (float(s.factor), float(s.low), float(s.high), float(s.original))
 
     def launches(self):
-        return ((self.theta, self.rotary_dim, self._scaling_key()), ()) if self._as_made(RotaryHalfSplit) else None
+        return ((self.theta, self.rotary_dim, self._scaling_key()), ()) if self._as_made(RotaryHalfSplit) and "fused_rotary" not in self.__dict__ else None
 
     def fused_rotary(self, step):
         # cosines and sines of this step's positions: made by the first layer that asks,
