@@ -776,7 +776,8 @@ __global__ __launch_bounds__(DELTA_THREADS) void delta_chunk_kernel(DeltaArgs a,
 // in order, so what is not on the chain S -> X S -> LDS -> w -> S is not in the chain's wavefronts.
 // What bounds it is that chain, 0.48 us a chunk (16 of the float32 matrix instruction's 32 cycles, a barrier, the trip through LDS): with
 // every wavefront taking its share of the read-outs 0.53, with a barrier that waits for loads 0.74; operands that are never
-// further than L2 change nothing.  32 heads of 64 x 64 with a decay per channel: the chunks' launch 28 us and this one 55 for 2048 tokens, walked 207.
+// further than L2 change nothing.  32 heads of 64 x 64 with a decay per channel: the chunks' launch 29 us and this one 59 for 2048 tokens (31 and
+// 72 behind a prompt's other launches, which leave no operand in a cache), walked 207.  A chunk whose corrections are not finite has its rows made one after the other.
 template <int NW, int AHEAD>
 __global__ __launch_bounds__(2 * NW * LLE_WAVE, NW / 2) void delta_chunk_walk_kernel(DeltaArgs a, int chunks, const float* __restrict__ work) {
     constexpr int KD = 16 * NW, TC = DELTA_TC;

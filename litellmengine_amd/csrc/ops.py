@@ -1145,7 +1145,12 @@ class HipOps:
         385 -> 246, 1375 -> 700 us, 300 tokens behind 4000 231 -> 131, 1000 behind 5000 914 -> 477, 512 behind 2048 beside 20 decoded
         tokens 468 -> 183.  Below two steps for every one of those workgroups, counted in whole blocks, a launch is the chain of one
         workgroup, which is longer here: 200 tokens 23 / 28, eight prompts of 100 23 / 24, 16 tokens behind 6000 34 / 39; 64 behind 2000,
-        at the line, 40 / 38."""
+        at the line, 40 / 38.
+        The longest request's keys stand for every row's, those of a short prompt beside long decoded requests too, whose own are not known here.
+        Measured at 32 / 8 heads, the other kernel -> this one: 32 tokens from an empty cache beside 4 / 20 / 63 decoded at 4096 46 -> 32, 178 -> 128,
+        371 -> 370; 200 beside 20 at 4096 236 -> 143; 200 behind 1000 beside 63 at 1000 184 -> 162.  It loses where the portion's own keys are few and the decoded
+        requests fill the chip, or are few: 200 from an empty cache beside 63 at 1000 117 -> 131, 32 behind 1000 beside 4 at 4096 46 -> 58 (the worst of
+        130 such steps; five lose over 3 %)."""
         group = nq // num_kv_heads
         if not plain or d != 128 or max_q_len * group <= 16:
             return 0
@@ -2190,9 +2195,10 @@ class HipOps:
 
     # Long requests of heads of 64 or 128 key channels go in chunks where their workgroups (one for a head and sixteen value channels) are no
     # more than the CUs: the walk's wavefronts, which share their SIMDs with one another well, are as fast or faster from there on (32
-    # heads of 64 x 64, chunks / walk in us: one request of 128, 256, 2048 tokens 15 / 17, 21 / 29, 83 / 209; two of 192, 1024 23 / 23,
+    # heads of 64 x 64, chunks / walk in us: one request of 128, 256, 2048 tokens 15 / 17, 24 / 29, 88 / 209; two of 192, 1024 23 / 23,
     # 64 / 108; four of 256, 1024 41 / 38, 134 / 129; 32 heads of 128 x 128: one of 128, 192, 2048 25 / 25, 29 / 33, 162 / 291; two of 512
-    # 95 / 96, four 194 / 175).
+    # 95 / 96, four 194 / 175).  A request's sums run in another order in chunks than walked: its last bits follow from how its prompt is cut and from how
+    # many long requests stand beside it; single tokens are always walked.
     DELTA_WALK = 160  # most tokens of a request that are always walked
     DELTA_CHUNK_FLOATS = 1 << 28  # of what the chunks of a step keep, 1 GiB (30000 tokens of 32 heads of 64 x 64); steps of more tokens are walked
 
